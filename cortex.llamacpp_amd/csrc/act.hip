@@ -49,13 +49,7 @@ __global__ __launch_bounds__(256) void norm_quant_kernel(const float *__restrict
         if (want_q8k) {
             uint32_t packed; int bs; float dq;
             wave_quant_q8k(vv, lane, packed, bs, dq);
-            *reinterpret_cast<uint32_t *>(q.qs + (size_t)row * n + e0) = packed;
-            if ((lane & 3) == 0) {
-                const size_t bi = (size_t)row * (n >> 4) + b * 16 + (lane >> 2);
-                q.bsums[bi] = (int16_t)bs;
-                if (bh) { const int hi = bs >> 6; bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }   // mmq_prep_kernel's split, for the MFMA kernels
-            }
-            if (lane == 0) q.d[(size_t)row * nblk + b] = dq;
+            store_q8k(q, row, n, b, lane, packed, bs, dq, bh, bl);
         }
         if (want_q80) {
             uint32_t packed; float d;
@@ -127,13 +121,7 @@ __global__ __launch_bounds__(1024) void norm_quant_wide_kernel(const float *__re
         if (want_q8k) {
             uint32_t packed; int bs; float dq;
             wave_quant_q8k(vv, lane, packed, bs, dq);
-            *reinterpret_cast<uint32_t *>(q.qs + (size_t)row * n + e0) = packed;
-            if ((lane & 3) == 0) {
-                const size_t bi = (size_t)row * (n >> 4) + b * 16 + (lane >> 2);
-                q.bsums[bi] = (int16_t)bs;
-                if (bh) { const int hi = bs >> 6; bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }
-            }
-            if (lane == 0) q.d[(size_t)row * nblk + b] = dq;
+            store_q8k(q, row, n, b, lane, packed, bs, dq, bh, bl);
         }
         if (want_q80) {
             uint32_t packed; float d;
@@ -177,8 +165,7 @@ static int quant_splits(int T, int n) {
 
 hipError_t launch_rmsnorm_quant(const float *x, const float *w, int n, int T, float eps, float *y_f32,
                                 const ActQuant *q, bool want_q8k, bool want_q80, hipStream_t st, int8_t *bh, int8_t *bl) {
-    ActQuant qq;
-    if (q) qq = *q;
+    const ActQuant qq = act_for(q, T);
     if (launch_wide(x, w, n, T, eps, 1, y_f32, qq, (int)(q && want_q8k), (int)(q && want_q80), (q && want_q8k) ? bh : nullptr, bl, st)) return hipGetLastError();
     const int splits = quant_splits(T, n);
     hipLaunchKernelGGL(norm_quant_kernel, dim3(T, splits), dim3(256), 0, st, x, w, n, eps, 1, y_f32, qq,
@@ -186,7 +173,8 @@ hipError_t launch_rmsnorm_quant(const float *x, const float *w, int n, int T, fl
     return hipGetLastError();
 }
 
-hipError_t launch_quantize(const float *x, int n, int T, const ActQuant &q, bool want_q8k, bool want_q80, hipStream_t st, int8_t *bh, int8_t *bl) {
+hipError_t launch_quantize(const float *x, int n, int T, const ActQuant &qa, bool want_q8k, bool want_q80, hipStream_t st, int8_t *bh, int8_t *bl) {
+    const ActQuant q = act_for(&qa, T);
     if (launch_wide(x, nullptr, n, T, 0.0f, 0, nullptr, q, (int)want_q8k, (int)want_q80, want_q8k ? bh : nullptr, bl, st)) return hipGetLastError();
     const int splits = quant_splits(T, n);
     hipLaunchKernelGGL(norm_quant_kernel, dim3(T, splits), dim3(256), 0, st, x, (const float *)nullptr, n, 0.0f, 0,
@@ -209,13 +197,7 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(const float *__restri
         if (want_q8k) {
             uint32_t packed; int bs; float dq;
             wave_quant_q8k(vv, lane, packed, bs, dq);
-            *reinterpret_cast<uint32_t *>(q.qs + (size_t)row * n + e0) = packed;
-            if ((lane & 3) == 0) {
-                const size_t bi = (size_t)row * (n >> 4) + b * 16 + (lane >> 2);
-                q.bsums[bi] = (int16_t)bs;
-                if (bh) { const int hi = bs >> 6; bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }
-            }
-            if (lane == 0) q.d[(size_t)row * nblk + b] = dq;
+            store_q8k(q, row, n, b, lane, packed, bs, dq, bh, bl);
         }
         if (want_q80) {
             uint32_t packed; float d;
@@ -229,7 +211,7 @@ hipError_t launch_swiglu_quant(const float *g, const float *u, int n, int T, con
                                int8_t *bh, int8_t *bl) {
     if ((n % 256) != 0 || T <= 0) return hipErrorInvalidValue;
     const int splits = quant_splits(T, n);
-    hipLaunchKernelGGL(swiglu_quant_kernel, dim3(T, splits), dim3(256), 0, st, g, u, n, q, (int)want_q8k, (int)want_q80, want_q8k ? bh : nullptr, bl);
+    hipLaunchKernelGGL(swiglu_quant_kernel, dim3(T, splits), dim3(256), 0, st, g, u, n, act_for(&q, T), (int)want_q8k, (int)want_q80, want_q8k ? bh : nullptr, bl);
     return hipGetLastError();
 }
 

@@ -542,13 +542,7 @@ __global__ __launch_bounds__(256) void flash_attn_combine_kernel(const float *pa
         if (want_q8k) {
             uint32_t packed; int bs; float dq;
             wave_quant_q8k(vv, lane, packed, bs, dq);
-            *reinterpret_cast<uint32_t *>(q.qs + (size_t)t * E + e0) = packed;
-            if ((lane & 3) == 0) {
-                const size_t bi = (size_t)t * (E >> 4) + b * 16 + (lane >> 2);
-                q.bsums[bi] = (int16_t)bs;
-                if (bh) { const int hi = bs >> 6; bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }   // mmq_prep_kernel's split, for the MFMA kernels
-            }
-            if (lane == 0) q.d[(size_t)t * nblk + b] = dq;
+            store_q8k(q, t, E, b, lane, packed, bs, dq, bh, bl);
         }
         if (want_q80) {
             uint32_t packed; float dd;
@@ -745,8 +739,7 @@ hipError_t launch_flash_attn_decode(const AttnArgs &a, const float *cs_table, Ro
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int nblk = (a.H * a.D) >> 8;
-    ActQuant qq;
-    if (a.out_q) qq = *a.out_q;
+    const ActQuant qq = act_for(a.out_q, a.T);
     hipLaunchKernelGGL(flash_attn_combine_kernel, dim3(nblk, a.T), dim3(256), (size_t)(256 / a.D) * a.splits * 4, st, a.part, a.out, a.H, a.D, a.splits,
                        qq, (int)(a.out_q && a.out_q8k), (int)(a.out_q && a.out_q80), a.tok_nchunks, a.out_q ? a.out_bh : nullptr, a.out_q ? a.out_bl : nullptr);
     return hipGetLastError();
@@ -839,7 +832,7 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
     if (e != hipSuccess || counters) return e;
     const int nblk = (a.H * a.D) >> 8;
     hipLaunchKernelGGL(flash_attn_combine_kernel, dim3(nblk, 1), dim3(256), (size_t)(256 / a.D) * a.splits * 4, st, a.part, a.out, a.H, a.D, a.splits,
-                       fz.q, fz.want_q8k, fz.want_q80, (const int32_t *)nullptr, (int8_t *)nullptr, (int8_t *)nullptr);
+                       act_for(a.out_q, 1), fz.want_q8k, fz.want_q80, (const int32_t *)nullptr, (int8_t *)nullptr, (int8_t *)nullptr);
     return hipGetLastError();
 }
 
@@ -887,13 +880,7 @@ __global__ __launch_bounds__(256) void flash_attn_combine_wave_kernel(const floa
     if (want_q8k) {
         uint32_t packed; int bs; float dq;
         wave_quant_q8k(acc, lane, packed, bs, dq);
-        *reinterpret_cast<uint32_t *>(q.qs + (size_t)t * E + e0) = packed;
-        if ((lane & 3) == 0) {
-            const size_t bi = (size_t)t * (E >> 4) + b * 16 + (lane >> 2);
-            q.bsums[bi] = (int16_t)bs;
-            if (bh) { const int hi = bs >> 6; bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }
-        }
-        if (lane == 0) q.d[(size_t)t * nblk + b] = dq;
+        store_q8k(q, t, E, b, lane, packed, bs, dq, bh, bl);
     }
     if (want_q80) {
         uint32_t packed; float dd;
@@ -909,8 +896,7 @@ size_t flash_attn_workspace_floats(int T, int H, int D, int splits) { return (si
 hipError_t launch_flash_attn_combine(const AttnArgs &a, int splits, hipStream_t st) {
     if (a.D != 64 && a.D != 128) return hipErrorInvalidValue;
     const int nblk = (a.H * a.D) >> 8;
-    ActQuant qq;
-    if (a.out_q) qq = *a.out_q;
+    const ActQuant qq = act_for(a.out_q, a.T);
     static const bool wave_off = getenv("MI355_ATTN_COMBINE_WAVE") && getenv("MI355_ATTN_COMBINE_WAVE")[0] == '0';
     if (!wave_off && a.T >= 32 && splits <= 64) {                 // prompt batches: one wave per block
         const dim3 grid((unsigned)((nblk + 3) / 4), (unsigned)a.T);
@@ -1104,8 +1090,7 @@ hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st) {
 #undef FA_CASE
     if (e != hipSuccess) return e;
     const int nblk = (a.H * a.D) >> 8;
-    ActQuant qq;
-    if (a.out_q) qq = *a.out_q;
+    const ActQuant qq = act_for(a.out_q, a.T);
     hipLaunchKernelGGL(flash_attn_combine_kernel, dim3(nblk, a.T), dim3(256), (size_t)(256 / a.D) * a.splits * 4, st, a.part, a.out, a.H, a.D, a.splits,
                        qq, (int)(a.out_q && a.out_q8k), (int)(a.out_q && a.out_q80), a.tok_nchunks, a.out_q ? a.out_bh : nullptr, a.out_q ? a.out_bl : nullptr);
     return hipGetLastError();

@@ -55,7 +55,7 @@ struct DecodeFuse {
     const float *knew, *vnew;      // [G*D] un-rotated K and V of the token
     const int32_t *tok_cell;       // [1]
     unsigned *counters;            // [G] words ATT_SYNC_STRIDE apart (a 128-byte line each), zero between launches
-    ActQuant q;
+    ActRows q;
     int want_q8k, want_q80;
     int neox;                      // rotary pairing (i, i + D / 2) instead of (2i, 2i + 1): qwen2-type files; the whole head rotates (n_rot == D)
     // diagnosis (MI355_ATTN_PROBE=1): 100 MHz wall-clock stamps.  [2 * wg], [2 * wg + 1] = start / partials-stored of every

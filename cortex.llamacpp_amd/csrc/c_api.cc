@@ -417,12 +417,13 @@ bool need_device() {
     return mi355_backend_init() == MI355_OK;
 }
 struct ActBufs {
-    DevBuf qs, d, bs, qs0, d0;
+    DevBuf qs, d, bs, qs0, d0, qf;
     ActQuant q;
-    ActBufs(size_t K, size_t T) : qs(T * K), d(T * (K / 256 + 1) * 4), bs(T * (K / 16 + 1) * 2), qs0(T * K), d0(T * (K / 32 + 1) * 2) {
+    ActBufs(size_t K, size_t T) : qs(T * K), d(T * (K / 256 + 1) * 4), bs(T * (K / 16 + 1) * 2), qs0(T * K), d0(T * (K / 32 + 1) * 2), qf(few_bytes((int64_t)K) + 16) {
+        if (few_bytes((int64_t)K)) q.qf = qf.as<uint8_t>();
         q.qs = qs.as<int8_t>(); q.d = d.as<float>(); q.bsums = bs.as<int16_t>(); q.qs0 = qs0.as<int8_t>(); q.d0 = d0.as<uint16_t>();
     }
-    bool ok() const { return qs.p && d.p && bs.p && qs0.p && d0.p; }
+    bool ok() const { return qs.p && d.p && bs.p && qs0.p && d0.p && qf.p; }
 };
 int hip_fail(hipError_t e, const char *what) {
     fail(std::string(what) + ": " + hipGetErrorString(e));
@@ -499,7 +500,7 @@ int mi355_op_mul_mat(int32_t type, const void *W, int64_t N, int64_t K, const fl
             if (e == hipSuccess) e = hipDeviceSynchronize();
             if (e != hipSuccess) return hip_fail(e, "mmq_q80 (copy)");
         } else
-        if (g_op_mmq_ksplit && mmq_ksplit_applicable(type, (int)K, (int)T)) {
+        if (g_op_mmq_ksplit && mmq_ksplit_applicable(type, (int)K, (int)T, ab.q.qf != nullptr)) {
             DevBuf bh(mmq_prep_bytes((int)K, (int)T)), bl(mmq_prep_bytes((int)K, (int)T));
             if (!bh.p || !bl.p) return MI355_ERR_OOM;
             e = launch_mmq_prep(ab.q, (int)K, (int)T, bh.as<int8_t>(), bl.as<int8_t>(), nullptr);

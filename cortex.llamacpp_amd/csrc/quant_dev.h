@@ -4,6 +4,7 @@
 #pragma once
 
 #include "dev_common.h"
+#include "kernels.h"
 
 namespace mi355 {
 
@@ -78,6 +79,26 @@ __device__ __forceinline__ void wave_quant_q8k_batch(const float (&vv)[N][4], in
         bs += dpp_i<DPP_QP_1032>(bs);
         bs += dpp_i<DPP_QP_2301>(bs);
         bsum16[i] = bs;
+    }
+}
+
+// Lane's share of one quantised block (wave_quant_q8k): block b of row `row` of n elements, in every layout that is asked for
+__device__ __forceinline__ void store_q8k(const ActQuant &q, int row, int n, int b, int lane, uint32_t packed, int bs, float d, int8_t *bh, int8_t *bl) {
+    const int nblk = n >> 8;
+    *reinterpret_cast<uint32_t *>(q.qs + (size_t)row * n + b * 256 + lane * 4) = packed;
+    const int hi = bs >> 6;                                    // mmq_prep_kernel's split, for the MFMA kernels
+    if ((lane & 3) == 0) {
+        const size_t bi = (size_t)row * (n >> 4) + b * 16 + (lane >> 2);
+        q.bsums[bi] = (int16_t)bs;
+        if (bh) { bh[bi] = (int8_t)hi; bl[bi] = (int8_t)(bs - 64 * hi); }
+    }
+    if (lane == 0) q.d[(size_t)row * nblk + b] = d;
+    if (q.qf) {
+        uint8_t *f = q.qf + (size_t)((row >> 4) * nblk + b) * FEW_BLOCK;
+        const int t = row & 15;
+        *reinterpret_cast<uint32_t *>(f + (lane >> 4) * 1024 + (t + 16 * (lane >> 1 & 3)) * 16 + (lane >> 3 & 1) * 8 + (lane & 1) * 4) = packed;
+        if ((lane & 3) == 0) { f[FEW_BH + t * 16 + (lane >> 2)] = (uint8_t)hi; f[FEW_BL + t * 16 + (lane >> 2)] = (uint8_t)(bs - 64 * hi); }
+        if (lane == 0) *reinterpret_cast<float *>(f + FEW_D + t * 4) = d;
     }
 }
 

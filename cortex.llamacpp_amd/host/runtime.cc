@@ -566,7 +566,7 @@ void *Context::dalloc(size_t bytes) {
     return p;
 }
 
-static void alloc_actq(ActQuant &q, size_t K, size_t T, bool k, bool z, std::vector<void *> &track, uint64_t &tot, bool &ok) {
+static void alloc_actq(ActQuant &q, size_t K, size_t T, bool k, bool z, std::vector<void *> &track, uint64_t &tot, bool &ok, bool few = false) {
     auto al = [&](size_t b) -> void * {
         void *p = nullptr;
         b = (b + 255) & ~(size_t)255;
@@ -579,6 +579,7 @@ static void alloc_actq(ActQuant &q, size_t K, size_t T, bool k, bool z, std::vec
         q.qs = (int8_t *)al(T * K);
         q.d = (float *)al(T * (K / 256) * 4);
         q.bsums = (int16_t *)al(T * (K / 16) * 2);
+        if (few && T >= 2 && few_bytes((int64_t)K)) q.qf = (uint8_t *)al(few_bytes((int64_t)K));
     }
     if (z) {
         q.qs0 = (int8_t *)al(T * K);
@@ -673,9 +674,9 @@ bool Context::init(std::string &err) {
         }
     }
     bool ok = true;
-    alloc_actq(aq_e_, E, T, true, true, allocs_, device_bytes, ok);
-    alloc_actq(aq_o_, E, T, true, true, allocs_, device_bytes, ok);
-    alloc_actq(aq_ff_, FF, T, true, true, allocs_, device_bytes, ok);
+    alloc_actq(aq_e_, E, T, true, true, allocs_, device_bytes, ok, true);
+    alloc_actq(aq_o_, E, T, true, true, allocs_, device_bytes, ok, true);
+    alloc_actq(aq_ff_, FF, T, true, true, allocs_, device_bytes, ok, true);
     const int prep_rows = (int)T * (hp.n_expert > 0 ? std::max(1, (int)hp.n_expert_used) : 1);   // (expert batches: every (token, rank) pair is a row)
     mmq_bh_ = (int8_t *)dalloc(mmq_prep_bytes((int)std::max(E, FF), prep_rows));
     mmq_bl_ = (int8_t *)dalloc(mmq_prep_bytes((int)std::max(E, FF), prep_rows));
@@ -949,8 +950,9 @@ static hipError_t mmvq_tokens(MMVQSeg *segs, int n_seg, int K, int T, int epi, c
     return hipSuccess;
 }
 
-hipError_t Context::ensure_prep(const ActQuant &aq, int K, int T) {
-    if (prep_owner_ == aq.qs && prep_K_ == K && prep_T_ == T && aq.qs) return hipSuccess;
+// few: the launch takes the quantiser's operand blocks (mmq_few.hip), which hold the block sums' planes already
+hipError_t Context::ensure_prep(const ActQuant &aq, int K, int T, bool few) {
+    if ((prep_owner_ == aq.qs && prep_K_ == K && prep_T_ == T && aq.qs) || few) return hipSuccess;
     HIP_TRY(launch_mmq_prep(aq, K, T, mmq_bh_, mmq_bl_, stream_));
     prep_written(aq, K, T);
     return hipSuccess;
@@ -969,8 +971,8 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
             return launch_mmq_q80(w.data, w.row_bytes, (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         // (bh_over_ / bl_over_: the caller prepared the block-sum planes of a larger batch that aq's rows are a slice of - the expert loop)
         const int8_t *bh = bh_over_ ? bh_over_ : mmq_bh_, *bl = bh_over_ ? bl_over_ : mmq_bl_;
-        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
-            if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T));
+        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, aq.qf != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
+            if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
             return launch_mmq_ksplit(w.type, w.data, w.row_bytes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         }
         if (mmq_applicable(w.type, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // prompt processing: MFMA path
@@ -998,9 +1000,9 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     for (int i = 0; i < n; i++) all_q &= is_quant(ws[i]->type);
     const int K = (int)ws[0]->K;
     bool all_mmq = true, all_ks = true;
-    for (int i = 0; i < n; i++) { all_mmq &= mmq_applicable(ws[i]->type, K, T); all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T); }
+    for (int i = 0; i < n; i++) { all_mmq &= mmq_applicable(ws[i]->type, K, T); all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T, aq.qf != nullptr); }
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
-        HIP_TRY(ensure_prep(aq, K, T));
+        HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
         MMQSeg sg[3];
         for (int i = 0; i < n; i++) sg[i] = MMQSeg{ws[i]->data, ws[i]->row_bytes, (int)ws[i]->N, ws[i]->type, outs[i], (int)ws[i]->N, nullptr, 0};
         return launch_mmq_ksplit_multi(sg, n, K, T, aq, mmq_bh_, mmq_bl_, false, stream_);
@@ -1694,18 +1696,19 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             bool swiglu_quantised = false;
             const bool ffn_mmq = (mmq_q80_applicable(L.gate.type, E, T) && mmq_q80_applicable(L.up.type, E, T)) ||
                                  (mmq_applicable(L.gate.type, E, T) && mmq_applicable(L.up.type, E, T)) ||
-                                 (mmq_ksplit_applicable(L.gate.type, E, T) && mmq_ksplit_applicable(L.up.type, E, T)) ||
+                                 (mmq_ksplit_applicable(L.gate.type, E, T, aq_e_.qf != nullptr) && mmq_ksplit_applicable(L.up.type, E, T, aq_e_.qf != nullptr)) ||
                                  (planes_small(L.gate, E, T) && planes_small(L.up, E, T)) || (q80_copy(L.gate, E, T) && q80_copy(L.up, E, T));
-            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, true) &&
-                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, true) && !fuse_ffn;
+            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, aq_e_.qf != nullptr, true) &&
+                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, aq_e_.qf != nullptr, true) && !fuse_ffn;
             if (gq && uq && L.gate.type == L.up.type && !ffn_mmq) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
                 HIP_TRY(mmvq_tokens(segs, 2, E, T, EPI_SWIGLU, aq_e_, stream_, fz));
             } else if (ffn_ks) {                               // batched decode step: gate and up in one launch
-                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, T));
+                const bool few = aq_e_.qf && T <= FEW_MAX_T;
+                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, T, few));
                 MMQSeg sg[2] = {{L.gate.data, L.gate.row_bytes, (int)L.gate.N, L.gate.type, ffn_, FF, nullptr, 0},
                                 {L.up.data, L.up.row_bytes, (int)L.up.N, L.up.type, ffn_u_, FF, nullptr, 0}};
-                const bool pair = T <= 32 && L.gate.type == L.up.type && L.gate.N == L.up.N;     // SwiGLU in the epilogue
+                const bool pair = (few || T <= 32) && L.gate.type == L.up.type && L.gate.N == L.up.N;     // SwiGLU in the epilogue
                 HIP_TRY(launch_mmq_ksplit_multi(sg, 2, E, T, aq_e_, mmq_bh_, mmq_bl_, pair, stream_));
                 if (!pair) {
                     if (is_quant(L.down.type) && (FF % 256) == 0) {

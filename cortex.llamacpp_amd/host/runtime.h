@@ -277,7 +277,7 @@ class Context {
     // the planes themselves, launch_mmq_prep runs only when they are not there (ensure_prep)
     const void *prep_owner_ = nullptr;
     int prep_K_ = 0, prep_T_ = 0;
-    hipError_t ensure_prep(const ActQuant &aq, int K, int T);
+    hipError_t ensure_prep(const ActQuant &aq, int K, int T, bool few = false);
     void prep_written(const ActQuant &aq, int K, int T) { prep_owner_ = aq.qs; prep_K_ = K; prep_T_ = T; }
     bool batch_distinct_ = false;                    // the micro-batch is one token each of different sequences (decode_ubatch)
     const int8_t *bh_over_ = nullptr, *bl_over_ = nullptr;   // linear(): block-sum planes prepared by the caller for a slice of a larger batch
