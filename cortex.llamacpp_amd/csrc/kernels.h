@@ -6,6 +6,8 @@
 
 namespace mi355 {
 
+struct KVLayerView;
+
 // ---------------------------------------------------------------- quantised activations (device)
 // Q8_K: codes + one f32 scale per 256 + int16 sums per 16 (ggml block_q8_K split into planes);
 // Q8_0: codes + one f16 scale per 32 (ggml block_q8_0 split into planes).
@@ -248,6 +250,11 @@ hipError_t launch_mmf16(const uint8_t *W, int n_rows, int K, const float *x, int
 // the same with the activation rows rounded to f16 beforehand (once per row instead of once per workgroup that reads it): xh [T][K] halves
 hipError_t launch_f32_to_f16(const float *x, void *y, size_t n, hipStream_t st);
 // y = resid + (W xh + bias) * scale - bias [n_rows], the scale and resid [T][ld_out] each optional (resid may be y itself)
+// the encoder's projections: few rows and columns, K shared by a workgroup's waves (mmf.hip mmf16_few_kernel)
+bool mmf16_few_applicable(int n_rows, int K, int T);
+hipError_t launch_mmf16_few(const uint8_t *W, int n_rows, int K, const void *x, bool x_f16, int T, float *out, const float *resid, const float *bias, hipStream_t st);
+hipError_t launch_mmf16_few_swiglu(const uint8_t *W_gate, const uint8_t *W_up, int n_rows, int K, const void *xh, int T, void *out_h, hipStream_t st);
+hipError_t launch_mmf16_few_qkv_rope(const uint8_t *W, int E, int K, const void *xh, int T, float *q, const float *cs, const int32_t *cell, struct KVLayerView kv, int n_ctx, hipStream_t st);
 hipError_t launch_mmf16_xh(const uint8_t *W, int n_rows, int K, const void *xh, int T, float *y, int ld_out, const float *resid, const float *bias, float scale, bool do_scale,
                            hipStream_t st);
 hipError_t launch_mmv_float(int type, const uint8_t *W, int n_rows, int K, const float *x, int T, float *y, int ld_out,

@@ -237,4 +237,201 @@ hipError_t launch_mmf16_xh(const uint8_t *W, int n_rows, int K, const void *xh, 
     return launch_mmf16_t<true>(W, n_rows, K, xh, T, y, ld_out, resid, bias, scale, do_scale, st);
 }
 
+namespace {
+// The encoder's projections (T tokens of one text against f16 weights of a few hundred to a few thousand columns): a product is 19 MB of weights at the most and
+// some microseconds of anything, so what counts is one trip to memory, enough workgroups and no launches around it.  Measured on nomic-embed (768 / 3072 columns)
+// at 187 tokens: 768 x 768 30 us with the 64 x 64 direct kernel above (36 workgroups, one load in flight, 32 lines per request).  Here:
+//   * 32 rows x 32 TT tokens per workgroup (432 workgroups for Q | K | V at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
+//     both operands - all of them for 768 columns - are requested before the first matrix step;
+//   * a request is whole 128-byte lines of eight rows; the operands (16 bytes of 32 rows) are made through LDS of the wave's own, rows padded to 144 bytes.  Asked for as
+//     operands, 32 lines per request: gate | up 20.8 us at 187 tokens and 92 at 1800;
+//   * partial tiles meet in LDS (rows padded to 36 floats: conflict-free both ways) and are summed in wave order;
+//   * two products of the same tokens share a workgroup (NP = 2): gate and up, which leave silu(gate) * up as f16, or the two halves of a head's 64 dimensions of
+//     Q | K | V, whose pairs (d, d + 32) are turned by their angle on the way out - Q to its rows, K and V straight into their cells of the f16 cache;
+//   * bias and residual are added on the way out.
+// XF: the activations are f32 rows, rounded to f16 in registers (the attention's output).
+enum { FEW_PLAIN, FEW_SWIGLU, FEW_ROPE };
+struct MMF16Few {
+    const _Float16 *W, *W2; const void *X;
+    float *out; _Float16 *out_h;
+    const float *resid, *bias;
+    int N, K, T;
+    const float *cs; const int32_t *cell; uint16_t *kc, *vc; int n_ctx;       // FEW_ROPE: cos, sin of every token's 32 pairs, the tokens' cells, the layer's cache planes
+};
+template <int NW, int EPI, int TT, int PD, bool XF>
+__global__ __launch_bounds__(64 * NW) void mmf16_few_kernel(const MMF16Few a) {
+    constexpr int NP = EPI == FEW_PLAIN ? 1 : 2, ROWS = EPI == FEW_ROPE ? 64 : 32;
+    constexpr int LD = 36, LDR = 72, STAGE = (NP + TT) * 32 * LDR;                                     // floats per row of a partial tile; halves per row of a staged chunk
+    constexpr int PART_BYTES = NW * NP * TT * 32 * LD * 4, STAGE_BYTES = NW * STAGE * 2;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[PART_BYTES > STAGE_BYTES ? PART_BYTES : STAGE_BYTES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m = lane & 31, kg = lane >> 5;
+    const int n0 = blockIdx.x * ROWS, t0 = blockIdx.y * (32 * TT), r8 = lane >> 3, c8 = 8 * (lane & 7);
+    float *part = reinterpret_cast<float *>(smem);
+    _Float16 *stage = reinterpret_cast<_Float16 *>(smem) + wave * STAGE;
+    // request i of an operand tile: row r8 + 8 i, its halves c8 .. of the chunk; rows past the end read the last one (their results are never stored)
+    unsigned wrow[4], xrow[TT][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int g = n0 + r8 + 8 * i;
+        wrow[i] = (unsigned)(g < a.N ? g : a.N - 1) * (unsigned)a.K + c8;
+#pragma unroll
+        for (int t = 0; t < TT; t++) { const int h = t0 + 32 * t + r8 + 8 * i; xrow[t][i] = (unsigned)(h < a.T ? h : a.T - 1) * (unsigned)a.K + c8; }
+    }
+    const _Float16 *W[NP] = {a.W};
+    if constexpr (NP == 2) W[1] = a.W2;
+    struct Slot { f16x8 w[NP][4]; f16x8 x[TT][XF ? 1 : 4]; f32x4 xf[TT][XF ? 8 : 1]; };
+    Slot s[PD];
+    const int nc = a.K >> 6, cn = wave < nc ? (nc - wave + NW - 1) / NW : 0;                          // this wave's chunks: wave, wave + NW, ..
+    const int last = nc - 1;
+    auto fetch = [&](Slot &v, int i) {
+        const unsigned k = 64u * (unsigned)(wave + NW * i < last ? wave + NW * i : last);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+#pragma unroll
+            for (int p = 0; p < NP; p++) v.w[p][j] = *reinterpret_cast<const f16x8 *>(W[p] + (wrow[j] + k));
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                if constexpr (XF) {
+                    const float *x = reinterpret_cast<const float *>(a.X) + (xrow[t][j] + k);
+                    v.xf[t][2 * j] = *reinterpret_cast<const f32x4 *>(x); v.xf[t][2 * j + 1] = *reinterpret_cast<const f32x4 *>(x + 4);
+                } else v.x[t][j] = *reinterpret_cast<const f16x8 *>(reinterpret_cast<const _Float16 *>(a.X) + (xrow[t][j] + k));
+            }
+        }
+    };
+    f32x16 acc[NP][TT];
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[p][t][r] = 0.0f;
+    auto put = [&](const Slot &v) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            _Float16 *d = stage + (r8 + 8 * j) * LDR + c8;
+#pragma unroll
+            for (int p = 0; p < NP; p++) *reinterpret_cast<f16x8 *>(d + p * 32 * LDR) = v.w[p][j];
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                f16x8 b;
+                if constexpr (XF) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) { b[e] = (_Float16)v.xf[t][2 * j][e]; b[4 + e] = (_Float16)v.xf[t][2 * j + 1][e]; }
+                } else b = v.x[t][j];
+                *reinterpret_cast<f16x8 *>(d + (NP + t) * 32 * LDR) = b;
+            }
+        }
+    };
+    auto use = [&]() {
+        const _Float16 *f = stage + m * LDR + 8 * kg;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            f16x8 w[NP];
+#pragma unroll
+            for (int p = 0; p < NP; p++) w[p] = *reinterpret_cast<const f16x8 *>(f + p * 32 * LDR + 16 * j);
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                const f16x8 b = *reinterpret_cast<const f16x8 *>(f + (NP + t) * 32 * LDR + 16 * j);
+#pragma unroll
+                for (int p = 0; p < NP; p++) acc[p][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[p], b, acc[p][t], 0, 0, 0);
+            }
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < PD; u++) { fetch(s[u], u); __builtin_amdgcn_sched_barrier(0); }               // (in the order of their use: a wait for one slot is not one for the next)
+    int i = 0;
+    for (; i + PD < cn; i += PD)                             // (no branch around a request: it would become a wait for all of them)
+#pragma unroll
+        for (int u = 0; u < PD; u++) {
+            put(s[u]);
+            __builtin_amdgcn_sched_barrier(0);               // (a wave's LDS accesses are made in order)
+            fetch(s[u], i + PD + u);
+            __builtin_amdgcn_sched_barrier(0);
+            use();
+        }
+#pragma unroll
+    for (int u = 0; u < PD; u++) if (i + u < cn) { put(s[u]); __builtin_amdgcn_wave_barrier(); use(); __builtin_amdgcn_wave_barrier(); }
+    __syncthreads();                                         // the partial tiles take the staging area's place
+    // register r of a lane: weight row (r & 3) + 8 (r >> 2) + 4 kg, token = lane & 31
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<f32x4 *>(part + (((wave * NP + p) * TT + t) * 32 + m) * LD + 8 * q + 4 * kg) =
+                    f32x4{acc[p][t][4 * q], acc[p][t][4 * q + 1], acc[p][t][4 * q + 2], acc[p][t][4 * q + 3]};
+    __syncthreads();
+    for (int e = tid; e < 1024 * TT; e += 64 * NW) {
+        const int row = e & 31, t = e >> 5, gt = t0 + t, n = n0 + row;
+        float v[NP];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            v[p] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NW; w++) v[p] += part[(((w * NP + p) * TT + (t >> 5)) * 32 + (t & 31)) * LD + row];
+        }
+        if (gt >= a.T || n >= a.N) continue;
+        if constexpr (EPI == FEW_ROPE) {
+            const int E = a.N / 3, s = n0 / E, c0 = n0 - s * E;         // (a head is a whole tile, a segment whole heads)
+            float y0 = v[0], y1 = v[1];
+            if (s < 2) {
+                const float c = a.cs[(size_t)gt * 64 + 2 * row], sn = a.cs[(size_t)gt * 64 + 2 * row + 1];
+                y0 = v[0] * c - v[1] * sn;
+                y1 = v[0] * sn + v[1] * c;
+            }
+            if (s == 0) { float *q = a.out + (size_t)gt * E + c0 + row; q[0] = y0; q[32] = y1; }
+            else { uint16_t *d = (s == 1 ? a.kc : a.vc) + ((size_t)(c0 >> 6) * a.n_ctx + a.cell[gt]) * 64 + row; d[0] = f2h(y0); d[32] = f2h(y1); }
+        } else {
+            const size_t o = (size_t)gt * a.N + n;
+            if constexpr (EPI == FEW_SWIGLU) a.out_h[o] = (_Float16)((v[0] / (1.0f + expf(-v[0]))) * v[1]);
+            else {
+                float y = v[0];
+                if (a.bias) y = y + a.bias[n];
+                if (a.resid) y = a.resid[o] + y;
+                a.out[o] = y;
+            }
+        }
+    }
+}
+template <int NW, int EPI, bool XF>
+void few_launch(const MMF16Few &a, hipStream_t st) {
+    const int rows = EPI == FEW_ROPE ? 64 : 32;
+    const unsigned gx = (unsigned)((a.N + rows - 1) / rows), gy = (unsigned)((a.T + 31) / 32);
+    // two token tiles per workgroup once there are more workgroups than the chip holds: the weights are read half as often
+    if (gx * gy * (rows / 32) >= 2048) hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 2, XF ? 1 : 2, XF>), dim3(gx, (gy + 1) / 2), dim3(64 * NW), 0, st, a);
+    else hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
+}
+}  // namespace
+
+bool mmf16_few_applicable(int n_rows, int K, int T) {
+    return T >= 8 && n_rows >= 32 && K % 64 == 0 && (size_t)n_rows * K < (1ull << 31) && (size_t)T * K < (1ull << 31);
+}
+// out[t][n_rows] = W X (+ bias) (+ resid); X: [T][K] halves (x_f16) or floats, rounded to f16
+hipError_t launch_mmf16_few(const uint8_t *W, int n_rows, int K, const void *x, bool x_f16, int T, float *out, const float *resid, const float *bias, hipStream_t st) {
+    MMF16Few a{};
+    a.W = reinterpret_cast<const _Float16 *>(W); a.X = x; a.N = n_rows; a.K = K; a.T = T; a.out = out; a.resid = resid; a.bias = bias;
+    const bool wide = K > 1024;                              // eight waves share a longer K
+    if (x_f16) { if (wide) few_launch<8, FEW_PLAIN, false>(a, st); else few_launch<4, FEW_PLAIN, false>(a, st); }
+    else { if (wide) few_launch<8, FEW_PLAIN, true>(a, st); else few_launch<4, FEW_PLAIN, true>(a, st); }
+    return hipGetLastError();
+}
+// out[t][n_rows] = f16(silu(W_gate x) * (W_up x)), x: [T][K] halves
+hipError_t launch_mmf16_few_swiglu(const uint8_t *W_gate, const uint8_t *W_up, int n_rows, int K, const void *xh, int T, void *out_h, hipStream_t st) {
+    MMF16Few a{};
+    a.W = reinterpret_cast<const _Float16 *>(W_gate); a.W2 = reinterpret_cast<const _Float16 *>(W_up); a.X = xh; a.N = n_rows; a.K = K; a.T = T;
+    a.out_h = reinterpret_cast<_Float16 *>(out_h);
+    if (K > 1024) few_launch<8, FEW_SWIGLU, false>(a, st); else few_launch<4, FEW_SWIGLU, false>(a, st);
+    return hipGetLastError();
+}
+// the projections of E = n_head * 64 rows each of W (Q | K | V) for x: [T][K] halves; rope pairs (d, d + 32) by cs[T][64]; q [T][E], k and v into the f16 cache
+hipError_t launch_mmf16_few_qkv_rope(const uint8_t *W, int E, int K, const void *xh, int T, float *q, const float *cs, const int32_t *cell, KVLayerView kv, int n_ctx, hipStream_t st) {
+    if (E % 64) return hipErrorInvalidValue;
+    MMF16Few a{};
+    a.W = reinterpret_cast<const _Float16 *>(W); a.W2 = a.W + (size_t)32 * K; a.X = xh; a.N = 3 * E; a.K = K; a.T = T;
+    a.out = q; a.cs = cs; a.cell = cell; a.kc = reinterpret_cast<uint16_t *>(kv.k); a.vc = reinterpret_cast<uint16_t *>(kv.v); a.n_ctx = n_ctx;
+    if (K > 1024) few_launch<8, FEW_ROPE, false>(a, st); else few_launch<4, FEW_ROPE, false>(a, st);
+    return hipGetLastError();
+}
+
 }  // namespace mi355

@@ -1304,7 +1304,20 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
                                     d_tok_, x_, stream_));
     if (model->tok_types.valid())      // token types are all zero: row 0 of the table on every token
         HIP_TRY(launch_add_qkv_bias(x_, nullptr, nullptr, (const float *)model->tok_types.data, nullptr, nullptr, E, 0, T, stream_));
-    HIP_TRY(launch_layer_norm(x_, (const float *)model->tok_norm.data, (const float *)model->tok_norm_b.data, E, T, hp.eps, x_, stream_));
+    // f16 projections of a batch: one launch for Q | K | V, one for gate | up with SwiGLU, bias and residual inside the others; the rows travel as f16 beside the
+    // f32 residual (what each product rounded its input to), in the feed-forward buffers that these launches leave unused
+    const auto f16_few = [&](const DevTensor &w, int rows, int K) {
+        return w.type == T_F16 && w.n_expert == 1 && mmf16_few_applicable(rows, K, T) && ((uintptr_t)w.data & 15) == 0;
+    };
+    const bool packed = E == H * D && G == H && [&] {
+        for (const LayerWeights &L : model->layers)
+            if (!f16_few(L.wqkv, 3 * E, E) || !f16_few(L.wo, E, E) || !f16_few(L.gate, FF, E) || !f16_few(L.up, FF, E) || !f16_few(L.down, E, FF)) return false;
+        return true;
+    }();
+    // ... with the rope and the cache store on the projections' way out (heads of 64, pairs a half apart)
+    const bool rope_out = packed && D == 64 && ra.neox && ra.n_rot == 64 && cp.type_k == T_F16 && cp.type_v == T_F16 && rope_cs_;
+    void *const xh = packed ? (void *)ffn_u_ : nullptr, *const hh = ffn_;
+    HIP_TRY(launch_layer_norm_h(x_, (const float *)model->tok_norm.data, (const float *)model->tok_norm_b.data, E, T, hp.eps, x_, xh, stream_));
     prof_mark("embed");
     // quantised weight tensors contract against a quantised copy of their input (Q8_K for K-quants, Q8_0 otherwise), float tensors against the f32 rows
     auto quantise_for = [&](const float *x, int K, ActQuant &aq, std::initializer_list<const DevTensor *> ws) -> hipError_t {
@@ -1316,12 +1329,19 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
     };
     for (int il = 0; il < hp.n_layer; il++) {
         const LayerWeights &L = model->layers[(size_t)il];
-        HIP_TRY(quantise_for(x_, E, aq_e_, {&L.wq, &L.wk, &L.wv}));
-        const DevTensor *ws[3] = {&L.wq, &L.wk, &L.wv};
         float *outs[3] = {q_, k_, v_};
-        HIP_TRY(linear_multi(ws, outs, 3, aq_e_, x_, T));
+        if (rope_out) {
+            HIP_TRY(launch_mmf16_few_qkv_rope(L.wqkv.data, E, E, xh, T, q_, rope_cs_, d_cell_, kv_[(size_t)il], (int)cp.n_ctx, stream_));
+        } else if (packed) {
+            const DevTensor *ws[3] = {&L.wq, &L.wk, &L.wv};
+            for (int i = 0; i < 3; i++) HIP_TRY(launch_mmf16_few(ws[i]->data, E, E, xh, true, T, outs[i], nullptr, nullptr, stream_));
+        } else {
+            HIP_TRY(quantise_for(x_, E, aq_e_, {&L.wq, &L.wk, &L.wv}));
+            const DevTensor *ws[3] = {&L.wq, &L.wk, &L.wv};
+            HIP_TRY(linear_multi(ws, outs, 3, aq_e_, x_, T));
+        }
         prof_mark("qkv");
-        HIP_TRY(launch_rope_kv_store(q_, k_, v_, T, H, G, D, d_pos_, d_cell_, ra, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, rope_cs_, stream_));
+        if (!rope_out) HIP_TRY(launch_rope_kv_store(q_, k_, v_, T, H, G, D, d_pos_, d_cell_, ra, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, rope_cs_, stream_));
         prof_mark("rope_kv");
         AttnArgs aa{};
         aa.q = q_; aa.out = att_; aa.kv = kv_[(size_t)il]; aa.type_k = cp.type_k; aa.type_v = cp.type_v;
@@ -1334,6 +1354,18 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
         while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
         HIP_TRY(launch_flash_attn(aa, stream_));
         prof_mark("attn");
+        if (packed) {
+            HIP_TRY(launch_mmf16_few(L.wo.data, E, E, att_, false, T, xn_, x_, L.bo.valid() ? (const float *)L.bo.data : nullptr, stream_));   // + bias, + the layer input
+            HIP_TRY(launch_layer_norm_h(xn_, (const float *)L.attn_out_norm.data, (const float *)L.attn_out_norm_b.data, E, T, hp.eps, xn_, xh, stream_));
+            prof_mark("attn_out");
+            HIP_TRY(launch_mmf16_few_swiglu(L.gate.data, L.up.data, FF, E, xh, T, hh, stream_));
+            prof_mark("ffn_gate_up");
+            HIP_TRY(launch_mmf16_few(L.down.data, E, FF, hh, true, T, x_, xn_, nullptr, stream_));
+            HIP_TRY(launch_layer_norm_h(x_, (const float *)L.layer_out_norm.data, (const float *)L.layer_out_norm_b.data, E, T, hp.eps, x_, xh, stream_));
+            prof_mark("ffn_down");
+            if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
+            continue;
+        }
         HIP_TRY(quantise_for(att_, H * D, aq_o_, {&L.wo}));
         HIP_TRY(linear(L.wo, aq_o_, att_, H * D, T, q_, E, nullptr, EPI_STORE));
         if (L.bo.valid()) HIP_TRY(launch_add_qkv_bias(q_, nullptr, nullptr, (const float *)L.bo.data, nullptr, nullptr, E, 0, T, stream_));
