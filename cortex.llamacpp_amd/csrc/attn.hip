@@ -139,8 +139,10 @@ __global__ void step_setup_kernel(const int32_t *tok_pos, int T, RopeArgs ra, fl
 __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *tok_pos, int T, RopeArgs ra, float theta_scale, float *cs_out, int32_t *cell_pos,
                                                                uint64_t *cell_seq, const int32_t *tok_cell, const uint64_t *tok_seqmask, unsigned *zero_word,
                                                                unsigned *epoch_word, int type, const uint8_t *table, int K, size_t row_bytes,
-                                                               const int32_t *ids, float *dst) {
+                                                               const int32_t *ids, float *dst, const uint32_t *stage_src, uint32_t *stage_dst, int stage_words) {
     const int lin = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+    // a step of one token: its staging block comes out of pinned host memory here (the arrays above point into it) and is left on the device for the launches behind
+    if (lin < stage_words) stage_dst[lin] = stage_src[lin];
     if (blockIdx.x == 0 && blockIdx.y == 0) {
         if (zero_word && threadIdx.x < 9) zero_word[threadIdx.x == 0 ? 0 : 32 * threadIdx.x] = 0u;
         if (epoch_word && threadIdx.x == 0) epoch_word[0] = epoch_word[0] + 1u;
@@ -164,13 +166,14 @@ __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *to
 }
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st) {
+                                   const int32_t *ids, float *dst, hipStream_t st, const void *stage_src, void *stage_dst, int stage_words) {
     const float theta_scale = powf(ra.freq_base, -2.0f / (float)ra.n_rot);
     int bx = (int)((K + 255) / 256);
     if (bx > 64) bx = 64;
     while ((long)bx * T * 256 < (long)T * (ra.n_rot >> 1)) bx++;          // (enough threads for the table: n_rot / 2 <= 256 * bx per token)
     hipLaunchKernelGGL(step_setup_embed_kernel, dim3(bx, T), dim3(256), 0, st, tok_pos, T, ra, theta_scale, cs_out, cell_pos, cell_seq, tok_cell, tok_seqmask,
-                       zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst);
+                       zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst, reinterpret_cast<const uint32_t *>(stage_src),
+                       reinterpret_cast<uint32_t *>(stage_dst), stage_words);
     return hipGetLastError();
 }
 hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,

@@ -607,7 +607,7 @@ hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *
 // launch_step_setup + launch_get_rows (the batch's embedding rows, dst[T][K]) in one launch
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table_dev, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st);
+                                   const int32_t *ids, float *dst, hipStream_t st, const void *stage_src = nullptr, void *stage_dst = nullptr, int stage_words = 0);
 hipError_t launch_rope_inplace(float *x, int T, int n_head, int D, const int32_t *tok_pos, RopeArgs ra, hipStream_t st);
 
 struct AttnArgs {

@@ -240,7 +240,8 @@ hipError_t launch_mmf16_xh(const uint8_t *W, int n_rows, int K, const void *xh, 
 namespace {
 // The encoder's projections (T tokens of one text against f16 weights of a few hundred to a few thousand columns): a product is 19 MB of weights at the most and
 // some microseconds of anything, so what counts is one trip to memory, enough workgroups and no launches around it.  Measured on nomic-embed (768 / 3072 columns)
-// at 187 tokens: 768 x 768 30 us with the 64 x 64 direct kernel above (36 workgroups, one load in flight, 32 lines per request).  Here:
+// at 187 tokens, us: 768 x 768 30 with the 64 x 64 direct
+// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; now Q | K | V 7.4, output 5.8, gate | up 11.5, down 8.9.  Here:
 //   * 32 rows x 32 TT tokens per workgroup (432 workgroups for Q | K | V at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
 //     both operands - all of them for 768 columns - are requested before the first matrix step;
 //   * a request is whole 128-byte lines of eight rows; the operands (16 bytes of 32 rows) are made through LDS of the wave's own, rows padded to 144 bytes.  Asked for as
@@ -398,9 +399,13 @@ template <int NW, int EPI, bool XF>
 void few_launch(const MMF16Few &a, hipStream_t st) {
     const int rows = EPI == FEW_ROPE ? 64 : 32;
     const unsigned gx = (unsigned)((a.N + rows - 1) / rows), gy = (unsigned)((a.T + 31) / 32);
-    // two token tiles per workgroup once there are more workgroups than the chip holds: the weights are read half as often
-    if (gx * gy * (rows / 32) >= 2048) hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 2, XF ? 1 : 2, XF>), dim3(gx, (gy + 1) / 2), dim3(64 * NW), 0, st, a);
-    else hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
+    // two token tiles per workgroup, the weights read half as often, once there are enough workgroups: gate | up at 187 tokens (576 workgroups of one tile) 11.5 us with one
+    // tile and 12.4 with two, at 700 (2112) 24.5 and 23.3; down at 700 (528) 21.2 and 22.0, at 1800 (1368) 42.3 and 34.8.  Not for f32 rows: 17.5 and 18.0 at 1800
+    if constexpr (!XF) if (gx * gy * (rows / 32) >= 1280) {
+        hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 2, 2, XF>), dim3(gx, (gy + 1) / 2), dim3(64 * NW), 0, st, a);
+        return;
+    }
+    hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
 }
 }  // namespace
 

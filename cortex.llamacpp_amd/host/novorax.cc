@@ -251,6 +251,8 @@ bool Context::init_novorax(std::string &err) {
     cells_.assign(NC, KVCell());
     d_cell_pos_ = (int32_t *)dalloc(NC * 4);
     d_cell_seq_ = (uint64_t *)dalloc(NC * 8);
+    if (hipHostMalloc((void **)&h_cell_pos_, NC * 4, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&h_cell_seq_, NC * 8, hipHostMallocDefault) != hipSuccess) { err = "staging allocation failed"; return false; }
     d_delta_ = (int32_t *)dalloc(NC * 4);
     const size_t Tp = (T + 1) & ~(size_t)1;
     stage_bytes_ = 16 + Tp * 4 * 5 + Tp * 8;

@@ -538,6 +538,8 @@ Context::~Context() {
     for (auto &pe : prof_events_) (void)hipEventDestroy(pe.second);
     for (void *p : allocs_) (void)hipFree(p);
     if (h_stage_) (void)hipHostFree(h_stage_);
+    if (h_cell_pos_) (void)hipHostFree(h_cell_pos_);
+    if (h_cell_seq_) (void)hipHostFree(h_cell_seq_);
     if (h_logits_) (void)hipHostFree(h_logits_);
     if (h_argmax_) (void)hipHostFree(h_argmax_);
     if (h_embd_) (void)hipHostFree(h_embd_);
@@ -623,6 +625,8 @@ bool Context::init(std::string &err) {
     }
     d_cell_pos_ = (int32_t *)dalloc(NC * 4);
     d_cell_seq_ = (uint64_t *)dalloc(NC * 8);
+    if (hipHostMalloc((void **)&h_cell_pos_, NC * 4, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&h_cell_seq_, NC * 8, hipHostMallocDefault) != hipSuccess) { err = "pinned alloc failed"; return false; }
     d_delta_ = (int32_t *)dalloc(NC * 4);
     // token staging block: [nkv x4][tok][pos][seq][cell][outrow][seqmask]
     const size_t Tp = (T + 1) & ~(size_t)1;   // keeps the u64 seqmask array 8-byte aligned
@@ -734,10 +738,12 @@ bool Context::init(std::string &err) {
 // ------------------------------------------------------------------------------------------ KV cells
 void Context::kv_clear() {
     if (model->nvx && stream_) nvx_state_reset(-1);
-    for (auto &c : cells_) c = KVCell();
+    for (int i = 0; i < (int)cells_.size(); i++) {
+        if (cells_[(size_t)i].pos >= 0) touch_cell(i);
+        cells_[(size_t)i] = KVCell();
+    }
     head_ = 0;
     has_shift_ = false;
-    meta_dirty_ = true;
     region_next_.clear();
 }
 bool Context::kv_seq_rm(int seq, int p0, int p1) {
@@ -753,17 +759,17 @@ bool Context::kv_seq_rm(int seq, int p0, int p1) {
         }
     }
     int new_head = (int)cells_.size();
-    for (int i = 0; i < (int)cells_.size(); i++) {
+    for (int i = 0; i < cells_end_; i++) {
         KVCell &c = cells_[(size_t)i];
         if (c.pos < p0 || c.pos >= p1) continue;
         if (seq < 0) c.seqs = 0;
         else if (c.seqs & (1ull << seq)) c.seqs &= ~(1ull << seq);
         else continue;
+        touch_cell(i);
         if (!c.seqs) { c.pos = -1; c.delta = 0; if (i < new_head) new_head = i; }
     }
     if (new_head < (int)cells_.size() && new_head < head_) head_ = new_head;
     if (new_head < (int)cells_.size()) region_next_.clear();   // cells came free: the next allocation starts at its region's lowest free cell
-    meta_dirty_ = true;
     return true;
 }
 void Context::kv_seq_cp(int src, int dst, int p0, int p1) {
@@ -771,9 +777,10 @@ void Context::kv_seq_cp(int src, int dst, int p0, int p1) {
     if (p0 < 0) p0 = 0;
     if (p1 < 0) p1 = 0x7fffffff;
     if (model->nvx && p0 == 0) nvx_state_copy(src, dst);             // the recurrent state goes with a copy of the whole sequence
-    for (auto &c : cells_)
-        if ((c.seqs & (1ull << src)) && c.pos >= p0 && c.pos < p1) c.seqs |= 1ull << dst;
-    meta_dirty_ = true;
+    for (int i = 0; i < cells_end_; i++) {
+        KVCell &c = cells_[(size_t)i];
+        if ((c.seqs & (1ull << src)) && c.pos >= p0 && c.pos < p1) { c.seqs |= 1ull << dst; touch_cell(i); }
+    }
 }
 void Context::kv_seq_add(int seq, int p0, int p1, int delta) {
     if (seq < 0 || seq >= 64) return;
@@ -781,14 +788,32 @@ void Context::kv_seq_add(int seq, int p0, int p1, int delta) {
     if (p0 < 0) p0 = 0;
     if (p1 < 0) p1 = 0x7fffffff;
     if (p0 == p1 || delta == 0) return;
-    for (auto &c : cells_) {
+    for (int i = 0; i < cells_end_; i++) {
+        KVCell &c = cells_[(size_t)i];
         if (!(c.seqs & (1ull << seq)) || c.pos < p0 || c.pos >= p1) continue;
+        touch_cell(i);
         has_shift_ = true;
         c.pos += delta;
         c.delta += delta;
         if (c.pos < 0) { c.pos = -1; c.seqs = 0; c.delta = 0; region_next_.clear(); }
     }
-    meta_dirty_ = true;
+}
+// (behind the wait for the staging event: the pinned mirror may still be on its way)
+int Context::upload_cells() {
+    const int NC = (int)cells_.size();
+    int lo = dirty_lo_, hi = std::min(dirty_hi_, NC), u0 = NC, u1 = 0;
+    if (!device_cells_known_) { lo = 0; hi = NC; }
+    for (int i = lo; i < hi; i++) {
+        const KVCell &c = cells_[(size_t)i];
+        if (device_cells_known_ && h_cell_pos_[i] == c.pos && h_cell_seq_[i] == c.seqs) continue;
+        h_cell_pos_[i] = c.pos; h_cell_seq_[i] = c.seqs;
+        u0 = std::min(u0, i); u1 = i + 1;
+    }
+    dirty_lo_ = dirty_hi_ = 0;
+    device_cells_known_ = true;
+    if (u0 >= u1) return 0;
+    return hipMemcpyAsync(d_cell_pos_ + u0, h_cell_pos_ + u0, (size_t)(u1 - u0) * 4, hipMemcpyHostToDevice, stream_) == hipSuccess &&
+           hipMemcpyAsync(d_cell_seq_ + u0, h_cell_seq_ + u0, (size_t)(u1 - u0) * 8, hipMemcpyHostToDevice, stream_) == hipSuccess ? 0 : -1;
 }
 int Context::kv_used_cells() const {
     int n = 0;
@@ -1418,8 +1443,10 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
     const bool engine = T == 1 && !mega && !profile_ && !debug_taps_ && !ub_embd_ && engine_prepare();
     last_layers_engine_ = engine;
     // cos / sin table, cell metadata and the tokens' embedding rows: one launch
-    HIP_TRY(launch_step_setup_embed(d_pos_, T, ra, rope_cs_, d_cell_pos_, d_cell_seq_, d_cell_, d_seqmask_, mega ? d_mega_sync_ : nullptr,
-                                    d_step_serial_, model->tok_embd.type, model->tok_embd.data, E, d_tok_, x_, stream_));
+    const auto staged = [&](const auto *d) { return stage_in_setup_ ? (decltype(d))(h_stage_ + ((const uint8_t *)d - d_stage_)) : d; };
+    HIP_TRY(launch_step_setup_embed(staged(d_pos_), T, ra, rope_cs_, d_cell_pos_, d_cell_seq_, staged(d_cell_), staged(d_seqmask_), mega ? d_mega_sync_ : nullptr,
+                                    d_step_serial_, model->tok_embd.type, model->tok_embd.data, E, staged(d_tok_), x_, stream_, h_stage_, d_stage_,
+                                    stage_in_setup_ ? (int)(stage_used_ / 4) : 0));
     // an embeddings batch: the caller's rows take the place of the looked-up ones (never inside a captured graph: decode_ubatch)
     if (ub_embd_) HIP_TRY(hipMemcpyAsync(x_, ub_embd_, (size_t)T * E * sizeof(float), hipMemcpyHostToDevice, stream_));
     prof_mark("embed");
@@ -1902,34 +1929,35 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
     if (!alloc_cells(n, seqmask, tcell)) return 1;
     for (int i = 0; i < n; i++) {
         KVCell &c = cells_[(size_t)tcell[(size_t)i]];
+        cells_undo_.emplace_back(tcell[(size_t)i], c);
         c.pos = pos[i]; c.seqs = seqmask[i]; c.delta = 0;
+        cells_end_ = std::max(cells_end_, tcell[(size_t)i] + 1);
     }
-    int hi = 0;
-    for (int i = (int)cells_.size() - 1; i >= 0; i--) if (cells_[(size_t)i].pos >= 0) { hi = i + 1; break; }
-    n_kv_ = std::min((int)cp.n_ctx, (hi + 31) & ~31);
+    while (cells_end_ > 0 && cells_[(size_t)cells_end_ - 1].pos < 0) cells_end_--;
+    n_kv_ = std::min((int)cp.n_ctx, (cells_end_ + 31) & ~31);
 
-    if (meta_dirty_) {   // sequence ops since the last batch: re-upload the whole cell table
-        std::vector<int32_t> cpos(cells_.size());
-        std::vector<uint64_t> cseq(cells_.size());
-        for (size_t i = 0; i < cells_.size(); i++) { cpos[i] = cells_[i].pos; cseq[i] = cells_[i].seqs; }
-        if (hipMemcpyAsync(d_cell_pos_, cpos.data(), cpos.size() * 4, hipMemcpyHostToDevice, stream_) != hipSuccess ||
-            hipMemcpyAsync(d_cell_seq_, cseq.data(), cseq.size() * 8, hipMemcpyHostToDevice, stream_) != hipSuccess ||
-            hipStreamSynchronize(stream_) != hipSuccess) { last_error = "cell table upload failed"; return -1; }
-        meta_dirty_ = false;
-    }
-    // stage token arrays (the pinned block may still be in flight from the previous micro-batch)
+    // stage token arrays and cell table (the pinned blocks may still be in flight from the previous micro-batch)
     if (stage_event_) (void)hipEventSynchronize(stage_event_);
-    const size_t T = ((size_t)cp.n_ubatch + 1) & ~(size_t)1;
+    if (device_cells_known_)
+        for (int i = 0; i < n; i++) { const int c = tcell[(size_t)i]; h_cell_pos_[c] = pos[i]; h_cell_seq_[c] = seqmask[i]; }   // the set-up launch writes these
+    if (upload_cells() != 0) { last_error = "cell table upload failed"; return -1; }
+    // the arrays one behind the other, as long as the batch: a step uploads some dozen bytes (the same addresses for every batch of one token: its graphs hold them)
+    const size_t T = ((size_t)n + 1) & ~(size_t)1;             // keeps the u64 seqmask array 8-byte aligned
     int32_t *h_nkv = (int32_t *)h_stage_;
     int32_t *h_tok = (int32_t *)(h_stage_ + 16), *h_pos = h_tok + T, *h_seq = h_pos + T, *h_cell = h_seq + T, *h_out = h_cell + T;
     uint64_t *h_mask = (uint64_t *)(h_out + T);
+    const auto on_device = [&](const void *h) { return d_stage_ + ((const uint8_t *)h - h_stage_); };
+    d_tok_ = (int32_t *)on_device(h_tok); d_pos_ = (int32_t *)on_device(h_pos); d_seq_ = (int32_t *)on_device(h_seq); d_cell_ = (int32_t *)on_device(h_cell);
+    d_outrow_ = (int32_t *)on_device(h_out); d_seqmask_ = (uint64_t *)on_device(h_mask);
     h_nkv[0] = n_kv_;
     int n_out = 0;
     for (int i = 0; i < n; i++) {
         h_tok[i] = tokens[i]; h_pos[i] = pos[i]; h_seq[i] = seq[i]; h_cell[i] = tcell[(size_t)i]; h_mask[i] = seqmask[i];
         if (flags[i]) h_out[n_out++] = i;
     }
-    if (hipMemcpyAsync(d_stage_, h_stage_, stage_bytes_, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "token upload failed"; return -1; }
+    stage_used_ = (size_t)((uint8_t *)(h_mask + n) - h_stage_);
+    stage_in_setup_ = n == 1 && !model->nvx && !model->hp.encoder;
+    if (!stage_in_setup_ && hipMemcpyAsync(d_stage_, h_stage_, stage_used_, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "token upload failed"; return -1; }
     // continuous-batching steps (a few tokens, usually one per sequence): each token scans only the 64-cell chunks that
     // hold cells of its own sequence instead of the whole cache
     chunk_lmax_ = 0;
@@ -1976,7 +2004,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         for (int i = 0; i < n; i++) nvx_seq_len_[(size_t)seq[i]] = std::max<uint64_t>(nvx_seq_len_[(size_t)seq[i]], (uint64_t)pos[i] + 1);
     }
     if (!stage_event_) (void)hipEventCreateWithFlags(&stage_event_, hipEventDisableTiming);
-    if (stage_event_) (void)hipEventRecord(stage_event_, stream_);
+    if (stage_event_ && !stage_in_setup_) (void)hipEventRecord(stage_event_, stream_);
 
     const int V = model->hp.n_vocab;
     const bool nvx = model->nvx != nullptr;
@@ -2004,6 +2032,8 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         if (!graph_exec_) {
             hipGraph_t g = nullptr;
             std::string inner;                                  // which launch refused, when one did (HIP_TRY's message)
+            // (a copy nobody waits for: an idle device is awake by the time the capture - some hundred microseconds of the host - is done)
+            if (stage_in_setup_) (void)hipMemcpyAsync(d_stage_, h_stage_, stage_used_, hipMemcpyHostToDevice, stream_);
             e = hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
                 last_error.clear();
@@ -2043,6 +2073,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             e = hipMemcpyAsync(h_logits_ + (size_t)out_base * V, d_logits_ + (size_t)out_base * V, (size_t)n_out * V * 4, hipMemcpyDeviceToHost, stream_);
         prof_end();
     }
+    if (stage_event_ && stage_in_setup_) (void)hipEventRecord(stage_event_, stream_);   // (read inside the step)
     if (e != hipSuccess) { last_error = std::string("decode failed: ") + hipGetErrorString(e) + " / " + last_error_string(); return -1; }
     if (n == 1 && (graph_ok ? graph_is_mega_[graph_exec_] : last_layers_mega_)) mega_steps++;
     if (n == 1 && (graph_ok ? graph_is_engine_[graph_exec_] : last_layers_engine_)) engine_steps++;
@@ -2153,7 +2184,7 @@ int Context::decode(int n_tokens, const int32_t *tokens, const int32_t *pos, con
     if (embeddings_enabled && (size_t)n_out > cp.n_ubatch) { last_error = "embeddings: more flagged rows than n_ubatch"; return -1; }
     argmax_fetched_ = false;
 
-    const std::vector<KVCell> saved = cells_;
+    cells_undo_.clear();
     const int saved_head = head_;
     int out_base = 0;
     for (int i0 = 0; i0 < n_tokens; i0 += (int)cp.n_ubatch) {
@@ -2162,7 +2193,8 @@ int Context::decode(int n_tokens, const int32_t *tokens, const int32_t *pos, con
         const int rc = decode_ubatch(n, tokens + i0, pos + i0, seq.data() + i0, mask.data() + i0, flags.data() + i0, out_base);
         ub_embd_ = nullptr;
         if (rc != 0) {
-            cells_ = saved; head_ = saved_head; meta_dirty_ = true; region_next_.clear();
+            for (size_t u = cells_undo_.size(); u-- > 0;) cells_[(size_t)cells_undo_[u].first] = cells_undo_[u].second;
+            head_ = saved_head; device_cells_known_ = false; region_next_.clear();
             return rc;
         }
         for (int i = 0; i < n; i++) out_base += flags[(size_t)(i0 + i)] ? 1 : 0;

@@ -243,7 +243,15 @@ class Context {
     std::vector<KVCell> cells_;
     int head_ = 0;
     bool has_shift_ = false;
-    bool meta_dirty_ = true;
+    // the device's cell table follows the host's: what it holds is mirrored in pinned memory, and a batch uploads the cells between dirty_lo_ and dirty_hi_ whose mirror
+    // differs and that the batch's own set-up launch does not write (a tail cut off and fed again: none)
+    int dirty_lo_ = 0, dirty_hi_ = 0, cells_end_ = 0;     // cells_end_: no cell at or above it is occupied
+    bool device_cells_known_ = false;
+    int32_t *h_cell_pos_ = nullptr;     // pinned
+    uint64_t *h_cell_seq_ = nullptr;
+    std::vector<std::pair<int, KVCell>> cells_undo_;      // what the decode call in progress has overwritten
+    void touch_cell(int i) { if (dirty_lo_ >= dirty_hi_) dirty_lo_ = i; dirty_lo_ = std::min(dirty_lo_, i); dirty_hi_ = std::max(dirty_hi_, i + 1); }
+    int upload_cells();
 
     // device state
     std::vector<KVLayerView> kv_;
@@ -255,7 +263,8 @@ class Context {
     int32_t *d_tok_ = nullptr, *d_pos_ = nullptr, *d_seq_ = nullptr, *d_cell_ = nullptr, *d_nkv_ = nullptr, *d_outrow_ = nullptr;
     uint64_t *d_seqmask_ = nullptr;
     uint8_t *h_stage_ = nullptr;    // pinned
-    size_t stage_bytes_ = 0;
+    size_t stage_bytes_ = 0, stage_used_ = 0;             // of the block; of the batch in it
+    bool stage_in_setup_ = false;                         // the set-up launch of a single-token step fetches the block itself (no copy in front of its graph)
     uint8_t *d_stage_ = nullptr;
     hipEvent_t stage_event_ = nullptr;
     // activations
