@@ -19,7 +19,7 @@ struct ActRows {
     uint16_t *d0 = nullptr;    // [T][K/32]
 };
 struct ActQuant : ActRows {
-    uint8_t *qf = nullptr;     // nullable: the q8_K blocks of a batch of 2 .. FEW_MAX_T rows once more, as mmq_few.hip's operands
+    uint8_t *qf = nullptr;     // nullable: the q8_K blocks of a batch of 3 .. FEW_MAX_T rows once more, as mmq_few.hip's operands
 };
 // mmq_few.hip: a block of qf is 16 rows (tokens) x one super-block, blocks [row tile][super-block].  Codes: element k of row t lies at
 // (k / 64) * 1024 + ((t & 15) + 16 * (k / 8 % 4)) * 16 + k / 32 % 2 * 8 + k % 8 - a lane's 16 bytes of a step of 64 are 8 of either half.  Behind them the block
@@ -28,7 +28,7 @@ constexpr int FEW_BH = 4096, FEW_BL = FEW_BH + 256, FEW_D = FEW_BL + 256, FEW_BL
 inline ActQuant act_for(const ActQuant *q, int T) {       // what a quantiser of T rows writes
     ActQuant r;
     if (q) r = *q;
-    if (T < 2 || T > FEW_MAX_T) r.qf = nullptr;
+    if (T < 3 || T > FEW_MAX_T) r.qf = nullptr;
     return r;
 }
 inline size_t few_bytes(int64_t K) { return K % 256 ? 0 : (size_t)(FEW_MAX_T / 16) * (size_t)(K / 256) * FEW_BLOCK; }
@@ -169,12 +169,12 @@ bool mmq_planes_mixed_ok(const int *seg_rows, int n_seg, int K, int T, MMQWorksp
 bool mmq_planes_swiglu_ok(int type_gate, int type_up, int n_rows, int K, int T);
 hipError_t launch_mmq_planes_swiglu(int type, const uint8_t *planes_gate, const uint8_t *planes_up, int n_rows, int K, int T, const ActQuant &q,
                                     float *out, int ld_out, hipStream_t st);
-bool mmq_ksplit_applicable(int type, int K, int T, bool few = false);   // few: the activation has its operand blocks (ActQuant::qf)
+bool mmq_ksplit_applicable(int type, int K, int T);
 // ... and preferred over the planes kernels for a tensor of n_rows rows (has_planes: its pre-expanded planes exist)
-bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool few, bool pair = false);
+bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool pair = false);
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                                    bool swiglu, hipStream_t st);
-hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);   // mmq_few.hip: 2 .. 64 tokens of the same
+hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);   // mmq_few.hip: 3 .. 64 tokens of the same
 hipError_t launch_mmq_ksplit(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q,
                              const int8_t *bh, const int8_t *bl, float *out, int ld_out, const float *resid, hipStream_t st);
 size_t mmq_prep_bytes(int K, int T);                       // bytes of each of the two block-sum planes

@@ -1632,11 +1632,11 @@ void mmq_p2_set_probe(unsigned long long *p) { (void)hipMemcpyToSymbol(HIP_SYMBO
 // (round 2: the LDS-form planes kernel moved the crossover down - whole prompt, K-split against planes: 13.8 vs 14.1 ms at 256 tokens,
 // 17.2 vs 15.2 at 320, 19.1 vs 15.5 at 384)
 static int g_ksplit_max = getenv("MI355_KSPLIT_MAX") ? atoi(getenv("MI355_KSPLIT_MAX")) : 256;
-bool mmq_ksplit_applicable(int type, int K, int T, bool few) {
+bool mmq_ksplit_applicable(int type, int K, int T) {
     // from 3 tokens: the mat-vec takes 4 + 2 + 1 tokens per pass over the weights, so 3 sequences cost 4.5 ms and 6 cost 6.4 ms a step against
-    // 3.7 ms through this kernel; for 2 the mat-vec pass is cheaper (3.2 ms) - than this kernel, not than mmq_few.hip's, which takes the batch where the quantiser
-    // left its operand blocks (few)
-    return (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K % 256) == 0 && T >= (few ? 2 : 3) && T <= g_ksplit_max;
+    // 3.7 ms through this kernel.  Two stay with the mat-vec, whose sums are the one-token step's bit for bit: a pair of conversations then spells the text that
+    // either spells alone (mmq_few.hip adds the super-blocks up in another order)
+    return (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K % 256) == 0 && T >= 3 && T <= g_ksplit_max;
 }
 
 // Which kernel takes a 3..256-token launch is a matter of shape (tools/exp_planes_shapes.py, Q5_K, us per launch):
@@ -1648,9 +1648,9 @@ bool mmq_ksplit_applicable(int type, int K, int T, bool few) {
 // (pair: gate | up of a dense layer go out as ONE K-split launch of 2 n_rows rows, which holds its own against two planes launches up to
 // 128 tokens - whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128; past that the LDS-form SwiGLU launch takes the pair:
 // 13.6 -> 10.6 ms at 200 tokens, 14.1 -> 11.1 at 256.)
-bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool few, bool pair) {
+bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool pair) {
     static const int env = getenv("MI355_KSPLIT_SHAPE") ? atoi(getenv("MI355_KSPLIT_SHAPE")) : 1;
-    if (!mmq_ksplit_applicable(type, K, T, few)) return false;
+    if (!mmq_ksplit_applicable(type, K, T)) return false;
     if (env && has_planes && T > (pair ? 128 : 64) && n_rows >= 8192 && mmq_applicable(type, K, T)) return false;
     return true;
 }

@@ -1,4 +1,4 @@
-// mmq_few.hip — the K-split contraction of 2 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
+// mmq_few.hip — the K-split contraction of 3 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
 // K-quant weights in their GGUF form, Q8_K activations, int8 matrix cores, the integer of ggml_vec_dot_q{4,5,6}_K_q8_K per (row, token, super-block).
 //
 // What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and in front of them the ~140 vector instructions per unit and token tile below (matrix
@@ -405,7 +405,7 @@ void few_type(const FewArgs &a, int blocks, hipStream_t st) {
 
 }  // namespace
 
-// segs as launch_mmq_ksplit_multi's (which sends 2 .. 64 tokens here): up to three tensors sharing the activation, or {gate, up} of one type and shape with swiglu
+// segs as launch_mmq_ksplit_multi's (which sends 3 .. 64 tokens here): up to three tensors sharing the activation, or {gate, up} of one type and shape with swiglu
 hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st) {
     if (!q.qf || T > FEW_MAX_T) return hipErrorInvalidValue;
     FewArgs a{};

@@ -581,7 +581,7 @@ static void alloc_actq(ActQuant &q, size_t K, size_t T, bool k, bool z, std::vec
         q.qs = (int8_t *)al(T * K);
         q.d = (float *)al(T * (K / 256) * 4);
         q.bsums = (int16_t *)al(T * (K / 16) * 2);
-        if (few && T >= 2 && few_bytes((int64_t)K)) q.qf = (uint8_t *)al(few_bytes((int64_t)K));
+        if (few && T >= 3 && few_bytes((int64_t)K)) q.qf = (uint8_t *)al(few_bytes((int64_t)K));
     }
     if (z) {
         q.qs0 = (int8_t *)al(T * K);
@@ -996,7 +996,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
             return launch_mmq_q80(w.data, w.row_bytes, (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         // (bh_over_ / bl_over_: the caller prepared the block-sum planes of a larger batch that aq's rows are a slice of - the expert loop)
         const int8_t *bh = bh_over_ ? bh_over_ : mmq_bh_, *bl = bh_over_ ? bl_over_ : mmq_bl_;
-        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, aq.qf != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
+        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
             if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
             return launch_mmq_ksplit(w.type, w.data, w.row_bytes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         }
@@ -1025,7 +1025,7 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     for (int i = 0; i < n; i++) all_q &= is_quant(ws[i]->type);
     const int K = (int)ws[0]->K;
     bool all_mmq = true, all_ks = true;
-    for (int i = 0; i < n; i++) { all_mmq &= mmq_applicable(ws[i]->type, K, T); all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T, aq.qf != nullptr); }
+    for (int i = 0; i < n; i++) { all_mmq &= mmq_applicable(ws[i]->type, K, T); all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T); }
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
         HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
         MMQSeg sg[3];
@@ -1755,10 +1755,10 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             bool swiglu_quantised = false;
             const bool ffn_mmq = (mmq_q80_applicable(L.gate.type, E, T) && mmq_q80_applicable(L.up.type, E, T)) ||
                                  (mmq_applicable(L.gate.type, E, T) && mmq_applicable(L.up.type, E, T)) ||
-                                 (mmq_ksplit_applicable(L.gate.type, E, T, aq_e_.qf != nullptr) && mmq_ksplit_applicable(L.up.type, E, T, aq_e_.qf != nullptr)) ||
+                                 (mmq_ksplit_applicable(L.gate.type, E, T) && mmq_ksplit_applicable(L.up.type, E, T)) ||
                                  (planes_small(L.gate, E, T) && planes_small(L.up, E, T)) || (q80_copy(L.gate, E, T) && q80_copy(L.up, E, T));
-            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, aq_e_.qf != nullptr, true) &&
-                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, aq_e_.qf != nullptr, true) && !fuse_ffn;
+            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, true) &&
+                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, true) && !fuse_ffn;
             if (gq && uq && L.gate.type == L.up.type && !ffn_mmq) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
                 HIP_TRY(mmvq_tokens(segs, 2, E, T, EPI_SWIGLU, aq_e_, stream_, fz));

@@ -1,4 +1,4 @@
-"""Batches of 2 .. 64 tokens against K-quant weights (csrc/mmq_few.hip): the contraction whose workgroups walk 16-row tiles with the quantiser's operand blocks."""
+"""Batches of 3 .. 64 tokens against K-quant weights (csrc/mmq_few.hip): the contraction whose workgroups walk 16-row tiles with the quantiser's operand blocks."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("K,N,T", [(4096, 40, 2), (256, 8210, 3),       # two tokens; one super-block, more row tiles than workgroups, a ragged last one
+@pytest.mark.parametrize("K,N,T", [(4096, 40, 4), (256, 8210, 3),       # a few rows; one super-block, more row tiles than workgroups, a ragged last one
                                    (4096, 4200, 16), (2048, 8193, 17),  # a full token tile and one token more; two super-blocks per wave and one, several tiles each
                                    (3584, 4130, 32), (11008, 50, 33),   # super-blocks that do not divide by the waves, up to two and more than two per wave
                                    (1024, 4113, 48), (4096, 17, 49), (5632, 4112, 64)])
