@@ -1,6 +1,6 @@
 // mmq.hip — batched prefill contraction  Y[t][r] = dot(W[r,:], act_q8K[t,:])  on the MFMA matrix cores.
 //
-// Stands in for ggml's mul_mat_q / the CPU backend's chunked mul_mat for prompt processing (SURVEY.md §8a row a10),
+// Stands in for ggml's mul_mat_q / the CPU backend's chunked mul_mat for prompt processing,
 // reached from the reference through llama_decode with n_tokens > 1 (src/llama_server_context.cc:1568-1607, 1635).
 //
 // Integer-exact by construction, and MFMA-bound rather than VALU-bound:
@@ -26,6 +26,7 @@
 // MT = 1: 256 rows x 32 tokens).  The activation tile of one super-block (tokens x 256 int8, + block-sum planes + scales) is
 // staged in LDS once per workgroup (row stride 272 B: ds_read_b128 conflict-free), the next tile's global loads are
 // issued before the MFMA work of the current one, and the raw weights of the next super-block likewise.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1021,20 +1022,26 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
     }
 }
 
-// ---- the same contraction with BOTH operands through LDS (prompts of a few hundred tokens and more on the wide tensors).
-// mmq_planes_kernel reads its B operand (the weight planes) per lane from L2: 2 KiB per K-step per wave for MT x 2 MFMAs, so
-// at MT = 2 the eight waves of a CU ask the vector L1 for 64 B / clk at full matrix-core rate - the L1's whole bandwidth - and
-// the matrix cores idle most of the time (16 % busy on gate/up of the 8B model).  Here a workgroup covers 128 rows x 256 tokens:
-// a wave owns 32 rows x 128 tokens (four token tiles: 8 MFMAs per pair of B registers), and each plane byte is fetched ONCE per
-// workgroup - by the LDS-DMA (global_load_lds_dwordx4, no register round trip), half a super-block (4 K-steps) per stage into one
-// of two 64 KiB buffers, the other one being read by the MFMAs:
-//   B  32 KiB = [row tile 0..3][K-step 0..3][plane hi, lo][lane][16 B]   - the layout mmq_expand_kernel writes, copied verbatim
-//   A  32 KiB = [token 0..255][8 pieces of 16 B]; piece p of token t sits in slot p ^ ((t >> 1) & 7) (the swizzle is applied on
-//               the SOURCE side of the DMA, whose LDS side is always lane-linear), so the 16 lanes of a ds_read_b128 phase hit 16
-//               different 16-B bank groups
-// Per stage and CU: 64 KiB over the L1 (32 B / clk at full rate), 192 KiB out of LDS (96 B / clk of 128), 256 MFMAs.
-// Per-super-block activation scales and block-sum planes are staged by ordinary loads one super-block ahead (two parities).
-// The integer sums, the fold and the f32 order over super-blocks are those of mmq_planes_kernel: results are bit-identical.
+// ---- the same contraction in 128-row x 256-token workgroup tiles: activations through LDS, planes straight into registers.
+// Eight waves: wave (rw, tw) owns 32 rows x 128 tokens of the tile, i.e. the 32-row tile rw of token half tw.  Per super-block a wave takes the 16 KiB of its planes ONCE,
+// as the sixteen MFMA operands they are laid out as, and holds them in 64 registers while it walks its four token tiles; both halves ask for the same planes at about
+// the same time, so the second finds them in the vector L1.  The 256 x 256 activation codes come by LDS-DMA one super-block ahead (two buffers, one barrier per super-block):
+//   codes  64 KiB = [token 0..255][16 pieces of 16 B]; piece p of token t sits in slot p ^ (t & 15) (applied on the SOURCE side of the DMA, whose LDS side is
+//          lane-linear), so the 16 lanes of a ds_read_b128 phase hit all 64 banks
+//   block sums 8 KiB (int16, turned into f16 in place by the wave that fetched them), the rows' d / dmin / mins words, and the tokens' scales (three sets: a fold
+//          reaches into the next super-block)
+// The f32 fold of a token tile (five vector instructions an output) runs BETWEEN the MFMAs of the next tile, two outputs per K-step, on the other of two accumulator
+// pairs: a wave in an MFMA phase of its own leaves the vector unit idle, and one in a fold of its own the matrix cores.
+//
+// What bounds it: the package's power.  gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens, random operands, launches back to back): a workgroup's loop takes
+// 119 k cycles, of which the matrix cores are busy 70 k, at 1.6 GHz; with all-zero operands the same loop runs at 2.15 GHz and the launch in 137 us instead of 167; without
+// the loads in the loop (hot operands) 126.  So what counts besides the MFMAs is what is moved: this split asks the L2 for 128 KiB per super-block and CU; as two
+// 128 x 128 workgroups per CU, each with planes of its own, the same loop asked for 192 and took 4 % longer, and 16 x 16 x 64 MFMA tiles, which read twice the registers
+// per product, the same again.  Measured inside a 512-token prompt: 167 -> 153 us (before: planes through LDS as well, half a super-block per barrier, folds beside the
+// other half's MFMAs); the experts of an 8x7B layer (611 tokens, 1222 rows): gate | up 628 -> 548 us, down 276 -> 253, where a batch of ~150 rows is now dealt evenly to both halves.
+// Touching the super-block after the next one, to have it in the L2: 12 % slower (64 lines an instruction).
+// The block-sum ("mins") term is one v_mfma_f32_32x32x16_f16 per tile: the 16 block sums (|.| <= 2032) and the 6-bit mins are exact in f16 and their 16 products sum to
+// < 2^24, so the f32 result IS the integer msum.  The integer sums, the fold and the f32 order over super-blocks are those of mmq_planes_kernel: results are bit-identical.
 __device__ __forceinline__ unsigned lds_addr32(const void *p) { return (unsigned)(uintptr_t)p; }
 // lane l: 16 B from gbase + voff (voff per lane) to LDS dst + 16 l
 __device__ __forceinline__ void dma16_s(const void *gbase, unsigned voff, unsigned lds_dst) {
@@ -1042,32 +1049,6 @@ __device__ __forceinline__ void dma16_s(const void *gbase, unsigned voff, unsign
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                  : "=&s"(keep) : "v"(voff), "s"(gbase), "s"(lds_dst) : "memory");
 }
-// lane l: 4 x 16 B from g, g + 1 KiB, g + 2 KiB, g + 3 KiB (g per lane) to dst + {0, 1, 2, 3} KiB + 16 l: the instruction
-// offset applies to the global and to the LDS address alike
-__device__ __forceinline__ void dma_4k(const void *g, unsigned lds_dst) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %1, off\n\t"
-                 "global_load_lds_dwordx4 %1, off offset:1024\n\t"
-                 "global_load_lds_dwordx4 %1, off offset:2048\n\t"
-                 "global_load_lds_dwordx4 %1, off offset:3072\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(g), "s"(lds_dst) : "memory");
-}
-
-// lane l: 16 B from g + OFF (g per lane) to LDS dst + OFF + 16 l
-template <int OFF> __device__ __forceinline__ void dma16_o(const void *g, unsigned lds_dst) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%c3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(g), "s"(lds_dst), "i"(OFF) : "memory");
-}
-
-constexpr int P2_ROWS = 128, P2_TOK = 256, P2_MT = 4;
-constexpr int P2_BUF = 65536, P2_A = 32768;                         // per buffer: B planes | A codes
-constexpr int P2_YD = 0, P2_BS = 1024, P2_META = 1024 + 8192;
-constexpr int P2_SBARR = P2_META + 2048;                            // per parity: yd[256] | bsums[256][16] (int16, then f16) | meta[4][32][16]
-constexpr int P2_LDS = 2 * P2_BUF + 2 * P2_SBARR;
-
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -1079,399 +1060,273 @@ __device__ __forceinline__ void dma4_s(const void *gbase, unsigned voff, unsigne
                  : "=&s"(keep) : "v"(voff), "s"(gbase), "s"(lds_dst) : "memory");
 }
 
-#ifdef MI355_P2_PROBE
-// tools/exp_p2.hip: per wave of workgroup 0, shader cycles spent per stage kind {first, second half} in {compute issue, DMA wait, barrier}
-__device__ unsigned long long *g_p2_probe = nullptr;
-#define P2_STAMP() __builtin_readcyclecounter()
-#endif
-#ifndef MI355_P2_PRIO
-#define MI355_P2_PRIO 0      // tools: s_setprio level of a wave inside its MFMA phase (0 = no instruction)
-#endif
-#ifndef MI355_P2_LATE_DMA
-#define MI355_P2_LATE_DMA 0  // tools: 1 = a stage's DMA issued behind the issuing half's MFMAs instead of in front of them
-#endif
-#ifndef MI355_P2_EXP
-#define MI355_P2_EXP 0       // tools: 1 = no fold, 2 = no DMA, 3 = no MFMA (timing experiments; results are garbage)
-#endif
-// Schedule.  A stage is half a super-block (4 K-steps); stage s is computed from buffer s & 1 while the DMA fills the other one;
-// one workgroup barrier per stage.  A SIMD holds two waves of the workgroup, one of each token half, and the f32 fold of a
-// super-block (VALU work, 40 % of the MFMA time) would leave the matrix cores idle if both did it at the same point.  So the
-// token halves fold at DIFFERENT points: waves 0-3 right after the super-block's last MFMAs (end of its second stage), waves 4-7
-// at the start of the next super-block's first stage - each half's fold runs beside the other half's MFMAs.
-// The block-sum ("mins") term is one v_mfma_f32_32x32x16_f16 per tile: the 16 block sums (|.| <= 2032) and the 6-bit mins are
-// exact in f16 and their 16 products sum to < 2^24, so the f32 result IS the integer msum - no shift, no conversion.
-// SWIGLU: `planes` = ffn_gate, `planes_up` = ffn_up (n_rows rows each, same type): a workgroup takes 64 rows of BOTH (row-waves 0, 1 the
-// gate rows, 2, 3 the same rows of up), the up waves hand their tile over through LDS at the end and the gate waves store
-// silu(gate . x) * (up . x) - one [T][n_rows] f32 result instead of two, and no separate SwiGLU pass over them
-template <bool MINS, bool SWIGLU>
-__device__ __forceinline__ void planes2_body(const uint8_t *planes, const uint8_t *planes_up, int n_rows, int K, int T, int n_row_tiles, int n_tok_tiles,
-                                             const int8_t *aq, const float *ad, const int16_t *absum,
-                                             const PlanesOut &po, const float *resid, float *ws, int n_split, int row_tile, int tok_tile, int zz) {
-    constexpr int MT = P2_MT;
-    constexpr int SH = MINS ? 5 : 6;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nb_all = K >> 8;                                 // super-blocks per row (strides); this workgroup's share is [sb_lo, sb_lo + nb)
-    const int sb_lo = (int)((long)nb_all * zz / n_split), nb = (int)((long)nb_all * (zz + 1) / n_split) - sb_lo;
-    const int rw = wave & 3, tw = wave >> 2;
-    const int n_rt32 = (n_rows + 31) >> 5;
-    // 32-row tile of row-wave index p (compute: p = rw; plane DMA: p = wave >> 1; row-word DMA: p = 2 (wave & 1) + kg) and its tensor
-    auto tile_of = [&](int p) { return SWIGLU ? row_tile * 2 + (p & 1) : row_tile * 4 + p; };
-    auto base_of = [&](int p) { return SWIGLU && (p >> 1) ? planes_up : planes; };
-    const int rt32 = tile_of(rw);
-    const bool tile_ok = rt32 < n_rt32;
-    const int row0 = rt32 * 32;
-    const int tok0 = tok_tile * P2_TOK;
-    const int n = lane & 31, kg = lane >> 5;
-    // a token half (128 tokens) past the end of the batch - 320 tokens leave the second workgroup tile 64 of 256 - keeps the DMA and
-    // barrier protocol and skips its MFMAs and folds: the other half then has the matrix cores to itself
-    const bool idle_half = tok0 + tw * 128 >= T;                // (wave-uniform)
+constexpr int P2_ROWS = 128, P2_TOK = 256;
+constexpr int P2_BS = 65536, P2_META = P2_BS + 8192, P2_BUF = P2_META + 4096, P2_YD = 2 * P2_BUF, P2_YDB = 640, P2_LDS = P2_YD + 6 * P2_YDB;
 
-    // ---- the DMA, in shares of a "virtual wave" vw = 0..7.  Per stage: 4 KiB of B (row tile vw / 2, K-steps 2 (vw & 1) .. + 1, both
-    // planes) and 4 KiB of A (32 tokens x 128 B, eight tokens per instruction).  Per super-block: 1 KiB of block sums (32 tokens x
-    // 32 B), activation scales (vw 0-3, 64 tokens each) and the row tiles' d / dmin / mins words (vw 4, 5: two row tiles each).
-    // Addresses are formed when a share is issued (a dozen VALU instructions) instead of living in eight registers, and WHO issues
-    // follows the schedule below: an LDS-DMA instruction costs its wave ~100 cycles of issue in a busy phase, so a stage's 64 + 14
-    // instructions go to the token half that is NOT folding in that stage (it waits at the barrier for the folding half anyway), or to
-    // the half that has no tokens at all.
-    const unsigned lds0 = lds_addr32(smem);
-    auto issue_v = [&](int s, int vw) {                         // stage s = (super-block s >> 1, half s & 1) into buffer s & 1
-        if (MI355_P2_EXP == 2) return;
-        int lane = tid & 63;
-        asm volatile("" : "+v"(lane));                          // (formed here, every time: hoisted out of the loop the offsets would cost 20 registers)
-        const unsigned buf = lds0 + (unsigned)(s & 1) * P2_BUF;
-        int drt = tile_of(vw >> 1);
-        if (drt >= n_rt32) drt = n_rt32 - 1;
-        const uint8_t *gb = base_of(vw >> 1) + ((size_t)drt * nb_all + sb_lo + (s >> 1)) * PL_BLOCK + (vw & 1) * 4096 + (s & 1) * 8192;
-        dma_4k(gb + lane * 16, buf + (unsigned)vw * 4096u);
-        const int8_t *ga = aq + (size_t)s * 128;
+struct P2Args {
+    const uint8_t *planes, *planes_up;
+    int n_rows, K, T;
+    const int8_t *aq; const float *ad; const int16_t *absum;
+    const float *resid; float *ws; int n_split;
+};
+typedef const __attribute__((address_space(1))) uint8_t gbytes;
+// a pointer that is the same in every lane, in scalar registers
+__device__ __forceinline__ gbytes *scalar_ptr(const void *p) {
+    const uint64_t v = (uint64_t)p;
+    return (gbytes *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
+}
+// NT: token tiles of 32; FULL: every token of the workgroup's tile exists
+template <bool MINS, int NT, bool FULL>
+__device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int sb_lo, int nb, int tok0, int tid, int tw, uint8_t *smem_wg, float (&facc)[4][16]) {
+    constexpr int SH = MINS ? 5 : 6;
+    // (a half's four waves stage their own tokens: `wave` is the wave's index in its half)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int n = lane & 31, kg = lane >> 5;
+    const int nb_all = a.K >> 8;
+    const uint8_t *sm_bs = smem_wg + P2_BS + tw * 4096, *sm_meta = smem_wg + P2_META + tw * 2048, *sm_yd = smem_wg + P2_YD + tw * P2_YDB, *sm_a = smem_wg + tw * 32768;
+    const unsigned lds0 = lds_addr32(smem_wg);
+    const int last = a.T - 1 - tok0;                            // (tokens past the end read the last one; never stored)
+    auto dma = [&](int sb, int buf, int y3) {                   // tokens 32 wave .. + 31 of super-block sb, and the scale words of the wave's rows
+        const unsigned dst = lds0 + (unsigned)buf * P2_BUF;
+        const uint8_t *mw = (const uint8_t *)scalar_ptr((const uint8_t *)blk0 + (size_t)sb * PL_BLOCK + 16384);
+        int l = lane;
+        asm volatile("" : "+v"(l));                             // (the offsets are formed here, every time: hoisted out of the loop they would cost ten registers)
+        dma4_s(mw, l * 4u, dst + P2_META + (unsigned)(tw * 2048 + wave * 512));
+        dma4_s(mw + 256, l * 4u, dst + P2_META + (unsigned)(tw * 2048 + wave * 512 + 256));
+        const size_t sbg = (size_t)(sb_lo + sb);
+        if (NT == 4 || wave < NT) {
+            const int q4 = l >> 4, p16 = l & 15;
+            if (FULL) {
+                const int8_t *g = (const int8_t *)scalar_ptr(a.aq + (size_t)(tok0 + 32 * wave) * a.K + sbg * 256);
+                const unsigned off = (unsigned)q4 * (unsigned)a.K + (unsigned)(p16 ^ q4) * 16u;      // of the wave's first four tokens
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int tk = 8 * (4 * vw + k) + (lane >> 3);
-            int gt = tok0 + tk;
-            if (gt >= T) gt = T - 1;
-            const int piece = (lane & 7) ^ ((tk >> 1) & 7);
-            dma16_s(ga, (unsigned)gt * (unsigned)K + (unsigned)sb_lo * 256u + (unsigned)piece * 16u, buf + P2_A + (unsigned)(4 * vw + k) * 1024u);
+                for (int k = 0; k < 8; k++) dma16_s(g + (size_t)(4 * k) * a.K, off ^ (64u * (k & 3)), dst + (unsigned)(32 * tw + 8 * wave + k) * 1024u);
+            } else {
+                const int8_t *g = (const int8_t *)scalar_ptr(a.aq + (size_t)tok0 * a.K + sbg * 256);
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const int t = 32 * wave + 4 * k + q4;
+                    dma16_s(g, (unsigned)(t < last ? t : last) * (unsigned)a.K + (unsigned)(p16 ^ (4 * (k & 3) + q4)) * 16u, dst + (unsigned)(32 * tw + 8 * wave + k) * 1024u);
+                }
+            }
+            const int bt = 32 * wave + (l >> 1), yt = 32 * wave + l;
+            if (MINS) dma16_s((const void *)scalar_ptr(a.absum + (size_t)tok0 * nb_all * 16 + sbg * 16), (unsigned)(bt < last ? bt : last) * (unsigned)nb_all * 32u + (unsigned)(l & 1) * 16u,
+                              dst + P2_BS + (unsigned)(4 * tw + wave) * 1024u);
+            // (scales of 64 tokens: the upper half are the next wave's, with the same values)
+            dma4_s((const void *)scalar_ptr(a.ad + (size_t)tok0 * nb_all + sbg), (unsigned)(yt < last ? yt : last) * (unsigned)nb_all * 4u, lds0 + P2_YD + (unsigned)((2 * y3 + tw) * P2_YDB + wave * 128));
         }
     };
-    auto issue_sb_v = [&](int sb, int vw) {                     // per-super-block words into parity sb & 1
-        if (MI355_P2_EXP == 2) return;
-        int lane = tid & 63;
-        asm volatile("" : "+v"(lane));
-        const int n = lane & 31, kg = lane >> 5;
-        const unsigned par = lds0 + 2 * P2_BUF + (unsigned)(sb & 1) * P2_SBARR;
-        if (MINS) {
-            int btok = tok0 + 32 * vw + (lane >> 1);
-            if (btok >= T) btok = T - 1;
-            dma16_s(absum + (size_t)sb * 16, ((unsigned)btok * (unsigned)nb_all + (unsigned)sb_lo) * 32u + (unsigned)(lane & 1) * 16u, par + P2_BS + (unsigned)vw * 1024u);
-        }
-        if (vw < 4) {
-            int ptok = tok0 + 64 * vw + lane;
-            if (ptok >= T) ptok = T - 1;
-            dma4_s(ad + sb, ((unsigned)ptok * (unsigned)nb_all + (unsigned)sb_lo) * 4u, par + P2_YD + (unsigned)vw * 256u);
-        } else if (vw < 6) {
-            const int p0 = 2 * (vw & 1);                         // first tile of this share's pair (SwiGLU: the pair is one tensor's)
-            int mb0 = tile_of(p0), mrt = tile_of(p0 + kg);
-            if (mb0 >= n_rt32) mb0 = n_rt32 - 1;
-            if (mrt >= n_rt32) mrt = n_rt32 - 1;
-            const uint8_t *mb = base_of(p0) + ((size_t)mb0 * nb_all + sb_lo + sb) * PL_BLOCK + 16384;
-            dma16_s(mb, (unsigned)(mrt - mb0) * (unsigned)nb_all * (unsigned)PL_BLOCK + (unsigned)n * 16u, par + P2_META + (unsigned)(vw - 4) * 1024u);
-        }
-    };
-    // the issuing half of a stage takes two shares per wave
-    auto issue = [&](int s, int issuer_tw) { if (tw == issuer_tw) { issue_v(s, rw); issue_v(s, rw + 4); } };
-    auto issue_sb = [&](int sb, int issuer_tw) { if (tw == issuer_tw) { issue_sb_v(sb, rw); issue_sb_v(sb, rw + 4); } };
-    auto convert_bs = [&](int sb) {                             // int16 block sums -> f16, in place (16 B per thread)
+    auto convert = [&](int buf) {                               // the wave's own share of the block sums, int16 -> f16 in place
         if (!MINS) return;
-        uint8_t *q = smem + 2 * P2_BUF + (sb & 1) * P2_SBARR + P2_BS + tid * 16;
+        uint8_t *q = smem_wg + buf * P2_BUF + P2_BS + (4 * tw + wave) * 1024 + lane * 16;
         const i16x8 v = *reinterpret_cast<const i16x8 *>(q);
         f16x8 f;
 #pragma unroll
         for (int e = 0; e < 8; e++) f[e] = (_Float16)v[e];
         *reinterpret_cast<f16x8 *>(q) = f;
     };
-
-    float facc[MT][16];
+    const unsigned b_off = (unsigned)lane * 16u;
+    i32x4 B[8][2];                                              // [K-step][plane]
+    dma(0, 0, 0);
+    auto ld_b = [&](gbytes *blk, int j) {
+        gbytes *q = blk + j * 2048;
+        asm("" : "+s"(q));
 #pragma unroll
-    for (int t = 0; t < MT; t++)
+        for (int p = 0; p < 2; p++) B[j][p] = *(const __attribute__((address_space(1))) i32x4 *)(q + b_off + p * 1024);
+    };
 #pragma unroll
-        for (int r = 0; r < 16; r++) facc[t][r] = 0.0f;
+    for (int j = 0; j < 8; j++) { ld_b(blk0, j); __builtin_amdgcn_sched_barrier(0); }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    convert(0);
+    __syncthreads();
+    const bool nib = MINS && __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(sm_meta + 12));       // Q2_K planes: sixteen 4-bit mins
 
-    // swizzled byte offset of this lane's A fragment for K-step j of a stage (same for every token tile: tiles start at multiples of 32)
-    const unsigned a_lane = (unsigned)(tw * 128 + n) * 128u;
-    const unsigned a_key = (unsigned)((n >> 1) & 7);
-    i32x16 H[MT], L[MT];
-
-    // fold of the super-block whose words sit in parity par, token tile by token tile
-    auto fold_all = [&](int par) {
-        if (MI355_P2_EXP == 1) return;
-        const uint8_t *pp = smem + 2 * P2_BUF + par * P2_SBARR;
-        const float *s_yd = reinterpret_cast<const float *>(pp + P2_YD);
-        const u32x4 mcur = *reinterpret_cast<const u32x4 *>(pp + P2_META + rw * 512 + n * 16);
-        const float dd = h2f((uint16_t)(mcur.x & 0xffff));
-        float ndm = 0.0f;
-        f16x8 bm8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    i32x16 H[2], L[2];                                          // [tile parity]
+    f32x16 ms;
+    f32x4 yd = {0.0f, 0.0f, 0.0f, 0.0f};
+    f16x8 as = {0, 0, 0, 0, 0, 0, 0, 0}, bm = as;
+    float dd = 0.0f, ndm = 0.0f;
+    // outputs 2 p, 2 p + 1 of a lane's sixteen of token tile t; ydn: where the tile's scales lie
+    auto fold = [&](int t, int pr, int p, const uint8_t *ydp) {
+#pragma unroll
+        for (int r = 2 * p; r < 2 * p + 2; r++) {
+            const float cf = (float)((H[pr][r] << SH) + L[pr][r]);
+            if (MINS) facc[t][r] = fmaf(yd[r & 3], fmaf(dd, cf, ndm * ms[r]), facc[t][r]);
+            else facc[t][r] = fmaf(yd[r & 3] * dd, cf, facc[t][r]);
+        }
+        if ((p & 1) && p < 7) yd = *reinterpret_cast<const f32x4 *>(ydp + (8 * ((p >> 1) + 1)) * 4);
+    };
+    // the block-sum term of the tile whose fold is next
+    auto mins = [&]() {
+        if (!MINS) return;
+        f32x16 zf;
+#pragma unroll
+        for (int r = 0; r < 16; r++) zf[r] = 0.0f;
+        ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(as, bm, zf, 0, 0, 0);
+    };
+    int y3 = 0;                                                 // sb % 3: three sets of token scales, the last tile's fold reaches into the next super-block
+    const uint8_t *yprev = sm_yd;
+    for (int sb = 0; sb < nb; sb++) {
+        const int sbuf = (sb & 1) * P2_BUF;
+        const int nxt = sb + 1 < nb ? sb + 1 : sb, y3n = y3 == 2 ? 0 : y3 + 1;
+        gbytes *blkn = blk0 + (size_t)nxt * PL_BLOCK;
+        const uint8_t *ys = sm_yd + y3 * 2 * P2_YDB + 16 * kg;
+        unsigned x = (unsigned)(n * 256 + ((kg ^ (n & 15)) * 16));
+        asm volatile("" : "+v"(x));
+        auto ld_a = [&](int t, int j) { return *reinterpret_cast<const i32x4 *>(sm_a + sbuf + t * 8192 + (x ^ (unsigned)(32 * j))); };
+        i32x4 A[2];
+        u32x4 meta = *reinterpret_cast<const u32x4 *>(sm_meta + sbuf + wave * 512 + n * 16);
+        A[0] = ld_a(0, 0); A[1] = ld_a(0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (sb) {                                               // the last tile of the super-block before, while the operands come
+            mins();
+#pragma unroll
+            for (int p = 0; p < 8; p++) fold(NT - 1, (NT - 1) & 1, p, yprev);
+        }
+        dd = h2f((uint16_t)(meta.x & 0xffff));
+        asm("" : "+v"(dd));                                  // (as f32: folded into v_fma_mix_f32 it costs twice the issue slots)
         if (MINS) {
-            ndm = -h2f((uint16_t)(mcur.x >> 16));
-            const unsigned w = kg ? mcur.z : mcur.y;            // mins 4 kg .. 4 kg + 3, each for two consecutive block sums
-            if (mcur.w) {                                       // Q2_K planes: eight 4-bit mins 8 kg .. 8 kg + 7, one per block sum
+            ndm = -h2f((uint16_t)(meta.x >> 16));
+            const unsigned w = kg ? meta.z : meta.y;            // mins 4 kg .. 4 kg + 3, each for two consecutive block sums
+            if (nib) {                                          // eight 4-bit mins 8 kg .., one per block sum
 #pragma unroll
-                for (int e = 0; e < 8; e++) bm8[e] = (_Float16)(float)((w >> (4 * e)) & 0xfu);
+                for (int e = 0; e < 8; e++) bm[e] = (_Float16)(float)((w >> (4 * e)) & 0xfu);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const _Float16 v = (_Float16)(float)((w >> (8 * e)) & 0xffu);
-                    bm8[2 * e] = v; bm8[2 * e + 1] = v;
+                    bm[2 * e] = v; bm[2 * e + 1] = v;
                 }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-            const int tl = (tw * MT + t) * 32;
-            f32x16 ms;
-            if (MINS) {
-                const f16x8 ab = *reinterpret_cast<const f16x8 *>(pp + P2_BS + (tl + n) * 32 + kg * 16);
-                f32x16 z;
-#pragma unroll
-                for (int r = 0; r < 16; r++) z[r] = 0.0f;
-                ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(ab, bm8, z, 0, 0, 0);
+        for (int t = 0; t < NT; t++) {
+            const int pr = t & 1;
+            if (t == (NT > 2 ? 1 : 0)) dma(nxt, (sb + 1) & 1, y3n);
+            if (t == NT - 1) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile has landed; the planes' requests below stay in flight over the barrier
+                convert((sb + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int rq = 0; rq < 4; rq++) {
-                const f32x4 yd4 = *reinterpret_cast<const f32x4 *>(s_yd + tl + 8 * rq + 4 * kg);
-#ifndef MI355_P2_SCALAR_FOLD
-                // the fold's f32 operations on pairs (v_pk_mul_f32 / v_pk_fma_f32: identical IEEE results, bit-identical to the scalar form below and to the
-                // per-lane kernel; measured 1 % (Q4_K) to 3 % (Q6_K) per launch)
-                typedef float f32x2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-                for (int rp = 0; rp < 2; rp++) {
-                    const int r0 = rq * 4 + 2 * rp, r1 = r0 + 1;
-                    const f32x2 cf = {(float)((H[t][r0] << SH) + L[t][r0]), (float)((H[t][r1] << SH) + L[t][r1])};
-                    const f32x2 yd2 = {yd4[2 * rp], yd4[2 * rp + 1]}, dd2 = {dd, dd};
-                    f32x2 acc = {facc[t][r0], facc[t][r1]};
-                    if (MINS) {
-                        const f32x2 ndm2 = {ndm, ndm}, ms2 = {ms[r0], ms[r1]};
-                        const f32x2 t0 = __builtin_elementwise_fma(dd2, cf, ndm2 * ms2);
-                        acc = __builtin_elementwise_fma(yd2, t0, acc);
-                    } else {
-                        acc = __builtin_elementwise_fma(yd2 * dd2, cf, acc);
-                    }
-                    facc[t][r0] = acc.x; facc[t][r1] = acc.y;
-                }
-#else
-#pragma unroll
-                for (int ri = 0; ri < 4; ri++) {
-                    const int r = rq * 4 + ri;
-                    const float yd = yd4[ri];
-                    const int isum = (H[t][r] << SH) + L[t][r];
-                    if (MINS) {
-                        // dd * isum - dmin * msum:  (-dmin) * msum is -(dmin * msum) bit for bit
-                        const float t0 = fmaf(dd, (float)isum, ndm * ms[r]);
-                        facc[t][r] = fmaf(yd, t0, facc[t][r]);
-                    } else {
-                        facc[t][r] = fmaf(yd * dd, (float)isum, facc[t][r]);
-                    }
-                }
-#endif
-            }
-#ifndef MI355_P2_NOFB
-            __builtin_amdgcn_sched_barrier(0);                   // one tile's block-sum accumulator at a time (four at once spill)
-#endif
-        }
-    };
-#ifdef MI355_P2_PROBE
-    unsigned long long pr_acc[2][3] = {{0, 0, 0}, {0, 0, 0}}, pr_t0 = P2_STAMP();
-    int pr_kind = 0;
-#endif
-    auto stage_end = [&]() {
-#ifdef MI355_P2_PROBE
-        const unsigned long long t1 = P2_STAMP();
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const unsigned long long t2 = P2_STAMP();
-        __syncthreads();
-        const unsigned long long t3 = P2_STAMP();
-        pr_acc[pr_kind][0] += t1 - pr_t0; pr_acc[pr_kind][1] += t2 - t1; pr_acc[pr_kind][2] += t3 - t2;
-        pr_t0 = t3;
-#else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // the next stage has landed (this wave's share; the barrier covers the rest)
-        __syncthreads();
-#endif
-    };
-    // the 4 K-steps of buffer h, K-step-major, as 8 groups of {two token tiles x two planes}; the operands of group g + 1 (and,
-    // every other group, the planes of the next K-step) are requested before the MFMAs of group g are issued: a lone wave
-    // otherwise waits out the LDS latency once per group with its matrix-core slot empty
-    auto mma_stage = [&](int h, bool first) {
-#if MI355_P2_PRIO
-        __builtin_amdgcn_s_setprio(MI355_P2_PRIO);              // tools: the wave in its MFMA phase ahead of the SIMD's other wave (folding / issuing DMA)
-#endif
-        const uint8_t *bs = smem + h * P2_BUF + rw * 8192 + lane * 16;
-        const uint8_t *as = smem + h * P2_BUF + P2_A + a_lane;
-        auto ld_a = [&](int t, int j) {
-            const unsigned slot = ((unsigned)(2 * j + kg) ^ a_key) * 16u;
-            return *reinterpret_cast<const i32x4 *>(as + t * 32 * 128 + slot);
-        };
-        i32x4 bh = *reinterpret_cast<const i32x4 *>(bs), bl = *reinterpret_cast<const i32x4 *>(bs + 1024);
-        i32x4 a0 = ld_a(0, 0), a1 = ld_a(1, 0);
-#pragma unroll
-        for (int g = 0; g < 8; g++) {
-            const int j = g >> 1, t0 = (g & 1) * 2;
-            i32x4 n0 = a0, n1 = a1, nbh = bh, nbl = bl;
-            if (g < 7) {
-                n0 = ld_a((t0 + 2) & 3, (g + 1) >> 1); n1 = ld_a((t0 + 3) & 3, (g + 1) >> 1);
-                if (g & 1) { nbh = *reinterpret_cast<const i32x4 *>(bs + (j + 1) * 2048); nbl = *reinterpret_cast<const i32x4 *>(bs + (j + 1) * 2048 + 1024); }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int t = t0 + u;
-                const i32x4 a = u ? a1 : a0;
-                if (MI355_P2_EXP == 3) {
-                    if (first && j == 0) { for (int r = 0; r < 16; r++) { H[t][r] = 0; L[t][r] = 0; } }
-                    H[t][j] += a.x + bh.y; L[t][j] += a.z + bl.w;
-                } else if (first && j == 0) {
+            for (int j = 0; j < 8; j++) {
+                if (t > 0 && j == 0) mins();
+                if (j == 0) {
                     i32x16 z;
 #pragma unroll
                     for (int r = 0; r < 16; r++) z[r] = 0;
-                    H[t] = mfma_i8(a, bh, z); L[t] = mfma_i8(a, bl, z);
-                } else { H[t] = mfma_i8(a, bh, H[t]); L[t] = mfma_i8(a, bl, L[t]); }
+                    H[pr] = mfma_i8(A[0], B[0][0], z); L[pr] = mfma_i8(A[0], B[0][1], z);
+                } else { H[pr] = mfma_i8(A[j & 1], B[j][0], H[pr]); L[pr] = mfma_i8(A[j & 1], B[j][1], L[pr]); }
+                if (j < 6) A[j & 1] = ld_a(t, j + 2);
+                else if (t + 1 < NT) A[j & 1] = ld_a(t + 1, j - 6);
+                if (MINS && j == 4) as = *reinterpret_cast<const f16x8 *>(sm_bs + sbuf + (32 * t + n) * 32 + kg * 16);
+                if (t == NT - 1) ld_b(blkn, j);
+                if (t > 0) fold(t - 1, pr ^ 1, j, ys + (t - 1) * 128);
+                if (j == 7) yd = *reinterpret_cast<const f32x4 *>(ys + t * 128);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
-            a0 = n0; a1 = n1; bh = nbh; bl = nbl;
         }
-#if MI355_P2_PRIO
-        __builtin_amdgcn_s_setprio(0);
-#endif
-    };
-
-    issue_v(0, wave);
-    issue_sb_v(0, wave);
-    stage_end();
-    // first-half stages: waves 4-7 fold there, so waves 0-3 issue - unless waves 4-7 have no tokens and nothing else to do;
-    // second-half stages: waves 0-3 fold, waves 4-7 issue
-    const int issuer0 = (tok0 + 128 >= T) ? 1 : 0, issuer1 = 1;
-    if (idle_half) {
-        for (int sb = 0; sb < nb; sb++) {
-            issue(2 * sb + 1, issuer0);
-            convert_bs(sb);
-            stage_end();
-            if (sb + 1 < nb) { issue(2 * sb + 2, issuer1); issue_sb(sb + 1, issuer1); }
-            stage_end();
-        }
-    } else
-    for (int sb = 0; sb < nb; sb++) {
-        // ---- first half (buffer 0).  The block sums of sb (landed with the barrier just passed) become f16 here, one barrier
-        // ahead of their first use; waves 4-7 fold super-block sb - 1 before they overwrite its accumulators.
-#ifdef MI355_P2_PROBE
-        pr_kind = 0;
-#endif
-#if MI355_P2_LATE_DMA
-        // tools: the issuing half runs its MFMAs FIRST and issues the next stage's DMA behind them (the folding half's MFMAs then find the pipe free);
-        // the DMA has less of the stage left to land in
-        convert_bs(sb);
-        if (tw == 1 && sb > 0) fold_all((sb - 1) & 1);
-        mma_stage(0, true);
-        issue(2 * sb + 1, issuer0);
-        stage_end();
-#else
-        issue(2 * sb + 1, issuer0);
-        convert_bs(sb);
-        if (tw == 1 && sb > 0) fold_all((sb - 1) & 1);
-        mma_stage(0, true);
-        stage_end();
-#endif
-        // ---- second half (buffer 1).  The words of super-block sb + 1 go to the other parity, which waves 4-7 finished
-        // reading in the stage just ended; waves 0-3 fold sb at the end of this one.
-#ifdef MI355_P2_PROBE
-        pr_kind = 1;
-#endif
-#if MI355_P2_LATE_DMA
-        mma_stage(1, false);
-        if (sb + 1 < nb) { issue(2 * sb + 2, issuer1); issue_sb(sb + 1, issuer1); }
-        if (tw == 0 || sb + 1 == nb) fold_all(sb & 1);
-        stage_end();
-#else
-        if (sb + 1 < nb) { issue(2 * sb + 2, issuer1); issue_sb(sb + 1, issuer1); }
-        mma_stage(1, false);
-        if (tw == 0 || sb + 1 == nb) fold_all(sb & 1);
-        stage_end();
-#endif
-    }
-    if (MI355_P2_EXP == 1) {
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) facc[t][r] = (float)(H[t][r] + L[t][r]);
-    }
-
-#ifdef MI355_P2_PROBE
-    if (g_p2_probe && blockIdx.x == 0 && lane == 0) {
-        const unsigned long long t4 = P2_STAMP();
-        unsigned long long *o = g_p2_probe + wave * 8;
-        for (int k = 0; k < 2; k++) for (int c = 0; c < 3; c++) o[k * 3 + c] = pr_acc[k][c];
-        o[6] = t4 - pr_t0;                                      // last fold
-    }
-#endif
-    if (SWIGLU) {                                               // the up tile crosses to the gate wave of the same rows and tokens
-        float *exch = reinterpret_cast<float *>(smem) + (size_t)((rw & 1) * 2 + tw) * (MT * 16 * 64) + lane;   // (both buffers are idle now)
-        if (rw >= 2) {
-#pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) exch[(t * 16 + r) * 64] = facc[t][r];
-        }
+        yprev = ys + (NT - 1) * 128;
+        y3 = y3n;
         __syncthreads();
-        if (rw < 2 && tile_ok && row0 + n < n_rows) {
+    }
+    mins();
+#pragma unroll
+    for (int p = 0; p < 8; p++) fold(NT - 1, (NT - 1) & 1, p, yprev);
+}
+
+// SWIGLU: `planes` = ffn_gate, `planes_up` = ffn_up (n_rows rows each, same type): a workgroup takes 64 rows of BOTH (row-waves 0, 1 the
+// gate rows, 2, 3 the same rows of up), the two waves of the same rows swap halves of their tiles through LDS at the end and store
+// silu(gate . x) * (up . x) - one [T][n_rows] f32 result instead of two, and no separate SwiGLU pass over them
+template <bool MINS, bool SWIGLU>
+__device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &po, int row_tile, int tok_tile, int n_tok_tiles, int zz) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb_all = a.K >> 8;
+    const int sb_lo = (int)((long)nb_all * zz / a.n_split), nb = (int)((long)nb_all * (zz + 1) / a.n_split) - sb_lo;
+    const int n_rows = a.n_rows, T = a.T;
+    const int n_rt32 = (n_rows + 31) >> 5;
+    const int rw = wave & 3, tw = wave >> 2;
+    const int rt32 = SWIGLU ? row_tile * 2 + (rw & 1) : row_tile * 4 + rw;
+    const uint8_t *base = SWIGLU && rw >= 2 ? a.planes_up : a.planes;
+    const bool tile_ok = rt32 < n_rt32;
+    // the batch's 32-token tiles, dealt evenly: to the workgroups' token tiles, and there to the two halves
+    const int units = (T + 31) >> 5, per = (units + n_tok_tiles - 1) / n_tok_tiles, mine_u = units - tok_tile * per < per ? units - tok_tile * per : per;
+    const int nt = mine_u <= 0 ? 0 : tw ? mine_u >> 1 : (mine_u + 1) >> 1;
+    const int row0 = rt32 * 32, tok0 = (tok_tile * per + (tw ? (mine_u + 1) >> 1 : 0)) * 32, n = lane & 31, kg = lane >> 5, row = row0 + n;
+    gbytes *blk0 = scalar_ptr(base + ((size_t)(tile_ok ? rt32 : n_rt32 - 1) * nb_all + sb_lo) * PL_BLOCK);
+    float facc[4][16];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) facc[t][r] = 0.0f;
+#define P2_LOOP(NTV, FULLV) planes2_loop<MINS, NTV, FULLV>(blk0, a, sb_lo, nb, tok0, tid, tw, smem, facc)
+    if (nt == 4 && T - tok0 >= 128) P2_LOOP(4, true);
+    else if (nt == 4) P2_LOOP(4, false);
+    else if (nt == 3) P2_LOOP(3, false);
+    else if (nt == 2) P2_LOOP(2, false);
+    else if (nt == 1) P2_LOOP(1, false);
+    else for (int i = 0; i <= nb; i++) __syncthreads();         // (a half without tokens keeps the barriers)
+#undef P2_LOOP
+    const bool all = nt == 4 && T - tok0 >= 128 && row0 + 32 <= n_rows;
+    const int t_end = tok0 + 32 * nt < T ? tok0 + 32 * nt : T;  // tokens of this half: [tok0, t_end)
+    auto token = [&](int t, int r) { return tok0 + 32 * t + (r & 3) + 8 * (r >> 2) + 4 * kg; };
+    if (SWIGLU) {                                               // waves w (gate rows) and w + 2 (the same rows of up) swap halves: w finishes tokens 0 .. 63, w + 2 the others
+        float *mine = reinterpret_cast<float *>(smem) + wave * 2048 + lane, *theirs = reinterpret_cast<float *>(smem) + (wave ^ 2) * 2048 + lane;
+        auto give = [&](int t0) {
+#pragma unroll
+            for (int i = 0; i < 32; i++) mine[i * 64] = facc[t0 + (i >> 4)][i & 15];
+        };
+        auto finish = [&](int t0, bool all_) {
             float *out = po.out[0];
             const int ld_out = po.ld[0];
 #pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int gt = tok0 + (tw * MT + t) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
-                    const float gv = facc[t][r], uv = exch[(t * 16 + r) * 64];
-                    if (gt < T) out[(size_t)gt * ld_out + row0 + n] = (gv / (1.0f + expf(-gv))) * uv;
-                }
-        }
+            for (int i = 0; i < 32; i++) {
+                const int t = t0 + (i >> 4), gt = token(t, i & 15);
+                const float own = facc[t][i & 15], oth = theirs[i * 64], gv = t0 ? oth : own, uv = t0 ? own : oth;
+                const float y = (gv / (1.0f + expf(-gv))) * uv;
+                if (all_ || (gt < t_end && row < n_rows)) out[(size_t)gt * ld_out + row] = y;
+            }
+        };
+        if (rw < 2) give(2); else give(0);
+        __syncthreads();
+        if (!tile_ok) return;
+        if (all) { if (rw < 2) finish(0, true); else finish(2, true); }
+        else { if (rw < 2) finish(0, false); else finish(2, false); }
         return;
     }
-    if (n_split > 1) {                                          // partial sums of this K range: ws[zz][token][row], no residual
-        if (tile_ok && row0 + n < n_rows) {
-            float *o = ws + (size_t)zz * T * n_rows;
+    if (!tile_ok) return;
+    int sg = 0;
+    if (po.n_seg > 1 && row0 >= po.row_end[0]) sg = 1;
+    if (po.n_seg > 2 && row0 >= po.row_end[1]) sg = 2;
+    const bool split = a.n_split > 1;                           // partial sums of this K range: ws[zz][token][row], no residual
+    float *out = split ? a.ws + (size_t)zz * T * n_rows : po.out[sg] - (sg ? po.row_end[sg - 1] : 0);
+    const int ld_out = split ? n_rows : po.ld[sg];
+    if (a.resid && !split) {
 #pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int gt = tok0 + (tw * MT + t) * 32 + (r & 3) + 8 * (r >> 2) + 4 * kg;
-                    if (gt < T) o[(size_t)gt * n_rows + row0 + n] = facc[t][r];
-                }
-        }
-        return;
-    }
-    if (tile_ok && row0 + n < n_rows) {
-        int sg = 0;
-        if (po.n_seg > 1 && row0 >= po.row_end[0]) sg = 1;
-        if (po.n_seg > 2 && row0 >= po.row_end[1]) sg = 2;
-        float *out = po.out[sg] - (sg ? po.row_end[sg - 1] : 0);
-        const int ld_out = po.ld[sg];
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-            float rv[16];
+        for (int t = 0; t < 4; t++) {
+            float rv[16];                                       // (all requested before the first add)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int m = (r & 3) + 8 * (r >> 2) + 4 * kg;
-                int gt = tok0 + (tw * MT + t) * 32 + m;
-                if (gt >= T) gt = T - 1;
-                rv[r] = resid ? resid[(size_t)gt * ld_out + row0 + n] : 0.0f;
+                const int gt = token(t, r);
+                rv[r] = a.resid[(size_t)(gt < T ? gt : T - 1) * ld_out + (row < n_rows ? row : n_rows - 1)];
             }
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = (r & 3) + 8 * (r >> 2) + 4 * kg;
-                const int gt = tok0 + (tw * MT + t) * 32 + m;
-                if (gt < T) out[(size_t)gt * ld_out + row0 + n] = rv[r] + facc[t][r];
-            }
+            for (int r = 0; r < 16; r++) facc[t][r] = rv[r] + facc[t][r];
         }
     }
+    auto store = [&](bool all_) {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int gt = token(t, r);
+                if (all_ || (gt < t_end && row < n_rows)) out[(size_t)gt * ld_out + row] = facc[t][r];
+            }
+    };
+    if (all) store(true); else store(false);
 }
 
 // MODE 0: Q6_K planes (signed codes, no block-sum term); 1: Q4_K / Q5_K; 2: per segment (po.mins_mask; segment boundaries at multiples of
@@ -1493,8 +1348,9 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *pl
         if (po.n_seg > 2 && row_tile * P2_ROWS >= po.row_end[1]) sg0 = 2;
         mins = (po.mins_mask >> sg0) & 1u;
     }
-    if (MODE == 1 || (MODE == 2 && mins)) planes2_body<true, false>(planes, nullptr, n_rows, K, T, n_row_tiles, n_tok_tiles, aq, ad, absum, po, resid, ws, n_split, row_tile, tok_tile, zz);
-    else planes2_body<false, false>(planes, nullptr, n_rows, K, T, n_row_tiles, n_tok_tiles, aq, ad, absum, po, resid, ws, n_split, row_tile, tok_tile, zz);
+    const P2Args a{planes, nullptr, n_rows, K, T, aq, ad, absum, resid, ws, n_split};
+    if (MODE == 1 || (MODE == 2 && mins)) planes2_body<true, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
+    else planes2_body<false, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
 }
 
 // ffn_gate and ffn_up with SwiGLU in the epilogue: n_rows rows of each, 64 per workgroup, out[t][row] = silu(gate) * up
@@ -1506,20 +1362,20 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_kernel(const uint
     const int tok_tile = loc % n_tok_tiles;
     const int row_tile = (loc / n_tok_tiles) * 8 + xcd;
     if (row_tile >= n_row_tiles) return;                       // workgroup-uniform
-    planes2_body<MINS, true>(planes_gate, planes_up, n_rows, K, T, n_row_tiles, n_tok_tiles, aq, ad, absum, po, nullptr, nullptr, 1, row_tile, tok_tile, 0);
+    planes2_body<MINS, true>(P2Args{planes_gate, planes_up, n_rows, K, T, aq, ad, absum, nullptr, nullptr, 1}, po, row_tile, tok_tile, n_tok_tiles, 0);
 }
 
 // ---- ggml_mul_mat_id on a prompt batch as ONE launch per projection (round 5).  The (token, rank) pairs of the batch are sorted by expert (moe_group_kernel: expert
 // e owns rows [meta[NE + e], + meta[e]) of the grouped activation / result arrays); a workgroup is (row tile, token-tile slot j): slot j is the j-th 256-token tile
 // of the concatenation of the experts' batches, found by walking the per-expert counts ON THE DEVICE - no host synchronisation to size per-expert launches, and
-// eight half-empty launches of ~128 tokens become one that fills the chip.  The body is planes2_body unchanged: the wrapper hands it the expert's planes, the
+// eight half-empty launches of ~128 tokens become one that fills the chip.  The body is planes2_body: the wrapper hands it the expert's planes, the
 // batch's rows as "the" token range (pointers offset to the batch's first row, T = the batch's length) and the tile index within the batch.
 struct MoeTiles { const int32_t *meta; int n_expert; size_t plane_stride; };     // meta: [0, NE) tokens per expert, [NE, 2 NE) first grouped row
 __device__ __forceinline__ bool moe_tile_of(const MoeTiles &m, int j, int &e_out, int &tile_out, int &r0_out, int &n_out) {
     for (int e = 0; e < m.n_expert; e++) {                      // (scalar: the counts are a few words of one cache line)
-        const int n_e = m.meta[e];
+        const int n_e = __builtin_amdgcn_readfirstlane(m.meta[e]);
         const int tiles = (n_e + P2_TOK - 1) / P2_TOK;
-        if (j < tiles) { e_out = e; tile_out = j; r0_out = m.meta[m.n_expert + e]; n_out = n_e; return true; }
+        if (j < tiles) { e_out = e; tile_out = j; r0_out = __builtin_amdgcn_readfirstlane(m.meta[m.n_expert + e]); n_out = n_e; return true; }
         j -= tiles;
     }
     return false;
@@ -1536,8 +1392,8 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_moe_kernel(const 
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
     po.out[0] += (size_t)r0 * po.ld[0];
-    planes2_body<MINS, true>(planes_gate + (size_t)e * mt.plane_stride, planes_up + (size_t)e * mt.plane_stride, n_rows, K, n_e, n_row_tiles, (n_e + P2_TOK - 1) / P2_TOK,
-                             aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), po, nullptr, nullptr, 1, row_tile, tile, 0);
+    planes2_body<MINS, true>(P2Args{planes_gate + (size_t)e * mt.plane_stride, planes_up + (size_t)e * mt.plane_stride, n_rows, K, n_e,
+                                    aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 template <bool MINS>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t *planes, int n_rows, int K, int n_row_tiles, int n_tile_slots,
@@ -1550,8 +1406,8 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
     po.out[0] += (size_t)r0 * po.ld[0];
-    planes2_body<MINS, false>(planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e, n_row_tiles, (n_e + P2_TOK - 1) / P2_TOK,
-                              aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), po, nullptr, nullptr, 1, row_tile, tile, 0);
+    planes2_body<MINS, false>(P2Args{planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e,
+                                     aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 
 // out[t][row] = (resid) + ws[0][t][row] + ws[1][t][row] + ... in split order (fixed, so results do not depend on timing)
@@ -1622,9 +1478,6 @@ hipError_t launch_type(const uint8_t *W, size_t row_bytes, int n_rows, int K, in
 void mmq_set_tiles(int mt) { g_mmq_mt = mt; }
 void mmq_set_split(int n) { g_mmq_split = n; }
 void mmq_set_lds_form(int on) { g_mmq_p2 = on; }
-#ifdef MI355_P2_PROBE
-void mmq_p2_set_probe(unsigned long long *p) { (void)hipMemcpyToSymbol(HIP_SYMBOL(g_p2_probe), &p, sizeof(p)); }
-#endif
 
 // continuous-batching decode steps and prompts up to a few hundred tokens: 3 <= T <= g_ksplit_max.  This kernel reads the GGUF
 // bytes (0.56 B / weight) and expands them in registers, the planes kernel reads 2 B / weight it need not expand: measured on the
@@ -1648,10 +1501,12 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
 // (pair: gate | up of a dense layer go out as ONE K-split launch of 2 n_rows rows, which holds its own against two planes launches up to
 // 128 tokens - whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128; past that the LDS-form SwiGLU launch takes the pair:
 // 13.6 -> 10.6 ms at 200 tokens, 14.1 -> 11.1 at 256.)
+// From 129 tokens on the 128 x 256 tiles with K split over the workgroups take every tensor that has planes: prompts of 140, 160, 200 and 256 tokens through eight layers of an
+// 8B model (Q4_K_M) 2.75, 2.81, 3.20 and 3.32 ms by the K-split kernel here, 1.95, 2.00, 2.26 and 2.36 by them; of a 7B model (Q5_K_M) 2.69 .. 3.26 against 1.84 .. 2.24.
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool pair) {
     static const int env = getenv("MI355_KSPLIT_SHAPE") ? atoi(getenv("MI355_KSPLIT_SHAPE")) : 1;
     if (!mmq_ksplit_applicable(type, K, T)) return false;
-    if (env && has_planes && T > (pair ? 128 : 64) && n_rows >= 8192 && mmq_applicable(type, K, T)) return false;
+    if (env && has_planes && (T > 128 || (T > 64 && !pair && n_rows >= 8192)) && mmq_applicable(type, K, T)) return false;
     return true;
 }
 
@@ -1725,18 +1580,18 @@ static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool
     const int env_p2 = g_mmq_p2 >= 0 ? g_mmq_p2 : env_p2_0;
     static const int env_sk = getenv("MI355_MMQ_SPLITK") ? atoi(getenv("MI355_MMQ_SPLITK")) : -1;   // 0 off, 2..4 forced
     const int nb = K >> 8;
-    const long wg4 = (long)((n_rows + P2_ROWS - 1) / P2_ROWS) * ((T + P2_TOK - 1) / P2_TOK);
+    const long wg = (long)((n_rows + P2_ROWS - 1) / P2_ROWS) * ((T + P2_TOK - 1) / P2_TOK);
+    // One workgroup fills a CU, so K is split while the parts still run side by side - at least four super-blocks each, for a workgroup's start and end cost two.  us a launch
+    // (Q4_K; unsplit / by this rule / one part more; the planes kernel below): 4096 x 4096 at 160, 512, 611, 1280 tokens 55 / 27 / -, 62 / 38 / -, 61 / 46 / 64,
+    // 71 / 71 / 92 against 53, 48, 78, 126; 4096 x 14336: 169 / 59 / -, 205 / 82 / -, 189 / 114 / 158, 217 / 217 / 247 against 145, 144, 249, 396;
+    // 6144 x 4096 at 160 and 512: 57 / 33 / -, 66 / 50 / 71 against 50, 93; 22016 x 4096 at 160 and 512: 63 / 63 / 81, 141 / 141 / 149 against 99, 213.
     int n_split = 1;
     if (g_mmq_split > 1 || env_sk > 1) n_split = g_mmq_split > 1 ? g_mmq_split : env_sk;
-    else if (wg4 * 4 < 3L * num_cu() && env_sk != 0 && g_mmq_split != 1) {
-        n_split = (int)((num_cu() + wg4 - 1) / wg4);
-        if (n_split > 4) n_split = 4;
-        if (n_split > nb / 8) n_split = nb / 8;                 // at least eight super-blocks per workgroup: a 4096-wide K split four ways
-                                                                // (40.9 us with its reduction) loses to the 256 x 32 tiles (37.9), a 14336-wide one wins (89.7 vs 120.9)
-    }
+    else if (env_sk != 0 && g_mmq_split != 1) n_split = (int)std::max(1L, std::min({num_cu() / wg, 4L, (long)nb / 4}));
     if (n_split > nb) n_split = nb;
     if (n_split < 1 || (n_rows % 4) != 0 || !wsp.p || (size_t)n_split * T * n_rows * sizeof(float) > wsp.bytes) n_split = 1;
-    *takes = g_mmq_mt == 4 || (g_mmq_mt == 0 && env_mt == 0 && env_p2 != 0 && T > 128 && wg4 * n_split * 4 >= 3L * num_cu());
+    // (an unsplit launch wants a third of the CUs: 11264 x 2048 at 160 and 256 tokens - 88 workgroups - 35 and 40 us against 31 and 56, 4096 x 4096 at 300 - 64 - 53 against 47)
+    *takes = g_mmq_mt == 4 || (g_mmq_mt == 0 && env_mt == 0 && env_p2 != 0 && T > 128 && (n_split > 1 || wg * 3 >= num_cu()));
     return n_split;
 }
 

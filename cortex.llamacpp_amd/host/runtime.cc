@@ -686,11 +686,10 @@ bool Context::init(std::string &err) {
     mmq_bl_ = (int8_t *)dalloc(mmq_prep_bytes((int)std::max(E, FF), prep_rows));
     // partial sums of the K-split prompt contraction: only tensors with few rows split (Q | K | V, attention output, FFN down),
     // up to four ways; tensors that do not fit fall back to an unsplit kernel
-    // A launch only splits while its 128 x 256 tiles number fewer than 3/4 of the CUs, and then into ceil(CUs / tiles) <= 4 parts (mmq.hip planes2_split):
-    // n_split * tiles < CUs + tiles < 7/4 CUs, i.e. never more than 7/4 * CUs tiles' worth of partial sums whatever the model (58.7 MB on 256 CUs;
-    // sized by the widest tensor instead it was 335 MB per context for Llama-3-70B at n_ubatch 2048)
+    // A launch splits into floor(CUs / tiles) <= 4 parts of its 128 x 256 tiles (mmq.hip planes2_split), i.e. never into more than CUs tiles' worth of partial
+    // sums whatever the model (33.6 MB on 256 CUs; sized by the widest tensor instead it was 335 MB per context for Llama-3-70B at n_ubatch 2048)
     mmq_ws_.bytes = std::min((size_t)4 * T * std::max<size_t>(E, (size_t)(hp.n_head + 2 * hp.n_head_kv) * D) * sizeof(float),
-                             (size_t)(num_cu() * 7 / 4) * 128 * 256 * sizeof(float));
+                             (size_t)num_cu() * 128 * 256 * sizeof(float));
     mmq_ws_.p = T >= 128 ? (float *)dalloc(mmq_ws_.bytes) : nullptr;
     if (!mmq_ws_.p) mmq_ws_.bytes = 0;
     if (!ok || !x_ || !ffn_u_) { err = "activation buffer allocation failed"; return false; }
@@ -1025,7 +1024,10 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     for (int i = 0; i < n; i++) all_q &= is_quant(ws[i]->type);
     const int K = (int)ws[0]->K;
     bool all_mmq = true, all_ks = true;
-    for (int i = 0; i < n; i++) { all_mmq &= mmq_applicable(ws[i]->type, K, T); all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T); }
+    for (int i = 0; i < n; i++) {
+        all_mmq &= mmq_applicable(ws[i]->type, K, T);
+        all_ks &= T > 128 ? mmq_ksplit_preferred(ws[i]->type, (int)ws[i]->N, K, T, ws[i]->planes != nullptr) : mmq_ksplit_applicable(ws[i]->type, K, T);
+    }
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
         HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
         MMQSeg sg[3];

@@ -1,0 +1,52 @@
+"""Prompt contraction in 128-row x 256-token workgroup tiles (csrc/mmq.hip mmq_planes2_kernel): how a batch's 32-token tiles are dealt to workgroups and to their halves."""
+import numpy as np
+import pytest
+
+import oracle_py as oq
+from test_gpu_ops import Q2_K, Q4_K, Q5_K, Q6_K, be, rand_weights  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q2_K])
+@pytest.mark.parametrize("K,N,T", [(768, 130, 32), (256, 96, 64), (1024, 33, 90),        # a half without tokens; one tile each; two and one, the last one ragged
+                                   (768, 160, 128), (512, 70, 160), (768, 128, 224),      # two and two, three and two, four and three
+                                   (1280, 129, 250), (768, 256, 256), (512, 40, 257),     # a full half beside a ragged one; both full; nine tiles over two workgroups
+                                   (256, 130, 611)])                                      # twenty tiles over three
+def test_token_tiles(be, t, K, N, T):  # noqa: F811
+    """Against the oracle (f32 order over super-blocks, each rounding half an ulp: 2e-5 of the largest output as for the other contractions) and bit for bit against the
+    kernel whose waves take two token tiles: same integers, same fold, same order."""
+    rng = np.random.default_rng(5 * K + N + T + t)
+    W = rand_weights(rng, t, N * K)
+    x = (rng.standard_normal((T, K)) * rng.uniform(0.1, 4.0, (T, 1))).astype(np.float32)
+    be.set_option("mmq_planes", 1)
+    be.set_option("mmq_ksplit", 0)
+    try:
+        be.set_option("mmq_tiles", 4)
+        be.set_option("mmq_split", 1)
+        y = be.mul_mat(t, W, N, K, x)
+        be.set_option("mmq_tiles", 2)
+        y2 = be.mul_mat(t, W, N, K, x)
+    finally:
+        be.set_option("mmq_tiles", 0)
+        be.set_option("mmq_split", 0)
+        be.set_option("mmq_ksplit", 1)
+    ref = oq.mul_mat(t, W, N, K, x)
+    assert np.abs(y - ref).max() <= 2e-5 * np.abs(ref).max() + 1e-6
+    assert np.array_equal(y, y2)
+
+
+@pytest.mark.parametrize("t", [Q5_K, Q6_K])
+@pytest.mark.parametrize("K,N,T", [(2048, 1030, 129), (4096, 516, 300), (1024, 4100, 700), (768, 260, 1040)])
+def test_split_by_rule(be, t, K, N, T):  # noqa: F811
+    """No tile or split set: K is split by the number of workgroups (four parts, two, none) - or not, below eight super-blocks."""
+    rng = np.random.default_rng(3 * K + N + T + t)
+    W = rand_weights(rng, t, N * K)
+    x = (rng.standard_normal((T, K)) * rng.uniform(0.1, 4.0, (T, 1))).astype(np.float32)
+    be.set_option("mmq_ksplit", 0)
+    try:
+        y = be.mul_mat(t, W, N, K, x)
+    finally:
+        be.set_option("mmq_ksplit", 1)
+    ref = oq.mul_mat(t, W, N, K, x)
+    assert np.abs(y - ref).max() <= 2e-5 * np.abs(ref).max() + 1e-6

@@ -1,6 +1,5 @@
 // tools/exp_p2.hip — the prompt contraction on pre-expanded planes: per-lane planes kernel (128 x 128 tiles) against the kernel with both
-// operands through LDS (128 x 256): bit-for-bit comparison on synthetic planes, time per launch (HIP events), and with
-// -DMI355_P2_PROBE the per-wave cycle split of workgroup 0.
+// operands through LDS (128 x 256): bit-for-bit comparison on synthetic planes and time per launch (HIP events).
 // build: tools/build_exp_p2.sh
 #include <cstdio>
 #include <cstdlib>
@@ -16,9 +15,6 @@ void set_num_cu(int n) { g_ncu = n; }
 int num_cu() { return g_ncu; }
 void mmq_set_tiles(int mt);
 void mmq_set_split(int n);
-#ifdef MI355_P2_PROBE
-void mmq_p2_set_probe(unsigned long long *p);
-#endif
 }
 using namespace mi355;
 #define CK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { printf("%s failed: %s (line %d)\n", #x, hipGetErrorString(e_), __LINE__); exit(1); } } while (0)
@@ -74,13 +70,7 @@ int main(int argc, char **argv) {
         return ms * 1e3f / reps;
     };
     const float us1 = run(1, o_old, 1), us2 = run(2, o_old, 1);
-#ifdef MI355_P2_PROBE
-    unsigned long long *probe; CK(hipMalloc(&probe, 64 * 8)); CK(hipMemset(probe, 0, 64 * 8)); mmq_p2_set_probe(probe);
-#endif
     const float us4 = run(4, o_new, 1);
-#ifdef MI355_P2_PROBE
-    unsigned long long hpz[64]; CK(hipMemcpy(hpz, probe, sizeof(hpz), hipMemcpyDeviceToHost));   // (of the unsplit launch)
-#endif
     float *o_sk; CK(hipMalloc(&o_sk, (size_t)T * N * 4));
     float us_sk[5] = {0, 0, 0, 0, 0};
     for (int sp = 2; sp <= 4; sp++) us_sk[sp] = run(4, o_sk, sp);
@@ -96,11 +86,5 @@ int main(int argc, char **argv) {
     const double top = 2.0 * N * K * T / 1e6;
     printf("N %d K %d T %d type %d: 256x32 %.1f us (%.0f TOP/s)  128x128 %.1f us (%.0f)  lds 128x256 %.1f us (%.0f)  mismatches %zu / %zu  sample %g\n",
            N, K, T, type, us1, top / us1, us2, top / us2, us4, top / us4, bad, a.size(), (double)b[12345 % b.size()]);
-#ifdef MI355_P2_PROBE
-    { unsigned long long *tk, htk = 0; CK(hipMalloc(&tk, 8)); hipLaunchKernelGGL(tick_kernel, dim3(1), dim3(64), 0, 0, tk); CK(hipMemcpy(&htk, tk, 8, hipMemcpyDeviceToHost));
-      printf("  s_memtime: %.1f ticks per us\n", htk / 100.0); }
-    printf("  workgroup 0, cycles per wave over %d super-blocks:   first half: compute / dma wait / barrier   second half: compute / dma wait / barrier   last fold\n", nb);
-    for (int w = 0; w < 8; w++) printf("   wave %d: %8llu %8llu %8llu    %8llu %8llu %8llu    %8llu\n", w, hpz[w * 8], hpz[w * 8 + 1], hpz[w * 8 + 2], hpz[w * 8 + 3], hpz[w * 8 + 4], hpz[w * 8 + 5], hpz[w * 8 + 6]);
-#endif
     return bad ? 1 : 0;
 }
