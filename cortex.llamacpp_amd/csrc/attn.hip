@@ -502,6 +502,17 @@ __global__ __launch_bounds__(256) void flash_attn_combine_kernel(const float *pa
     if (tok_nsplits) splits = tok_nsplits[t];
     const int hpb = 256 / D;                       // heads per block (D = 64 -> 4, D = 128 -> 2)
     const int h0 = b * hpb;
+    // the output element's first U partials are requested in front of the weights, the next U in front of the sum over these (read one by one behind the test of
+    // their weight they cost a round trip to memory each: 7.5 us for the eleven splits of 640 cells, 37 tokens, 32 heads)
+    constexpr int U = 8;
+    const int hl = tid / D;
+    const float *pe = part + ((size_t)t * H + h0 + hl) * stride_s * (D + 2) + (tid - hl * D);
+    auto fetch = [&](int s0, float (&v)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = pe[(size_t)(s0 + u < splits ? s0 + u : 0) * (D + 2)];
+    };
+    float v[U];
+    fetch(0, v);
     if (wave < hpb) {
         const float *p = part + ((size_t)t * H + h0 + wave) * stride_s * (D + 2);
         float M = -INFINITY;
@@ -526,17 +537,19 @@ __global__ __launch_bounds__(256) void flash_attn_combine_kernel(const float *pa
         for (int sidx = lane; sidx < splits; sidx += 64) wgt[wave * stride_s + sidx] *= inv;
     }
     __syncthreads();
-    {
-        const int e = tid, hl = e / D, d = e - hl * D;
-        const float *p = part + ((size_t)t * H + h0 + hl) * stride_s * (D + 2) + d;
-        float acc = 0.0f;
-        for (int s = 0; s < splits; s++) {
-            const float w = wgt[hl * stride_s + s];
-            if (w != 0.0f) acc += w * p[(size_t)s * (D + 2)];        // chunks with no visible cell publish only (m, l)
+    float acc = 0.0f;
+    for (int s0 = 0; s0 < splits; s0 += U) {
+        float nx[U];
+        fetch(s0 + U, nx);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float w = s0 + u < splits ? wgt[hl * stride_s + s0 + u] : 0.0f;
+            acc = w != 0.0f ? acc + w * v[u] : acc;                  // chunks with no visible cell publish only (m, l)
+            v[u] = nx[u];
         }
-        merged[e] = acc;
-        out[(size_t)t * E + b * 256 + e] = acc;
     }
+    merged[tid] = acc;
+    out[(size_t)t * E + b * 256 + tid] = acc;
     __syncthreads();
     if (wave == 0 && (want_q8k || want_q80)) {
         const float4 v4 = *reinterpret_cast<const float4 *>(merged + lane * 4);
