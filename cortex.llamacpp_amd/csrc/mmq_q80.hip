@@ -1,4 +1,4 @@
-// mmq_q80.hip — prompt batches against Q8_0 weights on the matrix cores (mul_mat_q for Q8_0, SURVEY.md §8 a10).
+// mmq_q80.hip — prompt batches against Q8_0 weights on the matrix cores (mul_mat_q for Q8_0).
 //
 //   out[t][r] = sum over 32-blocks b of  (float)isum_b * (d_w[r][b] * d_a[t][b]),   isum_b = sum_{k in b} w[r][k] * a[t][k]
 //
@@ -13,6 +13,8 @@
 // 16 x (convert, scale product, multiply-add): the fold is the bound (VALU), ~1/8 of the int8 matrix peak — against one
 // pass over the weights per 16 tokens with the tiled mat-vec this replaces for T >= 32.
 // Workgroup = 4 waves = 128 weight rows x 32 tokens; the four waves share the token tile (L1 hits on the activations).
+#include <type_traits>
+
 #include "kernels.h"
 #include "quant_dev.h"
 
@@ -24,6 +26,7 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int Q80_UNROLL = 4;
 
@@ -35,8 +38,8 @@ template <int MT>
 __global__ __launch_bounds__(256) void mmq_q80_kernel(const uint8_t *__restrict__ W, size_t row_bytes, int n_rows, int K, int T,
                                                       const int8_t *__restrict__ aq, const uint16_t *__restrict__ ad, float *__restrict__ out,
                                                       int ld_out, const float *__restrict__ resid) {
-    __shared__ __attribute__((aligned(16))) float s_da[Q80_KC * 32 * MT];      // [block of the chunk][token of the workgroup's tile]
-    constexpr int TT = 32 * MT;
+    constexpr int TT = 32 * MT, SD = TT + 4;
+    __shared__ __attribute__((aligned(16))) float s_da[Q80_KC * SD];           // [block of the chunk][token of the workgroup's tile]
     const int nb = K >> 5;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 31, kg = lane >> 5;
@@ -66,7 +69,7 @@ __global__ __launch_bounds__(256) void mmq_q80_kernel(const uint8_t *__restrict_
         const f32x2 dw2 = {dw, dw};
 #pragma unroll
         for (int rq = 0; rq < 4; rq++) {
-            const f32x4 da4 = *reinterpret_cast<const f32x4 *>(s_da + bl * TT + 32 * m + 8 * rq + 4 * kg);    // tokens 8 rq + 4 kg + (0..3) of tile m
+            const f32x4 da4 = *reinterpret_cast<const f32x4 *>(s_da + bl * SD + 32 * m + 8 * rq + 4 * kg);    // tokens 8 rq + 4 kg + (0..3) of tile m
 #pragma unroll
             for (int rp = 0; rp < 2; rp++) {
                 const f32x2 da2 = {da4[2 * rp], da4[2 * rp + 1]};
@@ -79,44 +82,63 @@ __global__ __launch_bounds__(256) void mmq_q80_kernel(const uint8_t *__restrict_
             }
         }
     };
+    // The codes of a group of four blocks - a 128-byte line of every row - are requested a step ahead: the weights of the next group at the start of a group, the
+    // activations of the next token tile (of the next group's first) before a tile's products.  Two register sets, chosen at compile time: groups come in pairs.
+    const int ng = nb / Q80_UNROLL;
+    i32x4 w[2][Q80_UNROLL], av[2][Q80_UNROLL];
+    u32x2 dh[2];
+    auto ask_w = [&](int g, int s) {
+        const int gc = g < ng ? g : ng - 1;                            // (past the end: the last group again)
+#pragma unroll
+        for (int u = 0; u < Q80_UNROLL; u++) w[s][u] = *reinterpret_cast<const i32x4 *>(wrow + (size_t)(gc * Q80_UNROLL + u) * 32);
+        dh[s] = *reinterpret_cast<const u32x2 *>(wd + gc * Q80_UNROLL);
+    };
+    auto ask_a = [&](int g, int m, int s) {
+        const int gc = g < ng ? g : ng - 1;
+#pragma unroll
+        for (int u = 0; u < Q80_UNROLL; u++) av[s][u] = *reinterpret_cast<const i32x4 *>(arow[m] + (size_t)(gc * Q80_UNROLL + u) * 32);
+    };
+    if (rows_ok && ng > 0) { ask_w(0, 0); ask_a(0, 0, 0); }
+    auto group = [&](auto par, int g, int bl) {                        // par: parity of the group in its chunk (a chunk is an even number of groups, all but the last)
+        constexpr int P = decltype(par)::value;
+        ask_w(g + 1, P ^ 1);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            constexpr int FLIP = MT == 1 ? P : 0;
+            const int s = FLIP ^ (m & 1);
+            if (m + 1 < MT) ask_a(g, m + 1, s ^ 1); else ask_a(g + 1, 0, s ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < Q80_UNROLL; u++) {
+                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s][u], w[P][u], z, 0, 0, 0);
+                fold(c, h2f((uint16_t)(dh[P][u >> 1] >> (16 * (u & 1)))), bl + u, m);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
     for (int b0 = 0; b0 < nb; b0 += Q80_KC) {
         const int nbc = nb - b0 < Q80_KC ? nb - b0 : Q80_KC;
         __syncthreads();                                               // everyone is done with the previous chunk's scales
-        for (int i = tid; i < nbc * TT; i += 256) {
-            const int b = i / TT, m = i - b * TT;
+        for (int i = tid; i < Q80_KC * TT; i += 256) {                 // (lanes along a token's scales)
+            const int m = i / Q80_KC, b = i - m * Q80_KC;
             const int t = t0 + m < T ? t0 + m : T - 1;
-            s_da[i] = h2f(ad[(size_t)t * nb + b0 + b]);
+            if (b < nbc) s_da[b * SD + m] = h2f(ad[(size_t)t * nb + b0 + b]);
         }
         __syncthreads();
         if (!rows_ok) continue;
         int b = 0;
-        for (; b + Q80_UNROLL <= nbc; b += Q80_UNROLL) {               // the loads of a group are issued before its first MFMA
-            i32x4 w[Q80_UNROLL];
-            uint16_t dh[Q80_UNROLL];
-#pragma unroll
-            for (int u = 0; u < Q80_UNROLL; u++) {
-                w[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(wrow + (size_t)(b0 + b + u) * 32));
-                dh[u] = wd[b0 + b + u];
-            }
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-                i32x4 a[Q80_UNROLL];
-#pragma unroll
-                for (int u = 0; u < Q80_UNROLL; u++) a[u] = *reinterpret_cast<const i32x4 *>(arow[m] + (size_t)(b0 + b + u) * 32);
-#pragma unroll
-                for (int u = 0; u < Q80_UNROLL; u++) {
-                    const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u], w[u], z, 0, 0, 0);
-                    fold(c, h2f(dh[u]), b + u, m);
-                }
-            }
+        for (; b + 2 * Q80_UNROLL <= nbc; b += 2 * Q80_UNROLL) {
+            group(std::integral_constant<int, 0>{}, (b0 + b) / Q80_UNROLL, b);
+            group(std::integral_constant<int, 1>{}, (b0 + b) / Q80_UNROLL + 1, b + Q80_UNROLL);
         }
+        if (b + Q80_UNROLL <= nbc) { group(std::integral_constant<int, 0>{}, (b0 + b) / Q80_UNROLL, b); b += Q80_UNROLL; }
         for (; b < nbc; b++) {
-            const i32x4 w = *reinterpret_cast<const i32x4 *>(wrow + (size_t)(b0 + b) * 32);
+            const i32x4 w1 = *reinterpret_cast<const i32x4 *>(wrow + (size_t)(b0 + b) * 32);
             const float dw = h2f(wd[b0 + b]);
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 const i32x4 a = *reinterpret_cast<const i32x4 *>(arow[m] + (size_t)(b0 + b) * 32);
-                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w, z, 0, 0, 0);
+                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w1, z, 0, 0, 0);
                 fold(c, dw, b, m);
             }
         }
