@@ -9,6 +9,8 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include <type_traits>
+
 #include "kernels.h"
 #include "quant_dev.h"
 
@@ -65,15 +67,17 @@ __global__ __launch_bounds__(256) void norm_quant_kernel(const float *__restrict
 // do_norm: the row's sum of squares must come out with the bits of the kernel above (whose thread tid adds the squares of float4 tid, tid + 256, tid + 512 ..
 // to ONE double, element by element): every thread leaves its products in LDS and the first 256 threads add them up in exactly that order, then the same wave sums
 // and the same four partial sums.  grid = (rows, parts): a part is 16 blocks of the row; do_norm needs the whole row in one workgroup (n <= 16 * 256 * NV).
-template <int NV>
-__global__ __launch_bounds__(1024) void norm_quant_wide_kernel(const float *__restrict__ x, const float *__restrict__ w, int n, float eps, int do_norm,
+// PARTS (do_norm): the n_part partial sums of a K-split product ([part][row][n]) are added to the row on the way in, x = x + ((part 0 + part 1) + (part 2 + part 3)), what
+// the reduction pass of that product (mmq.hip) does otherwise.  512 x 4096, four parts: 9.1 + 6.4 us as two launches, 11.7 as this one (52 MB at the rate of a large copy: 10)
+template <int NV, bool PARTS = false>
+__global__ __launch_bounds__(1024) void norm_quant_wide_kernel(std::conditional_t<PARTS, float *, const float *__restrict__> x, const float *__restrict__ part, int n_part, const float *__restrict__ w, int n, float eps, int do_norm,
                                                                 float *__restrict__ yf, ActQuant q, int want_q8k, int want_q80, int8_t *__restrict__ bh, int8_t *__restrict__ bl) {
     extern __shared__ float prod[];                       // do_norm: [n] squares, float4 index major
     __shared__ double red[4];
     __shared__ float s_scale;
     const int row = blockIdx.x, u = threadIdx.x, lane = u & 63, wave = u >> 6, nw = blockDim.x >> 6;
     const int nblk = n >> 8;
-    const float *xr = x + (size_t)row * n;
+    auto *xr = x + (size_t)row * n;
     float4 v[NV];
     int blk[NV];
 #pragma unroll
@@ -81,6 +85,19 @@ __global__ __launch_bounds__(1024) void norm_quant_wide_kernel(const float *__re
         blk[j] = (do_norm ? 0 : blockIdx.y * 16 * NV) + wave + nw * j;
         const int bc = blk[j] < nblk ? blk[j] : nblk - 1;
         v[j] = *reinterpret_cast<const float4 *>(xr + bc * 256 + lane * 4);
+        if constexpr (PARTS) {
+            const size_t stride = (size_t)gridDim.x * n;
+            const float *p = part + (size_t)row * n + bc * 256 + lane * 4;
+            float4 pv[4];                                    // (at most four parts; all requested before the first add)
+#pragma unroll
+            for (int z = 0; z < 4; z++) pv[z] = *reinterpret_cast<const float4 *>(p + (z < n_part ? z : 0) * stride);
+            auto add = [](float4 &a, const float4 &b) { a.x = a.x + b.x; a.y = a.y + b.y; a.z = a.z + b.z; a.w = a.w + b.w; };
+            if (n_part > 3) add(pv[2], pv[3]);
+            add(pv[0], pv[1]);
+            if (n_part > 2) add(pv[0], pv[2]);
+            add(v[j], pv[0]);
+            if (blk[j] < nblk) *reinterpret_cast<float4 *>(xr + blk[j] * 256 + lane * 4) = v[j];
+        }
     }
     float scale = 1.0f;
     if (do_norm) {
@@ -132,20 +149,29 @@ __global__ __launch_bounds__(1024) void norm_quant_wide_kernel(const float *__re
     }
 }
 // true: launched.  Rows of a prompt batch only (T >= 32); with the norm the row must fit one workgroup
-static bool launch_wide(const float *x, const float *w, int n, int T, float eps, int do_norm, float *yf, const ActQuant &qq, int k, int z, int8_t *bh, int8_t *bl, hipStream_t st) {
+static bool wide_ok(int n, int T, int do_norm) {
     static const bool off = getenv("MI355_QUANT_WIDE") && getenv("MI355_QUANT_WIDE")[0] == '0';
     const int nblk = n >> 8;
-    if (off || T < 32 || (n & 255) || nblk < 1) return false;
+    return !(off || T < 32 || (n & 255) || nblk < 1) && !(do_norm && (nblk > 32 || (n & 1023)));
+}
+bool rmsnorm_takes_parts(int n, int T) { return wide_ok(n, T, 1); }
+static bool launch_wide(const float *x, const float *w, int n, int T, float eps, int do_norm, float *yf, const ActQuant &qq, int k, int z, int8_t *bh, int8_t *bl, hipStream_t st,
+                        float *x_rw = nullptr, const float *part = nullptr, int n_part = 1) {
+    const int nblk = n >> 8;
+    if (!wide_ok(n, T, do_norm)) return false;
     if (do_norm) {
-        if (nblk > 32 || (n & 1023)) return false;
         const int nv = nblk > 16 ? 2 : 1, nwv = (nblk + nv - 1) / nv;
         const size_t lds = (size_t)n * sizeof(float);
-        if (nv == 1) hipLaunchKernelGGL(norm_quant_wide_kernel<1>, dim3(T, 1), dim3(64 * nwv), lds, st, x, w, n, eps, 1, yf, qq, k, z, bh, bl);
-        else hipLaunchKernelGGL(norm_quant_wide_kernel<2>, dim3(T, 1), dim3(64 * nwv), lds, st, x, w, n, eps, 1, yf, qq, k, z, bh, bl);
+        if (n_part > 1) {
+            if (nv == 1) hipLaunchKernelGGL((norm_quant_wide_kernel<1, true>), dim3(T, 1), dim3(64 * nwv), lds, st, x_rw, part, n_part, w, n, eps, 1, yf, qq, k, z, bh, bl);
+            else hipLaunchKernelGGL((norm_quant_wide_kernel<2, true>), dim3(T, 1), dim3(64 * nwv), lds, st, x_rw, part, n_part, w, n, eps, 1, yf, qq, k, z, bh, bl);
+        } else
+        if (nv == 1) hipLaunchKernelGGL((norm_quant_wide_kernel<1>), dim3(T, 1), dim3(64 * nwv), lds, st, x, part, 1, w, n, eps, 1, yf, qq, k, z, bh, bl);
+        else hipLaunchKernelGGL((norm_quant_wide_kernel<2>), dim3(T, 1), dim3(64 * nwv), lds, st, x, part, 1, w, n, eps, 1, yf, qq, k, z, bh, bl);
         return true;
     }
     const int parts = (nblk + 15) / 16, nwv = nblk < 16 ? nblk : 16;
-    hipLaunchKernelGGL(norm_quant_wide_kernel<1>, dim3(T, parts), dim3(64 * nwv), 0, st, x, w, n, eps, 0, yf, qq, k, z, bh, bl);
+    hipLaunchKernelGGL((norm_quant_wide_kernel<1>), dim3(T, parts), dim3(64 * nwv), 0, st, x, (const float *)nullptr, 1, w, n, eps, 0, yf, qq, k, z, bh, bl);
     return true;
 }
 
@@ -163,12 +189,13 @@ static int quant_splits(int T, int n) {
     return s < 1 ? 1 : s;
 }
 
-hipError_t launch_rmsnorm_quant(const float *x, const float *w, int n, int T, float eps, float *y_f32,
-                                const ActQuant *q, bool want_q8k, bool want_q80, hipStream_t st, int8_t *bh, int8_t *bl) {
+hipError_t launch_rmsnorm_quant(float *x, const float *w, int n, int T, float eps, float *y_f32,
+                                const ActQuant *q, bool want_q8k, bool want_q80, hipStream_t st, int8_t *bh, int8_t *bl, const float *part, int n_part) {
+    if (n_part > 4 || (n_part > 1 && (!part || !rmsnorm_takes_parts(n, T)))) return hipErrorInvalidValue;
     const ActQuant qq = act_for(q, T);
-    if (launch_wide(x, w, n, T, eps, 1, y_f32, qq, (int)(q && want_q8k), (int)(q && want_q80), (q && want_q8k) ? bh : nullptr, bl, st)) return hipGetLastError();
+    if (launch_wide(x, w, n, T, eps, 1, y_f32, qq, (int)(q && want_q8k), (int)(q && want_q80), (q && want_q8k) ? bh : nullptr, bl, st, x, part, n_part)) return hipGetLastError();
     const int splits = quant_splits(T, n);
-    hipLaunchKernelGGL(norm_quant_kernel, dim3(T, splits), dim3(256), 0, st, x, w, n, eps, 1, y_f32, qq,
+    hipLaunchKernelGGL(norm_quant_kernel, dim3(T, splits), dim3(256), 0, st, (const float *)x, w, n, eps, 1, y_f32, qq,
                        (int)(q && want_q8k), (int)(q && want_q80), (q && want_q8k) ? bh : nullptr, bl);
     return hipGetLastError();
 }

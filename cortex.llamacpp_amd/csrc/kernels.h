@@ -146,7 +146,8 @@ hipError_t launch_mmq_planes_swiglu_moe(int type, const uint8_t *planes_gate, co
 hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_stride, int n_expert, const int32_t *meta, int n_rows, int K, int rows_max,
                                  const ActQuant &q, float *out, int ld_out, hipStream_t st);
 hipError_t launch_mmq_planes(int type, const uint8_t *planes, int n_rows, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
-                             float *out, int ld_out, const float *resid, hipStream_t st, MMQWorkspace wsp = MMQWorkspace());
+                             float *out, int ld_out, const float *resid, hipStream_t st, MMQWorkspace wsp = MMQWorkspace(), int *parts = nullptr);
+// parts (nullable): a launch that splits K leaves its partial sums in the workspace ([part][T][n_rows]; `out` untouched) and their number here
 // small batches (continuous-batching decode steps, 8 <= T <= 64): K split over the waves of a workgroup, GGUF-form weights
 struct MMQSeg {
     const uint8_t *W; size_t row_bytes; int n_rows, type;
@@ -161,7 +162,7 @@ hipError_t launch_mmq_q80(const uint8_t *W, size_t row_bytes, int n_rows, int K,
 // launch over the concatenated rows; seg_rows[i] rows go to outs[i] (leading dimension lds_out[i])
 hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *seg_rows, float *const *outs, const int *lds_out, int n_seg, int K, int T,
                                    const ActQuant &q, const int8_t *bh, const int8_t *bl, const float *resid, hipStream_t st,
-                                   MMQWorkspace wsp = MMQWorkspace(), const int *seg_types = nullptr);
+                                   MMQWorkspace wsp = MMQWorkspace(), const int *seg_types = nullptr, int *parts = nullptr);
 // seg_types (per segment; nullptr = all `type`): Q4_K / Q5_K segments beside Q6_K ones in ONE launch where this says so (segments end on
 // 128-row tiles and the launch takes the 128 x 256 kernel)
 bool mmq_planes_mixed_ok(const int *seg_rows, int n_seg, int K, int T, MMQWorkspace wsp);
@@ -186,9 +187,12 @@ hipError_t launch_mmq(int type, const uint8_t *W, size_t row_bytes, int n_rows, 
 // y = rms_norm(x) * w  for T rows of n; optionally f32 out and/or q8_K / q8_0 planes
 // bh / bl (optional, with q8_K): also write the block sums split into the int8 planes the MFMA kernels contract
 // (bsum = 64 * bh + bl, what launch_mmq_prep computes as its own launch), [T][n / 16] each
-hipError_t launch_rmsnorm_quant(const float *x, const float *w, int n, int T, float eps,
+// part / n_part (n_part > 1; rmsnorm_takes_parts): x is the residual of a K-split product whose partial sums part[0 .. n_part)[T][n] are still to be added to it:
+// x += (part 0 + part 1) + (part 2 + part 3) on the way in, written back
+bool rmsnorm_takes_parts(int n, int T);
+hipError_t launch_rmsnorm_quant(float *x, const float *w, int n, int T, float eps,
                                 float *y_f32 /*nullable*/, const ActQuant *q /*nullable*/, bool want_q8k, bool want_q80,
-                                hipStream_t st, int8_t *bh = nullptr, int8_t *bl = nullptr);
+                                hipStream_t st, int8_t *bh = nullptr, int8_t *bl = nullptr, const float *part = nullptr, int n_part = 1);
 // quantise f32 rows
 hipError_t launch_quantize(const float *x, int n, int T, const ActQuant &q, bool want_q8k, bool want_q80, hipStream_t st,
                            int8_t *bh = nullptr, int8_t *bl = nullptr);

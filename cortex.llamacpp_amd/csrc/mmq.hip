@@ -1410,17 +1410,19 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t
                                      aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 
-// out[t][row] = (resid) + ws[0][t][row] + ws[1][t][row] + ... in split order (fixed, so results do not depend on timing)
+// out[t][row] = (resid) + ((part 0 + part 1) + (part 2 + part 3)) of ws[part][t][row] (a fixed order, so results do not depend on timing)
 __global__ __launch_bounds__(256) void mmq_splitk_reduce_kernel(const float *ws, int n_split, int T, int n_rows, const PlanesOut po, const float *resid) {
     const size_t i4 = (size_t)blockIdx.x * 256 + threadIdx.x, per_tok = (size_t)n_rows >> 2;      // n_rows % 4 == 0 (launcher)
     if (i4 >= per_tok * T) return;
     const int t = (int)(i4 / per_tok), row = (int)(i4 % per_tok) * 4;
     const size_t plane = (size_t)T * n_rows, at = (size_t)t * n_rows + row;
-    f32x4 acc = *reinterpret_cast<const f32x4 *>(ws + at);
-    for (int z = 1; z < n_split; z++) {
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(ws + z * plane + at);
-        acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-    }
+    f32x4 v[4];                                                // (at most four parts; all requested before the first add)
+#pragma unroll
+    for (int z = 0; z < 4; z++) v[z] = *reinterpret_cast<const f32x4 *>(ws + (size_t)(z < n_split ? z : 0) * plane + at);
+    f32x4 acc = v[0];
+    if (n_split > 3) v[2] = v[2] + v[3];
+    if (n_split > 1) acc = acc + v[1];
+    if (n_split > 2) acc = acc + v[2];
     int sg = 0;
     if (po.n_seg > 1 && row >= po.row_end[0]) sg = 1;
     if (po.n_seg > 2 && row >= po.row_end[1]) sg = 2;
@@ -1569,8 +1571,8 @@ hipError_t launch_mmq_expand(int type, const uint8_t *W, size_t row_bytes, int n
 }
 
 hipError_t launch_mmq_planes(int type, const uint8_t *planes, int n_rows, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
-                             float *out, int ld_out, const float *resid, hipStream_t st, MMQWorkspace wsp) {
-    return launch_mmq_planes_multi(type, planes, &n_rows, &out, &ld_out, 1, K, T, q, bh, bl, resid, st, wsp, nullptr);
+                             float *out, int ld_out, const float *resid, hipStream_t st, MMQWorkspace wsp, int *parts) {
+    return launch_mmq_planes_multi(type, planes, &n_rows, &out, &ld_out, 1, K, T, q, bh, bl, resid, st, wsp, nullptr, parts);
 }
 
 // the K split the 128 x 256 kernel would run a tensor (or concatenation) of n_rows rows with, and whether it takes the launch at all
@@ -1588,7 +1590,7 @@ static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool
     int n_split = 1;
     if (g_mmq_split > 1 || env_sk > 1) n_split = g_mmq_split > 1 ? g_mmq_split : env_sk;
     else if (env_sk != 0 && g_mmq_split != 1) n_split = (int)std::max(1L, std::min({num_cu() / wg, 4L, (long)nb / 4}));
-    if (n_split > nb) n_split = nb;
+    n_split = std::min({n_split, nb, 4});                       // (the reductions add four parts at most)
     if (n_split < 1 || (n_rows % 4) != 0 || !wsp.p || (size_t)n_split * T * n_rows * sizeof(float) > wsp.bytes) n_split = 1;
     // (an unsplit launch wants a third of the CUs: 11264 x 2048 at 160 and 256 tokens - 88 workgroups - 35 and 40 us against 31 and 56, 4096 x 4096 at 300 - 64 - 53 against 47)
     *takes = g_mmq_mt == 4 || (g_mmq_mt == 0 && env_mt == 0 && env_p2 != 0 && T > 128 && (n_split > 1 || wg * 3 >= num_cu()));
@@ -1674,7 +1676,7 @@ hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_s
 
 hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *seg_rows, float *const *outs, const int *lds_out, int n_seg, int K, int T,
                                    const ActQuant &q, const int8_t *bh, const int8_t *bl, const float *resid, hipStream_t st, MMQWorkspace wsp,
-                                   const int *seg_types) {
+                                   const int *seg_types, int *parts) {
     if (n_seg < 1 || n_seg > 3 || (n_seg > 1 && resid)) return hipErrorInvalidValue;
     PlanesOut po{};
     po.n_seg = n_seg;
@@ -1716,7 +1718,8 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
             (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
             hipLaunchKernelGGL((mmq_planes2_kernel<false>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split);
         }
-        if (n_split > 1) {
+        if (n_split > 1 && parts) *parts = n_split;
+        else if (n_split > 1) {
             const size_t n4 = (size_t)T * (n_rows >> 2);
             hipLaunchKernelGGL(mmq_splitk_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, wsp.p, n_split, T, n_rows, po, resid);
         }

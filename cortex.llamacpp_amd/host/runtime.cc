@@ -989,7 +989,7 @@ static bool q80_copy(const DevTensor &w, int K, int T) {
 static bool planes_small(const DevTensor &w, int K, int T) { return (w.type == T_Q2_K || w.type == T_Q3_K) && w.planes && T >= 32 && (K % 256) == 0; }
 
 hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *x_f32, int K, int T, float *out, int ld_out,
-                           const float *resid, int epi) {
+                           const float *resid, int epi, int *parts) {
     if (is_quant(w.type)) {
         if (mmq_q80_applicable(w.type, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU && aq.qs0)   // prompt processing, Q8_0 weights
             return launch_mmq_q80(w.data, w.row_bytes, (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
@@ -1001,7 +1001,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
         }
         if (mmq_applicable(w.type, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // prompt processing: MFMA path
             if ((w.type != T_Q6_K || !w.planes) && !bh_over_) HIP_TRY(ensure_prep(aq, K, T));
-            if (w.planes) return launch_mmq_planes(w.type, w.planes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_, mmq_ws_);
+            if (w.planes) return launch_mmq_planes(w.type, w.planes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_, mmq_ws_, parts);
             return launch_mmq(w.type, w.data, w.row_bytes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         }
         if (q80_copy(w, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU && aq.qs0)      // prompt processing of Q4_0 / Q5_0 / IQ4_NL tensors: their exact Q8_0-layout copy
@@ -1458,6 +1458,9 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                                   att_counters_, d_mega_sync_, h_mega_flag_, d_mega_probe_, mega_lds_, stream_);
 
     const bool tp = hp.tp_exchange;
+    // a prompt's K-split attn_output / ffn_down leaves its partial sums to the norm that reads x_ next (x_parts of them in mmq_ws_; x_ holds the residual till then)
+    const bool late_sum = rmsnorm_takes_parts(E, T) && !tp;
+    int x_parts = 1;
     for (int il = 0; il < hp.n_layer; il++) {
         const LayerWeights &L = model->layers[(size_t)il];
         // --- attention block
@@ -1529,7 +1532,8 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         } else {
             const bool pl = need_k && T >= 3;                  // the batched kernels will want the block-sum planes
             HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.attn_norm.data, E, T, hp.eps, any_f ? xn_ : nullptr, &aq_e_, need_k, need_0, stream_,
-                                         pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
+                                         pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr, mmq_ws_.p, x_parts));
+            x_parts = 1;
             prep_owner_ = nullptr;
             if (pl) prep_written(aq_e_, E, T);
             prof_mark("norm_quant");
@@ -1592,14 +1596,15 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, tp_part_, E, hp.tp_rank == 0 ? x_ : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
             HIP_TRY(tp_reduce_into_x(T));
         } else {
-            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, x_, E, x_, EPI_ADD));
+            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, x_, E, x_, EPI_ADD, late_sum ? &x_parts : nullptr));
         }
         prof_mark("attn_out");
 
         // --- feed-forward block
         if (hp.n_expert > 0) {
             HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, xn_, &aq_e_,
-                                         !act_is_q80(L.gate_exps.type) || !act_is_q80(L.up_exps.type), act_is_q80(L.gate_exps.type) || act_is_q80(L.up_exps.type), stream_));
+                                         !act_is_q80(L.gate_exps.type) || !act_is_q80(L.up_exps.type), act_is_q80(L.gate_exps.type) || act_is_q80(L.up_exps.type), stream_, nullptr, nullptr, mmq_ws_.p, x_parts));
+            x_parts = 1;
             prep_owner_ = nullptr;
             prof_mark("norm_quant");
             if (L.gate_inp.type == T_F32 || L.gate_inp.type == T_F16) {
@@ -1749,7 +1754,8 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             } else {
                 const bool pl = fk && T >= 3;
                 HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, (!gq || !uq) ? xn_ : nullptr, &aq_e_, fk, f0, stream_,
-                                             pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
+                                             pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr, mmq_ws_.p, x_parts));
+                x_parts = 1;
                 prep_owner_ = nullptr;
                 if (pl) prep_written(aq_e_, E, T);
                 prof_mark("norm_quant");
@@ -1841,7 +1847,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 pending_fuse_ = Fuse();
                 HIP_TRY(tp_reduce_into_x(T));
             } else {
-                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, T, x_, E, x_, EPI_ADD));
+                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, T, x_, E, x_, EPI_ADD, late_sum && il + 1 < hp.n_layer && !(debug_taps_ && dbg_) ? &x_parts : nullptr));
             }
             pending_fuse_ = Fuse();
             prof_mark("ffn_down");

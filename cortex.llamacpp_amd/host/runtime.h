@@ -230,7 +230,7 @@ class Context {
     std::vector<std::pair<int, int>> nvx_waves_;            // segment ranges [first, count) that may share a launch (no slot twice)
     hipError_t run_output(int n_out, int out_base);
     hipError_t linear(const DevTensor &w, const ActQuant &aq, const float *x_f32, int K, int T, float *out, int ld_out,
-                      const float *resid, int epi);
+                      const float *resid, int epi, int *parts = nullptr);     // parts: as launch_mmq_planes's (the partial sums are left in mmq_ws_)
     hipError_t linear_multi(const DevTensor *const *ws, float *const *outs, int n, const ActQuant &aq, const float *x_f32, int T);
     void prof_mark(const char *name);
     void prof_begin();
