@@ -614,16 +614,34 @@ __global__ __launch_bounds__(256) void kv_store_fast_kernel(const float *k, cons
 // Prompt batches: the same K / V part (grid row y >= q_parts) plus the rotation of q in place (rows y < q_parts, 1024 elements of the
 // token's H * D each), four consecutive elements = two rope pairs per thread.  Same arithmetic as rope_kv_store_kernel (one workgroup per
 // token, one element per thread and pass, byte stores into a q8_0 cache: 14 us per layer at 512 tokens against 6).
-template <int TK, int TV>
+// PARTS: q | k | v come as the n_part partial sums of a K-split product, part[z][t][HD + 2 GD], added here as that product's own reduction adds them
+// ((0 + 1) + (2 + 3)); q is written whole, k and v only into the cache.  512 tokens, 4096 + 2 x 1024 columns, two parts: 8.3 + 8.3 us as two launches, 10.1 as this one
+template <int TK, int TV, bool PARTS = false>
 __global__ __launch_bounds__(256) void rope_q_kv_store_fast_kernel(float *q, int HD, int q_parts, const float *k, const float *v, int GD, int D,
-                                                                   const float *cs_table, int n_rot, const int32_t *tok_cell, KVLayerView kv, int n_ctx) {
+                                                                   const float *cs_table, int n_rot, const int32_t *tok_cell, KVLayerView kv, int n_ctx,
+                                                                   const float *psum, int n_part) {
     const int t = blockIdx.x, part = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    auto total = [&](int col) {                                  // column col of the token's summed row
+        const int N = HD + 2 * GD;
+        const size_t stride = (size_t)gridDim.x * N;
+        const float *p = psum + (size_t)t * N + col;
+        float4 pv[4];
+#pragma unroll
+        for (int z = 0; z < 4; z++) pv[z] = *reinterpret_cast<const float4 *>(p + (z < n_part ? z : 0) * stride);
+        auto add = [](float4 &a, const float4 &b) { a.x = a.x + b.x; a.y = a.y + b.y; a.z = a.z + b.z; a.w = a.w + b.w; };
+        if (n_part > 3) add(pv[2], pv[3]);
+        if (n_part > 1) add(pv[0], pv[1]);
+        if (n_part > 2) add(pv[0], pv[2]);
+        return pv[0];
+    };
     if (part < q_parts) {
         const int e0 = part * 1024 + tid * 4;
         const int dd = e0 % D;
+        float4 *qp = reinterpret_cast<float4 *>(q + (size_t)t * HD + e0);
+        float4 x;
+        if constexpr (PARTS) { x = total(e0); if (dd >= n_rot) *qp = x; }
         if (dd < n_rot) {
-            float4 *qp = reinterpret_cast<float4 *>(q + (size_t)t * HD + e0);
-            float4 x = *qp;
+            if constexpr (!PARTS) x = *qp;
             const float4 cs = *reinterpret_cast<const float4 *>(cs_table + (size_t)t * n_rot + dd);   // c0 s0 c1 s1
             const float x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
             x.x = x0 * cs.x - x1 * cs.y; x.y = x0 * cs.y + x1 * cs.x;
@@ -635,8 +653,9 @@ __global__ __launch_bounds__(256) void rope_q_kv_store_fast_kernel(float *q, int
     const int cell = tok_cell[t];
     {
         const int e0 = (part - q_parts) * 1024 + tid * 4;
-        float4 kk = *reinterpret_cast<const float4 *>(k + (size_t)t * GD + e0);
-        const float4 vv4 = *reinterpret_cast<const float4 *>(v + (size_t)t * GD + e0);
+        float4 kk, vv4;
+        if constexpr (PARTS) { kk = total(HD + e0); vv4 = total(HD + GD + e0); }
+        else { kk = *reinterpret_cast<const float4 *>(k + (size_t)t * GD + e0); vv4 = *reinterpret_cast<const float4 *>(v + (size_t)t * GD + e0); }
         const int g = e0 / D, dd = e0 - g * D;
         if (dd < n_rot) {
             const float4 cs = *reinterpret_cast<const float4 *>(cs_table + (size_t)t * n_rot + dd);   // c0 s0 c1 s1
@@ -671,11 +690,13 @@ bool rope_q_kv_store_fast_applicable(int H, int G, int D, int type_k, int type_v
     return kv_store_fast_applicable(G, D, type_k, type_v, ra) && (H * D) % 1024 == 0 && D % 4 == 0;
 }
 hipError_t launch_rope_q_kv_store_fast(float *q, const float *k, const float *v, int T, int H, int G, int D, const float *cs_table, RopeArgs ra,
-                                       const int32_t *tok_cell, KVLayerView kv, int type_k, int type_v, int n_ctx, hipStream_t st) {
+                                       const int32_t *tok_cell, KVLayerView kv, int type_k, int type_v, int n_ctx, hipStream_t st, const float *psum, int n_part) {
+    if (n_part > 4 || (n_part > 1 && !psum)) return hipErrorInvalidValue;
     if (!cs_table || !rope_q_kv_store_fast_applicable(H, G, D, type_k, type_v, ra)) return hipErrorInvalidValue;
     const int q_parts = H * D / 1024, kv_parts = G * D / 1024;
     const dim3 grid((unsigned)T, (unsigned)(q_parts + kv_parts));
-#define RKS(TK, TV) hipLaunchKernelGGL((rope_q_kv_store_fast_kernel<TK, TV>), grid, dim3(256), 0, st, q, H * D, q_parts, k, v, G * D, D, cs_table, ra.n_rot, tok_cell, kv, n_ctx)
+#define RKS(TK, TV) do { if (n_part > 1) hipLaunchKernelGGL((rope_q_kv_store_fast_kernel<TK, TV, true>), grid, dim3(256), 0, st, q, H * D, q_parts, k, v, G * D, D, cs_table, ra.n_rot, tok_cell, kv, n_ctx, psum, n_part); \
+                         else hipLaunchKernelGGL((rope_q_kv_store_fast_kernel<TK, TV>), grid, dim3(256), 0, st, q, H * D, q_parts, k, v, G * D, D, cs_table, ra.n_rot, tok_cell, kv, n_ctx, psum, 1); } while (0)
     if (type_k == T_F16 && type_v == T_F16) RKS(T_F16, T_F16);
     else if (type_k == T_Q8_0 && type_v == T_Q8_0) RKS(T_Q8_0, T_Q8_0);
     else if (type_k == T_Q8_0 && type_v == T_F16) RKS(T_Q8_0, T_F16);

@@ -1019,7 +1019,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
     return launch_mmv_float(w.type, w.data, (int)w.N, K, x_f32, T, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
 }
 
-hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs, int n, const ActQuant &aq, const float *x_f32, int T) {
+hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs, int n, const ActQuant &aq, const float *x_f32, int T, int *parts) {
     bool all_q = true;
     for (int i = 0; i < n; i++) all_q &= is_quant(ws[i]->type);
     const int K = (int)ws[0]->K;
@@ -1055,7 +1055,7 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
             int rows[3], ldo[3], types[3];
             float *o[3];
             for (int i = 0; i < nf; i++) { rows[i] = (int)ws[i]->N; ldo[i] = (int)ws[i]->N; o[i] = outs[i]; types[i] = ws[i]->type; }
-            HIP_TRY(launch_mmq_planes_multi(ws[0]->type, ws[0]->planes, rows, o, ldo, nf, K, T, aq, mmq_bh_, mmq_bl_, nullptr, stream_, mmq_ws_, types));
+            HIP_TRY(launch_mmq_planes_multi(ws[0]->type, ws[0]->planes, rows, o, ldo, nf, K, T, aq, mmq_bh_, mmq_bl_, nullptr, stream_, mmq_ws_, types, nf == n ? parts : nullptr));
         } else nf = 0;
         for (int i = nf; i < n; i++) {
             if (ws[i]->planes) HIP_TRY(launch_mmq_planes(ws[i]->type, ws[i]->planes, (int)ws[i]->N, K, T, aq, mmq_bh_, mmq_bl_, outs[i], (int)ws[i]->N, nullptr, stream_, mmq_ws_));
@@ -1540,7 +1540,12 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         }
         const DevTensor *ws[3] = {&L.wq, &L.wk, &L.wv};
         float *outs[3] = {q_, k_, v_};
-        if (!(engine && il > 0) && !qkv_in_attn) HIP_TRY(linear_multi(ws, outs, 3, aq_e_, xn_, T));
+        // a prompt's K-split Q | K | V leaves its partial sums to the rope + cache store (qkv_parts of them in mmq_ws_)
+        static const bool rope_fast = !(getenv("MI355_ROPE_FAST") && getenv("MI355_ROPE_FAST")[0] == '0');
+        const bool rope_fast_ok = rope_fast && g_rope_fast && rope_cs_ && rope_q_kv_store_fast_applicable(H, G, D, cp.type_k, cp.type_v, ra);
+        int qkv_parts = 1;
+        if (!(engine && il > 0) && !qkv_in_attn)
+            HIP_TRY(linear_multi(ws, outs, 3, aq_e_, xn_, T, rope_fast_ok && !decode_attn && !(L.bq.valid() || L.bk.valid() || L.bv.valid()) ? &qkv_parts : nullptr));
         pending_fuse_ = Fuse();
         if (!qkv_in_attn && (L.bq.valid() || L.bk.valid() || L.bv.valid()))       // qwen2-style attention biases: all T rows of the three projections in one launch
             HIP_TRY(launch_add_qkv_bias(q_, k_, v_, L.bq.valid() ? (const float *)L.bq.data : nullptr, L.bk.valid() ? (const float *)L.bk.data : nullptr,
@@ -1569,9 +1574,8 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 HIP_TRY(launch_flash_attn_decode(aa, rope_cs_, ra, stream_));
             }
         } else {
-            static const bool rope_fast = !(getenv("MI355_ROPE_FAST") && getenv("MI355_ROPE_FAST")[0] == '0');
-            if (rope_fast && g_rope_fast && rope_cs_ && rope_q_kv_store_fast_applicable(H, G, D, cp.type_k, cp.type_v, ra))
-                HIP_TRY(launch_rope_q_kv_store_fast(q_, k_, v_, T, H, G, D, rope_cs_, ra, d_cell_, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, stream_));
+            if (rope_fast_ok)
+                HIP_TRY(launch_rope_q_kv_store_fast(q_, k_, v_, T, H, G, D, rope_cs_, ra, d_cell_, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, stream_, mmq_ws_.p, qkv_parts));
             else
                 HIP_TRY(launch_rope_kv_store(q_, k_, v_, T, H, G, D, d_pos_, d_cell_, ra, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, rope_cs_, stream_));
             prof_mark("rope_kv");

@@ -231,7 +231,7 @@ class Context {
     hipError_t run_output(int n_out, int out_base);
     hipError_t linear(const DevTensor &w, const ActQuant &aq, const float *x_f32, int K, int T, float *out, int ld_out,
                       const float *resid, int epi, int *parts = nullptr);     // parts: as launch_mmq_planes's (the partial sums are left in mmq_ws_)
-    hipError_t linear_multi(const DevTensor *const *ws, float *const *outs, int n, const ActQuant &aq, const float *x_f32, int T);
+    hipError_t linear_multi(const DevTensor *const *ws, float *const *outs, int n, const ActQuant &aq, const float *x_f32, int T, int *parts = nullptr);
     void prof_mark(const char *name);
     void prof_begin();
     void prof_end();
