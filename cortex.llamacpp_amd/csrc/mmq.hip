@@ -1365,7 +1365,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_kernel(const uint
     planes2_body<MINS, true>(P2Args{planes_gate, planes_up, n_rows, K, T, aq, ad, absum, nullptr, nullptr, 1}, po, row_tile, tok_tile, n_tok_tiles, 0);
 }
 
-// ---- ggml_mul_mat_id on a prompt batch as ONE launch per projection (round 5).  The (token, rank) pairs of the batch are sorted by expert (moe_group_kernel: expert
+// ---- ggml_mul_mat_id on a prompt batch as ONE launch per projection.  The (token, rank) pairs of the batch are sorted by expert (moe_group_kernel: expert
 // e owns rows [meta[NE + e], + meta[e]) of the grouped activation / result arrays); a workgroup is (row tile, token-tile slot j): slot j is the j-th 256-token tile
 // of the concatenation of the experts' batches, found by walking the per-expert counts ON THE DEVICE - no host synchronisation to size per-expert launches, and
 // eight half-empty launches of ~128 tokens become one that fills the chip.  The body is planes2_body: the wrapper hands it the expert's planes, the
@@ -1484,7 +1484,7 @@ void mmq_set_lds_form(int on) { g_mmq_p2 = on; }
 // continuous-batching decode steps and prompts up to a few hundred tokens: 3 <= T <= g_ksplit_max.  This kernel reads the GGUF
 // bytes (0.56 B / weight) and expands them in registers, the planes kernel reads 2 B / weight it need not expand: measured on the
 // 8B model the whole prompt takes 8.3 vs 13.7 ms at 128 tokens, 13.6 vs 16.7 at 256, 19.4 vs 21.0 at 384 and 22.7 vs 21.1 at 448
-// (round 2: the LDS-form planes kernel moved the crossover down - whole prompt, K-split against planes: 13.8 vs 14.1 ms at 256 tokens,
+// (the LDS-form planes kernel moved the crossover down - whole prompt, K-split against planes: 13.8 vs 14.1 ms at 256 tokens,
 // 17.2 vs 15.2 at 320, 19.1 vs 15.5 at 384)
 static int g_ksplit_max = getenv("MI355_KSPLIT_MAX") ? atoi(getenv("MI355_KSPLIT_MAX")) : 256;
 bool mmq_ksplit_applicable(int type, int K, int T) {
@@ -1701,8 +1701,8 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     if (env_mt == 1 || env_mt == 2) mt = env_mt;
     if (g_mmq_mt == 1 || g_mmq_mt == 2) mt = g_mmq_mt;
     const bool mins = planes_have_mins(type);
-    // both operands through LDS (128 rows x 256 tokens per workgroup) once that grid covers most of the chip; tensors with
-    // too few rows for that split K over 2..4 workgroups (partial sums in the caller's workspace, added up in split order)
+    // 128 rows x 256 tokens per workgroup from 129 tokens on; tensors with too few rows to cover the chip that way split K over 2..4 workgroups (partial sums in
+    // the caller's workspace, added up pairwise)
     bool p2 = false;
     const int n_split = planes2_split(n_rows, K, T, wsp, &p2);
     if (p2) {
