@@ -273,6 +273,8 @@ hipError_t launch_moe_router(int type, const uint8_t *W, int n_expert, int K, co
 // x[t][d] += sum_j eo[j][t][d] * w[t][j]   (experts added in rank order, then the residual)
 hipError_t launch_moe_combine(float *x, const float *eo, const float *w, int T, int E, int k, size_t eo_stride, hipStream_t st);
 hipError_t launch_gather_rows_f32(const float *src, const int32_t *rows, int n_rows, int n, float *dst, hipStream_t st);
+// n floats into pinned host memory (there when the stream has drained)
+hipError_t launch_rows_to_host(const float *src, float *pinned, size_t n, hipStream_t st);
 
 // ---- ggml_mul_mat_id for more than a few tokens (build_moe_ffn): the (token, rank) pairs are grouped
 // by the expert they selected, every expert then sees ONE contiguous batch of activation rows (its weights are read once

@@ -2051,7 +2051,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
                 last_error.clear();
                 hipError_t e2 = layers_of(1, bucket > 0 ? bucket : std::min((int)cp.n_ctx, chunk_cap_ * 64));
                 if (e2 == hipSuccess) e2 = output_of(1, 0);
-                if (e2 == hipSuccess && cp.logits_to_host && !logits_on_host_) e2 = hipMemcpyAsync(h_logits_, d_logits_, (size_t)V * 4, hipMemcpyDeviceToHost, stream_);
+                if (e2 == hipSuccess && cp.logits_to_host && !logits_on_host_) e2 = launch_rows_to_host(d_logits_, h_logits_, (size_t)V, stream_);
                 if (e2 != hipSuccess) inner = last_error;
                 e = hipStreamEndCapture(stream_, &g);
                 if (e2 != hipSuccess) e = e2;
@@ -2082,7 +2082,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         if (e == hipSuccess) e = output_of(n_out, out_base);
         if (profiler_safe) (void)hipStreamSynchronize(stream_);
         if (e == hipSuccess && n_out > 0 && cp.logits_to_host && !embeddings_enabled && !logits_on_host_)
-            e = hipMemcpyAsync(h_logits_ + (size_t)out_base * V, d_logits_ + (size_t)out_base * V, (size_t)n_out * V * 4, hipMemcpyDeviceToHost, stream_);
+            e = launch_rows_to_host(d_logits_ + (size_t)out_base * V, h_logits_ + (size_t)out_base * V, (size_t)n_out * V, stream_);
         prof_end();
     }
     if (stage_event_ && stage_in_setup_) (void)hipEventRecord(stage_event_, stream_);   // (read inside the step)
@@ -2239,7 +2239,7 @@ float *Context::logits_ith(int i) {
     if (i < 0 || i >= (int)out_row_of_batch_.size() || out_row_of_batch_[(size_t)i] < 0) return nullptr;
     if (!logits_fetched_) {
         if (!cp.logits_to_host &&
-            hipMemcpyAsync(h_logits_, d_logits_, (size_t)n_out_last_ * model->hp.n_vocab * 4, hipMemcpyDeviceToHost, stream_) != hipSuccess) return nullptr;
+            (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_logits_, h_logits_, (size_t)n_out_last_ * model->hp.n_vocab, stream_) != hipSuccess)) return nullptr;
         if (hipStreamSynchronize(stream_) != hipSuccess || !mega_check() || !stream_check()) return nullptr;
         logits_fetched_ = true;
     }
@@ -2252,7 +2252,7 @@ float *Context::embeddings_ith(int i) {
     if (i < 0 || i >= (int)out_row_of_batch_.size() || out_row_of_batch_[(size_t)i] < 0) return nullptr;
     const int E = model->hp.n_embd;
     if (!embd_fetched_) {
-        if (hipMemcpyAsync(h_embd_, d_embd_, (size_t)n_out_last_ * E * 4, hipMemcpyDeviceToHost, stream_) != hipSuccess) return nullptr;
+        if (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_embd_, h_embd_, (size_t)n_out_last_ * E, stream_) != hipSuccess) return nullptr;
         if (hipStreamSynchronize(stream_) != hipSuccess) return nullptr;
         embd_fetched_ = true;
     }
