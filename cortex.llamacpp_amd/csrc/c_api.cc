@@ -259,6 +259,14 @@ int64_t mi355_debug_mega_steps(const mi355_context *ctx) { return ctx->c->mega_s
 int64_t mi355_debug_engine_steps(const mi355_context *ctx) { return ctx->c->engine_steps; }
 int64_t mi355_debug_fused_skipped_steps(const mi355_context *ctx) { return ctx->c->fused_skipped_steps; }
 int64_t mi355_debug_qkv_attn_launches(const mi355_context *ctx) { return ctx->c->qkv_attn_launches; }
+int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int32_t n_tokens, int32_t pair, int32_t sum_free) {
+    MMQWorkspace wsp;
+    wsp.bytes = (size_t)num_cu() * 128 * 256 * sizeof(float);
+    wsp.p = reinterpret_cast<float *>(wsp.bytes);               // (looked at for being there)
+    if (n_rows < 1 || n_cols < 256 || n_cols % 256 || n_tokens < 1) return 0;
+    if (mmq_ksplit_preferred(type, n_rows, n_cols, n_tokens, mmq_planes_bytes(type, n_rows, n_cols) != 0, wsp, sum_free != 0, pair != 0)) return n_tokens <= FEW_MAX_T ? 1 : 2;
+    return mmq_applicable(type, n_cols, n_tokens) ? 3 : 0;
+}
 int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int32_t type_v, int32_t type_o, int32_t n_embd, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
                                   int32_t type_kv, int32_t n_kv, int32_t *slots_out) {
     int slots = 0;

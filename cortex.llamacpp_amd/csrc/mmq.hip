@@ -1494,6 +1494,7 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
     return (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K % 256) == 0 && T >= 3 && T <= g_ksplit_max;
 }
 
+static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool *takes);
 // Which kernel takes a 3..256-token launch is a matter of shape (tools/exp_planes_shapes.py, Q5_K, us per launch):
 //     N x K          T = 48     64     96    128    160    192    256
 //   14336 x 4096   K-split 29     30     56     58     83     86    103      planes 256x32: 34 34 35 37 67 68 70   128x128: 55 56 56 57 60 60 61
@@ -1503,13 +1504,29 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
 // (pair: gate | up of a dense layer go out as ONE K-split launch of 2 n_rows rows, which holds its own against two planes launches up to
 // 128 tokens - whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128; past that the LDS-form SwiGLU launch takes the pair:
 // 13.6 -> 10.6 ms at 200 tokens, 14.1 -> 11.1 at 256.)
-// From 129 tokens on the 128 x 256 tiles with K split over the workgroups take every tensor that has planes: prompts of 140, 160, 200 and 256 tokens through eight layers of an
-// 8B model (Q4_K_M) 2.75, 2.81, 3.20 and 3.32 ms by the K-split kernel here, 1.95, 2.00, 2.26 and 2.36 by them; of a 7B model (Q5_K_M) 2.69 .. 3.26 against 1.84 .. 2.24.
-bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, bool pair) {
+// From 129 tokens on the other side is the 128 x 256 tiles, K split over the workgroups where the workspace allows it, and the choice is by the two launches' times.  Both are
+// whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us, Q4_K; Q6_K costs the K-split kernel up to a quarter more): K-split, 32 rows x 64 tokens,
+// a wave's ceil(nb / 8) super-blocks of 4.3 and 3.5; tiles, the part's super-blocks of 3.0 (to 160 tokens) or 3.8 and 9, and 4 more where the parts' sum is a launch of its own.
+// Measured, K-split against tiles (with the sum's launch) at 130 and 256 tokens:
+//   2048 x 2048   9 / 18, 10 / 22      2048 x 5632  18 / 28, 20 / 34      1536 x 8960  24 / 36, 25 / 47      gate | up of 5632 x 2048  36 / 32, 45 / 38
+//   3072 x 3072  17 / 23, 19 / 27      3072 x 8192  39 / 35, 44 / 44      5120 x 5120  28 / 29, 42 / 35      gate | up of 8192 x 3072  55 / 46, 74 / 54
+//   4096 x 4096  23 / 24, 26 / 29      6144 x 4096  34 / 27, 37 / 33      4096 x 14336 64 / 54, 73 / 69      gate | up of 14336 x 4096 129 / 67, 172 / 79
+// Whole prompts of 130, 160 and 256 tokens: the 22 layers of a 2048-column model 2.68, 2.76, 3.20 ms with every tensor here, 3.20, 3.30, 3.75 with every tensor on tiles; eight
+// layers of an 8B model 2.75 (140 tokens), 2.81, 3.32 and 1.95, 2.00, 2.36.
+static bool tiles_beat_ksplit(int n_rows, int K, int T, MMQWorkspace wsp, bool pair, bool sum_free) {
+    bool takes = false;
+    const int rows = pair ? 2 * n_rows : n_rows, parts = planes2_split(rows, K, T, pair ? MMQWorkspace() : wsp, &takes), nb = K >> 8;
+    if (!takes) return n_rows >= 8192;                          // (then the planes kernel below: by rows, as under 129 tokens)
+    const auto up = [](long a, long b) { return (double)((a + b - 1) / b); };
+    const double here = up(up(rows, 32) * up(T, 64), num_cu()) * (4.3 * up(nb, 8) + 3.5);
+    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * ((T <= 160 ? 3.0 : 3.8) * up(nb, parts) + 9.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
+    return tiles < here;
+}
+bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair) {
     static const int env = getenv("MI355_KSPLIT_SHAPE") ? atoi(getenv("MI355_KSPLIT_SHAPE")) : 1;
     if (!mmq_ksplit_applicable(type, K, T)) return false;
-    if (env && has_planes && (T > 128 || (T > 64 && !pair && n_rows >= 8192)) && mmq_applicable(type, K, T)) return false;
-    return true;
+    if (!env || !has_planes || !mmq_applicable(type, K, T)) return true;
+    return T > 128 ? !tiles_beat_ksplit(n_rows, K, T, wsp, pair, sum_free) : T <= 64 || pair || n_rows < 8192;
 }
 
 // segs: up to 3 tensors sharing the activation; swiglu: segs = {gate, up} of one type and shape, out = silu(gate.x) * (up.x) into segs[0].out

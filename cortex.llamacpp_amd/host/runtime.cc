@@ -995,7 +995,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
             return launch_mmq_q80(w.data, w.row_bytes, (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         // (bh_over_ / bl_over_: the caller prepared the block-sum planes of a larger batch that aq's rows are a slice of - the expert loop)
         const int8_t *bh = bh_over_ ? bh_over_ : mmq_bh_, *bl = bh_over_ ? bl_over_ : mmq_bl_;
-        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
+        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, mmq_ws_, parts != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
             if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
             return launch_mmq_ksplit(w.type, w.data, w.row_bytes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         }
@@ -1023,11 +1023,15 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     bool all_q = true;
     for (int i = 0; i < n; i++) all_q &= is_quant(ws[i]->type);
     const int K = (int)ws[0]->K;
-    bool all_mmq = true, all_ks = true;
+    bool all_mmq = true, all_ks = true, all_planes = true;
+    int all_rows = 0;
     for (int i = 0; i < n; i++) {
         all_mmq &= mmq_applicable(ws[i]->type, K, T);
-        all_ks &= T > 128 ? mmq_ksplit_preferred(ws[i]->type, (int)ws[i]->N, K, T, ws[i]->planes != nullptr) : mmq_ksplit_applicable(ws[i]->type, K, T);
+        all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T);
+        all_planes &= ws[i]->planes != nullptr;
+        all_rows += (int)ws[i]->N;
     }
+    if (T > 128) all_ks = all_ks && mmq_ksplit_preferred(ws[0]->type, all_rows, K, T, all_planes, mmq_ws_, parts != nullptr);   // (up to 128 tokens one K-split launch beats three of any kind)
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
         HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
         MMQSeg sg[3];
@@ -1769,8 +1773,8 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                                  (mmq_applicable(L.gate.type, E, T) && mmq_applicable(L.up.type, E, T)) ||
                                  (mmq_ksplit_applicable(L.gate.type, E, T) && mmq_ksplit_applicable(L.up.type, E, T)) ||
                                  (planes_small(L.gate, E, T) && planes_small(L.up, E, T)) || (q80_copy(L.gate, E, T) && q80_copy(L.up, E, T));
-            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, true) &&
-                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, true) && !fuse_ffn;
+            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, mmq_ws_, false, true) &&
+                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, mmq_ws_, false, true) && !fuse_ffn;
             if (gq && uq && L.gate.type == L.up.type && !ffn_mmq) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
                 HIP_TRY(mmvq_tokens(segs, 2, E, T, EPI_SWIGLU, aq_e_, stream_, fz));

@@ -1,0 +1,35 @@
+"""Which contraction a batch takes (host logic: no GPU): the sides on which measured launches were the faster ones."""
+import ctypes as C
+
+import pytest
+
+Q4_K, Q5_K, Q6_K = 12, 13, 14
+MATVEC, FEW, KSPLIT, PLANES = 0, 1, 2, 3
+
+
+@pytest.fixture(scope="module")
+def plan(pkg):
+    lib = pkg.load_library()
+    return lambda *a: int(lib.mi355_debug_batch_plan(*a))
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("n", [129, 145, 200, 256])
+def test_from_129_tokens_by_time(plan, t, n):
+    """A tensor whose 128 x 256 tiles leave most of the chip idle stays with the K-split kernel; one that fills it (alone, K split, or as a SwiGLU pair) does not."""
+    for rows, cols in [(2048, 2048), (2560, 2048), (2048, 5632), (1536, 8960), (2560, 2560), (1024, 8192)]:
+        for sum_free in (0, 1):
+            assert plan(t, rows, cols, n, 0, sum_free) == KSPLIT, (rows, cols)
+    for rows, cols in [(6144, 4096), (4096, 14336), (4096, 11008), (8192, 8192), (8192, 28672), (8192, 1024), (32000, 4096)]:
+        for sum_free in (0, 1):
+            assert plan(t, rows, cols, n, 0, sum_free) == PLANES, (rows, cols)
+    for rows, cols in [(5632, 2048), (8960, 1536), (8192, 3072), (14336, 4096), (18944, 3584)]:
+        assert plan(t, rows, cols, n, 1, 0) == PLANES, (rows, cols)
+    assert plan(t, 1024, 2048, n, 1, 0) == KSPLIT
+
+
+def test_around_the_ranges_ends(plan):
+    """One and two rows are mat-vecs, whose sums a single step's are; from 257 tokens on the K-split kernel is out, whatever the shape."""
+    assert [plan(Q4_K, 2048, 2048, n, 0, 0) for n in (1, 2, 3, 128, 129, 256, 257)] == [MATVEC, MATVEC, FEW, KSPLIT, KSPLIT, KSPLIT, PLANES]
+    assert [plan(Q4_K, 8192, 4096, n, 0, 0) for n in (65, 128, 129)] == [PLANES] * 3
+    assert plan(Q4_K, 2048, 2000, 64, 0, 0) == MATVEC
