@@ -98,6 +98,7 @@ SYMBOLS = {
     "mi355_debug_layer_out": (_i32, [_vp, _i32, _vp, _sz]),
     "mi355_op_quantize_act": (C.c_int, [_i32, _vp, _i64, _i64, _vp]),
     "mi355_op_mul_mat": (C.c_int, [_i32, _vp, _i64, _i64, _vp, _i64, _vp, _vp, _vp]),
+    "mi355_op_mul_mat_batch": (C.c_int, [_i32, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i32, _vp]),
     "mi355_op_ffn_gate_up": (C.c_int, [_i32, _vp, _vp, _i64, _i64, _vp, _i64, _vp]),
     "mi355_op_rms_norm_mul": (C.c_int, [_vp, _vp, _i64, _i64, _f32, _vp]),
     "mi355_op_rope": (C.c_int, [_vp, _i32, _i32, _i32, _vp, _i64, _f32, _f32, _vp, _i32]),
@@ -177,8 +178,8 @@ def load_library(path: str | None = None):
         raise MI355Error(f"{p} not found: build it with `python cortex.llamacpp_amd/build.py` (hipcc, gfx950)")
     lib = C.CDLL(p)
     for name, (res, args) in SYMBOLS.items():
-        if name.startswith("mi355_debug_") and os.environ.get("MI355_LLAMA_LIB") and not hasattr(lib, name):
-            continue                     # (tools/ab_libs.sh: an older build of the library under MI355_LLAMA_LIB may lack a diagnosis getter)
+        if name.startswith(("mi355_debug_", "mi355_op_")) and os.environ.get("MI355_LLAMA_LIB") and not hasattr(lib, name):
+            continue                     # (tools/ab_libs.sh: an older build of the library under MI355_LLAMA_LIB may lack a diagnosis getter or an op of the tests)
         fn = getattr(lib, name)          # AttributeError if the .so does not export a declared symbol
         fn.restype = res
         fn.argtypes = args
@@ -234,6 +235,16 @@ class Backend:
             msum = np.zeros((T, N, nblk), np.int32)
         self._chk(self.lib.mi355_op_mul_mat(t, _ptr(W), N, K, _ptr(x), T, _ptr(y), _ptr(isum), _ptr(msum)), "op_mul_mat")
         return (y, isum, msum) if want_ints else y
+
+    def mul_mat_batch(self, types, Ws, Ns, K: int, x: np.ndarray, resid=None, swiglu: bool = False):
+        Ws = [np.ascontiguousarray(w.view(np.uint8).reshape(-1)) for w in Ws]
+        x = np.ascontiguousarray(x, np.float32).reshape(-1, K)
+        resid = None if resid is None else np.ascontiguousarray(resid, np.float32)
+        n, T = len(Ws), x.shape[0]
+        ys = [np.zeros((T, r), np.float32) for r in (Ns[:1] if swiglu else Ns)]
+        ptrs = lambda arrays: (C.c_void_p * n)(*[a.ctypes.data for a in arrays])  # noqa: E731
+        self._chk(self.lib.mi355_op_mul_mat_batch(n, (C.c_int32 * n)(*types), ptrs(Ws), (C.c_int64 * n)(*Ns), K, _ptr(x), T, _ptr(resid), int(swiglu), ptrs(ys)), "op_mul_mat_batch")
+        return ys
 
     def ffn_gate_up(self, t: int, Wg: np.ndarray, Wu: np.ndarray, N: int, K: int, x: np.ndarray) -> np.ndarray:
         Wg = np.ascontiguousarray(Wg.view(np.uint8).reshape(-1))

@@ -43,7 +43,7 @@ struct mi355_context {
 };
 
 static thread_local std::string t_err;
-static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1;
+static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1, g_op_mmq_few = -1;
 static bool g_backend_ok = false;
 
 static void fail(const std::string &s) { t_err = s; }
@@ -264,7 +264,13 @@ int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int
     wsp.bytes = (size_t)num_cu() * 128 * 256 * sizeof(float);
     wsp.p = reinterpret_cast<float *>(wsp.bytes);               // (looked at for being there)
     if (n_rows < 1 || n_cols < 256 || n_cols % 256 || n_tokens < 1) return 0;
-    if (mmq_ksplit_preferred(type, n_rows, n_cols, n_tokens, mmq_planes_bytes(type, n_rows, n_cols) != 0, wsp, sum_free != 0, pair != 0)) return n_tokens <= FEW_MAX_T ? 1 : 2;
+    if (mmq_ksplit_preferred(type, n_rows, n_cols, n_tokens, mmq_planes_bytes(type, n_rows, n_cols) != 0, wsp, sum_free != 0, pair != 0)) {
+        MMQSeg sg[2] = {};
+        for (MMQSeg &s : sg) { s.n_rows = n_rows; s.type = type; }
+        ActQuant q;
+        q.qf = reinterpret_cast<uint8_t *>(wsp.p);
+        return mmq_few_takes(sg, pair ? 2 : 1, n_cols, n_tokens, q, pair != 0) ? 1 : 2;
+    }
     return mmq_applicable(type, n_cols, n_tokens) ? 3 : 0;
 }
 int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int32_t type_v, int32_t type_o, int32_t n_embd, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
@@ -433,6 +439,12 @@ struct ActBufs {
     }
     bool ok() const { return qs.p && d.p && bs.p && qs0.p && d0.p && qf.p; }
 };
+// launch_mmq_ksplit_multi, with its choice of kernel for 3 .. 64 rows left to it or made here ("mmq_few")
+hipError_t small_batch(const MMQSeg *segs, int n_seg, int K, int T, ActQuant q, const int8_t *bh, const int8_t *bl, bool swiglu) {
+    if (g_op_mmq_few == 1 && T <= FEW_MAX_T) return launch_mmq_few(segs, n_seg, K, T, q, swiglu, nullptr);
+    if (g_op_mmq_few == 0) q.qf = nullptr;
+    return launch_mmq_ksplit_multi(segs, n_seg, K, T, q, bh, bl, swiglu, nullptr);
+}
 int hip_fail(hipError_t e, const char *what) {
     fail(std::string(what) + ": " + hipGetErrorString(e));
     return MI355_ERR_HIP;
@@ -482,6 +494,37 @@ int mi355_op_ffn_gate_up(int32_t type, const void *Wg, const void *Wu, int64_t N
     return dy.down(y, (size_t)N * T * 4) ? MI355_OK : MI355_ERR_HIP;
 }
 
+int mi355_op_mul_mat_batch(int32_t n_seg, const int32_t *types, const void *const *W, const int64_t *N, int64_t K, const float *x, int64_t T, const float *resid, int32_t swiglu,
+                           float *const *y) {
+    if (!need_device()) return MI355_ERR_NO_DEVICE;
+    if (n_seg < 1 || n_seg > 3 || K < 256 || K % 256 || (resid && n_seg > 1) || (swiglu && (n_seg != 2 || types[0] != types[1] || N[0] != N[1]))) { fail("bad segments / K"); return MI355_ERR_ARG; }
+    for (int i = 0; i < n_seg; i++) if (N[i] < 1 || !mmq_ksplit_applicable(types[i], (int)K, (int)T)) { fail("bad type / N / T"); return MI355_ERR_ARG; }
+    DevBuf dx((size_t)K * T * 4), bh(mmq_prep_bytes((int)K, (int)T)), bl(mmq_prep_bytes((int)K, (int)T)), dr(resid ? (size_t)N[0] * T * 4 : 16);
+    ActBufs ab((size_t)K, (size_t)T);
+    if (!dx.up(x, (size_t)K * T * 4) || !bh.p || !bl.p || !ab.ok() || !dr.p || (resid && !dr.up(resid, (size_t)N[0] * T * 4))) { fail("device alloc/copy failed"); return MI355_ERR_OOM; }
+    std::vector<std::unique_ptr<DevBuf>> w, out;
+    MMQSeg sg[3] = {};
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n_seg; i++) {
+        const size_t grow = ggml_row_bytes(types[i], K), drow = dev_row_bytes(types[i], K);
+        DevBuf src(grow * N[i]);
+        w.emplace_back(new DevBuf(drow * N[i]));
+        out.emplace_back(new DevBuf((size_t)N[i] * T * 4));
+        if (!src.up(W[i], grow * N[i]) || !w[i]->p || !out[i]->p) { fail("device alloc/copy failed"); return MI355_ERR_OOM; }
+        e = launch_repack_rows(types[i], src.as<uint8_t>(), w[i]->as<uint8_t>(), K, N[i], nullptr);
+        if (e == hipSuccess) e = hipDeviceSynchronize();
+        if (e != hipSuccess) return hip_fail(e, "repack");
+        sg[i] = MMQSeg{w[i]->as<uint8_t>(), drow, (int)N[i], types[i], out[i]->as<float>(), (int)N[i], resid ? dr.as<float>() : nullptr, 0};
+    }
+    e = launch_quantize(dx.as<float>(), (int)K, (int)T, ab.q, true, false, nullptr);
+    if (e == hipSuccess) e = launch_mmq_prep(ab.q, (int)K, (int)T, bh.as<int8_t>(), bl.as<int8_t>(), nullptr);
+    if (e == hipSuccess) e = small_batch(sg, n_seg, (int)K, (int)T, ab.q, bh.as<int8_t>(), bl.as<int8_t>(), swiglu != 0);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) return hip_fail(e, "mul_mat_batch");
+    for (int i = 0; i < (swiglu ? 1 : n_seg); i++) if (!out[i]->down(y[i], (size_t)N[i] * T * 4)) return MI355_ERR_HIP;
+    return MI355_OK;
+}
+
 int mi355_op_mul_mat(int32_t type, const void *W, int64_t N, int64_t K, const float *x, int64_t T, float *y, int32_t *isum, int32_t *msum) {
     if (!need_device()) return MI355_ERR_NO_DEVICE;
     const size_t grow = ggml_row_bytes(type, K), drow = dev_row_bytes(type, K);
@@ -512,7 +555,8 @@ int mi355_op_mul_mat(int32_t type, const void *W, int64_t N, int64_t K, const fl
             DevBuf bh(mmq_prep_bytes((int)K, (int)T)), bl(mmq_prep_bytes((int)K, (int)T));
             if (!bh.p || !bl.p) return MI355_ERR_OOM;
             e = launch_mmq_prep(ab.q, (int)K, (int)T, bh.as<int8_t>(), bl.as<int8_t>(), nullptr);
-            if (e == hipSuccess) e = launch_mmq_ksplit(type, wdev.as<uint8_t>(), drow, (int)N, (int)K, (int)T, ab.q, bh.as<int8_t>(), bl.as<int8_t>(), dy.as<float>(), (int)N, nullptr, nullptr);
+            const MMQSeg sg{wdev.as<uint8_t>(), drow, (int)N, type, dy.as<float>(), (int)N, nullptr, 0};
+            if (e == hipSuccess) e = small_batch(&sg, 1, (int)K, (int)T, ab.q, bh.as<int8_t>(), bl.as<int8_t>(), false);
             if (e == hipSuccess) e = hipDeviceSynchronize();
             if (e != hipSuccess) return hip_fail(e, "mmq_ksplit");
         } else
@@ -860,6 +904,7 @@ int mi355_debug_set_option(const char *name, int32_t value) {
     if (!strcmp(name, "mmq_split")) { mmq_set_split(value); return MI355_OK; }
     if (!strcmp(name, "mmq_lds_form")) { mmq_set_lds_form(value); return MI355_OK; }
     if (!strcmp(name, "mmq_ksplit")) { g_op_mmq_ksplit = value != 0; return MI355_OK; }
+    if (!strcmp(name, "mmq_few")) { g_op_mmq_few = value; return MI355_OK; }
     if (!strcmp(name, "attn_store_fuse")) { set_attn_store_fuse(value != 0); return MI355_OK; }
     if (!strcmp(name, "rope_fast")) { set_rope_fast(value != 0); return MI355_OK; }
     if (!strcmp(name, "decode_mega") || !strcmp(name, "decode_engine")) {

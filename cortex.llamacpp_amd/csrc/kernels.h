@@ -148,7 +148,7 @@ hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_s
 hipError_t launch_mmq_planes(int type, const uint8_t *planes, int n_rows, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                              float *out, int ld_out, const float *resid, hipStream_t st, MMQWorkspace wsp = MMQWorkspace(), int *parts = nullptr);
 // parts (nullable): a launch that splits K leaves its partial sums in the workspace ([part][T][n_rows]; `out` untouched) and their number here
-// small batches (continuous-batching decode steps, 8 <= T <= 64): K split over the waves of a workgroup, GGUF-form weights
+// batches of 3 .. 256 tokens (continuous-batching decode steps, short prompts): K split over the waves of a workgroup, GGUF-form weights
 struct MMQSeg {
     const uint8_t *W; size_t row_bytes; int n_rows, type;
     float *out; int ld_out; const float *resid;
@@ -176,9 +176,9 @@ bool mmq_ksplit_applicable(int type, int K, int T);
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair = false);
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                                    bool swiglu, hipStream_t st);
-hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);   // mmq_few.hip: 3 .. 64 tokens of the same
-hipError_t launch_mmq_ksplit(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q,
-                             const int8_t *bh, const int8_t *bl, float *out, int ld_out, const float *resid, hipStream_t st);
+// mmq_few.hip: 3 .. 64 tokens of the same, bit for bit; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
+bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu);
+hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);
 size_t mmq_prep_bytes(int K, int T);                       // bytes of each of the two block-sum planes
 hipError_t launch_mmq_prep(const ActQuant &q, int K, int T, int8_t *bh, int8_t *bl, hipStream_t st);
 hipError_t launch_mmq(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q,

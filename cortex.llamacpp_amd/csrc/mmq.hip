@@ -1529,12 +1529,12 @@ bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, M
     return T > 128 ? !tiles_beat_ksplit(n_rows, K, T, wsp, pair, sum_free) : T <= 64 || pair || n_rows < 8192;
 }
 
-// segs: up to 3 tensors sharing the activation; swiglu: segs = {gate, up} of one type and shape, out = silu(gate.x) * (up.x) into segs[0].out
+// segs: up to 3 tensors sharing the activation; swiglu (to 32 tokens, or where mmq_few_takes): segs = {gate, up} of one type and shape, out = silu(gate.x) * (up.x) into segs[0].out
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                                    bool swiglu, hipStream_t st) {
     if (n_seg < 1 || n_seg > 3) return hipErrorInvalidValue;
     if (swiglu && (n_seg != 2 || segs[0].type != segs[1].type || segs[0].n_rows != segs[1].n_rows)) return hipErrorInvalidValue;
-    if (q.qf && T <= FEW_MAX_T) return launch_mmq_few(segs, n_seg, K, T, q, swiglu, st);
+    if (mmq_few_takes(segs, n_seg, K, T, q, swiglu)) return launch_mmq_few(segs, n_seg, K, T, q, swiglu, st);
     KSplitArgs a{};
     a.n_seg = n_seg; a.K = K; a.T = T; a.swiglu = swiglu ? 1 : 0;
     a.aq = q.qs; a.ad = q.d; a.abh = bh; a.abl = bl;
@@ -1545,6 +1545,7 @@ hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, 
         if (!swiglu || i == 0) tiles += (segs[i].n_rows + 31) / 32;
     }
     const int mt = T <= 32 ? 1 : 2;
+    if (swiglu && mt > 1) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)((T + 32 * mt - 1) / (32 * mt)));
 #define KS(MTV, SW)                                                                                                  \
     {                                                                                                                \
@@ -1555,17 +1556,10 @@ hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, 
         if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_ksplit_kernel<MTV, SW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
         hipLaunchKernelGGL((mmq_ksplit_kernel<MTV, SW>), grid, dim3(NTHREADS), lds, st, a);                          \
     }
-    if (swiglu) { if (mt == 1) KS(1, true) else KS(2, true) }
-    else { if (mt == 1) KS(1, false) else KS(2, false) }
+    if (swiglu) KS(1, true)
+    else if (mt == 1) KS(1, false) else KS(2, false)
 #undef KS
     return hipGetLastError();
-}
-
-hipError_t launch_mmq_ksplit(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q,
-                             const int8_t *bh, const int8_t *bl, float *out, int ld_out, const float *resid, hipStream_t st) {
-    MMQSeg sg{};
-    sg.W = W; sg.row_bytes = row_bytes; sg.n_rows = n_rows; sg.type = type; sg.out = out; sg.ld_out = ld_out; sg.resid = resid;
-    return launch_mmq_ksplit_multi(&sg, 1, K, T, q, bh, bl, false, st);
 }
 
 size_t mmq_planes_bytes(int type, int64_t n_rows, int K) {

@@ -405,7 +405,23 @@ void few_type(const FewArgs &a, int blocks, hipStream_t st) {
 
 }  // namespace
 
-// segs as launch_mmq_ksplit_multi's (which sends 3 .. 64 tokens here): up to three tensors sharing the activation, or {gate, up} of one type and shape with swiglu
+// Whether a launch of T tokens is the faster one here (the sums are the same either way; us, here against the K-split kernel of mmq.hip):
+//   * to 16 tokens: 4.2 / 6.1 (2048 x 2048) .. 62 / 100 (128256 x 4096), Q6_K 104 / 139;
+//   * to 48: as long as the row tiles fill their rounds of CUs - 320 of 512 do not: 5120 x 5120 14.3 / 10.8 at 17 tokens, 17.9 / 16.4 at 33 - and, for Q6_K, whose units
+//     take twice the instructions, there is but one round: 4096 x 4096 10.8 / 13.3, but 6144 x 4096 15.6 / 14.1 and 152064 x 3584 270 / 242;
+//   * to 64, where the operands of four token tiles leave two units in flight: gate | up, 42 / 50 (14336 x 4096), and long rows, 32.7 / 39.5 (4096 x 14336) - but 13.5 / 12.7
+//     (4096 x 4096), 112 / 77 (8192 x 28672: 512 row tiles), 318 / 217 (152064 x 3584), and Q6_K never, 549 / 233.
+bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu) {
+    if (!q.qf || T > FEW_MAX_T) return false;
+    if (T <= 16) return true;
+    int tiles = 0, q6 = 0;
+    for (int i = 0; i < n_seg; i++) { if (!swiglu || i == 0) tiles += (segs[i].n_rows + 15) / 16; q6 += segs[i].type == T_Q6_K; }
+    const bool one_round = tiles <= num_cu();
+    if (T <= 48) return q6 == n_seg ? one_round : one_round || 2 * tiles >= 3 * num_cu();
+    return q6 == 0 && (swiglu || (one_round && K > 4096));
+}
+
+// segs as launch_mmq_ksplit_multi's (which comes here where mmq_few_takes says so): up to three tensors sharing the activation, or {gate, up} of one type and shape with swiglu
 hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st) {
     if (!q.qf || T > FEW_MAX_T) return hipErrorInvalidValue;
     FewArgs a{};

@@ -996,8 +996,9 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
         // (bh_over_ / bl_over_: the caller prepared the block-sum planes of a larger batch that aq's rows are a slice of - the expert loop)
         const int8_t *bh = bh_over_ ? bh_over_ : mmq_bh_, *bl = bh_over_ ? bl_over_ : mmq_bl_;
         if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, mmq_ws_, parts != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
-            if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
-            return launch_mmq_ksplit(w.type, w.data, w.row_bytes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
+            const MMQSeg sg{w.data, w.row_bytes, (int)w.N, w.type, out, ld_out, epi == EPI_ADD ? resid : nullptr, 0};
+            if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, mmq_few_takes(&sg, 1, K, T, aq, false)));
+            return launch_mmq_ksplit_multi(&sg, 1, K, T, aq, bh, bl, false, stream_);
         }
         if (mmq_applicable(w.type, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // prompt processing: MFMA path
             if ((w.type != T_Q6_K || !w.planes) && !bh_over_) HIP_TRY(ensure_prep(aq, K, T));
@@ -1033,9 +1034,9 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     }
     if (T > 128) all_ks = all_ks && mmq_ksplit_preferred(ws[0]->type, all_rows, K, T, all_planes, mmq_ws_, parts != nullptr);   // (up to 128 tokens one K-split launch beats three of any kind)
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
-        HIP_TRY(ensure_prep(aq, K, T, aq.qf && T <= FEW_MAX_T));
         MMQSeg sg[3];
         for (int i = 0; i < n; i++) sg[i] = MMQSeg{ws[i]->data, ws[i]->row_bytes, (int)ws[i]->N, ws[i]->type, outs[i], (int)ws[i]->N, nullptr, 0};
+        HIP_TRY(ensure_prep(aq, K, T, mmq_few_takes(sg, n, K, T, aq, false)));
         return launch_mmq_ksplit_multi(sg, n, K, T, aq, mmq_bh_, mmq_bl_, false, stream_);
     }
     if (all_mmq && pending_fuse_.mode == 0) {
@@ -1779,11 +1780,11 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
                 HIP_TRY(mmvq_tokens(segs, 2, E, T, EPI_SWIGLU, aq_e_, stream_, fz));
             } else if (ffn_ks) {                               // batched decode step: gate and up in one launch
-                const bool few = aq_e_.qf && T <= FEW_MAX_T;
-                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, T, few));
                 MMQSeg sg[2] = {{L.gate.data, L.gate.row_bytes, (int)L.gate.N, L.gate.type, ffn_, FF, nullptr, 0},
                                 {L.up.data, L.up.row_bytes, (int)L.up.N, L.up.type, ffn_u_, FF, nullptr, 0}};
-                const bool pair = (few || T <= 32) && L.gate.type == L.up.type && L.gate.N == L.up.N;     // SwiGLU in the epilogue
+                const bool alike = L.gate.type == L.up.type && L.gate.N == L.up.N;
+                const bool pair = alike && (T <= 32 || mmq_few_takes(sg, 2, E, T, aq_e_, true));          // SwiGLU in the epilogue
+                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, T, mmq_few_takes(sg, 2, E, T, aq_e_, pair)));
                 HIP_TRY(launch_mmq_ksplit_multi(sg, 2, E, T, aq_e_, mmq_bh_, mmq_bl_, pair, stream_));
                 if (!pair) {
                     if (is_quant(L.down.type) && (FF % 256) == 0) {

@@ -213,6 +213,10 @@ MI355_API int mi355_op_mul_mat(int32_t type, const void *W, int64_t N, int64_t K
  * epilogue, as the prompt path launches them (mmq_planes2_swiglu_kernel): y[t][n] = silu(Wg[n] . x[t]) * (Wu[n] . x[t]).
  * Shapes too small for that launch are refused unless the debug option "mmq_tiles" = 4 forces the kernel. */
 MI355_API int mi355_op_ffn_gate_up(int32_t type, const void *Wg, const void *Wu, int64_t N, int64_t K, const float *x, int64_t T, float *y);
+/* up to three K-quant tensors against the same 3 .. 256 rows in one launch, as a batch's Q | K | V (y[i]: [T][N[i]]); resid (nullable, one tensor): [T][N[0]] added to its
+   result; swiglu: W = {ffn_gate, ffn_up} of one type and shape, y[0] = silu(gate . x) * (up . x).  Option "mmq_few" as in mi355_op_mul_mat */
+MI355_API int mi355_op_mul_mat_batch(int32_t n_seg, const int32_t *types, const void *const *W, const int64_t *N, int64_t K, const float *x, int64_t T, const float *resid,
+                                     int32_t swiglu, float *const *y);
 MI355_API int mi355_op_rms_norm_mul(const float *x, const float *w, int64_t n, int64_t T, float eps, float *y);
 MI355_API int mi355_op_rope(float *x, int32_t n_head, int32_t head_dim, int32_t n_rot, const int32_t *pos, int64_t T,
                             float freq_base, float freq_scale, const float *freq_factors, int32_t neox);
@@ -295,8 +299,9 @@ MI355_API void mi355_engine_set_log_callback(mi355_engine *e, mi355_log_callback
 
 /* Test / tool switches of the per-op entry points: "mmq_planes" (1: mi355_op_mul_mat with T >= 32 expands the weight
  * into MFMA planes first, as a loaded model does; 0: expands on the fly inside the kernel), "mmq_tiles" (0 | 1 | 2
- * token tiles per wave), "mmq_ksplit" (1: 8 <= T <= 64 uses the K-split small-batch kernel, as the runtime does; 0: the
- * kernels the other T ranges use); and of contexts created afterwards: "decode_mega" (1: single-token steps of a dense
+ * token tiles per wave), "mmq_ksplit" (1: 3 <= T <= 256 uses the small-batch kernels, as the runtime does; 0: the
+ * kernels the other T ranges use), "mmq_few" (which of the small-batch kernels takes 3 <= T <= 64: 1 csrc/mmq_few.hip, 0 the K-split kernel of csrc/mmq.hip,
+ * -1, the default: by shape); and of contexts created afterwards: "decode_mega" (1: single-token steps of a dense
  * K-quant model with Llama-3-8B's layer geometry run every layer in one launch; 0, the default: one launch per operation
  * — both produce the same bits; the single launch measured slower); "moe_group_min" (batches of at least
  * this many tokens run a mixture-of-experts feed-forward grouped by expert, default 8; smaller ones loop over (token,

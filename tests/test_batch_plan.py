@@ -33,3 +33,14 @@ def test_around_the_ranges_ends(plan):
     assert [plan(Q4_K, 2048, 2048, n, 0, 0) for n in (1, 2, 3, 128, 129, 256, 257)] == [MATVEC, MATVEC, FEW, KSPLIT, KSPLIT, KSPLIT, PLANES]
     assert [plan(Q4_K, 8192, 4096, n, 0, 0) for n in (65, 128, 129)] == [PLANES] * 3
     assert plan(Q4_K, 2048, 2000, 64, 0, 0) == MATVEC
+
+
+def test_to_64_tokens_by_shape(plan):
+    """mmq_few.hip to 16 tokens; beyond, where its row tiles fill their rounds of CUs (Q6_K: one round), and from 49 on for gate | up and long rows of few tensors."""
+    assert all(plan(t, n, 4096, T, 0, 0) == FEW for t in (Q4_K, Q5_K, Q6_K) for n in (512, 5120, 128256) for T in (3, 16))
+    assert [plan(Q4_K, n, 5120, T, 0, 0) for n in (4096, 5120, 6144) for T in (17, 48)] == [FEW, FEW, KSPLIT, KSPLIT, FEW, FEW]
+    assert [plan(Q6_K, n, 4096, T, 0, 0) for n in (4096, 6144, 128256) for T in (17, 48)] == [FEW, FEW, KSPLIT, KSPLIT, KSPLIT, KSPLIT]
+    for T in (49, 64):
+        assert [plan(t, 4096, 14336, T, 0, 0) for t in (Q4_K, Q5_K, Q6_K)] == [FEW, FEW, KSPLIT]
+        assert [plan(Q4_K, r, c, T, 0, 0) for r, c in [(4096, 4096), (8192, 28672), (152064, 3584)]] == [KSPLIT] * 3
+        assert [plan(t, 14336, 4096, T, 1, 0) for t in (Q4_K, Q5_K, Q6_K)] == [FEW, FEW, KSPLIT]

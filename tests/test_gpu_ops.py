@@ -217,7 +217,11 @@ def test_mul_mat_small_batch_ksplit(be, t, K, N, T):
     rng = np.random.default_rng(K + N + T + t)
     W = rand_weights(rng, t, N * K)
     x = (rng.standard_normal((T, K)) * rng.uniform(0.1, 4.0, (T, 1))).astype(np.float32)
-    y = be.mul_mat(t, W, N, K, x)
+    be.set_option("mmq_few", 0)                                # (to 64 tokens the choice is by shape)
+    try:
+        y = be.mul_mat(t, W, N, K, x)
+    finally:
+        be.set_option("mmq_few", -1)
     ref = oq.mul_mat(t, W, N, K, x)
     assert np.abs(y - ref).max() <= 2e-5 * np.abs(ref).max() + 1e-6
 
