@@ -136,17 +136,20 @@ __global__ void step_setup_kernel(const int32_t *tok_pos, int T, RopeArgs ra, fl
 }
 // ... and the embedding rows of the batch's tokens (ggml_get_rows of token_embd, dequantised: get_rows_kernel of misc.hip) in the same launch: grid
 // (row parts, tokens) of 256 threads; the first T * n_rot / 2 threads of the grid also fill the cos / sin table, block (0, 0) the cell metadata
+// ONE: a single token, whose scalars are arguments (v) and go to `stage` for the launches behind
+template <bool ONE>
 __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *tok_pos, int T, RopeArgs ra, float theta_scale, float *cs_out, int32_t *cell_pos,
                                                                uint64_t *cell_seq, const int32_t *tok_cell, const uint64_t *tok_seqmask, unsigned *zero_word,
                                                                unsigned *epoch_word, int type, const uint8_t *table, int K, size_t row_bytes,
-                                                               const int32_t *ids, float *dst, const uint32_t *stage_src, uint32_t *stage_dst, int stage_words) {
+                                                               const int32_t *ids, float *dst, const StepBlock v, uint32_t *stage) {
     const int lin = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
-    // a step of one token: its staging block comes out of pinned host memory here (the arrays above point into it) and is left on the device for the launches behind
-    if (lin < stage_words) stage_dst[lin] = stage_src[lin];
+    if (ONE && lin < 16) stage[lin] = v.w[lin];
     if (blockIdx.x == 0 && blockIdx.y == 0) {
         if (zero_word && threadIdx.x < 9) zero_word[threadIdx.x == 0 ? 0 : 32 * threadIdx.x] = 0u;
         if (epoch_word && threadIdx.x == 0) epoch_word[0] = epoch_word[0] + 1u;
-        for (int t = threadIdx.x; t < T; t += blockDim.x) {
+        if (ONE) {
+            if (threadIdx.x == 0) { cell_pos[v.w[10]] = (int32_t)v.w[6]; cell_seq[v.w[10]] = (uint64_t)v.w[14] | (uint64_t)v.w[15] << 32; }
+        } else for (int t = threadIdx.x; t < T; t += blockDim.x) {
             cell_pos[tok_cell[t]] = tok_pos[t];
             cell_seq[tok_cell[t]] = tok_seqmask[t];
         }
@@ -155,25 +158,27 @@ __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *to
     if (lin < T * half) {
         const int t = lin / half, i = lin - t * half;
         float c, s;
-        rope_angle(i, tok_pos[t], theta_scale, ra, c, s);
+        rope_angle(i, ONE ? (int)v.w[6] : tok_pos[t], theta_scale, ra, c, s);
         cs_out[(size_t)t * ra.n_rot + 2 * i] = c;
         cs_out[(size_t)t * ra.n_rot + 2 * i + 1] = s;
     }
     const int i = blockIdx.y;
-    const uint8_t *row = table + (size_t)ids[i] * row_bytes;
+    const uint8_t *row = table + (size_t)(ONE ? (int32_t)v.w[4] : ids[i]) * row_bytes;
     for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < K; e += gridDim.x * blockDim.x)
         dst[(size_t)i * K + e] = dequant_elem(type, row, K, e);
 }
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st, const void *stage_src, void *stage_dst, int stage_words) {
+                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one, void *stage) {
+    if (one && (T != 1 || !stage)) return hipErrorInvalidValue;
     const float theta_scale = powf(ra.freq_base, -2.0f / (float)ra.n_rot);
     int bx = (int)((K + 255) / 256);
     if (bx > 64) bx = 64;
     while ((long)bx * T * 256 < (long)T * (ra.n_rot >> 1)) bx++;          // (enough threads for the table: n_rot / 2 <= 256 * bx per token)
-    hipLaunchKernelGGL(step_setup_embed_kernel, dim3(bx, T), dim3(256), 0, st, tok_pos, T, ra, theta_scale, cs_out, cell_pos, cell_seq, tok_cell, tok_seqmask,
-                       zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst, reinterpret_cast<const uint32_t *>(stage_src),
-                       reinterpret_cast<uint32_t *>(stage_dst), stage_words);
+    if (one) hipLaunchKernelGGL((step_setup_embed_kernel<true>), dim3(bx, 1), dim3(256), 0, st, nullptr, 1, ra, theta_scale, cs_out, cell_pos, cell_seq, nullptr, nullptr,
+                                zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), nullptr, dst, *one, reinterpret_cast<uint32_t *>(stage));
+    else hipLaunchKernelGGL((step_setup_embed_kernel<false>), dim3(bx, T), dim3(256), 0, st, tok_pos, T, ra, theta_scale, cs_out, cell_pos, cell_seq, tok_cell, tok_seqmask,
+                            zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst, StepBlock{}, (uint32_t *)nullptr);
     return hipGetLastError();
 }
 hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,

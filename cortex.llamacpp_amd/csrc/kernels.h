@@ -611,10 +611,13 @@ hipError_t launch_rope_table(const int32_t *tok_pos, int T, RopeArgs ra, float *
 // epoch_word (nullable): device word incremented once per call - the step serial the hand-over tags of decode_engine.hip are built from
 hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                              const uint64_t *tok_seqmask, unsigned *zero_word, hipStream_t st, unsigned *epoch_word = nullptr);
-// launch_step_setup + launch_get_rows (the batch's embedding rows, dst[T][K]) in one launch
+// the staging block of a batch of one token: n_kv in word 0; token, position, sequence, cell and output row in words 4, 6, 8, 10, 12; the sequence mask in 14 and 15
+struct StepBlock { uint32_t w[16]; };
+// launch_step_setup + launch_get_rows (the batch's embedding rows, dst[T][K]) in one launch.  one (T == 1): the block travels as the launch's argument, in place of the arrays,
+// and is left at `stage` on the device
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table_dev, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st, const void *stage_src = nullptr, void *stage_dst = nullptr, int stage_words = 0);
+                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one = nullptr, void *stage = nullptr);
 hipError_t launch_rope_inplace(float *x, int T, int n_head, int D, const int32_t *tok_pos, RopeArgs ra, hipStream_t st);
 
 struct AttnArgs {

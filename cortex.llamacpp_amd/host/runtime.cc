@@ -535,6 +535,7 @@ Context::~Context() {
     }
     for (auto &ge : graphs_) (void)hipGraphExecDestroy(ge.second);
     if (stage_event_) (void)hipEventDestroy(stage_event_);
+    for (hipEvent_t ev : step_done_) if (ev) (void)hipEventDestroy(ev);
     for (auto &pe : prof_events_) (void)hipEventDestroy(pe.second);
     for (void *p : allocs_) (void)hipFree(p);
     if (h_stage_) (void)hipHostFree(h_stage_);
@@ -811,6 +812,7 @@ int Context::upload_cells() {
     dirty_lo_ = dirty_hi_ = 0;
     device_cells_known_ = true;
     if (u0 >= u1) return 0;
+    stage_pending_ = true;
     return hipMemcpyAsync(d_cell_pos_ + u0, h_cell_pos_ + u0, (size_t)(u1 - u0) * 4, hipMemcpyHostToDevice, stream_) == hipSuccess &&
            hipMemcpyAsync(d_cell_seq_ + u0, h_cell_seq_ + u0, (size_t)(u1 - u0) * 8, hipMemcpyHostToDevice, stream_) == hipSuccess ? 0 : -1;
 }
@@ -1419,6 +1421,11 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
     return hipSuccess;
 }
 
+hipError_t Context::launch_setup(int T, bool mega) {
+    return launch_step_setup_embed(d_pos_, T, rope_args(*model, true), rope_cs_, d_cell_pos_, d_cell_seq_, d_cell_, d_seqmask_, mega ? d_mega_sync_ : nullptr, d_step_serial_,
+                                   model->tok_embd.type, model->tok_embd.data, model->hp.n_embd, d_tok_, x_, stream_, one_token_ ? &step_block_ : nullptr, d_stage_);
+}
+
 hipError_t Context::run_layers(int T, int n_kv_cap) {
     if (model->hp.encoder) return run_layers_encoder(T, n_kv_cap);
     cur_T_ = T;
@@ -1450,10 +1457,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
     const bool engine = T == 1 && !mega && !profile_ && !debug_taps_ && !ub_embd_ && engine_prepare();
     last_layers_engine_ = engine;
     // cos / sin table, cell metadata and the tokens' embedding rows: one launch
-    const auto staged = [&](const auto *d) { return stage_in_setup_ ? (decltype(d))(h_stage_ + ((const uint8_t *)d - d_stage_)) : d; };
-    HIP_TRY(launch_step_setup_embed(staged(d_pos_), T, ra, rope_cs_, d_cell_pos_, d_cell_seq_, staged(d_cell_), staged(d_seqmask_), mega ? d_mega_sync_ : nullptr,
-                                    d_step_serial_, model->tok_embd.type, model->tok_embd.data, E, staged(d_tok_), x_, stream_, h_stage_, d_stage_,
-                                    stage_in_setup_ ? (int)(stage_used_ / 4) : 0));
+    if (!setup_launched_) HIP_TRY(launch_setup(T, mega));
     // an embeddings batch: the caller's rows take the place of the looked-up ones (never inside a captured graph: decode_ubatch)
     if (ub_embd_) HIP_TRY(hipMemcpyAsync(x_, ub_embd_, (size_t)T * E * sizeof(float), hipMemcpyHostToDevice, stream_));
     prof_mark("embed");
@@ -1954,16 +1958,21 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
     n_kv_ = std::min((int)cp.n_ctx, (cells_end_ + 31) & ~31);
 
     // stage token arrays and cell table (the pinned blocks may still be in flight from the previous micro-batch)
-    if (stage_event_) (void)hipEventSynchronize(stage_event_);
+    one_token_ = n == 1 && !model->nvx && !model->hp.encoder;
+    setup_launched_ = false;
+    if (stage_pending_ && stage_event_) { (void)hipEventSynchronize(stage_event_); stage_pending_ = false; }
+    if (one_token_ && step_done_[step_turn_]) (void)hipEventSynchronize(step_done_[step_turn_]);
     if (device_cells_known_)
         for (int i = 0; i < n; i++) { const int c = tcell[(size_t)i]; h_cell_pos_[c] = pos[i]; h_cell_seq_[c] = seqmask[i]; }   // the set-up launch writes these
     if (upload_cells() != 0) { last_error = "cell table upload failed"; return -1; }
     // the arrays one behind the other, as long as the batch: a step uploads some dozen bytes (the same addresses for every batch of one token: its graphs hold them)
     const size_t T = ((size_t)n + 1) & ~(size_t)1;             // keeps the u64 seqmask array 8-byte aligned
-    int32_t *h_nkv = (int32_t *)h_stage_;
-    int32_t *h_tok = (int32_t *)(h_stage_ + 16), *h_pos = h_tok + T, *h_seq = h_pos + T, *h_cell = h_seq + T, *h_out = h_cell + T;
+    static_assert(sizeof(StepBlock) == 16 + 5 * 2 * 4 + 8, "a batch of one token");
+    uint8_t *const block = one_token_ ? (uint8_t *)&step_block_ : h_stage_;
+    int32_t *h_nkv = (int32_t *)block;
+    int32_t *h_tok = (int32_t *)(block + 16), *h_pos = h_tok + T, *h_seq = h_pos + T, *h_cell = h_seq + T, *h_out = h_cell + T;
     uint64_t *h_mask = (uint64_t *)(h_out + T);
-    const auto on_device = [&](const void *h) { return d_stage_ + ((const uint8_t *)h - h_stage_); };
+    const auto on_device = [&](const void *h) { return d_stage_ + ((const uint8_t *)h - block); };
     d_tok_ = (int32_t *)on_device(h_tok); d_pos_ = (int32_t *)on_device(h_pos); d_seq_ = (int32_t *)on_device(h_seq); d_cell_ = (int32_t *)on_device(h_cell);
     d_outrow_ = (int32_t *)on_device(h_out); d_seqmask_ = (uint64_t *)on_device(h_mask);
     h_nkv[0] = n_kv_;
@@ -1972,9 +1981,10 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         h_tok[i] = tokens[i]; h_pos[i] = pos[i]; h_seq[i] = seq[i]; h_cell[i] = tcell[(size_t)i]; h_mask[i] = seqmask[i];
         if (flags[i]) h_out[n_out++] = i;
     }
-    stage_used_ = (size_t)((uint8_t *)(h_mask + n) - h_stage_);
-    stage_in_setup_ = n == 1 && !model->nvx && !model->hp.encoder;
-    if (!stage_in_setup_ && hipMemcpyAsync(d_stage_, h_stage_, stage_used_, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "token upload failed"; return -1; }
+    if (!one_token_) {
+        stage_pending_ = true;
+        if (hipMemcpyAsync(d_stage_, h_stage_, (size_t)((uint8_t *)(h_mask + n) - h_stage_), hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "token upload failed"; return -1; }
+    }
     // continuous-batching steps (a few tokens, usually one per sequence): each token scans only the 64-cell chunks that
     // hold cells of its own sequence instead of the whole cache
     chunk_lmax_ = 0;
@@ -2010,6 +2020,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             chunk_lmax_ = std::max(chunk_lmax_, c);
         }
         if (chunk_lmax_ < 1) chunk_lmax_ = 1;
+        stage_pending_ = true;
         if (hipMemcpyAsync(d_chunks_, h_chunks_, (size_t)64 * (chunk_stride_ + 1) * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "chunk list upload failed"; return -1; }
     }
     // rocprofv3 --pmc does not keep copy-engine transfers ordered with the kernels it serialises (observed: kernels reading
@@ -2021,7 +2032,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         for (int i = 0; i < n; i++) nvx_seq_len_[(size_t)seq[i]] = std::max<uint64_t>(nvx_seq_len_[(size_t)seq[i]], (uint64_t)pos[i] + 1);
     }
     if (!stage_event_) (void)hipEventCreateWithFlags(&stage_event_, hipEventDisableTiming);
-    if (stage_event_ && !stage_in_setup_) (void)hipEventRecord(stage_event_, stream_);
+    if (stage_event_ && stage_pending_) (void)hipEventRecord(stage_event_, stream_);
 
     const int V = model->hp.n_vocab;
     const bool nvx = model->nvx != nullptr;
@@ -2044,13 +2055,18 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             chunk_cap_ = std::min(chunk_stride_, (chunk_lmax_ + 3) & ~3);
             bucket = -chunk_cap_;                              // separate key space from the cell-count buckets
         }
+        // the step's set-up goes out by itself, its scalars as arguments: nothing of a queued step lies in host memory, and the graph behind it is the same for every step.  us a step
+        // queued unread, and read (eight layers of an 8B model; six of a 2048-column one): 435 and 449; 258 and 273.  With the block fetched from pinned memory inside the graph,
+        // where the next call had to wait for the whole step: 442 and 447; 265 and 272.  With the block copied in front of the graph: 454 and 466; 277 and 286
+        if (one_token_) {
+            if ((e = launch_setup(1, true)) != hipSuccess) { last_error = std::string("set-up launch failed: ") + hipGetErrorString(e); return -1; }
+            setup_launched_ = true;
+        }
         auto git = graphs_.find(bucket);
         graph_exec_ = git == graphs_.end() ? nullptr : git->second;
         if (!graph_exec_) {
             hipGraph_t g = nullptr;
             std::string inner;                                  // which launch refused, when one did (HIP_TRY's message)
-            // (a copy nobody waits for: an idle device is awake by the time the capture - some hundred microseconds of the host - is done)
-            if (stage_in_setup_) (void)hipMemcpyAsync(d_stage_, h_stage_, stage_used_, hipMemcpyHostToDevice, stream_);
             e = hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
                 last_error.clear();
@@ -2090,7 +2106,11 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             e = launch_rows_to_host(d_logits_ + (size_t)out_base * V, h_logits_ + (size_t)out_base * V, (size_t)n_out * V, stream_);
         prof_end();
     }
-    if (stage_event_ && stage_in_setup_) (void)hipEventRecord(stage_event_, stream_);   // (read inside the step)
+    if (one_token_) {
+        if (!step_done_[step_turn_]) (void)hipEventCreateWithFlags(&step_done_[step_turn_], hipEventDisableTiming);
+        if (step_done_[step_turn_]) (void)hipEventRecord(step_done_[step_turn_], stream_);
+        step_turn_ ^= 1;
+    }
     if (e != hipSuccess) { last_error = std::string("decode failed: ") + hipGetErrorString(e) + " / " + last_error_string(); return -1; }
     if (n == 1 && (graph_ok ? graph_is_mega_[graph_exec_] : last_layers_mega_)) mega_steps++;
     if (n == 1 && (graph_ok ? graph_is_engine_[graph_exec_] : last_layers_engine_)) engine_steps++;

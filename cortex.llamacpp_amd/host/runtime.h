@@ -263,8 +263,13 @@ class Context {
     int32_t *d_tok_ = nullptr, *d_pos_ = nullptr, *d_seq_ = nullptr, *d_cell_ = nullptr, *d_nkv_ = nullptr, *d_outrow_ = nullptr;
     uint64_t *d_seqmask_ = nullptr;
     uint8_t *h_stage_ = nullptr;    // pinned
-    size_t stage_bytes_ = 0, stage_used_ = 0;             // of the block; of the batch in it
-    bool stage_in_setup_ = false;                         // the set-up launch of a single-token step fetches the block itself (no copy in front of its graph)
+    size_t stage_bytes_ = 0;
+    StepBlock step_block_{};                              // a single-token step's block: an argument of its set-up launch, so nothing of a queued step lies in host memory
+    bool one_token_ = false, setup_launched_ = false;     // this batch is such a step; its set-up went out in front of its graph
+    bool stage_pending_ = false;                          // copies out of pinned memory since stage_event_ was last waited for
+    hipEvent_t step_done_[2] = {nullptr, nullptr};        // the last two single-token steps: a third is not queued behind them
+    int step_turn_ = 0;
+    hipError_t launch_setup(int T, bool mega);
     uint8_t *d_stage_ = nullptr;
     hipEvent_t stage_event_ = nullptr;
     // activations
