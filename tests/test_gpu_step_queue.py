@@ -65,3 +65,21 @@ def test_a_step_is_queued_behind_unfinished_work(pkg, model):
         share.append((t1 - t0) / (time.perf_counter() - t0))
     assert min(share[1:]) < 0.5, share                             # (the first pass captures the step's graph)
     c.close()
+
+
+@pytest.mark.parametrize("n_seq", [1, 2])
+def test_first_step_of_a_bucket_and_its_replays(pkg, model, n_seq):
+    """A bucket's first step runs by launches, later ones by the graph that was captured behind it: the same token at the same place gives the same row, in the bucket of the
+    first 256 cells and in the next."""
+    c = pkg.Context(model, n_ctx=1024, n_batch=512, n_ubatch=512, n_seq_max=n_seq)
+    rng = np.random.default_rng(8)
+    for past in (5, 300):
+        c.kv_clear()
+        assert c.decode(rng.integers(0, model.n_vocab, past), np.arange(past)) == 0
+        rows = []
+        for _ in range(4):
+            assert c.decode([17], [past]) == 0
+            rows.append(c.logits())
+            c.kv_seq_rm(0, past, -1)
+        assert all(np.array_equal(rows[0], r) for r in rows[1:])
+    c.close()
