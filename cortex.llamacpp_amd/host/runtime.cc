@@ -1343,7 +1343,7 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
     const auto f16_few = [&](const DevTensor &w, int rows, int K) {
         return w.type == T_F16 && w.n_expert == 1 && mmf16_few_applicable(rows, K, T) && ((uintptr_t)w.data & 15) == 0;
     };
-    const bool packed = E == H * D && G == H && [&] {
+    const bool packed = E == H * D && G == H && E <= 2 * FF && [&] {       // (the f16 rows, E halves a token, lie in ffn_u_, FF floats a token)
         for (const LayerWeights &L : model->layers)
             if (!f16_few(L.wqkv, 3 * E, E) || !f16_few(L.wo, E, E) || !f16_few(L.gate, FF, E) || !f16_few(L.up, FF, E) || !f16_few(L.down, E, FF)) return false;
         return true;
