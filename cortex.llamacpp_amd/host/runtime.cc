@@ -1100,6 +1100,8 @@ static bool store_fuse_enabled() {
     static const bool env_off = getenv("MI355_ATTN_STORE_FUSE") && getenv("MI355_ATTN_STORE_FUSE")[0] == '0';
     return g_store_fuse && !env_off;
 }
+static bool g_late_sums = true;
+void set_late_sums(bool on) { g_late_sums = on; }
 static bool g_rope_fast = true;
 void set_rope_fast(bool on) { g_rope_fast = on; }
 void set_decode_mega(bool on) { g_decode_mega = on ? 1 : 0; }
@@ -1468,7 +1470,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
 
     const bool tp = hp.tp_exchange;
     // a prompt's K-split attn_output / ffn_down leaves its partial sums to the norm that reads x_ next (x_parts of them in mmq_ws_; x_ holds the residual till then)
-    const bool late_sum = rmsnorm_takes_parts(E, T) && !tp;
+    const bool late_sum = g_late_sums && rmsnorm_takes_parts(E, T) && !tp;
     int x_parts = 1;
     for (int il = 0; il < hp.n_layer; il++) {
         const LayerWeights &L = model->layers[(size_t)il];
@@ -1554,7 +1556,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         const bool rope_fast_ok = rope_fast && g_rope_fast && rope_cs_ && rope_q_kv_store_fast_applicable(H, G, D, cp.type_k, cp.type_v, ra);
         int qkv_parts = 1;
         if (!(engine && il > 0) && !qkv_in_attn)
-            HIP_TRY(linear_multi(ws, outs, 3, aq_e_, xn_, T, rope_fast_ok && !decode_attn && !(L.bq.valid() || L.bk.valid() || L.bv.valid()) ? &qkv_parts : nullptr));
+            HIP_TRY(linear_multi(ws, outs, 3, aq_e_, xn_, T, g_late_sums && rope_fast_ok && !decode_attn && !(L.bq.valid() || L.bk.valid() || L.bv.valid()) ? &qkv_parts : nullptr));
         pending_fuse_ = Fuse();
         if (!qkv_in_attn && (L.bq.valid() || L.bk.valid() || L.bv.valid()))       // qwen2-style attention biases: all T rows of the three projections in one launch
             HIP_TRY(launch_add_qkv_bias(q_, k_, v_, L.bq.valid() ? (const float *)L.bq.data : nullptr, L.bk.valid() ? (const float *)L.bk.data : nullptr,

@@ -1034,11 +1034,12 @@ def test_embeddings_match_oracle_hidden_state(be, pkg, tmp_models):
     c.close(); m.close(); oc.close(); om.close()
 
 
-@pytest.mark.parametrize("ftype,kv,n_prompt", [("q4_k_m", "q8_0", 300), ("q5_k_m", "q8_0", 96), ("q8_0", "q8_0", 40)])
+@pytest.mark.parametrize("ftype,kv,n_prompt", [("q4_k_m", "q8_0", 300), ("q5_k_m", "q8_0", 96), ("q8_0", "q8_0", 40),
+                                               ("q4_k_m", "q8_0", 20), ("q5_k_m", "q8_0", 31), ("q6_k", "q8_0", 16)])
 def test_moe_prompt_batches_grouped_by_expert(be, pkg, tmp_models, ftype, kv, n_prompt):
     """ggml_mul_mat_id on a prompt batch (build_moe_ffn): the (token, rank) pairs are grouped by expert and every expert
     runs ONE batched contraction over its tokens (300 tokens / 8 experts top-2: ~75 rows per expert -> the MFMA kernels;
-    96 -> the K-split small-batch kernel; Q8_0 experts -> the tiled mat-vec).  Checked against the CPU oracle per layer
+    to 31 tokens -> a launch an expert: the K-split small-batch kernel from three rows, the mat-vec below; Q8_0 experts -> the tiled mat-vec).  Checked against the CPU oracle per layer
     and on the logits, and against the per-(token, expert) mat-vec loop the single-token steps use (same integer sums)."""
     path = make(pkg, tmp_models, "tiny-moe", ftype)
     rng = np.random.default_rng(9)

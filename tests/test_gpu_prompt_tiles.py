@@ -70,3 +70,35 @@ def test_partial_sums_left_to_the_norm(pkg, tmp_path, cfg, n):
         c.close()
     m.close()
     assert np.isfinite(rows[0]).all() and np.abs(rows[0] - rows[1]).max() <= 3e-2 * np.abs(rows[1]).max()
+
+
+@pytest.mark.parametrize("parts", [2, 3, 4])
+@pytest.mark.parametrize("cfg,kv,n_rot", [("tiny-8b-attn-2l", 8, 128), ("tiny-7b-attn-2l", 1, 128), ("tiny-8b-attn-2l", 1, 64)])
+def test_partial_sums_by_whichever_launch(be, pkg, tmp_path, cfg, kv, n_rot, parts):  # noqa: F811
+    """Two, three and four parts of Q | K | V, attn_output and ffn_down, added by the rope + cache store and the norms or by a launch of their own: the same order, so the same
+    bits - in the prompt's last row and, through the cache, in a step's behind it.  q8_0 and f16 caches, kv heads as many as query heads, half a head rotated."""
+    path = tmp_path / "m.gguf"
+    pkg.gguf_synth.write_synthetic_llama(str(path), cfg, "q4_k_m", seed=5, with_vocab=False)
+    raw = bytearray(path.read_bytes())
+    at = raw.index(b"llama.rope.dimension_count") + len(b"llama.rope.dimension_count")
+    assert int.from_bytes(raw[at:at + 4], "little") == 4 and int.from_bytes(raw[at + 4:at + 8], "little") == 128       # (a u32, the head size)
+    raw[at + 4:at + 8] = n_rot.to_bytes(4, "little")
+    path.write_bytes(raw)
+    m = pkg.Model(str(path))
+    toks = np.random.default_rng(parts).integers(0, m.n_vocab, 300)
+    rows = []
+    be.set_option("mmq_split", parts)
+    try:
+        for late in (1, 0):
+            be.set_option("late_sums", late)
+            c = pkg.Context(m, n_ctx=512, n_batch=512, n_ubatch=512, type_k=kv, type_v=kv)
+            assert c.decode(toks, np.arange(300)) == 0
+            rows.append([c.logits()])
+            assert c.decode([7], [300]) == 0
+            rows[-1].append(c.logits())
+            c.close()
+    finally:
+        be.set_option("mmq_split", 0)
+        be.set_option("late_sums", 1)
+    m.close()
+    assert np.isfinite(rows[0]).all() and np.array_equal(rows[0], rows[1])
