@@ -136,12 +136,14 @@ __global__ void step_setup_kernel(const int32_t *tok_pos, int T, RopeArgs ra, fl
 }
 // ... and the embedding rows of the batch's tokens (ggml_get_rows of token_embd, dequantised: get_rows_kernel of misc.hip) in the same launch: grid
 // (row parts, tokens) of 256 threads; the first T * n_rot / 2 threads of the grid also fill the cos / sin table, block (0, 0) the cell metadata
-// ONE: a single token, whose scalars are arguments (v) and go to `stage` for the launches behind
-template <bool ONE>
+// MODE 1: a single token, whose scalars are arguments (v) and go to `stage` for the launches behind; 2: they lie in pinned memory
+template <int MODE>
 __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *tok_pos, int T, RopeArgs ra, float theta_scale, float *cs_out, int32_t *cell_pos,
                                                                uint64_t *cell_seq, const int32_t *tok_cell, const uint64_t *tok_seqmask, unsigned *zero_word,
                                                                unsigned *epoch_word, int type, const uint8_t *table, int K, size_t row_bytes,
-                                                               const int32_t *ids, float *dst, const StepBlock v, uint32_t *stage) {
+                                                               const int32_t *ids, float *dst, const StepBlock by_value, uint32_t *stage, const StepBlock *ring, const unsigned *turn) {
+    constexpr bool ONE = MODE != 0;
+    const StepBlock &v = MODE == 2 ? ring[*turn & 1u] : by_value;
     const int lin = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
     if (ONE && lin < 16) stage[lin] = v.w[lin];
     if (blockIdx.x == 0 && blockIdx.y == 0) {
@@ -169,16 +171,18 @@ __global__ __launch_bounds__(256) void step_setup_embed_kernel(const int32_t *to
 }
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one, void *stage) {
-    if (one && (T != 1 || !stage)) return hipErrorInvalidValue;
+                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one, void *stage, const StepBlock *ring, const unsigned *turn) {
+    if ((one || ring) && (T != 1 || !stage || (ring && !turn))) return hipErrorInvalidValue;
     const float theta_scale = powf(ra.freq_base, -2.0f / (float)ra.n_rot);
     int bx = (int)((K + 255) / 256);
     if (bx > 64) bx = 64;
     while ((long)bx * T * 256 < (long)T * (ra.n_rot >> 1)) bx++;          // (enough threads for the table: n_rot / 2 <= 256 * bx per token)
-    if (one) hipLaunchKernelGGL((step_setup_embed_kernel<true>), dim3(bx, 1), dim3(256), 0, st, nullptr, 1, ra, theta_scale, cs_out, cell_pos, cell_seq, nullptr, nullptr,
-                                zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), nullptr, dst, *one, reinterpret_cast<uint32_t *>(stage));
-    else hipLaunchKernelGGL((step_setup_embed_kernel<false>), dim3(bx, T), dim3(256), 0, st, tok_pos, T, ra, theta_scale, cs_out, cell_pos, cell_seq, tok_cell, tok_seqmask,
-                            zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst, StepBlock{}, (uint32_t *)nullptr);
+    if (ring) hipLaunchKernelGGL((step_setup_embed_kernel<2>), dim3(bx, 1), dim3(256), 0, st, nullptr, 1, ra, theta_scale, cs_out, cell_pos, cell_seq, nullptr, nullptr,
+                                 zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), nullptr, dst, StepBlock{}, reinterpret_cast<uint32_t *>(stage), ring, turn);
+    else if (one) hipLaunchKernelGGL((step_setup_embed_kernel<1>), dim3(bx, 1), dim3(256), 0, st, nullptr, 1, ra, theta_scale, cs_out, cell_pos, cell_seq, nullptr, nullptr,
+                                zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), nullptr, dst, *one, reinterpret_cast<uint32_t *>(stage), nullptr, nullptr);
+    else hipLaunchKernelGGL((step_setup_embed_kernel<0>), dim3(bx, T), dim3(256), 0, st, tok_pos, T, ra, theta_scale, cs_out, cell_pos, cell_seq, tok_cell, tok_seqmask,
+                            zero_word, epoch_word, type, table, (int)K, dev_row_bytes(type, K), ids, dst, StepBlock{}, (uint32_t *)nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,

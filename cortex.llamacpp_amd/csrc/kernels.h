@@ -222,7 +222,7 @@ hipError_t launch_get_rows(int type, const uint8_t *table_dev, int64_t K, const 
 hipError_t launch_get_rows_pair(int type, const uint8_t *table_dev, const uint8_t *table2_dev, int64_t K, const int32_t *ids, const int32_t *ids2, int n_ids, float *dst,
                                 hipStream_t st, float scale = 1.0f);
 // scratch: cap_rows * 129 words, zero-filled once: [cap_rows ticket words | cap_rows * 64 part values | cap_rows * 64 part indices]; rows <= cap_rows
-hipError_t launch_argmax_rows(const float *x, int n, int rows, int32_t *out, float *scratch, int cap_rows, hipStream_t st);
+hipError_t launch_argmax_rows(const float *x, int n, int rows, int32_t *out, float *scratch, int cap_rows, hipStream_t st, unsigned *turn = nullptr);   // turn (one row): += 1
 // ---- device-side sampling front end (reference call site common_sampler_sample, src/llama_server_context.cc:1679-1698): the k best
 // candidates of a logits row after logit_bias and the repetition / frequency / presence penalties, so that k (token, logit) pairs cross to the host
 // instead of the 513 KB row.  Order = the host sampler's (host/sampling.cc `better`): higher logit first, lower token id on ties.  Exact: the same f32
@@ -613,11 +613,12 @@ hipError_t launch_step_setup(const int32_t *tok_pos, int T, RopeArgs ra, float *
                              const uint64_t *tok_seqmask, unsigned *zero_word, hipStream_t st, unsigned *epoch_word = nullptr);
 // the staging block of a batch of one token: n_kv in word 0; token, position, sequence, cell and output row in words 4, 6, 8, 10, 12; the sequence mask in 14 and 15
 struct StepBlock { uint32_t w[16]; };
-// launch_step_setup + launch_get_rows (the batch's embedding rows, dst[T][K]) in one launch.  one (T == 1): the block travels as the launch's argument, in place of the arrays,
-// and is left at `stage` on the device
+// launch_step_setup + launch_get_rows (the batch's embedding rows, dst[T][K]) in one launch.  T == 1: the block in place of the arrays, left at `stage` on the device - either as
+// the launch's argument (one), or from pinned memory (ring), where it is the one of two whose number is *turn's parity when the launch runs
 hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, float *cs_out, int32_t *cell_pos, uint64_t *cell_seq, const int32_t *tok_cell,
                                    const uint64_t *tok_seqmask, unsigned *zero_word, unsigned *epoch_word, int type, const uint8_t *table_dev, int64_t K,
-                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one = nullptr, void *stage = nullptr);
+                                   const int32_t *ids, float *dst, hipStream_t st, const StepBlock *one = nullptr, void *stage = nullptr,
+                                   const StepBlock *ring = nullptr, const unsigned *turn = nullptr);
 hipError_t launch_rope_inplace(float *x, int T, int n_head, int D, const int32_t *tok_pos, RopeArgs ra, hipStream_t st);
 
 struct AttnArgs {

@@ -154,7 +154,7 @@ __device__ __forceinline__ void argmax_block_reduce(float &best, int &idx, float
 }
 // One launch: every workgroup reduces its part, takes a ticket on the row's counter, and the LAST arriver reduces the 64 parts (device-coherent loads
 // of what the others wrote, no cache-wide fence) and writes the winner - the second launch this replaced cost ~4.5 us of every decoded token.
-__global__ __launch_bounds__(256) void argmax_part_kernel(const float *x, int n, float *pv, int *pi, unsigned *cnt, int32_t *out) {
+__global__ __launch_bounds__(256) void argmax_part_kernel(const float *x, int n, float *pv, int *pi, unsigned *cnt, int32_t *out, unsigned *turn) {
     __shared__ float bv[4];
     __shared__ int bi[4];
     __shared__ int last_sh;
@@ -187,17 +187,20 @@ __global__ __launch_bounds__(256) void argmax_part_kernel(const float *x, int n,
         const int oi = __shfl_xor(i2, o, 64);
         if (ov > b2 || (ov == b2 && oi < i2)) { b2 = ov; i2 = oi; }
     }
-    if (tid == 0) out[row] = i2;
+    if (tid == 0) {
+        out[row] = i2;
+        if (turn) *turn = *turn + 1u;                           // (one row: one thread of the launch gets here)
+    }
 }
 // scratch: cap_rows ticket words (zero between launches) | cap_rows * 64 part values | cap_rows * 64 part indices.  The ticket words sit at the HEAD of the
 // scratch, at an address that does not depend on `rows`: behind the parts they moved with the row count, and a launch with fewer rows than its predecessor
 // found a part value of the earlier launch where its (zero) counter should be (multi-slot serving: 2 generating slots, then 1).
-hipError_t launch_argmax_rows(const float *x, int n, int rows, int32_t *out, float *scratch, int cap_rows, hipStream_t st) {
-    if (rows < 1 || rows > cap_rows) return hipErrorInvalidValue;
+hipError_t launch_argmax_rows(const float *x, int n, int rows, int32_t *out, float *scratch, int cap_rows, hipStream_t st, unsigned *turn) {
+    if (rows < 1 || rows > cap_rows || (turn && rows != 1)) return hipErrorInvalidValue;
     unsigned *cnt = reinterpret_cast<unsigned *>(scratch);
     float *pv = scratch + cap_rows;
     int *pi = reinterpret_cast<int *>(scratch + cap_rows + (size_t)cap_rows * ARGMAX_PARTS);
-    hipLaunchKernelGGL(argmax_part_kernel, dim3(ARGMAX_PARTS, rows), dim3(256), 0, st, x, n, pv, pi, cnt, out);
+    hipLaunchKernelGGL(argmax_part_kernel, dim3(ARGMAX_PARTS, rows), dim3(256), 0, st, x, n, pv, pi, cnt, out, turn);
     return hipGetLastError();
 }
 

@@ -535,10 +535,11 @@ Context::~Context() {
     }
     for (auto &ge : graphs_) (void)hipGraphExecDestroy(ge.second);
     if (stage_event_) (void)hipEventDestroy(stage_event_);
-    for (hipEvent_t ev : step_done_) if (ev) (void)hipEventDestroy(ev);
+    if (step_mark_) (void)hipEventDestroy(step_mark_);
     for (auto &pe : prof_events_) (void)hipEventDestroy(pe.second);
     for (void *p : allocs_) (void)hipFree(p);
     if (h_stage_) (void)hipHostFree(h_stage_);
+    if (h_ring_) (void)hipHostFree(h_ring_);
     if (h_cell_pos_) (void)hipHostFree(h_cell_pos_);
     if (h_cell_seq_) (void)hipHostFree(h_cell_seq_);
     if (h_logits_) (void)hipHostFree(h_logits_);
@@ -687,7 +688,7 @@ bool Context::init(std::string &err) {
     mmq_bl_ = (int8_t *)dalloc(mmq_prep_bytes((int)std::max(E, FF), prep_rows));
     // partial sums of the K-split prompt contraction: only tensors with few rows split (Q | K | V, attention output, FFN down),
     // up to four ways; tensors that do not fit fall back to an unsplit kernel
-    // A launch splits into floor(CUs / tiles) <= 4 parts of its 128 x 256 tiles (mmq.hip planes2_split), i.e. never into more than CUs tiles' worth of partial
+    // A launch splits into floor(CUs / tiles) <= 4 parts, of four super-blocks at least, of its 128 x 256 tiles (mmq.hip planes2_split), i.e. never into more than CUs tiles' worth of partial
     // sums whatever the model (33.6 MB on 256 CUs; sized by the widest tensor instead it was 335 MB per context for Llama-3-70B at n_ubatch 2048)
     mmq_ws_.bytes = std::min((size_t)4 * T * std::max<size_t>(E, (size_t)(hp.n_head + 2 * hp.n_head_kv) * D) * sizeof(float),
                              (size_t)num_cu() * 128 * 256 * sizeof(float));
@@ -709,10 +710,12 @@ bool Context::init(std::string &err) {
     if (!att_part_ || !att_counters_) { err = "attention workspace allocation failed"; return false; }
     if (hipMemset(att_counters_, 0, 64 * ATT_SYNC_STRIDE * sizeof(unsigned)) != hipSuccess) { err = "hipMemset failed"; return false; }
     d_step_serial_ = (unsigned *)dalloc(64);
+    d_turn_ = (unsigned *)dalloc(64);
+    if (hipHostMalloc((void **)&h_ring_, 2 * sizeof(StepBlock), hipHostMallocDefault) != hipSuccess) { err = "pinned alloc failed"; return false; }
     d_ao_flags_ = (unsigned *)dalloc((size_t)std::max(1, hp.n_layer) * 64 * ATT_SYNC_STRIDE * sizeof(unsigned));
     d_ao_gran_ = (unsigned long long *)dalloc(attn_out_granule_words((int)(hp.n_head * D)) * 8);
     d_qkv_gran_ = (unsigned long long *)dalloc(qkv_attn_granule_words((int)(hp.n_head * D), (int)(hp.n_head_kv * D)) * 8);
-    if (!d_step_serial_ || !d_ao_flags_ || !d_ao_gran_ || !d_qkv_gran_) { err = "step serial / flag allocation failed"; return false; }
+    if (!d_step_serial_ || !d_turn_ || !d_ao_flags_ || !d_ao_gran_ || !d_qkv_gran_) { err = "step serial / flag allocation failed"; return false; }
     d_argmax_ = (int32_t *)dalloc(T * 4);
     argmax_scratch_ = (float *)dalloc(T * 129 * 4);     // T ticket words at the head, then per row 64 part values and 64 part indices (zero-filled: dalloc)
     rope_cs_ = (float *)dalloc(T * (size_t)hp.n_rot * 4);
@@ -1425,7 +1428,8 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
 
 hipError_t Context::launch_setup(int T, bool mega) {
     return launch_step_setup_embed(d_pos_, T, rope_args(*model, true), rope_cs_, d_cell_pos_, d_cell_seq_, d_cell_, d_seqmask_, mega ? d_mega_sync_ : nullptr, d_step_serial_,
-                                   model->tok_embd.type, model->tok_embd.data, model->hp.n_embd, d_tok_, x_, stream_, one_token_ ? &step_block_ : nullptr, d_stage_);
+                                   model->tok_embd.type, model->tok_embd.data, model->hp.n_embd, d_tok_, x_, stream_, one_token_ ? &step_block_ : nullptr, d_stage_,
+                                   one_token_ && capturing_ ? h_ring_ : nullptr, d_turn_);
 }
 
 hipError_t Context::run_layers(int T, int n_kv_cap) {
@@ -1459,7 +1463,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
     const bool engine = T == 1 && !mega && !profile_ && !debug_taps_ && !ub_embd_ && engine_prepare();
     last_layers_engine_ = engine;
     // cos / sin table, cell metadata and the tokens' embedding rows: one launch
-    if (!setup_launched_) HIP_TRY(launch_setup(T, mega));
+    HIP_TRY(launch_setup(T, mega));
     // an embeddings batch: the caller's rows take the place of the looked-up ones (never inside a captured graph: decode_ubatch)
     if (ub_embd_) HIP_TRY(hipMemcpyAsync(x_, ub_embd_, (size_t)T * E * sizeof(float), hipMemcpyHostToDevice, stream_));
     prof_mark("embed");
@@ -1937,7 +1941,7 @@ hipError_t Context::run_output(int n_out, int out_base) {
     for (int r0 = 0; r0 < n_out; r0 += (int)cp.n_ubatch) {
         const int nr = std::min((int)cp.n_ubatch, n_out - r0);
         // the winner goes straight into pinned host memory (visible once the stream has drained): no copy node
-        HIP_TRY(launch_argmax_rows(lg + (size_t)r0 * V, V, nr, h_argmax_ + out_base + r0, argmax_scratch_, (int)cp.n_ubatch, stream_));
+        HIP_TRY(launch_argmax_rows(lg + (size_t)r0 * V, V, nr, h_argmax_ + out_base + r0, argmax_scratch_, (int)cp.n_ubatch, stream_, one_token_ && capturing_ ? d_turn_ : nullptr));
     }
     prof_mark("argmax");
     return hipSuccess;
@@ -1961,9 +1965,12 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
 
     // stage token arrays and cell table (the pinned blocks may still be in flight from the previous micro-batch)
     one_token_ = n == 1 && !model->nvx && !model->hp.encoder;
-    setup_launched_ = false;
     if (stage_pending_ && stage_event_) { (void)hipEventSynchronize(stage_event_); stage_pending_ = false; }
-    if (one_token_ && step_done_[step_turn_]) (void)hipEventSynchronize(step_done_[step_turn_]);
+    if (one_token_ && unread_steps_ > 0) {                     // (a caller that reads its rows never gets here)
+        if (!step_mark_) (void)hipEventCreateWithFlags(&step_mark_, hipEventDisableTiming);
+        if (unread_steps_ > 1 && step_mark_) (void)hipEventSynchronize(step_mark_);
+        if (!step_mark_ || hipEventRecord(step_mark_, stream_) != hipSuccess) (void)hipStreamSynchronize(stream_);
+    }
     if (device_cells_known_)
         for (int i = 0; i < n; i++) { const int c = tcell[(size_t)i]; h_cell_pos_[c] = pos[i]; h_cell_seq_[c] = seqmask[i]; }   // the set-up launch writes these
     if (upload_cells() != 0) { last_error = "cell table upload failed"; return -1; }
@@ -2058,13 +2065,6 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             chunk_cap_ = std::min(chunk_stride_, (chunk_lmax_ + 3) & ~3);
             bucket = -chunk_cap_;                              // separate key space from the cell-count buckets
         }
-        // the step's set-up goes out by itself, its scalars as arguments: nothing of a queued step lies in host memory, and the graph behind it is the same for every step.  us a step
-        // queued unread, and read (eight layers of an 8B model; six of a 2048-column one): 435 and 449; 258 and 273.  With the block fetched from pinned memory inside the graph,
-        // where the next call had to wait for the whole step: 442 and 447; 265 and 272.  With the block copied in front of the graph: 454 and 466; 277 and 286
-        if (one_token_) {
-            if ((e = launch_setup(1, true)) != hipSuccess) { last_error = std::string("set-up launch failed: ") + hipGetErrorString(e); return -1; }
-            setup_launched_ = true;
-        }
         auto git = graphs_.find(bucket);
         graph_exec_ = git == graphs_.end() ? nullptr : git->second;
         if (!graph_exec_) {
@@ -2089,7 +2089,9 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             e = hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal);
             if (e == hipSuccess) {
                 last_error.clear();
+                capturing_ = true;
                 const hipError_t e2 = issue();
+                capturing_ = false;
                 if (e2 != hipSuccess) inner = last_error;
                 e = hipStreamEndCapture(stream_, &g);
                 if (e2 != hipSuccess) e = e2;
@@ -2111,7 +2113,13 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
                 graph_is_engine_[graph_exec_] = last_layers_engine_;
             }
         }
-        if (graph_ok && !issued) e = hipGraphLaunch(graph_exec_, stream_);
+        if (graph_ok && !issued) {
+            // us a step queued unread, and read (eight layers of an 8B model; six of a 2048-column one): 436 and 448; 259 and 272.  One block, and a wait for the whole step in front of the next call: 442
+            // and 447; 265 and 272.  The block as arguments of a launch in front of the graph: 433 and 447; 258 and 273.  Copied there: 454 and 466; 277 and 286
+            if (one_token_) h_ring_[replays_ & 1u] = step_block_;
+            e = hipGraphLaunch(graph_exec_, stream_);
+            if (one_token_ && e == hipSuccess) replays_++;
+        }
     }
     if (!graph_ok && !issued) {
         prof_begin();
@@ -2123,11 +2131,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             e = launch_rows_to_host(d_logits_ + (size_t)out_base * V, h_logits_ + (size_t)out_base * V, (size_t)n_out * V, stream_);
         prof_end();
     }
-    if (one_token_) {
-        if (!step_done_[step_turn_]) (void)hipEventCreateWithFlags(&step_done_[step_turn_], hipEventDisableTiming);
-        if (step_done_[step_turn_]) (void)hipEventRecord(step_done_[step_turn_], stream_);
-        step_turn_ ^= 1;
-    }
+    if (one_token_ && unread_steps_ < 2) unread_steps_++;
     if (e != hipSuccess) { last_error = std::string("decode failed: ") + hipGetErrorString(e) + " / " + last_error_string(); return -1; }
     if (n == 1 && (graph_ok ? graph_is_mega_[graph_exec_] : last_layers_mega_)) mega_steps++;
     if (n == 1 && (graph_ok ? graph_is_engine_[graph_exec_] : last_layers_engine_)) engine_steps++;
@@ -2257,7 +2261,7 @@ int Context::decode(int n_tokens, const int32_t *tokens, const int32_t *pos, con
     return 0;
 }
 
-void Context::synchronize() { (void)hipStreamSynchronize(stream_); fused_release(); }
+void Context::synchronize() { (void)hipStreamSynchronize(stream_); unread_steps_ = 0; fused_release(); }
 
 int Context::force_moe_ids(const int32_t *ids, int n_layer, int T, int k) {
     const HParams &hp = model->hp;
@@ -2283,6 +2287,7 @@ float *Context::logits_ith(int i) {
         if (!cp.logits_to_host &&
             (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_logits_, h_logits_, (size_t)n_out_last_ * model->hp.n_vocab, stream_) != hipSuccess)) return nullptr;
         if (hipStreamSynchronize(stream_) != hipSuccess || !mega_check() || !stream_check()) return nullptr;
+        unread_steps_ = 0;
         logits_fetched_ = true;
     }
     return h_logits_ + (size_t)out_row_of_batch_[(size_t)i] * model->hp.n_vocab;
@@ -2296,6 +2301,7 @@ float *Context::embeddings_ith(int i) {
     if (!embd_fetched_) {
         if (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_embd_, h_embd_, (size_t)n_out_last_ * E, stream_) != hipSuccess) return nullptr;
         if (hipStreamSynchronize(stream_) != hipSuccess) return nullptr;
+        unread_steps_ = 0;
         embd_fetched_ = true;
     }
     return h_embd_ + (size_t)out_row_of_batch_[(size_t)i] * E;
@@ -2306,6 +2312,7 @@ int32_t Context::argmax_ith(int i) {
     if (i < 0 || i >= (int)out_row_of_batch_.size() || out_row_of_batch_[(size_t)i] < 0) return -1;
     if (!argmax_fetched_) {
         if (hipStreamSynchronize(stream_) != hipSuccess || !mega_check() || !stream_check()) return -1;
+        unread_steps_ = 0;
         argmax_fetched_ = true;
     }
     return h_argmax_[out_row_of_batch_[(size_t)i]];
@@ -2357,6 +2364,7 @@ int Context::topk_rows(int n, const int *is, const int *ks, const TopkAdj *adjs,
     if (launch_topk_rows(d_logits_, V, n, reinterpret_cast<const int *>(d_topk_adj_ + rows_off), kmax, reinterpret_cast<const TopkAdj *>(d_topk_adj_), topk_scratch_, h_topk_,
                          stream_) != hipSuccess) { last_error = "top-k launch failed"; return -1; }
     if (hipStreamSynchronize(stream_) != hipSuccess || !mega_check() || !stream_check()) return -1;
+    unread_steps_ = 0;
     for (int r = 0; r < n; r++)
         for (int j = 0; j < ks[r]; j++) {
             const unsigned long long key = h_topk_[(size_t)r * TOPK_MAX_K + (size_t)j];

@@ -265,11 +265,16 @@ class Context {
     uint64_t *d_seqmask_ = nullptr;
     uint8_t *h_stage_ = nullptr;    // pinned
     size_t stage_bytes_ = 0;
-    StepBlock step_block_{};                              // a single-token step's block: an argument of its set-up launch, so nothing of a queued step lies in host memory
-    bool one_token_ = false, setup_launched_ = false;     // this batch is such a step; its set-up went out in front of its graph
+    // a single-token step's block: an argument of its set-up launch or, for the steps that are graph replays, one of two in pinned memory that they take in turn - the last launch
+    // of a replay moves the turn on, so a step can be queued behind another whose block has not been read yet
+    StepBlock step_block_{};
+    StepBlock *h_ring_ = nullptr;                         // pinned
+    unsigned *d_turn_ = nullptr;
+    unsigned replays_ = 0;                                // issued: what *d_turn_ will be
+    bool one_token_ = false, capturing_ = false;
     bool stage_pending_ = false;                          // copies out of pinned memory since stage_event_ was last waited for
-    hipEvent_t step_done_[2] = {nullptr, nullptr};        // the last two single-token steps: a third is not queued behind them
-    int step_turn_ = 0;
+    int unread_steps_ = 0;                                // single-token steps since the stream was last drained for a reader: a third is not queued behind two
+    hipEvent_t step_mark_ = nullptr;                      // the end of the step before the last one of them
     hipError_t launch_setup(int T, bool mega);
     uint8_t *d_stage_ = nullptr;
     hipEvent_t stage_event_ = nullptr;
