@@ -1,6 +1,6 @@
 // tools/exp_p2.hip — the prompt contraction on pre-expanded planes: per-lane planes kernel (128 x 128 tiles) against the kernel with both
 // operands through LDS (128 x 256): bit-for-bit comparison on synthetic planes and time per launch (HIP events).
-// build: tools/build_exp_p2.sh
+// build: tools/build_exp_p2.sh; usage: exp_p2 [rows] [columns] [tokens] [type] [launches] [1: all operands zero]
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -32,6 +32,7 @@ __global__ void tick_kernel(unsigned long long *o) {          // s_memtime ticks
 int main(int argc, char **argv) {
     const int N = argc > 1 ? atoi(argv[1]) : 4096, K = argc > 2 ? atoi(argv[2]) : 4096, T = argc > 3 ? atoi(argv[3]) : 2048;
     const int type = argc > 4 ? atoi(argv[4]) : T_Q4_K, reps = argc > 5 ? atoi(argv[5]) : 20;
+    const bool zeros = argc > 6 && atoi(argv[6]);
     const int nb = K / 256, n_rt = (N + 31) / 32;
     const size_t PLB = 8 * 2 * 1024 + 32 * 16;
     std::vector<uint8_t> hp((size_t)n_rt * nb * PLB);
@@ -44,9 +45,10 @@ int main(int argc, char **argv) {
             m[1] = rnd() & 0x3f3f3f3f; m[2] = (rnd() * 77u) & 0x3f3f3f3f; m[3] = 0;
         }
     }
+    if (zeros) std::fill(hp.begin(), hp.end(), 0);
     uint8_t *planes; CK(hipMalloc(&planes, hp.size())); CK(hipMemcpy(planes, hp.data(), hp.size(), hipMemcpyHostToDevice));
     std::vector<int8_t> haq((size_t)T * K); std::vector<float> had((size_t)T * nb); std::vector<int16_t> hbs((size_t)T * K / 16);
-    for (auto &v : haq) v = (int8_t)((int)(rnd() % 255) - 127);
+    for (auto &v : haq) v = zeros ? 0 : (int8_t)((int)(rnd() % 255) - 127);
     for (auto &v : had) v = 0.01f + (rnd() & 1023) * 1e-4f;
     for (size_t i = 0; i < hbs.size(); i++) { int sum = 0; for (int k = 0; k < 16; k++) sum += haq[i * 16 + k]; hbs[i] = (int16_t)sum; }
     ActQuant q{};

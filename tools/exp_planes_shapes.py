@@ -33,7 +33,7 @@ pkg = ge.load_pkg(); be = pkg.Backend()
 from test_gpu_ops import rand_weights
 from oracle_py import Q5_K
 rng = np.random.default_rng(1)
-be.set_option("mmq_planes", 1); be.set_option("mmq_lds_form", 0)
+be.set_option("mmq_planes", 1); be.set_option("mmq_lds_form", 0); be.set_option("mmq_few", 0)
 for N, K in SHAPES:
     W = rand_weights(rng, Q5_K, N * K)
     for T in TOKENS:
@@ -44,4 +44,4 @@ for N, K in SHAPES:
             for _ in range(REPS):
                 be.mul_mat(Q5_K, W, N, K, x)
         print("done", N, K, T, flush=True)
-be.set_option("mmq_lds_form", -1); be.set_option("mmq_tiles", 0); be.set_option("mmq_ksplit", 1)
+be.set_option("mmq_lds_form", -1); be.set_option("mmq_tiles", 0); be.set_option("mmq_ksplit", 1); be.set_option("mmq_few", -1)
