@@ -1033,11 +1033,12 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
 // The f32 fold of a token tile (five vector instructions an output) runs BETWEEN the MFMAs of the next tile, two outputs per K-step, on the other of two accumulator
 // pairs: a wave in an MFMA phase of its own leaves the vector unit idle, and one in a fold of its own the matrix cores.
 //
-// What bounds it: the package's power.  gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens, random operands, launches back to back): a workgroup's loop takes
-// 119 k cycles, of which the matrix cores are busy 70 k, at 1.6 GHz; with all-zero operands the same loop runs at 2.15 GHz and the launch in 137 us instead of 167; without
-// the loads in the loop (hot operands) 126.  So what counts besides the MFMAs is what is moved: this split asks the L2 for 128 KiB per super-block and CU; as two
-// 128 x 128 workgroups per CU, each with planes of its own, the same loop asked for 192 and took 4 % longer, and 16 x 16 x 64 MFMA tiles, which read twice the registers
-// per product, the same again.  Measured inside a 512-token prompt: 167 -> 153 us (before: planes through LDS as well, half a super-block per barrier, folds beside the
+// What bounds it: gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens) is 448 workgroups, two rounds of the 256 CUs of which the second is three quarters full;
+// in each a SIMD issues 2176 MFMAs of 32 cycles, so both rounds are 58 us at 2.4 GHz, 39 % of the 148 us that a launch takes back to back.  The clock is one part of the rest: with
+// all-zero operands, the same instructions and the same bytes, 127 us.  Counters over a 512-token prompt: matrix cores busy in 0.39 of the launch, 6.8 vector instructions an MFMA,
+// waves waiting in 0.38 of their cycles (for the planes, which both token halves ask the L2 for, 128 KiB per super-block and CU, or at the barrier behind the codes: not told
+// apart).  Tried, and slower: two 128 x 128 workgroups per CU, each with planes of its own (192 KiB), by 4 %; 16 x 16 x 64 MFMA tiles, which read twice the registers per product, the same.
+// Inside a 512-token prompt: 167 -> 153 us (before: planes through LDS as well, half a super-block per barrier, folds beside the
 // other half's MFMAs); the experts of an 8x7B layer (611 tokens, 1222 rows): gate | up 628 -> 548 us, down 276 -> 253, where a batch of ~150 rows is now dealt evenly to both halves.
 // Touching the super-block after the next one, to have it in the L2: 12 % slower (64 lines an instruction).
 // The block-sum ("mins") term is one v_mfma_f32_32x32x16_f16 per tile: the 16 block sums (|.| <= 2032) and the 6-bit mins are exact in f16 and their 16 products sum to
@@ -1481,11 +1482,9 @@ void mmq_set_tiles(int mt) { g_mmq_mt = mt; }
 void mmq_set_split(int n) { g_mmq_split = n; }
 void mmq_set_lds_form(int on) { g_mmq_p2 = on; }
 
-// continuous-batching decode steps and prompts up to a few hundred tokens: 3 <= T <= g_ksplit_max.  This kernel reads the GGUF
-// bytes (0.56 B / weight) and expands them in registers, the planes kernel reads 2 B / weight it need not expand: measured on the
-// 8B model the whole prompt takes 8.3 vs 13.7 ms at 128 tokens, 13.6 vs 16.7 at 256, 19.4 vs 21.0 at 384 and 22.7 vs 21.1 at 448
-// (the LDS-form planes kernel moved the crossover down - whole prompt, K-split against planes: 13.8 vs 14.1 ms at 256 tokens,
-// 17.2 vs 15.2 at 320, 19.1 vs 15.5 at 384)
+// continuous-batching decode steps and prompts up to a few hundred tokens: 3 <= T <= g_ksplit_max.  This kernel reads the GGUF bytes (0.56 B / weight) and expands them in
+// registers, once per 64 tokens; the planes kernels read 2 B / weight that they need not expand, the fewer times the more tokens there are.  Behind 256 tokens every tensor with
+// planes goes to them: a whole 8B prompt of 320 tokens took 17.2 ms here and 15.2 there, of 384 19.1 and 15.5, before the tiles became faster.
 static int g_ksplit_max = getenv("MI355_KSPLIT_MAX") ? atoi(getenv("MI355_KSPLIT_MAX")) : 256;
 bool mmq_ksplit_applicable(int type, int K, int T) {
     // from 3 tokens: the mat-vec takes 4 + 2 + 1 tokens per pass over the weights, so 3 sequences cost 4.5 ms and 6 cost 6.4 ms a step against
@@ -1495,15 +1494,14 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
 }
 
 static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool *takes);
-// Which kernel takes a 3..256-token launch is a matter of shape (tools/exp_planes_shapes.py, Q5_K, us per launch):
+// Which kernel takes a launch of 65 .. 256 tokens is a matter of shape (tools/exp_planes_shapes.py, Q5_K, us per launch; to 64 tokens mmq_few_takes chooses):
 //     N x K          T = 48     64     96    128    160    192    256
 //   14336 x 4096   K-split 29     30     56     58     83     86    103      planes 256x32: 34 34 35 37 67 68 70   128x128: 55 56 56 57 60 60 61
 //    4096 x 14336  K-split 38     39     41     43     77     80     83      planes 256x32: 99 .. 102              128x128: 166 .. 172
 // a tensor of >= 8192 rows has enough 256-row tiles for the planes kernels to fill the chip from 65 tokens on (56 x 3 workgroups) and
 // they read pre-expanded operands; a tensor of 4096 rows does not, and the K-split kernel's waves share its long K instead.
 // (pair: gate | up of a dense layer go out as ONE K-split launch of 2 n_rows rows, which holds its own against two planes launches up to
-// 128 tokens - whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128; past that the LDS-form SwiGLU launch takes the pair:
-// 13.6 -> 10.6 ms at 200 tokens, 14.1 -> 11.1 at 256.)
+// 128 tokens: whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128)
 // From 129 tokens on the other side is the 128 x 256 tiles, K split over the workgroups where the workspace allows it, and the choice is by the two launches' times.  Both are
 // whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us, Q4_K; Q6_K costs the K-split kernel up to a quarter more): K-split, 32 rows x 64 tokens,
 // a wave's ceil(nb / 8) super-blocks of 4.3 and 3.5; tiles, the part's super-blocks of 3.0 (to 160 tokens) or 3.8 and 9, and 4 more where the parts' sum is a launch of its own.

@@ -14,8 +14,8 @@
 //     128-byte line is asked for by four or five requests: gate | up of an 8B layer took 29 us that way.
 //   * The activations come as operand blocks laid out by the quantiser (ActQuant::qf).  Read from rows of K bytes instead, sixteen lanes hit sixteen lines a power
 //     of two apart: 34 us at 4 tokens, 43 at 16.  A wave meets the same super-blocks in every tile: up to 4096 columns and 32 tokens they stay in registers.
-//   * The eight partial sums of an output are added in wave order through LDS, so results do not depend on timing - and they are the sums the 65 .. 256 token
-//     kernel (mmq.hip) makes, bit for bit: an integer per super-block, the same fold, the same order.
+//   * The eight partial sums of an output are added in wave order through LDS, so results do not depend on timing - and they are the sums the K-split
+//     kernel of mmq.hip makes, bit for bit: an integer per super-block, the same fold, the same order.
 #include <algorithm>
 
 #include "kernels.h"
