@@ -303,7 +303,7 @@ MI355_API void mi355_engine_set_log_callback(mi355_engine *e, mi355_log_callback
  * kernels the other T ranges use), "mmq_few" (which of the small-batch kernels takes 3 <= T <= 64: 1 csrc/mmq_few.hip, 0 the K-split kernel of csrc/mmq.hip,
  * -1, the default: by shape); and of contexts created afterwards: "decode_mega" (1: single-token steps of a dense
  * K-quant model with Llama-3-8B's layer geometry run every layer in one launch; 0, the default: one launch per operation
- * — both produce the same bits; the single launch measured slower, see DESIGN.md); "late_sums" (0: the partial sums of a K-split prompt
+ * — both produce the same bits; the single launch measured slower); "late_sums" (0: the partial sums of a K-split prompt
  * contraction are added by a launch of their own, 1: by the norm or the rope + cache store that follows; the same bits); "moe_group_min" (batches of at least
  * this many tokens run a mixture-of-experts feed-forward grouped by expert, default 8; smaller ones loop over (token,
  * expert) with the mat-vec); "tp_null_group" (measurement aid: the process becomes rank 0 of a row-split group of `value`
