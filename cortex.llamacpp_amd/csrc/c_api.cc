@@ -44,6 +44,7 @@ struct mi355_context {
 
 static thread_local std::string t_err;
 static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1, g_op_mmq_few = -1;
+int g_op_attn_cols = 0;            // 0: the call's own kernel
 static bool g_backend_ok = false;
 
 static void fail(const std::string &s) { t_err = s; }
@@ -771,7 +772,11 @@ int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t
     a.pf_splits = flash_attn_prefill_splits((int)T, H, G, D, n_cells);
     DevBuf part(flash_attn_workspace_floats((int)T, H, D, std::max(a.splits, a.pf_splits)) * 4);
     a.part = part.as<float>();
-    hipError_t e = launch_flash_attn(a, nullptr);
+    const bool cols = g_op_attn_cols > 0;
+    if (cols && !flash_attn_cols_applicable(a)) { fail("attn_cols: no form for this call"); return MI355_ERR_ARG; }
+    DevBuf cpart(cols ? flash_attn_workspace_floats((int)T, H, D, g_op_attn_cols) * 4 : 16);
+    if (cols) { a.part = cpart.as<float>(); a.pf_splits = g_op_attn_cols; }
+    hipError_t e = cols ? launch_flash_attn_cols(a, nullptr) : launch_flash_attn(a, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) return hip_fail(e, "flash_attn");
     return dout.down(out, (size_t)T * H * D * 4) ? MI355_OK : MI355_ERR_HIP;
@@ -906,6 +911,7 @@ int mi355_debug_set_option(const char *name, int32_t value) {
     if (!strcmp(name, "mmq_ksplit")) { g_op_mmq_ksplit = value != 0; return MI355_OK; }
     if (!strcmp(name, "mmq_few")) { g_op_mmq_few = value; return MI355_OK; }
     if (!strcmp(name, "attn_store_fuse")) { set_attn_store_fuse(value != 0); return MI355_OK; }
+    if (!strcmp(name, "attn_cols")) { g_op_attn_cols = value < 0 || value > 64 ? 0 : value; return MI355_OK; }     // mi355_op_flash_attn: attn_cols.hip with so many shares of the keys
     if (!strcmp(name, "late_sums")) { set_late_sums(value != 0); return MI355_OK; }
     if (!strcmp(name, "rope_fast")) { set_rope_fast(value != 0); return MI355_OK; }
     if (!strcmp(name, "decode_mega") || !strcmp(name, "decode_engine")) {

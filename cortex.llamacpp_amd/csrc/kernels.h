@@ -645,6 +645,9 @@ struct AttnArgs {
     const ActQuant *out_q;     // nullable: also quantise the merged rows (for attn_output)
     bool out_q8k, out_q80;
     int8_t *out_bh = nullptr, *out_bl = nullptr;   // nullable (with out_q, Q8_K): the block sums also as the int8 planes the MFMA kernels take (launch_mmq_prep's)
+    // a batch of one sequence: the 64-cell chunks that hold its cells; nullptr = every chunk of the scanned range
+    const int32_t *chunks = nullptr;
+    int n_chunks = 0;
 };
 hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st);
 // parity mode for an f16 K / V cache: the reference CPU path's cell-by-cell arithmetic with V accumulated in fp16 (attn.hip); 1 / 0, -1 = MI355_FA_V_ACC=f16
@@ -654,6 +657,11 @@ bool fa_v_acc_f16_enabled();
 bool flash_attn_prefill_applicable(const AttnArgs &a);
 int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max);
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st);
+// a short batch of one sequence, a short text through the encoder: the same in another split of the work (attn_cols.hip); pf_splits = flash_attn_cols_splits
+bool flash_attn_cols_applicable(const AttnArgs &a);
+bool flash_attn_cols_takes(const AttnArgs &a, bool one_token_kernel);      // one_token_kernel: the batch of a decoder, which has kernels for one token at a time
+int flash_attn_cols_splits(const AttnArgs &a);
+hipError_t launch_flash_attn_cols(const AttnArgs &a, hipStream_t st);
 // merge of [T][H][splits][D+2] partial records into a.out (+ quantised rows when a.out_q): attn.hip
 hipError_t launch_flash_attn_combine(const AttnArgs &a, int splits, hipStream_t st);
 // decode-step variants (attn.hip): single round trip per workgroup; q passed UN-rotated (rope fused), NORM rope, D = 128

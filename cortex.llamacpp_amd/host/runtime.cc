@@ -1389,9 +1389,10 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
         aa.n_kv_dev = d_nkv_; aa.n_kv_max = n_kv_max; aa.scale = kq_scale; aa.part = att_part_;
         aa.out_q = nullptr; aa.out_q8k = false; aa.out_q80 = false;
         aa.splits = att_splits_;
-        aa.pf_splits = flash_attn_prefill_splits(T, H, G, D, n_kv_max);
+        const bool cols = !(fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16) && flash_attn_cols_takes(aa, false);
+        aa.pf_splits = cols ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(T, H, G, D, n_kv_max);
         while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
-        HIP_TRY(launch_flash_attn(aa, stream_));
+        HIP_TRY(cols ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_));
         prof_mark("attn");
         if (packed) {
             HIP_TRY(launch_mmf16_few(L.wo.data, E, E, att_, false, T, xn_, x_, L.bo.valid() ? (const float *)L.bo.data : nullptr, stream_));   // + bias, + the layer input
@@ -1499,7 +1500,10 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         bool fused_step = false, attn_out_done = false;
         // (parity mode for an f16 cache: the generic launch below dispatches to the cell-by-cell kernel with fp16 V accumulation)
         const bool v16 = fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16;
-        const bool decode_attn = !v16 && flash_attn_decode_applicable(aa, ra);
+        // a batch of one sequence: (token, head) pairs as columns of one product against its keys (attn_cols.hip)
+        const bool cols = attn_cols_;
+        if (cols) { aa.chunks = d_chunks_; aa.n_chunks = chunk_lmax_; }
+        const bool decode_attn = !v16 && !cols && flash_attn_decode_applicable(aa, ra);
         if (decode_attn) {
             aa.splits = flash_attn_decode_splits(n_kv_max);
             if (chunk_lmax_ > 0) {                             // per-token chunk lists (decode_ubatch): batched steps, or regions in use
@@ -1598,9 +1602,9 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             // (splits balance the causal tiles of ONE long sequence: sized by what a query of this batch can see - its position + 1 -
             // not by the cache's high-water mark: 32 sequences of 50-token prompts in a 32000-cell cache need none, and every
             // extra workgroup would scan the whole cell table)
-            aa.pf_splits = flash_attn_prefill_splits(T, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
+            aa.pf_splits = cols ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(T, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
             while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
-            HIP_TRY(launch_flash_attn(aa, stream_));
+            HIP_TRY(cols ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_));
         }
         prof_mark("attn");
         if (o_pl) prep_written(aq_o_, (int)L.wo.K, T);          // the attention just re-quantised its output, planes included
@@ -2007,30 +2011,42 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         }
     }
     bool lists_usable = false;                                 // only the split-per-chunk attention kernels walk the lists
-    if (!model->nvx) {
+    attn_cols_ = false;                                        // every token of one and the same sequence: one list, and attn_cols.hip where it has a form for the batch
+    AttnArgs aa{};
+    if (!model->nvx && !model->hp.encoder) {
         const HParams &hp = model->hp;
         RopeArgs ra = rope_args(*model, false);
-        AttnArgs aa{};
-        aa.T = n; aa.H = hp.n_head; aa.G = hp.n_head_kv; aa.D = hp.head_dim; aa.n_kv_max = n_kv_; aa.type_k = cp.type_k; aa.type_v = cp.type_v;
+        aa.T = n; aa.H = hp.n_head; aa.G = hp.n_head_kv; aa.D = hp.head_dim; aa.n_ctx = (int)cp.n_ctx; aa.n_kv_max = n_kv_; aa.type_k = cp.type_k; aa.type_v = cp.type_v;
         lists_usable = n <= 64 && flash_attn_decode_applicable(aa, ra) && kv_store_fast_applicable(aa.G, aa.D, cp.type_k, cp.type_v, ra);
+        attn_cols_ = n >= 2 && seqmask[0] != 0 && (seqmask[0] & (seqmask[0] - 1)) == 0 && std::all_of(seqmask, seqmask + n, [&](uint64_t m) { return m == seqmask[0]; }) &&
+                     !(fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16);
     }
-    if ((n >= 2 || cp.n_seq_max > 1) && lists_usable) {
+    if (attn_cols_ || ((n >= 2 || cp.n_seq_max > 1) && lists_usable)) {
         const int nch = (n_kv_ + 63) / 64;
         std::vector<uint64_t> seq_of_chunk((size_t)nch, 0ull);
         for (int i = 0; i < n_kv_ && i < (int)cells_.size(); i++)
             if (cells_[(size_t)i].pos >= 0) seq_of_chunk[(size_t)(i >> 6)] |= cells_[(size_t)i].seqs;
         int32_t *cnt = h_chunks_ + (size_t)64 * chunk_stride_;
-        for (int t = 0; t < n; t++) {
+        for (int t = 0; t < (lists_usable ? n : 1); t++) {
             int32_t *lst = h_chunks_ + (size_t)t * chunk_stride_;
             int c = 0;
             const uint64_t bit = 1ull << (seq[t] & 63);
             for (int ch = 0; ch < nch; ch++) if (seq_of_chunk[(size_t)ch] & bit) lst[c++] = ch;
             cnt[t] = c;
             chunk_lmax_ = std::max(chunk_lmax_, c);
+            if (attn_cols_) {                                  // (by what the sequence holds, wherever its cells are: a conversation's sums do not depend on its neighbours)
+                aa.chunks = d_chunks_; aa.n_chunks = c;
+                attn_cols_ = c > 0 && flash_attn_cols_takes(aa, true);
+                if (attn_cols_) break;
+            }
         }
         if (chunk_lmax_ < 1) chunk_lmax_ = 1;
-        stage_pending_ = true;
-        if (hipMemcpyAsync(d_chunks_, h_chunks_, (size_t)64 * (chunk_stride_ + 1) * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "chunk list upload failed"; return -1; }
+        const size_t words = attn_cols_ ? (size_t)chunk_lmax_ : (size_t)64 * (chunk_stride_ + 1);
+        if (!attn_cols_ && !lists_usable) chunk_lmax_ = 0;     // (a long batch for the prompt kernel: no lists)
+        else {
+            stage_pending_ = true;
+            if (hipMemcpyAsync(d_chunks_, h_chunks_, words * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "chunk list upload failed"; return -1; }
+        }
     }
     // rocprofv3 --pmc does not keep copy-engine transfers ordered with the kernels it serialises (observed: kernels reading
     // the previous step's token / position block); MI355_PROFILER_SAFE=1 drains the stream around the transfers

@@ -303,6 +303,7 @@ class Context {
     const int8_t *bh_over_ = nullptr, *bl_over_ = nullptr;   // linear(): block-sum planes prepared by the caller for a slice of a larger batch
     float *att_part_ = nullptr;
     size_t att_part_floats_ = 0;
+    bool attn_cols_ = false;                         // the micro-batch being decoded is of one sequence and goes through attn_cols.hip; its chunk list is the first
     int cur_max_pos_ = 0;                            // largest position of the micro-batch being decoded
     float *d_embd_ = nullptr, *h_embd_ = nullptr;   // [n_ubatch][n_embd], embeddings mode
     bool embd_fetched_ = false, last_was_embd_ = false;

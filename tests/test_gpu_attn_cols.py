@@ -1,0 +1,89 @@
+"""Attention of short batches of one sequence (csrc/attn_cols.hip): (token, head) pairs as the columns of 32-wide tiles, waves and workgroups sharing the keys."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle_py as oq
+from test_gpu_ops import F16, Q8_0, be  # noqa: F401
+from test_oracle_encoder import bert_forward_f64
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tkv", [Q8_0, F16])
+@pytest.mark.parametrize("H,G,D,n_cells,T,shares", [
+    (8, 8, 128, 1, 1, 1), (8, 2, 128, 32, 8, 1), (8, 2, 128, 33, 9, 1),         # one cell; a full tile and chunk; one column tile more, a chunk of one cell
+    (32, 8, 128, 129, 5, 1), (4, 4, 64, 300, 33, 1), (32, 4, 64, 257, 3, 1),    # four chunks a workgroup and more than that; eight heads a group
+    (6, 2, 128, 70, 21, 1), (14, 2, 128, 200, 11, 3), (24, 8, 64, 90, 7, 1),    # groups whose heads do not divide a tile
+    (8, 2, 128, 300, 40, 2), (32, 8, 128, 700, 37, 6), (12, 12, 64, 1000, 64, 5), (4, 2, 64, 100, 50, 4),    # shares, some with fewer chunks than waves
+])
+def test_against_the_oracle(be, tkv, H, G, D, n_cells, T, shares):  # noqa: F811
+    """Holes in the cache, a query that sees one cell, ragged tiles and chunks.  q8_0: the scores' integers are exact; f16: the CPU's sums of V are made in f32 for the comparison.
+    What differs is the order of f32 sums over D and over the cells and the device's exp2: 2e-5 of the largest output, as for the prompt kernel."""
+    rng = np.random.default_rng(H * 1000 + n_cells + T)
+    kf = rng.standard_normal((n_cells, G * D)).astype(np.float32)
+    vf = (rng.standard_normal((n_cells, G * D)) * rng.uniform(0.2, 3.0, (n_cells, 1))).astype(np.float32)
+    kc, vc = np.stack([oq.quantize(tkv, r) for r in kf]), np.stack([oq.quantize(tkv, r) for r in vf])
+    cell_pos = np.arange(n_cells, dtype=np.int32)
+    cell_pos[rng.random(n_cells) < 0.1] = -1
+    cell_pos[0] = 0
+    q_pos = np.sort(rng.integers(0, n_cells, T)).astype(np.int32)
+    q_pos[0], q_pos[-1] = 0, n_cells - 1
+    q = rng.standard_normal((T, H, D)).astype(np.float32)
+    scale = 1 / np.sqrt(D)
+    be.set_option("attn_cols", shares)
+    try:
+        out = be.flash_attn(q, H, G, D, tkv, kc, tkv, vc, cell_pos, q_pos, scale)
+    finally:
+        be.set_option("attn_cols", 0)
+    oq.set_fa_v_acc_f32(1 if tkv == F16 else 0)
+    try:
+        for i in range(T):
+            cells = np.nonzero((cell_pos >= 0) & (cell_pos <= q_pos[i]))[0].astype(np.int32)
+            ref = oq.flash_attn(q[i], H, G, D, tkv, kc, tkv, vc, cells, scale)
+            assert np.abs(out[i] - ref).max() <= 2e-5 * max(1.0, float(np.abs(ref).max())), (i, np.abs(out[i] - ref).max())
+    finally:
+        oq.set_fa_v_acc_f32(0)
+
+
+@pytest.mark.parametrize("kv", [1, 8])
+@pytest.mark.parametrize("past,n", [(0, 2), (70, 21), (900, 5), (300, 150)])
+def test_a_turn_among_other_conversations(pkg, tmp_path, kv, past, n):
+    """A conversation alone, and with its cells dealt out among two others' (chunks of its list that hold their cells, chunks left out): the same sums over the same cells in other
+    chunks.  f16 weights, so that only a q8_0 cache rounds in between; a logit's share of a flipped code is below 1e-3 of the largest."""
+    path = str(tmp_path / "m.gguf")
+    cfg = dataclasses.replace(pkg.gguf_synth.CONFIGS["tinyllama-1.1b"], n_layer=2, n_vocab=900)
+    pkg.gguf_synth.write_synthetic_llama(path, cfg, "f16", seed=4, with_vocab=False)
+    m = pkg.Model(path)
+    rng = np.random.default_rng(past + n)
+    talk, other = rng.integers(3, 900, past + n), rng.integers(3, 900, 2500)
+    out = []
+    for alone in (True, False):
+        c = pkg.Context(m, n_ctx=4096, n_batch=512, n_ubatch=512, n_seq_max=3, type_k=kv, type_v=kv)
+        for i in range(0, past, 45):
+            part = talk[i:min(past, i + 45)]
+            assert c.decode(part, np.arange(i, i + part.size), 1) == 0
+            for s in (() if alone else (0, 2)):
+                assert c.decode(other[i:i + 45], np.arange(i, i + 45), s) == 0
+        assert c.decode(talk[past:], np.arange(past, past + n), 1) == 0
+        out.append(c.logits().copy())
+        c.close()
+    m.close()
+    assert np.abs(out[0] - out[1]).max() <= 1e-3 * np.abs(out[0]).max()
+
+
+@pytest.mark.parametrize("n", [5, 40, 200])
+def test_texts_of_two_sequences_in_one_batch(pkg, tmp_path, n):
+    """The encoder with two texts interleaved token by token: tiles whose columns see different cells.  Tolerance as in test_gpu_encoder_few."""
+    path = str(tmp_path / "m.gguf")
+    pkg.gguf_synth.write_synthetic_llama(path, "nomic-embed-2l", "f16", seed=4, with_vocab=False)
+    m = pkg.Model(path)
+    c = pkg.Context(m, n_ctx=4096, n_batch=2048, n_ubatch=2048, n_seq_max=2)
+    toks = np.random.default_rng(n).integers(5, m.n_vocab, (n, 2))
+    assert c.decode(toks.reshape(-1), np.repeat(np.arange(n), 2), [0, 1] * n, np.ones(2 * n, np.int8)) == 0
+    got = np.stack([c.embeddings(i) for i in range(2 * n)]).astype(np.float64).reshape(n, 2, -1)
+    for s in (0, 1):
+        ref = bert_forward_f64(path, toks[:, s], np.arange(n))[-1]
+        assert np.linalg.norm(got[:, s] - ref) / np.linalg.norm(ref) <= 1.6e-3
+    c.close(); m.close()
