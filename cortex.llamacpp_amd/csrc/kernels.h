@@ -179,6 +179,12 @@ hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, 
 // mmq_few.hip: 3 .. 64 tokens of the same, bit for bit; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
 bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu);
 hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);
+// the same as the output head: 3 .. HEAD_MAX_T rows of logits are stored to `host` too ([T][ld_out] of pinned memory; nullable) while the weights stream, and each row's arg-max
+// (the lowest index of equals) to win[t].  scratch: mmq_few_head_scratch() words, zero before the first launch
+constexpr int HEAD_MAX_T = 32;
+size_t mmq_few_head_scratch();
+bool mmq_few_head_takes(int type, int K, int T, const ActQuant &q);
+hipError_t launch_mmq_few_head(const MMQSeg &seg, int K, int T, const ActQuant &q, float *host, float *scratch, int32_t *win, hipStream_t st);
 size_t mmq_prep_bytes(int K, int T);                       // bytes of each of the two block-sum planes
 hipError_t launch_mmq_prep(const ActQuant &q, int K, int T, int8_t *bh, int8_t *bl, hipStream_t st);
 hipError_t launch_mmq(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q,

@@ -128,6 +128,11 @@ struct FewArgs {
     MMQSeg seg[3];
     int n_seg, K, T;
     const uint8_t *qf;
+    // the output head (launch_mmq_few_head): rows for the host, [T][ld_out]; the workgroups' best logits of each row, and whose ticket is the last
+    float *host, *best;
+    int *best_row;
+    unsigned *ticket;
+    int32_t *win;
 };
 
 // One lane's activation operands of one super-block, as the quantiser laid them out (kernels.h FEW_BLOCK): token 16 * tile + (lane & 15) as the A operand - element
@@ -238,11 +243,21 @@ template <int TYPE, int MT, int NP> constexpr int few_lds = few_stage<TYPE, NP> 
 // CN > 0: every wave has (up to) CN <= PD super-blocks of a tile and keeps their activation operands in registers across tiles.  CN = 0: any number, the operands
 // are read (from the caches) a unit ahead.
 // NP = 2: gate and up rows of one SwiGLU pair against the same activation operands.
-template <int TYPE, int MT, int NP, int PD, int CN>
+// HEAD: see mmq_few_head_kernel
+constexpr int HEAD_RUN = 4;                                  // row tiles whose results are stored to the host together, a wave's width of rows (two: 16 rows 20 us slower; eight: 4 and 16 rows 8 us)
+template <int MT> constexpr int head_lds = 2 * 16 * MT * HEAD_RUN * 64;
+template <int TYPE, int MT, int NP, int PD, int CN, bool HEAD = false>
 __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int tile, int n_blocks, uint8_t *smem, int stage_bytes) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, kq = lane >> 4;
-    const int nb = a.K >> 8, T = a.T, tiles = (sg.n_rows + 15) >> 4;
+    const int nb = a.K >> 8, T = a.T;
+    int tiles = (sg.n_rows + 15) >> 4;
+    if constexpr (HEAD) {                                    // (a run of neighbours)
+        const int b = tile, all = tiles, each = n_blocks;
+        tile = (int)((long long)all * b / each); tiles = (int)((long long)all * (b + 1) / each);
+        n_blocks = 1;
+    }
+    const int tile0 = tile;
     uint8_t *stage = smem + wave * (NP * Raw<TYPE>::LDS);
     float *part = reinterpret_cast<float *>(smem + stage_bytes);
     // token tiles are worked on two at a time (the registers of their operands); the operands of a pair that is read again stay a unit ahead
@@ -291,6 +306,18 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
         }
     };
     int set = 0;
+    // HEAD: results wait in LDS for the other tiles of their run, [run parity][token][row]; a thread's outputs are all of one token
+    float *const run = part + few_sets<MT, NP> * NW * NP * MT * 256;
+    float top = -INFINITY;
+    int top_row = 0x7fffffff;
+    auto to_host = [&](int done) {                           // the run that ends in front of `done`, behind a barrier
+        if (!a.host) return;
+        const int k0 = (done - tile0 - 1) / HEAD_RUN * HEAD_RUN, n = (done - tile0 - k0) * 16;
+        const float *const r0 = run + (k0 / HEAD_RUN & 1) * 16 * MT * (HEAD_RUN * 16);
+        const int row0 = (tile0 + k0) * 16, rows = sg.n_rows - row0 < n ? sg.n_rows - row0 : n;
+        for (int t = wave; t < T; t += NW)
+            if (lane < rows) a.host[(size_t)t * sg.ld_out + row0 + lane] = r0[t * (HEAD_RUN * 16) + lane];
+    };
     auto finish = [&](int row_tile) {
         float *ps = part + set * (NW * NP * MT * 256);
         set ^= few_sets<MT, NP> - 1;
@@ -301,6 +328,7 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
 #pragma unroll
                 for (int r = 0; r < 4; r++) ps[((wave * NP + p) * MT * 4 + t * 4 + r) * 64 + lane] = facc[p][t][r];
         __syncthreads();
+        if constexpr (HEAD) if (row_tile > tile0 && (row_tile - tile0) % HEAD_RUN == 0) to_host(row_tile);
 #pragma unroll
         for (int j = 0; j < NE; j++) {
             const int e = tid + NT * j;
@@ -314,6 +342,11 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
                 }
                 if constexpr (NP == 2) sg.out[o] = (sum / (1.0f + expf(-sum))) * sum2;
                 else sg.out[o] = sg.resid ? rv[j] + sum : sum;
+                if constexpr (HEAD) {
+                    const int k = row_tile - tile0, gt = (e >> 8) * 16 + 4 * ((e & 63) >> 4) + (e >> 6 & 3), row = row_tile * 16 + (e & 15);
+                    run[((k / HEAD_RUN & 1) * 16 * MT + gt) * (HEAD_RUN * 16) + (k % HEAD_RUN) * 16 + (e & 15)] = sum;
+                    if (sum > top || (sum == top && row < top_row)) { top = sum; top_row = row; }
+                }
             }
         }
         if constexpr (few_sets<MT, NP> == 1) __syncthreads();
@@ -359,9 +392,42 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     for (int s = 0; s < S; s += PD) {
 #pragma unroll
         for (int u = 0; u < PD; u++) {
-            if (CN > 0 ? u % (CN > 0 ? CN : 1) == 0 && s + u >= S : s + u >= S) return;
+            if (CN > 0 ? u % (CN > 0 ? CN : 1) == 0 && s + u >= S : s + u >= S) goto done;
             unit(R[u], A[CN > 0 ? u % (CN > 0 ? CN : 1) : u % PA], CN > 0 ? u % (CN > 0 ? CN : 1) : i);
             if (CN > 0 ? (u + 1) % (CN > 0 ? CN : 1) == 0 : ++i == cn) { i = 0; finish(tile); tile += n_blocks; residual(tile < tiles ? tile : 0); }
+        }
+    }
+done:
+    if constexpr (HEAD) {
+        __syncthreads();
+        if (tiles > tile0) to_host(tiles);
+        // the best of the workgroup's rows: a token's results are sixteen neighbouring lanes'
+        static_assert(NE == 1, "a thread's results are of one token");
+        const auto better = [&](float v, int r) { if (v > top || (v == top && r < top_row)) { top = v; top_row = r; } };
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) { const float v = __shfl_xor(top, o, 64); const int r = __shfl_xor(top_row, o, 64); better(v, r); }
+        const int gt = (tid >> 8) * 16 + 4 * (lane >> 4) + (tid >> 6 & 3), blocks = (int)gridDim.x;
+        if (tid < MT * 256 && (lane & 15) == 0 && gt < T) {
+            __hip_atomic_store(a.best + gt * blocks + blockIdx.x, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.best_row + gt * blocks + blockIdx.x, top_row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (the write-through stores have left before the ticket is taken)
+        int *const last = reinterpret_cast<int *>(smem);
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned t = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *last = t == (unsigned)blocks - 1u;
+            if (*last) __hip_atomic_store(a.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // re-armed for the next launch
+        }
+        __syncthreads();
+        if (!*last) return;
+        for (int t = wave; t < T; t += NW) {
+            top = -INFINITY; top_row = 0x7fffffff;
+            for (int b = lane; b < blocks; b += 64)
+                better(__hip_atomic_load(a.best + t * blocks + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __hip_atomic_load(a.best_row + t * blocks + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) { const float v = __shfl_xor(top, o, 64); const int r = __shfl_xor(top_row, o, 64); better(v, r); }
+            if (lane == 0) a.win[t] = top_row;
         }
     }
 }
@@ -383,6 +449,23 @@ __global__ __launch_bounds__(NT, 2) void mmq_few_kernel(const FewArgs a) {
         case T_Q6_K: few_body<T_Q6_K, MT, NP, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
         default: break;
     }
+}
+
+// The output head of a tick: a workgroup takes a run of neighbouring row tiles, and stores the results of HEAD_RUN of them at a time - 256 consecutive bytes a token - to the
+// host's rows while its weights stream: PCIe bounds it from a dozen rows on.  The rows' arg-max is made of what the threads hold anyway.  128256 rows of 4096 columns (Q6_K), us, here /
+// the head, the arg-max and a launch that copies the rows one behind the other: 4 tokens 110 / 99 + 10 + 38, 16 tokens 206 / 104 + 19 + 149.
+template <int TYPE, int MT, int CN>
+__global__ __launch_bounds__(NT, 2) void mmq_few_head_kernel(const FewArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, 1> + head_lds<MT>];
+    few_body<TYPE, MT, 1, 4, CN, true>(a, a.seg[0], (int)blockIdx.x, (int)gridDim.x, smem, few_stage<TYPE, 1>);
+}
+template <int TYPE>
+void few_head(const FewArgs &a, int blocks, hipStream_t st) {
+    const int cn = ((a.K >> 8) + NW - 1) / NW;
+#define GO(MT, CN) hipLaunchKernelGGL((mmq_few_head_kernel<TYPE, MT, CN>), dim3((unsigned)blocks), dim3(NT), 0, st, a)
+    if (a.T <= 16) { if (cn == 1) GO(1, 1); else if (cn == 2) GO(1, 2); else GO(1, 0); }
+    else if (cn == 1) GO(2, 1); else if (cn == 2) GO(2, 2); else GO(2, 0);
+#undef GO
 }
 
 template <int TYPE, int MT, int NP, int PD, int CN>
@@ -449,6 +532,31 @@ hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const Act
         case T_Q5_K: few_type<T_Q5_K, 1>(a, blocks, st); break;
         case T_Q6_K: few_type<T_Q6_K, 1>(a, blocks, st); break;
         default: few_type<0, 1>(a, blocks, st); break;
+    }
+    return hipGetLastError();
+}
+
+static int head_blocks(int n_rows) { return std::min((n_rows + 15) / 16, num_cu()); }
+size_t mmq_few_head_scratch() { return 1 + 2 * (size_t)HEAD_MAX_T * (size_t)num_cu(); }
+bool mmq_few_head_takes(int type, int K, int T, const ActQuant &q) {
+    return q.qf && (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K & 255) == 0 && T >= 3 && T <= HEAD_MAX_T;
+}
+hipError_t launch_mmq_few_head(const MMQSeg &seg, int K, int T, const ActQuant &q, float *host, float *scratch, int32_t *win, hipStream_t st) {
+    if (!mmq_few_head_takes(seg.type, K, T, q) || !scratch || !win || seg.resid || seg.n_rows < 1) return hipErrorInvalidValue;
+    FewArgs a{};
+    a.n_seg = 1; a.K = K; a.T = T;
+    a.qf = q.qf;
+    a.seg[0] = seg;
+    a.seg[0].tile0 = 0;
+    const int blocks = head_blocks(seg.n_rows);
+    a.host = host; a.win = win;
+    a.ticket = reinterpret_cast<unsigned *>(scratch);
+    a.best = scratch + 1;
+    a.best_row = reinterpret_cast<int *>(a.best + (size_t)HEAD_MAX_T * num_cu());
+    switch (seg.type) {
+        case T_Q4_K: few_head<T_Q4_K>(a, blocks, st); break;
+        case T_Q5_K: few_head<T_Q5_K>(a, blocks, st); break;
+        default: few_head<T_Q6_K>(a, blocks, st); break;
     }
     return hipGetLastError();
 }

@@ -879,7 +879,7 @@ hipError_t launch_mmvq(MMVQArgs a, hipStream_t st) {
         if (a.n_seg != 1 || a.T != 1) return hipErrorInvalidValue;
         const hipError_t e = launch_mmvq(a, st);
         if (e != hipSuccess) return e;
-        return hipMemcpyAsync(oh, a.seg[0].out, (size_t)a.seg[0].n_rows * 4, hipMemcpyDeviceToHost, st);
+        return launch_rows_to_host(a.seg[0].out, oh, (size_t)a.seg[0].n_rows, st);
     }
     if (fast_on && mmvq_fast_applicable(a)) return launch_mmvq_fast(a, st);
     if ((a.T == 16 || a.T == 8) && a.fuse_mode == 0) {

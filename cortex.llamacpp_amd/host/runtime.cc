@@ -718,6 +718,7 @@ bool Context::init(std::string &err) {
     if (!d_step_serial_ || !d_turn_ || !d_ao_flags_ || !d_ao_gran_ || !d_qkv_gran_) { err = "step serial / flag allocation failed"; return false; }
     d_argmax_ = (int32_t *)dalloc(T * 4);
     argmax_scratch_ = (float *)dalloc(T * 129 * 4);     // T ticket words at the head, then per row 64 part values and 64 part indices (zero-filled: dalloc)
+    head_scratch_ = (float *)dalloc(mmq_few_head_scratch() * 4);
     rope_cs_ = (float *)dalloc(T * (size_t)hp.n_rot * 4);
     chunk_stride_ = (int)((NC + 63) / 64);
     d_chunks_ = (int32_t *)dalloc((size_t)64 * (chunk_stride_ + 1) * 4);
@@ -1904,10 +1905,10 @@ hipError_t Context::run_output(int n_out, int out_base) {
         return hipSuccess;
     }
     const bool oq = is_quant(model->output.type);
-    // a single-token step whose logits row is wanted on the host: the head's launch stores it into the pinned row itself (the row crosses PCIe under the
-    // launch; a copy node behind it cost 9 - 12 us of every step, tools/host_gap.py)
+    // one logits row that is wanted on the host: the head's launch stores it into the pinned row itself (the row crosses PCIe under the launch; a copy node behind
+    // it cost 9 - 12 us of every step, tools/host_gap.py, a copying launch 10 of a prompt)
     static const bool zc_env = !(getenv("MI355_LOGITS_ZERO_COPY") && getenv("MI355_LOGITS_ZERO_COPY")[0] == '0');
-    logits_on_host_ = zc_env && oq && cur_T_ == 1 && n_out == 1 && cp.logits_to_host && !hp.tp_exchange && h_logits_ != nullptr;
+    logits_on_host_ = zc_env && oq && n_out == 1 && cp.logits_to_host && !hp.tp_exchange && h_logits_ != nullptr;
     if (oq && can_fuse(E, n_out)) {
         pending_fuse_.mode = 1; pending_fuse_.x = xo; pending_fuse_.w = (const float *)model->out_norm.data; pending_fuse_.eps = hp.eps;
     } else {
@@ -1937,6 +1938,15 @@ hipError_t Context::run_output(int n_out, int out_base) {
             HIP_TRY(hipMemcpy2DAsync(lg + (size_t)r * VL, (size_t)V * 4, tp_logits_ + (size_t)r * n_out * VL, (size_t)VL * 4, (size_t)VL * 4, (size_t)n_out,
                                      hipMemcpyDeviceToDevice, stream_));
     } else {
+        // a tick's rows: the head's launch stores them to the host and finds their arg-max (mmq_few_head_kernel)
+        if (oq && pending_fuse_.mode == 0 && mmq_few_head_takes(model->output.type, E, n_out, aq_e_) &&
+            mmq_ksplit_preferred(model->output.type, V, E, n_out, model->output.planes != nullptr, mmq_ws_, false)) {
+            logits_on_host_ = zc_env && cp.logits_to_host && h_logits_ != nullptr;
+            const MMQSeg sg{model->output.data, model->output.row_bytes, V, model->output.type, lg, V, nullptr, 0};
+            HIP_TRY(launch_mmq_few_head(sg, E, n_out, aq_e_, logits_on_host_ ? h_logits_ + (size_t)out_base * V : nullptr, head_scratch_, h_argmax_ + out_base, stream_));
+            prof_mark("lm_head");
+            return hipSuccess;
+        }
         if (logits_on_host_) pending_fuse_.out_host = h_logits_ + (size_t)out_base * V;
         HIP_TRY(linear(model->output, aq_e_, xn_, E, n_out, lg, V, nullptr, EPI_STORE));
     }
