@@ -1455,14 +1455,19 @@ bool attn_out_fused_enabled() {
 size_t attn_out_granule_words(int K) { return (size_t)(K / 256) * AO_GPB + 64; }
 void attn_out_set_error_word(unsigned *w) { (void)hipMemcpyToSymbol(HIP_SYMBOL(g_st_err_word), &w, sizeof(w)); }
 
-// chunk size the launch will use for a scan of n_kv_max cells: 64 cells while that gives every CU at most one item, 128 beyond
+// chunk size the launch will use for a scan of n_kv_max cells: 64 cells while that gives every CU at most one item, 128 beyond.  With a query head to every kv head the items are many
+// and small, and a second one on a CU waits for the whole chain of the first: the smallest chunk that needs no second, 256 where all do.  us a step, eight layers of 32 heads, f16, 128 / 192 /
+// 256 cells an item: behind 600 cells 445 453 462, 900 450 460 468, 1201 496 463 472, 1500 501 471 477, 2000 524 538 491, 3900 641 620 589 (384 and 512: 658 and 583, and 20 to 50 more to 2000)
 int attn_out_fused_chunk(const AttnArgs &a) {
     const int s64 = (a.n_kv_max + 63) / 64;
     if (a.tok_chunks) return 64;                      // (the per-token chunk lists count 64-cell chunks)
 #ifdef MI355_AO_FORCE_C
     if (MI355_AO_FORCE_C == 128 || MI355_AO_FORCE_C == 64) return (MI355_AO_FORCE_C == 64 && s64 > 64) ? 128 : MI355_AO_FORCE_C;   // (tools: A/B of the chunk size)
 #endif
-    return s64 * a.G <= num_cu() && s64 <= 64 ? 64 : 128;
+    if (s64 * a.G <= num_cu() && s64 <= 64) return 64;
+    if (a.H != a.G) return 128;
+    for (int c = 128; c < 256; c += 64) if ((a.n_kv_max + c - 1) / c * a.G <= num_cu()) return c;
+    return 256;
 }
 int attn_out_fused_splits(const AttnArgs &a) {
     const int C = attn_out_fused_chunk(a);
@@ -1573,12 +1578,13 @@ static hipError_t launch_ao(const AttnArgs &a, const float *cs_table, RopeArgs r
     } while (0)
 #define AO_K(RR, TK, TV, CC) do { if (!qf) AO_LAUNCH(RR, TK, TV, CC); else if (qf->kb == 1) QF_LAUNCH(RR, TK, TV, CC, 1); else QF_LAUNCH(RR, TK, TV, CC, 2); } while (0)
 #define AO_C(RR, TK, TV) do { if (C == 64) AO_K(RR, TK, TV, 64); else AO_K(RR, TK, TV, 128); } while (0)
+#define AO_C1(TK, TV) do { if (C == 256) AO_K(1, TK, TV, 256); else if (C == 192) AO_K(1, TK, TV, 192); else AO_C(1, TK, TV); } while (0)
 #define AO_T(RR) do { if (a.type_k == T_F16) AO_C(RR, T_F16, T_F16); else AO_C(RR, T_Q8_0, T_Q8_0); } while (0)
 #ifdef MI355_AO_DEV      // (development builds: one form only, seconds to compile)
     if (R == 4 && a.type_k == T_Q8_0 && C == 64) AO_K(4, T_Q8_0, T_Q8_0, 64); else return hipErrorInvalidValue;
 #else
     switch (R) {
-        case 1: AO_T(1); break;
+        case 1: if (a.type_k == T_F16) AO_C1(T_F16, T_F16); else AO_C1(T_Q8_0, T_Q8_0); break;
         case 2: AO_T(2); break;
         case 4: AO_T(4); break;
         case 8: AO_T(8); break;
@@ -1586,6 +1592,7 @@ static hipError_t launch_ao(const AttnArgs &a, const float *cs_table, RopeArgs r
     }
 #endif
 #undef AO_T
+#undef AO_C1
 #undef AO_C
 #undef AO_K
 #undef QF_LAUNCH
@@ -1654,7 +1661,7 @@ static QFPlan qf_plan(const AttnArgs &a, const MMVQSeg &wo, int K, const QKVFuse
     const int R = a.H / a.G, C = attn_out_fused_chunk(a);
     size_t attn_bytes = 0;
 #define QF_SZ(RR) attn_bytes = C == 64 ? sizeof(AOSmemQ<RR, 64>) : sizeof(AOSmemQ<RR, 128>)
-    switch (R) { case 1: QF_SZ(1); break; case 2: QF_SZ(2); break; case 4: QF_SZ(4); break; case 8: QF_SZ(8); break; default: return p; }
+    switch (R) { case 1: if (C == 256) attn_bytes = sizeof(AOSmemQ<1, 256>); else if (C == 192) attn_bytes = sizeof(AOSmemQ<1, 192>); else QF_SZ(1); break; case 2: QF_SZ(2); break; case 4: QF_SZ(4); break; case 8: QF_SZ(8); break; default: return p; }
 #undef QF_SZ
     const AOLayout ql = ao_layout((unsigned)wo_lds, K, attn_bytes, AO_QF_HDR, f.qkv_lds);
     const size_t accs_bytes = (size_t)AO_NCG * R * AO_D * 4;
