@@ -1,10 +1,10 @@
 // mmq_few.hip — the K-split contraction of 3 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
 // K-quant weights in their GGUF form, Q8_K activations, int8 matrix cores, the integer of ggml_vec_dot_q{4,5,6}_K_q8_K per (row, token, super-block).
 //
-// What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and in front of them the ~140 vector instructions per unit and token tile below (matrix
-// pipe and memory idle half of the time at two waves per SIMD).  Measured on an 8B Q4_K_M model, kernel times before -> now: gate | up (66 MB) at 4 tokens
-// 27.2 -> 18.7 us, at 37 tokens 51.4 -> 37.0; attn_output and ffn_down together 19.1 -> 12.3 a launch at 4; the head (431 MB) 129 -> 98; before is the 32 x 32
-// form of mmq.hip, whose waves had no load in flight while they computed and which left half of the CUs without a row tile.
+// What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and beside them the vector instructions per unit and token tile below, ~130 for Q4_K and 270 for Q6_K at
+// sixteen tokens (two waves per SIMD, whose waits the other wave's instructions do not fill: sixteen waves a CU are no faster).  An 8B Q4_K_M model, kernel times before -> now (before is the
+// 32 x 32 form of mmq.hip, whose waves had no load in flight while they computed and which left half of the CUs without a row tile): gate | up (66 MB) at 4 tokens 27.2 -> 15.5 us, at 37
+// 51.4 -> 34.1; ffn_down at 4, Q4_K and Q6_K, 12.8 and 18.9; Q | K | V at 37 14.1 -> 11.2; the head (431 MB) at 4 129 -> 97, its rows on the host.
 //   * A unit of work is 16 weight rows x one super-block (v_mfma_i32_16x16x32_i8: M = 16 tokens, N = 16 rows, K = the 32 weights of one scale group of Q4_K / Q5_K):
 //     a 4096-row tensor is 256 row tiles, one per CU, and 16 tokens pad to 16, 37 to 48.
 //   * One workgroup per CU walks its row tiles; its eight waves take a tile's super-blocks round-robin, and the weights of the next PD units - of the next tile
@@ -13,7 +13,9 @@
 //     own (a row's stride of 36, 44 or 52 words: no bank conflicts, no barrier).  Asked for as operands directly - 32 bytes of sixteen rows per request - every
 //     128-byte line is asked for by four or five requests: gate | up of an 8B layer took 29 us that way.
 //   * The activations come as operand blocks laid out by the quantiser (ActQuant::qf).  Read from rows of K bytes instead, sixteen lanes hit sixteen lines a power
-//     of two apart: 34 us at 4 tokens, 43 at 16.  A wave meets the same super-blocks in every tile: up to 4096 columns and 32 tokens they stay in registers.
+//     of two apart: 34 us at 4 tokens, 43 at 16.  A wave meets the same super-blocks in every tile: up to 4096 columns and 48 tokens they stay in registers.
+//   * To 8 and 4 tokens the operand's sixteen rows are two and four scale groups of a token (Act): half and a quarter of the multiplications by scales, the same integers.  Whole ticks of
+//     eight layers of an 8B model, four conversations 790 -> 715 us (with PAIR 1 below), seven 797 -> 745.
 //   * The eight partial sums of an output are added in wave order through LDS, so results do not depend on timing - and they are the sums the K-split
 //     kernel of mmq.hip makes, bit for bit: an integer per super-block, the same fold, the same order.
 #include <algorithm>
@@ -28,7 +30,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef short i16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int NW = 8, NT = 64 * NW;
 
@@ -36,25 +38,48 @@ __device__ __forceinline__ u32x4 ldg16(const void *p) { return *reinterpret_cast
 __device__ __forceinline__ u32x2 ldg8(const void *p) { return *reinterpret_cast<const u32x2 *>(p); }
 __device__ __forceinline__ long as_long(u32x2 v) { return __builtin_bit_cast(long, v); }
 __device__ __forceinline__ i32x4 mfma32(u32x2 a, u32x2 b, i32x4 c) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(as_long(a), as_long(b), c, 0, 0, 0); }
+__device__ __forceinline__ i32x4 mfma64(u32x4 a, u32x4 b, i32x4 c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0); }
 
-// A unit, 16 rows x one super-block, as it is asked for: piece p = lane + 64 i is 16 bytes of row p / PIECES; rows past the end read the last one (never stored)
-template <int TYPE> struct Raw {
+// A unit, 16 rows x one super-block, as it is asked for: piece p = lane + 64 i is 16 bytes of row p / PIECES.  What of a piece's address is the lane's own stays in registers, the
+// tile's and the super-block's share is scalar.  Tiles past the end of a tensor begin early enough to be whole (few_body), so rows are clamped only where there are fewer than sixteen
+template <int TYPE, bool PAIR> struct Raw {
     static constexpr int PIECES = TYPE == T_Q4_K ? 9 : TYPE == T_Q5_K ? 11 : 13, N = (16 * PIECES + 63) / 64, LDS = N * 1024, STRIDE = 16 * PIECES;
-    u32x4 v[N];
-    uint32_t d16 = 0;                                        // Q6_K: the row's scale, which lies apart
-    __device__ __forceinline__ void load(const uint8_t *W, int rows, unsigned row_bytes, int nb, int sb, int lane) {
+    struct Where {                                           // PAIR: eight rows of two tensors, so whole addresses; else offsets from a scalar base
+        unsigned o[N], u[N], d;                              // u: of a super-block (Q6_K: row planes ql, qh, scales, d, each with a step of its own)
+        const uint8_t *b[PAIR ? N : 1], *bd;
+    };
+    static __device__ __forceinline__ void where(Where &w, const uint8_t *W, const uint8_t *W2, int rows, unsigned row_bytes, int nb, int lane) {
+        const auto row = [&](int r) { return (unsigned)(PAIR ? (r & 7) < rows ? r & 7 : rows - 1 : r < rows ? r : rows - 1) * row_bytes; };
 #pragma unroll
         for (int i = 0; i < N; i++) {
             const int q = lane + 64 * i, p = q < STRIDE ? q : 0, r = p / PIECES, c = p - r * PIECES;    // (lanes past the unit: its first piece)
-            unsigned o = (unsigned)(r < rows ? r : rows - 1) * row_bytes;
-            if constexpr (TYPE == T_Q6_K)                    // row planes: ql (8 pieces), qh (4), scales (1)
-                o += c < 8 ? (unsigned)sb * 128u + 16u * c : c < 12 ? (unsigned)nb * 128u + (unsigned)sb * 64u + 16u * (c - 8) : (unsigned)nb * 192u + (unsigned)sb * 16u;
-            else o += (unsigned)sb * (unsigned)STRIDE + 16u * c;
-            v[i] = ldg16(W + o);
+            w.o[i] = row(r) + (TYPE != T_Q6_K || c < 8 ? 16u * c : c < 12 ? (unsigned)nb * 128u + 16u * (c - 8) : (unsigned)nb * 192u);
+            w.u[i] = TYPE != T_Q6_K ? (unsigned)STRIDE : c < 8 ? 128u : c < 12 ? 64u : 16u;
+            if constexpr (PAIR) w.b[i] = (r < 8 ? W : W2) + w.o[i];
         }
         if constexpr (TYPE == T_Q6_K) {
             const int r = lane & 15;
-            d16 = *reinterpret_cast<const uint16_t *>(W + (unsigned)(r < rows ? r : rows - 1) * row_bytes + (unsigned)nb * 208u + (unsigned)sb * 2u);
+            w.d = row(r) + (unsigned)nb * 208u;
+            if constexpr (PAIR) w.bd = (r < 8 ? W : W2) + w.d;
+        }
+    }
+    u32x4 v[N];
+    uint32_t d16 = 0;                                        // Q6_K: the row's scale, which lies apart
+    // at: what the tile's first row is away from the tensor's (bytes)
+    __device__ __forceinline__ void load(const Where &w, const uint8_t *W, size_t at, int sb, int lane) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            if constexpr (TYPE == T_Q6_K) {
+                const unsigned x = (unsigned)sb * w.u[i];
+                v[i] = PAIR ? ldg16(w.b[PAIR ? i : 0] + at + x) : ldg16(W + at + (w.o[i] + x));
+            } else {
+                const size_t x = at + (unsigned)sb * (unsigned)STRIDE;
+                v[i] = PAIR ? ldg16(w.b[PAIR ? i : 0] + x) : ldg16(W + x + w.o[i]);
+            }
+        }
+        if constexpr (TYPE == T_Q6_K) {
+            const size_t x = at + (unsigned)sb * 2u;
+            d16 = *reinterpret_cast<const uint16_t *>(PAIR ? w.bd + x : W + x + w.d);
         }
     }
     __device__ __forceinline__ void put(uint8_t *lds, int lane) const {
@@ -136,50 +161,95 @@ struct FewArgs {
 };
 
 // One lane's activation operands of one super-block, as the quantiser laid them out (kernels.h FEW_BLOCK): token 16 * tile + (lane & 15) as the A operand - element
-// pair (2 S, 2 S + 1) of scale groups per 16 bytes -, its block sums' two int8 planes, and the block scales of the four tokens whose results the lane holds
-template <int MT> struct Act {
+// pair (2 S, 2 S + 1) of scale groups per 16 bytes -, its block sums' two int8 planes, and the block scales of the four tokens whose results the lane holds.
+// G = 2, 4 (to 8 and 4 tokens, one tile): the operand's row G t + g is token t with the weights of all scale groups but every G-th zeroed, so one MFMA makes the sums of G groups at
+// once, and all of them are a lane's own 4 / G tokens': a G-th of the multiplications by scales.
+template <int MT, int TYPE, int G> struct Act {
     u32x4 a[MT][4];
     u32x2 bh[MT], bl[MT];
-    f32x4 yd[MT];
+    float yd[MT][4 / G];
     __device__ __forceinline__ void load(const uint8_t *qf, int tile0, int nb, int sb, int lane, int n) {    // the first n of the tiles
+        const int m = lane & 15, tk = m / G, kq = lane >> 4;
 #pragma unroll
         for (int t = 0; t < MT; t++) {
             if (t >= n) continue;
             const uint8_t *p = qf + (size_t)((unsigned)((tile0 + t) * nb + sb) * (unsigned)FEW_BLOCK);     // (wave-uniform)
 #pragma unroll
-            for (int s = 0; s < 4; s++) a[t][s] = ldg16(p + s * 1024 + lane * 16);
-            const int o = (lane & 15) * 16 + (lane >> 4 & 1) * 8;
+            for (int s = 0; s < 4; s++) a[t][s] = ldg16(p + s * 1024 + (kq * 16 + tk) * 16);
+            const int o = tk * 16 + (kq & 1) * 8;
             bh[t] = ldg8(p + FEW_BH + o); bl[t] = ldg8(p + FEW_BL + o);
-            yd[t] = *reinterpret_cast<const f32x4 *>(p + FEW_D + (lane >> 4) * 16);
+            if constexpr (G == 1) { const f32x4 y = *reinterpret_cast<const f32x4 *>(p + FEW_D + kq * 16); yd[t][0] = y.x; yd[t][1] = y.y; yd[t][2] = y.z; yd[t][3] = y.w; }
+            else if constexpr (G == 2) { const f32x2 y = *reinterpret_cast<const f32x2 *>(p + FEW_D + kq * 8); yd[t][0] = y.x; yd[t][1] = y.y; }
+            else yd[t][0] = *reinterpret_cast<const float *>(p + FEW_D + kq * 4);
+        }
+    }
+    // G > 1, behind the loads: the other groups' weights zeroed
+    __device__ __forceinline__ void mask(int lane) {
+        if constexpr (G > 1) {
+            const int g = lane & (G - 1), kq = lane >> 4;
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                uint32_t lo, hi;                             // the 16 bytes' first and second 32 weights
+                if constexpr (TYPE == T_Q6_K) {              // groups of sixteen: k-quarters 0, 1 and 2, 3 of each 32
+                    const bool h = (kq >> 1) == (g & 1);
+                    lo = h && (G == 2 || g < 2) ? ~0u : 0u; hi = h && (G == 2 || g >= 2) ? ~0u : 0u;
+                } else {
+                    const int x = G == 2 ? g : g - 2 * (s & 1);
+                    lo = x == 0 ? ~0u : 0u; hi = x == 1 ? ~0u : 0u;
+                }
+                a[0][s] &= u32x4{lo, lo, hi, hi};
+            }
         }
     }
 };
 
 // the first MT token tiles of A
-template <int TYPE, int MT, int M>
-__device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M> &A, int kq, bool take, float (*facc)[4]) {
+template <int TYPE, int MT, int M, int G>
+__device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M, TYPE, G> &A, int kq, bool take, float (*facc)[4 / G]) {
+    constexpr int TPL = 4 / G;                               // a lane's tokens
     const i32x4 z = {0, 0, 0, 0};
+    int isum[MT][TPL];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < TPL; r++) isum[t][r] = 0;
+#define HALF(J, t) ((J & 1) ? u32x2{A.a[t][J >> 1].z, A.a[t][J >> 1].w} : u32x2{A.a[t][J >> 1].x, A.a[t][J >> 1].y})
+#define BOTH(S) ({ const u32x2 b0_ = R.template codes<2 * (S)>(), b1_ = R.template codes<2 * (S) + 1>(); u32x4{b0_.x, b0_.y, b1_.x, b1_.y}; })
     if constexpr (Frag<TYPE>::GROUPS) {
         // header: d, dmin, twelve bytes of 6-bit scales and mins
         const uint32_t sc_lo = R.h.y & 0x3f3f3f3fu, mn_lo = R.h.z & 0x3f3f3f3fu;
         const uint32_t sc_hi = (R.h.w & 0x0f0f0f0fu) | ((R.h.y >> 2) & 0x30303030u), mn_hi = ((R.h.w >> 4) & 0x0f0f0f0fu) | ((R.h.z >> 2) & 0x30303030u);
-        int isum[MT][4];
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) isum[t][r] = 0;
+        const auto scale = [&](int J) { return (int)(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff); };
+        if constexpr (G == 1) {
 #define STEP(J)                                                                                              \
         {                                                                                                    \
             const u32x2 b = R.template codes<J>();                                                           \
-            const int sc = (int)(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff);                         \
+            const int sc = scale(J);                                                                         \
             _Pragma("unroll") for (int t = 0; t < MT; t++) {                                                 \
-                const i32x4 I = mfma32((J & 1) ? u32x2{A.a[t][J >> 1].z, A.a[t][J >> 1].w} : u32x2{A.a[t][J >> 1].x, A.a[t][J >> 1].y}, b, z);                                                    \
+                const i32x4 I = mfma32(HALF(J, t), b, z);                                                    \
                 _Pragma("unroll") for (int r = 0; r < 4; r++) isum[t][r] = __mul24(I[r], sc) + isum[t][r];   \
                 if constexpr (M > 1) { _Pragma("unroll") for (int r = 0; r < 4; r++) asm volatile("" : "+v"(isum[t][r])); }   /* (the sums are reassociated otherwise, every product alive) */ \
             }                                                                                                \
         }
         STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
 #undef STEP
+        } else if constexpr (G == 2) {
+#define STEP(S)                                                                                              \
+        {                                                                                                    \
+            const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                                   \
+            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * S + (r & 1))) + isum[0][r >> 1]; \
+        }
+        STEP(0) STEP(1) STEP(2) STEP(3)
+#undef STEP
+        } else {
+#define STEP(C)                                                                                              \
+        {                                                                                                    \
+            const i32x4 I = mfma64(A.a[0][2 * C + 1], BOTH(2 * C + 1), mfma64(A.a[0][2 * C], BOTH(2 * C), z)); \
+            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * C + r)) + isum[0][0]; \
+        }
+        STEP(0) STEP(1)
+#undef STEP
+        }
         // the mins against the sixteen block sums: min j meets sums 2 j and 2 j + 1; k-quarters 0 and 1 hold them, 2 and 3 are zero
         const uint32_t mw = kq == 0 ? mn_lo : mn_hi;
         u32x2 bm = {__builtin_amdgcn_perm(0, mw, 0x01010000u), __builtin_amdgcn_perm(0, mw, 0x03030202u)};
@@ -193,26 +263,22 @@ __device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M> &A,
             for (int r = 0; r < 4; r++) ms[r] <<= 6;
             ms = mfma32(A.bl[t], bm, ms);
 #pragma unroll
-            for (int r = 0; r < 4; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)isum[t][r] - (dm * A.yd[t][r]) * (float)ms[r];
+            for (int r = 0; r < TPL; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)isum[t][r] - (dm * A.yd[t][r]) * (float)ms[G * r];
         }
     } else {
         // The raw codes against the activations, 16-group by 16-group (a step of 32 weights is two of them: the k-quarters of the other one are
         // zeroed), the signed scale on the four results; the code's "- 32" is the scales against the block sums.  (The scale in the weight, as two int8 planes of
         // sc * (q - 32): 20 instructions per four weights, the head of an 8B model - 431 MB - at 4 tokens 131 us; this form 8 and 16 per token tile: 109 us)
-        int isum[MT][4];
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) isum[t][r] = 0;
+        const auto scale = [&](int j) { return (int)(int8_t)((R.sc[j >> 2] >> (8 * (j & 3))) & 0xff); };
+        if constexpr (G == 1) {
         const uint32_t m0 = kq < 2 ? ~0u : 0u, m1 = ~m0;
 #define STEP(J)                                                                                              \
         {                                                                                                    \
             const u32x2 b = R.template codes<J>();                                                           \
-            const uint32_t w = (J >> 1) == 0 ? R.sc.x : (J >> 1) == 1 ? R.sc.y : (J >> 1) == 2 ? R.sc.z : R.sc.w; \
-            const int s0 = (int)(int8_t)((w >> (16 * (J & 1))) & 0xff), s1 = (int)(int8_t)((w >> (16 * (J & 1) + 8)) & 0xff); \
+            const int s0 = scale(2 * J), s1 = scale(2 * J + 1);                                              \
             const u32x2 b0 = {b.x & m0, b.y & m0}, b1 = {b.x & m1, b.y & m1};                                \
             _Pragma("unroll") for (int t = 0; t < MT; t++) {                                                 \
-                const u32x2 av = (J & 1) ? u32x2{A.a[t][J >> 1].z, A.a[t][J >> 1].w} : u32x2{A.a[t][J >> 1].x, A.a[t][J >> 1].y}; \
+                const u32x2 av = HALF(J, t);                                                                 \
                 const i32x4 I0 = mfma32(av, b0, z), I1 = mfma32(av, b1, z);                                  \
                 _Pragma("unroll") for (int r = 0; r < 4; r++) isum[t][r] = __mul24(I1[r], s1) + (__mul24(I0[r], s0) + isum[t][r]); \
                 if constexpr (M > 1 || J == 3) { _Pragma("unroll") for (int r = 0; r < 4; r++) asm volatile("" : "+v"(isum[t][r])); } \
@@ -220,6 +286,23 @@ __device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M> &A,
         }
         STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
 #undef STEP
+        } else if constexpr (G == 2) {
+#define STEP(J)                                                                                              \
+        {                                                                                                    \
+            const i32x4 I = mfma32(HALF(J, 0), R.template codes<J>(), z);                                    \
+            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * J + (r & 1))) + isum[0][r >> 1]; \
+        }
+        STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
+#undef STEP
+        } else {
+#define STEP(S)                                                                                              \
+        {                                                                                                    \
+            const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                                   \
+            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * S + r)) + isum[0][0]; \
+        }
+        STEP(0) STEP(1) STEP(2) STEP(3)
+#undef STEP
+        }
         u32x2 bm = kq == 0 ? u32x2{R.sc.x, R.sc.y} : u32x2{R.sc.z, R.sc.w};
         if (kq >= 2) bm = u32x2{0, 0};
         const float dd = h2f((uint16_t)(take ? R.d16 : 0u));
@@ -230,84 +313,95 @@ __device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M> &A,
             for (int r = 0; r < 4; r++) ms[r] <<= 6;
             ms = mfma32(A.bl[t], bm, ms);
 #pragma unroll
-            for (int r = 0; r < 4; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)(isum[t][r] - 32 * ms[r]);
+            for (int r = 0; r < TPL; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)(isum[t][r] - 32 * ms[G * r]);
         }
     }
+#undef HALF
+#undef BOTH
 }
 
-// LDS of a workgroup: every wave's staging area (NP units), then the sets of partial sums [wave][pair][tile * 4 + r][lane]
-template <int TYPE, int NP> constexpr int few_stage = NW * NP * Raw<TYPE == 0 ? T_Q6_K : TYPE>::LDS;
+// LDS of a workgroup: every wave's staging area (NP units), then the sets of partial sums [wave][unit][tile * 4 / G + r][lane]
+template <int TYPE, int NP> constexpr int few_stage = NW * NP * Raw<TYPE == 0 ? T_Q6_K : TYPE, false>::LDS;
 template <int MT, int NP> constexpr int few_sets = MT * NP == 1 ? 2 : 1;  // two in turn: one barrier per tile
-template <int TYPE, int MT, int NP> constexpr int few_lds = few_stage<TYPE, NP> + few_sets<MT, NP> * NW * NP * MT * 1024;
+template <int TYPE, int MT, int G, int NP> constexpr int few_lds = few_stage<TYPE, NP> + few_sets<MT, NP> * NW * NP * MT * (1024 / G);
 
 // CN > 0: every wave has (up to) CN <= PD super-blocks of a tile and keeps their activation operands in registers across tiles.  CN = 0: any number, the operands
 // are read (from the caches) a unit ahead.
-// NP = 2: gate and up rows of one SwiGLU pair against the same activation operands.
+// out = silu(gate . x) * (up . x): PAIR 1, a tile is eight rows of ffn_gate and the same eight of ffn_up, one unit; PAIR 2, sixteen rows of each, two units against the same
+// activation operands.  14336 rows are seven tiles a CU of the first kind and three and a half, four for half of them, of the second; but where the operands are read again for every tile
+// the first reads them twice as often (few_pair).
 // HEAD: see mmq_few_head_kernel
 constexpr int HEAD_RUN = 4;                                  // row tiles whose results are stored to the host together, a wave's width of rows (two: 16 rows 20 us slower; eight: 4 and 16 rows 8 us)
 template <int MT> constexpr int head_lds = 2 * 16 * MT * HEAD_RUN * 64;
-template <int TYPE, int MT, int NP, int PD, int CN, bool HEAD = false>
+template <int TYPE, int MT, int G, int PAIR, int PD, int CN, bool HEAD = false>
 __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int tile, int n_blocks, uint8_t *smem, int stage_bytes) {
+    constexpr int TR = PAIR == 1 ? 8 : 16, TPL = 4 / G, NP = PAIR == 2 ? 2 : 1;           // a tile's rows (of each tensor), a lane's tokens of a token tile, a tile's units
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, kq = lane >> 4;
     const int nb = a.K >> 8, T = a.T;
-    int tiles = (sg.n_rows + 15) >> 4;
+    int tiles = (sg.n_rows + TR - 1) / TR;
     if constexpr (HEAD) {                                    // (a run of neighbours)
         const int b = tile, all = tiles, each = n_blocks;
         tile = (int)((long long)all * b / each); tiles = (int)((long long)all * (b + 1) / each);
         n_blocks = 1;
     }
     const int tile0 = tile;
-    uint8_t *stage = smem + wave * (NP * Raw<TYPE>::LDS);
+    const int row_max = sg.n_rows > TR ? sg.n_rows - TR : 0; // a tile's first row at most: the last tile begins early enough to be whole, and stores the rows that are its own
+    uint8_t *stage = smem + wave * (NP * Raw<TYPE, PAIR == 1>::LDS);
     float *part = reinterpret_cast<float *>(smem + stage_bytes);
     // token tiles are worked on two at a time (the registers of their operands); the operands of a pair that is read again stay a unit ahead
     constexpr int NC = (MT + 1) / 2, PA = CN > 0 ? CN : MT == 1 ? 2 : 1;
-    static_assert(CN == 0 || NC == 1, "operands of more than two token tiles are not kept");
+    static_assert(CN == 0 || MT <= 3, "operands of four token tiles are not kept");
+    static_assert(G == 1 || MT == 1, "one token tile");
     const int cn = CN > 0 ? CN : (nb + NW - 1) / NW;
-    float facc[NP][MT][4];
+    float facc[NP][MT][TPL];
     auto clear = [&]() {
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) facc[p][t][r] = 0.0f;
+                for (int r = 0; r < TPL; r++) facc[p][t][r] = 0.0f;
     };
     clear();
-    Raw<TYPE> R[PD][NP];
-    Act<MT == 1 ? 1 : 2> A[PA][NC];
+    typedef Raw<TYPE, PAIR == 1> RawT;
+    typedef Act<MT == 1 ? 1 : 2, TYPE, G> ActT;
+    typename RawT::Where where;
+    RawT::where(where, sg.W, PAIR == 1 ? a.seg[1].W : nullptr, sg.n_rows < TR ? sg.n_rows : TR, (unsigned)sg.row_bytes, nb, lane);
+    RawT R[PD][NP];
+    ActT A[PA][NC];
     // the unit the next request is for; past the end it stays on the last one
     int l_tile = tile, l_i = 0;
-    auto request = [&](Raw<TYPE> (&r)[NP]) {
-        const int row0 = l_tile * 16, rows = sg.n_rows - row0 < 16 ? sg.n_rows - row0 : 16;
+    auto request = [&](RawT (&r)[NP]) {
+        const int row0 = l_tile * TR < row_max ? l_tile * TR : row_max;
         const int sb = wave + NW * l_i < nb ? wave + NW * l_i : nb - 1;
-        r[0].load(sg.W + (size_t)row0 * sg.row_bytes, rows, (unsigned)sg.row_bytes, nb, sb, lane);
-        if constexpr (NP == 2) r[1].load(a.seg[1].W + (size_t)row0 * a.seg[1].row_bytes, rows, (unsigned)a.seg[1].row_bytes, nb, sb, lane);
+        r[0].load(where, sg.W, (size_t)row0 * sg.row_bytes, sb, lane);
+        if constexpr (NP == 2) r[1].load(where, a.seg[1].W, (size_t)row0 * sg.row_bytes, sb, lane);
         if (l_i + 1 < cn) l_i++;
         else if (l_tile + n_blocks < tiles) { l_tile += n_blocks; l_i = 0; }
     };
-    auto act = [&](Act<MT == 1 ? 1 : 2> &x, int c, int i) {
+    auto act = [&](ActT &x, int c, int i) {
         const int sb = wave + NW * i;
         x.load(a.qf, blockIdx.y * MT + 2 * c, nb, sb < nb ? sb : nb - 1, lane, MT - 2 * c);
     };
-    // an output of a finished tile: element e = tid + NT j of [tile * 4 + r][lane].  Its residual is requested a tile ahead, in front of the weights that follow
-    constexpr int NE = (MT * 256 + NT - 1) / NT;
+    // an output of a finished tile: element e = tid + NT j of [tile * TPL + r][lane].  Its residual is requested a tile ahead, in front of the weights that follow
+    constexpr int NS = MT * TPL * 64, NE = (NS + NT - 1) / NT;
     float rv[NE];
+    auto token = [&](int e) { const int tr = e >> 6; return (tr / TPL) * 16 + TPL * ((e & 63) >> 4) + tr % TPL; };
     auto place = [&](int e, int row_tile, size_t &o) {
-        const int ln = e & 63, tr = e >> 6;
-        const int gt = blockIdx.y * 16 * MT + (tr >> 2) * 16 + 4 * (ln >> 4) + (tr & 3), row = row_tile * 16 + (ln & 15);
+        const int gt = blockIdx.y * 16 * MT + token(e), row0 = row_tile * TR < row_max ? row_tile * TR : row_max, row = row0 + (e & (TR - 1));
         o = (size_t)gt * sg.ld_out + row;
-        return e < MT * 256 && gt < T && row < sg.n_rows;
+        return e < NS && gt < T && row >= row_tile * TR && row < sg.n_rows && (e & 15) < TR;
     };
     auto residual = [&](int row_tile) {
-        if constexpr (NP == 1) if (sg.resid) {
+        if constexpr (PAIR == 0) if (sg.resid) {
 #pragma unroll
             for (int j = 0; j < NE; j++) { size_t o; const bool in = place(tid + NT * j, row_tile, o); rv[j] = sg.resid[in ? o : 0]; }
         }
     };
     int set = 0;
     // HEAD: results wait in LDS for the other tiles of their run, [run parity][token][row]; a thread's outputs are all of one token
-    float *const run = part + few_sets<MT, NP> * NW * NP * MT * 256;
+    float *const run = part + few_sets<MT, NP> * NW * NP * NS;
     float top = -INFINITY;
     int top_row = 0x7fffffff;
     auto to_host = [&](int done) {                           // the run that ends in front of `done`, behind a barrier
@@ -319,14 +413,14 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
             if (lane < rows) a.host[(size_t)t * sg.ld_out + row0 + lane] = r0[t * (HEAD_RUN * 16) + lane];
     };
     auto finish = [&](int row_tile) {
-        float *ps = part + set * (NW * NP * MT * 256);
+        float *ps = part + set * (NW * NP * NS);
         set ^= few_sets<MT, NP> - 1;
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) ps[((wave * NP + p) * MT * 4 + t * 4 + r) * 64 + lane] = facc[p][t][r];
+                for (int r = 0; r < TPL; r++) ps[(wave * NP + p) * NS + (t * TPL + r) * 64 + lane] = facc[p][t][r];
         __syncthreads();
         if constexpr (HEAD) if (row_tile > tile0 && (row_tile - tile0) % HEAD_RUN == 0) to_host(row_tile);
 #pragma unroll
@@ -337,14 +431,14 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
                 float sum = 0.0f, sum2 = 0.0f;
 #pragma unroll
                 for (int w = 0; w < NW; w++) {
-                    sum += ps[(w * NP) * MT * 256 + e];
-                    if constexpr (NP == 2) sum2 += ps[(w * NP + 1) * MT * 256 + e];
+                    sum += ps[w * NP * NS + e];
+                    if constexpr (PAIR) sum2 += ps[PAIR == 1 ? w * NS + e + 8 : (w * NP + 1) * NS + e];
                 }
-                if constexpr (NP == 2) sg.out[o] = (sum / (1.0f + expf(-sum))) * sum2;
+                if constexpr (PAIR) sg.out[o] = (sum / (1.0f + expf(-sum))) * sum2;
                 else sg.out[o] = sg.resid ? rv[j] + sum : sum;
                 if constexpr (HEAD) {
-                    const int k = row_tile - tile0, gt = (e >> 8) * 16 + 4 * ((e & 63) >> 4) + (e >> 6 & 3), row = row_tile * 16 + (e & 15);
-                    run[((k / HEAD_RUN & 1) * 16 * MT + gt) * (HEAD_RUN * 16) + (k % HEAD_RUN) * 16 + (e & 15)] = sum;
+                    const int k = row_tile - tile0, gt = token(e), row = (int)(o - (size_t)gt * sg.ld_out);
+                    run[((k / HEAD_RUN & 1) * 16 * MT + gt) * (HEAD_RUN * 16) + (k % HEAD_RUN) * 16 + (row - row_tile * 16)] = sum;
                     if (sum > top || (sum == top && row < top_row)) { top = sum; top_row = row; }
                 }
             }
@@ -362,24 +456,27 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     for (int u = 0; u < PD; u++) { __builtin_amdgcn_sched_barrier(0); request(R[u]); __builtin_amdgcn_sched_barrier(0); }
     static_assert(CN == 0 || PD % CN == 0, "a slot belongs to one super-block of the tile");
     static_assert(CN > 0 || PD % PA == 0, "activation slots turn with the weight slots");
-    int i = 0;
-    auto unit = [&](Raw<TYPE> (&r)[NP], Act<MT == 1 ? 1 : 2> (&x)[NC], int i) {
-        const bool take = wave + NW * i < nb;                              // (a tile of nb super-blocks does not divide by the waves: the last unit's share is multiplied by a zero scale, not branched around)
+    if constexpr (CN > 0) {
 #pragma unroll
-        for (int p = 0; p < NP; p++) r[p].put(stage + p * Raw<TYPE>::LDS, lane);
+        for (int i = 0; i < PA; i++) A[i][0].mask(lane);
+    }
+    int i = 0;
+    auto unit = [&](RawT (&r)[NP], ActT (&x)[NC], int i) {
+        const bool take = wave + NW * i < nb;                              // (a tile of nb super-blocks does not divide by the waves: the last unit's share is multiplied by a zero scale, not branched around)
         uint32_t d16[NP];
 #pragma unroll
-        for (int p = 0; p < NP; p++) d16[p] = r[p].d16;
+        for (int p = 0; p < NP; p++) { r[p].put(stage + p * RawT::LDS, lane); d16[p] = r[p].d16; }
         __builtin_amdgcn_sched_barrier(0);                                 // (a wave's LDS accesses are made in order)
         request(r);                                                        // the slot's next unit, in flight across this one's arithmetic
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (CN == 0) x[0].mask(lane);
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             constexpr int LAST = MT - 2 * (NC - 1);
 #pragma unroll
             for (int p = 0; p < NP; p++) {
                 Frag<TYPE> f;
-                f.get(stage + p * Raw<TYPE>::LDS, d16[p], n, kq);
+                f.get(stage + p * RawT::LDS, d16[p], n, kq);
                 if (c < NC - 1 || LAST == 2) superblock<TYPE, MT == 1 ? 1 : 2>(f, x[c], kq, take, facc[p] + 2 * c);
                 else superblock<TYPE, 1>(f, x[c], kq, take, facc[p] + 2 * c);
             }
@@ -406,8 +503,8 @@ done:
         const auto better = [&](float v, int r) { if (v > top || (v == top && r < top_row)) { top = v; top_row = r; } };
 #pragma unroll
         for (int o = 8; o > 0; o >>= 1) { const float v = __shfl_xor(top, o, 64); const int r = __shfl_xor(top_row, o, 64); better(v, r); }
-        const int gt = (tid >> 8) * 16 + 4 * (lane >> 4) + (tid >> 6 & 3), blocks = (int)gridDim.x;
-        if (tid < MT * 256 && (lane & 15) == 0 && gt < T) {
+        const int gt = token(tid), blocks = (int)gridDim.x;
+        if (tid < NS && (lane & 15) == 0 && gt < T) {
             __hip_atomic_store(a.best + gt * blocks + blockIdx.x, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(a.best_row + gt * blocks + blockIdx.x, top_row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -433,20 +530,21 @@ done:
 }
 
 // TYPE: the segments' common type, or 0 where they differ (Q | K | V of a layer whose attn_v is wider)
-template <int TYPE, int MT, int NP, int PD, int CN>
+template <int TYPE, int MT, int G, int PAIR, int PD, int CN>
 __global__ __launch_bounds__(NT, 2) void mmq_few_kernel(const FewArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, NP>];
+    constexpr int NP = PAIR == 2 ? 2 : 1;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, G, NP>];
     int s = 0;
-    if constexpr (NP == 1) {
+    if constexpr (!PAIR) {
         if (a.n_seg > 1 && (int)blockIdx.x >= a.seg[1].tile0) s = 1;
         if (a.n_seg > 2 && (int)blockIdx.x >= a.seg[2].tile0) s = 2;
     }
-    const int first = (int)blockIdx.x - a.seg[s].tile0, n_blocks = (s + 1 < a.n_seg && NP == 1 ? a.seg[s + 1].tile0 : (int)gridDim.x) - a.seg[s].tile0;
-    if constexpr (TYPE != 0) few_body<TYPE, MT, NP, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>);
+    const int first = (int)blockIdx.x - a.seg[s].tile0, n_blocks = (s + 1 < a.n_seg && !PAIR ? a.seg[s + 1].tile0 : (int)gridDim.x) - a.seg[s].tile0;
+    if constexpr (TYPE != 0) few_body<TYPE, MT, G, PAIR, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>);
     else switch (a.seg[s].type) {
-        case T_Q4_K: few_body<T_Q4_K, MT, NP, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
-        case T_Q5_K: few_body<T_Q5_K, MT, NP, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
-        case T_Q6_K: few_body<T_Q6_K, MT, NP, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
+        case T_Q4_K: few_body<T_Q4_K, MT, G, PAIR, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
+        case T_Q5_K: few_body<T_Q5_K, MT, G, PAIR, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
+        case T_Q6_K: few_body<T_Q6_K, MT, G, PAIR, PD, CN>(a, a.seg[s], first, n_blocks, smem, few_stage<TYPE, NP>); break;
         default: break;
     }
 }
@@ -454,35 +552,40 @@ __global__ __launch_bounds__(NT, 2) void mmq_few_kernel(const FewArgs a) {
 // The output head of a tick: a workgroup takes a run of neighbouring row tiles, and stores the results of HEAD_RUN of them at a time - 256 consecutive bytes a token - to the
 // host's rows while its weights stream: PCIe bounds it from a dozen rows on.  The rows' arg-max is made of what the threads hold anyway.  128256 rows of 4096 columns (Q6_K), us, here /
 // the head, the arg-max and a launch that copies the rows one behind the other: 4 tokens 110 / 99 + 10 + 38, 16 tokens 206 / 104 + 19 + 149.
-template <int TYPE, int MT, int CN>
+template <int TYPE, int MT, int G, int CN>
 __global__ __launch_bounds__(NT, 2) void mmq_few_head_kernel(const FewArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, 1> + head_lds<MT>];
-    few_body<TYPE, MT, 1, 4, CN, true>(a, a.seg[0], (int)blockIdx.x, (int)gridDim.x, smem, few_stage<TYPE, 1>);
+    __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, G, 1> + head_lds<MT>];
+    few_body<TYPE, MT, G, 0, 4, CN, true>(a, a.seg[0], (int)blockIdx.x, (int)gridDim.x, smem, few_stage<TYPE, 1>);
 }
 template <int TYPE>
 void few_head(const FewArgs &a, int blocks, hipStream_t st) {
     const int cn = ((a.K >> 8) + NW - 1) / NW;
-#define GO(MT, CN) hipLaunchKernelGGL((mmq_few_head_kernel<TYPE, MT, CN>), dim3((unsigned)blocks), dim3(NT), 0, st, a)
-    if (a.T <= 16) { if (cn == 1) GO(1, 1); else if (cn == 2) GO(1, 2); else GO(1, 0); }
-    else if (cn == 1) GO(2, 1); else if (cn == 2) GO(2, 2); else GO(2, 0);
+#define GO(MT, G, CN) hipLaunchKernelGGL((mmq_few_head_kernel<TYPE, MT, G, CN>), dim3((unsigned)blocks), dim3(NT), 0, st, a)
+#define GO_CN(MT, G) do { if (cn == 1) GO(MT, G, 1); else if (cn == 2) GO(MT, G, 2); else GO(MT, G, 0); } while (0)
+    if (a.T <= 4) GO_CN(1, 4); else if (a.T <= 8) GO_CN(1, 2); else if (a.T <= 16) GO_CN(1, 1); else GO_CN(2, 1);
+#undef GO_CN
 #undef GO
 }
 
-template <int TYPE, int MT, int NP, int PD, int CN>
-void few_go(const FewArgs &a, int blocks, hipStream_t st) {
-    hipLaunchKernelGGL((mmq_few_kernel<TYPE, MT, NP, PD, CN>), dim3((unsigned)blocks, (unsigned)((a.T + 16 * MT - 1) / (16 * MT))), dim3(NT), 0, st, a);
-}
-template <int TYPE, int NP>
+// The form of a gate | up launch: the operands of up to 48 tokens stay in registers to 4096 columns, and to eight tokens they are few.  us a pass, PAIR 1 / 2: three layers of 5120 columns
+// at 4 and 12 tokens 395 / 437, 492 / 497, two of 8192 at 4, 12, 24 and 40 625 / 683, 747 / 736, 986 / 942, 790 / 752; 37.2 / 34.1 a launch of 14336 x 4096 at 37
+int few_pair(int K, int T) { return T <= 8 || (K <= 2 * NW * 256 && T <= 48) ? 1 : 2; }
+
+template <int TYPE, int PAIR>
 void few_type(const FewArgs &a, int blocks, hipStream_t st) {
-    const int mt = a.T <= 16 ? 1 : a.T <= 32 ? 2 : a.T <= 48 ? 3 : 4, cn = ((a.K >> 8) + NW - 1) / NW;
-    constexpr int PD = 4 / NP;                                             // four units of weights in flight per wave: 74 KB per CU
-#define GO(MT, CN) few_go<TYPE, MT, NP, PD, CN>(a, blocks, st)
-    switch (mt) {
-        case 1: if (cn == 1) GO(1, 1); else if (cn == 2) GO(1, 2); else GO(1, 0); break;
-        case 2: if (cn == 1) GO(2, 1); else if (cn == 2) GO(2, 2); else GO(2, 0); break;
-        case 3: few_go<TYPE, 3, NP, 2 / NP, 0>(a, blocks, st); break;           // (three and four token tiles: their operands take the registers)
-        default: few_go<TYPE, 4, NP, 2 / NP, 0>(a, blocks, st); break;
-    }
+    const int cn = ((a.K >> 8) + NW - 1) / NW;
+    // four units of weights in flight per wave: 74 KB per CU (three and four token tiles: two, their operands take the registers)
+#define GO(MT, G, PD, CN) hipLaunchKernelGGL((mmq_few_kernel<TYPE, MT, G, PAIR, PD, CN>), dim3((unsigned)blocks, (unsigned)((a.T + 16 * MT - 1) / (16 * MT))), dim3(NT), 0, st, a)
+#define GO_CN(MT, G) do { if (cn == 1) GO(MT, G, 4, 1); else if (cn == 2) GO(MT, G, 4, 2); else GO(MT, G, 4, 0); } while (0)
+    if constexpr (PAIR == 2) {
+        if (a.T <= 16) GO(1, 1, 2, 0); else if (a.T <= 32) GO(2, 1, 2, 0); else if (a.T <= 48) GO(3, 1, 1, 0); else GO(4, 1, 1, 0);
+    } else if (a.T <= 4) GO_CN(1, 4);
+    else if (a.T <= 8) GO_CN(1, 2);
+    else if (a.T <= 16) { if (cn == 1) GO(1, 1, 4, 1); else if (cn == 2) GO(1, 1, 4, 2); else if constexpr (PAIR == 0) GO(1, 1, 4, 0); }
+    else if (a.T <= 32) { if (cn == 1) GO(2, 1, 4, 1); else if (cn == 2) GO(2, 1, 4, 2); else if constexpr (PAIR == 0) GO(2, 1, 4, 0); }
+    else if (a.T <= 48) { if (cn == 1) GO(3, 1, 2, 1); else if (cn == 2) GO(3, 1, 2, 2); else if constexpr (PAIR == 0) GO(3, 1, 2, 0); }
+    else if constexpr (PAIR == 0) GO(4, 1, 2, 0);
+#undef GO_CN
 #undef GO
 }
 
@@ -510,28 +613,40 @@ hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const Act
     FewArgs a{};
     a.n_seg = n_seg; a.K = K; a.T = T;
     a.qf = q.qf;
-    // one workgroup per CU where there are more row tiles than that: a segment's share of them by its rows
-    const int ns = swiglu ? 1 : n_seg;
-    int tiles = 0, type = segs[0].type, blocks = 0;
-    for (int i = 0; i < ns; i++) { tiles += (segs[i].n_rows + 15) / 16; if (segs[i].type != type) type = 0; }
+    // one workgroup per CU where there are more row tiles than that.  Segments of different types: as few rounds as a Q6_K tile of one and a half others' allow (Q | K | V with a
+    // Q6_K attn_v, 256 + 64 + 64 tiles, us at 4 and 16 tokens: 12.1, 12.2 where every tensor gets its share by rows - V's tiles two to a workgroup - here 8.6, 9.6); the CUs left over by rows
+    const int ns = swiglu ? 1 : n_seg, pair = swiglu ? few_pair(K, T) : 0, tr = pair == 1 ? 8 : 16;
+    int tiles = 0, type = segs[0].type, t[3] = {0, 0, 0}, n[3] = {0, 0, 0};
+    for (int i = 0; i < ns; i++) { tiles += t[i] = (segs[i].n_rows + tr - 1) / tr; if (segs[i].type != type) type = 0; }
     const int cap = std::max(ns, std::min(tiles, num_cu()));
-    for (int i = 0, seen = 0; i < n_seg; i++) {
+    const auto cost = [&](int i) { return segs[i].type == T_Q6_K ? 3 : 2; };
+    for (int budget = 3;; budget++) {
+        int sum = 0;
+        for (int i = 0; i < ns; i++) { const int each = std::max(1, budget / cost(i)); sum += n[i] = (t[i] + each - 1) / each; }
+        if (sum <= cap || budget > 3 * tiles) break;
+    }
+    for (int left = cap - n[0] - n[1] - n[2]; left > 0; left--) {
+        int k = 0;
+        for (int i = 1; i < ns; i++) if ((long long)t[i] * cost(i) * n[k] > (long long)t[k] * cost(k) * n[i]) k = i;
+        if (n[k] >= t[k]) break;
+        n[k]++;
+    }
+    int blocks = 0;
+    for (int i = 0; i < n_seg; i++) {
         a.seg[i] = segs[i];
         a.seg[i].tile0 = blocks;
-        if (i >= ns) continue;
-        seen += (segs[i].n_rows + 15) / 16;
-        blocks = std::max(blocks + 1, (int)((long long)cap * seen / tiles));
+        if (i < ns) blocks += n[i];
     }
     if (swiglu) switch (type) {
-        case T_Q4_K: few_type<T_Q4_K, 2>(a, blocks, st); break;
-        case T_Q5_K: few_type<T_Q5_K, 2>(a, blocks, st); break;
-        case T_Q6_K: few_type<T_Q6_K, 2>(a, blocks, st); break;
+        case T_Q4_K: if (pair == 1) few_type<T_Q4_K, 1>(a, blocks, st); else few_type<T_Q4_K, 2>(a, blocks, st); break;
+        case T_Q5_K: if (pair == 1) few_type<T_Q5_K, 1>(a, blocks, st); else few_type<T_Q5_K, 2>(a, blocks, st); break;
+        case T_Q6_K: if (pair == 1) few_type<T_Q6_K, 1>(a, blocks, st); else few_type<T_Q6_K, 2>(a, blocks, st); break;
         default: return hipErrorInvalidValue;
     } else switch (type) {
-        case T_Q4_K: few_type<T_Q4_K, 1>(a, blocks, st); break;
-        case T_Q5_K: few_type<T_Q5_K, 1>(a, blocks, st); break;
-        case T_Q6_K: few_type<T_Q6_K, 1>(a, blocks, st); break;
-        default: few_type<0, 1>(a, blocks, st); break;
+        case T_Q4_K: few_type<T_Q4_K, 0>(a, blocks, st); break;
+        case T_Q5_K: few_type<T_Q5_K, 0>(a, blocks, st); break;
+        case T_Q6_K: few_type<T_Q6_K, 0>(a, blocks, st); break;
+        default: few_type<0, 0>(a, blocks, st); break;
     }
     return hipGetLastError();
 }
