@@ -274,9 +274,10 @@ hipError_t launch_mmv_float(int type, const uint8_t *W, int n_rows, int K, const
 // MoE router: softmax over n_expert logits per token, top-k (first index wins ties), weights renormalised
 // forced (nullable, tests): [T][k] expert ids to take instead of the k most probable (weights = this side's probabilities of them, renormalised)
 hipError_t launch_moe_route(const float *logits, int T, int n_expert, int k, int32_t *ids, float *w, hipStream_t st, const int32_t *forced = nullptr);
-// the two above in one launch (f32 / f16 gate_inp), same arithmetic; logits_out may be null
+// the two above in one launch (f32 / f16 gate_inp); nw (nullable; one token, moe_router_norms): x is the row in front of the RMS norm with these weights
+bool moe_router_norms(int type, int n_expert, int K);
 hipError_t launch_moe_router(int type, const uint8_t *W, int n_expert, int K, const float *x, int T, int k, float *logits_out, int32_t *ids, float *w,
-                             hipStream_t st, const int32_t *forced = nullptr);
+                             hipStream_t st, const int32_t *forced = nullptr, const float *nw = nullptr, float eps = 0.0f);
 // x[t][d] += sum_j eo[j][t][d] * w[t][j]   (experts added in rank order, then the residual)
 hipError_t launch_moe_combine(float *x, const float *eo, const float *w, int T, int E, int k, size_t eo_stride, hipStream_t st);
 hipError_t launch_gather_rows_f32(const float *src, const int32_t *rows, int n_rows, int n, float *dst, hipStream_t st);
@@ -688,7 +689,7 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
 // (never reset: they hold the tag of the step that raised them); serial: device word the step's set-up launch increments (never 0).
 void set_attn_out_fused(int on);                          // tests / A-B runs: 0 = the two launches, 1 = fused, -1 = environment (MI355_ATTN_OUT_FUSED, default on)
 bool attn_out_fused_enabled();
-int attn_out_fused_chunk(const AttnArgs &a);              // cells per attention item: 64, or 128 from the context length on where 64 would give a CU two items
+int attn_out_fused_chunk(const AttnArgs &a);              // cells per attention item: 64, and 128 .. 256 where fewer would give a CU two items
 int attn_out_fused_splits(const AttnArgs &a);
 bool attn_out_fused_applicable(const AttnArgs &a, const RopeArgs &ra, const MMVQSeg &wo, int K, int epi);
 // gran: attn_out_granule_words(K) 8-byte words shared by the layers of a step (zero once); layer: 0 .. 254, part of the hand-over tag

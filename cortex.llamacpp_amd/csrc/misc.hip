@@ -374,66 +374,150 @@ hipError_t launch_moe_route(const float *logits, int T, int n_expert, int k, int
     hipLaunchKernelGGL(moe_route_kernel, dim3((T + 63) / 64), dim3(64), 0, st, logits, T, n_expert, k, ids, w, forced);
     return hipGetLastError();
 }
-// Router of a mixture-of-experts layer in ONE launch: logits = gate_inp . x (the arithmetic of mmv_float_kernel: lane l adds
-// the products k = l, l + 64, ... in a double, waves reduced the same way), then the selection of moe_route_kernel, per
-// token.  Workgroup = token; wave w computes experts w, w + 4, ...; thread 0 selects.  Same bits as the two launches.
-__global__ __launch_bounds__(256) void moe_router_kernel(int type, const uint8_t *W, int n_expert, int K, const float *x, int k, float *logits_out,
-                                                         int32_t *ids, float *w, const int32_t *forced) {
-    __shared__ float lg[64];
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float *xr = x + (size_t)t * K;
-    constexpr int UN = 16;
-    for (int e = wave; e < n_expert; e += 4) {
+// Router of a mixture-of-experts layer in ONE launch: logits = gate_inp . x, products in f32 and their sums in double, then the selection of moe_route_kernel.
+// What bounds it is latency: 131 KB of weights (8 experts of 4096 columns) for a token.  So sixteen waves, an expert's columns shared by as many as there are; a wave's first
+// eight pieces of weights are in flight before the row's norm is known; the selection is a wave's, a lane an expert.  NTOK rows share a workgroup's weights.
+// NORM (one token): x is the row in front of the norm, so that a step needs no launch that norms it (its expert kernels norm for themselves).
+// us, one token, 8 experts: 7.5, and 5.2 of a norm launch + 9.7 with four waves that walked two experts each and one thread that selected.
+template <int NTOK, bool NORM>
+__global__ __launch_bounds__(1024) void moe_router_kernel(int type, const uint8_t *W, int n_expert, int K, const float *x, const float *nw, float eps, int T, int k, float *logits_out,
+                                                          int32_t *ids, float *w, const int32_t *forced) {
+    extern __shared__ __attribute__((aligned(16))) float xs[];          // [NTOK][K]
+    __shared__ double part[64 * NTOK], red[16];
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t0 = blockIdx.x * NTOK;
+    const int each = n_expert <= 8 ? 16 / n_expert : 1;                  // waves of an expert
+    const int np = K >> 8, per = (np + each - 1) / each;                // pieces of 256 columns, of a wave's share
+    constexpr int UN = 8;
+    u32x4 pre[UN];
+    const auto piece = [&](int e, int q) {                               // four weights of the lane
+        const size_t at = (size_t)e * K + q * 256 + lane * 4;
+        if (type == T_F32) return *reinterpret_cast<const u32x4 *>(W + at * 4);
+        const u32x2 h = *reinterpret_cast<const u32x2 *>(W + at * 2);
+        return u32x4{h.x, h.y, 0u, 0u};
+    };
+    const int e0 = wave / each, q0 = (wave % each) * per;
+    if (e0 < n_expert) {
+#pragma unroll
+        for (int u = 0; u < UN; u++) pre[u] = piece(e0, q0 + u < np ? q0 + u : np - 1);
+    }
+    if constexpr (NORM) {
+        constexpr int NV = 4;                                            // (rows of up to 16384 columns)
+        f32x4 v[NV], g[NV];
         double s = 0.0;
-        if (type == T_F32) {
-            const float *wr = reinterpret_cast<const float *>(W) + (size_t)e * K;
-            for (int k0 = lane; k0 < K; k0 += 64 * UN) {
-                float wv[UN], xv[UN];
 #pragma unroll
-                for (int j = 0; j < UN; j++) { const int kk = k0 + 64 * j, kc = kk < K ? kk : lane; wv[j] = wr[kc]; xv[j] = xr[kc]; }
-#pragma unroll
-                for (int j = 0; j < UN; j++) if (k0 + 64 * j < K) s += (double)(wv[j] * xv[j]);
-            }
-        } else {
-            const uint16_t *wr = reinterpret_cast<const uint16_t *>(W) + (size_t)e * K;
-            for (int k0 = lane; k0 < K; k0 += 64 * UN) {
-                uint16_t wv[UN]; float xv[UN];
-#pragma unroll
-                for (int j = 0; j < UN; j++) { const int kk = k0 + 64 * j, kc = kk < K ? kk : lane; wv[j] = wr[kc]; xv[j] = xr[kc]; }
-#pragma unroll
-                for (int j = 0; j < UN; j++) if (k0 + 64 * j < K) s += (double)(h2f(wv[j]) * h2f(f2h(xv[j])));
-            }
+        for (int j = 0; j < NV; j++) {
+            const int i = (tid + 1024 * j) * 4;
+            if (i < K) { v[j] = *reinterpret_cast<const f32x4 *>(x + i); g[j] = *reinterpret_cast<const f32x4 *>(nw + i); }
         }
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+            if ((tid + 1024 * j) * 4 < K) { s += (double)(v[j].x * v[j].x); s += (double)(v[j].y * v[j].y); s += (double)(v[j].z * v[j].z); s += (double)(v[j].w * v[j].w); }
         s = wave_sum(s);
-        if (lane == 0) { lg[e] = (float)s; if (logits_out) logits_out[(size_t)t * n_expert + e] = (float)s; }
+        if (lane == 0) red[wave] = s;
+        __syncthreads();
+        double tot = 0.0;
+#pragma unroll
+        for (int i = 0; i < 16; i++) tot += red[i];
+        const float scale = 1.0f / sqrtf((float)(tot / (double)K) + eps);
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = (tid + 1024 * j) * 4;
+            if (i < K) *reinterpret_cast<f32x4 *>(xs + i) = f32x4{(v[j].x * scale) * g[j].x, (v[j].y * scale) * g[j].y, (v[j].z * scale) * g[j].z, (v[j].w * scale) * g[j].w};
+        }
+    } else {
+        for (int i = tid * 4; i < NTOK * K; i += 4096) {
+            const int t = t0 + i / K;
+            *reinterpret_cast<f32x4 *>(xs + i) = *reinterpret_cast<const f32x4 *>(x + (size_t)(t < T ? t : T - 1) * K + i % K);
+        }
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    float p[64];
-    float mx = -INFINITY;
-    for (int e = 0; e < n_expert; e++) mx = fmaxf(mx, lg[e]);
-    double sum = 0.0;
-    for (int e = 0; e < n_expert; e++) { p[e] = expf(lg[e] - mx); sum += (double)p[e]; }
-    const float inv = (float)(1.0 / sum);
-    for (int e = 0; e < n_expert; e++) p[e] *= inv;
-    unsigned long long used = 0;
-    float wsum = 0.0f;
-    for (int j = 0; j < k; j++) {
-        int best = -1;
-        for (int e = 0; e < n_expert; e++)
-            if (!((used >> e) & 1ull) && (best < 0 || p[e] > p[best])) best = e;
-        if (forced) { best = forced[(size_t)t * k + j]; best = best < 0 ? 0 : best >= n_expert ? n_expert - 1 : best; }
-        used |= 1ull << best;
-        ids[(size_t)t * k + j] = best;
-        w[(size_t)t * k + j] = p[best];
-        wsum += p[best];
+    for (int task = wave; task < n_expert * each; task += 16) {
+        const int e = task / each, q1 = (task % each) * per, q2 = q1 + per < np ? q1 + per : np;
+        double s[NTOK];
+#pragma unroll
+        for (int t = 0; t < NTOK; t++) s[t] = 0.0;
+        for (int q = q1; q < q2; q += UN) {
+            if (task != wave || q != q1) {
+#pragma unroll
+                for (int u = 0; u < UN; u++) pre[u] = piece(e, q + u < np ? q + u : np - 1);
+            }
+#pragma unroll
+            for (int u = 0; u < UN; u++) {
+                if (q + u >= q2) break;
+                float wv[4];
+                if (type == T_F32) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) wv[i] = __uint_as_float(pre[u][i]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) wv[i] = h2f((uint16_t)(pre[u][i >> 1] >> (16 * (i & 1))));
+                }
+#pragma unroll
+                for (int t = 0; t < NTOK; t++) {
+                    const f32x4 xv = *reinterpret_cast<const f32x4 *>(xs + (size_t)t * K + (q + u) * 256 + lane * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) s[t] += (double)(wv[i] * (type == T_F32 ? xv[i] : h2f(f2h(xv[i]))));
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < NTOK; t++) {
+            s[t] = wave_sum(s[t]);
+            if (lane == 0) part[task * NTOK + t] = s[t];
+        }
     }
-    for (int j = 0; j < k; j++) w[(size_t)t * k + j] /= wsum;
+    __syncthreads();
+    const int t = t0 + wave;
+    if (wave >= NTOK || t >= T) return;
+    float p = 0.0f, lg = -INFINITY;
+    if (lane < n_expert) {
+        double s = 0.0;
+        for (int i = 0; i < each; i++) s += part[(lane * each + i) * NTOK + wave];
+        lg = (float)s;
+        if (logits_out) logits_out[(size_t)t * n_expert + lane] = lg;
+    }
+    const float mx = wave_max(lg);
+    if (lane < n_expert) p = expf(lg - mx);
+    const double sum = wave_sum((double)p);
+    p *= (float)(1.0 / sum);
+    // the k most probable, the lower of equals first; a NaN is the least, and still an expert
+    int key = lane < n_expert ? (p == p ? (int)__float_as_uint(p) + 1 : 0) : -1;
+    float wsum = 0.0f, mine = 0.0f;
+    int id = 0;
+    for (int j = 0; j < k; j++) {
+        int bk = key, be = lane;
+        for (int o = n_expert <= 8 ? 4 : 32; o > 0; o >>= 1) {           // (lanes 0 .. 7 among themselves, and lane 0 tells the others)
+            const int ok = __shfl_xor(bk, o, 64), oe = __shfl_xor(be, o, 64);
+            if (ok > bk || (ok == bk && oe < be)) { bk = ok; be = oe; }
+        }
+        be = __builtin_amdgcn_readfirstlane(be);
+        if (forced) { be = forced[(size_t)t * k + j]; be = be < 0 ? 0 : be >= n_expert ? n_expert - 1 : be; }
+        if (lane == be) key = -1;
+        const float pb = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), __builtin_amdgcn_readfirstlane(be)));
+        if (lane == j) { id = be; mine = pb; }
+        wsum += pb;
+    }
+    if (lane < k) { ids[(size_t)t * k + lane] = id; w[(size_t)t * k + lane] = mine / wsum; }
 }
+bool moe_router_norms(int type, int n_expert, int K) { return (type == T_F32 || type == T_F16) && n_expert <= 64 && (K & 255) == 0 && K <= 16384; }
 hipError_t launch_moe_router(int type, const uint8_t *W, int n_expert, int K, const float *x, int T, int k, float *logits_out, int32_t *ids, float *w,
-                             hipStream_t st, const int32_t *forced) {
-    if (n_expert > 64 || (type != T_F32 && type != T_F16) || T <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(moe_router_kernel, dim3(T), dim3(256), 0, st, type, W, n_expert, K, x, k, logits_out, ids, w, forced);
+                             hipStream_t st, const int32_t *forced, const float *nw, float eps) {
+    if (n_expert < 1 || n_expert > 64 || k > n_expert || (type != T_F32 && type != T_F16) || T <= 0 || (nw && (T != 1 || !moe_router_norms(type, n_expert, K)))) return hipErrorInvalidValue;
+    if (nw) hipLaunchKernelGGL((moe_router_kernel<1, true>), dim3(1), dim3(1024), (size_t)K * 4, st, type, W, n_expert, K, x, nw, eps, T, k, logits_out, ids, w, forced);
+    else if (T >= 64 && (K & 255) == 0 && K <= 8192) {
+        const size_t lds = (size_t)4 * K * 4;
+        if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_router_kernel<4, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipLaunchKernelGGL((moe_router_kernel<4, false>), dim3((T + 3) / 4), dim3(1024), lds, st, type, W, n_expert, K, x, nullptr, 0.0f, T, k, logits_out, ids, w, forced);
+    } else if ((K & 255) == 0 && K <= 16384)
+        hipLaunchKernelGGL((moe_router_kernel<1, false>), dim3(T), dim3(1024), (size_t)K * 4, st, type, W, n_expert, K, x, nullptr, 0.0f, T, k, logits_out, ids, w, forced);
+    else {
+        if (!logits_out) return hipErrorInvalidValue;
+        const hipError_t e = launch_mmv_float(type, W, n_expert, K, x, T, logits_out, n_expert, nullptr, st);
+        return e != hipSuccess ? e : launch_moe_route(logits_out, T, n_expert, k, ids, w, st, forced);
+    }
     return hipGetLastError();
 }
 __global__ void moe_combine_kernel(float *x, const float *eo, const float *w, int T, int E, int k, size_t eo_stride) {

@@ -1626,23 +1626,43 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
 
         // --- feed-forward block
         if (hp.n_expert > 0) {
-            HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, xn_, &aq_e_,
+            const int KU = hp.n_expert_used, group_min = g_moe_group_min;
+            // a single-token step: the token's selected experts share one launch per projection (the workgroups are divided
+            // among them; each reads its own expert index on the device): gate/up with SwiGLU, then down with the Q8_K
+            // quantisation of its own expert's activation in the prologue
+            MMVQArgs one_gu{}, one_down{};
+            bool one_step = false;
+            if (T == 1 && KU >= 2 && KU <= 8 && (int)cp.n_ubatch >= KU && L.gate_exps.type == L.up_exps.type) {
+                MMVQArgs &a = one_gu, &d = one_down;
+                a.n_seg = 2; a.K = E; a.T = 1; a.epi = EPI_SWIGLU; a.n_sel = KU; a.sel_out_stride = FF;
+                a.seg[0] = make_seg(L.gate_exps, ffn_, FF, nullptr, moe_ids_);
+                a.seg[1] = make_seg(L.up_exps, ffn_u_, FF, nullptr, moe_ids_);
+                chunk_act(a, aq_e_, E, 0);
+                // (RMSNorm + quantise again in the launch's prologue - the arithmetic of the norm_quant launch, so the same codes: the
+                // weight stream's gate | up form takes its activation that way, and with it the selected experts stream like the dense feed-forward does)
+                if (can_fuse(E, 1) && !act_is_q80(L.gate_exps.type)) { a.fuse_mode = 1; a.nx = x_; a.nw = (const float *)L.ffn_norm.data; a.neps = hp.eps; }
+                d.n_seg = 1; d.K = FF; d.T = 1; d.epi = EPI_STORE; d.fuse_mode = 2; d.nx = ffn_; d.n_sel = KU; d.sel_nx_stride = FF; d.sel_out_stride = E;
+                d.seg[0] = make_seg(L.down_exps, moe_out_, E, nullptr, moe_ids_);
+                chunk_act(d, aq_ff_, FF, 0);
+                one_step = mmvq_fast_applicable(a) && mmvq_fast_applicable(d);
+            }
+            // (then the norm is the router's own, and nobody reads a normed or quantised row)
+            const bool router_norm = one_step && one_gu.fuse_mode == 1 && T < group_min && x_parts == 1 && moe_router_norms(L.gate_inp.type, hp.n_expert, E);
+            if (!router_norm) HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, xn_, &aq_e_,
                                          !act_is_q80(L.gate_exps.type) || !act_is_q80(L.up_exps.type), act_is_q80(L.gate_exps.type) || act_is_q80(L.up_exps.type), stream_, nullptr, nullptr, mmq_ws_.p, x_parts));
             x_parts = 1;
             prep_owner_ = nullptr;
             prof_mark("norm_quant");
             if (L.gate_inp.type == T_F32 || L.gate_inp.type == T_F16) {
-                HIP_TRY(launch_moe_router(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, xn_, T, hp.n_expert_used, router_, moe_ids_, moe_w_, stream_,
-                                          moe_forced_T_ == T ? d_moe_forced_ + (size_t)il * T * hp.n_expert_used : nullptr));
+                HIP_TRY(launch_moe_router(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, router_norm ? x_ : xn_, T, hp.n_expert_used, router_, moe_ids_, moe_w_, stream_,
+                                          moe_forced_T_ == T ? d_moe_forced_ + (size_t)il * T * hp.n_expert_used : nullptr, router_norm ? (const float *)L.ffn_norm.data : nullptr, hp.eps));
             } else {
                 HIP_TRY(launch_mmv_float(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, xn_, T, router_, hp.n_expert, nullptr, stream_));
                 HIP_TRY(launch_moe_route(router_, T, hp.n_expert, hp.n_expert_used, moe_ids_, moe_w_, stream_,
                                          moe_forced_T_ == T ? d_moe_forced_ + (size_t)il * T * hp.n_expert_used : nullptr));
             }
             prof_mark("moe_route");
-            const int KU = hp.n_expert_used;
             const bool exps_q = is_quant(L.gate_exps.type) && is_quant(L.up_exps.type) && is_quant(L.down_exps.type);
-            const int group_min = g_moe_group_min;
             if (exps_q && T >= group_min && aq_eg_.qs) {
                 // ggml_mul_mat_id on a batch: group the (token, rank) pairs by expert, one contiguous activation batch per
                 // expert (its weights are read once per batch, through the same batched kernels as the dense projections)
@@ -1713,30 +1733,11 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
                 continue;
             }
-            // single-token step: the token's selected experts share one launch per projection (the workgroups are divided
-            // among them; each reads its own expert index on the device): gate/up with SwiGLU, then down with the Q8_K
-            // quantisation of its own expert's activation in the prologue
-            bool experts_done = false;
-            if (T == 1 && KU >= 2 && KU <= 8 && (int)cp.n_ubatch >= KU && L.gate_exps.type == L.up_exps.type) {
-                MMVQArgs a{};
-                a.n_seg = 2; a.K = E; a.T = 1; a.epi = EPI_SWIGLU; a.n_sel = KU; a.sel_out_stride = FF;
-                a.seg[0] = make_seg(L.gate_exps, ffn_, FF, nullptr, moe_ids_);
-                a.seg[1] = make_seg(L.up_exps, ffn_u_, FF, nullptr, moe_ids_);
-                chunk_act(a, aq_e_, E, 0);
-                // (RMSNorm + quantise again in the launch's prologue - the same arithmetic as the norm_quant launch that fed the router, so the same codes: the
-                // weight stream's gate | up form takes its activation that way, and with it the selected experts stream like the dense feed-forward does)
-                if (can_fuse(E, 1) && !act_is_q80(L.gate_exps.type)) { a.fuse_mode = 1; a.nx = x_; a.nw = (const float *)L.ffn_norm.data; a.neps = hp.eps; }
-                MMVQArgs d{};
-                d.n_seg = 1; d.K = FF; d.T = 1; d.epi = EPI_STORE; d.fuse_mode = 2; d.nx = ffn_; d.n_sel = KU; d.sel_nx_stride = FF; d.sel_out_stride = E;
-                d.seg[0] = make_seg(L.down_exps, moe_out_, E, nullptr, moe_ids_);
-                chunk_act(d, aq_ff_, FF, 0);
-                if (mmvq_fast_applicable(a) && mmvq_fast_applicable(d)) {
-                    HIP_TRY(launch_mmvq(a, stream_));          // the weight stream where it has a form for the shape, else the register ring (bit-identical)
-                    HIP_TRY(launch_mmvq(d, stream_));
-                    experts_done = true;
-                }
+            if (one_step) {
+                HIP_TRY(launch_mmvq(one_gu, stream_));         // the weight stream where it has a form for the shape, else the register ring (bit-identical)
+                HIP_TRY(launch_mmvq(one_down, stream_));
             }
-            for (int t = 0; t < T && !experts_done; t++) {
+            for (int t = 0; t < T && !one_step; t++) {
                 for (int j = 0; j < KU; j++) {
                     const int32_t *esel = moe_ids_ + (size_t)t * KU + j;
                     MMVQArgs a{};
