@@ -346,14 +346,58 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float *x, const f
         if (yh) yh[(size_t)blockIdx.x * n + i] = (_Float16)v;
     }
 }
-hipError_t launch_layer_norm(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, hipStream_t st) {
-    hipLaunchKernelGGL(layer_norm_kernel, dim3((unsigned)T), dim3(256), 0, st, x, w, b, n, eps, y, (_Float16 *)nullptr);
+// The same with a wave to a row that stays in registers: one trip to memory instead of three, no barriers.  187 rows of 768: 4.3 -> 2.9 us.
+// yp (optional): the row once more, in pinned host memory (the encoder's last layer; 187 rows: 12.6 us, PCIe's time, and no gathering, copying and storing launches behind it, 17).
+template <int NV>
+__global__ __launch_bounds__(256) void layer_norm_wave_kernel(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, _Float16 *yh, float *yp) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), n4 = n >> 2;
+    if (row >= T) return;
+    const f32x4 *xr = reinterpret_cast<const f32x4 *>(x + (size_t)row * n), *w4 = reinterpret_cast<const f32x4 *>(w), *b4 = reinterpret_cast<const f32x4 *>(b);
+    f32x4 v[NV], g[NV], h[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) { const int i = lane + 64 * j < n4 ? lane + 64 * j : n4 - 1; v[j] = xr[i]; g[j] = w4[i]; h[j] = b4[i]; }
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < NV; j++) if (lane + 64 * j < n4) s += ((double)v[j].x + (double)v[j].y) + ((double)v[j].z + (double)v[j].w);
+    s = wave_sum(s);
+    const float mean = (float)(s / (double)n);
+    double s2 = 0.0;
+#pragma unroll
+    for (int j = 0; j < NV; j++)
+        if (lane + 64 * j < n4) {
+            v[j] -= mean;
+            s2 += ((double)(v[j].x * v[j].x) + (double)(v[j].y * v[j].y)) + ((double)(v[j].z * v[j].z) + (double)(v[j].w * v[j].w));
+        }
+    s2 = wave_sum(s2);
+    const float scale = 1.0f / sqrtf((float)(s2 / (double)n) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = lane + 64 * j;
+        if (i >= n4) break;
+        const f32x4 o = (v[j] * scale) * g[j] + h[j];
+        reinterpret_cast<f32x4 *>(y + (size_t)row * n)[i] = o;
+        if (yh) reinterpret_cast<f16x4 *>(yh + (size_t)row * n)[i] = f16x4{(_Float16)o.x, (_Float16)o.y, (_Float16)o.z, (_Float16)o.w};
+        if (yp) reinterpret_cast<f32x4 *>(yp + (size_t)row * n)[i] = o;
+    }
+}
+hipError_t launch_layer_norm_h(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, void *yh, hipStream_t st, float *yp) {
+    const uintptr_t at = (uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)y | (uintptr_t)yp | ((uintptr_t)yh << 1);
+    const dim3 rows((unsigned)((T + 3) / 4)), t(256);
+    _Float16 *h = reinterpret_cast<_Float16 *>(yh);
+    if ((n & 3) != 0 || (at & 15) != 0 || n > 2048) {
+        hipLaunchKernelGGL(layer_norm_kernel, dim3((unsigned)T), dim3(256), 0, st, x, w, b, n, eps, y, h);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess || !yp ? e : launch_rows_to_host(y, yp, (size_t)T * n, st);
+    }
+    if (n <= 256) hipLaunchKernelGGL(layer_norm_wave_kernel<1>, rows, t, 0, st, x, w, b, n, T, eps, y, h, yp);
+    else if (n <= 768) hipLaunchKernelGGL(layer_norm_wave_kernel<3>, rows, t, 0, st, x, w, b, n, T, eps, y, h, yp);
+    else if (n <= 1024) hipLaunchKernelGGL(layer_norm_wave_kernel<4>, rows, t, 0, st, x, w, b, n, T, eps, y, h, yp);
+    else hipLaunchKernelGGL(layer_norm_wave_kernel<8>, rows, t, 0, st, x, w, b, n, T, eps, y, h, yp);
     return hipGetLastError();
 }
-hipError_t launch_layer_norm_h(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, void *yh, hipStream_t st) {
-    hipLaunchKernelGGL(layer_norm_kernel, dim3((unsigned)T), dim3(256), 0, st, x, w, b, n, eps, y, reinterpret_cast<_Float16 *>(yh));
-    return hipGetLastError();
-}
+hipError_t launch_layer_norm(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, hipStream_t st) { return launch_layer_norm_h(x, w, b, n, T, eps, y, nullptr, st); }
 
 // row softmax: y = softmax(x*scale + mask)   (ggml_soft_max_ext, max_bias = 0)
 __global__ __launch_bounds__(256) void soft_max_kernel(const float *x, const float *mask, float *y, int n, float scale) {

@@ -260,9 +260,9 @@ struct MMF16Few {
     const float *cs; const int32_t *cell; uint16_t *kc, *vc; int n_ctx;       // FEW_ROPE: cos, sin of every token's 32 pairs, the tokens' cells, the layer's cache planes
 };
 template <int NW, int EPI, int TT, int PD, bool XF>
-__global__ __launch_bounds__(64 * NW) void mmf16_few_kernel(const MMF16Few a) {
+__global__ __launch_bounds__(64 * NW, EPI == FEW_SWIGLU && NW == 4 && TT == 1 ? 3 : 1) void mmf16_few_kernel(const MMF16Few a) {
     constexpr int NP = EPI == FEW_PLAIN ? 1 : 2, ROWS = EPI == FEW_ROPE ? 64 : 32;
-    constexpr int LD = 36, LDR = 72, STAGE = (NP + TT) * 32 * LDR;                                     // floats per row of a partial tile; halves per row of a staged chunk
+    constexpr int LD = 36, LDR = 64, STAGE = (NP + TT) * 32 * LDR;                                     // floats per row of a partial tile; halves per row of a staged chunk
     constexpr int PART_BYTES = NW * NP * TT * 32 * LD * 4, STAGE_BYTES = NW * STAGE * 2;
     __shared__ __attribute__((aligned(16))) uint8_t smem[PART_BYTES > STAGE_BYTES ? PART_BYTES : STAGE_BYTES];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m = lane & 31, kg = lane >> 5;
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(64 * NW) void mmf16_few_kernel(const MMF16Few a) {
     auto put = [&](const Slot &v) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            _Float16 *d = stage + (r8 + 8 * j) * LDR + c8;
+            _Float16 *d = stage + (r8 + 8 * j) * LDR + (c8 ^ (8 * r8));          // (piece c of row r at c ^ (r & 7): no bank conflicts, and no padding)
 #pragma unroll
             for (int p = 0; p < NP; p++) *reinterpret_cast<f16x8 *>(d + p * 32 * LDR) = v.w[p][j];
 #pragma unroll
@@ -324,15 +324,16 @@ __global__ __launch_bounds__(64 * NW) void mmf16_few_kernel(const MMF16Few a) {
         }
     };
     auto use = [&]() {
-        const _Float16 *f = stage + m * LDR + 8 * kg;
+        const _Float16 *f = stage + m * LDR;
+        const int x = 8 * (m & 7);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             f16x8 w[NP];
 #pragma unroll
-            for (int p = 0; p < NP; p++) w[p] = *reinterpret_cast<const f16x8 *>(f + p * 32 * LDR + 16 * j);
+            for (int p = 0; p < NP; p++) w[p] = *reinterpret_cast<const f16x8 *>(f + p * 32 * LDR + ((16 * j + 8 * kg) ^ x));
 #pragma unroll
             for (int t = 0; t < TT; t++) {
-                const f16x8 b = *reinterpret_cast<const f16x8 *>(f + (NP + t) * 32 * LDR + 16 * j);
+                const f16x8 b = *reinterpret_cast<const f16x8 *>(f + (NP + t) * 32 * LDR + ((16 * j + 8 * kg) ^ x));
 #pragma unroll
                 for (int p = 0; p < NP; p++) acc[p][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[p], b, acc[p][t], 0, 0, 0);
             }
@@ -405,7 +406,7 @@ void few_launch(const MMF16Few &a, hipStream_t st) {
         hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 2, 2, XF>), dim3(gx, (gy + 1) / 2), dim3(64 * NW), 0, st, a);
         return;
     }
-    hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF || (EPI == FEW_SWIGLU && NW == 4) ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
 }
 }  // namespace
 

@@ -1402,7 +1402,8 @@ hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
             HIP_TRY(launch_mmf16_few_swiglu(L.gate.data, L.up.data, FF, E, xh, T, hh, stream_));
             prof_mark("ffn_gate_up");
             HIP_TRY(launch_mmf16_few(L.down.data, E, FF, hh, true, T, x_, xn_, nullptr, stream_));
-            HIP_TRY(launch_layer_norm_h(x_, (const float *)L.layer_out_norm.data, (const float *)L.layer_out_norm_b.data, E, T, hp.eps, x_, xh, stream_));
+            HIP_TRY(launch_layer_norm_h(x_, (const float *)L.layer_out_norm.data, (const float *)L.layer_out_norm_b.data, E, T, hp.eps, x_, xh, stream_, il == hp.n_layer - 1 ? embd_out_ : nullptr));
+            embd_on_host_ = il == hp.n_layer - 1 && embd_out_;
             prof_mark("ffn_down");
             if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
             continue;
@@ -1891,6 +1892,7 @@ hipError_t Context::run_output(int n_out, int out_base) {
     if (n_out <= 0) return hipSuccess;
     const HParams &hp = model->hp;
     const int E = hp.n_embd, V = hp.n_vocab;
+    if (embd_on_host_) return hipSuccess;                    // (the last layer's norm stored them)
     // (a single-token step has one row and it is the flagged one: no gather launch)
     float *const xo = cur_T_ == 1 && n_out == 1 ? x_ : xo_;
     if (xo != x_) HIP_TRY(launch_gather_rows_f32(x_, d_outrow_, n_out, E, xo_, stream_));
@@ -2005,6 +2007,8 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         h_tok[i] = tokens[i]; h_pos[i] = pos[i]; h_seq[i] = seq[i]; h_cell[i] = tcell[(size_t)i]; h_mask[i] = seqmask[i];
         if (flags[i]) h_out[n_out++] = i;
     }
+    embd_out_ = model->hp.encoder && n_out == n && out_base == 0 ? h_embd_ : nullptr;
+    embd_on_host_ = false;
     if (!one_token_) {
         stage_pending_ = true;
         if (hipMemcpyAsync(d_stage_, h_stage_, (size_t)((uint8_t *)(h_mask + n) - h_stage_), hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "token upload failed"; return -1; }
@@ -2326,7 +2330,7 @@ float *Context::embeddings_ith(int i) {
     if (i < 0 || i >= (int)out_row_of_batch_.size() || out_row_of_batch_[(size_t)i] < 0) return nullptr;
     const int E = model->hp.n_embd;
     if (!embd_fetched_) {
-        if (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_embd_, h_embd_, (size_t)n_out_last_ * E, stream_) != hipSuccess) return nullptr;
+        if (!embd_on_host_ && (hipSetDevice(model->device) != hipSuccess || launch_rows_to_host(d_embd_, h_embd_, (size_t)n_out_last_ * E, stream_) != hipSuccess)) return nullptr;
         if (hipStreamSynchronize(stream_) != hipSuccess) return nullptr;
         unread_steps_ = 0;
         embd_fetched_ = true;

@@ -307,6 +307,8 @@ class Context {
     int cur_max_pos_ = 0;                            // largest position of the micro-batch being decoded
     float *d_embd_ = nullptr, *h_embd_ = nullptr;   // [n_ubatch][n_embd], embeddings mode
     bool embd_fetched_ = false, last_was_embd_ = false;
+    float *embd_out_ = nullptr;                      // an encoder's batch whose tokens are all flagged: where its last norm stores their rows, too (h_embd_)
+    bool embd_on_host_ = false;                      // ... and did
     // batched single-token steps: per-token lists of the 64-cell chunks that hold cells of the token's sequence
     int32_t *h_chunks_ = nullptr, *d_chunks_ = nullptr;     // [64][chunk_stride_] lists, then [64] counts
     int chunk_stride_ = 0, chunk_lmax_ = 0, chunk_cap_ = 0;   // cap = grid size used for the lists (>= lmax; rounded up for graph reuse)                 // lmax = longest list of the current batch (0 = lists not in use)
