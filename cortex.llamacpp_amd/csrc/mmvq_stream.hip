@@ -221,10 +221,9 @@ MI355_ST_KERNEL(mmvq_stream_head)
 void mmvq_stream_set_probe(unsigned long long *p) { (void)hipMemcpyToSymbol(HIP_SYMBOL(g_stream_probe), &p, sizeof(p)); }
 #endif
 
-#ifndef MI355_STREAM_Q80_MIN_MB
-#define MI355_STREAM_Q80_MIN_MB 16
-#endif
-static constexpr size_t STREAM_Q80_MIN_BYTES = (size_t)MI355_STREAM_Q80_MIN_MB << 20;   // launches of Q8_0 tensors only: below this the register ring (TinyLlama: 850 vs 816 tok/s)
+// Launches of Q8_0 tensors only: from here on the stream is the faster one.  us, stream / register ring, of a 2048-column model: Q | K | V (5.6 MB) 5.2 / 7.0, ffn_down (12.3 MB) 6.1 / 9.3,
+// attn_output (4.5 MB), which then quantises its input itself, 4.8 / 6.1; smaller tensors have not been timed
+static constexpr size_t STREAM_Q80_MIN_BYTES = (size_t)4 << 20;
 
 bool mmvq_stream_applicable(const MMVQArgs &a) {
     if (a.T != 1 || a.K <= 0 || (a.K % 256) != 0) return false;      // (whole super-blocks; a partial last pass decodes zero-scale slices, as on the register ring)
@@ -243,10 +242,7 @@ bool mmvq_stream_applicable(const MMVQArgs &a) {
     if (swiglu && a.fuse_mode != 1) return false;
     if (swiglu && (a.n_seg != 2 || a.seg[0].type != a.seg[1].type || a.seg[0].n_rows != a.seg[1].n_rows || a.seg[0].row_bytes != a.seg[1].row_bytes)) return false;
     const int n = swiglu ? 1 : a.n_seg;
-    // Q8_0 tensors: 1.06 B per weight through LDS and no shorter decode; measured on TinyLlama-1.1B Q8_0 the register ring is 4 %
-    // faster (850 vs 816 tok/s), so launches made of Q8_0 tensors only stay there (a Q8_0 attn_k / attn_v beside a K-quant attn_q
-    // of an 8-expert file streams with it)
-    // (round 4: from STREAM_Q80_MIN_BYTES on they stream too - at Llama-3-8B's sizes the launch is bound by its bytes like any other)
+    // (a Q8_0 attn_k / attn_v beside a K-quant attn_q of an 8-expert file streams with it)
     bool all_q80 = true;
     size_t launch_bytes = 0;
     for (int s = 0; s < (swiglu ? 2 : n); s++) { all_q80 = all_q80 && a.seg[s].type == T_Q8_0; launch_bytes += (size_t)a.seg[s].n_rows * a.seg[s].row_bytes; }

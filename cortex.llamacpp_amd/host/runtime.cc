@@ -1615,13 +1615,23 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             HIP_TRY(launch_decode_engine(d_engine_layers_ + il, E, FF, d_engine_gran_, d_engine_epoch_, il, il == engine_probe_layer_ ? d_engine_probe_ : nullptr, stream_));
             continue;
         }
+        // a step's Q8_0 attn_output where it can be a weight stream: that form quantises its input itself
+        bool o_fuse = false;
+        if (T == 1 && !attn_out_done && !tp && L.wo.type == T_Q8_0) {
+            MMVQArgs o{};
+            o.n_seg = 1; o.K = (int)L.wo.K; o.T = 1; o.epi = EPI_ADD; o.fuse_mode = 2; o.nx = att_;
+            o.seg[0] = make_seg(L.wo, x_, E, x_, nullptr);
+            o_fuse = mmvq_stream_applicable(o);
+        }
         if (attn_out_done) {   // the mat-vec ran inside the attention launch (attn_out.hip)
             if (tp) HIP_TRY(tp_reduce_into_x(T));
         } else if (tp) {   // this rank's partial sum (rank 0 carries the residual), then the exchange: x = sum over ranks
             HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, tp_part_, E, hp.tp_rank == 0 ? x_ : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
             HIP_TRY(tp_reduce_into_x(T));
         } else {
+            if (o_fuse) { pending_fuse_.mode = 2; pending_fuse_.x = att_; }
             HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, x_, E, x_, EPI_ADD, late_sum ? &x_parts : nullptr));
+            pending_fuse_ = Fuse();
         }
         prof_mark("attn_out");
 
