@@ -1,6 +1,8 @@
 // attn_decode_dev.h — device side of the decode attention (one 64-cell chunk of one kv head per 256-thread workgroup).
 // Shared by attn.hip (one launch per layer) and decode_mega.hip (a phase of the whole-step kernel).
 #pragma once
+#include <type_traits>
+
 #include "kernels.h"
 #include "quant_dev.h"
 
@@ -105,9 +107,10 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     if (tid < C && c_lo + tid < n_ctx) { cpos = a.cell_pos[c_lo + tid]; cseq = a.cell_seq[c_lo + tid]; }
     const int32_t tpos = a.tok_pos[t];
     const int tseq = a.tok_seq[t];
-    if (a.T > 1) {   // (FUSED with T > 1 is the store-fused form of a batched step: no tickets, the merge is its own launch)
-        // batched steps (one token per sequence): most chunks hold other sequences' cells only.  Decide that before
-        // touching K / V: such a chunk publishes (m, l) = (-inf, 0) and leaves; the merge skips it.
+    if (a.T > 1 && !a.tok_chunks) {
+        // batched steps (one token per sequence) without chunk lists: most chunks hold other sequences' cells only.  Decide that before
+        // touching K / V: such a chunk publishes (m, l) = (-inf, 0) and leaves; the merge skips it.  (A list names the chunks that hold cells of the token's sequence, and
+        // the cells' answer would be a trip to memory in front of K's and V's)
         const int mine = (tid < C && cpos >= 0 && cpos <= tpos && ((cseq >> tseq) & 1ull)) ? 1 : 0;
         if (!__syncthreads_or(mine)) {
             if (tid < R) {
@@ -392,7 +395,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
         if (d == 0) { cstf<COH>(dst + D, ml[2 * r]); cstf<COH>(dst + D + 1, ml[2 * r + 1]); }
     }
     if (!FUSED) return;
-    if (fz.counters == nullptr) return;               // store-fused only: the merge runs as its own launch
+    if (fz.counters == nullptr) return;               // store-fused only: the merge runs as its own launch (batched steps: in this launch it takes as long, ticks of 2 to 16 tokens 1 % slower to 1 % faster)
     if (fz.probe && tid == 0) fz.probe[2 * (sp * a.G + g) + 1] = wall_clock64();
 
     // ---- FUSED: ticket; the last workgroup of this kv head merges.  The merge also quantises whole 256-element blocks of
@@ -422,11 +425,13 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     float *merged = accs;                              // [RM * D]
     float *wgt = GP > 1 ? accs + RM * D : S;           // [RM][64] split weights (S is free now, but holds R * C floats only)
     // The merge is a chain of memory round trips (~1.5 us each: the partials come from other XCDs).  Every output still
-    // sums its splits in order (the combine kernel's arithmetic), but the partials of the first 32 splits of all of this
+    // sums its splits in order (the combine kernel's arithmetic), but the partials of the first UB splits of all of this
     // thread's outputs are requested BEFORE the (m, l) pairs, so the weight computation runs under them: ticket, one trip
-    // for (m, l) + 32 splits, one more per further 32 splits (it was ticket + (m, l) + one trip per 8 splits and output).
-    constexpr int NE = (RM * D + 255) / 256, UB = NE > 4 ? 16 : 32;     // (NE * UB partials in registers per thread)
-    float macc[NE], x[NE][UB];
+    // for (m, l) + UB splits, one more per further UB (it was ticket + (m, l) + one trip per 8 splits and output).  UB by the splits there are: a load past them is one more
+    // trip of the fabric's (us a launch of a step, 4 kv heads of 8 heads of 64 behind 93 cells: 10.0 with thirty-two loads an output for four splits and the argument
+    // segment read field by field, 8.6)
+    constexpr int NE = (RM * D + 255) / 256;
+    float macc[NE];
     const float *pp[NE];
     int wr[NE];
 #pragma unroll
@@ -436,43 +441,49 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
         wr[j] = r * 64;
         macc[j] = 0.0f;
     }
-    auto request = [&](int s0) {
+    const auto merge = [&](auto ub) __attribute__((always_inline)) {
+        constexpr int UB = decltype(ub)::value;        // (NE * UB partials in registers per thread)
+        float x[NE][UB];
+        auto request = [&](int s0) {
 #pragma unroll
-        for (int u = 0; u < UB; u++) {
-            const int s2 = s0 + u < splits ? s0 + u : splits - 1;              // clamped: straight-line loads
+            for (int u = 0; u < UB; u++) {
+                const int s2 = s0 + u < splits ? s0 + u : splits - 1;          // clamped: straight-line loads
 #pragma unroll
-            for (int j = 0; j < NE; j++) x[j][u] = __hip_atomic_load(pp[j] + (size_t)s2 * (D + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int j = 0; j < NE; j++) x[j][u] = __hip_atomic_load(pp[j] + (size_t)s2 * (D + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        };
+        request(0);
+        for (int r = wave; r < RM; r += 4) {           // same arithmetic as flash_attn_combine_kernel
+            const float *p = a.part + ((size_t)hb + r) * stride_s * (D + 2);
+            float m = -INFINITY, l = 0.0f;
+            if (lane < splits) {
+                m = __hip_atomic_load(p + (size_t)lane * (D + 2) + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                l = __hip_atomic_load(p + (size_t)lane * (D + 2) + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            const float M = wave_max(m);
+            const float w = (lane < splits && m != -INFINITY) ? expf(m - M) : 0.0f;
+            const float den = wave_sum(w * l);
+            const float inv = 1.0f / den;
+            wgt[r * 64 + lane] = w * inv;
+        }
+        __syncthreads();
+        if (fz.probe && tid == 0) fz.probe[4096 + 8 * g + 1] = wall_clock64();
+        for (int s0 = 0;;) {
+#pragma unroll
+            for (int u = 0; u < UB; u++) {
+                if (s0 + u < splits) {                                         // workgroup-uniform
+#pragma unroll
+                    for (int j = 0; j < NE; j++) macc[j] += wgt[wr[j] + s0 + u] * x[j][u];
+                }
+            }
+            s0 += UB;
+            if (s0 >= splits) break;
+            request(s0);
         }
     };
-    request(0);
-    for (int r = wave; r < RM; r += 4) {               // same arithmetic as flash_attn_combine_kernel
-        const float *p = a.part + ((size_t)hb + r) * stride_s * (D + 2);
-        float m = -INFINITY, l = 0.0f;
-        if (lane < splits) {
-            m = __hip_atomic_load(p + (size_t)lane * (D + 2) + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            l = __hip_atomic_load(p + (size_t)lane * (D + 2) + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        const float M = wave_max(m);
-        const float w = (lane < splits && m != -INFINITY) ? expf(m - M) : 0.0f;
-        const float den = wave_sum(w * l);
-        const float inv = 1.0f / den;
-        wgt[r * 64 + lane] = w * inv;
-    }
-    __syncthreads();
-    if (fz.probe && tid == 0) fz.probe[4096 + 8 * g + 1] = wall_clock64();
-    const int E = H * D;
-    for (int s0 = 0;;) {
-#pragma unroll
-        for (int u = 0; u < UB; u++) {
-            if (s0 + u < splits) {                                             // workgroup-uniform
-#pragma unroll
-                for (int j = 0; j < NE; j++) macc[j] += wgt[wr[j] + s0 + u] * x[j][u];
-            }
-        }
-        s0 += UB;
-        if (s0 >= splits) break;
-        request(s0);
-    }
+    if (splits <= 4) merge(std::integral_constant<int, 4>());
+    else if (splits <= 12) merge(std::integral_constant<int, 12>());
+    else merge(std::integral_constant<int, (NE > 4 ? 16 : 32)>());
 #pragma unroll
     for (int j = 0; j < NE; j++) {
         const int e = tid + 256 * j;
@@ -502,7 +513,6 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
             }
         }
     }
-    (void)E;
     if (fz.probe) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (tid == 0) fz.probe[4096 + 8 * g + 3] = wall_clock64();
@@ -511,6 +521,15 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
 
 template <int R, int TK, int TV, bool FUSED, bool COH = false, int D = 128>
 __global__ __launch_bounds__(256) void flash_attn_decode_kernel(const AttnArgs a, const float *cs_table, int n_rot, const DecodeFuse fz) {
+    // (the argument segment is cold at every launch: a read of each of its lines at once, instead of one behind the other where a field is first used)
+    {
+        struct KArgs { AttnArgs a; const float *cs; int n_rot; DecodeFuse fz; };
+        const __attribute__((address_space(4))) unsigned *ka = (const __attribute__((address_space(4))) unsigned *)__builtin_amdgcn_kernarg_segment_ptr();
+        unsigned acc = 0;
+#pragma unroll
+        for (int i = 0; i < (int)((sizeof(KArgs) + 63) / 64); i++) acc ^= ka[i * 16];
+        asm volatile("" :: "s"(acc));
+    }
     flash_attn_decode_item<R, TK, TV, FUSED, COH, D>(a, cs_table, n_rot, fz, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
