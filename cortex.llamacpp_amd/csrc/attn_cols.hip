@@ -47,7 +47,7 @@ template <> struct VWord<8> { typedef u32x2 T; };
 template <int DH> constexpr int cols_merge_words = (DH / 32) * 16 * 65;      // a wave's O, [16 * tile + register][lane], rows of 65: the readers take registers, not lanes, side by side
 template <int DH> constexpr int cols_wave_words = (DH / 32) * CK * 2 + CK + 2 * CK;      // a chunk's scales [k, v][block][key], positions, sequence masks
 template <bool F16, int DH> constexpr int cols_q_stride = (F16 ? 2 * DH : DH) + 16;                            // bytes of a column's query as an operand
-template <bool F16, int DH, int NW> constexpr int cols_lds_words = NW * cols_merge_words<DH> + std::max(NW * 64, CK * cols_q_stride<F16, DH> / 4 + CK * (DH / 32));
+template <bool F16, int DH, int NW> constexpr int cols_lds_words = NW * cols_merge_words<DH> + std::max(NW * 64 + CK, CK * cols_q_stride<F16, DH> / 4 + CK * (DH / 32));
 
 struct ColsArgs {
     AttnArgs a;
@@ -335,7 +335,9 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
     const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
 #pragma unroll
     for (int w = 0; w < NW; w++) l_all += s_ml[w * 64 + 32 + n] * __builtin_amdgcn_exp2f(s_ml[w * 64 + n] - m_ref);
-    const float own = __builtin_amdgcn_exp2f(m_run - m_ref), f = c.nsp > 1 ? own : own / l_all;
+    const float f = __builtin_amdgcn_exp2f(m_run - m_ref);
+    float *const s_l = s_ml + NW * 64;                       // (a column's sum, for the end)
+    if (wave == 0 && kg == 0) s_l[n] = l_all;
 #pragma unroll
     for (int db = 0; db < NB; db++)
 #pragma unroll
@@ -350,14 +352,19 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
     const int cw = lane / LPC, d0 = (lane - cw * LPC) * 4;
     for (int b = wave; b < CK / CPB; b += NW) {
         const int cb = b * CPB + cw, gc = blockIdx.y * CK + cb;
+        const float l = c.nsp > 1 ? 1.0f : s_l[cb];          // (divided by once, behind the sum over the waves)
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int d = d0 + e, m = d / DPL, db = d - m * DPL, r = (m & 3) + 4 * (m >> 3), o = (db * 16 + r) * 65 + cb + 32 * ((m >> 2) & 1);
-            float x = 0.0f;
+            float x[NW];                                     // (in pairs: three roundings instead of seven)
 #pragma unroll
-            for (int w = 0; w < NW; w++) x += smem[w * cols_merge_words<DH> + o];
-            v[e] = x;
+            for (int w = 0; w < NW; w++) x[w] = smem[w * cols_merge_words<DH> + o];
+#pragma unroll
+            for (int h = NW / 2; h >= 1; h >>= 1)
+#pragma unroll
+                for (int w = 0; w < h; w++) x[w] += x[w + h];
+            v[e] = x[0] / l;
         }
         if (blockIdx.y * CK + b * CPB >= n_cols) break;      // (wave-uniform)
         const bool in = gc < n_cols;
