@@ -21,16 +21,28 @@ __global__ __launch_bounds__(256) void norm_quant_kernel(const float *__restrict
                                                          int n, float eps, int do_norm, float *__restrict__ yf,
                                                          ActQuant q, int want_q8k, int want_q80, int8_t *__restrict__ bh, int8_t *__restrict__ bl) {
     __shared__ double red[4];
-    // grid = (rows, splits): each workgroup re-derives the row scale (cheap, L2-resident) and quantises its share of blocks
+    // grid = (rows, splits): each workgroup re-derives the row scale (cheap, L2-resident) and quantises its share of blocks.  A wave's first block and the whole row are requested
+    // together (rows of up to 8192): one trip to memory, where the sum's loads, the block and the weights were three (us, 4 rows of 4096: 4.2 -> 3.85)
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *xr = x + (size_t)row * n;
+    const int nblk = n >> 8, b0 = blockIdx.y * 4 + wave, e1 = (b0 < nblk ? b0 : nblk > 0 ? nblk - 1 : 0) * 256 + lane * 4;
+    float4 v1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), w1 = v1;
+    if (nblk > 0) { v1 = *reinterpret_cast<const float4 *>(xr + e1); if (do_norm) w1 = *reinterpret_cast<const float4 *>(w + e1); }
     float scale = 1.0f;
     if (do_norm) {
         double s = 0.0;
-        for (int i = tid * 4; i < n; i += 256 * 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(xr + i);
-            s += (double)(v.x * v.x); s += (double)(v.y * v.y); s += (double)(v.z * v.z); s += (double)(v.w * v.w);
-        }
+        const auto add = [&](const float4 &v) { s += (double)(v.x * v.x); s += (double)(v.y * v.y); s += (double)(v.z * v.z); s += (double)(v.w * v.w); };
+        const auto held = [&](auto nv) __attribute__((always_inline)) {
+            constexpr int NV = decltype(nv)::value;
+            float4 v[NV];
+#pragma unroll
+            for (int j = 0; j < NV; j++) v[j] = *reinterpret_cast<const float4 *>(xr + (tid * 4 + 1024 * j < n ? tid * 4 + 1024 * j : 0));
+#pragma unroll
+            for (int j = 0; j < NV; j++) if (tid * 4 + 1024 * j < n) add(v[j]);
+        };
+        if (n <= 4096) held(std::integral_constant<int, 4>());
+        else if (n <= 8192) held(std::integral_constant<int, 8>());
+        else for (int i = tid * 4; i < n; i += 256 * 4) add(*reinterpret_cast<const float4 *>(xr + i));
         s = wave_sum(s);
         if (lane == 0) red[wave] = s;
         __syncthreads();
@@ -38,12 +50,11 @@ __global__ __launch_bounds__(256) void norm_quant_kernel(const float *__restrict
         const float mean = (float)(tot / (double)n);
         scale = 1.0f / sqrtf(mean + eps);
     }
-    const int nblk = n >> 8;
-    for (int b = blockIdx.y * 4 + wave; b < nblk; b += 4 * gridDim.y) {
+    for (int b = b0; b < nblk; b += 4 * gridDim.y) {
         const int e0 = b * 256 + lane * 4;
-        float4 v = *reinterpret_cast<const float4 *>(xr + e0);
+        float4 v = b == b0 ? v1 : *reinterpret_cast<const float4 *>(xr + e0);
         if (do_norm) {
-            const float4 ww = *reinterpret_cast<const float4 *>(w + e0);
+            const float4 ww = b == b0 ? w1 : *reinterpret_cast<const float4 *>(w + e0);
             v.x = (v.x * scale) * ww.x; v.y = (v.y * scale) * ww.y; v.z = (v.z * scale) * ww.z; v.w = (v.w * scale) * ww.w;
         }
         if (yf) *reinterpret_cast<float4 *>(yf + (size_t)row * n + e0) = v;
@@ -181,7 +192,7 @@ static bool launch_wide(const float *x, const float *w, int n, int T, float eps,
 #define MI355_QUANT_SPLIT_BLOCKS 8
 #endif
 static int quant_splits(int T, int n) {
-    if (T < 8) return ((n >> 8) + 3) / 4;
+    if (T < 32) return ((n >> 8) + 3) / 4;               // a block a wave: few rows are bound by the row's chain (16 rows of 4096, us: two blocks and more a wave 4.8, one 3.9)
     const int nblk = n >> 8;
     int s = (nblk + MI355_QUANT_SPLIT_BLOCKS - 1) / MI355_QUANT_SPLIT_BLOCKS;      // blocks per workgroup <= 8 (two per wave)
     if (T < 64 && s < 2) s = 2;
@@ -346,7 +357,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const float *x, const f
         if (yh) yh[(size_t)blockIdx.x * n + i] = (_Float16)v;
     }
 }
-// The same with a wave to a row that stays in registers: one trip to memory instead of three, no barriers.  187 rows of 768: 4.3 -> 2.9 us.
+// The same with a wave to a row that stays in registers: one trip to memory instead of three, no barriers.  187 rows of 768: 4.3 -> 3.8 us.
 // yp (optional): the row once more, in pinned host memory (the encoder's last layer; 187 rows: 12.6 us, PCIe's time, and no gathering, copying and storing launches behind it, 17).
 template <int NV>
 __global__ __launch_bounds__(256) void layer_norm_wave_kernel(const float *x, const float *w, const float *b, int n, int T, float eps, float *y, _Float16 *yh, float *yp) {
