@@ -1465,7 +1465,7 @@ int attn_out_fused_chunk(const AttnArgs &a) {
     if (MI355_AO_FORCE_C == 128 || MI355_AO_FORCE_C == 64) return (MI355_AO_FORCE_C == 64 && s64 > 64) ? 128 : MI355_AO_FORCE_C;   // (tools: A/B of the chunk size)
 #endif
     if (s64 * a.G <= num_cu() && s64 <= 64) return 64;
-    if (a.H != a.G) return 128;
+    if (a.H != a.G || a.n_kv_max > 64 * 128) return 128;     // (over 64 items a head the launch is refused: longer scans than measured are left where they were)
     for (int c = 128; c < 256; c += 64) if ((a.n_kv_max + c - 1) / c * a.G <= num_cu()) return c;
     return 256;
 }

@@ -717,8 +717,8 @@ bool Context::init(std::string &err) {
     d_qkv_gran_ = (unsigned long long *)dalloc(qkv_attn_granule_words((int)(hp.n_head * D), (int)(hp.n_head_kv * D)) * 8);
     if (!d_step_serial_ || !d_turn_ || !d_ao_flags_ || !d_ao_gran_ || !d_qkv_gran_) { err = "step serial / flag allocation failed"; return false; }
     d_argmax_ = (int32_t *)dalloc(T * 4);
-    argmax_scratch_ = (float *)dalloc(T * 129 * 4);     // T ticket words at the head, then per row 64 part values and 64 part indices (zero-filled: dalloc)
-    head_scratch_ = (float *)dalloc(mmq_few_head_scratch() * 4);
+    argmax_scratch_ = (float *)dalloc((T * 129 + mmq_few_head_scratch()) * 4);     // T ticket words at the head, then per row 64 part values and 64 part indices (zero-filled: dalloc)
+    head_scratch_ = argmax_scratch_ ? argmax_scratch_ + T * 129 : nullptr;          // ... and what a tick's head needs
     rope_cs_ = (float *)dalloc(T * (size_t)hp.n_rot * 4);
     chunk_stride_ = (int)((NC + 63) / 64);
     d_chunks_ = (int32_t *)dalloc((size_t)64 * (chunk_stride_ + 1) * 4);
