@@ -1,7 +1,12 @@
 // attn_cols.hip — attention of a short batch of one conversation (its next turn, a short prompt) and of a text through the encoder, on the matrix cores.
 //
-// The arithmetic is the prompt kernel's (attn_prefill.hip: int8 scores against q8_0 keys or f16 ones, online softmax in log2 units, P as f16 hi + lo, V exact), the
-// split of the work another.  What bounds such a call is latency: a kv head's few hundred keys are tens of kilobytes, and a workgroup that stages chunk after chunk in LDS
+// Scores are the prompt kernel's (attn_prefill.hip: int8 products against q8_0 keys, f16 ones else), the softmax is online in log2 units.  The sums over V are the prompt kernel's for batches
+// that it would take, over 64 tokens: weights and q8_0 values as pairs of f16.  Shorter ones come from kernels that hold weights and values in f32, and are no less exact here (EXACT):
+// a weight is three f16 parts of 2^15 times itself - with all of f16 below it - and a q8_0 value two, exact from the block's scale and code at any size (pairs of 2^-9 of the values
+// where a scale is 512 and more); every product of parts that f32 would see is made.  Error against 64 bits, here with four shares / one-token kernel, geometric mean of 24 conversations at
+// 5, 20 and 7 tokens over 100, 700 and 2500 cells, queries of 1 to 10 times unit size: f16 0.81 to 0.94, q8_0 0.88 to 1.01 and with heads of 64 0.96 to 1.04 (as pairs, with one chain of
+// eight products for an f16 score: 1.0 to 1.4, and weights under 1e-7 of the largest lost).  It costs 0.3 to 1.2 us a launch.
+// The split of the work is another.  What bounds such a call is latency: a kv head's few hundred keys are tens of kilobytes, and a workgroup that stages chunk after chunk in LDS
 // for a tile of 32 tokens leaves most of the chip idle behind a chain of barriers.  Here
 //   * the columns of a tile are (token, query head of the kv group) pairs, so eight tokens of a 4-heads-per-group model fill one;
 //   * a wave takes whole 32-key chunks by itself: K rows ARE the matrix core's A operand and are loaded as such; V rows are loaded four (two) dimensions per lane and
@@ -29,6 +34,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int CK = 32;                                       // keys per chunk, columns per tile
+constexpr unsigned V_BIG = 0x6000;                           // f16 512: a block of codes with a smaller scale is within f16
 
 __device__ __forceinline__ float xhalf_max(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -53,12 +59,15 @@ struct ColsArgs {
     AttnArgs a;
     ActQuant q;                                              // the merged rows quantised as well (quant: 1 Q8_K, 2 Q8_0); nsp = 1 only
     int quant, nsp, n_chunks;                                // n_chunks: of 32 cells
+    float scale_l2;                                          // EXACT: the scores' scale in log2 units, rounded once
     const int32_t *list;                                     // 64-cell chunks to walk (two of 32 each); nullptr: all of [0, n_chunks)
 };
 
-template <bool F16, int DH, int NW>
+// EXACT: the products of weights and values as f32 has them (three f16 parts of a weight, a q8_0 value of any size); else as attn_prefill.hip has them
+template <bool F16, int DH, int NW, bool EXACT>
 __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsArgs c) {
     constexpr int D = DH, NB = DH / 32, NKS = DH / 16, DPL = DH / 32;
+    constexpr float P_ONE = EXACT ? 32768.0f : 1.0f;         // what a weight of one is as an operand: with all of f16 below it
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const AttnArgs &a = c.a;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -182,8 +191,8 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
     }
     const bool one = (seqs & (seqs - 1)) == 0ull;            // (then a cell of another sequence is hidden like an empty one)
     float m_run = -INFINITY, l_run = 0.0f;
-    const float scale_l2 = a.scale * 1.4426950408889634f;
-    f32x16 O[NB];
+    const float scale_l2 = EXACT ? c.scale_l2 : a.scale * 1.4426950408889634f;
+    f32x16 O[NB];                                            // P_ONE times the sums
 #pragma unroll
     for (int db = 0; db < NB; db++)
 #pragma unroll
@@ -195,6 +204,13 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
         const bool live = cell < n_kv && cp >= 0 && cp <= maxpos && (cs & seqs) != 0ull;
         const bool open = __all(cell < n_kv && cp >= 0 && cp <= minpos && (cs & seqs) == seqs);
         const bool more = ci + step < c.n_chunks, see = __any(live);     // (wave-uniform)
+        bool big = false;                                    // a value of the chunk may be beyond f16
+        if constexpr (EXACT && !F16) {
+            unsigned top = 0;
+#pragma unroll
+            for (int b = 0; b < NB; b++) top = max(top, (sq[b >> 1] >> (16 * (b & 1))) & 0x7fffu);
+            big = __any(kg == 1 && top >= V_BIG);
+        }
         if (kg == 0) { s_pos[n] = live ? cp : -1; if (!one) s_seq[n] = cs; }
         if constexpr (!F16) {
 #pragma unroll
@@ -204,13 +220,16 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
         float sc[16];
         if (see) {
         if constexpr (F16) {
-            f32x16 sa;
+            constexpr int CH = EXACT ? 2 : 1;                 // (sums of half of the dimensions each: a chain of eight loses more than the one-token kernel's)
+            f32x16 sa[CH];
 #pragma unroll
-            for (int r = 0; r < 16; r++) sa[r] = 0.0f;
+            for (int k = 0; k < CH; k++)
 #pragma unroll
-            for (int j = 0; j < NKS; j++) sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, kq[j]), qh[j], sa, 0, 0, 0);
+                for (int r = 0; r < 16; r++) sa[k][r] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) sc[r] = sa[r];
+            for (int j = 0; j < NKS; j++) sa[j * CH / NKS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, kq[j]), qh[j], sa[j * CH / NKS], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] = CH > 1 ? sa[0][r] + sa[CH - 1][r] : sa[0][r];
         } else {
 #pragma unroll
             for (int r = 0; r < 16; r++) sc[r] = 0.0f;
@@ -237,7 +256,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
         float mloc = -INFINITY;
         if (open) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) { sc[r] *= scale_l2; mloc = fmaxf(mloc, sc[r]); }
+            for (int r = 0; r < 16; r++) { if constexpr (!EXACT) sc[r] *= scale_l2; mloc = fmaxf(mloc, sc[r]); }
         } else {
 #pragma unroll
             for (int rq = 0; rq < 4; rq++) {
@@ -247,20 +266,27 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
                     const int r = 4 * rq + ri;
                     bool vis = (unsigned)kp[ri] <= (unsigned)tpos;       // (-1: hidden from all)
                     if (!one) vis = vis & ((s_seq[8 * rq + 4 * kg + ri] >> tseq & 1ull) != 0ull);
-                    sc[r] = vis ? sc[r] * scale_l2 : -INFINITY;
+                    sc[r] = vis ? EXACT ? sc[r] : sc[r] * scale_l2 : -INFINITY;
                     mloc = fmaxf(mloc, sc[r]);
                 }
             }
         }
         mloc = xhalf_max(mloc);
+        if constexpr (EXACT) mloc *= scale_l2;
         const float m_new = fmaxf(m_run, mloc);
         const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
         float p[16], lsum = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; r++) { p[r] = __builtin_amdgcn_exp2f(sc[r] - m_ref); lsum += p[r]; }
+        for (int r = 0; r < 16; r++) { p[r] = __builtin_amdgcn_exp2f(EXACT ? __builtin_fmaf(sc[r], scale_l2, -m_ref) : sc[r] - m_ref); if constexpr (!EXACT) lsum += p[r]; }
+        if constexpr (EXACT) {                               // (in pairs: what the sum loses is every dimension's loss)
+            float t[8];
+#pragma unroll
+            for (int r = 0; r < 8; r++) t[r] = p[2 * r] + p[2 * r + 1];
+            lsum = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        }
         lsum = xhalf_sum(lsum);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
-        l_run = l_run * alpha + lsum;
+        l_run = EXACT ? __builtin_fmaf(l_run, alpha, lsum) : l_run * alpha + lsum;
         m_run = m_new;
         if (!__all(alpha == 1.0f)) {
 #pragma unroll
@@ -268,54 +294,91 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
 #pragma unroll
                 for (int r = 0; r < 16; r++) O[db][r] *= alpha;
         }
+        // (a chunk whose values may be beyond f16 is added in two turns, the larger values as 2^-9 of theirs)
+#pragma unroll 1
+        for (int turn = 0; turn <= (int)big; turn++) {
+            if (turn) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            f16x8 ph, pl;
+                for (int db = 0; db < NB; db++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const float v = p[8 * j + i];
-                ph[i] = (_Float16)v;
-                pl[i] = (_Float16)(v - (float)ph[i]);
+                    for (int r = 0; r < 16; r++) O[db][r] *= 0x1p-9f;
             }
-            // output tile db, row m: dimension DPL m + db
-            if constexpr (F16) {
 #pragma unroll
-                for (int db = 0; db < NB; db++) {
-                    u32x4 w;
+            for (int j = 0; j < 2; j++) {
+                f16x8 ph, pm, pl;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        uint32_t lo, hi;
-                        if constexpr (DPL == 4) { lo = vq[j][2 * i][db >> 1]; hi = vq[j][2 * i + 1][db >> 1]; }
-                        else { lo = vq[j][2 * i]; hi = vq[j][2 * i + 1]; }
-                        w[i] = __builtin_amdgcn_perm(hi, lo, (db & 1) ? 0x07060302u : 0x05040100u);
+                for (int i = 0; i < 8; i++) {
+                    if constexpr (EXACT && !F16) asm volatile("" : "+v"(p[8 * j + i]), "+v"(vq[j][i]));        // (nothing made of them is kept from turn to turn)
+                    const float v = EXACT ? p[8 * j + i] * P_ONE : p[8 * j + i];
+                    ph[i] = (_Float16)v;
+                    const float w = v - (float)ph[i];
+                    pm[i] = (_Float16)w;
+                    if constexpr (EXACT) pl[i] = (_Float16)(w - (float)pm[i]);
+                }
+                // output tile db, row m: dimension DPL m + db
+                if constexpr (F16) {
+#pragma unroll
+                    for (int db = 0; db < NB; db++) {
+                        u32x4 w;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            uint32_t lo, hi;
+                            if constexpr (DPL == 4) { lo = vq[j][2 * i][db >> 1]; hi = vq[j][2 * i + 1][db >> 1]; }
+                            else { lo = vq[j][2 * i]; hi = vq[j][2 * i + 1]; }
+                            w[i] = __builtin_amdgcn_perm(hi, lo, (db & 1) ? 0x07060302u : 0x05040100u);
+                        }
+                        const f16x8 av = __builtin_bit_cast(f16x8, w);
+                        if constexpr (EXACT) {
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pl, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pm, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, ph, O[db], 0, 0, 0);
+                        } else {
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, ph, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pm, O[db], 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    const f16x8 av = __builtin_bit_cast(f16x8, w);
-                    O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, ph, O[db], 0, 0, 0);
-                    O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, pl, O[db], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
-                float dv[8];
+                } else {
+                    float dv[8];
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const f32x4 x = *reinterpret_cast<const f32x4 *>(s_sc + (NB + ((DPL * n) >> 5)) * CK + 16 * j + 8 * q + 4 * kg);
+                    for (int q = 0; q < 2; q++) {
+                        const f32x4 x = *reinterpret_cast<const f32x4 *>(s_sc + (NB + ((DPL * n) >> 5)) * CK + 16 * j + 8 * q + 4 * kg);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) dv[4 * q + e] = x[e];
-                }
-#pragma unroll
-                for (int db = 0; db < NB; db++) {
-                    f16x8 vh, vl;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        const float v = (float)(int8_t)((vq[j][i] >> (8 * db)) & 0xff) * dv[i];
-                        vh[i] = (_Float16)v;
-                        vl[i] = (_Float16)(v - (float)vh[i]);
+                        for (int e = 0; e < 4; e++) dv[4 * q + e] = x[e];
                     }
-                    O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph, O[db], 0, 0, 0);
-                    O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl, O[db], 0, 0, 0);
-                    O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph, O[db], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (big) {
+#pragma unroll
+                        for (int i = 0; i < 8; i++) { const bool small = fabsf(dv[i]) < 512.0f; dv[i] = turn ? small ? 0.0f : dv[i] * 0x1p-9f : small ? dv[i] : 0.0f; }
+                    }
+#pragma unroll
+                    for (int db = 0; db < NB; db++) {
+                        f16x8 vh, vl;
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            const float v = (float)(int8_t)((vq[j][i] >> (8 * db)) & 0xff) * dv[i];
+                            vh[i] = (_Float16)v;
+                            vl[i] = (_Float16)(v - (float)vh[i]);
+                        }
+                        if constexpr (EXACT) {               // (the small ones first: the other way round q8_0 is up to 0.1 further off)
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, pm, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pm, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph, O[db], 0, 0, 0);
+                        } else {
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pm, O[db], 0, 0, 0);
+                            O[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph, O[db], 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
+            }
+            if (turn) {
+#pragma unroll
+                for (int db = 0; db < NB; db++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) O[db][r] *= 0x1p9f;
             }
         }
         }
@@ -335,7 +398,10 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
     const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
 #pragma unroll
     for (int w = 0; w < NW; w++) l_all += s_ml[w * 64 + 32 + n] * __builtin_amdgcn_exp2f(s_ml[w * 64 + n] - m_ref);
-    const float f = __builtin_amdgcn_exp2f(m_run - m_ref);
+    // (the merge of the shares works in natural-log units: what the record's maximum loses by its rounding goes into the sums)
+    const float m_nat = m_all * 0.6931471805599453f;
+    const float adj = EXACT && c.nsp > 1 && m_all != -INFINITY ? __builtin_amdgcn_exp2f(__builtin_fmaf(-m_nat, 1.925963033500e-08f, __builtin_fmaf(-m_nat, 1.44269502162933349609375f, m_all))) : 1.0f;
+    const float f = __builtin_amdgcn_exp2f(m_run - m_ref) * (adj * (1.0f / P_ONE));
     float *const s_l = s_ml + NW * 64;                       // (a column's sum, for the end)
     if (wave == 0 && kg == 0) s_l[n] = l_all;
 #pragma unroll
@@ -344,7 +410,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
         for (int r = 0; r < 16; r++) mine[(db * 16 + r) * 65 + lane] = O[db][r] * f;
     if (wave == 0 && kg == 0 && c.nsp > 1 && q_ok) {
         float *rec = a.part + (((size_t)tok * a.H + h) * c.nsp + blockIdx.z) * (D + 2);
-        rec[D] = m_all * 0.6931471805599453f; rec[D + 1] = l_all;        // (the merge works in natural-log units)
+        rec[D] = m_nat; rec[D + 1] = l_all * adj;
     }
     __syncthreads();
     // a wave per 256 values: 256 / D columns, four consecutive dimensions per lane
@@ -440,12 +506,12 @@ bool flash_attn_cols_takes(const AttnArgs &a, bool one_token_kernel) {
     return !one_token_kernel || a.T >= 32 || a.T * ((cols_chunks(a) + 1) / 2) >= 64;
 }
 
-template <bool F16, int DH, int NW>
+template <bool F16, int DH, int NW, bool EXACT>
 static void cols_go(const ColsArgs &c, hipStream_t st) {
     const AttnArgs &a = c.a;
     constexpr int lds = cols_lds_words<F16, DH, NW> * 4;
-    if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_cols_kernel<F16, DH, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL((flash_attn_cols_kernel<F16, DH, NW>), dim3((unsigned)a.G, (unsigned)(cols_tiles(a) / a.G), (unsigned)c.nsp), dim3(64 * NW), lds, st, c);
+    if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_cols_kernel<F16, DH, NW, EXACT>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL((flash_attn_cols_kernel<F16, DH, NW, EXACT>), dim3((unsigned)a.G, (unsigned)(cols_tiles(a) / a.G), (unsigned)c.nsp), dim3(64 * NW), lds, st, c);
 }
 
 hipError_t launch_flash_attn_cols(const AttnArgs &a, hipStream_t st) {
@@ -453,16 +519,20 @@ hipError_t launch_flash_attn_cols(const AttnArgs &a, hipStream_t st) {
     ColsArgs c{};
     c.a = a;
     c.nsp = a.pf_splits > 1 && a.part ? a.pf_splits : 1;
+    c.scale_l2 = (float)((double)a.scale * 1.4426950408889634);
     c.n_chunks = cols_chunks(a);
     c.list = a.chunks;
     const bool here = c.nsp == 1 && a.out_q && cols_quantises(a);
     if (here) { c.q = act_for(a.out_q, a.T); c.quant = (a.out_q8k ? 1 : 0) | (a.out_q80 ? 2 : 0); }
     const bool wide = c.n_chunks > 4 * c.nsp;
-#define GO(F, DD) do { if (wide) cols_go<F, DD, 8>(c, st); else cols_go<F, DD, 4>(c, st); } while (0)
+    const bool exact = a.T <= 64 || !flash_attn_prefill_applicable(a);
+#define GO1(F, DD, X) do { if (wide) cols_go<F, DD, 8, X>(c, st); else cols_go<F, DD, 4, X>(c, st); } while (0)
+#define GO(F, DD) do { if (exact) GO1(F, DD, true); else GO1(F, DD, false); } while (0)
     if (a.type_k == T_F16) { if (a.D == 128) GO(true, 128); else GO(true, 64); }
     else if (a.D == 128) GO(false, 128);
     else GO(false, 64);
 #undef GO
+#undef GO1
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (c.nsp > 1) return launch_flash_attn_combine(a, c.nsp, st);

@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
     (32, 8, 128, 129, 5, 1), (4, 4, 64, 300, 33, 1), (32, 4, 64, 257, 3, 1),    # four chunks a workgroup and more than that; eight heads a group
     (6, 2, 128, 70, 21, 1), (14, 2, 128, 200, 11, 3), (24, 8, 64, 90, 7, 1),    # groups whose heads do not divide a tile
     (8, 2, 128, 300, 40, 2), (32, 8, 128, 700, 37, 6), (12, 12, 64, 1000, 64, 5), (4, 2, 64, 100, 50, 4),    # shares, some with fewer chunks than waves
+    (8, 2, 128, 300, 70, 2), (4, 4, 128, 90, 65, 1), (12, 12, 64, 200, 66, 1), (8, 1, 64, 700, 130, 3), (12, 4, 64, 150, 67, 1),    # over 64 tokens: pairs of f16; three heads of 64 a group do not go to the prompt kernel
 ])
 def test_against_the_oracle(be, tkv, H, G, D, n_cells, T, shares):  # noqa: F811
     """Holes in the cache, a query that sees one cell, ragged tiles and chunks.  q8_0: the scores' integers are exact; f16: the CPU's sums of V are made in f32 for the comparison.
@@ -43,6 +44,46 @@ def test_against_the_oracle(be, tkv, H, G, D, n_cells, T, shares):  # noqa: F811
             cells = np.nonzero((cell_pos >= 0) & (cell_pos <= q_pos[i]))[0].astype(np.int32)
             ref = oq.flash_attn(q[i], H, G, D, tkv, kc, tkv, vc, cells, scale)
             assert np.abs(out[i] - ref).max() <= 2e-5 * max(1.0, float(np.abs(ref).max())), (i, np.abs(out[i] - ref).max())
+    finally:
+        oq.set_fa_v_acc_f32(0)
+
+
+@pytest.mark.parametrize("tkv", [Q8_0, F16])
+@pytest.mark.parametrize("H,G,D,shares", [(8, 2, 128, 1), (8, 2, 128, 3), (8, 1, 64, 1), (8, 8, 64, 2)])
+@pytest.mark.parametrize("what", ["small weights", "large values"])
+def test_weights_and_values_as_in_f32(be, tkv, H, G, D, shares, what):  # noqa: F811
+    """Small weights: every query's largest score, 16 over the others, is a cell's whose values are zero, so the output is the others', of weights near 1e-7.  Large values: up to 3e6 in a
+    q8_0 cache (the blocks of a row of very different size, a hidden cell among them), 6e4 in an f16 one.  The bound is of the output's own largest: a score of 16 is 2e-6 off in f32, the
+    oracle's sum over 300 cells in f32 about as much, together below 2e-5."""
+    n, T = 300, 9
+    rng = np.random.default_rng(D + H + shares)
+    kf = (0.2 * rng.standard_normal((n, G, D))).astype(np.float32)
+    vf = rng.standard_normal((n, G, D)).astype(np.float32)
+    q = rng.choice([-1.0, 1.0], D) + 0.05 * rng.standard_normal((T, H, D))
+    scale = 1 / np.sqrt(D)
+    if what == "small weights":
+        kf[40] = np.sign(q[0, 0]) * 16 * scale
+        vf[40] = 0.0
+    else:
+        vf *= 10.0 ** rng.uniform(-3, 4.5 if tkv == F16 else 6, (n, G, 1))
+        vf[::7, :, D // 2:] *= 1e-3
+        vf = np.clip(vf, -6e4, 6e4) if tkv == F16 else np.clip(vf, -3e6, 3e6)
+        vf[77] = 6e4 if tkv == F16 else 3e6
+    vf = vf.astype(np.float32)
+    kc, vc = np.stack([oq.quantize(tkv, r.reshape(-1)) for r in kf]), np.stack([oq.quantize(tkv, r.reshape(-1)) for r in vf])
+    cell_pos = np.arange(n, dtype=np.int32)
+    cell_pos[77] = -1
+    q, q_pos = q.astype(np.float32), np.linspace(100, n - 1, T).astype(np.int32)
+    be.set_option("attn_cols", shares)
+    try:
+        out = be.flash_attn(q, H, G, D, tkv, kc, tkv, vc, cell_pos, q_pos, scale)
+    finally:
+        be.set_option("attn_cols", 0)
+    oq.set_fa_v_acc_f32(1 if tkv == F16 else 0)
+    try:
+        for i in range(T):
+            ref = oq.flash_attn(q[i], H, G, D, tkv, kc, tkv, vc, np.nonzero((cell_pos >= 0) & (cell_pos <= q_pos[i]))[0].astype(np.int32), scale)
+            assert np.abs(out[i] - ref).max() <= 2e-5 * float(np.abs(ref).max()), (i, np.abs(out[i] - ref).max() / np.abs(ref).max())
     finally:
         oq.set_fa_v_acc_f32(0)
 
