@@ -493,17 +493,33 @@ bool flash_attn_cols_applicable(const AttnArgs &a) {
     return (f16 || q8) && (int64_t)a.T * (a.H / a.G) <= (65535LL * CK) && (a.H * a.D) % 256 == 0;
 }
 
-// Two rounds of workgroups, four with heads of 64 (us, here / attn_prefill.hip):
-//   32 / 8 heads of 128, q8_0   64 tokens behind 677 cells 16 / 38, 256 / 0 11.1 / 30, 512 / 0 27 / 41, 512 / 2488 109 / 112, 777 / 0 62 / 59, 1024 / 0 73 / 76, 2048 / 0 225 / 150
-//   32 / 32 heads of 128, f16   256 / 0 13.7 / 28, 512 / 0 28 / 38, 777 / 0 66 / 59, 1024 / 0 71 / 61
-//   32 / 4 heads of 64, f16     256 / 0 7.0 / 23, 1024 / 0 41 / 49, 2048 / 0 124 / 101            12 / 12 heads of 64, f16 (a text)   187 6.2 / 16, 2000 53 / 90
-// Behind it, fewer than 32 tokens of few chunks stay with the one-token kernel, a (token, 64-cell chunk) at a time with a merge, whose sums are a step's: here / there
-// 5 tokens behind 59 cells 8.8 / 9.8, behind 195 10.2 / 10.0, behind 1495 11.9 / 13.9; 12 behind 188 10.7 / 10.6, behind 665 11.7 / 14.5; 37 behind 163 10.8 / 14.7, behind 640
-// 15.0 / 27.0, behind 3863 26 / 97.  (The encoder has no such kernel.)
+// Long batches, here / attn_prefill.hip with its merge (us a layer):
+//   32 / 8 heads of 128, q8_0   64 tokens behind 613 cells 18 / 39, 256 / 0 15 / 29, 256 / 3500 88 / 98, 450 / 3400 163 / 195, 512 / 0 34 / 44, 512 / 1500 101 / 102, 512 / 2488 145 / 137,
+//                               512 / 3400 169 / 161
+//   32 / 32 heads of 128, f16   256 / 2000 53 / 63, 300 / 2000 85 / 103, 512 / 0 28 / 41, 512 / 1000 67 / 69, 512 / 1500 86 / 83, 400 / 2500 113 / 101, 450 / 1500 82 / 77, 512 / 2500 122 / 109
+//   32 / 4 heads of 64, f16     256 / 0 8 / 24, 768 / 1200 66 / 80, 850 / 0 44 / 45, 1024 / 0 51 / 50, 1024 / 900 86 / 75      12 / 12 heads of 64, f16 (a text)   187 6.6 / 17, 2000 58 / 92
+// So with heads of 64 three rounds of workgroups; with heads of 128 two as long as the keys are few, to 1536 cells with a query head to every kv head and to 2048 else, and with more keys
+// 11 / 8 and 15 / 8 rounds.
+static bool cols_long(const AttnArgs &a) {
+    const int eighths = 8 * cols_tiles(a), cu = num_cu(), ch = cols_chunks(a);
+    if (a.D == 64) return eighths <= 24 * cu;
+    return eighths <= (a.H == a.G ? ch <= 48 ? 16 : 11 : ch <= 64 ? 16 : 15) * cu;
+}
+// Short ones beside the one-token kernel, a (token, 64-cell chunk) at a time with a merge, whose sums are a step's: here / there, T tokens behind so many cells, each with its merge
+//   32 / 8 heads of 128, q8_0   2 / 2100 13.2 / 13.6, 3 / 1900 14.1 / 14.7, 5 / 900 14.1 / 12.9, 5 / 1495 14.8 / 15.7, 8 / 700 14.2 / 13.3, 12 / 400 14.3 / 12.6, 14 / 700 14.7 / 17.3,
+//                               22 / 200 13.3 / 12.6, 31 / 150 13.7 / 12.9, 31 / 200 13.1 / 14.6, 32 / 0 11.4 / 10.8, 40 / 0 11.3 / 11.2, 64 / 0 11.0 / 11.4
+//   32 / 32 heads of 128, f16   2 / 2100 20.4 / 17.0, 2 / 3000 21.2 / 24.0, 2 / 3900 22 / 29, 3 / 1900 17.0 / 19.2, 5 / 900 13.5 / 16.8, 12 / 400 12.3 / 16.5, 32 / 0 8.3 / 10.7
+//   32 / 4 heads of 64, f16     3 / 1900 11.7 / 15.6, 8 / 700 10.1 / 14.6, 22 / 200 7.4 / 14.4
+// (The encoder has no such kernel: 3 tokens 5.7 / 7.9 with the general one.)
+static bool cols_short(const AttnArgs &a) {
+    const int ch = (cols_chunks(a) + 1) / 2, work = a.T * ch;
+    const bool wide = a.D == 128, q8 = a.type_k == T_Q8_0;
+    if (a.T >= (wide && q8 ? 40 : 32)) return true;
+    return work >= (!wide ? 64 : q8 ? ch < 28 ? 104 : 64 : a.T < 3 ? 80 : 64);
+}
 bool flash_attn_cols_takes(const AttnArgs &a, bool one_token_kernel) {
     static const bool off = getenv("MI355_ATTN_COLS") && getenv("MI355_ATTN_COLS")[0] == '0';
-    if (off || !flash_attn_cols_applicable(a) || cols_tiles(a) > (a.D == 64 ? 4 : 2) * num_cu()) return false;
-    return !one_token_kernel || a.T >= 32 || a.T * ((cols_chunks(a) + 1) / 2) >= 64;
+    return !off && flash_attn_cols_applicable(a) && cols_long(a) && (!one_token_kernel || cols_short(a));
 }
 
 template <bool F16, int DH, int NW, bool EXACT>

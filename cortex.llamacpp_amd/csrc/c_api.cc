@@ -274,6 +274,11 @@ int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int
     }
     return mmq_applicable(type, n_cols, n_tokens) ? 3 : 0;
 }
+int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder) {
+    AttnArgs a{};
+    a.T = n_tokens; a.H = n_head; a.G = n_head_kv; a.D = head_dim; a.n_ctx = a.n_kv_max = n_cells; a.type_k = a.type_v = type_kv;
+    return flash_attn_cols_takes(a, !encoder) ? flash_attn_cols_splits(a) : 0;
+}
 int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int32_t type_v, int32_t type_o, int32_t n_embd, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
                                   int32_t type_kv, int32_t n_kv, int32_t *slots_out) {
     int slots = 0;

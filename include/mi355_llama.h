@@ -179,6 +179,9 @@ MI355_API int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int3
 /* host logic only: which contraction a batch of n_tokens rows against a K-quant tensor of n_rows x n_cols takes in a context of n_ubatch >= 128 (pair: n_rows rows each of ffn_gate and
    ffn_up; sum_free: the launch that follows adds a K split's partial sums).  0 mat-vec, 1 csrc/mmq_few.hip, 2 K-split, 3 planes */
 MI355_API int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int32_t n_tokens, int32_t pair, int32_t sum_free);
+/* host logic only: does the attention of n_tokens of one conversation (encoder: of a text) over n_cells cells of type_kv go through csrc/attn_cols.hip?  Returns the number of workgroups
+   that share a tile's keys there, 0 = the one-token or the prompt kernel */
+MI355_API int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder);
 /* llama_set_embeddings (ctx.cc:299) */
 MI355_API void    mi355_set_embeddings(mi355_context *ctx, int32_t enabled);
 /* llama_get_embeddings_ith (ctx.cc:1042-1044): final-norm hidden state (n_embd floats, host memory) of batch row i of the

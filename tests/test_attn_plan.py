@@ -1,0 +1,33 @@
+"""Which attention a batch of one conversation takes (host logic: no GPU): the sides on which measured launches were the faster ones."""
+import pytest
+
+F16, Q8_0 = 1, 8
+L8, L7, SMALL, TEXT = (Q8_0, 32, 8, 128), (F16, 32, 32, 128), (F16, 32, 4, 64), (F16, 12, 12, 64)
+
+
+@pytest.fixture(scope="module")
+def takes(pkg):
+    lib = pkg.load_library()
+    return lambda model, n, past, encoder=0: int(lib.mi355_debug_attn_plan(*model, n, past + n, encoder)) > 0
+
+
+@pytest.mark.parametrize("model,yes,no", [
+    (L8, [(2, 2100), (3, 1900), (5, 1495), (14, 700), (31, 200), (40, 0), (37, 160), (64, 613)], [(2, 700), (5, 900), (8, 700), (12, 400), (22, 200), (31, 150), (32, 0), (1, 3900)]),
+    (L7, [(2, 3000), (3, 1900), (5, 900), (12, 400), (32, 0)], [(2, 2100), (14, 200)]),
+    (SMALL, [(3, 1900), (8, 700), (22, 200)], [(14, 200), (2, 700)]),
+])
+def test_short_batches(takes, model, yes, no):
+    assert [c for c in yes if not takes(model, *c)] == [] and [c for c in no if takes(model, *c)] == []
+
+
+@pytest.mark.parametrize("model,yes,no", [
+    (L8, [(256, 3500), (450, 3400), (512, 0), (512, 700), (512, 1400)], [(512, 2488), (512, 3400), (513, 0)]),
+    (L7, [(256, 3500), (300, 2000), (512, 0), (512, 1000)], [(400, 2500), (450, 1500), (512, 1500), (512, 2500)]),
+    (SMALL, [(256, 0), (700, 900), (768, 1200)], [(850, 0), (1024, 900)]),
+])
+def test_long_batches(takes, model, yes, no):
+    assert [c for c in yes if not takes(model, *c)] == [] and [c for c in no if takes(model, *c)] == []
+
+
+def test_texts(takes):
+    assert all(takes(TEXT, n, 0, 1) for n in (3, 20, 187, 700, 2000, 2048))
