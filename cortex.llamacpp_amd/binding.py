@@ -108,6 +108,7 @@ SYMBOLS = {
     "mi355_op_swiglu": (C.c_int, [_vp, _vp, _i64, _vp]),
     "mi355_op_soft_max": (C.c_int, [_vp, _vp, _i64, _i64, _f32, _vp]),
     "mi355_op_moe_route": (C.c_int, [_vp, _i64, _i32, _i32, _vp, _vp]),
+    "mi355_op_moe_router": (C.c_int, [_i32, _vp, _i32, _i64, _vp, _i64, _i32, _vp, _f32, _vp, _vp, _vp]),
     "mi355_op_flash_attn": (C.c_int, [_vp, _i64, _i32, _i32, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _vp, _f32, _vp]),
     "mi355_op_attn_step": (C.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i32, _f32, _i32, _f32, _i32, _vp, _i64, _vp, _i32,
                                      _vp, _vp, _vp, _vp]),
@@ -308,6 +309,15 @@ class Backend:
         ids = np.zeros((T, k), np.int32); w = np.zeros((T, k), np.float32)
         self._chk(self.lib.mi355_op_moe_route(_ptr(x), T, ne, k, _ptr(ids), _ptr(w)), "op_moe_route")
         return ids, w
+
+    def moe_router(self, t: int, W: np.ndarray, x: np.ndarray, k: int, norm_w: np.ndarray | None = None, eps: float = 0.0):
+        """logits [T][n_expert], ids and weights [T][k]; W [n_expert][K] as float32 (t = 0) or float16 (t = 1)."""
+        W = np.ascontiguousarray(W, np.float32 if t == 0 else np.float16); x = np.ascontiguousarray(x, np.float32)
+        T, ne = x.shape[0], W.shape[0]
+        nw = None if norm_w is None else np.ascontiguousarray(norm_w, np.float32)
+        lg = np.zeros((T, ne), np.float32); ids = np.zeros((T, k), np.int32); w = np.zeros((T, k), np.float32)
+        self._chk(self.lib.mi355_op_moe_router(t, _ptr(W), ne, W.shape[1], _ptr(x), T, k, None if nw is None else _ptr(nw), eps, _ptr(lg), _ptr(ids), _ptr(w)), "op_moe_router")
+        return lg, ids, w
 
     def flash_attn(self, q: np.ndarray, n_head: int, n_head_kv: int, hd: int, type_k: int, k_rows: np.ndarray, type_v: int,
                    v_rows: np.ndarray, cell_pos, q_pos, scale: float) -> np.ndarray:

@@ -716,6 +716,20 @@ int mi355_op_moe_route(const float *logits, int64_t T, int32_t n_expert, int32_t
     return di.down(ids, (size_t)T * k * 4) && dw.down(w, (size_t)T * k * 4) ? MI355_OK : MI355_ERR_HIP;
 }
 
+int mi355_op_moe_router(int32_t type, const void *W, int32_t n_expert, int64_t K, const float *x, int64_t T, int32_t k, const float *norm_w, float eps, float *logits, int32_t *ids, float *w) {
+    if (!need_device()) return MI355_ERR_NO_DEVICE;
+    if (T <= 0 || K <= 0 || n_expert <= 0 || n_expert > 64 || k <= 0 || k > n_expert || (type != T_F32 && type != T_F16)) { fail("moe_router: bad shape"); return MI355_ERR_ARG; }
+    if (norm_w && (T != 1 || !moe_router_norms(type, n_expert, (int)K))) { fail("moe_router: no form that norms"); return MI355_ERR_ARG; }
+    const size_t wb = (size_t)n_expert * K * (type == T_F32 ? 4 : 2);
+    DevBuf dW(wb), dx((size_t)T * K * 4), dn((size_t)K * 4), dl((size_t)T * n_expert * 4), di((size_t)T * k * 4), dw((size_t)T * k * 4);
+    if (!dW.up(W, wb) || !dx.up(x, (size_t)T * K * 4) || (norm_w && !dn.up(norm_w, (size_t)K * 4)) || !dl.p || !di.p || !dw.p) return MI355_ERR_OOM;
+    hipError_t e = launch_moe_router(type, dW.as<uint8_t>(), n_expert, (int)K, dx.as<float>(), (int)T, k, dl.as<float>(), di.as<int32_t>(), dw.as<float>(), nullptr, nullptr,
+                                     norm_w ? dn.as<float>() : nullptr, eps);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) return hip_fail(e, "moe_router");
+    return dl.down(logits, (size_t)T * n_expert * 4) && di.down(ids, (size_t)T * k * 4) && dw.down(w, (size_t)T * k * 4) ? MI355_OK : MI355_ERR_HIP;
+}
+
 int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t D, int32_t type_k, const void *k, int32_t type_v,
                         const void *v, int32_t n_cells, const int32_t *cell_pos, const int32_t *q_pos, float scale, float *out) {
     if (!need_device()) return MI355_ERR_NO_DEVICE;

@@ -515,22 +515,27 @@ __global__ __launch_bounds__(1024) void moe_router_kernel(int type, const uint8_
     if (lane < k) { ids[(size_t)t * k + lane] = id; w[(size_t)t * k + lane] = mine / wsum; }
 }
 bool moe_router_norms(int type, int n_expert, int K) { return (type == T_F32 || type == T_F16) && n_expert <= 64 && (K & 255) == 0 && K <= 16384; }
+struct RouterCall { int type; const uint8_t *W; int n_expert, K; const float *x, *nw; float eps; int T, k; float *logits; int32_t *ids; float *w; const int32_t *forced; };
+template <int NTOK, bool NORM>
+static hipError_t router_go(const RouterCall &c, hipStream_t st) {
+    const size_t rows = (size_t)NTOK * c.K * 4, arrays = (64 * NTOK + 16) * sizeof(double);         // dynamic LDS, and the kernel's own arrays
+    if (rows + arrays > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_router_kernel<NTOK, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((moe_router_kernel<NTOK, NORM>), dim3((c.T + NTOK - 1) / NTOK), dim3(1024), rows, st, c.type, c.W, c.n_expert, c.K, c.x, c.nw, c.eps, c.T, c.k, c.logits, c.ids, c.w, c.forced);
+    return hipGetLastError();
+}
 hipError_t launch_moe_router(int type, const uint8_t *W, int n_expert, int K, const float *x, int T, int k, float *logits_out, int32_t *ids, float *w,
                              hipStream_t st, const int32_t *forced, const float *nw, float eps) {
     if (n_expert < 1 || n_expert > 64 || k > n_expert || (type != T_F32 && type != T_F16) || T <= 0 || (nw && (T != 1 || !moe_router_norms(type, n_expert, K)))) return hipErrorInvalidValue;
-    if (nw) hipLaunchKernelGGL((moe_router_kernel<1, true>), dim3(1), dim3(1024), (size_t)K * 4, st, type, W, n_expert, K, x, nw, eps, T, k, logits_out, ids, w, forced);
-    else if (T >= 64 && (K & 255) == 0 && K <= 8192) {
-        const size_t lds = (size_t)4 * K * 4;
-        if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_router_kernel<4, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        hipLaunchKernelGGL((moe_router_kernel<4, false>), dim3((T + 3) / 4), dim3(1024), lds, st, type, W, n_expert, K, x, nullptr, 0.0f, T, k, logits_out, ids, w, forced);
-    } else if ((K & 255) == 0 && K <= 16384)
-        hipLaunchKernelGGL((moe_router_kernel<1, false>), dim3(T), dim3(1024), (size_t)K * 4, st, type, W, n_expert, K, x, nullptr, 0.0f, T, k, logits_out, ids, w, forced);
-    else {
-        if (!logits_out) return hipErrorInvalidValue;
-        const hipError_t e = launch_mmv_float(type, W, n_expert, K, x, T, logits_out, n_expert, nullptr, st);
-        return e != hipSuccess ? e : launch_moe_route(logits_out, T, n_expert, k, ids, w, st, forced);
-    }
-    return hipGetLastError();
+    const RouterCall c{type, W, n_expert, K, x, nw, eps, T, k, logits_out, ids, w, forced};
+    if (nw) return router_go<1, true>(c, st);
+    if (T >= 64 && (K & 255) == 0 && K <= 8192) return router_go<4, false>(c, st);
+    if ((K & 255) == 0 && K <= 16384) return router_go<1, false>(c, st);
+    if (!logits_out) return hipErrorInvalidValue;
+    const hipError_t e = launch_mmv_float(type, W, n_expert, K, x, T, logits_out, n_expert, nullptr, st);
+    return e != hipSuccess ? e : launch_moe_route(logits_out, T, n_expert, k, ids, w, st, forced);
 }
 __global__ void moe_combine_kernel(float *x, const float *eo, const float *w, int T, int E, int k, size_t eo_stride) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

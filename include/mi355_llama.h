@@ -234,6 +234,10 @@ MI355_API int mi355_op_soft_max(const float *x, const float *mask, int64_t n, in
 /* build_moe_ffn's expert selection: softmax over n_expert router logits per token, the k largest (first index wins ties), weights
    renormalised; ids [T][k], w [T][k] */
 MI355_API int mi355_op_moe_route(const float *logits, int64_t T, int32_t n_expert, int32_t k, int32_t *ids, float *w);
+/* the router of a mixture-of-experts layer: logits [T][n_expert] of W [n_expert][K] (F32 / F16) and rows x [T][K], and the selection above; norm_w (nullable, T = 1): x is the row in front
+   of the RMS norm with these weights */
+MI355_API int mi355_op_moe_router(int32_t type, const void *W, int32_t n_expert, int64_t K, const float *x, int64_t T, int32_t k, const float *norm_w, float eps, float *logits, int32_t *ids,
+                                  float *w);
 /* flash_attn_ext for T query tokens: K/V given as ggml-layout rows [n_cells][n_head_kv*head_dim] of type_k/type_v;
  * visibility: cell c is visible to token t iff cell_pos[c] >= 0 && cell_pos[c] <= q_pos[t]. */
 MI355_API int mi355_op_flash_attn(const float *q, int64_t T, int32_t n_head, int32_t n_head_kv, int32_t head_dim,

@@ -87,3 +87,35 @@ def test_router_token_by_token_and_in_batches(pkg, tmp_path, experts, used):
     for r in rows[1:]:
         assert (np.linalg.norm(r - rows[0], axis=1) <= 0.02 * np.linalg.norm(rows[0], axis=1)).all()
     c.close(); m.close()
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("experts,used,K,T,norm", [
+    (8, 2, 4096, 1, True), (2, 1, 256, 1, True), (60, 4, 2304, 1, True), (64, 8, 16384, 1, True),          # the norm within; two and one waves to an expert; 64 KB of a row
+    (8, 2, 4096, 3, False), (3, 3, 768, 5, False), (64, 6, 16384, 2, False),                                # a token a workgroup
+    (8, 2, 4096, 66, False), (5, 2, 8192, 65, False), (64, 4, 256, 64, False),                              # four tokens, the last workgroup's ragged; 128 KB of rows
+    (8, 2, 320, 3, False), (8, 2, 16640, 2, False), (4, 1, 8448, 70, False),                                # two launches: columns that are no multiple of 256, rows longer than 64 KB; and 64 rows too long for four
+])
+def test_router_against_float64(be, f16, experts, used, K, T, norm):  # noqa: F811
+    """Products are f32 (f16 weights: of the row's f16 roundings, which numpy makes from the same f32 norm), sums double: half an ulp of every product and of the logit.  Experts are
+    compared where the k-th is apart from the next by more than that; the weights follow from the logits, an exponential and two divisions in f32: 1e-6 and twice a logit's error."""
+    rng = np.random.default_rng(experts * 1000 + K + T)
+    W = (rng.standard_normal((experts, K)) / np.sqrt(K)).astype(np.float16 if f16 else np.float32)
+    x = (rng.standard_normal((T, K)) * 3).astype(np.float32)
+    nw = rng.uniform(0.5, 1.5, K).astype(np.float32) if norm else None
+    lg, ids, w = be.moe_router(1 if f16 else 0, W, x, used, nw, 1e-5)
+    if norm:
+        mean = np.float32((x * x).astype(np.float64).sum() / K)
+        x = (x * (np.float32(1) / np.sqrt(mean + np.float32(1e-5)))) * nw
+    x = x.astype(np.float16) if f16 else x
+    prod = W.astype(np.float64)[None] * x.astype(np.float64)[:, None]
+    ref = prod.sum(-1)
+    err = 2.0 ** -24 * (np.abs(prod).sum(-1) + np.abs(ref)) * (4 if norm else 1)          # (the norm: a root and a reciprocal of one ulp each)
+    assert (np.abs(lg - ref) <= err).all()
+    for t in range(T):
+        order = np.argsort(-ref[t], kind="stable")
+        gap = ref[t][order][:-1] - ref[t][order][1:]
+        if (gap[:used] > 2 * err[t].max()).all() if used < experts else (gap > 2 * err[t].max()).all():
+            assert ids[t].tolist() == order[:used].tolist()
+        p = np.exp(ref[t][ids[t]] - ref[t].max())
+        assert np.allclose(w[t], p / p.sum(), rtol=1e-6 + 2 * err[t].max(), atol=0)
