@@ -51,7 +51,9 @@ template <> struct VWord<2> { typedef uint16_t T; };
 template <> struct VWord<8> { typedef u32x2 T; };
 
 template <int DH> constexpr int cols_merge_words = (DH / 32) * 16 * 65;      // a wave's O, [16 * tile + register][lane], rows of 65: the readers take registers, not lanes, side by side
-template <int DH> constexpr int cols_wave_words = (DH / 32) * CK * 2 + CK + 2 * CK;      // a chunk's scales [k, v][block][key], positions, sequence masks
+template <int DH> constexpr int cols_wave_words = (DH / 32) * CK * 2 + CK + 2 * CK;      // a chunk's scales [k, v][block][key], positions, sequence masks, in the space of the sums
+static_assert(cols_wave_words<64> <= cols_merge_words<64> && cols_wave_words<128> <= cols_merge_words<128>, "a chunk's words fit where the wave's sums go");
+static_assert(cols_merge_words<64> % 4 == 0 && cols_merge_words<128> % 4 == 0 && CK % 4 == 0, "read 16 and 8 bytes at a time");
 template <bool F16, int DH> constexpr int cols_q_stride = (F16 ? 2 * DH : DH) + 16;                            // bytes of a column's query as an operand
 template <bool F16, int DH, int NW> constexpr int cols_lds_words = NW * cols_merge_words<DH> + std::max(NW * 64 + CK, CK * cols_q_stride<F16, DH> / 4 + CK * (DH / 32));
 
@@ -472,10 +474,13 @@ bool cols_quantises(const AttnArgs &a) {
 static int cols_chunks(const AttnArgs &a) { return a.chunks ? 2 * a.n_chunks : (std::min(a.n_kv_max, a.n_ctx) + CK - 1) / CK; }
 static int cols_tiles(const AttnArgs &a) { return a.G * ((a.T * (a.H / a.G) + CK - 1) / CK); }
 // How many workgroups share a tile's keys.  A workgroup fills a CU; of its time (us, as the tables below have it) a part is its start and its end, the rest goes by the rounds
-// of chunks that its waves walk, and sharing costs the records and the launch that merges them.  Four waves where a share is no more than four chunks.  Measured (us, attention and merge):
+// of chunks that its waves walk, and sharing costs the records and the launch that merges them.  Four waves where a share is no more than four chunks.  Measured (us, attention and merge, weights
+// as pairs; EXACT adds 0.3 to 1.2):
 //   32 / 8 heads of 128, q8_0      37 tokens, 677 cells: 1 share 19.8, 2 19.8, 3 15.1, 6 15.0, 12 15.9      64, 677: 20.1, 20.4, 16.0, 18.5, 21.0
 //                                  37, 3900: 1 71.7, 3 34.4, 6 26.3, 8 36.0, 16 38.6                        5, 3900: 1 70.3, 6 21.9, 16 13.8, 32 13.4
 //   32 / 4 heads of 64, f16        37, 677: 1 11.4, 3 12.3, 6 12.8                                          2, 677: 1 10.5, 3 9.4, 6 8.2
+// The tiles are those of the caller's kv heads: a rank of a row split, with a part of them, shares its keys in another number of parts than the whole model does, and its sums differ from the
+// whole's by the order of f32 additions - as its attn_output and ffn_down, summed over the ranks, do anyway.  Greedy answers of a split model can part from the unsplit one's at a near tie.
 static double cols_time(const AttnArgs &a, int nsp) {
     const int per = (cols_chunks(a) + nsp - 1) / nsp, nw = per > 4 ? 8 : 4, walks = (per + nw - 1) / nw, rounds = (cols_tiles(a) * nsp + num_cu() - 1) / num_cu();
     const double start = a.D == 128 ? 6.5 : 5.0, walk = a.D == 128 ? 4.0 : 2.1, merge = 2.5 + 2.5 * std::min(a.T, 32) / 32;

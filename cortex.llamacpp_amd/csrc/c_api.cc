@@ -44,7 +44,7 @@ struct mi355_context {
 
 static thread_local std::string t_err;
 static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1, g_op_mmq_few = -1;
-int g_op_attn_cols = 0;            // 0: the call's own kernel
+static int g_op_attn_cols = 0;     // mi355_op_flash_attn: 0 the call's own kernel, else attn_cols.hip with so many shares of the keys
 static bool g_backend_ok = false;
 
 static void fail(const std::string &s) { t_err = s; }

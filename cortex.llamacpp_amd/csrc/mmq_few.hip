@@ -551,7 +551,7 @@ __global__ __launch_bounds__(NT, 2) void mmq_few_kernel(const FewArgs a) {
 
 // The output head of a tick: a workgroup takes a run of neighbouring row tiles, and stores the results of HEAD_RUN of them at a time - 256 consecutive bytes a token - to the
 // host's rows while its weights stream: PCIe bounds it from a dozen rows on.  The rows' arg-max is made of what the threads hold anyway.  128256 rows of 4096 columns (Q6_K), us, here /
-// the head, the arg-max and a launch that copies the rows one behind the other: 4 tokens 110 / 99 + 10 + 38, 16 tokens 206 / 104 + 19 + 149.
+// the head, the arg-max and a launch that copies the rows one behind the other: 4 tokens 97 / 99 + 10 + 38, 16 tokens 205 / 104 + 19 + 149.
 template <int TYPE, int MT, int G, int CN>
 __global__ __launch_bounds__(NT, 2) void mmq_few_head_kernel(const FewArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[few_lds<TYPE, MT, G, 1> + head_lds<MT>];
@@ -653,6 +653,11 @@ hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const Act
 
 static int head_blocks(int n_rows) { return std::min((n_rows + 15) / 16, num_cu()); }
 size_t mmq_few_head_scratch() { return 1 + 2 * (size_t)HEAD_MAX_T * (size_t)num_cu(); }
+// Over its whole range the faster one, also where 17 rows and more of Q6_K are the K-split kernel's otherwise (mmq_few_takes), and where the rows stay on the device: us a call of one
+// layer and the head, here / that kernel or mmq_few_kernel with the arg-max, and the copy, behind it
+//   128256 x 4096, rows on the host    3: 219 / 252, 8: 245 / 317, 16: 352 / 424, 17: 390 / 482, 24: 477 / 564, 32: 572 / 668      left on the device   3: 221 / 227, 16: 260 / 274, 17: 310 / 329, 32: 340 / 365
+//   32000 x 4096                       3: 152 / 163, 8: 173 / 188, 16: 214 / 237, 17: 245 / 268, 24: 271 / 302, 32: 315 / 346                           3: 148 / 155, 16: 185 / 199, 17: 216 / 227, 32: 255 / 267
+//   32000 x 2048                       3: 115 / 119, 8: 131 / 144, 16: 167 / 186, 17: 182 / 197, 24: 210 / 227, 32: 251 / 273                           3: 108 / 111, 16: 133 / 147, 17: 148 / 156, 32: 186 / 195
 bool mmq_few_head_takes(int type, int K, int T, const ActQuant &q) {
     return q.qf && (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K & 255) == 0 && T >= 3 && T <= HEAD_MAX_T;
 }

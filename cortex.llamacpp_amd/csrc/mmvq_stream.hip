@@ -222,7 +222,9 @@ void mmvq_stream_set_probe(unsigned long long *p) { (void)hipMemcpyToSymbol(HIP_
 #endif
 
 // Launches of Q8_0 tensors only: from here on the stream is the faster one.  us, stream / register ring, of a 2048-column model: Q | K | V (5.6 MB) 5.2 / 7.0, ffn_down (12.3 MB) 6.1 / 9.3,
-// attn_output (4.5 MB), which then quantises its input itself, 4.8 / 6.1; smaller tensors have not been timed
+// attn_output (4.5 MB), which then quantises its input itself, 4.8 / 6.1.  Steps of twelve layers (columns / ffn columns), us, with the line at 4 / 4.5 / 16 MB: 2048 / 5632 384 / 407 / 481,
+// 2048 / 8192 390 / 415 / 448, 1024 / 4096 350 / 387 / 412, 1024 / 3584 384 / 383 / 406, 1792 / 4864 445 / 472 / 507, 2560 / 6912 448 / 447 / 467, 3072 / 8192 496 / 497 / 540.  Tensors of 2 to 4 MB
+// gain too (1792 / 4864 418, 1024 / 3584 350 with the line at 2)
 static constexpr size_t STREAM_Q80_MIN_BYTES = (size_t)4 << 20;
 
 bool mmvq_stream_applicable(const MMVQArgs &a) {

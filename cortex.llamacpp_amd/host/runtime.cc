@@ -2059,7 +2059,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             for (int ch = 0; ch < nch; ch++) if (seq_of_chunk[(size_t)ch] & bit) lst[c++] = ch;
             cnt[t] = c;
             chunk_lmax_ = std::max(chunk_lmax_, c);
-            if (attn_cols_) {                                  // (by what the sequence holds, wherever its cells are: a conversation's sums do not depend on its neighbours)
+            if (attn_cols_) {                                  // (by the chunks that hold its cells; which those are, and with them the order of the sums, follows the cells it was dealt)
                 aa.chunks = d_chunks_; aa.n_chunks = c;
                 attn_cols_ = c > 0 && flash_attn_cols_takes(aa, true);
                 if (attn_cols_) break;

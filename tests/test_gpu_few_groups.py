@@ -21,7 +21,8 @@ def test_types_share_the_workgroups(be, types, K, Ns, T):  # noqa: F811
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("K,N,T", [(256, 5, 3), (4096, 4100, 4), (11008, 12, 4), (2048, 4097, 8), (5632, 9, 6), (4096, 7, 16), (4096, 4111, 30), (2304, 20, 32), (4352, 4100, 16)])
+@pytest.mark.parametrize("K,N,T", [(256, 5, 3), (4096, 4100, 4), (11008, 12, 4), (2048, 4097, 8), (5632, 9, 6), (4096, 7, 16), (4096, 4111, 30), (2304, 20, 32), (4352, 4100, 16),
+                                   (4096, 4111, 37), (2304, 20, 48), (2048, 9, 33)])         # three token tiles: two super-blocks a wave, all whole and the second ragged; one
 def test_gate_up(be, t, K, N, T):  # noqa: F811
     """Fewer rows than a tile of eight, and a last tile that begins among the rows of the one before."""
     few.test_gate_up_pair(be, t, K, N, T)
