@@ -429,7 +429,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     // thread's outputs are requested BEFORE the (m, l) pairs, so the weight computation runs under them: ticket, one trip
     // for (m, l) + UB splits, one more per further UB (it was ticket + (m, l) + one trip per 8 splits and output).  UB by the splits there are: a load past them is one more
     // trip of the fabric's (us a launch of a step, 4 kv heads of 8 heads of 64 behind 93 cells: 10.0 with thirty-two loads an output for four splits and the argument
-    // segment read field by field, 8.6)
+    // segment read field by field, 8.6 in a replayed step; launched eagerly 9.5)
     constexpr int NE = (RM * D + 255) / 256;
     float macc[NE];
     const float *pp[NE];

@@ -390,7 +390,7 @@ hipError_t launch_moe_route(const float *logits, int T, int n_expert, int k, int
 // What bounds it is latency: 131 KB of weights (8 experts of 4096 columns) for a token.  So sixteen waves, an expert's columns shared by as many as there are; a wave's first
 // eight pieces of weights are in flight before the row's norm is known; the selection is a wave's, a lane an expert.  NTOK rows share a workgroup's weights.
 // NORM (one token): x is the row in front of the norm, so that a step needs no launch that norms it (its expert kernels norm for themselves).
-// us, one token, 8 experts: 7.5, and 5.2 of a norm launch + 9.7 with four waves that walked two experts each and one thread that selected.
+// us, one token, 8 experts, in a replayed step: 7.3 (8.6 launched eagerly), and 5.2 of a norm launch + 9.7 with four waves that walked two experts each and one thread that selected.
 template <int NTOK, bool NORM>
 __global__ __launch_bounds__(1024) void moe_router_kernel(int type, const uint8_t *W, int n_expert, int K, const float *x, const float *nw, float eps, int T, int k, float *logits_out,
                                                           int32_t *ids, float *w, const int32_t *forced) {

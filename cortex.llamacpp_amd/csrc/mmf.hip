@@ -241,7 +241,7 @@ namespace {
 // The encoder's projections (T tokens of one text against f16 weights of a few hundred to a few thousand columns): a product is 19 MB of weights at the most and
 // some microseconds of anything, so what counts is one trip to memory, enough workgroups and no launches around it.  Measured on nomic-embed (768 / 3072 columns)
 // at 187 tokens, us: 768 x 768 30 with the 64 x 64 direct
-// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; now Q | K | V 7.3, output 6.25, gate | up 11.2, down 9.4.  Here:
+// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; now Q | K | V 7.6, output 6.1, gate | up 11.6, down 9.6.  Here:
 //   * 32 rows x 32 TT tokens per workgroup (432 workgroups for Q | K | V at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
 //     both operands - all of them for 768 columns - are requested before the first matrix step;
 //   * a request is whole 128-byte lines of eight rows; the operands (16 bytes of 32 rows) are made through LDS of the wave's own, pieces of a row turned by its number.  Asked for as
