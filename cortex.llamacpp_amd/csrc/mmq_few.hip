@@ -1,10 +1,11 @@
 // mmq_few.hip — the K-split contraction of 3 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
 // K-quant weights in their GGUF form, Q8_K activations, int8 matrix cores, the integer of ggml_vec_dot_q{4,5,6}_K_q8_K per (row, token, super-block).
 //
-// What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and beside them the vector instructions per unit and token tile below, ~130 for Q4_K and 270 for Q6_K at
-// sixteen tokens (two waves per SIMD, whose waits the other wave's instructions do not fill: sixteen waves a CU are no faster).  An 8B Q4_K_M model, kernel times before -> now (before is the
-// 32 x 32 form of mmq.hip, whose waves had no load in flight while they computed and which left half of the CUs without a row tile): gate | up (66 MB) at 4 tokens 27.2 -> 15.5 us, at 37
-// 51.4 -> 34.1; ffn_down at 4, Q4_K and Q6_K, 12.8 and 18.9; Q | K | V at 37 14.1 -> 11.2; the head (431 MB) at 4 129 -> 97, its rows on the host.
+// What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and beside them the vector instructions per unit, ~200 for Q4_K and 280 for Q6_K at 48 tokens and their waits (two
+// waves per SIMD; sixteen waves a CU are no faster); long rows of 37 tokens, 4096 x 14336, the activations' operands, which every workgroup reads: 290 MB from the L2 in 21 us.
+// An 8B Q4_K_M model, kernel times (in front of them the 32 x 32 form of mmq.hip, whose waves had no load in flight while they computed and which left half of the CUs without a row
+// tile): gate | up (66 MB) at 4 tokens 27.2 / 15.3 us, at 37 51.4 / 28.3; ffn_down at 4, Q4_K and Q6_K, 13.6 and 19.0, at 37 20.9 and 24.2; Q | K | V at 37 14.1 / 10.3; the head (431 MB) at 4
+// 129 / 97, its rows on the host.
 //   * A unit of work is 16 weight rows x one super-block (v_mfma_i32_16x16x32_i8: M = 16 tokens, N = 16 rows, K = the 32 weights of one scale group of Q4_K / Q5_K):
 //     a 4096-row tensor is 256 row tiles, one per CU, and 16 tokens pad to 16, 37 to 48.
 //   * One workgroup per CU walks its row tiles; its eight waves take a tile's super-blocks round-robin, and the weights of the next PD units - of the next tile
@@ -14,6 +15,9 @@
 //     128-byte line is asked for by four or five requests: gate | up of an 8B layer took 29 us that way.
 //   * The activations come as operand blocks laid out by the quantiser (ActQuant::qf).  Read from rows of K bytes instead, sixteen lanes hit sixteen lines a power
 //     of two apart: 34 us at 4 tokens, 43 at 16.  A wave meets the same super-blocks in every tile: up to 4096 columns and 48 tokens they stay in registers.
+//   * From 17 tokens on (Q6_K from 9, Q5_K from 33) the groups' scales are folded into the weights, two codes a multiplication (Planes, few_planes): a super-block is two chains of MFMAs
+//     of 64 weights, its integer one shift.  Before, an MFMA a group and four multiplications by its scale a tile: gate | up at 37 tokens 33.9 us, ffn_down of Q6_K 31.2, a prompt turn
+//     of 37 tokens through eight layers of an 8B model 995 -> 903.
 //   * To 8 and 4 tokens the operand's sixteen rows are two and four scale groups of a token (Act): half and a quarter of the multiplications by scales, the same integers.  Whole ticks of
 //     eight layers of an 8B model, four conversations 790 -> 715 us (with PAIR 1 below), seven 797 -> 745.
 //   * The eight partial sums of an output are added in wave order through LDS, so results do not depend on timing - and they are the sums the K-split
@@ -93,7 +97,7 @@ template <int TYPE> struct Frag;
 
 // Q4_K / Q5_K: step J is scale group J (32 weights), the lane's 8 of them are bytes 8 kq .. of the group's 32-byte chunk (low / high nibbles)
 template <> struct Frag<T_Q4_K> {
-    static constexpr bool GROUPS = true;
+    static constexpr bool MINS = true;
     u32x4 h;
     u32x2 q[4];
     __device__ __forceinline__ void get(const uint8_t *lds, uint32_t, int n, int kq) {
@@ -108,7 +112,7 @@ template <> struct Frag<T_Q4_K> {
     }
 };
 template <> struct Frag<T_Q5_K> {
-    static constexpr bool GROUPS = true;
+    static constexpr bool MINS = true;
     u32x4 h;
     u32x2 q[4], qh;
     __device__ __forceinline__ void get(const uint8_t *lds, uint32_t, int n, int kq) {
@@ -126,7 +130,7 @@ template <> struct Frag<T_Q5_K> {
 };
 // Q6_K: step J is quarter J & 3 of half J >> 2 (low nibbles of ql for quarters 0 and 1, high for 2 and 3; two bits of qh), 16-groups 2 J and 2 J + 1
 template <> struct Frag<T_Q6_K> {
-    static constexpr bool GROUPS = false;                    // (two scales per step)
+    static constexpr bool MINS = false;
     u32x2 l[4], h[2];
     u32x4 sc;
     uint32_t d16;
@@ -149,6 +153,48 @@ template <> struct Frag<T_Q6_K> {
     }
 };
 
+// Group scales folded into the weights: of a unit's 64 weights of step S, a lane's sixteen as two int8 planes with  scale * code = (hi << SHIFT) + lo  (+ 128 in both planes of Q5_K),
+// so that a super-block is two chains of MFMAs and one shift, and nothing is multiplied per output and group.  Two codes are multiplied at once, as bytes of a 16-bit lane:
+//   Q4_K / Q5_K: scale = 8 s1 + s0, and a code times three bits stays in its byte (15 * 7, 31 * 7 = 217: the latter with 128 taken off, which the caller adds again as
+//   128 * (8 + 1) times the sum of the activations);
+//   Q6_K: (code - 32) * scale + 128 in 16 bits; its high byte is the one plane, its low one, the 128 taken off again, the other.
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2 as_u16(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+__device__ __forceinline__ uint32_t as_u32(u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+template <int TYPE> struct Planes {
+    static constexpr int SHIFT = TYPE == T_Q6_K ? 8 : 3;
+    uint32_t s0[2], s1[2];                                   // Q4_K / Q5_K: the scales' low and high three bits, a byte a group
+    __device__ __forceinline__ void scales(uint32_t sc_lo, uint32_t sc_hi) {
+        s0[0] = sc_lo & 0x07070707u; s0[1] = sc_hi & 0x07070707u;
+        s1[0] = (sc_lo >> 3) & 0x07070707u; s1[1] = (sc_hi >> 3) & 0x07070707u;
+    }
+    template <int S> __device__ __forceinline__ void step(const Frag<TYPE> &R, int kq, u32x4 &hi, u32x4 &lo) const {
+        const u32x2 c[2] = {R.template codes<2 * S>(), R.template codes<2 * S + 1>()};
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int J = 2 * S + g;
+            if constexpr (TYPE == T_Q6_K) {                  // groups of sixteen: a lane's eight weights of 32 are of group 2 J + (kq >> 1)
+                const int sc = __builtin_amdgcn_sbfe((int)R.sc[J >> 1], 8 * (2 * (J & 1) + (kq >> 1)), 8), off = 128 - 32 * sc;
+                const u16x2 m = {(unsigned short)sc, (unsigned short)sc}, o = {(unsigned short)off, (unsigned short)off};
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t pe = as_u32(as_u16(c[g][i] & 0x00ff00ffu) * m + o), po = as_u32((as_u16(c[g][i]) >> (unsigned short)8) * m + o);
+                    hi[2 * g + i] = __builtin_amdgcn_perm(po, pe, 0x07030501u);
+                    lo[2 * g + i] = __builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u;
+                }
+            } else {
+                const u16x2 w = as_u16(__builtin_amdgcn_perm(s1[J >> 2], s0[J >> 2], 0x0c040c00u + 0x00010001u * (J & 3)));
+                const u16x2 m0 = {w.x, w.x}, m1 = {w.y, w.y};
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    hi[2 * g + i] = as_u32(as_u16(c[g][i]) * m1); lo[2 * g + i] = as_u32(as_u16(c[g][i]) * m0);
+                    if constexpr (TYPE == T_Q5_K) { hi[2 * g + i] ^= 0x80808080u; lo[2 * g + i] ^= 0x80808080u; }
+                }
+            }
+        }
+    }
+};
+
 struct FewArgs {
     MMQSeg seg[3];
     int n_seg, K, T;
@@ -168,20 +214,31 @@ template <int MT, int TYPE, int G> struct Act {
     u32x4 a[MT][4];
     u32x2 bh[MT], bl[MT];
     float yd[MT][4 / G];
-    __device__ __forceinline__ void load(const uint8_t *qf, int tile0, int nb, int sb, int lane, int n) {    // the first n of the tiles
+    // (of the last tile's tokens past the batch, whose results are dropped, the last one's codes: other lines of the caches are not asked for)
+    __device__ __forceinline__ void load_codes(const uint8_t *qf, int tile0, int nb, int sb, int lane, int s, int live) {
+        const int m = lane & 15, kq = lane >> 4;
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            const int tk = t == MT - 1 ? m / G < live ? m / G : live - 1 : m;
+            a[t][s] = ldg16(qf + (size_t)((unsigned)((tile0 + t) * nb + sb) * (unsigned)FEW_BLOCK) + s * 1024 + (kq * 16 + tk) * 16);     // (the block is wave-uniform)
+        }
+    }
+    __device__ __forceinline__ void load_rest(const uint8_t *qf, int tile0, int nb, int sb, int lane) {
         const int m = lane & 15, tk = m / G, kq = lane >> 4;
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            if (t >= n) continue;
-            const uint8_t *p = qf + (size_t)((unsigned)((tile0 + t) * nb + sb) * (unsigned)FEW_BLOCK);     // (wave-uniform)
-#pragma unroll
-            for (int s = 0; s < 4; s++) a[t][s] = ldg16(p + s * 1024 + (kq * 16 + tk) * 16);
+            const uint8_t *p = qf + (size_t)((unsigned)((tile0 + t) * nb + sb) * (unsigned)FEW_BLOCK);
             const int o = tk * 16 + (kq & 1) * 8;
             bh[t] = ldg8(p + FEW_BH + o); bl[t] = ldg8(p + FEW_BL + o);
             if constexpr (G == 1) { const f32x4 y = *reinterpret_cast<const f32x4 *>(p + FEW_D + kq * 16); yd[t][0] = y.x; yd[t][1] = y.y; yd[t][2] = y.z; yd[t][3] = y.w; }
             else if constexpr (G == 2) { const f32x2 y = *reinterpret_cast<const f32x2 *>(p + FEW_D + kq * 8); yd[t][0] = y.x; yd[t][1] = y.y; }
             else yd[t][0] = *reinterpret_cast<const float *>(p + FEW_D + kq * 4);
         }
+    }
+    __device__ __forceinline__ void load(const uint8_t *qf, int tile0, int nb, int sb, int lane, int live) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) load_codes(qf, tile0, nb, sb, lane, s, live);
+        load_rest(qf, tile0, nb, sb, lane);
     }
     // G > 1, behind the loads: the other groups' weights zeroed
     __device__ __forceinline__ void mask(int lane) {
@@ -203,54 +260,119 @@ template <int MT, int TYPE, int G> struct Act {
     }
 };
 
-// the first MT token tiles of A
-template <int TYPE, int MT, int M, int G>
-__device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M, TYPE, G> &A, int kq, bool take, float (*facc)[4 / G]) {
+// Scales in the weights, or on the sums of each group: 16 tokens of Q4_K and Q5_K need no fewer instructions with the former (us a pass of eight layers at 12 tokens, an 8B Q4_K_M and a 7B
+// Q5_K_M model: 722 and 763 with it, 716 and 730 without; at 24, 37 and 48 of the former 806, 911 and 925, before 825, 994 and 1011)
+template <int TYPE, int MT, int G> constexpr bool few_planes = G == 1 && (TYPE == T_Q6_K || MT > (TYPE == T_Q5_K ? 2 : 1));
+// next(s): the operands of step s (4: the rest) are used, others may be asked for
+template <int TYPE, int MT, int G, typename NEXT>
+__device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<MT, TYPE, G> &A, int kq, bool take, float (*facc)[4 / G], NEXT next) {
     constexpr int TPL = 4 / G;                               // a lane's tokens
+    constexpr bool MINS = Frag<TYPE>::MINS;
     const i32x4 z = {0, 0, 0, 0};
     int isum[MT][TPL];
+    // header of Q4_K / Q5_K: d, dmin, twelve bytes of 6-bit scales and mins
+    uint32_t sc_lo = 0, sc_hi = 0, mn_lo = 0, mn_hi = 0;
+    if constexpr (MINS) {
+        sc_lo = R.h.y & 0x3f3f3f3fu; mn_lo = R.h.z & 0x3f3f3f3fu;
+        sc_hi = (R.h.w & 0x0f0f0f0fu) | ((R.h.y >> 2) & 0x30303030u); mn_hi = ((R.h.w >> 4) & 0x0f0f0f0fu) | ((R.h.z >> 2) & 0x30303030u);
+    }
+    if constexpr (few_planes<TYPE, MT, G>) {
+        Planes<TYPE> P;
+        if constexpr (MINS) P.scales(sc_lo, sc_hi);
+        i32x4 H[MT], L[MT];
 #pragma unroll
-    for (int t = 0; t < MT; t++)
+        for (int t = 0; t < MT; t++) {
+            H[t] = z; L[t] = z;
+            if constexpr (TYPE == T_Q5_K) {                  // the sum of the token's activations: its sixteen block sums, in k-quarters 0 and 1
+                const u32x2 one = kq < 2 ? u32x2{0x01010101u, 0x01010101u} : u32x2{0, 0};
+                i32x4 v = mfma32(A.bh[t], one, z);
 #pragma unroll
-        for (int r = 0; r < TPL; r++) isum[t][r] = 0;
-#define HALF(J, t) ((J & 1) ? u32x2{A.a[t][J >> 1].z, A.a[t][J >> 1].w} : u32x2{A.a[t][J >> 1].x, A.a[t][J >> 1].y})
-#define BOTH(S) ({ const u32x2 b0_ = R.template codes<2 * (S)>(), b1_ = R.template codes<2 * (S) + 1>(); u32x4{b0_.x, b0_.y, b1_.x, b1_.y}; })
-    if constexpr (Frag<TYPE>::GROUPS) {
-        // header: d, dmin, twelve bytes of 6-bit scales and mins
-        const uint32_t sc_lo = R.h.y & 0x3f3f3f3fu, mn_lo = R.h.z & 0x3f3f3f3fu;
-        const uint32_t sc_hi = (R.h.w & 0x0f0f0f0fu) | ((R.h.y >> 2) & 0x30303030u), mn_hi = ((R.h.w >> 4) & 0x0f0f0f0fu) | ((R.h.z >> 2) & 0x30303030u);
-        const auto scale = [&](int J) { return (int)(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff); };
-        if constexpr (G == 1) {
-#define STEP(J)                                                                                              \
-        {                                                                                                    \
-            const u32x2 b = R.template codes<J>();                                                           \
-            const int sc = scale(J);                                                                         \
-            _Pragma("unroll") for (int t = 0; t < MT; t++) {                                                 \
-                const i32x4 I = mfma32(HALF(J, t), b, z);                                                    \
-                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[t][r] = __mul24(I[r], sc) + isum[t][r];   \
-                if constexpr (M > 1) { _Pragma("unroll") for (int r = 0; r < 4; r++) asm volatile("" : "+v"(isum[t][r])); }   /* (the sums are reassociated otherwise, every product alive) */ \
-            }                                                                                                \
+                for (int r = 0; r < 4; r++) v[r] <<= 6;
+                v = mfma32(A.bl[t], one, v);
+#pragma unroll
+                for (int r = 0; r < 4; r++) L[t][r] = __mul24(v[r], 128 * 9);
+            }
         }
-        STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
-#undef STEP
-        } else if constexpr (G == 2) {
-#define STEP(S)                                                                                              \
-        {                                                                                                    \
-            const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                                   \
-            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * S + (r & 1))) + isum[0][r >> 1]; \
+#define STEP(S)                                                                                                                      \
+        {                                                                                                                            \
+            u32x4 hi, lo;                                                                                                            \
+            P.template step<S>(R, kq, hi, lo);                                                                                       \
+            _Pragma("unroll") for (int t = 0; t < MT; t++) { H[t] = mfma64(A.a[t][S], hi, H[t]); L[t] = mfma64(A.a[t][S], lo, L[t]); } \
+            next(S);                                                                                                                 \
         }
         STEP(0) STEP(1) STEP(2) STEP(3)
 #undef STEP
-        } else {
-#define STEP(C)                                                                                              \
-        {                                                                                                    \
-            const i32x4 I = mfma64(A.a[0][2 * C + 1], BOTH(2 * C + 1), mfma64(A.a[0][2 * C], BOTH(2 * C), z)); \
-            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * C + r)) + isum[0][0]; \
-        }
-        STEP(0) STEP(1)
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) isum[t][r] = (H[t][r] << Planes<TYPE>::SHIFT) + L[t][r];
+    } else {
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < TPL; r++) isum[t][r] = 0;
+#define HALF(J, t) ((J & 1) ? u32x2{A.a[t][J >> 1].z, A.a[t][J >> 1].w} : u32x2{A.a[t][J >> 1].x, A.a[t][J >> 1].y})
+#define BOTH(S) ({ const u32x2 b0_ = R.template codes<2 * (S)>(), b1_ = R.template codes<2 * (S) + 1>(); u32x4{b0_.x, b0_.y, b1_.x, b1_.y}; })
+        if constexpr (MINS) {
+            const auto scale = [&](int J) { return (int)(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff); };
+            if constexpr (G == 1) {
+#define STEP(J)                                                                                              \
+            {                                                                                                \
+                const int sc = scale(J);                                                                     \
+                const u32x2 b = R.template codes<J>();                                                       \
+                _Pragma("unroll") for (int t = 0; t < MT; t++) {                                             \
+                    const i32x4 I = mfma32(HALF(J, t), b, z);                                                \
+                    _Pragma("unroll") for (int r = 0; r < 4; r++) isum[t][r] = __mul24(I[r], sc) + isum[t][r]; \
+                    if constexpr (MT > 1) { _Pragma("unroll") for (int r = 0; r < 4; r++) asm volatile("" : "+v"(isum[t][r])); }   /* (the sums are reassociated otherwise, every product alive) */ \
+                }                                                                                            \
+            }
+            STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
 #undef STEP
+            } else if constexpr (G == 2) {
+#define STEP(S)                                                                                              \
+            {                                                                                                \
+                const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                               \
+                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * S + (r & 1))) + isum[0][r >> 1]; \
+            }
+            STEP(0) STEP(1) STEP(2) STEP(3)
+#undef STEP
+            } else {
+#define STEP(C)                                                                                              \
+            {                                                                                                \
+                const i32x4 I = mfma64(A.a[0][2 * C + 1], BOTH(2 * C + 1), mfma64(A.a[0][2 * C], BOTH(2 * C), z)); \
+                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * C + r)) + isum[0][0]; \
+            }
+            STEP(0) STEP(1)
+#undef STEP
+            }
+        } else {
+            // the raw codes, 16-group by 16-group, the signed scale on the four results
+            const auto scale = [&](int j) { return (int)(int8_t)((R.sc[j >> 2] >> (8 * (j & 3))) & 0xff); };
+            if constexpr (G == 2) {
+#define STEP(J)                                                                                              \
+            {                                                                                                \
+                const i32x4 I = mfma32(HALF(J, 0), R.template codes<J>(), z);                                   \
+                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * J + (r & 1))) + isum[0][r >> 1]; \
+            }
+            STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
+#undef STEP
+            } else {
+#define STEP(S)                                                                                              \
+            {                                                                                                \
+                const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                               \
+                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * S + r)) + isum[0][0]; \
+            }
+            STEP(0) STEP(1) STEP(2) STEP(3)
+#undef STEP
+            }
         }
-        // the mins against the sixteen block sums: min j meets sums 2 j and 2 j + 1; k-quarters 0 and 1 hold them, 2 and 3 are zero
+#undef HALF
+#undef BOTH
+#pragma unroll
+        for (int s = 0; s < 4; s++) next(s);
+    }
+    // the block sums: against the mins (min j meets sums 2 j and 2 j + 1), or for the code's "- 32" against the scales; k-quarters 0 and 1 hold them, 2 and 3 are zero
+    if constexpr (MINS) {
         const uint32_t mw = kq == 0 ? mn_lo : mn_hi;
         u32x2 bm = {__builtin_amdgcn_perm(0, mw, 0x01010000u), __builtin_amdgcn_perm(0, mw, 0x03030202u)};
         if (kq >= 2) bm = u32x2{0, 0};
@@ -266,58 +388,23 @@ __device__ __forceinline__ void superblock(const Frag<TYPE> &R, const Act<M, TYP
             for (int r = 0; r < TPL; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)isum[t][r] - (dm * A.yd[t][r]) * (float)ms[G * r];
         }
     } else {
-        // The raw codes against the activations, 16-group by 16-group (a step of 32 weights is two of them: the k-quarters of the other one are
-        // zeroed), the signed scale on the four results; the code's "- 32" is the scales against the block sums.  (The scale in the weight, as two int8 planes of
-        // sc * (q - 32): 20 instructions per four weights, the head of an 8B model - 431 MB - at 4 tokens 131 us; this form 8 and 16 per token tile: 109 us)
-        const auto scale = [&](int j) { return (int)(int8_t)((R.sc[j >> 2] >> (8 * (j & 3))) & 0xff); };
-        if constexpr (G == 1) {
-        const uint32_t m0 = kq < 2 ? ~0u : 0u, m1 = ~m0;
-#define STEP(J)                                                                                              \
-        {                                                                                                    \
-            const u32x2 b = R.template codes<J>();                                                           \
-            const int s0 = scale(2 * J), s1 = scale(2 * J + 1);                                              \
-            const u32x2 b0 = {b.x & m0, b.y & m0}, b1 = {b.x & m1, b.y & m1};                                \
-            _Pragma("unroll") for (int t = 0; t < MT; t++) {                                                 \
-                const u32x2 av = HALF(J, t);                                                                 \
-                const i32x4 I0 = mfma32(av, b0, z), I1 = mfma32(av, b1, z);                                  \
-                _Pragma("unroll") for (int r = 0; r < 4; r++) isum[t][r] = __mul24(I1[r], s1) + (__mul24(I0[r], s0) + isum[t][r]); \
-                if constexpr (M > 1 || J == 3) { _Pragma("unroll") for (int r = 0; r < 4; r++) asm volatile("" : "+v"(isum[t][r])); } \
-            }                                                                                                \
-        }
-        STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
-#undef STEP
-        } else if constexpr (G == 2) {
-#define STEP(J)                                                                                              \
-        {                                                                                                    \
-            const i32x4 I = mfma32(HALF(J, 0), R.template codes<J>(), z);                                    \
-            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][r >> 1] = __mul24(I[r], scale(2 * J + (r & 1))) + isum[0][r >> 1]; \
-        }
-        STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5) STEP(6) STEP(7)
-#undef STEP
-        } else {
-#define STEP(S)                                                                                              \
-        {                                                                                                    \
-            const i32x4 I = mfma64(A.a[0][S], BOTH(S), z);                                                   \
-            _Pragma("unroll") for (int r = 0; r < 4; r++) isum[0][0] = __mul24(I[r], scale(4 * S + r)) + isum[0][0]; \
-        }
-        STEP(0) STEP(1) STEP(2) STEP(3)
-#undef STEP
-        }
-        u32x2 bm = kq == 0 ? u32x2{R.sc.x, R.sc.y} : u32x2{R.sc.z, R.sc.w};
-        if (kq >= 2) bm = u32x2{0, 0};
         const float dd = h2f((uint16_t)(take ? R.d16 : 0u));
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-            i32x4 ms = mfma32(A.bh[t], bm, z);
+        if constexpr (G > 1) {
+            u32x2 bm = kq == 0 ? u32x2{R.sc.x, R.sc.y} : u32x2{R.sc.z, R.sc.w};
+            if (kq >= 2) bm = u32x2{0, 0};
+            i32x4 ms = mfma32(A.bh[0], bm, z);
 #pragma unroll
             for (int r = 0; r < 4; r++) ms[r] <<= 6;
-            ms = mfma32(A.bl[t], bm, ms);
+            ms = mfma32(A.bl[0], bm, ms);
 #pragma unroll
-            for (int r = 0; r < TPL; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)(isum[t][r] - 32 * ms[G * r]);
+            for (int r = 0; r < TPL; r++) isum[0][r] -= 32 * ms[G * r];
         }
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < TPL; r++) facc[t][r] += (dd * A.yd[t][r]) * (float)isum[t][r];
     }
-#undef HALF
-#undef BOTH
+    next(4);
 }
 
 // LDS of a workgroup: every wave's staging area (NP units), then the sets of partial sums [wave][unit][tile * 4 / G + r][lane]
@@ -349,8 +436,8 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     const int row_max = sg.n_rows > TR ? sg.n_rows - TR : 0; // a tile's first row at most: the last tile begins early enough to be whole, and stores the rows that are its own
     uint8_t *stage = smem + wave * (NP * Raw<TYPE, PAIR == 1>::LDS);
     float *part = reinterpret_cast<float *>(smem + stage_bytes);
-    // token tiles are worked on two at a time (the registers of their operands); the operands of a pair that is read again stay a unit ahead
-    constexpr int NC = (MT + 1) / 2, PA = CN > 0 ? CN : MT == 1 ? 2 : 1;
+    // operands that are read again stay a unit or two ahead
+    constexpr int PA = CN > 0 ? CN : MT == 1 ? 2 : 1;
     static_assert(CN == 0 || MT <= 3, "operands of four token tiles are not kept");
     static_assert(G == 1 || MT == 1, "one token tile");
     const int cn = CN > 0 ? CN : (nb + NW - 1) / NW;
@@ -365,11 +452,11 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     };
     clear();
     typedef Raw<TYPE, PAIR == 1> RawT;
-    typedef Act<MT == 1 ? 1 : 2, TYPE, G> ActT;
+    typedef Act<MT, TYPE, G> ActT;
     typename RawT::Where where;
     RawT::where(where, sg.W, PAIR == 1 ? a.seg[1].W : nullptr, sg.n_rows < TR ? sg.n_rows : TR, (unsigned)sg.row_bytes, nb, lane);
     RawT R[PD][NP];
-    ActT A[PA][NC];
+    ActT A[PA];
     // the unit the next request is for; past the end it stays on the last one
     int l_tile = tile, l_i = 0;
     auto request = [&](RawT (&r)[NP]) {
@@ -380,10 +467,8 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
         if (l_i + 1 < cn) l_i++;
         else if (l_tile + n_blocks < tiles) { l_tile += n_blocks; l_i = 0; }
     };
-    auto act = [&](ActT &x, int c, int i) {
-        const int sb = wave + NW * i;
-        x.load(a.qf, blockIdx.y * MT + 2 * c, nb, sb < nb ? sb : nb - 1, lane, MT - 2 * c);
-    };
+    const int live = T - 16 * (MT * (int)blockIdx.y + MT - 1) < 1 ? 1 : T - 16 * (MT * (int)blockIdx.y + MT - 1);
+    const auto act_sb = [&](int i) { const int sb = wave + NW * i; return sb < nb ? sb : nb - 1; };
     // an output of a finished tile: element e = tid + NT j of [tile * TPL + r][lane].  Its residual is requested a tile ahead, in front of the weights that follow
     constexpr int NS = MT * TPL * 64, NE = (NS + NT - 1) / NT;
     float rv[NE];
@@ -448,9 +533,7 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     };
     residual(tile);
 #pragma unroll
-    for (int i = 0; i < PA; i++)
-#pragma unroll
-        for (int c = 0; c < NC; c++) act(A[i][c], c, i < cn ? i : 0);
+    for (int i = 0; i < PA; i++) A[i].load(a.qf, blockIdx.y * MT, nb, act_sb(i < cn ? i : 0), lane, live);
     // (the requests in the order of their use, none moved past another: a wait for one slot must not be a wait for the others)
 #pragma unroll
     for (int u = 0; u < PD; u++) { __builtin_amdgcn_sched_barrier(0); request(R[u]); __builtin_amdgcn_sched_barrier(0); }
@@ -458,10 +541,10 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
     static_assert(CN > 0 || PD % PA == 0, "activation slots turn with the weight slots");
     if constexpr (CN > 0) {
 #pragma unroll
-        for (int i = 0; i < PA; i++) A[i][0].mask(lane);
+        for (int i = 0; i < PA; i++) A[i].mask(lane);
     }
     int i = 0;
-    auto unit = [&](RawT (&r)[NP], ActT (&x)[NC], int i) {
+    auto unit = [&](RawT (&r)[NP], ActT &x, int i) {
         const bool take = wave + NW * i < nb;                              // (a tile of nb super-blocks does not divide by the waves: the last unit's share is multiplied by a zero scale, not branched around)
         uint32_t d16[NP];
 #pragma unroll
@@ -469,20 +552,19 @@ __device__ __forceinline__ void few_body(const FewArgs &a, const MMQSeg &sg, int
         __builtin_amdgcn_sched_barrier(0);                                 // (a wave's LDS accesses are made in order)
         request(r);                                                        // the slot's next unit, in flight across this one's arithmetic
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (CN == 0) x[0].mask(lane);
+        if constexpr (CN == 0) x.mask(lane);
+        const int j = i + PA, then = act_sb(j < cn ? j : j - cn < cn ? j - cn : 0);
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            constexpr int LAST = MT - 2 * (NC - 1);
-#pragma unroll
-            for (int p = 0; p < NP; p++) {
-                Frag<TYPE> f;
-                f.get(stage + p * RawT::LDS, d16[p], n, kq);
-                if (c < NC - 1 || LAST == 2) superblock<TYPE, MT == 1 ? 1 : 2>(f, x[c], kq, take, facc[p] + 2 * c);
-                else superblock<TYPE, 1>(f, x[c], kq, take, facc[p] + 2 * c);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (CN == 0) { const int j = i + PA; act(x[c], c, j < cn ? j : j - cn < cn ? j - cn : 0); __builtin_amdgcn_sched_barrier(0); }
+        for (int p = 0; p < NP; p++) {
+            Frag<TYPE> f;
+            f.get(stage + p * RawT::LDS, d16[p], n, kq);
+            superblock<TYPE, MT, G>(f, x, kq, take, facc[p], [&](int s) {
+                if (CN > 0 || p < NP - 1) return;
+                if (s < 4) x.load_codes(a.qf, blockIdx.y * MT, nb, then, lane, s, live); else x.load_rest(a.qf, blockIdx.y * MT, nb, then, lane);
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
+        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_wave_barrier();
     };
     const int mine = (tiles - tile + n_blocks - 1) / n_blocks, S = mine * cn;
