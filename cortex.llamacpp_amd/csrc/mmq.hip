@@ -144,15 +144,15 @@ template <> struct RowSB<T_Q5_K> {
         return i32x4{Q5C(v.x, qh.x), Q5C(v.y, qh.y), Q5C(v.z, qh.z), Q5C(v.w, qh.w)};
 #undef Q5C
     }
-    template <int J> __device__ __forceinline__ void bop(uint32_t sc, i32x4 &bh, i32x4 &bl) const {
+    template <int J, int S = 5> __device__ __forceinline__ void bop(uint32_t sc, i32x4 &bh, i32x4 &bl) const {
         const u32x4 v = (J >> 1) == 0 ? q0 : (J >> 1) == 1 ? q1 : (J >> 1) == 2 ? q2 : q3;
         constexpr int sh = (J & 1) * 4;
         uint32_t hx, lx;
 #define Q5W(vv, hh) ((((vv) >> sh) & 0x0f0f0f0f) | ((((hh) >> J) & 0x01010101u) << 4))
-        planes_u<5>(Q5W(v.x, qh.x), sc, hx, lx); bh.x = (int)hx; bl.x = (int)lx;
-        planes_u<5>(Q5W(v.y, qh.y), sc, hx, lx); bh.y = (int)hx; bl.y = (int)lx;
-        planes_u<5>(Q5W(v.z, qh.z), sc, hx, lx); bh.z = (int)hx; bl.z = (int)lx;
-        planes_u<5>(Q5W(v.w, qh.w), sc, hx, lx); bh.w = (int)hx; bl.w = (int)lx;
+        planes_u<S>(Q5W(v.x, qh.x), sc, hx, lx); bh.x = (int)hx; bl.x = (int)lx;
+        planes_u<S>(Q5W(v.y, qh.y), sc, hx, lx); bh.y = (int)hx; bl.y = (int)lx;
+        planes_u<S>(Q5W(v.z, qh.z), sc, hx, lx); bh.z = (int)hx; bl.z = (int)lx;
+        planes_u<S>(Q5W(v.w, qh.w), sc, hx, lx); bh.w = (int)hx; bl.w = (int)lx;
 #undef Q5W
     }
 };
@@ -668,12 +668,10 @@ __global__ __launch_bounds__(NTHREADS) void mmq_ksplit_kernel(const KSplitArgs a
 // exactly as the MFMA B operands are consumed, so the prefill kernel does no per-weight VALU work at all:
 //   block(rt, sb) = 32 rows x one super-block:  [K-step J 0..7][plane 0 = hi, 1 = lo][lane 0..63][16 B]  (16 KB)
 //                                               [row n 0..31][16 B meta: d | dmin << 16 (f16 bits), mins 0-3, mins 4-7, 0]
-// 2 bytes per weight + 1/16 B meta (Q4_K: 3.7x the GGUF bytes).  Q6_K planes carry the SIGNED code (q - 32), so that
-// type needs no block-sum term at all.
+// 2 bytes per weight + 1/16 B meta.  Q6_K planes carry the SIGNED code (q - 32), so that type needs no block-sum term at all.  (Q4_K and Q5_K: as codes, below)
 constexpr int PL_BLOCK = 8 * 2 * 1024 + 32 * 16;
 
-template <int TYPE>
-__global__ __launch_bounds__(256) void mmq_expand_kernel(const uint8_t *W, size_t row_bytes, int n_rows, int nb, int n_rt, uint8_t *planes) {
+__global__ __launch_bounds__(256) void mmq_expand_kernel(const uint8_t *W, size_t row_bytes, int n_rows, int nb, int n_rt, uint8_t *planes) {      // Q6_K
     const int lane = threadIdx.x & 63;
     const int idx = blockIdx.x * 4 + (threadIdx.x >> 6);     // (row tile, super-block)
     if (idx >= n_rt * nb) return;
@@ -681,27 +679,19 @@ __global__ __launch_bounds__(256) void mmq_expand_kernel(const uint8_t *W, size_
     const int n = lane & 31, kg = lane >> 5;
     int row = rt * 32 + n;
     if (row >= n_rows) row = n_rows - 1;
-    RowSB<TYPE> R;
+    RowSB<T_Q6_K> R;
     R.load(W + (size_t)row * row_bytes, nb, sb, kg);
     uint8_t *blk = planes + (size_t)idx * PL_BLOCK;
-    uint32_t sc_lo = 0, sc_hi = 0, mn_lo = 0, mn_hi = 0;
-    if constexpr (TYPE != T_Q6_K) R.scales(sc_lo, sc_hi, mn_lo, mn_hi);
 #define EXP(J)                                                                                                 \
     {                                                                                                          \
         i32x4 bh, bl;                                                                                          \
-        if constexpr (TYPE == T_Q6_K) R.template bop_signed<J>(R.scale_pk(8 * (J >> 2) + 2 * (J & 3) + kg), bh, bl); \
-        else R.template bop<J>(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff, bh, bl);                     \
+        R.template bop_signed<J>(R.scale_pk(8 * (J >> 2) + 2 * (J & 3) + kg), bh, bl);                         \
         *reinterpret_cast<i32x4 *>(blk + (J * 2) * 1024 + lane * 16) = bh;                                     \
         *reinterpret_cast<i32x4 *>(blk + (J * 2 + 1) * 1024 + lane * 16) = bl;                                 \
     }
     EXP(0) EXP(1) EXP(2) EXP(3) EXP(4) EXP(5) EXP(6) EXP(7)
 #undef EXP
-    if (kg == 0) {
-        u32x4 m = {0, 0, 0, 0};
-        if constexpr (TYPE == T_Q6_K) m.x = R.d16;
-        else { m.x = R.h.x; m.y = mn_lo; m.z = mn_hi; }
-        *reinterpret_cast<u32x4 *>(blk + 16384 + n * 16) = m;
-    }
+    if (kg == 0) *reinterpret_cast<u32x4 *>(blk + 16384 + n * 16) = u32x4{R.d16, 0, 0, 0};
 }
 
 // Q2_K and Q3_K into the same plane format (their prompts then run on the kernels below; there is no expand-on-the-fly form for them):
@@ -778,8 +768,69 @@ __global__ __launch_bounds__(256) void mmq_expand_small_kernel(const uint8_t *W,
         *reinterpret_cast<u32x4 *>(blk + 16384 + n * 16) = m;
     }
 }
-// which fold a plane set takes: the block-sum ("mins") form with shift 5, or the signed form with shift 6
-__host__ __device__ constexpr bool planes_have_mins(int type) { return type == T_Q4_K || type == T_Q5_K || type == T_Q2_K; }
+// Q4_K as codes, the kernels make the planes of them a super-block ahead: a scale is 8 s1 + s0, and a code times three bits stays in its byte, so one 16-bit multiplication makes two
+// products:  isum = 8 (s1 q . a) + (s0 q . a).  Q5_K with the seven low bits of p as one plane and the four high ones as nibbles of two K-steps:  isum = 128 (hi . a) + (lo . a).
+//   block(rt, sb) = 32 rows x one super-block:  Q4_K [codes of K-steps 2 c and 2 c + 1, a nibble each: c 0..3][lane][16 B]      [row n][16 B: s0, s1 of the eight groups]
+//                                               Q5_K [low plane of K-step 0..7][lane][16 B][high nibbles of K-steps 2 c, 2 c + 1][lane][16 B]
+//                                               [row n][16 B meta as above]
+enum PlaneForm { PF_SIGNED, PF_MINS, PF_CODES, PF_NIBBLES };
+__host__ __device__ constexpr PlaneForm plane_form(int type) { return type == T_Q4_K ? PF_CODES : type == T_Q5_K ? PF_NIBBLES : type == T_Q2_K ? PF_MINS : PF_SIGNED; }
+__host__ __device__ constexpr int plane_words(int form) { return form == PF_CODES ? 4096 : form == PF_NIBBLES ? 12288 : 16384; }        // bytes of a block in front of its rows' words
+__host__ __device__ constexpr int plane_block(int form) { return plane_words(form) + (form == PF_CODES ? 1024 : 512); }
+__host__ __device__ constexpr int plane_shift(int form) { return form == PF_SIGNED ? 6 : form == PF_MINS ? 5 : form == PF_NIBBLES ? 7 : 3; }
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+// K-step J of what a lane holds of a block: codes, its 16 B of them and the scales of K-steps 2 (J / 2) and + 1 -> both planes; nibbles -> the high one
+template <int FORM, int J>
+__device__ __forceinline__ void expand_words(u32x4 raw, uint32_t sw, i32x4 &hi, i32x4 &lo) {
+    const u16x2 s = __builtin_bit_cast(u16x2, perm(0, sw, J & 1 ? 0x0c030c02u : 0x0c010c00u)), s0 = {s.x, s.x}, s1 = {s.y, s.y};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t q = (J & 1 ? raw[e] >> 4 : raw[e]) & 0x0f0f0f0fu;
+        if (FORM == PF_NIBBLES) { hi[e] = (int)q; continue; }
+        hi[e] = (int)__builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, q) * s1));
+        lo[e] = (int)__builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, q) * s0));
+    }
+}
+template <int TYPE>
+__global__ __launch_bounds__(256) void mmq_pack_kernel(const uint8_t *W, size_t row_bytes, int n_rows, int nb, int n_rt, uint8_t *planes) {
+    constexpr int FORM = plane_form(TYPE), WORDS = plane_words(FORM), BLOCK = plane_block(FORM);
+    const int lane = threadIdx.x & 63;
+    const int idx = blockIdx.x * 4 + (threadIdx.x >> 6);     // (row tile, super-block)
+    if (idx >= n_rt * nb) return;
+    const int rt = idx / nb, sb = idx - rt * nb;
+    const int n = lane & 31, kg = lane >> 5;
+    int row = rt * 32 + n;
+    if (row >= n_rows) row = n_rows - 1;
+    RowSB<TYPE> R;
+    R.load(W + (size_t)row * row_bytes, nb, sb, kg);
+    uint8_t *blk = planes + (size_t)idx * BLOCK;
+    u32x4 *o = reinterpret_cast<u32x4 *>(blk) + lane;
+    uint32_t sc_lo, sc_hi, mn_lo, mn_hi;
+    R.scales(sc_lo, sc_hi, mn_lo, mn_hi);
+    if constexpr (FORM == PF_CODES) {
+        o[0] = R.q0; o[64] = R.q1; o[128] = R.q2; o[192] = R.q3;
+        u32x4 v;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint32_t w = (c < 2 ? sc_lo : sc_hi) >> (16 * (c & 1)), a = w & 0xff, b = (w >> 8) & 0xff;
+            v[c] = (a & 7) | (a >> 3) << 8 | (b & 7) << 16 | (b >> 3) << 24;
+        }
+        if (kg) *reinterpret_cast<u32x4 *>(blk + WORDS + n * 16) = v;
+    } else {
+        u32x4 hi;                                               // of a pair of K-steps
+#define OUT(J)                                                                                                 \
+        {                                                                                                      \
+            i32x4 h, l;                                                                                        \
+            R.template bop<J, 7>(((J < 4 ? sc_lo : sc_hi) >> (8 * (J & 3))) & 0xff, h, l);                     \
+            o[64 * J] = __builtin_bit_cast(u32x4, l);                                                          \
+            _Pragma("unroll") for (int e = 0; e < 4; e++) hi[e] = J & 1 ? hi[e] | (uint32_t)h[e] << 4 : (uint32_t)h[e]; \
+            if (J & 1) o[64 * (8 + J / 2)] = hi;                                                               \
+        }
+        OUT(0) OUT(1) OUT(2) OUT(3) OUT(4) OUT(5) OUT(6) OUT(7)
+#undef OUT
+    }
+    if (kg == 0) *reinterpret_cast<u32x4 *>(blk + BLOCK - 512 + n * 16) = u32x4{R.h.x, mn_lo, mn_hi, 0};
+}
 
 // Several tensors that share the activation and whose plane sets lie back to back in memory (attn_q | attn_k | attn_v) run as
 // ONE launch over the concatenated rows: rows [row_end[s-1], row_end[s]) go to out[s] with leading dimension ld[s] (segment
@@ -790,16 +841,17 @@ struct PlanesOut {
     int ld[3];
     int row_end[3];
     int n_seg;
-    unsigned mins_mask;     // bit s: segment s is Q4_K / Q5_K (block-sum term, shift 5); mmq_planes2_kernel<2> only
+    int form[3];            // PlaneForm of a segment, and where its blocks begin: mmq_planes2_kernel<2> and <3> only
+    size_t at[3];
 };
 
-// MINS: Q4_K / Q5_K (block-sum term, shift 5); otherwise Q6_K (shift 6, nothing else)
-template <bool MINS, int MT>
+template <int FORM, int MT>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *planes, int n_rows, int K, int T, int n_row_tiles, int n_tok_tiles,
                                                               const int8_t *aq, const float *ad, const int8_t *abh, const int8_t *abl,
                                                               const PlanesOut po, const float *resid) {
     using G = Geo<MT>;
-    constexpr int SH = MINS ? 5 : 6;
+    constexpr bool MINS = FORM != PF_SIGNED, PACKED = FORM >= PF_CODES;
+    constexpr int SH = plane_shift(FORM), BLOCK = plane_block(FORM), WORDS = plane_words(FORM);
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     // two activation tiles: super-block sb is read from buffer sb & 1 while sb + 1 is written into the other one, so one
     // barrier per super-block suffices and the LDS writes overlap the other waves' MFMA work
@@ -824,7 +876,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
     const int tok0 = tok_tile * G::TOK_TILE;
     const int n = lane & 31, kg = lane >> 5;
     const bool tile_ok = rt32 < n_rt32;
-    const uint8_t *blk0 = planes + (size_t)(tile_ok ? rt32 : n_rt32 - 1) * nb * PL_BLOCK;
+    const uint8_t *blk0 = planes + (size_t)(tile_ok ? rt32 : n_rt32 - 1) * nb * BLOCK;
     const unsigned b_off = (unsigned)lane * 16u;
 
     unsigned st_g[G::NST], st_l[G::NST];
@@ -852,13 +904,14 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
     // ring of K-steps: 4 (half a super-block ahead) where two token tiles per wave leave no registers for more; 8 (a whole
     // super-block ahead) with one tile per wave, whose 2 MFMAs per K-step otherwise cover only 256 cycles of the planes' latency
     constexpr int RING = MT == 1 ? 8 : 4;
-    i32x4 Bh[RING], Bl[RING];
+    i32x4 Bh[RING], Bl[RING];                                   // (a slot's Bh holds codes and nibbles as they are)
+    auto ld_b = [&](const uint8_t *blk, int j, int slot) {
+        Bh[slot] = *reinterpret_cast<const i32x4 *>(blk + (FORM == PF_CODES ? j >> 1 : FORM == PF_NIBBLES ? 8 + (j >> 1) : 2 * j) * 1024 + b_off);
+        if (FORM != PF_CODES) Bl[slot] = *reinterpret_cast<const i32x4 *>(blk + (FORM == PF_NIBBLES ? j : 2 * j + 1) * 1024 + b_off);
+    };
 #pragma unroll
-    for (int j = 0; j < RING; j++) {
-        Bh[j] = *reinterpret_cast<const i32x4 *>(blk0 + (j * 2) * 1024 + b_off);
-        Bl[j] = *reinterpret_cast<const i32x4 *>(blk0 + (j * 2 + 1) * 1024 + b_off);
-    }
-    u32x4 meta = ldg16(blk0 + 16384 + n * 16);
+    for (int j = 0; j < RING; j++) ld_b(blk0, j, j);
+    u32x4 meta = ldg16(blk0 + BLOCK - 512 + n * 16), scales = FORM == PF_CODES ? ldg16(blk0 + WORDS + n * 16) : meta;
     {
         u32x4 tmp[G::NST];
 #pragma unroll
@@ -879,7 +932,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
         s_aq = p_aq(sb & 1); s_bh = p_bh(sb & 1); s_bl = p_bl(sb & 1); s_yd = p_yd(sb & 1);
         const bool more = sb + 1 < nb;
         const int sbn = more ? sb + 1 : sb;
-        const uint8_t *blkn = blk0 + (size_t)sbn * PL_BLOCK;
+        const uint8_t *blkn = blk0 + (size_t)sbn * BLOCK;
         // next activation tile: request now, park in registers across the MFMA work
         u32x4 nxt[G::NST];
 #pragma unroll
@@ -893,12 +946,13 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
                 nbl = ldg16(abl + ((size_t)pl_g + (unsigned)sbn) * 16);
             }
         }
-        const u32x4 mcur = meta;
-        meta = ldg16(blkn + 16384 + n * 16);
+        const u32x4 mcur = meta, scur = scales;
+        meta = ldg16(blkn + BLOCK - 512 + n * 16);
+        if (FORM == PF_CODES) scales = ldg16(blkn + WORDS + n * 16);
 
         i32x16 H[MT], L[MT];
         const int8_t *abase = s_aq + (tw * MT * 32 + n) * A_STRIDE + 16 * kg;
-        const uint8_t *blkc = blk0 + (size_t)sb * PL_BLOCK;
+        const uint8_t *blkc = blk0 + (size_t)sb * BLOCK;
         // K-step J: MFMAs on ring slot J & 3, then the slot is refilled with the operand four K-steps ahead (same
         // super-block for J < 4, the next one otherwise): every B register waits half an iteration before its use
         // A fragments are read one K-step ahead of the MFMAs that use them (two register sets)
@@ -911,17 +965,16 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
                 _Pragma("unroll") for (int t = 0; t < MT; t++)                                                \
                     ANXT[t] = *reinterpret_cast<const i32x4 *>(abase + t * 32 * A_STRIDE + 32 * (J + 1));     \
             }                                                                                                 \
+            i32x4 bh = Bh[J & (RING - 1)], bl = Bl[J & (RING - 1)];                                           \
+            if constexpr (PACKED) expand_words<FORM, J>(__builtin_bit_cast(u32x4, bh), scur[J >> 1], bh, bl); \
             _Pragma("unroll") for (int t = 0; t < MT; t++) {                                                  \
                 if (J == 0) {                                                                                 \
                     i32x16 z;                                                                                 \
                     _Pragma("unroll") for (int r = 0; r < 16; r++) z[r] = 0;                                  \
-                    H[t] = mfma_i8(ACUR[t], Bh[J & (RING - 1)], z); L[t] = mfma_i8(ACUR[t], Bl[J & (RING - 1)], z); \
-                } else { H[t] = mfma_i8(ACUR[t], Bh[J & (RING - 1)], H[t]); L[t] = mfma_i8(ACUR[t], Bl[J & (RING - 1)], L[t]); } \
+                    H[t] = mfma_i8(ACUR[t], bh, z); L[t] = mfma_i8(ACUR[t], bl, z);                           \
+                } else { H[t] = mfma_i8(ACUR[t], bh, H[t]); L[t] = mfma_i8(ACUR[t], bl, L[t]); }              \
             }                                                                                                 \
-            const uint8_t *src = RING == 8 ? blkn + (J * 2) * 1024 + b_off                                    \
-                                           : (J < 4 ? blkc : blkn) + (((J + 4) & 7) * 2) * 1024 + b_off;       \
-            Bh[J & (RING - 1)] = *reinterpret_cast<const i32x4 *>(src);                                       \
-            Bl[J & (RING - 1)] = *reinterpret_cast<const i32x4 *>(src + 1024);                                \
+            ld_b(RING == 8 ? blkn : J < 4 ? blkc : blkn, RING == 8 ? J : (J + 4) & 7, J & (RING - 1));         \
         }
         KSTEP(0, a0, a1) KSTEP(1, a1, a0) KSTEP(2, a0, a1) KSTEP(3, a1, a0) KSTEP(4, a0, a1) KSTEP(5, a1, a0) KSTEP(6, a0, a1) KSTEP(7, a1, a0)
 #undef KSTEP
@@ -1022,25 +1075,27 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
     }
 }
 
-// ---- the same contraction in 128-row x 256-token workgroup tiles: activations through LDS, planes straight into registers.
-// Eight waves: wave (rw, tw) owns 32 rows x 128 tokens of the tile, i.e. the 32-row tile rw of token half tw.  Per super-block a wave takes the 16 KiB of its planes ONCE,
-// as the sixteen MFMA operands they are laid out as, and holds them in 64 registers while it walks its four token tiles; both halves ask for the same planes at about
-// the same time, so the second finds them in the vector L1.  The 256 x 256 activation codes come by LDS-DMA one super-block ahead (two buffers, one barrier per super-block):
+// ---- the same contraction in 128-row x 256-token workgroup tiles: activations through LDS, weights straight into registers.
+// Eight waves: wave (rw, tw) owns 32 rows x 128 tokens of the tile, i.e. the 32-row tile rw of token half tw.  Per super-block a wave has its planes as the sixteen MFMA operands that they
+// are, in 64 registers, while it walks its four token tiles; both halves ask for the same words at about the same time, so the second finds them in the vector L1.  The words of the next
+// super-block are asked for in the last token tile, as the operands' registers come free; of packed forms they wait in the registers of the operands that are made of them, K-step by K-step two
+// steps ahead of the first token tile.  The 256 x 256 activation codes come by LDS-DMA one super-block ahead (two buffers, one barrier per super-block):
 //   codes  64 KiB = [token 0..255][16 pieces of 16 B]; piece p of token t sits in slot p ^ (t & 15) (applied on the SOURCE side of the DMA, whose LDS side is
 //          lane-linear), so the 16 lanes of a ds_read_b128 phase hit all 64 banks
-//   block sums 8 KiB (int16, turned into f16 in place by the wave that fetched them), the rows' d / dmin / mins words, and the tokens' scales (three sets: a fold
-//          reaches into the next super-block)
+//   block sums 8 KiB (int16, turned into f16 in place by the wave that fetched them), the rows' words (scales, d / dmin / mins; once, for both halves), and the tokens' scales (three sets: a
+//          fold reaches into the next super-block)
 // The f32 fold of a token tile (five vector instructions an output) runs BETWEEN the MFMAs of the next tile, two outputs per K-step, on the other of two accumulator
 // pairs: a wave in an MFMA phase of its own leaves the vector unit idle, and one in a fold of its own the matrix cores.
 //
-// What bounds it: gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens) is 448 workgroups, two rounds of the 256 CUs of which the second is three quarters full;
-// in each a SIMD issues 2176 MFMAs of 32 cycles, so both rounds are 58 us at 2.4 GHz, 39 % of the 148 us that a launch takes back to back.  The clock is one part of the rest: with
-// all-zero operands, the same instructions and the same bytes, 127 us.  Counters over a 512-token prompt: matrix cores busy in 0.39 of the launch, 6.8 vector instructions an MFMA,
-// waves waiting in 0.38 of their cycles (for the planes, which both token halves ask the L2 for, 128 KiB per super-block and CU, or at the barrier behind the codes: not told
-// apart).  Tried, and slower: two 128 x 128 workgroups per CU, each with planes of its own (192 KiB), by 4 %; 16 x 16 x 64 MFMA tiles, which read twice the registers per product, the same.
-// Inside a 512-token prompt: 167 -> 153 us (before: planes through LDS as well, half a super-block per barrier, folds beside the
-// other half's MFMAs); the experts of an 8x7B layer (611 tokens, 1222 rows): gate | up 628 -> 548 us, down 276 -> 253, where a batch of ~150 rows is now dealt evenly to both halves.
-// Touching the super-block after the next one, to have it in the L2: 12 % slower (64 lines an instruction).
+// What bounds it: gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens) is 448 workgroups, two rounds of the 256 CUs of which the second is three quarters full; in each a SIMD issues
+// 2176 MFMAs of 32 cycles, so both rounds are 58 us at 2.4 GHz; but MFMAs of random operands alone run at 1.9 GHz here, with ten f32 instructions a pair of them at 1.5: the card's power.  What
+// instructions and bytes cost comes on top of the MFMAs, whichever unit has room: of a round of 73 us (2048 tokens) the MFMAs are 47, the fold 15, the expansion of codes 6, the activations'
+// way to LDS 3 to 6.  So bytes were taken out where instructions do not cost as much (us, before -> now, with weights from HBM): planes of 2 B a weight against Q4_K codes of 0.63 B: gate | up at 130, 256
+// and 512 tokens 70 -> 49, 79 -> 61, 159 -> 153; Q5_K as 1.5 B (a byte and a nibble: 6 instructions a K-step; as codes of a byte, 17, eight layers of a 7B model at 512 tokens 3179 us, as planes 3035,
+// so 2956): experts of an 8x7B layer, 611 tokens, gate | up 544 -> 455.
+// Tried, and slower: two 128 x 128 workgroups per CU, each with planes of its own (192 KiB), by 4 %; 16 x 16 x 64 MFMA tiles, which read twice the registers per product, the same; touching the
+// super-block after the next one, to have it in the L2 (64 lines an instruction), 12 %; the DMA's requests spread over the K-steps, 3 %; workgroups that walk equal shares of 64-token
+// pairs, by 12 % at 512 tokens: the CUs that the second round leaves idle cost nothing while the others' bytes and power bound it.  One MFMA a group and the scale on its sixteen results: a fifth more.
 // The block-sum ("mins") term is one v_mfma_f32_32x32x16_f16 per tile: the 16 block sums (|.| <= 2032) and the 6-bit mins are exact in f16 and their 16 products sum to
 // < 2^24, so the f32 result IS the integer msum.  The integer sums, the fold and the f32 order over super-blocks are those of mmq_planes_kernel: results are bit-identical.
 __device__ __forceinline__ unsigned lds_addr32(const void *p) { return (unsigned)(uintptr_t)p; }
@@ -1077,23 +1132,27 @@ __device__ __forceinline__ gbytes *scalar_ptr(const void *p) {
     return (gbytes *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
 // NT: token tiles of 32; FULL: every token of the workgroup's tile exists
-template <bool MINS, int NT, bool FULL>
+template <int FORM, int NT, bool FULL>
 __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int sb_lo, int nb, int tok0, int tid, int tw, uint8_t *smem_wg, float (&facc)[4][16]) {
-    constexpr int SH = MINS ? 5 : 6;
+    constexpr bool MINS = FORM != PF_SIGNED, PACKED = FORM >= PF_CODES;
+    constexpr int SH = plane_shift(FORM), BLOCK = plane_block(FORM), WORDS = plane_words(FORM);
     // (a half's four waves stage their own tokens: `wave` is the wave's index in its half)
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
     const int n = lane & 31, kg = lane >> 5;
     const int nb_all = a.K >> 8;
-    const uint8_t *sm_bs = smem_wg + P2_BS + tw * 4096, *sm_meta = smem_wg + P2_META + tw * 2048, *sm_yd = smem_wg + P2_YD + tw * P2_YDB, *sm_a = smem_wg + tw * 32768;
+    const uint8_t *sm_bs = smem_wg + P2_BS + tw * 4096, *sm_meta = smem_wg + P2_META, *sm_yd = smem_wg + P2_YD + tw * P2_YDB, *sm_a = smem_wg + tw * 32768;
     const unsigned lds0 = lds_addr32(smem_wg);
     const int last = a.T - 1 - tok0;                            // (tokens past the end read the last one; never stored)
     auto dma = [&](int sb, int buf, int y3) {                   // tokens 32 wave .. + 31 of super-block sb, and the scale words of the wave's rows
         const unsigned dst = lds0 + (unsigned)buf * P2_BUF;
-        const uint8_t *mw = (const uint8_t *)scalar_ptr((const uint8_t *)blk0 + (size_t)sb * PL_BLOCK + 16384);
         int l = lane;
         asm volatile("" : "+v"(l));                             // (the offsets are formed here, every time: hoisted out of the loop they would cost ten registers)
-        dma4_s(mw, l * 4u, dst + P2_META + (unsigned)(tw * 2048 + wave * 512));
-        dma4_s(mw + 256, l * 4u, dst + P2_META + (unsigned)(tw * 2048 + wave * 512 + 256));
+        if (tw == 0) {                                          // (both halves' rows are the same)
+            const uint8_t *mw = (const uint8_t *)scalar_ptr((const uint8_t *)blk0 + (size_t)sb * BLOCK + WORDS);
+            const unsigned to = dst + P2_META + (unsigned)wave * 1024u;
+            if (FORM == PF_CODES) dma16_s(mw, l * 16u, to);
+            else { dma4_s(mw, l * 4u, to + 512u); dma4_s(mw + 256, l * 4u, to + 768u); }
+        }
         const size_t sbg = (size_t)(sb_lo + sb);
         if (NT == 4 || wave < NT) {
             const int q4 = l >> 4, p16 = l & 15;
@@ -1128,19 +1187,28 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
     };
     const unsigned b_off = (unsigned)lane * 16u;
     i32x4 B[8][2];                                              // [K-step][plane]
+    u32x4 raw[4];                                               // codes, nibbles: as they are, of K-steps 2 c and 2 c + 1
     dma(0, 0, 0);
+    typedef const __attribute__((address_space(1))) i32x4 g_i32x4;
     auto ld_b = [&](gbytes *blk, int j) {
-        gbytes *q = blk + j * 2048;
-        asm("" : "+s"(q));
-#pragma unroll
-        for (int p = 0; p < 2; p++) B[j][p] = *(const __attribute__((address_space(1))) i32x4 *)(q + b_off + p * 1024);
+        if (FORM != PF_CODES) {
+            gbytes *q = blk + (FORM == PF_NIBBLES ? j : 2 * j) * 1024;
+            asm("" : "+s"(q));
+            if (!PACKED) B[j][0] = *(g_i32x4 *)(q + b_off);
+            B[j][1] = *(g_i32x4 *)(q + b_off + (PACKED ? 0 : 1024));
+        }
+        if (PACKED && (j & 1)) {
+            gbytes *q = blk + (FORM == PF_CODES ? j >> 1 : 8 + (j >> 1)) * 1024;
+            asm("" : "+s"(q));
+            raw[j >> 1] = __builtin_bit_cast(u32x4, *(g_i32x4 *)(q + b_off));
+        }
     };
 #pragma unroll
     for (int j = 0; j < 8; j++) { ld_b(blk0, j); __builtin_amdgcn_sched_barrier(0); }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     convert(0);
     __syncthreads();
-    const bool nib = MINS && __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(sm_meta + 12));       // Q2_K planes: sixteen 4-bit mins
+    const bool nib = FORM == PF_MINS && __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(sm_meta + 512 + 12));       // Q2_K planes: sixteen 4-bit mins
 
     i32x16 H[2], L[2];                                          // [tile parity]
     f32x16 ms;
@@ -1170,20 +1238,26 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
     for (int sb = 0; sb < nb; sb++) {
         const int sbuf = (sb & 1) * P2_BUF;
         const int nxt = sb + 1 < nb ? sb + 1 : sb, y3n = y3 == 2 ? 0 : y3 + 1;
-        gbytes *blkn = blk0 + (size_t)nxt * PL_BLOCK;
+        gbytes *blkn = blk0 + (size_t)nxt * BLOCK;
         const uint8_t *ys = sm_yd + y3 * 2 * P2_YDB + 16 * kg;
         unsigned x = (unsigned)(n * 256 + ((kg ^ (n & 15)) * 16));
         asm volatile("" : "+v"(x));
         auto ld_a = [&](int t, int j) { return *reinterpret_cast<const i32x4 *>(sm_a + sbuf + t * 8192 + (x ^ (unsigned)(32 * j))); };
         i32x4 A[2];
-        u32x4 meta = *reinterpret_cast<const u32x4 *>(sm_meta + sbuf + wave * 512 + n * 16);
+        u32x4 meta = *reinterpret_cast<const u32x4 *>(sm_meta + sbuf + wave * 1024 + 512 + n * 16);
         A[0] = ld_a(0, 0); A[1] = ld_a(0, 1);
+        uint32_t sw = 0;
+        auto scales = [&](int c) { if (FORM == PF_CODES) sw = *reinterpret_cast<const uint32_t *>(sm_meta + sbuf + wave * 1024 + n * 16 + c * 4); };
+        auto expand = [&](auto J) { constexpr int j = J.value; if constexpr (PACKED) expand_words<FORM, j>(raw[j >> 1], sw, B[j][0], B[j][1]); };
+        scales(0);
         __builtin_amdgcn_sched_barrier(0);
         if (sb) {                                               // the last tile of the super-block before, while the operands come
             mins();
 #pragma unroll
             for (int p = 0; p < 8; p++) fold(NT - 1, (NT - 1) & 1, p, yprev);
         }
+        expand(std::integral_constant<int, 0>()); expand(std::integral_constant<int, 1>());
+        scales(1);
         dd = h2f((uint16_t)(meta.x & 0xffff));
         asm("" : "+v"(dd));                                  // (as f32: folded into v_fma_mix_f32 it costs twice the issue slots)
         if (MINS) {
@@ -1222,6 +1296,17 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
                 if (j < 6) A[j & 1] = ld_a(t, j + 2);
                 else if (t + 1 < NT) A[j & 1] = ld_a(t + 1, j - 6);
                 if (MINS && j == 4) as = *reinterpret_cast<const f16x8 *>(sm_bs + sbuf + (32 * t + n) * 32 + kg * 16);
+                if (PACKED && t == 0) {                         // two K-steps ahead
+                    switch (j) {
+                        case 0: expand(std::integral_constant<int, 2>()); break;
+                        case 1: expand(std::integral_constant<int, 3>()); scales(2); break;
+                        case 2: expand(std::integral_constant<int, 4>()); break;
+                        case 3: expand(std::integral_constant<int, 5>()); scales(3); break;
+                        case 4: expand(std::integral_constant<int, 6>()); break;
+                        case 5: expand(std::integral_constant<int, 7>()); break;
+                        default: break;
+                    }
+                }
                 if (t == NT - 1) ld_b(blkn, j);
                 if (t > 0) fold(t - 1, pr ^ 1, j, ys + (t - 1) * 128);
                 if (j == 7) yd = *reinterpret_cast<const f32x4 *>(ys + t * 128);
@@ -1240,7 +1325,7 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
 // SWIGLU: `planes` = ffn_gate, `planes_up` = ffn_up (n_rows rows each, same type): a workgroup takes 64 rows of BOTH (row-waves 0, 1 the
 // gate rows, 2, 3 the same rows of up), the two waves of the same rows swap halves of their tiles through LDS at the end and store
 // silu(gate . x) * (up . x) - one [T][n_rows] f32 result instead of two, and no separate SwiGLU pass over them
-template <bool MINS, bool SWIGLU>
+template <int FORM, bool SWIGLU>
 __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &po, int row_tile, int tok_tile, int n_tok_tiles, int zz) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1257,13 +1342,13 @@ __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &p
     const int units = (T + 31) >> 5, per = (units + n_tok_tiles - 1) / n_tok_tiles, mine_u = units - tok_tile * per < per ? units - tok_tile * per : per;
     const int nt = mine_u <= 0 ? 0 : tw ? mine_u >> 1 : (mine_u + 1) >> 1;
     const int row0 = rt32 * 32, tok0 = (tok_tile * per + (tw ? (mine_u + 1) >> 1 : 0)) * 32, n = lane & 31, kg = lane >> 5, row = row0 + n;
-    gbytes *blk0 = scalar_ptr(base + ((size_t)(tile_ok ? rt32 : n_rt32 - 1) * nb_all + sb_lo) * PL_BLOCK);
+    gbytes *blk0 = scalar_ptr(base + ((size_t)(tile_ok ? rt32 : n_rt32 - 1) * nb_all + sb_lo) * plane_block(FORM));
     float facc[4][16];
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) facc[t][r] = 0.0f;
-#define P2_LOOP(NTV, FULLV) planes2_loop<MINS, NTV, FULLV>(blk0, a, sb_lo, nb, tok0, tid, tw, smem, facc)
+#define P2_LOOP(NTV, FULLV) planes2_loop<FORM, NTV, FULLV>(blk0, a, sb_lo, nb, tok0, tid, tw, smem, facc)
     if (nt == 4 && T - tok0 >= 128) P2_LOOP(4, true);
     else if (nt == 4) P2_LOOP(4, false);
     else if (nt == 3) P2_LOOP(3, false);
@@ -1330,9 +1415,9 @@ __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &p
     if (all) store(true); else store(false);
 }
 
-// MODE 0: Q6_K planes (signed codes, no block-sum term); 1: Q4_K / Q5_K; 2: per segment (po.mins_mask; segment boundaries at multiples of
-// 128 rows, so a workgroup's row tile is of one kind) - Q | K | V of the layers whose attn_v is Q6_K, in one launch.  MODE 2 carries both
-// bodies behind one workgroup-uniform branch (a run-time flag inside ONE body costs 92 bytes of scratch per lane and 2.3x the time).
+// MODE < 4: that PlaneForm; otherwise per segment (po.form; segment boundaries at multiples of 128 rows, so a workgroup's row tile is of one kind), of the forms in MODE >> 4 - Q | K | V of
+// the layers whose attn_v is Q6_K, in one launch.  The bodies lie behind workgroup-uniform branches (a run-time flag inside ONE body costs 92 bytes of scratch per lane and 2.3x the time).
+constexpr int P2_MIXED = 4, P2_MIXED_PACKED = P2_MIXED | (1 << PF_CODES | 1 << PF_NIBBLES | 1 << PF_SIGNED) << 4, P2_MIXED_PLANES = P2_MIXED | (1 << PF_MINS | 1 << PF_SIGNED) << 4;
 template <int MODE>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *planes, int n_rows, int K, int T, int n_row_tiles, int n_tok_tiles,
                                                                const int8_t *aq, const float *ad, const int16_t *absum,
@@ -1342,20 +1427,23 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *pl
     const int zz = (loc / n_tok_tiles) % n_split;              // K split: partial sums go to ws[zz], mmq_splitk_reduce_kernel adds them up
     const int row_tile = (loc / (n_tok_tiles * n_split)) * 8 + xcd;
     if (row_tile >= n_row_tiles) return;                       // workgroup-uniform
-    bool mins = MODE == 1;
-    if (MODE == 2) {
-        int sg0 = 0;
-        if (po.n_seg > 1 && row_tile * P2_ROWS >= po.row_end[0]) sg0 = 1;
-        if (po.n_seg > 2 && row_tile * P2_ROWS >= po.row_end[1]) sg0 = 2;
-        mins = (po.mins_mask >> sg0) & 1u;
+    P2Args a{planes, nullptr, n_rows, K, T, aq, ad, absum, resid, ws, n_split};
+    if constexpr (MODE < P2_MIXED) planes2_body<MODE, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
+    else {
+        int sg = 0;
+        if (po.n_seg > 1 && row_tile * P2_ROWS >= po.row_end[0]) sg = 1;
+        if (po.n_seg > 2 && row_tile * P2_ROWS >= po.row_end[1]) sg = 2;
+        // where block 0 of the launch would lie if all were of this segment's form
+        const int form = __builtin_amdgcn_readfirstlane(po.form[sg]);
+        a.planes = planes + po.at[sg] - (size_t)(sg ? po.row_end[sg - 1] >> 5 : 0) * (size_t)(K >> 8) * plane_block(form);
+#define P2_FORM(F) if constexpr (((MODE >> 4) >> F) & 1) if (form == F) planes2_body<F, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz)
+        P2_FORM(PF_SIGNED); P2_FORM(PF_MINS); P2_FORM(PF_CODES); P2_FORM(PF_NIBBLES);
+#undef P2_FORM
     }
-    const P2Args a{planes, nullptr, n_rows, K, T, aq, ad, absum, resid, ws, n_split};
-    if (MODE == 1 || (MODE == 2 && mins)) planes2_body<true, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
-    else planes2_body<false, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
 }
 
 // ffn_gate and ffn_up with SwiGLU in the epilogue: n_rows rows of each, 64 per workgroup, out[t][row] = silu(gate) * up
-template <bool MINS>
+template <int FORM>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_kernel(const uint8_t *planes_gate, const uint8_t *planes_up, int n_rows, int K, int T,
                                                                       int n_row_tiles, int n_tok_tiles, const int8_t *aq, const float *ad,
                                                                       const int16_t *absum, const PlanesOut po) {
@@ -1363,7 +1451,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_kernel(const uint
     const int tok_tile = loc % n_tok_tiles;
     const int row_tile = (loc / n_tok_tiles) * 8 + xcd;
     if (row_tile >= n_row_tiles) return;                       // workgroup-uniform
-    planes2_body<MINS, true>(P2Args{planes_gate, planes_up, n_rows, K, T, aq, ad, absum, nullptr, nullptr, 1}, po, row_tile, tok_tile, n_tok_tiles, 0);
+    planes2_body<FORM, true>(P2Args{planes_gate, planes_up, n_rows, K, T, aq, ad, absum, nullptr, nullptr, 1}, po, row_tile, tok_tile, n_tok_tiles, 0);
 }
 
 // ---- ggml_mul_mat_id on a prompt batch as ONE launch per projection.  The (token, rank) pairs of the batch are sorted by expert (moe_group_kernel: expert
@@ -1381,7 +1469,7 @@ __device__ __forceinline__ bool moe_tile_of(const MoeTiles &m, int j, int &e_out
     }
     return false;
 }
-template <bool MINS>
+template <int FORM>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_moe_kernel(const uint8_t *planes_gate, const uint8_t *planes_up, int n_rows, int K, int n_row_tiles,
                                                                           int n_tile_slots, const int8_t *aq, const float *ad, const int16_t *absum, PlanesOut po,
                                                                           const MoeTiles mt) {
@@ -1393,10 +1481,10 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_moe_kernel(const 
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
     po.out[0] += (size_t)r0 * po.ld[0];
-    planes2_body<MINS, true>(P2Args{planes_gate + (size_t)e * mt.plane_stride, planes_up + (size_t)e * mt.plane_stride, n_rows, K, n_e,
+    planes2_body<FORM, true>(P2Args{planes_gate + (size_t)e * mt.plane_stride, planes_up + (size_t)e * mt.plane_stride, n_rows, K, n_e,
                                     aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
-template <bool MINS>
+template <int FORM>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t *planes, int n_rows, int K, int n_row_tiles, int n_tile_slots,
                                                                    const int8_t *aq, const float *ad, const int16_t *absum, PlanesOut po, const MoeTiles mt) {
     const int bid = blockIdx.x, xcd = bid & 7, loc = bid >> 3;
@@ -1407,7 +1495,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
     po.out[0] += (size_t)r0 * po.ld[0];
-    planes2_body<MINS, false>(P2Args{planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e,
+    planes2_body<FORM, false>(P2Args{planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e,
                                      aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 
@@ -1562,16 +1650,18 @@ hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, 
 
 size_t mmq_planes_bytes(int type, int64_t n_rows, int K) {
     if ((type != T_Q4_K && type != T_Q5_K && type != T_Q6_K && type != T_Q2_K && type != T_Q3_K) || (K % 256) != 0) return 0;
-    return (size_t)((n_rows + 31) / 32) * (size_t)(K >> 8) * PL_BLOCK;
+    return (size_t)((n_rows + 31) / 32) * (size_t)(K >> 8) * plane_block(plane_form(type));
 }
+
+bool mmq_planes_same_form(int type_a, int type_b) { return plane_form(type_a) == plane_form(type_b); }
 
 hipError_t launch_mmq_expand(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, uint8_t *planes, hipStream_t st) {
     const int nb = K >> 8, n_rt = (n_rows + 31) / 32;
     const dim3 grid((unsigned)((n_rt * nb + 3) / 4));
     switch (type) {
-        case T_Q4_K: hipLaunchKernelGGL(mmq_expand_kernel<T_Q4_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
-        case T_Q5_K: hipLaunchKernelGGL(mmq_expand_kernel<T_Q5_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
-        case T_Q6_K: hipLaunchKernelGGL(mmq_expand_kernel<T_Q6_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
+        case T_Q4_K: hipLaunchKernelGGL(mmq_pack_kernel<T_Q4_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
+        case T_Q5_K: hipLaunchKernelGGL(mmq_pack_kernel<T_Q5_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
+        case T_Q6_K: hipLaunchKernelGGL(mmq_expand_kernel, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
         case T_Q2_K: hipLaunchKernelGGL(mmq_expand_small_kernel<T_Q2_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
         case T_Q3_K: hipLaunchKernelGGL(mmq_expand_small_kernel<T_Q3_K>, grid, dim3(256), 0, st, W, row_bytes, n_rows, nb, n_rt, planes); break;
         default: return hipErrorInvalidValue;
@@ -1633,13 +1723,15 @@ hipError_t launch_mmq_planes_swiglu(int type, const uint8_t *planes_gate, const 
     po.n_seg = 1; po.out[0] = out; po.ld[0] = ld_out; po.row_end[0] = n_rows;
     const int nrt = (n_rows + 63) / 64, ntt = (T + P2_TOK - 1) / P2_TOK;
     const dim3 grid((unsigned)(((nrt + 7) / 8) * ntt * 8));
-    if (planes_have_mins(type)) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_swiglu_kernel<true>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po);
-    } else {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_swiglu_kernel<false>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po);
+#define GO(F) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_kernel<F>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
+                hipLaunchKernelGGL((mmq_planes2_swiglu_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po); }
+    switch (plane_form(type)) {
+        case PF_CODES: GO(PF_CODES) break;
+        case PF_NIBBLES: GO(PF_NIBBLES) break;
+        case PF_MINS: GO(PF_MINS) break;
+        default: GO(PF_SIGNED) break;
     }
+#undef GO
     return hipGetLastError();
 }
 
@@ -1656,13 +1748,14 @@ hipError_t launch_mmq_planes_swiglu_moe(int type, const uint8_t *planes_gate, co
     const int nrt = (n_rows + 63) / 64, slots = (rows_max + P2_TOK - 1) / P2_TOK + n_expert;     // every expert may end in a partial tile
     const dim3 grid((unsigned)(((nrt + 7) / 8) * slots * 8));
     const MoeTiles mt{meta, n_expert, plane_stride};
-    if (planes_have_mins(type)) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_moe_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_swiglu_moe_kernel<true>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt);
-    } else {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_moe_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_swiglu_moe_kernel<false>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt);
+#define GO(F) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_moe_kernel<F>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
+                hipLaunchKernelGGL((mmq_planes2_swiglu_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt); }
+    switch (plane_form(type)) {
+        case PF_CODES: GO(PF_CODES) break;
+        case PF_NIBBLES: GO(PF_NIBBLES) break;
+        default: GO(PF_SIGNED) break;
     }
+#undef GO
     return hipGetLastError();
 }
 hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_stride, int n_expert, const int32_t *meta, int n_rows, int K, int rows_max,
@@ -1673,13 +1766,14 @@ hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_s
     const int nrt = (n_rows + P2_ROWS - 1) / P2_ROWS, slots = (rows_max + P2_TOK - 1) / P2_TOK + n_expert;
     const dim3 grid((unsigned)(((nrt + 7) / 8) * slots * 8));
     const MoeTiles mt{meta, n_expert, plane_stride};
-    if (planes_have_mins(type)) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_moe_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_moe_kernel<true>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt);
-    } else {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_moe_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-        hipLaunchKernelGGL((mmq_planes2_moe_kernel<false>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt);
+#define GO(F) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_moe_kernel<F>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
+                hipLaunchKernelGGL((mmq_planes2_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt); }
+    switch (plane_form(type)) {
+        case PF_CODES: GO(PF_CODES) break;
+        case PF_NIBBLES: GO(PF_NIBBLES) break;
+        default: GO(PF_SIGNED) break;
     }
+#undef GO
     return hipGetLastError();
 }
 
@@ -1690,15 +1784,21 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     PlanesOut po{};
     po.n_seg = n_seg;
     int n_rows = 0;
-    bool mixed = false;
+    bool mixed = false, packed = false, mins = false;
+    size_t at = 0;
     for (int i = 0; i < n_seg; i++) {
         if (i + 1 < n_seg && (seg_rows[i] % 32) != 0) return hipErrorInvalidValue;
         n_rows += seg_rows[i];
         po.out[i] = outs[i]; po.ld[i] = lds_out[i]; po.row_end[i] = n_rows;
         const int ti = seg_types ? seg_types[i] : type;
-        if (planes_have_mins(ti)) po.mins_mask |= 1u << i;
-        mixed = mixed || planes_have_mins(ti) != planes_have_mins(type);
+        po.form[i] = plane_form(ti);
+        po.at[i] = at;
+        at += (mmq_planes_bytes(ti, seg_rows[i], K) + 255) & ~(size_t)255;
+        mixed = mixed || po.form[i] != plane_form(type);
+        packed = packed || po.form[i] >= PF_CODES;
+        mins = mins || po.form[i] == PF_MINS;
     }
+    if (mixed && packed && mins) return hipErrorInvalidValue;   // (no launch has both bodies)
     if (mixed && !mmq_planes_mixed_ok(seg_rows, n_seg, K, T, wsp)) return hipErrorInvalidValue;
     static const int env_mt = getenv("MI355_MMQ_MT") ? atoi(getenv("MI355_MMQ_MT")) : 0;
     // 128 x 128 workgroup tiles (two token tiles per wave) when that still yields ~2 workgroups per CU, else 256 x 32
@@ -1709,7 +1809,6 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     if (n_seg > 1 && T > 32 && wg2 * 4 >= 3L * num_cu()) mt = 2;       // concatenated Q | K | V: 192 workgroups of 128 x 128 beat 384 of 256 x 32 (59 vs 71 us)
     if (env_mt == 1 || env_mt == 2) mt = env_mt;
     if (g_mmq_mt == 1 || g_mmq_mt == 2) mt = g_mmq_mt;
-    const bool mins = planes_have_mins(type);
     // 128 rows x 256 tokens per workgroup from 129 tokens on; tensors with too few rows to cover the chip that way split K over 2..4 workgroups (partial sums in
     // the caller's workspace, added up pairwise)
     bool p2 = false;
@@ -1717,16 +1816,17 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     if (p2) {
         const int nrt = (n_rows + P2_ROWS - 1) / P2_ROWS, ntt = (T + P2_TOK - 1) / P2_TOK;
         const dim3 grid((unsigned)(((nrt + 7) / 8) * ntt * n_split * 8));
-        if (mixed) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-            hipLaunchKernelGGL((mmq_planes2_kernel<2>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split);
-        } else if (mins) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-            hipLaunchKernelGGL((mmq_planes2_kernel<true>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split);
-        } else {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS);
-            hipLaunchKernelGGL((mmq_planes2_kernel<false>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split);
+#define GO(M) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<M>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
+                hipLaunchKernelGGL((mmq_planes2_kernel<M>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split); }
+        if (mixed && packed) GO(P2_MIXED_PACKED)
+        else if (mixed) GO(P2_MIXED_PLANES)
+        else switch (plane_form(type)) {
+            case PF_CODES: GO(PF_CODES) break;
+            case PF_NIBBLES: GO(PF_NIBBLES) break;
+            case PF_MINS: GO(PF_MINS) break;
+            default: GO(PF_SIGNED) break;
         }
+#undef GO
         if (n_split > 1 && parts) *parts = n_split;
         else if (n_split > 1) {
             const size_t n4 = (size_t)T * (n_rows >> 2);
@@ -1734,18 +1834,22 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
         }
         return hipGetLastError();
     }
-#define PLN(MINSV, MTV)                                                                                                   \
+#define PLN(FORMV, MTV)                                                                                                   \
     {                                                                                                                     \
         using G = Geo<MTV>;                                                                                               \
         const int nrt = (n_rows + G::ROW_TILE - 1) / G::ROW_TILE, ntt = (T + G::TOK_TILE - 1) / G::TOK_TILE;              \
         const dim3 grid((unsigned)(((nrt + 7) / 8) * ntt * 8));                                                           \
         const size_t lds2 = 2 * (size_t)G::LDS_BYTES;                                                                     \
-        if (lds2 > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes_kernel<MINSV, MTV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2); \
-        hipLaunchKernelGGL((mmq_planes_kernel<MINSV, MTV>), grid, dim3(NTHREADS), lds2, st, planes, n_rows, K, T, nrt, ntt, \
+        if (lds2 > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes_kernel<FORMV, MTV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2); \
+        hipLaunchKernelGGL((mmq_planes_kernel<FORMV, MTV>), grid, dim3(NTHREADS), lds2, st, planes, n_rows, K, T, nrt, ntt, \
                            q.qs, q.d, bh, bl, po, resid);                                                                 \
     }
-    if (mins) { if (mt == 1) PLN(true, 1) else PLN(true, 2) }
-    else { if (mt == 1) PLN(false, 1) else PLN(false, 2) }
+    switch (plane_form(type)) {
+        case PF_CODES: if (mt == 1) PLN(PF_CODES, 1) else PLN(PF_CODES, 2) break;
+        case PF_NIBBLES: if (mt == 1) PLN(PF_NIBBLES, 1) else PLN(PF_NIBBLES, 2) break;
+        case PF_MINS: if (mt == 1) PLN(PF_MINS, 1) else PLN(PF_MINS, 2) break;
+        default: if (mt == 1) PLN(PF_SIGNED, 1) else PLN(PF_SIGNED, 2) break;
+    }
 #undef PLN
     return hipGetLastError();
 }

@@ -385,8 +385,8 @@ Model *model_load(const std::string &path, int main_gpu, std::string &err, int &
     m->device_bytes = total;
     m->host_bytes = 0;
 
-    // prompt-processing copy of the per-layer projection weights: both int8 MFMA operand planes of every K-step,
-    // expanded once here (2 B per weight) so that the prefill kernel spends nothing per weight (mmq.hip).  288 GB of HBM
+    // prompt-processing copy of the per-layer projection weights: the MFMA operand planes of every K-step, laid out once here
+    // (2 B per weight; Q4_K 0.6 as codes and Q5_K 1.6, of which the kernel makes the planes: mmq.hip).  288 GB of HBM
     // is what makes this the default; it is skipped (the prefill kernel then expands on the fly) when memory is short.
     if (const char *e = getenv("MI355_PREFILL_PLANES")) prefill_planes = atoi(e);
     if (prefill_planes != 0) {
@@ -1048,12 +1048,11 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     if (all_mmq && pending_fuse_.mode == 0) {
         HIP_TRY(ensure_prep(aq, K, T));
         // Q | K | V (or Q | K) as one launch over the concatenated rows where their plane sets are adjacent in the arena and
-        // of one plane format (Q4_K and Q5_K share it; the Q6_K attn_v of the "more bits" layers runs on its own)
-        auto mins = [](int t) { return t != T_Q6_K; };
+        // of one plane format (the Q6_K attn_v of the "more bits" layers runs on its own)
         auto adjacent = [&](int i) { return ws[i]->planes && ws[i - 1]->planes && ws[i]->planes == ws[i - 1]->planes + ws[i - 1]->planes_bytes &&
                                             (ws[i - 1]->N % 32) == 0 && ws[i]->n_expert == 1; };
         int nf = 1;
-        while (nf < n && nf < 3 && adjacent(nf) && mins(ws[nf]->type) == mins(ws[0]->type)) nf++;
+        while (nf < n && nf < 3 && adjacent(nf) && mmq_planes_same_form(ws[nf]->type, ws[0]->type)) nf++;
         // the "more bits" layers (Q6_K attn_v beside Q4_K / Q5_K attn_q, attn_k): still one launch where the 128 x 256 kernel takes it
         int nm = nf;
         while (nm < n && nm < 3 && adjacent(nm)) nm++;

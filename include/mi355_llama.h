@@ -68,7 +68,7 @@ typedef struct mi355_model_params {
     /* row split over RCCL (see mi355_tp_init below; new keys proposed in SURVEY.md §2b) */
     int32_t tp_rank;        /* 0 when tp_size <= 1 */
     int32_t tp_size;        /* 1 = whole model on this GPU */
-    /* prompt-processing copy of the projection weights as pre-expanded int8 MFMA operand planes (2 B / weight):
+    /* prompt-processing copy of the projection weights as pre-expanded int8 MFMA operand planes (up to 2 B / weight):
      * -1 = keep it when device memory allows (default), 0 = never (expand on the fly), 1 = required */
     int32_t prefill_planes;
 } mi355_model_params;
