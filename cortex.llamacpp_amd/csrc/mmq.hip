@@ -1582,37 +1582,29 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
 }
 
 static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool *takes);
-// Which kernel takes a launch of 65 .. 256 tokens is a matter of shape (tools/exp_planes_shapes.py, Q5_K, us per launch; to 64 tokens mmq_few_takes chooses):
-//     N x K          T = 48     64     96    128    160    192    256
-//   14336 x 4096   K-split 29     30     56     58     83     86    103      planes 256x32: 34 34 35 37 67 68 70   128x128: 55 56 56 57 60 60 61
-//    4096 x 14336  K-split 38     39     41     43     77     80     83      planes 256x32: 99 .. 102              128x128: 166 .. 172
-// a tensor of >= 8192 rows has enough 256-row tiles for the planes kernels to fill the chip from 65 tokens on (56 x 3 workgroups) and
-// they read pre-expanded operands; a tensor of 4096 rows does not, and the K-split kernel's waves share its long K instead.
-// (pair: gate | up of a dense layer go out as ONE K-split launch of 2 n_rows rows, which holds its own against two planes launches up to
-// 128 tokens: whole 8B prompt 8.8 vs 9.0 ms at 100 tokens, 9.0 vs 9.2 at 128)
-// From 129 tokens on the other side is the 128 x 256 tiles, K split over the workgroups where the workspace allows it, and the choice is by the two launches' times.  Both are
-// whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us, Q4_K; Q6_K costs the K-split kernel up to a quarter more): K-split, 32 rows x 64 tokens,
-// a wave's ceil(nb / 8) super-blocks of 4.3 and 3.5; tiles, the part's super-blocks of 3.0 (to 160 tokens) or 3.8 and 9, and 4 more where the parts' sum is a launch of its own.
-// Measured, K-split against tiles (with the sum's launch) at 130 and 256 tokens:
-//   2048 x 2048   9 / 18, 10 / 22      2048 x 5632  18 / 28, 20 / 34      1536 x 8960  24 / 36, 25 / 47      gate | up of 5632 x 2048  36 / 32, 45 / 38
-//   3072 x 3072  17 / 23, 19 / 27      3072 x 8192  39 / 35, 44 / 44      5120 x 5120  28 / 29, 42 / 35      gate | up of 8192 x 3072  55 / 46, 74 / 54
-//   4096 x 4096  23 / 24, 26 / 29      6144 x 4096  34 / 27, 37 / 33      4096 x 14336 64 / 54, 73 / 69      gate | up of 14336 x 4096 129 / 67, 172 / 79
-// Whole prompts of 130, 160 and 256 tokens: the 22 layers of a 2048-column model 2.68, 2.76, 3.20 ms with every tensor here, 3.20, 3.30, 3.75 with every tensor on tiles; eight
-// layers of an 8B model 2.75 (140 tokens), 2.81, 3.32 and 1.95, 2.00, 2.36.
+// Which kernel takes a launch of 65 .. 256 tokens is a matter of shape (to 64 tokens mmq_few_takes chooses): this one, or the 128 x 256 tiles, K split over the workgroups where the
+// workspace allows it.  The choice is by the two launches' times.  Both are whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us): K-split, 32 rows x 64
+// tokens, an eighth of the super-blocks of 5.2 and 3.5; tiles, the part's super-blocks of 1.5 + T / 128 and 7, and 4 more where the parts' sum is a launch of its own.
+// Measured with weights from HBM, Q4_K, K-split / tiles without the sum's launch, at 72, 128 and 256 tokens (Q5_K and Q6_K cost either kernel a tenth more):
+//   2048 x 2048   9/13 9/15 10/18     2048 x 5632  18/18 19/20 20/24    1536 x 8960   23/23 27/27 26/34     gate | up of 5632 x 2048    25/24 25/27 44/32
+//   3072 x 3072  11/14 12/16 19/19    3072 x 8192  24/22 24/25 43/31    5120 x 5120   28/17 28/19 42/24     gate | up of 8192 x 3072    40/32 41/37 74/44
+//   4096 x 4096  15/15 15/16 26/20    6144 x 4096  25/15 25/17 37/21    4096 x 14336  40/35 40/40 72/50     gate | up of 14336 x 4096   89/43 91/49 166/61
+// (tiles of planes, before Q4_K came as codes: gate | up of 14336 x 4096 at 130 tokens 70, 6144 x 4096 25.)  Whole prompts of eight layers of an 8B model, us, K-split to 128 tokens and now:
+// 65 tokens 1624, 1083; 96 1672, 1128; 128 1727, 1227.
 static bool tiles_beat_ksplit(int n_rows, int K, int T, MMQWorkspace wsp, bool pair, bool sum_free) {
     bool takes = false;
     const int rows = pair ? 2 * n_rows : n_rows, parts = planes2_split(rows, K, T, pair ? MMQWorkspace() : wsp, &takes), nb = K >> 8;
-    if (!takes) return n_rows >= 8192;                          // (then the planes kernel below: by rows, as under 129 tokens)
+    if (!takes) return n_rows >= 8192 && !(pair && T <= 128);  // (then the planes kernel below, by rows; ffn_gate | ffn_up are one launch here and two there)
     const auto up = [](long a, long b) { return (double)((a + b - 1) / b); };
-    const double here = up(up(rows, 32) * up(T, 64), num_cu()) * (4.3 * up(nb, 8) + 3.5);
-    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * ((T <= 160 ? 3.0 : 3.8) * up(nb, parts) + 9.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
+    const double here = up(up(rows, 32) * up(T, 64), num_cu()) * (5.2 * nb / 8 + 3.5);
+    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * ((1.5 + T / 128.0) * up(nb, parts) + 7.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
     return tiles < here;
 }
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair) {
     static const int env = getenv("MI355_KSPLIT_SHAPE") ? atoi(getenv("MI355_KSPLIT_SHAPE")) : 1;
     if (!mmq_ksplit_applicable(type, K, T)) return false;
     if (!env || !has_planes || !mmq_applicable(type, K, T)) return true;
-    return T > 128 ? !tiles_beat_ksplit(n_rows, K, T, wsp, pair, sum_free) : T <= 64 || pair || n_rows < 8192;
+    return T <= 64 || !tiles_beat_ksplit(n_rows, K, T, wsp, pair, sum_free);
 }
 
 // segs: up to 3 tensors sharing the activation; swiglu (to 32 tokens, or where mmq_few_takes): segs = {gate, up} of one type and shape, out = silu(gate.x) * (up.x) into segs[0].out
@@ -1692,7 +1684,7 @@ static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool
     n_split = std::min({n_split, nb, 4});                       // (the reductions add four parts at most)
     if (n_split < 1 || (n_rows % 4) != 0 || !wsp.p || (size_t)n_split * T * n_rows * sizeof(float) > wsp.bytes) n_split = 1;
     // (an unsplit launch wants a third of the CUs: 11264 x 2048 at 160 and 256 tokens - 88 workgroups - 35 and 40 us against 31 and 56, 4096 x 4096 at 300 - 64 - 53 against 47)
-    *takes = g_mmq_mt == 4 || (g_mmq_mt == 0 && env_mt == 0 && env_p2 != 0 && T > 128 && (n_split > 1 || wg * 3 >= num_cu()));
+    *takes = g_mmq_mt == 4 || (g_mmq_mt == 0 && env_mt == 0 && env_p2 != 0 && T > 64 && (n_split > 1 || wg * 3 >= num_cu()));
     return n_split;
 }
 

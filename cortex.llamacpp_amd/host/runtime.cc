@@ -1038,7 +1038,22 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
         all_planes &= ws[i]->planes != nullptr;
         all_rows += (int)ws[i]->N;
     }
-    if (T > 128) all_ks = all_ks && mmq_ksplit_preferred(ws[0]->type, all_rows, K, T, all_planes, mmq_ws_, parts != nullptr);   // (up to 128 tokens one K-split launch beats three of any kind)
+    // Q | K | V (or Q | K) as one launch over the concatenated rows where their plane sets are adjacent in the arena and
+    // of one plane format (the Q6_K attn_v of the "more bits" layers runs on its own)
+    auto adjacent = [&](int i) { return ws[i]->planes && ws[i - 1]->planes && ws[i]->planes == ws[i - 1]->planes + ws[i - 1]->planes_bytes &&
+                                        (ws[i - 1]->N % 32) == 0 && ws[i]->n_expert == 1; };
+    int nf = 1;
+    while (nf < n && nf < 3 && adjacent(nf) && mmq_planes_same_form(ws[nf]->type, ws[0]->type)) nf++;
+    // the "more bits" layers (Q6_K attn_v beside Q4_K / Q5_K attn_q, attn_k): still one launch where the 128 x 256 kernel takes it
+    int nm = nf;
+    while (nm < n && nm < 3 && adjacent(nm)) nm++;
+    if (nm > nf) {
+        int rows[3];
+        for (int i = 0; i < nm; i++) rows[i] = (int)ws[i]->N;
+        if (mmq_planes_mixed_ok(rows, nm, K, T, mmq_ws_)) nf = nm;
+    }
+    // (up to 128 tokens one K-split launch beats several of any kind)
+    if (T > (nf == n ? 64 : 128)) all_ks = all_ks && mmq_ksplit_preferred(ws[0]->type, all_rows, K, T, all_planes, mmq_ws_, parts != nullptr);
     if (all_ks && pending_fuse_.mode == 0 && n <= 3) {         // batched decode step: Q, K, V in one launch
         MMQSeg sg[3];
         for (int i = 0; i < n; i++) sg[i] = MMQSeg{ws[i]->data, ws[i]->row_bytes, (int)ws[i]->N, ws[i]->type, outs[i], (int)ws[i]->N, nullptr, 0};
@@ -1047,20 +1062,6 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     }
     if (all_mmq && pending_fuse_.mode == 0) {
         HIP_TRY(ensure_prep(aq, K, T));
-        // Q | K | V (or Q | K) as one launch over the concatenated rows where their plane sets are adjacent in the arena and
-        // of one plane format (the Q6_K attn_v of the "more bits" layers runs on its own)
-        auto adjacent = [&](int i) { return ws[i]->planes && ws[i - 1]->planes && ws[i]->planes == ws[i - 1]->planes + ws[i - 1]->planes_bytes &&
-                                            (ws[i - 1]->N % 32) == 0 && ws[i]->n_expert == 1; };
-        int nf = 1;
-        while (nf < n && nf < 3 && adjacent(nf) && mmq_planes_same_form(ws[nf]->type, ws[0]->type)) nf++;
-        // the "more bits" layers (Q6_K attn_v beside Q4_K / Q5_K attn_q, attn_k): still one launch where the 128 x 256 kernel takes it
-        int nm = nf;
-        while (nm < n && nm < 3 && adjacent(nm)) nm++;
-        if (nm > nf) {
-            int rows[3];
-            for (int i = 0; i < nm; i++) rows[i] = (int)ws[i]->N;
-            if (mmq_planes_mixed_ok(rows, nm, K, T, mmq_ws_)) nf = nm;
-        }
         if (nf >= 2) {
             int rows[3], ldo[3], types[3];
             float *o[3];

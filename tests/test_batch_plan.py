@@ -44,3 +44,16 @@ def test_to_64_tokens_by_shape(plan):
         assert [plan(t, 4096, 14336, T, 0, 0) for t in (Q4_K, Q5_K, Q6_K)] == [FEW, FEW, KSPLIT]
         assert [plan(Q4_K, r, c, T, 0, 0) for r, c in [(4096, 4096), (8192, 28672), (152064, 3584)]] == [KSPLIT] * 3
         assert [plan(t, 14336, 4096, T, 1, 0) for t in (Q4_K, Q5_K, Q6_K)] == [FEW, FEW, KSPLIT]
+
+
+@pytest.mark.parametrize("n", [65, 96, 128])
+def test_from_65_tokens_by_time(plan, n):
+    """The 128 x 256 tiles take what fills the chip, K split, from 65 tokens on: at these sizes measured at half to nine tenths of the K-split kernel's time."""
+    for t in (Q4_K, Q5_K, Q6_K):
+        for rows, cols in [(2048, 2048), (2560, 2048), (2048, 5632), (4096, 4096), (3072, 3072)]:
+            assert [plan(t, rows, cols, n, 0, s) for s in (0, 1)] == [KSPLIT] * 2, (rows, cols)
+        for rows, cols in [(6144, 4096), (12288, 4096), (5120, 5120), (8192, 8192)]:
+            assert [plan(t, rows, cols, n, 0, s) for s in (0, 1)] == [PLANES] * 2, (rows, cols)
+        for rows, cols in [(8192, 3072), (14336, 4096), (28672, 8192)]:
+            assert plan(t, rows, cols, n, 1, 0) == PLANES, (rows, cols)
+        assert plan(t, 1024, 2048, n, 1, 0) == KSPLIT
