@@ -5,16 +5,8 @@
 // exactly ggml_vec_dot_q8_0_q8_0: integer block sums, one f32 multiply-add per block, blocks added in order — so unlike
 // the K-quant kernels (whose super-block sums are re-associated) this one reproduces the CPU result bit for bit.
 //
-// v_mfma_i32_32x32x32_i8 contracts K = 32 per instruction = one Q8_0 block: A = 32 tokens x 32 codes (lane = token
-// lane & 31, k-half lane >> 5, 16 bytes straight from the activation plane), B = 32 weight rows x 32 codes (lane = row,
-// k-half; 16 bytes straight from the device row [codes K][scales K/32]).  The result tile holds 16 tokens of one weight
-// row per lane, so d_w is a per-lane scalar and the 16 activation scales of the block come from LDS (staged once per
-// workgroup as f32, [block][token]: four broadcast ds_read_b128 per block).  Every block costs one MFMA (32 cycles) and
-// 16 x (convert, scale product, multiply-add): the fold is the bound (VALU), ~1/8 of the int8 matrix peak — against one
-// pass over the weights per 16 tokens with the tiled mat-vec this replaces for T >= 32.
-// Workgroup = 4 waves = 128 weight rows x 32 tokens; the four waves share the token tile (L1 hits on the activations).
-#include <type_traits>
-
+// An MFMA contracts K = 32 = one Q8_0 block (v_mfma_i32_32x32x32_i8 or 16x16x32): A = tokens x 32 codes, B = weight rows x
+// 32 codes, so the result tile holds some tokens of one weight row per lane.
 #include "kernels.h"
 #include "quant_dev.h"
 
@@ -25,135 +17,172 @@ namespace {
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int Q80_UNROLL = 4;
+// up to three tensors of K columns that share the activations, one launch: tensor i is the workgroups from tile0[i] on
+struct Q80Args {
+    const uint8_t *W[3]; size_t row_bytes;
+    float *out[3];
+    int n_rows[3], ld_out[3], tile0[3];
+    int n_seg, K, T;
+    const int8_t *aq; const uint16_t *ad; const float *resid;
+};
 
-// MT token tiles of 32 per wave: a workgroup covers 128 weight rows x 32 MT tokens, so every weight byte is fetched T / (32 MT) times instead of T / 32
-// (with MT = 1 an 8B-shaped prompt is bound by those re-reads out of L2: 8.5k tok/s).  The activation scales are staged per chunk of Q80_KC blocks.
-constexpr int Q80_KC = 64;
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <int SZ> struct Tile;
+template <> struct Tile<32> {
+    using Codes = i32x4; using Ints = i32x16; using Floats = f32x16;
+    __device__ static Ints dot(const Codes &x, const Codes &w, const Ints &z) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(x, w, z, 0, 0, 0); }
+    __device__ static Floats outer(f16x4 x, f16x4 w, const Floats &z) { return __builtin_amdgcn_mfma_f32_32x32x8f16(x, w, z, 0, 0, 0); }
+};
+template <> struct Tile<16> {
+    using Codes = long; using Ints = i32x4; using Floats = f32x4;
+    __device__ static Ints dot(const Codes &x, const Codes &w, const Ints &z) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(x, w, z, 0, 0, 0); }
+    __device__ static Floats outer(f16x4 x, f16x4 w, const Floats &z) { return __builtin_amdgcn_mfma_f32_16x16x16f16(x, w, z, 0, 0, 0); }
+};
 
-template <int MT>
-__global__ __launch_bounds__(256) void mmq_q80_kernel(const uint8_t *__restrict__ W, size_t row_bytes, int n_rows, int K, int T,
-                                                      const int8_t *__restrict__ aq, const uint16_t *__restrict__ ad, float *__restrict__ out,
-                                                      int ld_out, const float *__restrict__ resid) {
-    constexpr int TT = 32 * MT, SD = TT + 4;
-    __shared__ __attribute__((aligned(16))) float s_da[Q80_KC * SD];           // [block of the chunk][token of the workgroup's tile]
-    const int nb = K >> 5;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = lane & 31, kg = lane >> 5;
-    const int t0 = blockIdx.y * TT, r0 = blockIdx.x * 128 + wave * 32;
-    const bool rows_ok = r0 < n_rows;                                  // (wave-uniform; such a wave still takes part in the barriers)
-    const int row = r0 + n < n_rows ? r0 + n : n_rows - 1;
-    const uint8_t *wrow = W + (size_t)row * row_bytes + 16 * kg;
-    const uint16_t *wd = reinterpret_cast<const uint16_t *>(W + (size_t)row * row_bytes + K);
-    const int8_t *arow[MT];
+// lane l: 16 B (4 B) from base + off to LDS to + 16 l (4 l)
+__device__ __forceinline__ void dma16(const void *base, unsigned off, unsigned to) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+}
+__device__ __forceinline__ void dma4(const void *base, unsigned off, unsigned to) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+}
+__device__ __forceinline__ const void *uniform_ptr(const void *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const void *)((uint64_t)hi << 32 | lo);
+}
+
+// Rows come in steps of 128 bytes, four blocks.  A lane that reads its own row from memory costs the CU's address unit a clock a lane, and in the matrix unit's layout every lane is another
+// line: a row of 64 blocks took 20 us however few the tiles (2048 x 2048, 40 tokens; its products are 5).  So a wave instruction brings eight rows' 128 bytes into LDS - S steps of them in
+// turn, the 16-byte pieces of row i in the order p ^ (i & 7), so that the matrix unit's reads meet no bank twice -, and the four waves share both operands.  The scales come the same way, and
+// their products from the matrix unit too: one f16 contraction of which all elements but one are zero IS d_w * d_a of every output, exactly (22 bits in f32, subnormals kept), in place of a
+// vector instruction a result.  What is left to the vector unit is convert, multiply, add - the CPU's three roundings an output and block in the CPU's order -: 48 instructions a 32 x 32
+// tile and block, its bound (5632 x 2048, 2000 tokens: 63 us of 102).
+// Wave = W x W tiles of SZ x SZ, workgroup = 2 x 2 waves.  us, 40 / 611 / 2000 tokens, this | every lane its own row, scales from LDS: 2048 x 2048 8 / 17 / 42 | 21 / 35 / 61, 5632 x 2048
+// 11 / 37 / 102 | 22 / 60 / 151, 4096 x 14336 43 / 156 / 448 | 133 / 349 / 582, 1024 x 4096 13 / 22 / 37 | 38 / 38 / 69.
+// (Tried: rows straight from memory in tiles of 16, or two to four steps ahead: the same 20 us.  The products of the next tile asked for before the fold of this one: nothing.)
+template <int SZ, int W, int S>
+__global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) {
+    using TL = Tile<SZ>;
+    using Codes = typename TL::Codes;
+    constexpr int ROWS = 2 * SZ * W, STEP = 256 * ROWS, SCALES = 16 * ROWS, STAGE = STEP + SCALES;   // rows of either operand; 128 B of codes and 8 of scales a row
+    constexpr int NR = SZ * SZ / 64, NC = ROWS / 32, NS = SCALES >= 1024 ? SCALES / 1024 : 1, LOADS = 2 * NC + NS;
+    __shared__ __attribute__((aligned(1024))) uint8_t sm[S * STAGE];
+    int sg = 0;
+    if (a.n_seg > 1 && (int)blockIdx.x >= a.tile0[1]) sg = 1;
+    if (a.n_seg > 2 && (int)blockIdx.x >= a.tile0[2]) sg = 2;
+    const int n_rows = a.n_rows[sg], K = a.K, T = a.T, nb = K >> 5, steps = nb >> 2;
+    const int l = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), n = l & (SZ - 1), kg = l / SZ;
+    const int t0 = blockIdx.y * ROWS, r0 = ((int)blockIdx.x - a.tile0[sg]) * ROWS;
+    const int last_r = (n_rows - r0 < ROWS ? n_rows - r0 : ROWS) - 1, last_t = (T - t0 < ROWS ? T - t0 : ROWS) - 1;
+    const uint8_t *const wbase = (const uint8_t *)uniform_ptr(a.W[sg] + (size_t)r0 * a.row_bytes);
+    const uint8_t *const xbase = (const uint8_t *)uniform_ptr(a.aq + (size_t)t0 * K), *const dbase = (const uint8_t *)uniform_ptr(a.ad + (size_t)t0 * nb);
+    // a request: eight rows' 128 B of codes, the 16-byte pieces of row i in the order p ^ (i & 7); or 32 rows' 8 B of scales
+    unsigned woff[NC], xoff[NC], soff[NS];
+    const unsigned piece = 16u * ((l & 7) ^ (l >> 3));
 #pragma unroll
-    for (int m = 0; m < MT; m++) {
-        const int tok = t0 + 32 * m + n < T ? t0 + 32 * m + n : T - 1;
-        arow[m] = aq + (size_t)tok * K + 16 * kg;
+    for (int i = 0; i < NC; i++) {
+        const int r = (wave + 4 * i) * 8 + (l >> 3);
+        woff[i] = (unsigned)(r < last_r ? r : last_r) * (unsigned)a.row_bytes + piece;
+        xoff[i] = (unsigned)(r < last_t ? r : last_t) * (unsigned)K + piece;
     }
-    float facc[MT][16];
+    constexpr int SR = ROWS / 32;                                      // scale requests an operand
+    bool sw[NS];
+    unsigned sto[NS];
 #pragma unroll
-    for (int m = 0; m < MT; m++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) facc[m][r] = 0.0f;
-    i32x16 z;
-#pragma unroll
-    for (int r = 0; r < 16; r++) z[r] = 0;
-
-    // per output and block: scale = d_w * d_a (exact: two f16 values), product = (float)isum * scale, sum += product - the CPU's three roundings in the CPU's
-    // order; written on pairs so that the multiplies and the add become v_pk_mul_f32 / v_pk_add_f32 (two outputs per instruction, same IEEE results)
-    auto fold = [&](const i32x16 &c, float dw, int bl, int m) {        // bl: block within the chunk
-        const f32x2 dw2 = {dw, dw};
-#pragma unroll
-        for (int rq = 0; rq < 4; rq++) {
-            const f32x4 da4 = *reinterpret_cast<const f32x4 *>(s_da + bl * SD + 32 * m + 8 * rq + 4 * kg);    // tokens 8 rq + 4 kg + (0..3) of tile m
-#pragma unroll
-            for (int rp = 0; rp < 2; rp++) {
-                const f32x2 da2 = {da4[2 * rp], da4[2 * rp + 1]};
-                const f32x2 cf = {(float)c[rq * 4 + 2 * rp], (float)c[rq * 4 + 2 * rp + 1]};
-                const f32x2 sc = dw2 * da2;
-                const f32x2 pr = cf * sc;
-                f32x2 acc = {facc[m][rq * 4 + 2 * rp], facc[m][rq * 4 + 2 * rp + 1]};
-                acc = acc + pr;
-                facc[m][rq * 4 + 2 * rp] = acc.x; facc[m][rq * 4 + 2 * rp + 1] = acc.y;
-            }
-        }
-    };
-    // The codes of a group of four blocks - a 128-byte line of every row - are requested a step ahead: the weights of the next group at the start of a group, the
-    // activations of the next token tile (of the next group's first) before a tile's products.  Two register sets, chosen at compile time: groups come in pairs.
-    const int ng = nb / Q80_UNROLL;
-    i32x4 w[2][Q80_UNROLL], av[2][Q80_UNROLL];
-    u32x2 dh[2];
-    auto ask_w = [&](int g, int s) {
-        const int gc = g < ng ? g : ng - 1;                            // (past the end: the last group again)
-#pragma unroll
-        for (int u = 0; u < Q80_UNROLL; u++) w[s][u] = *reinterpret_cast<const i32x4 *>(wrow + (size_t)(gc * Q80_UNROLL + u) * 32);
-        dh[s] = *reinterpret_cast<const u32x2 *>(wd + gc * Q80_UNROLL);
-    };
-    auto ask_a = [&](int g, int m, int s) {
-        const int gc = g < ng ? g : ng - 1;
-#pragma unroll
-        for (int u = 0; u < Q80_UNROLL; u++) av[s][u] = *reinterpret_cast<const i32x4 *>(arow[m] + (size_t)(gc * Q80_UNROLL + u) * 32);
-    };
-    if (rows_ok && ng > 0) { ask_w(0, 0); ask_a(0, 0, 0); }
-    auto group = [&](auto par, int g, int bl) {                        // par: parity of the group in its chunk (a chunk is an even number of groups, all but the last)
-        constexpr int P = decltype(par)::value;
-        ask_w(g + 1, P ^ 1);
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            constexpr int FLIP = MT == 1 ? P : 0;
-            const int s = FLIP ^ (m & 1);
-            if (m + 1 < MT) ask_a(g, m + 1, s ^ 1); else ask_a(g + 1, 0, s ^ 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < Q80_UNROLL; u++) {
-                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s][u], w[P][u], z, 0, 0, 0);
-                fold(c, h2f((uint16_t)(dh[P][u >> 1] >> (16 * (u & 1)))), bl + u, m);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    for (int b0 = 0; b0 < nb; b0 += Q80_KC) {
-        const int nbc = nb - b0 < Q80_KC ? nb - b0 : Q80_KC;
-        __syncthreads();                                               // everyone is done with the previous chunk's scales
-        for (int i = tid; i < Q80_KC * TT; i += 256) {                 // (lanes along a token's scales)
-            const int m = i / Q80_KC, b = i - m * Q80_KC;
-            const int t = t0 + m < T ? t0 + m : T - 1;
-            if (b < nbc) s_da[b * SD + m] = h2f(ad[(size_t)t * nb + b0 + b]);
-        }
-        __syncthreads();
-        if (!rows_ok) continue;
-        int b = 0;
-        for (; b + 2 * Q80_UNROLL <= nbc; b += 2 * Q80_UNROLL) {
-            group(std::integral_constant<int, 0>{}, (b0 + b) / Q80_UNROLL, b);
-            group(std::integral_constant<int, 1>{}, (b0 + b) / Q80_UNROLL + 1, b + Q80_UNROLL);
-        }
-        if (b + Q80_UNROLL <= nbc) { group(std::integral_constant<int, 0>{}, (b0 + b) / Q80_UNROLL, b); b += Q80_UNROLL; }
-        for (; b < nbc; b++) {
-            const i32x4 w1 = *reinterpret_cast<const i32x4 *>(wrow + (size_t)(b0 + b) * 32);
-            const float dw = h2f(wd[b0 + b]);
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-                const i32x4 a = *reinterpret_cast<const i32x4 *>(arow[m] + (size_t)(b0 + b) * 32);
-                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w1, z, 0, 0, 0);
-                fold(c, dw, b, m);
-            }
-        }
+    for (int i = 0; i < NS; i++) {
+        const int q = (wave + 4 * i) % (2 * SR), r = (q % SR) * 32 + (l >> 1);
+        sw[i] = q < SR;
+        sto[i] = STEP + q * 256;
+        soff[i] = sw[i] ? (unsigned)(r < last_r ? r : last_r) * (unsigned)a.row_bytes + (unsigned)K + 4u * (l & 1) : (unsigned)(r < last_t ? r : last_t) * (unsigned)nb * 2u + 4u * (l & 1);
     }
-    if (rows_ok && r0 + n < n_rows) {
+    const unsigned lds = __builtin_amdgcn_readfirstlane((int)(unsigned)(uintptr_t)sm);
+    const auto ask = [&](int step, int buf) {
+        const int s = step < steps ? step : steps - 1;                 // (past the end: the last again, never read)
+        const unsigned to = lds + buf * STAGE;
 #pragma unroll
-        for (int m = 0; m < MT; m++)
+        for (int i = 0; i < NC; i++) dma16(wbase + (size_t)s * 128, woff[i], to + (wave + 4 * i) * 1024);
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int t = t0 + 32 * m + 8 * (r >> 2) + 4 * kg + (r & 3);
-                if (t < T) {
-                    const size_t o = (size_t)t * ld_out + row;
-                    out[o] = resid ? resid[o] + facc[m][r] : facc[m][r];
+        for (int i = 0; i < NC; i++) dma16(xbase + (size_t)s * 128, xoff[i], to + STEP / 2 + (wave + 4 * i) * 1024);
+#pragma unroll
+        for (int i = 0; i < NS; i++) dma4((sw[i] ? wbase : dbase) + (size_t)s * 8, soff[i], to + sto[i]);
+    };
+    const int wr = (wave & 1) * SZ * W, wt = (wave >> 1) * SZ * W;     // the wave's tiles in the workgroup's
+    const uint32_t first = kg == 0 ? 0x0000ffffu : 0u, second = kg == 0 ? 0xffff0000u : 0u;
+    const auto one = [&](const u32x2 &d, int u) { return __builtin_bit_cast(f16x4, u32x2{d[u >> 1] & ((u & 1) ? second : first), 0u}); };
+    float acc[W][W][NR];
+#pragma unroll
+    for (int i = 0; i < W; i++)
+#pragma unroll
+        for (int j = 0; j < W; j++)
+#pragma unroll
+            for (int r = 0; r < NR; r++) acc[i][j][r] = 0.0f;
+    const typename TL::Ints zi = {};
+    const typename TL::Floats zf = {};
+#pragma unroll
+    for (int s = 0; s + 1 < S; s++) ask(s, s);
+    int buf = 0;
+    for (int step = 0; step < steps; step++) {
+        asm volatile("s_waitcnt vmcnt(%c0) lgkmcnt(0)\n\ts_barrier" :: "i"(LOADS * (S - 2)) : "memory");
+        ask(step + S - 1, buf ? buf - 1 : S - 1);
+        const uint8_t *const at = sm + buf * STAGE;
+        buf = buf + 1 < S ? buf + 1 : 0;
+        u32x2 dw[W], da[W];
+#pragma unroll
+        for (int i = 0; i < W; i++) {
+            dw[i] = *reinterpret_cast<const u32x2 *>(at + STEP + (wr + SZ * i + n) * 8);
+            da[i] = *reinterpret_cast<const u32x2 *>(at + STEP + SCALES / 2 + (wt + SZ * i + n) * 8);
+        }
+        const auto codes = [&](const uint8_t *op, int row, int u) {
+            if constexpr (SZ == 32) return *reinterpret_cast<const Codes *>(op + row * 128 + (((2 * u + kg) ^ (n & 7)) * 16));
+            else return *reinterpret_cast<const Codes *>(op + row * 128 + (((2 * u + (kg >> 1)) ^ (n & 7)) * 16) + (kg & 1) * 8);
+        };
+        Codes w[2][W], x[2][W];
+        const auto read = [&](int u) {
+#pragma unroll
+            for (int i = 0; i < W; i++) { w[u & 1][i] = codes(at, wr + SZ * i + n, u); x[u & 1][i] = codes(at + STEP / 2, wt + SZ * i + n, u); }
+        };
+        read(0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (u + 1 < 4) read(u + 1);
+#pragma unroll
+            for (int i = 0; i < W; i++)
+#pragma unroll
+                for (int j = 0; j < W; j++) {
+                    const auto c = TL::dot(x[u & 1][j], w[u & 1][i], zi);
+                    const auto sc = TL::outer(one(da[j], u), one(dw[i], u), zf);
+#pragma unroll
+                    for (int r = 0; r < NR; r++) acc[i][j][r] = acc[i][j][r] + (float)c[r] * sc[r];
                 }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // nothing lands in LDS after the workgroup's end
+    const int ld = a.ld_out[sg];
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        const int row = r0 + wr + SZ * i + n;
+        if (row >= n_rows) continue;
+        float *const out = a.out[sg] + row;
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const auto token = [&](int r) { return t0 + wt + SZ * j + (SZ == 32 ? 8 * (r >> 2) + 4 * kg + (r & 3) : 4 * kg + r); };
+            if (a.resid) {                                             // (may be out itself; the tile's are requested before its first is stored)
+                float old[NR];
+#pragma unroll
+                for (int r = 0; r < NR; r++) old[r] = a.resid[(size_t)(token(r) < T ? token(r) : T - 1) * ld + row];
+#pragma unroll
+                for (int r = 0; r < NR; r++) acc[i][j][r] = old[r] + acc[i][j][r];
             }
+#pragma unroll
+            for (int r = 0; r < NR; r++)
+                if (token(r) < T) out[(size_t)token(r) * ld] = acc[i][j][r];
+        }
     }
 }
 
@@ -199,24 +228,45 @@ hipError_t launch_expand_q80_copy(int type, const uint8_t *W, size_t row_bytes, 
     return hipGetLastError();
 }
 
-bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && T >= 32 && K >= 32 && (K % 32) == 0 && K <= 16384; }
+// The mat-vec takes one, two or four tokens to a pass over the weights; everything between goes here (us of a batch, mat-vec | tiles, 2 / 3 / 4 / 5 / 16 / 31 tokens: six TinyLlama-1.1B
+// Q8_0 layers 387 553 452 617 1057 2137 | 466 466 466 466 470 487, four 8B ones 507 722 672 891 1568 3291 | 635 626 629 629 644 671; as Q4_0 with the copy above 464 - 654 - 1648 3320 |
+// 625 - 620 - 623 646).
+bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && (T == 3 || T >= 5) && K >= 128 && (K % 128) == 0 && K <= 16384; }
+
+template <int SZ, int W, int S> static void tiles_launch(Q80Args &a, hipStream_t st) {
+    constexpr int R = 2 * SZ * W;
+    int tiles = 0;
+    for (int i = 0; i < a.n_seg; i++) { a.tile0[i] = tiles; tiles += (a.n_rows[i] + R - 1) / R; }
+    hipLaunchKernelGGL((mmq_q80_tiles_kernel<SZ, W, S>), dim3((unsigned)tiles, (unsigned)((a.T + R - 1) / R)), dim3(256), 0, st, a);
+}
+
+hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st) {
+    if (!mmq_q80_applicable(T_Q8_0, K, T) || !q.qs0 || !q.d0 || n < 1 || n > 3) return hipErrorInvalidValue;
+    for (int i = 0; i < n; i++)                                        // (16-byte requests of the codes, 4-byte ones of the scales)
+        if (sg[i].row_bytes != sg[0].row_bytes || ((((uintptr_t)sg[i].W | sg[i].row_bytes | (uintptr_t)q.qs0) & 15) | ((uintptr_t)q.d0 & 3))) return hipErrorInvalidValue;
+    Q80Args a{};
+    a.row_bytes = sg[0].row_bytes; a.n_seg = n; a.K = K; a.T = T; a.aq = q.qs0; a.ad = q.d0; a.resid = resid;
+    const auto count = [&](int r) {
+        long c = 0;
+        for (int i = 0; i < n; i++) c += (sg[i].n_rows + r - 1) / r;
+        return c * ((T + r - 1) / r);
+    };
+    for (int i = 0; i < n; i++) { a.W[i] = sg[i].W; a.out[i] = sg[i].out; a.n_rows[i] = sg[i].n_rows; a.ld_out[i] = sg[i].ld_out; }
+    // Up to two 32 x 32 workgroups a CU it is one wave's way through its row that counts, a third shorter in tiles of 16 (us, 16 | 32: 5632 x 2048, 40 tokens = 352 workgroups 11.0 | 12.9;
+    // 4096 x 14336, 100 = 512 56 | 74; 2048 x 2048, 320 = 640 13.8 | 12.8).  Four tiles of 32 a wave read half as much of LDS, but need 1.7 workgroups of 128 x 128 a CU and no more
+    // than a tenth more padding (us, one tile | four: 5632 x 2048, 1200 tokens = 440 workgroups 69 | 65; 4096 x 14336, 2000 = 512 490 | 448, 1200 = 320 292 | 335;
+    // 32000 x 2048, 320 = 750, a fifth more padding 92 | 100).
+    const long c32 = count(32), c64 = count(64), c128 = count(128);
+    if (c32 <= 2L * num_cu()) tiles_launch<16, 1, 4>(a, st);
+    else if (c128 * 10 >= 17L * num_cu() && c128 * 40 <= c64 * 11) tiles_launch<32, 2, 2>(a, st);
+    else tiles_launch<32, 1, 3>(a, st);
+    return hipGetLastError();
+}
 
 hipError_t launch_mmq_q80(const uint8_t *W, size_t row_bytes, int n_rows, int K, int T, const ActQuant &q, float *out, int ld_out,
                           const float *resid, hipStream_t st) {
-    if (!mmq_q80_applicable(T_Q8_0, K, T) || !q.qs0 || !q.d0) return hipErrorInvalidValue;
-    // four token tiles per wave once that still leaves a workgroup per CU; each output keeps its own block order, so the result does not depend on MT
-    const long wg4 = (long)((n_rows + 127) / 128) * ((T + 127) / 128);
-    if (T >= 128 && wg4 >= num_cu()) {
-        const dim3 grid((unsigned)((n_rows + 127) / 128), (unsigned)((T + 127) / 128));
-        hipLaunchKernelGGL((mmq_q80_kernel<4>), grid, dim3(256), 0, st, W, row_bytes, n_rows, K, T, q.qs0, q.d0, out, ld_out, resid);
-    } else if (T >= 64 && wg4 * 2 >= num_cu()) {
-        const dim3 grid((unsigned)((n_rows + 127) / 128), (unsigned)((T + 63) / 64));
-        hipLaunchKernelGGL((mmq_q80_kernel<2>), grid, dim3(256), 0, st, W, row_bytes, n_rows, K, T, q.qs0, q.d0, out, ld_out, resid);
-    } else {
-        const dim3 grid((unsigned)((n_rows + 127) / 128), (unsigned)((T + 31) / 32));
-        hipLaunchKernelGGL((mmq_q80_kernel<1>), grid, dim3(256), 0, st, W, row_bytes, n_rows, K, T, q.qs0, q.d0, out, ld_out, resid);
-    }
-    return hipGetLastError();
+    const Q80Seg sg{W, row_bytes, n_rows, out, ld_out};
+    return launch_mmq_q80_multi(&sg, 1, K, T, q, resid, st);
 }
 
 }  // namespace mi355

@@ -992,6 +992,10 @@ hipError_t Context::ensure_prep(const ActQuant &aq, int K, int T, bool few) {
 static bool q80_copy(const DevTensor &w, int K, int T) {
     return (w.type == T_Q4_0 || w.type == T_Q5_0 || w.type == T_IQ4_NL) && w.planes && w.n_expert == 1 && mmq_q80_applicable(T_Q8_0, K, T);
 }
+static bool q80_rows(const DevTensor &w, int K, int T) { return mmq_q80_applicable(w.type, K, T) || q80_copy(w, K, T); }
+static Q80Seg q80_seg(const DevTensor &w, int K, float *out, int ld_out) {
+    return w.type == T_Q8_0 ? Q80Seg{w.data, w.row_bytes, (int)w.N, out, ld_out} : Q80Seg{w.planes, dev_row_bytes(T_Q8_0, K), (int)w.N, out, ld_out};
+}
 static bool planes_small(const DevTensor &w, int K, int T) { return (w.type == T_Q2_K || w.type == T_Q3_K) && w.planes && T >= 32 && (K % 256) == 0; }
 
 hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *x_f32, int K, int T, float *out, int ld_out,
@@ -1081,8 +1085,15 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
         for (int i = 0; i < n; i++) segs[i] = make_seg(*ws[i], outs[i], (int)ws[i]->N, nullptr, nullptr);
         return mmvq_tokens(segs, n, K, T, EPI_STORE, aq, stream_, pending_fuse_);
     }
-    // a prompt batch with mixed types (8-expert files keep attn_k / attn_v in Q8_0): every tensor takes its own best path
+    // a prompt batch of Q8_0 tensors, or with mixed types (8-expert files keep attn_k / attn_v in Q8_0): the Q8_0 ones in one launch, every other tensor on its own best path
+    Q80Seg q80[3];
+    int n8 = 0;
+    if (n <= 3 && pending_fuse_.mode == 0 && aq.qs0)
+        for (int i = 0; i < n; i++)
+            if (q80_rows(*ws[i], K, T)) q80[n8++] = q80_seg(*ws[i], K, outs[i], (int)ws[i]->N);
+    if (n8) HIP_TRY(launch_mmq_q80_multi(q80, n8, K, T, aq, nullptr, stream_));
     for (int i = 0; i < n; i++) {
+        if (n8 && q80_rows(*ws[i], K, T)) continue;
         hipError_t e = linear(*ws[i], aq, x_f32, K, T, outs[i], (int)ws[i]->N, nullptr, EPI_STORE);
         if (e != hipSuccess) return e;
     }
@@ -1838,8 +1849,13 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                     swiglu_quantised = true;
                 }
             } else {
-                HIP_TRY(linear(L.gate, aq_e_, xn_, E, T, ffn_, FF, nullptr, EPI_STORE));
-                HIP_TRY(linear(L.up, aq_e_, xn_, E, T, ffn_u_, FF, nullptr, EPI_STORE));
+                if (!fuse_ffn && pending_fuse_.mode == 0 && aq_e_.qs0 && q80_rows(L.gate, E, T) && q80_rows(L.up, E, T)) {
+                    const Q80Seg sg[2] = {q80_seg(L.gate, E, ffn_, FF), q80_seg(L.up, E, ffn_u_, FF)};
+                    HIP_TRY(launch_mmq_q80_multi(sg, 2, E, T, aq_e_, nullptr, stream_));
+                } else {
+                    HIP_TRY(linear(L.gate, aq_e_, xn_, E, T, ffn_, FF, nullptr, EPI_STORE));
+                    HIP_TRY(linear(L.up, aq_e_, xn_, E, T, ffn_u_, FF, nullptr, EPI_STORE));
+                }
                 // prompt batch: SwiGLU and the quantisation for the down projection in one pass (no f32 round trip of T x FF)
                 if (T > 1 && is_quant(L.down.type) && (FF % 256) == 0) {
                     const bool pl = !act_is_q80(L.down.type) && T >= 3;
