@@ -42,26 +42,11 @@ template <> struct Tile<16> {
     __device__ static Floats outer(f16x4 x, f16x4 w, const Floats &z) { return __builtin_amdgcn_mfma_f32_16x16x16f16(x, w, z, 0, 0, 0); }
 };
 
-// lane l: 16 B (4 B) from base + off to LDS to + 16 l (4 l)
-__device__ __forceinline__ void dma16(const void *base, unsigned off, unsigned to) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
-}
-__device__ __forceinline__ void dma4(const void *base, unsigned off, unsigned to) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
-}
-__device__ __forceinline__ const void *uniform_ptr(const void *p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (const void *)((uint64_t)hi << 32 | lo);
-}
-
 // Rows come in steps of 128 bytes, four blocks.  A lane that reads its own row from memory costs the CU's address unit a clock a lane, and in the matrix unit's layout every lane is another
 // line: a row of 64 blocks took 20 us however few the tiles (2048 x 2048, 40 tokens; its products are 5).  So a wave instruction brings eight rows' 128 bytes into LDS - S steps of them in
 // turn, the 16-byte pieces of row i in the order p ^ (i & 7), so that the matrix unit's reads meet no bank twice -, and the four waves share both operands.  The scales come the same way, and
 // their products from the matrix unit too: one f16 contraction of which all elements but one are zero IS d_w * d_a of every output, exactly (22 bits in f32, subnormals kept), in place of a
-// vector instruction a result.  What is left to the vector unit is convert, multiply, add - the CPU's three roundings an output and block in the CPU's order -: 48 instructions a 32 x 32
+// vector instruction a result.  What is left to the vector unit is convert (or subtract), multiply, add - the CPU's three roundings an output and block in the CPU's order -: 48 instructions a 32 x 32
 // tile and block, its bound (5632 x 2048, 2000 tokens: 63 us of 102).
 // Wave = W x W tiles of SZ x SZ, workgroup = 2 x 2 waves.  us, 40 / 611 / 2000 tokens, this | every lane its own row, scales from LDS: 2048 x 2048 8 / 17 / 42 | 21 / 35 / 61, 5632 x 2048
 // 11 / 37 / 102 | 22 / 60 / 151, 4096 x 14336 43 / 156 / 448 | 133 / 349 / 582, 1024 x 4096 13 / 22 / 37 | 38 / 38 / 69.
@@ -106,11 +91,11 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
         const int s = step < steps ? step : steps - 1;                 // (past the end: the last again, never read)
         const unsigned to = lds + buf * STAGE;
 #pragma unroll
-        for (int i = 0; i < NC; i++) dma16(wbase + (size_t)s * 128, woff[i], to + (wave + 4 * i) * 1024);
+        for (int i = 0; i < NC; i++) lds_dma16(wbase + (size_t)s * 128, woff[i], to + (wave + 4 * i) * 1024);
 #pragma unroll
-        for (int i = 0; i < NC; i++) dma16(xbase + (size_t)s * 128, xoff[i], to + STEP / 2 + (wave + 4 * i) * 1024);
+        for (int i = 0; i < NC; i++) lds_dma16(xbase + (size_t)s * 128, xoff[i], to + STEP / 2 + (wave + 4 * i) * 1024);
 #pragma unroll
-        for (int i = 0; i < NS; i++) dma4((sw[i] ? wbase : dbase) + (size_t)s * 8, soff[i], to + sto[i]);
+        for (int i = 0; i < NS; i++) lds_dma4((sw[i] ? wbase : dbase) + (size_t)s * 8, soff[i], to + sto[i]);
     };
     const int wr = (wave & 1) * SZ * W, wt = (wave >> 1) * SZ * W;     // the wave's tiles in the workgroup's
     const uint32_t first = kg == 0 ? 0x0000ffffu : 0u, second = kg == 0 ? 0xffff0000u : 0u;
@@ -122,7 +107,9 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
         for (int j = 0; j < W; j++)
 #pragma unroll
             for (int r = 0; r < NR; r++) acc[i][j][r] = 0.0f;
-    const typename TL::Ints zi = {};
+    // (with the bias as the sums' start a subtraction converts them: 4096 x 14336 at 40 tokens, tiles of 16, 44 -> 41 us, at 2000, four of 32 a wave, 430 -> 415; one of 32 a wave is 4 % slower for it)
+    constexpr bool BIAS = SZ == 16 || W == 2;
+    const typename TL::Ints zi = (typename TL::Ints)(BIAS ? INT_BIAS : 0);
     const typename TL::Floats zf = {};
 #pragma unroll
     for (int s = 0; s + 1 < S; s++) ask(s, s);
@@ -158,7 +145,7 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
                     const auto c = TL::dot(x[u & 1][j], w[u & 1][i], zi);
                     const auto sc = TL::outer(one(da[j], u), one(dw[i], u), zf);
 #pragma unroll
-                    for (int r = 0; r < NR; r++) acc[i][j][r] = acc[i][j][r] + (float)c[r] * sc[r];
+                    for (int r = 0; r < NR; r++) acc[i][j][r] = acc[i][j][r] + (BIAS ? biased_f32(c[r]) : (float)c[r]) * sc[r];
                 }
         }
     }

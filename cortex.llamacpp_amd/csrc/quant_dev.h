@@ -193,5 +193,37 @@ __device__ __forceinline__ float dequant_elem(int type, const uint8_t *row, int 
     return 0.0f;
 }
 
+// An integer below 2^22 in magnitude as f32: with INT_BIAS as the sum's start its bits are 1.5 * 2^23 + n in f32, and one subtraction is exact.  v_sub_f32 takes 1.25 ns a wave instruction at
+// two waves a SIMD, v_cvt_f32_i32 2.9 (conversions go at half rate).
+constexpr int INT_BIAS = 0x4b400000;
+__device__ __forceinline__ float biased_f32(int n) { return __uint_as_float((uint32_t)n) - 12582912.0f; }
+
+// memory straight into LDS: lane l's 16 B (4 B) from base + off to LDS to + 16 l (4 l); base and to uniform
+__device__ __forceinline__ void lds_dma16(const void *base, unsigned off, unsigned to) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+}
+__device__ __forceinline__ void lds_dma4(const void *base, unsigned off, unsigned to) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+}
+// the same, N kilobytes one behind the other
+template <int N> __device__ __forceinline__ void lds_dma16_n(const void *base, unsigned off, unsigned to) {
+    static_assert(N == 1 || N == 2 || N == 4, "");
+    unsigned keep;
+    if constexpr (N == 1) lds_dma16(base, off, to);
+    else if constexpr (N == 2)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\ts_mov_b32 m0, %0"
+                     : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %1, %2 offset:2048\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072\n\ts_mov_b32 m0, %0"
+                     : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
+}
+__device__ __forceinline__ const void *uniform_ptr(const void *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const void *)((uint64_t)hi << 32 | lo);
+}
 
 }  // namespace mi355
