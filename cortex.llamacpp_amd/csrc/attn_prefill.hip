@@ -68,6 +68,61 @@ __device__ __forceinline__ float xhalf_sum(float x) {
 // key index (0..31) of MFMA K-slot (j, kg, i): the order the score tile leaves its 16 keys per lane in registers
 __device__ __forceinline__ int slot_key(int j, int kg, int i) { return 16 * j + 8 * (i >> 2) + 4 * kg + (i & 3); }
 
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// A chunk whose V planes are in memory already (flash_attn_planes_kernel), in LDS: K rows as the cache has them, the planes, 32 x NB f16 scales, positions, sequences
+template <bool F16, int DH> struct PlaneChunk {
+    static constexpr int NB = DH / 32, ROW = F16 ? 2 * DH : DH, PIECES = ROW / 16, KREQ = CK * ROW / 1024, VPL = NB * 2 * 2 * 32 * 8, VBYTES = VPL * (F16 ? 2 : 4), VREQ = VBYTES / 1024;
+    static constexpr int V = CK * ROW, DK = V + VBYTES, CPOS = DK + 256, CSEQ = CPOS + 256, BYTES = CSEQ + 256;
+    // eight neighbouring rows' piece p in different banks: 256 bytes are all of them, four rows of 64
+    __device__ static constexpr int swz(int r) { return PIECES >= 8 ? r & 7 : (r >> 2) & 3; }
+};
+static size_t plane_chunk_bytes(bool f16, int D) { return (size_t)D * CK * (f16 ? 2 : 4); }
+
+// The V planes of a prompt batch, once for all its query tiles: workgroup = (chunk, kv head), in the order the matrix cores take them (Chunk's vh and, for a q8_0 cache, vl: V' = code * d_v
+// split exactly in two halves).  4096 cells of eight kv heads, q8_0: 17 MB, 6 us - where every tile converted every chunk it walked, for 3.1 of a chunk's 7.8 kilocycles.
+template <bool F16, int DH>
+__global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a) {
+    constexpr int NB = DH / 32;
+    using PC = PlaneChunk<F16, DH>;
+    __shared__ __attribute__((aligned(16))) _Float16 sm[PC::VBYTES / 2];
+    const int c = blockIdx.x, g = blockIdx.y, n_ctx = a.n_ctx;
+    if (c * CK >= *a.n_kv_dev) return;                          // (no tile marks it)
+    for (int u = threadIdx.x; u < 2 * DH; u += 256) {           // four consecutive keys x four dims
+        const int kgp = u / (DH / 4), dg = u % (DH / 4);
+        const int j = kgp >> 2, kgs = kgp & 1, slot0 = ((kgp >> 1) & 1) * 4;
+        uint64_t v[4];
+        float d[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int cell = c * CK + 4 * kgp + kk;
+            const size_t row = (size_t)g * n_ctx + (cell < n_ctx ? cell : n_ctx - 1);
+            if (F16) v[kk] = *reinterpret_cast<const uint64_t *>(a.kv.v + row * DH * 2 + 8 * dg);
+            else { v[kk] = *reinterpret_cast<const uint32_t *>(a.kv.v + row * DH + 4 * dg); d[kk] = h2f(a.kv.vd[row * NB + (dg >> 3)]); }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int dim = 4 * dg + e, o = ((((dim >> 5) * 2 + j) * 2 + kgs) * 32 + ((dim & 31) ^ (dim >> 5))) * 8 + slot0;
+            f16x4 hi, lo;
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                if (F16) hi[kk] = __builtin_bit_cast(_Float16, (uint16_t)(v[kk] >> (16 * e)));
+                else {
+                    const float x = (float)(int8_t)((v[kk] >> (8 * e)) & 0xff) * d[kk];
+                    hi[kk] = (_Float16)x;
+                    lo[kk] = (_Float16)(x - (float)hi[kk]);
+                }
+            }
+            *reinterpret_cast<f16x4 *>(sm + o) = hi;
+            if (!F16) *reinterpret_cast<f16x4 *>(sm + PC::VPL + o) = lo;
+        }
+    }
+    __syncthreads();
+    u32x4 *const out = reinterpret_cast<u32x4 *>(reinterpret_cast<uint8_t *>(a.pf_planes) + ((size_t)g * ((n_ctx + CK - 1) / CK) + c) * PC::VBYTES);
+    for (int i = threadIdx.x; i < PC::VBYTES / 16; i += 256) out[i] = reinterpret_cast<const u32x4 *>(sm)[i];
+}
+
 #ifdef MI355_FA_PROBE
 // tools/build_fa_probe.sh: shader-clock split of one workgroup (printed by the last tile's first split): prologue | per chunk: scores,
 // softmax, P.V, barrier, store, barrier
@@ -84,7 +139,11 @@ __device__ __forceinline__ int slot_key(int j, int kg, int i) { return 16 * j + 
 // Q4 (with F16 = false): a q4_0 K / V cache (cache_type "q4_0", src/llama_engine.cc:272-285).  Only the staging differs: a 16-byte piece of a K row is one
 // 32-block of nibbles, unpacked to the int8 codes nibble - 8 on its way into LDS (elements 0..15 from the low nibbles, 16..31 from the high ones), V codes
 // likewise; scores (vec_dot_q4_0_q8_0: the same integer dot with those codes), scales and the f16 hi / lo split of V' = code * d_v are the q8_0 path's.
-template <int R, bool F16, int KH, int QS, int DH = 128, bool Q4 = false>
+// PL (q8_0 and f16 caches): V's planes are in memory (flash_attn_planes_kernel), so a chunk goes to LDS as it is - no registers, no conversion, no scattered LDS stores: those were 3.1 of the
+// 7.8 kilocycles of a pair of chunks and made most of the 1.1 at the barrier; now 5.2, of which the two waves of a SIMD have 2 in matrix products and 3.3 in vector instructions, which bound
+// it (probe, 32 / 8 heads of 128, q8_0; 1919 tokens behind 2048: 382 -> 276 us, 2048 behind none 174 -> 134).  The block scales' products come from the matrix unit.  The same bits.
+// (Tried: one of a SIMD's two waves half a chunk behind, its P.V beside the other's scores, in a third buffer: nothing.  Integer sums that start at the f32 bias: nothing.)
+template <int R, bool F16, int KH, int QS, int DH = 128, bool Q4 = false, bool PL = false>
 __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel(const AttnArgs a) {
     // head width: 128 or 64 (TinyLlama, Llama-3.2-1B, nomic-embed): everything below is written in 32-dim blocks (NB of them) and 16-dim matrix-core steps
     constexpr int D = DH, NB = DH / 32, K_STRIDE = DH + 16, KF_STRIDE = 2 * DH + 16, NKS = DH / 16, VPL = NB * 2 * 2 * 32 * 8, NVU = 2 * DH;
@@ -98,6 +157,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
     constexpr int KVROW = Q4 ? D / 2 : D;                         // bytes of a quantised K / V row
     constexpr int CHUNK_LDS = CK * KS + NB * CK * 4 + 2 * VPL * 2 + CK * 4 + CK * 8;   // one staged chunk (launcher: one per half)
     static_assert(CHUNK_LDS % 16 == 0, "chunk buffers stay 16-byte aligned");
+    using PC = PlaneChunk<F16, DH>;
     constexpr int NT = 64 * R * QS;                   // threads of one half: the staging roles below are per half
     const int tid_all = threadIdx.x, lane = tid_all & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(tid_all >> 6);
@@ -106,6 +166,16 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
     const int tid = tid_all - half * NT;
     auto chunk_at = [&](int par) {                    // buffer par of this half
         Chunk S;
+        if constexpr (PL) {
+            uint8_t *base = smem + (half * 2 + par) * PC::BYTES;
+            S.k = reinterpret_cast<int8_t *>(base);
+            S.dk = nullptr;
+            S.vh = reinterpret_cast<_Float16 *>(base + PC::V);
+            S.vl = S.vh + VPL;
+            S.cpos = reinterpret_cast<int *>(base + PC::CPOS);
+            S.cseq = reinterpret_cast<unsigned long long *>(base + PC::CSEQ);
+            return S;
+        }
         uint8_t *base = smem + (half * 2 + par) * CHUNK_LDS;
         S.k = reinterpret_cast<int8_t *>(base);
         S.dk = reinterpret_cast<float *>(base + CK * KS);
@@ -155,6 +225,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
     //      f16 cache: round to f16, lane holds dims 16 j + 8 kg .. + 7 of K-step j
     i32x4 qc[NB];
     float dq[NB];
+    uint32_t dqh[NB / 2] = {};                                 // the scales as f16 pairs
     f16x8 qh[F16 ? NKS : 1];
     if constexpr (F16) {
         const float *qrow = a.q + ((size_t)qt * H + h) * D;
@@ -187,6 +258,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
             }
             qc[b].x = w[0]; qc[b].y = w[1]; qc[b].z = w[2]; qc[b].w = w[3];
             dq[b] = h2f(f2h(d));
+            dqh[b >> 1] |= (uint32_t)f2h(d) << (16 * (b & 1));
         }
     }
 
@@ -330,6 +402,40 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
             if (lane == 0) { s_chunk_open[par] = all_open ? 1 : 0; if (QS > 1) s_chunk_minpos[par] = mp; }
         }
     };
+    // PL: chunk c -> buffer par of this half, by the half's waves in turn: K rows as they are (1 KB = 1024 / ROW of them a request, the 16-byte pieces of row r in the order
+    // p ^ swz(r)), V's planes, the cells' positions and sequences, the K scales.  What a request needs beside c is made once.
+    constexpr int NW = R * QS, KI = (PC::KREQ + NW - 1) / NW, VN = PC::VREQ >= 4 * NW ? 4 : PC::VREQ >= 2 * NW ? 2 : 1, VI = (PC::VREQ / VN + NW - 1) / NW, SW = NB / 2;   // (SW: dwords of a row's scales)
+    const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(uintptr_t)smem + (unsigned)(half * 2 * PC::BYTES)));
+    const void *kbase = nullptr, *vbase = nullptr, *sbase = nullptr, *pbase = nullptr, *qbase = nullptr;
+    unsigned kr[KI] = {}, krow_last = 0;
+    if constexpr (PL) {
+        kbase = uniform_ptr(a.kv.k + head_row0 * PC::ROW);
+        vbase = uniform_ptr(reinterpret_cast<const uint8_t *>(a.pf_planes) + (size_t)g * ((n_ctx + CK - 1) / CK) * PC::VBYTES);
+        sbase = F16 ? nullptr : uniform_ptr(a.kv.kd + head_row0 * NB);
+        pbase = uniform_ptr(a.cell_pos); qbase = uniform_ptr(a.cell_seq);
+        krow_last = (unsigned)(n_ctx - 1);                     // (cells past the table's end: the last one's, never visible)
+#pragma unroll
+        for (int i = 0; i < KI; i++) kr[i] = (wave + NW * i) * (1024 / PC::ROW) + lane / PC::PIECES;
+    }
+    auto request = [&](int c, int par) {
+        const unsigned to = lds0 + par * PC::BYTES, cell0 = (unsigned)__builtin_amdgcn_readfirstlane(c) * CK;
+        const auto cell = [&](unsigned i) { return min(cell0 + i, krow_last); };
+#pragma unroll
+        for (int i = 0; i < KI; i++)
+            if (KI * NW == PC::KREQ || wave + NW * i < PC::KREQ)
+                lds_dma16(kbase, cell(kr[i]) * PC::ROW + 16u * ((lane % PC::PIECES) ^ PC::swz(kr[i])), to + (wave + NW * i) * 1024);
+#pragma unroll
+        for (int i = 0; i < VI; i++)
+            if (VI * NW * VN == PC::VREQ || (wave + NW * i) * VN < PC::VREQ)
+                lds_dma16_n<VN>(vbase, cell0 / CK * PC::VBYTES + (wave + NW * i) * VN * 1024 + lane * 16u, to + PC::V + (wave + NW * i) * VN * 1024);
+#pragma unroll
+        for (int i = 0; i < (F16 ? 2 : 3); i++) {
+            if (wave != i % NW) continue;
+            if (i == 0) lds_dma4(pbase, cell(lane & 31) * 4u, to + PC::CPOS);
+            if (i == 1) lds_dma4(qbase, cell(lane >> 1) * 8u + 4u * (lane & 1), to + PC::CSEQ);
+            if (i == 2) lds_dma4(sbase, cell(min(lane / SW, CK - 1)) * (4u * SW) + 4u * (lane % SW), to + PC::DK);
+        }
+    };
     auto next_visible = [&](int from) -> int {                   // first marked chunk >= from, or n_chunks
         int c = from;
         while (c < n_chunks) {
@@ -351,21 +457,21 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
 
     __syncthreads();                                            // tile bounds complete
     // ---- which chunks matter: one pass over the cell table (a wave's 64 cells = two chunks per ballot)
-    for (int cell0 = 0; cell0 < n_chunks * CK; cell0 += NT * KH) {
-        const int cell = cell0 + tid_all;
-        int mine = 0;
-        if (cell < n_kv) {
-            const int cp = a.cell_pos[cell];
-            const unsigned long long cs = a.cell_seq[cell];
-            mine = (cp >= 0 && cp <= s_tile_maxpos && (cs & s_tile_seqs) != 0ull) ? 1 : 0;
+    //      (eight groups of cells requested before the first is looked at: one behind the other they were 16 of the prologue's 36 kilocycles at 4096 cells)
+    for (int base = 0; base < n_chunks * CK; base += NT * KH * 8) {
+        int cps[8];
+        unsigned long long css[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int cell = base + NT * KH * i + tid_all;
+            cps[i] = -1; css[i] = 0;
+            if (cell < n_kv) { cps[i] = a.cell_pos[cell]; css[i] = a.cell_seq[cell]; }
         }
-        const unsigned long long bal = __ballot(mine);
-        if (lane == 0) {
-            const int c0 = (cell0 + wave_all * 64) / CK;
-            if (c0 < MAX_CHUNKS) {
-                unsigned bits = ((unsigned)(bal & 0xffffffffull) != 0u ? 1u : 0u) | ((unsigned)(bal >> 32) != 0u ? 2u : 0u);
-                if (bits) atomicOr(&s_vis[c0 >> 5], bits << (c0 & 31));
-            }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const unsigned long long bal = __ballot(cps[i] >= 0 && cps[i] <= s_tile_maxpos && (css[i] & s_tile_seqs) != 0ull);
+            const int c0 = (base + NT * KH * i + wave_all * 64) / CK;
+            if (lane == 0 && bal && c0 < MAX_CHUNKS) atomicOr(&s_vis[c0 >> 5], (((unsigned)bal ? 1u : 0u) | ((unsigned)(bal >> 32) ? 2u : 0u)) << (c0 & 31));
         }
     }
     __syncthreads();
@@ -392,26 +498,65 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
     const int n_it = (left + KH - 1) / KH;                      // iterations of the workgroup (the barriers are everybody's)
     // two buffers per half: chunk c is on the matrix cores from one while chunk c + 1 (requested an iteration ago) is converted into the
     // other and chunk c + 2's requests go out: ONE barrier per chunk (eight waves meet at it; the second one cost 0.5 kilocycles a chunk)
-    auto next_mine = [&](int cur) -> int { int x = next_visible(cur + 1); if (KH == 2) x = next_visible(x + 1); return x; };
+    // PL: the marks after chunk c, a word at a time
+    int vis_i = c >> 5;
+    unsigned vis_w = PL && c < n_chunks ? (unsigned)__builtin_amdgcn_readfirstlane((int)(s_vis[vis_i] & ~((2u << (c & 31)) - 1u))) : 0u;
+    auto next_marked = [&]() -> int {
+        while (vis_w == 0) {
+            if (++vis_i * 32 >= n_chunks) return n_chunks;
+            vis_w = (unsigned)__builtin_amdgcn_readfirstlane((int)s_vis[vis_i]);
+        }
+        const int b = __builtin_ctz(vis_w);
+        vis_w &= vis_w - 1;
+        return vis_i * 32 + b;
+    };
+    auto next_mine = [&](int cur) -> int {
+        if constexpr (PL) { if (KH == 2) (void)next_marked(); return next_marked(); }
+        int x = next_visible(cur + 1); if (KH == 2) x = next_visible(x + 1); return x; };
     int cn = n_chunks, par = 0;
     const int sub_maxpos = s_sub_maxpos[sub];
     const bool sub_live = (tile * QS + sub) * QT < a.T;         // (a ragged last tile may leave a sub-tile without queries)
-    if (mine > 0) { load_data(c); store_chunk(0); }
-    if (mine > 1) { cn = next_mine(c); load_data(cn); }
-    __syncthreads();
+    const int tile_minpos = __builtin_amdgcn_readfirstlane(s_tile_minpos);
+    const unsigned long long tile_seqs = s_tile_seqs;
+    if constexpr (PL) {
+        if (mine > 0) request(c, 0);
+        if (mine > 1) cn = next_mine(c);
+    } else {
+        if (mine > 0) { load_data(c); store_chunk(0); }
+        if (mine > 1) { cn = next_mine(c); load_data(cn); }
+        __syncthreads();
+    }
     FA_T(0);
     for (int it = 0; it < n_it; it++) {
 #ifdef MI355_FA_PROBE
         fa_chunks++;
 #endif
         int cnn = n_chunks;
-        if (it + 1 < mine) {
-            store_chunk(par ^ 1);
-            if (it + 2 < mine) { cnn = next_mine(cn); load_data(cnn); }     // in flight while this chunk and the next conversion run
+        const Chunk S = chunk_at(par);
+        bool open = false, live = it < mine;                    // (wave-uniform) every cell visible to every query of the tile; some cell to some query of the sub-tile
+        int cp = -1;                                            // PL: lane n's cell
+        unsigned long long cs = 0;
+        bool held = false;
+        if constexpr (PL) {
+            // this chunk has landed, and nobody reads the other buffer any more
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (it + 1 < mine) {
+                request(cn, par ^ 1);
+                if (it + 2 < mine) cnn = next_mine(cn);
+            }
+            cp = S.cpos[n]; cs = S.cseq[n];
+            held = c * CK + n < n_kv && cp >= 0;
+            if (QS > 1) live = live && sub_live && __any(held && cp <= sub_maxpos);
+        } else {
+            if (it + 1 < mine) {
+                store_chunk(par ^ 1);
+                if (it + 2 < mine) { cnn = next_mine(cn); load_data(cnn); }     // in flight while this chunk and the next conversion run
+            }
+            open = s_chunk_open[par] != 0;
+            if (QS > 1) live = live && sub_live && (open || s_chunk_minpos[par] <= sub_maxpos);
         }
         FA_T(5);
-        if (it < mine && (QS == 1 || (sub_live && (s_chunk_open[par] || s_chunk_minpos[par] <= sub_maxpos)))) {   // (wave-uniform)
-            const Chunk S = chunk_at(par);
+        if (live) {
             // ---- scores S^T[key][query] of this chunk
             float sc[16];
 #pragma unroll
@@ -422,14 +567,31 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
                 for (int r = 0; r < 16; r++) sa[r] = 0.0f;
 #pragma unroll
                 for (int j = 0; j < NKS; j++) {
-                    const f16x8 ak = *reinterpret_cast<const f16x8 *>(S.k + n * KS + (16 * j + 8 * kg) * 2);
+                    const f16x8 ak = *reinterpret_cast<const f16x8 *>(PL ? S.k + n * PC::ROW + 16 * ((2 * j + kg) ^ PC::swz(n)) : S.k + n * KS + (16 * j + 8 * kg) * 2);
                     sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qh[j], sa, 0, 0, 0);
                 }
 #pragma unroll
                 for (int r = 0; r < 16; r++) sc[r] = sa[r];
             }
+            if constexpr (PL && !F16) {
+                // d_q * d_k of every score is one f16 contraction with a single element that is not zero: exact, and no vector instructions
+                uint32_t dk[NB / 2];
 #pragma unroll
-            for (int b = 0; b < (F16 ? 0 : NB); b++) {
+                for (int w = 0; w < NB / 2; w++) dk[w] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(S.k) + PC::DK + n * (2 * NB) + 4 * w);
+                const auto one = [&](uint32_t d, int b) { return __builtin_bit_cast(f16x4, u32x2{d & (kg ? 0u : (b & 1) ? 0xffff0000u : 0xffffu), 0u}); };
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const i32x4 ak = *reinterpret_cast<const i32x4 *>(S.k + n * PC::ROW + 16 * ((2 * b + kg) ^ PC::swz(n)));
+                    const i32x16 zi = {};
+                    const f32x16 zf = {};
+                    const i32x16 I = __builtin_amdgcn_mfma_i32_32x32x32_i8(ak, qc[b], zi, 0, 0, 0);
+                    const f32x16 dd = __builtin_amdgcn_mfma_f32_32x32x8f16(one(dk[b >> 1], b), one(dqh[b >> 1], b), zf, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) sc[r] += (float)I[r] * dd[r];
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < (F16 || PL ? 0 : NB); b++) {
                 const i32x4 ak = *reinterpret_cast<const i32x4 *>(S.k + n * K_STRIDE + 32 * b + 16 * kg);
                 i32x16 z;
 #pragma unroll
@@ -447,7 +609,8 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
             // (scores and the running maximum are kept in log2 units: exp(s - m) is one v_exp_f32 of (s - m) * log2(e), which is
             // folded into the softmax scale; exp2(-inf) = 0 does the masking; the record a split leaves converts m back)
             float mloc = -INFINITY;
-            if (s_chunk_open[par]) {                                          // (uniform over the half)
+            if constexpr (PL) open = __all(held && cp <= tile_minpos && (cs & tile_seqs) == tile_seqs);
+            if (open) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) { sc[r] *= scale_l2; mloc = fmaxf(mloc, sc[r]); }
             } else {
@@ -456,7 +619,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
                     const int key = (r & 3) + 8 * (r >> 2) + 4 * kg;
                     const int cp = S.cpos[key];
                     const unsigned long long cs = S.cseq[key];
-                    const bool vis = q_ok && cp >= 0 && cp <= tpos && ((cs >> tseq) & 1ull);
+                    const bool vis = q_ok && cp >= 0 && cp <= tpos && ((cs >> tseq) & 1ull) && (!PL || c * CK + key < n_kv);
                     sc[r] = vis ? sc[r] * scale_l2 : -INFINITY;
                     mloc = fmaxf(mloc, sc[r]);
                 }
@@ -489,7 +652,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
                     const float v = p[8 * j + i];
                     const _Float16 hi = (_Float16)v;
                     ph[j][i] = hi;
-                    pl[j][i] = (_Float16)(v - (float)hi);
+                    pl[j][i] = (_Float16)__builtin_fmaf((float)hi, -1.0f, v);
                 }
             FA_T(2);
             // ---- O^T[d][query] += V'^T . P^T
@@ -506,10 +669,11 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
                 }
         }
         FA_T(3);
-        __syncthreads();                                        // chunk c consumed, chunk cn staged
+        if constexpr (!PL) __syncthreads();                     // chunk c consumed, chunk cn staged
         FA_T(4);
         c = cn; cn = cnn; par ^= 1;
     }
+    if constexpr (PL) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the last chunk consumed (the hand-over below takes its place)
     if constexpr (KH == 2) {
         // ---- the second half's partial (O, m, l) -> LDS (the chunk buffers are done with) -> merged into the first half's: two softmax
         // partials over disjoint keys, O = O_a 2^(m_a - m) + O_b 2^(m_b - m)
@@ -611,14 +775,59 @@ int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max) {
     return s < 1 ? 1 : s;
 }
 
+// (a context's workspace: 4 KB a cell for eight kv heads of 128 in a q8_0 cache, half of that in an f16 one)
+size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int D, int G, int n_ctx) {
+    const bool f16 = type_k == T_F16 && type_v == T_F16;
+    if (!(f16 || (type_k == T_Q8_0 && type_v == T_Q8_0)) || (D != 64 && D != 128) || G < 1 || n_ctx < 1) return 0;
+    const size_t b = (size_t)((n_ctx + CK - 1) / CK) * G * plane_chunk_bytes(f16, D);
+    return b <= ((size_t)256 << 20) ? b : 0;
+}
+// The planes of the scanned cells cost 6 us a layer at 4096 cells of eight kv heads, and spare a query tile 2 of 5 parts of its time: from eight tiles on that see all the cells, or as many more
+// as they see less of them (us, planes / every tile on its own: 1919 tokens behind 2048 a layer 276 + 7 / 382; four tiles break even).
+bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible) {
+    const int tiles = (T + QT * fa_sub_tiles(H / G) - 1) / (QT * fa_sub_tiles(H / G));
+    return (long)tiles * std::min(n_kv, visible) >= 8L * n_kv;
+}
+
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st) {
     const int R = a.H / a.G, kh = fa_key_halves(R), qs = fa_sub_tiles(R);
     const int nsp = (a.pf_splits > 1 && a.part) ? a.pf_splits : 1;
+    const bool planes = a.pf_planes && flash_attn_prefill_planes_bytes(a.type_k, a.type_v, a.D, a.G, a.n_ctx) && kh == (R <= 4 ? 2 : 1) && qs == (R == 1 ? 4 : R == 2 ? 2 : 1);
     const dim3 grid((unsigned)a.G, (unsigned)((a.T + QT * qs - 1) / (QT * qs)), (unsigned)nsp);
     const bool f16 = a.type_k == T_F16;
     const int nb = a.D / 32;
     const size_t chunk = (size_t)CK * (f16 ? 2 * a.D + 16 : a.D + 16) + nb * CK * 4 + 2 * (size_t)(nb * 2 * 2 * 32 * 8) * 2 + CK * 4 + CK * 8;
-    const size_t lds = kh == 2 ? std::max(4 * chunk, (size_t)R * qs * (16 * nb + 2) * 64 * 4) : 2 * chunk;   // two chunk buffers per half, later the hand-over of the second half
+    const size_t pchunk = (size_t)CK * (f16 ? 2 * a.D : a.D) + plane_chunk_bytes(f16, a.D) + 768;
+    const size_t lds = kh == 2 ? std::max(4 * (planes ? pchunk : chunk), (size_t)R * qs * (16 * nb + 2) * 64 * 4) : 2 * (planes ? pchunk : chunk);   // two chunk buffers per half, later the hand-over of the second half
+    if (planes) {
+        const dim3 pg((unsigned)((std::min(a.n_kv_max, a.n_ctx) + CK - 1) / CK), (unsigned)a.G);
+#define FAPL(F, DD) hipLaunchKernelGGL((flash_attn_planes_kernel<F, DD>), pg, dim3(256), 0, st, a)
+        if (f16) { if (a.D == 128) FAPL(true, 128); else FAPL(true, 64); }
+        else { if (a.D == 128) FAPL(false, 128); else FAPL(false, 64); }
+#undef FAPL
+#define FAPP(RR, F, KK, QQ, DD) do { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, F, KK, QQ, DD, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+                                     hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, F, KK, QQ, DD, false, true>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } while (0)
+#define FAPT(RR, KK, QQ, DD) do { if (f16) FAPP(RR, true, KK, QQ, DD); else FAPP(RR, false, KK, QQ, DD); } while (0)
+        if (a.D == 64) switch (R) {
+            case 1: FAPT(1, 2, 4, 64); break;
+            case 2: FAPT(2, 2, 2, 64); break;
+            case 4: FAPT(4, 2, 1, 64); break;
+            case 8: FAPT(8, 1, 1, 64); break;
+            default: return hipErrorInvalidValue;
+        } else switch (R) {
+            case 1: FAPT(1, 2, 4, 128); break;
+            case 2: FAPT(2, 2, 2, 128); break;
+            case 3: FAPT(3, 2, 1, 128); break;
+            case 4: FAPT(4, 2, 1, 128); break;
+            case 5: FAPT(5, 1, 1, 128); break;
+            case 6: FAPT(6, 1, 1, 128); break;
+            case 7: FAPT(7, 1, 1, 128); break;
+            case 8: FAPT(8, 1, 1, 128); break;
+            default: return hipErrorInvalidValue;
+        }
+#undef FAPT
+#undef FAPP
+    } else
 #define FAP_D(RR, KK, QQ, DD) do { \
         if (f16) { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, true, KK, QQ, DD>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
                    hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, true, KK, QQ, DD>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } \

@@ -44,6 +44,7 @@ struct mi355_context {
 
 static thread_local std::string t_err;
 static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1, g_op_mmq_few = -1;
+static int g_op_attn_planes = 0;   // mi355_op_flash_attn: 1 a prompt batch's V planes made once for all its query tiles
 static int g_op_attn_cols = 0;     // mi355_op_flash_attn: 0 the call's own kernel, else attn_cols.hip with so many shares of the keys
 static bool g_backend_ok = false;
 
@@ -791,6 +792,8 @@ int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t
     a.pf_splits = flash_attn_prefill_splits((int)T, H, G, D, n_cells);
     DevBuf part(flash_attn_workspace_floats((int)T, H, D, std::max(a.splits, a.pf_splits)) * 4);
     a.part = part.as<float>();
+    DevBuf planes(g_op_attn_planes ? flash_attn_prefill_planes_bytes(type_k, type_v, D, G, n_cells) : 0);
+    a.pf_planes = g_op_attn_planes ? planes.as<void>() : nullptr;
     const bool cols = g_op_attn_cols > 0;
     if (cols && !flash_attn_cols_applicable(a)) { fail("attn_cols: no form for this call"); return MI355_ERR_ARG; }
     DevBuf cpart(cols ? flash_attn_workspace_floats((int)T, H, D, g_op_attn_cols) * 4 : 16);
@@ -930,6 +933,7 @@ int mi355_debug_set_option(const char *name, int32_t value) {
     if (!strcmp(name, "mmq_ksplit")) { g_op_mmq_ksplit = value != 0; return MI355_OK; }
     if (!strcmp(name, "mmq_few")) { g_op_mmq_few = value; return MI355_OK; }
     if (!strcmp(name, "attn_store_fuse")) { set_attn_store_fuse(value != 0); return MI355_OK; }
+    if (!strcmp(name, "attn_planes")) { g_op_attn_planes = value > 0; return MI355_OK; }
     if (!strcmp(name, "attn_cols")) { g_op_attn_cols = value < 0 || value > 64 ? 0 : value; return MI355_OK; }     // mi355_op_flash_attn: attn_cols.hip with so many shares of the keys
     if (!strcmp(name, "late_sums")) { set_late_sums(value != 0); return MI355_OK; }
     if (!strcmp(name, "rope_fast")) { set_rope_fast(value != 0); return MI355_OK; }

@@ -706,6 +706,9 @@ bool Context::init(std::string &err) {
         ws = std::max(ws, flash_attn_workspace_floats(t, hp.n_head, (int)D, flash_attn_prefill_splits(t, hp.n_head, (int)G, (int)D, (int)NC)));
     att_part_ = (float *)dalloc(ws * 4);
     att_part_floats_ = ws;
+    const size_t planes = T >= 32 && D * (size_t)hp.n_head_kv > 0 ? flash_attn_prefill_planes_bytes(cp.type_k, cp.type_v, (int)D, (int)G, (int)NC) : 0;
+    att_planes_ = planes ? dalloc(planes) : nullptr;             // (without: every query tile converts the chunks it walks)
+    if (planes && !att_planes_) (void)hipGetLastError();
     att_counters_ = (unsigned *)dalloc(64 * ATT_SYNC_STRIDE * sizeof(unsigned));
     if (!att_part_ || !att_counters_) { err = "attention workspace allocation failed"; return false; }
     if (hipMemset(att_counters_, 0, 64 * ATT_SYNC_STRIDE * sizeof(unsigned)) != hipSuccess) { err = "hipMemset failed"; return false; }
@@ -1617,6 +1620,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             // extra workgroup would scan the whole cell table)
             aa.pf_splits = cols ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(T, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
             while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
+            if (!cols && flash_attn_prefill_planes_pay(T, H, G, n_kv_max, cur_max_pos_ + 1)) aa.pf_planes = att_planes_;
             HIP_TRY(cols ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_));
         }
         prof_mark("attn");
