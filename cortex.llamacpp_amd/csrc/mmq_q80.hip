@@ -42,64 +42,70 @@ template <> struct Tile<16> {
     __device__ static Floats outer(f16x4 x, f16x4 w, const Floats &z) { return __builtin_amdgcn_mfma_f32_16x16x16f16(x, w, z, 0, 0, 0); }
 };
 
-// Rows come in steps of 128 bytes, four blocks.  A lane that reads its own row from memory costs the CU's address unit a clock a lane, and in the matrix unit's layout every lane is another
-// line: a row of 64 blocks took 20 us however few the tiles (2048 x 2048, 40 tokens; its products are 5).  So a wave instruction brings eight rows' 128 bytes into LDS - S steps of them in
+// Rows come in steps of U blocks, 128 or 256 bytes.  A lane that reads its own row from memory costs the CU's address unit a clock a lane, and in the matrix unit's layout every lane is another
+// line: a row of 64 blocks took 20 us however few the tiles (2048 x 2048, 40 tokens; its products are 5).  So a wave instruction brings eight (four) rows' steps into LDS - S of them in
 // turn, the 16-byte pieces of row i in the order p ^ (i & 7), so that the matrix unit's reads meet no bank twice -, and the four waves share both operands.  The scales come the same way, and
 // their products from the matrix unit too: one f16 contraction of which all elements but one are zero IS d_w * d_a of every output, exactly (22 bits in f32, subnormals kept), in place of a
 // vector instruction a result.  What is left to the vector unit is convert (or subtract), multiply, add - the CPU's three roundings an output and block in the CPU's order -: 48 instructions a 32 x 32
-// tile and block, its bound (5632 x 2048, 2000 tokens: 63 us of 102).
-// Wave = W x W tiles of SZ x SZ, workgroup = 2 x 2 waves.  us, 40 / 611 / 2000 tokens, this | every lane its own row, scales from LDS: 2048 x 2048 8 / 17 / 42 | 21 / 35 / 61, 5632 x 2048
-// 11 / 37 / 102 | 22 / 60 / 151, 4096 x 14336 43 / 156 / 448 | 133 / 349 / 582, 1024 x 4096 13 / 22 / 37 | 38 / 38 / 69.
+// tile and block, its bound (5632 x 2048, 2000 tokens: 63 us of 97).
+// Wave = W x W tiles of SZ x SZ, workgroup = 2 x 2 waves.  Tiles of 16 take steps of eight blocks: what they wait for is a barrier and two LDS reads a step (four / eight, 40 tokens:
+// 2048 x 2048 7.3 / 6.5, 2048 x 5632 16.8 / 14.6, 4096 x 14336 41 / 35; tiles of 32 the same either way).
+// us, 40 / 611 / 2000 tokens, this | every lane its own row, scales from LDS: 2048 x 2048 6.5 / 17 / 39 | 21 / 35 / 61, 5632 x 2048 9.6 / 35 / 97 | 22 / 60 / 151, 4096 x 14336
+// 35 / 152 / 415 | 133 / 349 / 582, 1024 x 4096 10.6 / 22 / 37 | 38 / 38 / 69.
 // (Tried: rows straight from memory in tiles of 16, or two to four steps ahead: the same 20 us.  The products of the next tile asked for before the fold of this one: nothing.)
-template <int SZ, int W, int S>
+template <int SZ, int W, int S, int U>
 __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) {
     using TL = Tile<SZ>;
     using Codes = typename TL::Codes;
-    constexpr int ROWS = 2 * SZ * W, STEP = 256 * ROWS, SCALES = 16 * ROWS, STAGE = STEP + SCALES;   // rows of either operand; 128 B of codes and 8 of scales a row
-    constexpr int NR = SZ * SZ / 64, NC = ROWS / 32, NS = SCALES >= 1024 ? SCALES / 1024 : 1, LOADS = 2 * NC + NS;
+    // rows of either operand, 32 U B of codes and 2 U of scales each; a scale request brings SQ rows'
+    constexpr int ROWS = 2 * SZ * W, RB = 32 * U, PIECES = 2 * U, STEP = 2 * RB * ROWS, SB = 2 * U, SQ = U == 4 ? 32 : 64, SOP = (ROWS + SQ - 1) / SQ * SQ * SB, STAGE = STEP + 2 * SOP;
+    constexpr int NR = SZ * SZ / 64, NC = ROWS * RB / 4096, SR = (ROWS + SQ - 1) / SQ, NS = SR > 2 ? SR / 2 : 1, LOADS = 2 * NC + NS;
     __shared__ __attribute__((aligned(1024))) uint8_t sm[S * STAGE];
     int sg = 0;
     if (a.n_seg > 1 && (int)blockIdx.x >= a.tile0[1]) sg = 1;
     if (a.n_seg > 2 && (int)blockIdx.x >= a.tile0[2]) sg = 2;
-    const int n_rows = a.n_rows[sg], K = a.K, T = a.T, nb = K >> 5, steps = nb >> 2;
+    const int n_rows = a.n_rows[sg], K = a.K, T = a.T, nb = K >> 5, steps = nb / U;
     const int l = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), n = l & (SZ - 1), kg = l / SZ;
     const int t0 = blockIdx.y * ROWS, r0 = ((int)blockIdx.x - a.tile0[sg]) * ROWS;
     const int last_r = (n_rows - r0 < ROWS ? n_rows - r0 : ROWS) - 1, last_t = (T - t0 < ROWS ? T - t0 : ROWS) - 1;
     const uint8_t *const wbase = (const uint8_t *)uniform_ptr(a.W[sg] + (size_t)r0 * a.row_bytes);
     const uint8_t *const xbase = (const uint8_t *)uniform_ptr(a.aq + (size_t)t0 * K), *const dbase = (const uint8_t *)uniform_ptr(a.ad + (size_t)t0 * nb);
-    // a request: eight rows' 128 B of codes, the 16-byte pieces of row i in the order p ^ (i & 7); or 32 rows' 8 B of scales
+    // a request: 1 KB of codes, the 16-byte pieces of row i in the order p ^ (i & 7); or SQ rows' scales
     unsigned woff[NC], xoff[NC], soff[NS];
-    const unsigned piece = 16u * ((l & 7) ^ (l >> 3));
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        const int r = (wave + 4 * i) * 8 + (l >> 3);
+        const int r = (wave + 4 * i) * (1024 / RB) + l / PIECES;
+        const unsigned piece = 16u * ((l % PIECES) ^ (r & 7));
         woff[i] = (unsigned)(r < last_r ? r : last_r) * (unsigned)a.row_bytes + piece;
         xoff[i] = (unsigned)(r < last_t ? r : last_t) * (unsigned)K + piece;
     }
-    constexpr int SR = ROWS / 32;                                      // scale requests an operand
     bool sw[NS];
     unsigned sto[NS];
 #pragma unroll
     for (int i = 0; i < NS; i++) {
-        const int q = (wave + 4 * i) % (2 * SR), r = (q % SR) * 32 + (l >> 1);
+        const int q = (wave + 4 * i) % (2 * SR), r = (q % SR) * SQ + (U == 4 ? l >> 1 : l);
+        const unsigned half = U == 4 ? 4u * (l & 1) : 0u;
         sw[i] = q < SR;
-        sto[i] = STEP + q * 256;
-        soff[i] = sw[i] ? (unsigned)(r < last_r ? r : last_r) * (unsigned)a.row_bytes + (unsigned)K + 4u * (l & 1) : (unsigned)(r < last_t ? r : last_t) * (unsigned)nb * 2u + 4u * (l & 1);
+        sto[i] = STEP + q * (SQ * SB);
+        soff[i] = sw[i] ? (unsigned)(r < last_r ? r : last_r) * (unsigned)a.row_bytes + (unsigned)K + half : (unsigned)(r < last_t ? r : last_t) * (unsigned)nb * 2u + half;
     }
     const unsigned lds = __builtin_amdgcn_readfirstlane((int)(unsigned)(uintptr_t)sm);
     const auto ask = [&](int step, int buf) {
         const int s = step < steps ? step : steps - 1;                 // (past the end: the last again, never read)
         const unsigned to = lds + buf * STAGE;
 #pragma unroll
-        for (int i = 0; i < NC; i++) lds_dma16(wbase + (size_t)s * 128, woff[i], to + (wave + 4 * i) * 1024);
+        for (int i = 0; i < NC; i++) lds_dma16(wbase + (size_t)s * RB, woff[i], to + (wave + 4 * i) * 1024);
 #pragma unroll
-        for (int i = 0; i < NC; i++) lds_dma16(xbase + (size_t)s * 128, xoff[i], to + STEP / 2 + (wave + 4 * i) * 1024);
+        for (int i = 0; i < NC; i++) lds_dma16(xbase + (size_t)s * RB, xoff[i], to + STEP / 2 + (wave + 4 * i) * 1024);
 #pragma unroll
-        for (int i = 0; i < NS; i++) lds_dma4((sw[i] ? wbase : dbase) + (size_t)s * 8, soff[i], to + sto[i]);
+        for (int i = 0; i < NS; i++) {
+            if constexpr (U == 4) lds_dma4((sw[i] ? wbase : dbase) + (size_t)s * SB, soff[i], to + sto[i]);
+            else lds_dma16((sw[i] ? wbase : dbase) + (size_t)s * SB, soff[i], to + sto[i]);
+        }
     };
     const int wr = (wave & 1) * SZ * W, wt = (wave >> 1) * SZ * W;     // the wave's tiles in the workgroup's
     const uint32_t first = kg == 0 ? 0x0000ffffu : 0u, second = kg == 0 ? 0xffff0000u : 0u;
-    const auto one = [&](const u32x2 &d, int u) { return __builtin_bit_cast(f16x4, u32x2{d[u >> 1] & ((u & 1) ? second : first), 0u}); };
+    const auto one = [&](const auto &d, int u) { return __builtin_bit_cast(f16x4, u32x2{d[u >> 1] & ((u & 1) ? second : first), 0u}); };
     float acc[W][W][NR];
 #pragma unroll
     for (int i = 0; i < W; i++)
@@ -107,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
         for (int j = 0; j < W; j++)
 #pragma unroll
             for (int r = 0; r < NR; r++) acc[i][j][r] = 0.0f;
-    // (with the bias as the sums' start a subtraction converts them: 4096 x 14336 at 40 tokens, tiles of 16, 44 -> 41 us, at 2000, four of 32 a wave, 430 -> 415; one of 32 a wave is 4 % slower for it)
+    // (with the bias as the sums' start a subtraction converts them: 4096 x 14336 at 40 tokens, tiles of 16 in steps of four blocks, 44 -> 41 us, at 2000, four of 32 a wave, 430 -> 415; one of 32 a wave is 4 % slower for it)
     constexpr bool BIAS = SZ == 16 || W == 2;
     const typename TL::Ints zi = (typename TL::Ints)(BIAS ? INT_BIAS : 0);
     const typename TL::Floats zf = {};
@@ -119,15 +125,16 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
         ask(step + S - 1, buf ? buf - 1 : S - 1);
         const uint8_t *const at = sm + buf * STAGE;
         buf = buf + 1 < S ? buf + 1 : 0;
-        u32x2 dw[W], da[W];
+        typedef unsigned int scales __attribute__((ext_vector_type(U / 2)));
+        scales dw[W], da[W];
 #pragma unroll
         for (int i = 0; i < W; i++) {
-            dw[i] = *reinterpret_cast<const u32x2 *>(at + STEP + (wr + SZ * i + n) * 8);
-            da[i] = *reinterpret_cast<const u32x2 *>(at + STEP + SCALES / 2 + (wt + SZ * i + n) * 8);
+            dw[i] = *reinterpret_cast<const scales *>(at + STEP + (wr + SZ * i + n) * SB);
+            da[i] = *reinterpret_cast<const scales *>(at + STEP + SOP + (wt + SZ * i + n) * SB);
         }
         const auto codes = [&](const uint8_t *op, int row, int u) {
-            if constexpr (SZ == 32) return *reinterpret_cast<const Codes *>(op + row * 128 + (((2 * u + kg) ^ (n & 7)) * 16));
-            else return *reinterpret_cast<const Codes *>(op + row * 128 + (((2 * u + (kg >> 1)) ^ (n & 7)) * 16) + (kg & 1) * 8);
+            if constexpr (SZ == 32) return *reinterpret_cast<const Codes *>(op + row * RB + (((2 * u + kg) ^ (n & 7)) * 16));
+            else return *reinterpret_cast<const Codes *>(op + row * RB + (((2 * u + (kg >> 1)) ^ (n & 7)) * 16) + (kg & 1) * 8);
         };
         Codes w[2][W], x[2][W];
         const auto read = [&](int u) {
@@ -136,8 +143,8 @@ __global__ __launch_bounds__(256, 2) void mmq_q80_tiles_kernel(const Q80Args a) 
         };
         read(0);
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (u + 1 < 4) read(u + 1);
+        for (int u = 0; u < U; u++) {
+            if (u + 1 < U) read(u + 1);
 #pragma unroll
             for (int i = 0; i < W; i++)
 #pragma unroll
@@ -215,16 +222,16 @@ hipError_t launch_expand_q80_copy(int type, const uint8_t *W, size_t row_bytes, 
     return hipGetLastError();
 }
 
-// The mat-vec takes one, two or four tokens to a pass over the weights; everything between goes here (us of a batch, mat-vec | tiles, 2 / 3 / 4 / 5 / 16 / 31 tokens: six TinyLlama-1.1B
-// Q8_0 layers 387 553 452 617 1057 2137 | 466 466 466 466 470 487, four 8B ones 507 722 672 891 1568 3291 | 635 626 629 629 644 671; as Q4_0 with the copy above 464 - 654 - 1648 3320 |
-// 625 - 620 - 623 646).
-bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && (T == 3 || T >= 5) && K >= 128 && (K % 128) == 0 && K <= 16384; }
+// The mat-vec takes one, two or four tokens to a pass over the weights; from three on they go here (us of a batch, mat-vec | tiles, 3 / 4 / 5 / 16 / 31 tokens: six TinyLlama-1.1B Q8_0 layers
+// 533 444 604 1056 2138 | 422 428 426 434 451, four 8B ones 723 671 888 1571 3294 | 583 577 577 590 614, as Q4_0 with the copy above 615 655 - 1651 3327 | 571 569 - 570 598; two tokens,
+// in steps of four blocks, 387 | 466).
+bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && T >= 3 && K >= 256 && (K % 256) == 0 && K <= 16384; }
 
-template <int SZ, int W, int S> static void tiles_launch(Q80Args &a, hipStream_t st) {
+template <int SZ, int W, int S, int U> static void tiles_launch(Q80Args &a, hipStream_t st) {
     constexpr int R = 2 * SZ * W;
     int tiles = 0;
     for (int i = 0; i < a.n_seg; i++) { a.tile0[i] = tiles; tiles += (a.n_rows[i] + R - 1) / R; }
-    hipLaunchKernelGGL((mmq_q80_tiles_kernel<SZ, W, S>), dim3((unsigned)tiles, (unsigned)((a.T + R - 1) / R)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((mmq_q80_tiles_kernel<SZ, W, S, U>), dim3((unsigned)tiles, (unsigned)((a.T + R - 1) / R)), dim3(256), 0, st, a);
 }
 
 hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st) {
@@ -239,14 +246,14 @@ hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const Act
         return c * ((T + r - 1) / r);
     };
     for (int i = 0; i < n; i++) { a.W[i] = sg[i].W; a.out[i] = sg[i].out; a.n_rows[i] = sg[i].n_rows; a.ld_out[i] = sg[i].ld_out; }
-    // Up to two 32 x 32 workgroups a CU it is one wave's way through its row that counts, a third shorter in tiles of 16 (us, 16 | 32: 5632 x 2048, 40 tokens = 352 workgroups 11.0 | 12.9;
-    // 4096 x 14336, 100 = 512 56 | 74; 2048 x 2048, 320 = 640 13.8 | 12.8).  Four tiles of 32 a wave read half as much of LDS, but need 1.7 workgroups of 128 x 128 a CU and no more
-    // than a tenth more padding (us, one tile | four: 5632 x 2048, 1200 tokens = 440 workgroups 69 | 65; 4096 x 14336, 2000 = 512 490 | 448, 1200 = 320 292 | 335;
+    // Up to two 32 x 32 workgroups a CU it is one wave's way through its row that counts, half as long in tiles of 16 (us, 16 | 32: 5632 x 2048, 40 tokens = 352 workgroups 9.6 | 12.9;
+    // 4096 x 14336, 100 = 512 48 | 74; 2048 x 2048, 320 = 640 13.1 | 13.0; 5632 x 2048, 100 = 704 14.1 | 13.3).  Four tiles of 32 a wave read half as much of LDS, but need 1.7 workgroups of 128 x 128 a CU and no more
+    // than a tenth more padding (us, one tile | four: 5632 x 2048, 1200 tokens = 440 workgroups 66 | 64; 4096 x 14336, 2000 = 512 470 | 415, 1200 = 320 283 | 330;
     // 32000 x 2048, 320 = 750, a fifth more padding 92 | 100).
     const long c32 = count(32), c64 = count(64), c128 = count(128);
-    if (c32 <= 2L * num_cu()) tiles_launch<16, 1, 4>(a, st);
-    else if (c128 * 10 >= 17L * num_cu() && c128 * 40 <= c64 * 11) tiles_launch<32, 2, 2>(a, st);
-    else tiles_launch<32, 1, 3>(a, st);
+    if (c32 <= 2L * num_cu()) tiles_launch<16, 1, 3, 8>(a, st);
+    else if (c128 * 10 >= 17L * num_cu() && c128 * 40 <= c64 * 11) tiles_launch<32, 2, 2, 4>(a, st);
+    else tiles_launch<32, 1, 3, 4>(a, st);
     return hipGetLastError();
 }
 
