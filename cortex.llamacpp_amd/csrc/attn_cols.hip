@@ -503,6 +503,8 @@ bool flash_attn_cols_applicable(const AttnArgs &a) {
 //                               512 / 3400 169 / 161
 //   32 / 32 heads of 128, f16   256 / 2000 53 / 63, 300 / 2000 85 / 103, 512 / 0 28 / 41, 512 / 1000 67 / 69, 512 / 1500 86 / 83, 400 / 2500 113 / 101, 450 / 1500 82 / 77, 512 / 2500 122 / 109
 //   32 / 4 heads of 64, f16     256 / 0 8 / 24, 768 / 1200 66 / 80, 850 / 0 44 / 45, 1024 / 0 51 / 50, 1024 / 900 86 / 75      12 / 12 heads of 64, f16 (a text)   187 6.6 / 17, 2000 58 / 92
+// (These are the prompt kernel's with every tile converting V for itself.  With the planes made once a layer it is ahead at 512 / 1000 and 512 / 1400 q8_0 by 8 and 10 us a layer and at 450 / 3400 by
+// 4, behind at 512 / 0, 350 / 3500, 256 / 2000 by 10, 10 and 7 and at 300 / 2000 f16 by 20: one to two hundredths of a pass on either side of a line, which stays.)
 // So with heads of 64 three rounds of workgroups; with heads of 128 two as long as the keys are few, to 1536 cells with a query head to every kv head and to 2048 else, and with more keys
 // 11 / 8 and 15 / 8 rounds.
 static bool cols_long(const AttnArgs &a) {
