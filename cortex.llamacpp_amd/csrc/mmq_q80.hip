@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void expand_nib32_q80_kernel(int type, const u
     }
 }
 size_t mmq_q80_copy_bytes(int type, int64_t n_rows, int K) {
-    if ((type != T_Q4_0 && type != T_Q5_0 && type != T_IQ4_NL) || (K % 32) != 0 || K > 16384) return 0;
+    if ((type != T_Q4_0 && type != T_Q5_0 && type != T_IQ4_NL) || (K % 32) != 0 || K > 65536) return 0;
     return (size_t)n_rows * dev_row_bytes(T_Q8_0, K);
 }
 hipError_t launch_expand_q80_copy(int type, const uint8_t *W, size_t row_bytes, int n_rows, int K, uint8_t *dst, hipStream_t st) {
@@ -225,7 +225,9 @@ hipError_t launch_expand_q80_copy(int type, const uint8_t *W, size_t row_bytes, 
 // The mat-vec takes one, two or four tokens to a pass over the weights; from three on they go here (us of a batch, mat-vec | tiles, 3 / 4 / 5 / 16 / 31 tokens: six TinyLlama-1.1B Q8_0 layers
 // 533 444 604 1056 2138 | 422 428 426 434 451, four 8B ones 723 671 888 1571 3294 | 583 577 577 590 614, as Q4_0 with the copy above 615 655 - 1651 3327 | 571 569 - 570 598; two tokens,
 // in steps of four blocks, 387 | 466).
-bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && T >= 3 && K >= 256 && (K % 256) == 0 && K <= 16384; }
+// Rows of any length that 32-bit offsets within a workgroup's 128 allow, by far (28672 columns left to the mat-vec: two 70B layers of Q8_0 at 5, 40 and 512 tokens 1264, 3008, 23941 us; here
+// 762, 900, 3449).
+bool mmq_q80_applicable(int type, int K, int T) { return type == T_Q8_0 && T >= 3 && K >= 256 && (K % 256) == 0 && K <= 65536; }
 
 template <int SZ, int W, int S, int U> static void tiles_launch(Q80Args &a, hipStream_t st) {
     constexpr int R = 2 * SZ * W;

@@ -19,7 +19,7 @@ def scaled(rng, W, N, K):
     return W
 
 
-@pytest.mark.parametrize("K,N,T", [(256, 1, 3), (512, 40, 5), (768, 65, 16), (256, 1, 32), (256, 33, 33), (768, 40, 63), (2048, 130, 47), (5632, 70, 40),   # 16 x 16 tiles: fewer steps than buffers, ragged rows and tokens
+@pytest.mark.parametrize("K,N,T", [(256, 1, 3), (512, 40, 5), (768, 65, 16), (256, 1, 32), (256, 33, 33), (768, 40, 63), (2048, 130, 47), (5632, 70, 40), (28672, 40, 35),   # 16 x 16 tiles: fewer steps than buffers, ragged rows and tokens
                                    (256, 2049, 257), (768, 1100, 513), (2048, 2000, 323),                           # one 32 x 32 tile a wave
                                    (256, 14000, 513), (768, 8193, 897)])                                            # four
 def test_q80_tiles_bit_exact(be, K, N, T):  # noqa: F811
