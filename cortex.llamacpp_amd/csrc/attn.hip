@@ -1120,10 +1120,10 @@ static hipError_t launch_fa_v16(const AttnArgs &a, hipStream_t st) {
     return hipSuccess;
 }
 
-hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st) {
+hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st, void *planes) {
     if (fa_v_acc_f16_enabled() && a.type_k == T_F16 && a.type_v == T_F16) return launch_fa_v16(a, st);
     static const bool mfma_prefill = !(getenv("MI355_ATTN_PREFILL_MFMA") && getenv("MI355_ATTN_PREFILL_MFMA")[0] == '0');
-    if (mfma_prefill && flash_attn_prefill_applicable(a)) return launch_flash_attn_prefill(a, st);   // prompt processing: matrix cores
+    if (mfma_prefill && flash_attn_prefill_applicable(a)) return launch_flash_attn_prefill(a, st, planes);   // prompt processing: matrix cores
     const int R = a.H / a.G;
     hipError_t e = hipErrorInvalidValue;
     if ((size_t)a.splits * ATT_MAX_CHUNK < (size_t)a.n_kv_max) return hipErrorInvalidValue;

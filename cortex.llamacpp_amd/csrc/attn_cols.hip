@@ -64,6 +64,7 @@ struct ColsArgs {
     float scale_l2;                                          // EXACT: the scores' scale in log2 units, rounded once
     const int32_t *list;                                     // 64-cell chunks to walk (two of 32 each); nullptr: all of [0, n_chunks)
 };
+static_assert(sizeof(ColsArgs) == 288, "eight bytes more in AttnArgs: 0.2 us a launch at 187 tokens of 12 heads, 0.8 at 65 of 32 / 4");
 
 // EXACT: the products of weights and values as f32 has them (three f16 parts of a weight, a q8_0 value of any size); else as attn_prefill.hip has them
 template <bool F16, int DH, int NW, bool EXACT>

@@ -83,7 +83,7 @@ static size_t plane_chunk_bytes(bool f16, int D) { return (size_t)D * CK * (f16 
 // The V planes of a prompt batch, once for all its query tiles: workgroup = (chunk, kv head), in the order the matrix cores take them (Chunk's vh and, for a q8_0 cache, vl: V' = code * d_v
 // split exactly in two halves).  4096 cells of eight kv heads, q8_0: 17 MB, 6 us - where every tile converted every chunk it walked, for 3.1 of a chunk's 7.8 kilocycles.
 template <bool F16, int DH>
-__global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a, void *planes) {
     constexpr int NB = DH / 32;
     using PC = PlaneChunk<F16, DH>;
     __shared__ __attribute__((aligned(16))) _Float16 sm[PC::VBYTES / 2];
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a
         }
     }
     __syncthreads();
-    u32x4 *const out = reinterpret_cast<u32x4 *>(reinterpret_cast<uint8_t *>(a.pf_planes) + ((size_t)g * ((n_ctx + CK - 1) / CK) + c) * PC::VBYTES);
+    u32x4 *const out = reinterpret_cast<u32x4 *>(reinterpret_cast<uint8_t *>(planes) + ((size_t)g * ((n_ctx + CK - 1) / CK) + c) * PC::VBYTES);
     for (int i = threadIdx.x; i < PC::VBYTES / 16; i += 256) out[i] = reinterpret_cast<const u32x4 *>(sm)[i];
 }
 
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a
 // it (probe, 32 / 8 heads of 128, q8_0; 1919 tokens behind 2048: 382 -> 276 us, 2048 behind none 174 -> 134).  The block scales' products come from the matrix unit.  The same bits.
 // (Tried: one of a SIMD's two waves half a chunk behind, its P.V beside the other's scores, in a third buffer: nothing.  Integer sums that start at the f32 bias: nothing.)
 template <int R, bool F16, int KH, int QS, int DH = 128, bool Q4 = false, bool PL = false>
-__global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel(const AttnArgs a, const void *planes) {
     // head width: 128 or 64 (TinyLlama, Llama-3.2-1B, nomic-embed): everything below is written in 32-dim blocks (NB of them) and 16-dim matrix-core steps
     constexpr int D = DH, NB = DH / 32, K_STRIDE = DH + 16, KF_STRIDE = 2 * DH + 16, NKS = DH / 16, VPL = NB * 2 * 2 * 32 * 8, NVU = 2 * DH;
 #ifdef MI355_FA_PROBE
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
     unsigned kr[KI] = {}, krow_last = 0;
     if constexpr (PL) {
         kbase = uniform_ptr(a.kv.k + head_row0 * PC::ROW);
-        vbase = uniform_ptr(reinterpret_cast<const uint8_t *>(a.pf_planes) + (size_t)g * ((n_ctx + CK - 1) / CK) * PC::VBYTES);
+        vbase = uniform_ptr(reinterpret_cast<const uint8_t *>(planes) + (size_t)g * ((n_ctx + CK - 1) / CK) * PC::VBYTES);
         sbase = F16 ? nullptr : uniform_ptr(a.kv.kd + head_row0 * NB);
         pbase = uniform_ptr(a.cell_pos); qbase = uniform_ptr(a.cell_seq);
         krow_last = (unsigned)(n_ctx - 1);                     // (cells past the table's end: the last one's, never visible)
@@ -789,10 +789,10 @@ bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible) {
     return (long)tiles * std::min(n_kv, visible) >= 8L * n_kv;
 }
 
-hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st) {
+hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *v_planes) {
     const int R = a.H / a.G, kh = fa_key_halves(R), qs = fa_sub_tiles(R);
     const int nsp = (a.pf_splits > 1 && a.part) ? a.pf_splits : 1;
-    const bool planes = a.pf_planes && flash_attn_prefill_planes_bytes(a.type_k, a.type_v, a.D, a.G, a.n_ctx) && kh == (R <= 4 ? 2 : 1) && qs == (R == 1 ? 4 : R == 2 ? 2 : 1);
+    const bool planes = v_planes && flash_attn_prefill_planes_bytes(a.type_k, a.type_v, a.D, a.G, a.n_ctx) && kh == (R <= 4 ? 2 : 1) && qs == (R == 1 ? 4 : R == 2 ? 2 : 1);
     const dim3 grid((unsigned)a.G, (unsigned)((a.T + QT * qs - 1) / (QT * qs)), (unsigned)nsp);
     const bool f16 = a.type_k == T_F16;
     const int nb = a.D / 32;
@@ -801,12 +801,12 @@ hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st) {
     const size_t lds = kh == 2 ? std::max(4 * (planes ? pchunk : chunk), (size_t)R * qs * (16 * nb + 2) * 64 * 4) : 2 * (planes ? pchunk : chunk);   // two chunk buffers per half, later the hand-over of the second half
     if (planes) {
         const dim3 pg((unsigned)((std::min(a.n_kv_max, a.n_ctx) + CK - 1) / CK), (unsigned)a.G);
-#define FAPL(F, DD) hipLaunchKernelGGL((flash_attn_planes_kernel<F, DD>), pg, dim3(256), 0, st, a)
+#define FAPL(F, DD) hipLaunchKernelGGL((flash_attn_planes_kernel<F, DD>), pg, dim3(256), 0, st, a, v_planes)
         if (f16) { if (a.D == 128) FAPL(true, 128); else FAPL(true, 64); }
         else { if (a.D == 128) FAPL(false, 128); else FAPL(false, 64); }
 #undef FAPL
 #define FAPP(RR, F, KK, QQ, DD) do { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, F, KK, QQ, DD, false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-                                     hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, F, KK, QQ, DD, false, true>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } while (0)
+                                     hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, F, KK, QQ, DD, false, true>), grid, dim3(64 * RR * KK * QQ), lds, st, a, v_planes); } while (0)
 #define FAPT(RR, KK, QQ, DD) do { if (f16) FAPP(RR, true, KK, QQ, DD); else FAPP(RR, false, KK, QQ, DD); } while (0)
         if (a.D == 64) switch (R) {
             case 1: FAPT(1, 2, 4, 64); break;
@@ -830,12 +830,12 @@ hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st) {
     } else
 #define FAP_D(RR, KK, QQ, DD) do { \
         if (f16) { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, true, KK, QQ, DD>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-                   hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, true, KK, QQ, DD>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } \
+                   hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, true, KK, QQ, DD>), grid, dim3(64 * RR * KK * QQ), lds, st, a, v_planes); } \
         else { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, false, KK, QQ, DD>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-               hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, false, KK, QQ, DD>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } } while (0)
+               hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, false, KK, QQ, DD>), grid, dim3(64 * RR * KK * QQ), lds, st, a, v_planes); } } while (0)
 #define FAP(RR, KK, QQ) FAP_D(RR, KK, QQ, 128)
 #define FAP_Q4(RR, KK, QQ) do { if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&flash_attn_prefill_kernel<RR, false, KK, QQ, 128, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-                                hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, false, KK, QQ, 128, true>), grid, dim3(64 * RR * KK * QQ), lds, st, a); } while (0)
+                                hipLaunchKernelGGL((flash_attn_prefill_kernel<RR, false, KK, QQ, 128, true>), grid, dim3(64 * RR * KK * QQ), lds, st, a, v_planes); } while (0)
     if (a.type_k == T_Q4_0) {                                   // head_dim 128, the default wave arrangement of the power-of-two head ratios
         if (R == 1 && kh == 2 && qs == 4) FAP_Q4(1, 2, 4);
         else if (R == 2 && kh == 2 && qs == 2) FAP_Q4(2, 2, 2);

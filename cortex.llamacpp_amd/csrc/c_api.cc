@@ -793,12 +793,11 @@ int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t
     DevBuf part(flash_attn_workspace_floats((int)T, H, D, std::max(a.splits, a.pf_splits)) * 4);
     a.part = part.as<float>();
     DevBuf planes(g_op_attn_planes ? flash_attn_prefill_planes_bytes(type_k, type_v, D, G, n_cells) : 0);
-    a.pf_planes = g_op_attn_planes ? planes.as<void>() : nullptr;
     const bool cols = g_op_attn_cols > 0;
     if (cols && !flash_attn_cols_applicable(a)) { fail("attn_cols: no form for this call"); return MI355_ERR_ARG; }
     DevBuf cpart(cols ? flash_attn_workspace_floats((int)T, H, D, g_op_attn_cols) * 4 : 16);
     if (cols) { a.part = cpart.as<float>(); a.pf_splits = g_op_attn_cols; }
-    hipError_t e = cols ? launch_flash_attn_cols(a, nullptr) : launch_flash_attn(a, nullptr);
+    hipError_t e = cols ? launch_flash_attn_cols(a, nullptr) : launch_flash_attn(a, nullptr, g_op_attn_planes ? planes.as<void>() : nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) return hip_fail(e, "flash_attn");
     return dout.down(out, (size_t)T * H * D * 4) ? MI355_OK : MI355_ERR_HIP;

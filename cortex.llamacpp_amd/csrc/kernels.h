@@ -659,16 +659,17 @@ struct AttnArgs {
     // a batch of one sequence: the 64-cell chunks that hold its cells; nullptr = every chunk of the scanned range
     const int32_t *chunks = nullptr;
     int n_chunks = 0;
-    void *pf_planes = nullptr; // prompt kernel (attn_prefill.hip), nullable: flash_attn_prefill_planes_bytes() for the V planes of the scanned cells, made once for all query tiles
 };
-hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st);
+// planes: for launch_flash_attn_prefill.  (A field of AttnArgs it moved what ColsArgs holds behind them: attn_cols.hip 6.7 -> 6.95 us a launch at 187 tokens of 12 heads, 7.9 -> 8.7 at 65 of 32 / 4)
+hipError_t launch_flash_attn(const AttnArgs &a, hipStream_t st, void *planes = nullptr);
 // parity mode for an f16 K / V cache: the reference CPU path's cell-by-cell arithmetic with V accumulated in fp16 (attn.hip); 1 / 0, -1 = MI355_FA_V_ACC=f16
 void set_fa_v_acc_f16(int on);
 bool fa_v_acc_f16_enabled();
 // prompt processing on the matrix cores (attn_prefill.hip): D = 128, q8_0 K / V, T >= 32; q already rotated
 bool flash_attn_prefill_applicable(const AttnArgs &a);
 int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max);
-hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st);
+// planes (nullable): flash_attn_prefill_planes_bytes() for the V planes of the scanned cells, made once for all query tiles
+hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *planes = nullptr);
 size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int D, int G, int n_ctx);      // of a cache; 0: no such form, or more than 256 MiB
 bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible);               // n_kv cells scanned, of which a query can see at most `visible`
 // a short batch of one sequence, a short text through the encoder: the same in another split of the work (attn_cols.hip); pf_splits = flash_attn_cols_splits

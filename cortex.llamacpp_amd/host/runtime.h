@@ -302,7 +302,7 @@ class Context {
     bool batch_distinct_ = false;                    // the micro-batch is one token each of different sequences (decode_ubatch)
     const int8_t *bh_over_ = nullptr, *bl_over_ = nullptr;   // linear(): block-sum planes prepared by the caller for a slice of a larger batch
     float *att_part_ = nullptr;
-    void *att_planes_ = nullptr;        // a prompt batch's V planes (AttnArgs::pf_planes); null: no such form
+    void *att_planes_ = nullptr;        // a prompt batch's V planes (launch_flash_attn); null: no such form
     size_t att_part_floats_ = 0;
     bool attn_cols_ = false;                         // the micro-batch being decoded is of one sequence and goes through attn_cols.hip; its chunk list is the first
     int cur_max_pos_ = 0;                            // largest position of the micro-batch being decoded
