@@ -1584,27 +1584,30 @@ bool mmq_ksplit_applicable(int type, int K, int T) {
 static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool *takes);
 // Which kernel takes a launch of 65 .. 256 tokens is a matter of shape (to 64 tokens mmq_few_takes chooses): this one, or the 128 x 256 tiles, K split over the workgroups where the
 // workspace allows it.  The choice is by the two launches' times.  Both are whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us): K-split, 32 rows x 64
-// tokens, an eighth of the super-blocks of 5.2 and 3.5; tiles, the part's super-blocks of 1.5 + T / 128 and 7, and 4 more where the parts' sum is a launch of its own.
-// Measured with weights from HBM, Q4_K, K-split / tiles without the sum's launch, at 72, 128 and 256 tokens (Q5_K and Q6_K cost either kernel a tenth more):
+// tokens, an eighth of the super-blocks of 5.2 and 3.5; tiles, the part's super-blocks of 1.5 + T / 128, to 128 tokens of Q6_K, which they read as two bytes a weight, 2 + T / 128, and 7, and 4
+// more where the parts' sum is a launch of its own.
+// Measured with weights from HBM, Q4_K, K-split / tiles without the sum's launch, at 72, 128 and 256 tokens (Q5_K costs either kernel a tenth more):
 //   2048 x 2048   9/13 9/15 10/18     2048 x 5632  18/18 19/20 20/24    1536 x 8960   23/23 27/27 26/34     gate | up of 5632 x 2048    25/24 25/27 44/32
 //   3072 x 3072  11/14 12/16 19/19    3072 x 8192  24/22 24/25 43/31    5120 x 5120   28/17 28/19 42/24     gate | up of 8192 x 3072    40/32 41/37 74/44
 //   4096 x 4096  15/15 15/16 26/20    6144 x 4096  25/15 25/17 37/21    4096 x 14336  40/35 40/40 72/50     gate | up of 14336 x 4096   89/43 91/49 166/61
+// Q6_K at 65, 96 and 128 tokens:  2048 x 5632  20/21 20/21 20/23    4096 x 14336  46/45 43/45 43/47    3584 x 18944  55/55 53/57 54/59    6144 x 4096  27/19 27/20 27/21
+//   gate | up of 5632 x 2048  25/28 25/28 25/30    of 8192 x 3072  43/41 43/41 44/43    of 14336 x 4096  101/58 95/56 96/61
 // (tiles of planes, before Q4_K came as codes: gate | up of 14336 x 4096 at 130 tokens 70, 6144 x 4096 25.)  Whole prompts of eight layers of an 8B model, us, K-split to 128 tokens and now:
 // 65 tokens 1624, 1083; 96 1672, 1128; 128 1727, 1227.
-static bool tiles_beat_ksplit(int n_rows, int K, int T, MMQWorkspace wsp, bool pair, bool sum_free) {
+static bool tiles_beat_ksplit(int type, int n_rows, int K, int T, MMQWorkspace wsp, bool pair, bool sum_free) {
     bool takes = false;
     const int rows = pair ? 2 * n_rows : n_rows, parts = planes2_split(rows, K, T, pair ? MMQWorkspace() : wsp, &takes), nb = K >> 8;
     if (!takes) return n_rows >= 8192 && !(pair && T <= 128);  // (then the planes kernel below, by rows; ffn_gate | ffn_up are one launch here and two there)
     const auto up = [](long a, long b) { return (double)((a + b - 1) / b); };
     const double here = up(up(rows, 32) * up(T, 64), num_cu()) * (5.2 * nb / 8 + 3.5);
-    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * ((1.5 + T / 128.0) * up(nb, parts) + 7.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
+    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * (((type == T_Q6_K && T <= 128 ? 2.0 : 1.5) + T / 128.0) * up(nb, parts) + 7.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
     return tiles < here;
 }
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair) {
     static const int env = getenv("MI355_KSPLIT_SHAPE") ? atoi(getenv("MI355_KSPLIT_SHAPE")) : 1;
     if (!mmq_ksplit_applicable(type, K, T)) return false;
     if (!env || !has_planes || !mmq_applicable(type, K, T)) return true;
-    return T <= 64 || !tiles_beat_ksplit(n_rows, K, T, wsp, pair, sum_free);
+    return T <= 64 || !tiles_beat_ksplit(type, n_rows, K, T, wsp, pair, sum_free);
 }
 
 // segs: up to 3 tensors sharing the activation; swiglu (to 32 tokens, or where mmq_few_takes): segs = {gate, up} of one type and shape, out = silu(gate.x) * (up.x) into segs[0].out

@@ -57,3 +57,21 @@ def test_from_65_tokens_by_time(plan, n):
         for rows, cols in [(8192, 3072), (14336, 4096), (28672, 8192)]:
             assert plan(t, rows, cols, n, 1, 0) == PLANES, (rows, cols)
         assert plan(t, 1024, 2048, n, 1, 0) == KSPLIT
+
+
+@pytest.mark.parametrize("n", [65, 80, 96, 112, 128])
+def test_from_65_tokens_by_the_bytes_of_a_type(plan, n):
+    """Q6_K reaches the tiles as two bytes a weight: gate | up of 5632 x 2048, and the long rows of few tensors, stay with the K-split kernel where a Q4_K tensor does not."""
+    assert plan(Q6_K, 5632, 2048, n, 1, 0) == KSPLIT
+    for rows, cols in [(2048, 5632), (1536, 8960), (3072, 8192), (4096, 11008), (4096, 14336), (3584, 18944)]:
+        assert plan(Q6_K, rows, cols, n, 0, 1) == KSPLIT, (rows, cols)
+    if n < 112:
+        assert [plan(t, 5632, 2048, n, 1, 0) for t in (Q4_K, Q5_K)] == [PLANES] * 2
+        assert [plan(t, 4096, 14336, n, 0, 1) for t in (Q4_K, Q5_K)] == [PLANES] * 2
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("n", [161, 180, 212, 256])
+def test_the_square_tensor_of_4096_columns(plan, t, n):
+    """attn_output of an 8B model from 161 tokens on: 24 to 28 us with the K-split kernel, 17 to 22 on tiles."""
+    assert [plan(t, 4096, 4096, n, 0, s) for s in (0, 1)] == [PLANES] * 2
