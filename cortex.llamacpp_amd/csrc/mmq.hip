@@ -1324,8 +1324,9 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
 
 // SWIGLU: `planes` = ffn_gate, `planes_up` = ffn_up (n_rows rows each, same type): a workgroup takes 64 rows of BOTH (row-waves 0, 1 the
 // gate rows, 2, 3 the same rows of up), the two waves of the same rows swap halves of their tiles through LDS at the end and store
-// silu(gate . x) * (up . x) - one [T][n_rows] f32 result instead of two, and no separate SwiGLU pass over them
-template <int FORM, bool SWIGLU>
+// silu(gate . x) * (up . x) - one [T][n_rows] f32 result instead of two, and no separate SwiGLU pass over them.  ONE: one segment, known here (a struct made in the kernel and indexed
+// at run time is scratch: 96 bytes a lane of mmq_planes2_moe_kernel)
+template <int FORM, bool SWIGLU, bool ONE = SWIGLU>
 __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &po, int row_tile, int tok_tile, int n_tok_tiles, int zz) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1385,8 +1386,8 @@ __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &p
     }
     if (!tile_ok) return;
     int sg = 0;
-    if (po.n_seg > 1 && row0 >= po.row_end[0]) sg = 1;
-    if (po.n_seg > 2 && row0 >= po.row_end[1]) sg = 2;
+    if (!ONE && po.n_seg > 1 && row0 >= po.row_end[0]) sg = 1;
+    if (!ONE && po.n_seg > 2 && row0 >= po.row_end[1]) sg = 2;
     const bool split = a.n_split > 1;                           // partial sums of this K range: ws[zz][token][row], no residual
     float *out = split ? a.ws + (size_t)zz * T * n_rows : po.out[sg] - (sg ? po.row_end[sg - 1] : 0);
     const int ld_out = split ? n_rows : po.ld[sg];
@@ -1469,9 +1470,15 @@ __device__ __forceinline__ bool moe_tile_of(const MoeTiles &m, int j, int &e_out
     }
     return false;
 }
+// an expert's rows of the grouped output
+__device__ __forceinline__ PlanesOut moe_out(float *out, int ld_out, int r0, int n_rows) {
+    PlanesOut po{};
+    po.n_seg = 1; po.out[0] = out + (size_t)r0 * ld_out; po.ld[0] = ld_out; po.row_end[0] = n_rows;
+    return po;
+}
 template <int FORM>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_moe_kernel(const uint8_t *planes_gate, const uint8_t *planes_up, int n_rows, int K, int n_row_tiles,
-                                                                          int n_tile_slots, const int8_t *aq, const float *ad, const int16_t *absum, PlanesOut po,
+                                                                          int n_tile_slots, const int8_t *aq, const float *ad, const int16_t *absum, float *out, int ld_out,
                                                                           const MoeTiles mt) {
     const int bid = blockIdx.x, xcd = bid & 7, loc = bid >> 3;
     const int slot = loc % n_tile_slots;
@@ -1480,13 +1487,13 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_swiglu_moe_kernel(const 
     int e, tile, r0, n_e;
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
-    po.out[0] += (size_t)r0 * po.ld[0];
+    const PlanesOut po = moe_out(out, ld_out, r0, n_rows);
     planes2_body<FORM, true>(P2Args{planes_gate + (size_t)e * mt.plane_stride, planes_up + (size_t)e * mt.plane_stride, n_rows, K, n_e,
                                     aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 template <int FORM>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t *planes, int n_rows, int K, int n_row_tiles, int n_tile_slots,
-                                                                   const int8_t *aq, const float *ad, const int16_t *absum, PlanesOut po, const MoeTiles mt) {
+                                                                   const int8_t *aq, const float *ad, const int16_t *absum, float *out, int ld_out, const MoeTiles mt) {
     const int bid = blockIdx.x, xcd = bid & 7, loc = bid >> 3;
     const int slot = loc % n_tile_slots;
     const int row_tile = (loc / n_tile_slots) * 8 + xcd;
@@ -1494,8 +1501,8 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_moe_kernel(const uint8_t
     int e, tile, r0, n_e;
     if (!moe_tile_of(mt, slot, e, tile, r0, n_e)) return;
     const size_t nb = (size_t)(K >> 8);
-    po.out[0] += (size_t)r0 * po.ld[0];
-    planes2_body<FORM, false>(P2Args{planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e,
+    const PlanesOut po = moe_out(out, ld_out, r0, n_rows);
+    planes2_body<FORM, false, true>(P2Args{planes + (size_t)e * mt.plane_stride, nullptr, n_rows, K, n_e,
                                      aq + (size_t)r0 * K, ad + (size_t)r0 * nb, absum + (size_t)r0 * (K >> 4), nullptr, nullptr, 1}, po, row_tile, tile, (n_e + P2_TOK - 1) / P2_TOK, 0);
 }
 
@@ -1738,13 +1745,11 @@ bool mmq_planes_moe_ok(int type, int n_rows, int K) {
 hipError_t launch_mmq_planes_swiglu_moe(int type, const uint8_t *planes_gate, const uint8_t *planes_up, size_t plane_stride, int n_expert, const int32_t *meta,
                                         int n_rows, int K, int rows_max, const ActQuant &q, float *out, int ld_out, hipStream_t st) {
     if (!mmq_planes_moe_ok(type, n_rows, K) || n_expert < 1 || !meta || !q.qs || !q.d || !q.bsums) return hipErrorInvalidValue;
-    PlanesOut po{};
-    po.n_seg = 1; po.out[0] = out; po.ld[0] = ld_out; po.row_end[0] = n_rows;
     const int nrt = (n_rows + 63) / 64, slots = (rows_max + P2_TOK - 1) / P2_TOK + n_expert;     // every expert may end in a partial tile
     const dim3 grid((unsigned)(((nrt + 7) / 8) * slots * 8));
     const MoeTiles mt{meta, n_expert, plane_stride};
 #define GO(F) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_swiglu_moe_kernel<F>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
-                hipLaunchKernelGGL((mmq_planes2_swiglu_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt); }
+                hipLaunchKernelGGL((mmq_planes2_swiglu_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes_gate, planes_up, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, out, ld_out, mt); }
     switch (plane_form(type)) {
         case PF_CODES: GO(PF_CODES) break;
         case PF_NIBBLES: GO(PF_NIBBLES) break;
@@ -1756,13 +1761,11 @@ hipError_t launch_mmq_planes_swiglu_moe(int type, const uint8_t *planes_gate, co
 hipError_t launch_mmq_planes_moe(int type, const uint8_t *planes, size_t plane_stride, int n_expert, const int32_t *meta, int n_rows, int K, int rows_max,
                                  const ActQuant &q, float *out, int ld_out, hipStream_t st) {
     if (!mmq_planes_moe_ok(type, n_rows, K) || n_expert < 1 || !meta || !q.qs || !q.d || !q.bsums) return hipErrorInvalidValue;
-    PlanesOut po{};
-    po.n_seg = 1; po.out[0] = out; po.ld[0] = ld_out; po.row_end[0] = n_rows;
     const int nrt = (n_rows + P2_ROWS - 1) / P2_ROWS, slots = (rows_max + P2_TOK - 1) / P2_TOK + n_expert;
     const dim3 grid((unsigned)(((nrt + 7) / 8) * slots * 8));
     const MoeTiles mt{meta, n_expert, plane_stride};
 #define GO(F) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_moe_kernel<F>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
-                hipLaunchKernelGGL((mmq_planes2_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, po, mt); }
+                hipLaunchKernelGGL((mmq_planes2_moe_kernel<F>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, nrt, slots, q.qs, q.d, q.bsums, out, ld_out, mt); }
     switch (plane_form(type)) {
         case PF_CODES: GO(PF_CODES) break;
         case PF_NIBBLES: GO(PF_NIBBLES) break;
