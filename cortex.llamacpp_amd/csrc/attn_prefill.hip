@@ -776,9 +776,10 @@ int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max) {
 }
 
 // (a context's workspace: 4 KB a cell for eight kv heads of 128 in a q8_0 cache, half of that in an f16 one)
-size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int D, int G, int n_ctx) {
+size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int H, int G, int D, int n_ctx) {
     const bool f16 = type_k == T_F16 && type_v == T_F16;
-    if (!(f16 || (type_k == T_Q8_0 && type_v == T_Q8_0)) || (D != 64 && D != 128) || G < 1 || n_ctx < 1) return 0;
+    const int R = G > 0 ? H / G : 0;
+    if (!(f16 || (type_k == T_Q8_0 && type_v == T_Q8_0)) || (D != 64 && D != 128) || R < 1 || R > 8 || (D == 64 && (R & (R - 1))) || n_ctx < 1) return 0;
     const size_t b = (size_t)((n_ctx + CK - 1) / CK) * G * plane_chunk_bytes(f16, D);
     return b <= ((size_t)256 << 20) ? b : 0;
 }
@@ -788,11 +789,15 @@ bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible) {
     const int tiles = (T + QT * fa_sub_tiles(H / G) - 1) / (QT * fa_sub_tiles(H / G));
     return (long)tiles * std::min(n_kv, visible) >= 8L * n_kv;
 }
+size_t flash_attn_prefill_planes_wanted(int type_k, int type_v, int H, int G, int D, int n_ctx, int n_ubatch) {
+    const size_t b = flash_attn_prefill_planes_bytes(type_k, type_v, H, G, D, n_ctx);
+    return b && flash_attn_prefill_planes_pay(n_ubatch, H, G, 1, 1) ? b : 0;
+}
 
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *v_planes) {
     const int R = a.H / a.G, kh = fa_key_halves(R), qs = fa_sub_tiles(R);
     const int nsp = (a.pf_splits > 1 && a.part) ? a.pf_splits : 1;
-    const bool planes = v_planes && flash_attn_prefill_planes_bytes(a.type_k, a.type_v, a.D, a.G, a.n_ctx) && kh == (R <= 4 ? 2 : 1) && qs == (R == 1 ? 4 : R == 2 ? 2 : 1);
+    const bool planes = v_planes && flash_attn_prefill_planes_bytes(a.type_k, a.type_v, a.H, a.G, a.D, a.n_ctx) && kh == (R <= 4 ? 2 : 1) && qs == (R == 1 ? 4 : R == 2 ? 2 : 1);
     const dim3 grid((unsigned)a.G, (unsigned)((a.T + QT * qs - 1) / (QT * qs)), (unsigned)nsp);
     const bool f16 = a.type_k == T_F16;
     const int nb = a.D / 32;

@@ -280,6 +280,9 @@ int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv
     a.T = n_tokens; a.H = n_head; a.G = n_head_kv; a.D = head_dim; a.n_ctx = a.n_kv_max = n_cells; a.type_k = a.type_v = type_kv;
     return flash_attn_cols_takes(a, !encoder) ? flash_attn_cols_splits(a) : 0;
 }
+int64_t mi355_debug_attn_planes_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_ctx, int32_t n_ubatch) {
+    return (int64_t)flash_attn_prefill_planes_wanted(type_kv, type_kv, n_head, n_head_kv, head_dim, n_ctx, n_ubatch);
+}
 int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int32_t type_v, int32_t type_o, int32_t n_embd, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
                                   int32_t type_kv, int32_t n_kv, int32_t *slots_out) {
     int slots = 0;
@@ -792,7 +795,7 @@ int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t
     a.pf_splits = flash_attn_prefill_splits((int)T, H, G, D, n_cells);
     DevBuf part(flash_attn_workspace_floats((int)T, H, D, std::max(a.splits, a.pf_splits)) * 4);
     a.part = part.as<float>();
-    DevBuf planes(g_op_attn_planes ? flash_attn_prefill_planes_bytes(type_k, type_v, D, G, n_cells) : 0);
+    DevBuf planes(g_op_attn_planes ? flash_attn_prefill_planes_bytes(type_k, type_v, H, G, D, n_cells) : 0);
     const bool cols = g_op_attn_cols > 0;
     if (cols && !flash_attn_cols_applicable(a)) { fail("attn_cols: no form for this call"); return MI355_ERR_ARG; }
     DevBuf cpart(cols ? flash_attn_workspace_floats((int)T, H, D, g_op_attn_cols) * 4 : 16);

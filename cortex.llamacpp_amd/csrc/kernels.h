@@ -670,8 +670,9 @@ bool flash_attn_prefill_applicable(const AttnArgs &a);
 int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max);
 // planes (nullable): flash_attn_prefill_planes_bytes() for the V planes of the scanned cells, made once for all query tiles
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *planes = nullptr);
-size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int D, int G, int n_ctx);      // of a cache; 0: no such form, or more than 256 MiB
+size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int H, int G, int D, int n_ctx);     // of a cache; 0: no such form, or more than 256 MiB
 bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible);               // n_kv cells scanned, of which a query can see at most `visible`
+size_t flash_attn_prefill_planes_wanted(int type_k, int type_v, int H, int G, int D, int n_ctx, int n_ubatch);      // by a decoder's context: 0 too where no batch is long enough for them to pay
 // a short batch of one sequence, a short text through the encoder: the same in another split of the work (attn_cols.hip); pf_splits = flash_attn_cols_splits
 bool flash_attn_cols_applicable(const AttnArgs &a);
 bool flash_attn_cols_takes(const AttnArgs &a, bool one_token_kernel);      // one_token_kernel: the batch of a decoder, which has kernels for one token at a time

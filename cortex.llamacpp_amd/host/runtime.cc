@@ -706,7 +706,7 @@ bool Context::init(std::string &err) {
         ws = std::max(ws, flash_attn_workspace_floats(t, hp.n_head, (int)D, flash_attn_prefill_splits(t, hp.n_head, (int)G, (int)D, (int)NC)));
     att_part_ = (float *)dalloc(ws * 4);
     att_part_floats_ = ws;
-    const size_t planes = T >= 32 && !hp.encoder && D * (size_t)hp.n_head_kv > 0 ? flash_attn_prefill_planes_bytes(cp.type_k, cp.type_v, (int)D, (int)G, (int)NC) : 0;
+    const size_t planes = hp.encoder ? 0 : flash_attn_prefill_planes_wanted(cp.type_k, cp.type_v, hp.n_head, (int)G, (int)D, (int)NC, (int)T);
     att_planes_ = planes ? dalloc(planes) : nullptr;             // (without: every query tile converts the chunks it walks)
     if (planes && !att_planes_) (void)hipGetLastError();
     att_counters_ = (unsigned *)dalloc(64 * ATT_SYNC_STRIDE * sizeof(unsigned));

@@ -182,6 +182,9 @@ MI355_API int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n
 /* host logic only: does the attention of n_tokens of one conversation (encoder: of a text) over n_cells cells of type_kv go through csrc/attn_cols.hip?  Returns the number of workgroups
    that share a tile's keys there, 0 = the one-token or the prompt kernel */
 MI355_API int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder);
+/* host logic only: bytes that a decoder's context of n_ctx cells (K and V of type_kv) and n_ubatch tokens a micro-batch keeps for the V planes of a prompt's attention
+   (csrc/attn_prefill.hip); 0 where no micro-batch takes that form */
+MI355_API int64_t mi355_debug_attn_planes_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_ctx, int32_t n_ubatch);
 /* llama_set_embeddings (ctx.cc:299) */
 MI355_API void    mi355_set_embeddings(mi355_context *ctx, int32_t enabled);
 /* llama_get_embeddings_ith (ctx.cc:1042-1044): final-norm hidden state (n_embd floats, host memory) of batch row i of the

@@ -31,3 +31,18 @@ def test_long_batches(takes, model, yes, no):
 
 def test_texts(takes):
     assert all(takes(TEXT, n, 0, 1) for n in (3, 20, 187, 700, 2000, 2048))
+
+
+@pytest.mark.parametrize("model,n,bytes_", [
+    (L8, 225, 4096 * 8 * 128 * 4), (L7, 897, 4096 * 32 * 128 * 2), ((Q8_0, 16, 8, 128), 449, 4096 * 8 * 128 * 4), (SMALL, 225, 4096 * 4 * 64 * 2), ((Q8_0, 56, 8, 128), 225, 4096 * 8 * 128 * 4)])
+def test_planes_workspace(pkg, model, n, bytes_):
+    """A context keeps the V planes' workspace from the first micro-batch of eight query tiles (of 128, 64, 32 tokens with 1, 2, more query heads to a kv head) on, and not below."""
+    plan = pkg.load_library().mi355_debug_attn_planes_plan
+    assert [plan(*model, 4096, t) for t in (1, 32, n - 1)] == [0] * 3
+    assert [plan(*model, 4096, t) for t in (n, 2048)] == [bytes_] * 2
+
+
+@pytest.mark.parametrize("model", [(Q8_0, 12, 4, 64), (F16, 28, 4, 64), (F16, 10, 2, 64), (2, 32, 8, 128), (Q8_0, 32, 2, 128), (Q8_0, 32, 8, 96)])
+def test_no_planes_workspace_without_a_form(pkg, model):
+    """64-wide heads in threes, fives, sixes, sevens; a q4_0 cache; more than eight query heads to a kv head; other widths."""
+    assert pkg.load_library().mi355_debug_attn_planes_plan(*model, 4096, 2048) == 0
