@@ -45,6 +45,7 @@ struct mi355_context {
 static thread_local std::string t_err;
 static int g_op_mmq_planes = 1, g_op_mmq_ksplit = 1, g_op_mmq_few = -1;
 static int g_op_attn_planes = 0;   // mi355_op_flash_attn: 1 a prompt batch's V planes made once for all its query tiles
+static int g_op_attn_seqs = 1, g_op_attn_spare = 0;   // ... : the tokens are so many sequences' in turn, every fifth cell all of theirs and the others one's; the last so many cells lie behind the scan's end
 static int g_op_attn_cols = 0;     // mi355_op_flash_attn: 0 the call's own kernel, else attn_cols.hip with so many shares of the keys
 static bool g_backend_ok = false;
 
@@ -782,7 +783,11 @@ int mi355_op_flash_attn(const float *q, int64_t T, int32_t H, int32_t G, int32_t
     if (!vs.empty()) dvs.up(vs.data(), vs.size() * 2);
     std::vector<uint64_t> seqm((size_t)n_cells, 1ull);
     std::vector<int32_t> tseq((size_t)T, 0);
-    int32_t nkv = n_cells;
+    if (const int s = g_op_attn_seqs; s > 1) {
+        for (int c = 0; c < n_cells; c++) seqm[(size_t)c] = c % 5 == 0 ? (1ull << s) - 1 : 1ull << (c % s);
+        for (int64_t t = 0; t < T; t++) tseq[(size_t)t] = (int32_t)(t * s / T);
+    }
+    const int32_t nkv = std::max(1, n_cells - g_op_attn_spare);
     dcp.up(cell_pos, (size_t)n_cells * 4); dcs.up(seqm.data(), (size_t)n_cells * 8); dtp.up(q_pos, (size_t)T * 4); dts.up(tseq.data(), (size_t)T * 4);
     dn.up(&nkv, 4);
     AttnArgs a{};
@@ -936,6 +941,8 @@ int mi355_debug_set_option(const char *name, int32_t value) {
     if (!strcmp(name, "mmq_few")) { g_op_mmq_few = value; return MI355_OK; }
     if (!strcmp(name, "attn_store_fuse")) { set_attn_store_fuse(value != 0); return MI355_OK; }
     if (!strcmp(name, "attn_planes")) { g_op_attn_planes = value > 0; return MI355_OK; }
+    if (!strcmp(name, "attn_seqs")) { g_op_attn_seqs = value < 1 || value > 32 ? 1 : value; return MI355_OK; }
+    if (!strcmp(name, "attn_spare")) { g_op_attn_spare = value < 0 ? 0 : value; return MI355_OK; }
     if (!strcmp(name, "attn_cols")) { g_op_attn_cols = value < 0 || value > 64 ? 0 : value; return MI355_OK; }     // mi355_op_flash_attn: attn_cols.hip with so many shares of the keys
     if (!strcmp(name, "late_sums")) { set_late_sums(value != 0); return MI355_OK; }
     if (!strcmp(name, "rope_fast")) { set_rope_fast(value != 0); return MI355_OK; }
