@@ -86,6 +86,7 @@ SYMBOLS = {
     "mi355_debug_qkv_attn_launches": (C.c_int64, [_vp]),
     "mi355_debug_qkv_attn_plan": (C.c_int64, [C.c_int32] * 10 + [C.POINTER(C.c_int32)]),
     "mi355_debug_batch_plan": (_i32, [_i32] * 6),
+    "mi355_debug_q80_plan": (_i32, [_i32] * 3),
     "mi355_debug_attn_plan": (_i32, [_i32] * 7),
     "mi355_debug_attn_planes_plan": (C.c_int64, [_i32] * 6),
     "mi355_set_embeddings": (None, [_vp, _i32]),

@@ -276,6 +276,10 @@ int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int
     }
     return mmq_applicable(type, n_cols, n_tokens) ? 3 : 0;
 }
+int32_t mi355_debug_q80_plan(int32_t n_rows, int32_t n_cols, int32_t n_tokens) {
+    const int rows = n_rows;
+    return n_rows >= 1 && mmq_q80_applicable(T_Q8_0, n_cols, n_tokens) ? mmq_q80_form(&rows, 1, n_tokens) : 0;
+}
 int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder) {
     AttnArgs a{};
     a.T = n_tokens; a.H = n_head; a.G = n_head_kv; a.D = head_dim; a.n_ctx = a.n_kv_max = n_cells; a.type_k = a.type_v = type_kv;

@@ -161,6 +161,7 @@ hipError_t launch_mmq_q80(const uint8_t *W, size_t row_bytes, int n_rows, int K,
                           const float *resid, hipStream_t st);
 // up to three tensors of the same K and row size (Q | K | V, gate | up) in one launch; resid (nullable) has out's layout and may be out
 struct Q80Seg { const uint8_t *W; size_t row_bytes; int n_rows; float *out; int ld_out; };
+int mmq_q80_form(const int *n_rows, int n, int T);          // rows and tokens of a wave: 16, 32, or 64 as 2 x 2 tiles of 32
 hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st);
 // up to three tensors of one plane format (Q4_K / Q5_K together, or Q6_K) whose plane sets are contiguous in memory, as one
 // launch over the concatenated rows; seg_rows[i] rows go to outs[i] (leading dimension lds_out[i])

@@ -236,26 +236,32 @@ template <int SZ, int W, int S, int U> static void tiles_launch(Q80Args &a, hipS
     hipLaunchKernelGGL((mmq_q80_tiles_kernel<SZ, W, S, U>), dim3((unsigned)tiles, (unsigned)((a.T + R - 1) / R)), dim3(256), 0, st, a);
 }
 
+// Up to two 32 x 32 workgroups a CU it is one wave's way through its row that counts, half as long in tiles of 16 (us, 16 | 32: 5632 x 2048, 40 tokens = 352 workgroups 9.6 | 12.9;
+// 4096 x 14336, 100 = 512 48 | 74; 2048 x 2048, 320 = 640 13.1 | 13.0; 5632 x 2048, 100 = 704 14.1 | 13.3).  Four tiles of 32 a wave read half as much of LDS, but need 1.7 workgroups of 128 x 128 a CU and no more
+// than a tenth more padding (us, one tile | four: 5632 x 2048, 1200 tokens = 440 workgroups 66 | 64; 4096 x 14336, 2000 = 512 470 | 415, 1200 = 320 283 | 330;
+// 32000 x 2048, 320 = 750, a fifth more padding 92 | 100).
+int mmq_q80_form(const int *n_rows, int n, int T) {
+    const auto count = [&](int r) {
+        long c = 0;
+        for (int i = 0; i < n; i++) c += (n_rows[i] + r - 1) / r;
+        return c * ((T + r - 1) / r);
+    };
+    const long c32 = count(32), c64 = count(64), c128 = count(128);
+    return c32 <= 2L * num_cu() ? 16 : c128 * 10 >= 17L * num_cu() && c128 * 40 <= c64 * 11 ? 64 : 32;
+}
+
 hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st) {
     if (!mmq_q80_applicable(T_Q8_0, K, T) || !q.qs0 || !q.d0 || n < 1 || n > 3) return hipErrorInvalidValue;
     for (int i = 0; i < n; i++)                                        // (16-byte requests of the codes, 4-byte ones of the scales)
         if (sg[i].row_bytes != sg[0].row_bytes || ((((uintptr_t)sg[i].W | sg[i].row_bytes | (uintptr_t)q.qs0) & 15) | ((uintptr_t)q.d0 & 3))) return hipErrorInvalidValue;
     Q80Args a{};
     a.row_bytes = sg[0].row_bytes; a.n_seg = n; a.K = K; a.T = T; a.aq = q.qs0; a.ad = q.d0; a.resid = resid;
-    const auto count = [&](int r) {
-        long c = 0;
-        for (int i = 0; i < n; i++) c += (sg[i].n_rows + r - 1) / r;
-        return c * ((T + r - 1) / r);
-    };
     for (int i = 0; i < n; i++) { a.W[i] = sg[i].W; a.out[i] = sg[i].out; a.n_rows[i] = sg[i].n_rows; a.ld_out[i] = sg[i].ld_out; }
-    // Up to two 32 x 32 workgroups a CU it is one wave's way through its row that counts, half as long in tiles of 16 (us, 16 | 32: 5632 x 2048, 40 tokens = 352 workgroups 9.6 | 12.9;
-    // 4096 x 14336, 100 = 512 48 | 74; 2048 x 2048, 320 = 640 13.1 | 13.0; 5632 x 2048, 100 = 704 14.1 | 13.3).  Four tiles of 32 a wave read half as much of LDS, but need 1.7 workgroups of 128 x 128 a CU and no more
-    // than a tenth more padding (us, one tile | four: 5632 x 2048, 1200 tokens = 440 workgroups 66 | 64; 4096 x 14336, 2000 = 512 470 | 415, 1200 = 320 283 | 330;
-    // 32000 x 2048, 320 = 750, a fifth more padding 92 | 100).
-    const long c32 = count(32), c64 = count(64), c128 = count(128);
-    if (c32 <= 2L * num_cu()) tiles_launch<16, 1, 3, 8>(a, st);
-    else if (c128 * 10 >= 17L * num_cu() && c128 * 40 <= c64 * 11) tiles_launch<32, 2, 2, 4>(a, st);
-    else tiles_launch<32, 1, 3, 4>(a, st);
+    switch (mmq_q80_form(a.n_rows, n, T)) {
+        case 16: tiles_launch<16, 1, 3, 8>(a, st); break;
+        case 64: tiles_launch<32, 2, 2, 4>(a, st); break;
+        default: tiles_launch<32, 1, 3, 4>(a, st);
+    }
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-"""Prompt batches against Q8_0 weights (csrc/mmq_q80.hip): groups of four blocks requested a step ahead, in pairs, in chunks of sixteen."""
+"""Prompt batches against Q8_0 weights (csrc/mmq_q80.hip): rows of one, eight and nine steps in tiles of 16, of two, four and eighteen in tiles of 32."""
 import numpy as np
 import pytest
 
@@ -8,8 +8,8 @@ from test_gpu_ops import Q8_0, be, rand_weights  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K,N,T", [(256, 129, 32), (2048, 40, 33), (2304, 130, 65),       # one pair of groups; a chunk; a chunk and a pair
-                                   (512, 8200, 250), (256, 16390, 250), (2304, 16384, 129)])  # two and four token tiles a wave, ragged rows and tokens
+@pytest.mark.parametrize("K,N,T", [(256, 129, 32), (2048, 40, 33), (2304, 130, 65),       # tiles of 16, ragged rows and tokens
+                                   (512, 8200, 250), (256, 16390, 250), (2304, 16384, 129)])  # a tile of 32 a wave
 def test_q80_groups_bit_exact(be, K, N, T):  # noqa: F811
     """Integer block sums, three roundings a block, blocks in order: the oracle's bits."""
     rng = np.random.default_rng(K + N + T)
