@@ -899,7 +899,7 @@ def main() -> int:
         },
         "prefill_roofline": {
             "bound": "mfma",
-            "kernel": "mmq_planes2_kernel / mmq_planes_kernel (int8 v_mfma_i32_32x32x32_i8, weights pre-expanded into two exact int8 planes)",
+            "kernel": "mmq_planes2_kernel / mmq_planes_kernel (int8 v_mfma_i32_32x32x32_i8, two exact int8 planes of every weight, made at load or, of Q4_K and Q5_K, in the kernel)",
             "achieved": round(prefill_tops, 1),
             "peak": MFMA_I8_PEAK_TOPS,
             "unit": "TOP/s",

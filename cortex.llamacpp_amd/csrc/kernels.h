@@ -163,7 +163,7 @@ hipError_t launch_mmq_q80(const uint8_t *W, size_t row_bytes, int n_rows, int K,
 struct Q80Seg { const uint8_t *W; size_t row_bytes; int n_rows; float *out; int ld_out; };
 int mmq_q80_form(const int *n_rows, int n, int T);          // rows and tokens of a wave: 16, 32, or 64 as 2 x 2 tiles of 32
 hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st);
-// up to three tensors of one plane format (Q4_K / Q5_K together, or Q6_K) whose plane sets are contiguous in memory, as one
+// up to three tensors of one plane form, or of the forms of Q4_K, Q5_K and Q6_K where mmq_planes_mixed_ok, whose plane sets are contiguous in memory, as one
 // launch over the concatenated rows; seg_rows[i] rows go to outs[i] (leading dimension lds_out[i])
 hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *seg_rows, float *const *outs, const int *lds_out, int n_seg, int K, int T,
                                    const ActQuant &q, const int8_t *bh, const int8_t *bl, const float *resid, hipStream_t st,

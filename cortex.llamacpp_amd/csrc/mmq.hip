@@ -841,7 +841,7 @@ struct PlanesOut {
     int ld[3];
     int row_end[3];
     int n_seg;
-    int form[3];            // PlaneForm of a segment, and where its blocks begin: mmq_planes2_kernel<2> and <3> only
+    int form[3];            // PlaneForm of a segment, and where its blocks begin: mmq_planes2_kernel<P2_MIXED> only
     size_t at[3];
 };
 
@@ -1416,9 +1416,9 @@ __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &p
     if (all) store(true); else store(false);
 }
 
-// MODE < 4: that PlaneForm; otherwise per segment (po.form; segment boundaries at multiples of 128 rows, so a workgroup's row tile is of one kind), of the forms in MODE >> 4 - Q | K | V of
-// the layers whose attn_v is Q6_K, in one launch.  The bodies lie behind workgroup-uniform branches (a run-time flag inside ONE body costs 92 bytes of scratch per lane and 2.3x the time).
-constexpr int P2_MIXED = 4, P2_MIXED_PACKED = P2_MIXED | (1 << PF_CODES | 1 << PF_NIBBLES | 1 << PF_SIGNED) << 4, P2_MIXED_PLANES = P2_MIXED | (1 << PF_MINS | 1 << PF_SIGNED) << 4;
+// MODE a PlaneForm, or P2_MIXED: per segment (po.form, of Q4_K, Q5_K or Q6_K; segment boundaries at multiples of 128 rows, so a workgroup's row tile is of one kind) - Q | K | V of
+// the layers whose attn_v has more bits, in one launch.  The bodies lie behind workgroup-uniform branches (a run-time flag inside ONE body costs 92 bytes of scratch per lane and 2.3x the time).
+constexpr int P2_MIXED = 4;
 template <int MODE>
 __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *planes, int n_rows, int K, int T, int n_row_tiles, int n_tok_tiles,
                                                                const int8_t *aq, const float *ad, const int16_t *absum,
@@ -1429,7 +1429,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *pl
     const int row_tile = (loc / (n_tok_tiles * n_split)) * 8 + xcd;
     if (row_tile >= n_row_tiles) return;                       // workgroup-uniform
     P2Args a{planes, nullptr, n_rows, K, T, aq, ad, absum, resid, ws, n_split};
-    if constexpr (MODE < P2_MIXED) planes2_body<MODE, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
+    if constexpr (MODE != P2_MIXED) planes2_body<MODE, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
     else {
         int sg = 0;
         if (po.n_seg > 1 && row_tile * P2_ROWS >= po.row_end[0]) sg = 1;
@@ -1437,9 +1437,9 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes2_kernel(const uint8_t *pl
         // where block 0 of the launch would lie if all were of this segment's form
         const int form = __builtin_amdgcn_readfirstlane(po.form[sg]);
         a.planes = planes + po.at[sg] - (size_t)(sg ? po.row_end[sg - 1] >> 5 : 0) * (size_t)(K >> 8) * plane_block(form);
-#define P2_FORM(F) if constexpr (((MODE >> 4) >> F) & 1) if (form == F) planes2_body<F, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz)
-        P2_FORM(PF_SIGNED); P2_FORM(PF_MINS); P2_FORM(PF_CODES); P2_FORM(PF_NIBBLES);
-#undef P2_FORM
+        if (form == PF_SIGNED) planes2_body<PF_SIGNED, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
+        if (form == PF_CODES) planes2_body<PF_CODES, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
+        if (form == PF_NIBBLES) planes2_body<PF_NIBBLES, false>(a, po, row_tile, tok_tile, n_tok_tiles, zz);
     }
 }
 
@@ -1578,7 +1578,7 @@ void mmq_set_split(int n) { g_mmq_split = n; }
 void mmq_set_lds_form(int on) { g_mmq_p2 = on; }
 
 // continuous-batching decode steps and prompts up to a few hundred tokens: 3 <= T <= g_ksplit_max.  This kernel reads the GGUF bytes (0.56 B / weight) and expands them in
-// registers, once per 64 tokens; the planes kernels read 2 B / weight that they need not expand, the fewer times the more tokens there are.  Behind 256 tokens every tensor with
+// registers, once per 64 tokens; the planes kernels read 0.6 to 2 B / weight that they need expand less or not at all, the fewer times the more tokens there are.  Behind 256 tokens every tensor with
 // planes goes to them: a whole 8B prompt of 320 tokens took 17.2 ms here and 15.2 there, of 384 19.1 and 15.5, before the tiles became faster.
 static int g_ksplit_max = getenv("MI355_KSPLIT_MAX") ? atoi(getenv("MI355_KSPLIT_MAX")) : 256;
 bool mmq_ksplit_applicable(int type, int K, int T) {
@@ -1698,7 +1698,7 @@ static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool
     return n_split;
 }
 
-// Q4_K / Q5_K segments beside Q6_K ones in one launch: only the 128 x 256 kernel has that form, and segments must end on its row tiles
+// Segments of several forms in one launch: only the 128 x 256 kernel has that form, and segments must end on its row tiles
 bool mmq_planes_mixed_ok(const int *seg_rows, int n_seg, int K, int T, MMQWorkspace wsp) {
     static const bool env_on = !(getenv("MI355_MMQ_MIXED") && getenv("MI355_MMQ_MIXED")[0] == '0');
     if (!env_on) return false;
@@ -1782,7 +1782,7 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     PlanesOut po{};
     po.n_seg = n_seg;
     int n_rows = 0;
-    bool mixed = false, packed = false, mins = false;
+    bool mixed = false, mins = false;
     size_t at = 0;
     for (int i = 0; i < n_seg; i++) {
         if (i + 1 < n_seg && (seg_rows[i] % 32) != 0) return hipErrorInvalidValue;
@@ -1793,11 +1793,9 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
         po.at[i] = at;
         at += (mmq_planes_bytes(ti, seg_rows[i], K) + 255) & ~(size_t)255;
         mixed = mixed || po.form[i] != plane_form(type);
-        packed = packed || po.form[i] >= PF_CODES;
         mins = mins || po.form[i] == PF_MINS;
     }
-    if (mixed && packed && mins) return hipErrorInvalidValue;   // (no launch has both bodies)
-    if (mixed && !mmq_planes_mixed_ok(seg_rows, n_seg, K, T, wsp)) return hipErrorInvalidValue;
+    if (mixed && (mins || !mmq_planes_mixed_ok(seg_rows, n_seg, K, T, wsp))) return hipErrorInvalidValue;
     static const int env_mt = getenv("MI355_MMQ_MT") ? atoi(getenv("MI355_MMQ_MT")) : 0;
     // 128 x 128 workgroup tiles (two token tiles per wave) when that still yields ~2 workgroups per CU, else 256 x 32
     // tiles, which quadruple the workgroup count (measured on the 8B shapes: gate/up 297 vs 383 us, N = 4096 tensors
@@ -1807,7 +1805,7 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
     if (n_seg > 1 && T > 32 && wg2 * 4 >= 3L * num_cu()) mt = 2;       // concatenated Q | K | V: 192 workgroups of 128 x 128 beat 384 of 256 x 32 (59 vs 71 us)
     if (env_mt == 1 || env_mt == 2) mt = env_mt;
     if (g_mmq_mt == 1 || g_mmq_mt == 2) mt = g_mmq_mt;
-    // 128 rows x 256 tokens per workgroup from 129 tokens on; tensors with too few rows to cover the chip that way split K over 2..4 workgroups (partial sums in
+    // 128 rows x 256 tokens per workgroup from 65 tokens on; tensors with too few rows to cover the chip that way split K over 2..4 workgroups (partial sums in
     // the caller's workspace, added up pairwise)
     bool p2 = false;
     const int n_split = planes2_split(n_rows, K, T, wsp, &p2);
@@ -1816,8 +1814,7 @@ hipError_t launch_mmq_planes_multi(int type, const uint8_t *planes, const int *s
         const dim3 grid((unsigned)(((nrt + 7) / 8) * ntt * n_split * 8));
 #define GO(M) { (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&mmq_planes2_kernel<M>), hipFuncAttributeMaxDynamicSharedMemorySize, P2_LDS); \
                 hipLaunchKernelGGL((mmq_planes2_kernel<M>), grid, dim3(NTHREADS), (size_t)P2_LDS, st, planes, n_rows, K, T, nrt, ntt, q.qs, q.d, q.bsums, po, resid, wsp.p, n_split); }
-        if (mixed && packed) GO(P2_MIXED_PACKED)
-        else if (mixed) GO(P2_MIXED_PLANES)
+        if (mixed) GO(P2_MIXED)
         else switch (plane_form(type)) {
             case PF_CODES: GO(PF_CODES) break;
             case PF_NIBBLES: GO(PF_NIBBLES) break;

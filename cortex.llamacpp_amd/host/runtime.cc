@@ -1021,7 +1021,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
         if (q80_copy(w, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU && aq.qs0)      // prompt processing of Q4_0 / Q5_0 / IQ4_NL tensors: their exact Q8_0-layout copy
             return launch_mmq_q80(w.planes, dev_row_bytes(T_Q8_0, K), (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         if (planes_small(w, K, T) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU && aq.qs) {
-            // prompt processing of Q2_K / Q3_K tensors: their plane sets (expanded at load in the Q4_K / Q6_K plane formats, mmq.hip) on the same kernels
+            // prompt processing of Q2_K / Q3_K tensors: their plane sets (both planes, expanded at load, mmq.hip) on the same kernels
             if (w.type == T_Q2_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T));
             return launch_mmq_planes(w.type, w.planes, (int)w.N, K, T, aq, bh, bl, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_, mmq_ws_);
         }
@@ -1046,7 +1046,7 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
         all_rows += (int)ws[i]->N;
     }
     // Q | K | V (or Q | K) as one launch over the concatenated rows where their plane sets are adjacent in the arena and
-    // of one plane format (the Q6_K attn_v of the "more bits" layers runs on its own)
+    // of one plane form (an attn_v of more bits: below)
     auto adjacent = [&](int i) { return ws[i]->planes && ws[i - 1]->planes && ws[i]->planes == ws[i - 1]->planes + ws[i - 1]->planes_bytes &&
                                         (ws[i - 1]->N % 32) == 0 && ws[i]->n_expert == 1; };
     int nf = 1;
