@@ -252,8 +252,8 @@ int mmq_q80_form(const int *n_rows, int n, int T) {
 
 hipError_t launch_mmq_q80_multi(const Q80Seg *sg, int n, int K, int T, const ActQuant &q, const float *resid, hipStream_t st) {
     if (!mmq_q80_applicable(T_Q8_0, K, T) || !q.qs0 || !q.d0 || n < 1 || n > 3) return hipErrorInvalidValue;
-    for (int i = 0; i < n; i++)                                        // (16-byte requests of the codes, 4-byte ones of the scales)
-        if (sg[i].row_bytes != sg[0].row_bytes || ((((uintptr_t)sg[i].W | sg[i].row_bytes | (uintptr_t)q.qs0) & 15) | ((uintptr_t)q.d0 & 3))) return hipErrorInvalidValue;
+    for (int i = 0; i < n; i++)                                        // (16-byte requests of the codes and, in tiles of 16, of the scales)
+        if (sg[i].row_bytes != sg[0].row_bytes || (((uintptr_t)sg[i].W | sg[i].row_bytes | (uintptr_t)q.qs0 | (uintptr_t)q.d0) & 15)) return hipErrorInvalidValue;
     Q80Args a{};
     a.row_bytes = sg[0].row_bytes; a.n_seg = n; a.K = K; a.T = T; a.aq = q.qs0; a.ad = q.d0; a.resid = resid;
     for (int i = 0; i < n; i++) { a.W[i] = sg[i].W; a.out[i] = sg[i].out; a.n_rows[i] = sg[i].n_rows; a.ld_out[i] = sg[i].ld_out; }

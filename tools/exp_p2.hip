@@ -1,5 +1,6 @@
-// tools/exp_p2.hip — the prompt contraction on pre-expanded planes: per-lane planes kernel (128 x 128 tiles) against the kernel with both
-// operands through LDS (128 x 256): bit-for-bit comparison on synthetic planes and time per launch (HIP events).
+// tools/exp_p2.hip — the prompt contraction on a tensor's plane set: per-lane planes kernel (256 x 32 and 128 x 128 tiles) against the kernel with the activations through LDS
+// (128 x 256): bit-for-bit comparison on random GGUF rows, laid out as at load, and time per launch (HIP events; the launches read copies of the tensor in turn, more than the last
+// level of cache holds).
 // build: tools/build_exp_p2.sh; usage: exp_p2 [rows] [columns] [tokens] [type] [launches] [1: all operands zero]
 #include <cstdio>
 #include <cstdlib>
@@ -33,20 +34,23 @@ int main(int argc, char **argv) {
     const int N = argc > 1 ? atoi(argv[1]) : 4096, K = argc > 2 ? atoi(argv[2]) : 4096, T = argc > 3 ? atoi(argv[3]) : 2048;
     const int type = argc > 4 ? atoi(argv[4]) : T_Q4_K, reps = argc > 5 ? atoi(argv[5]) : 20;
     const bool zeros = argc > 6 && atoi(argv[6]);
-    const int nb = K / 256, n_rt = (N + 31) / 32;
-    const size_t PLB = 8 * 2 * 1024 + 32 * 16;
-    std::vector<uint8_t> hp((size_t)n_rt * nb * PLB);
-    for (size_t b = 0; b < (size_t)n_rt * nb; b++) {
-        uint8_t *blk = hp.data() + b * PLB;
-        for (int i = 0; i < 16384; i++) blk[i] = (uint8_t)(rnd() & (type == T_Q6_K ? 0xff : 0x3f));
-        for (int r = 0; r < 32; r++) {
-            uint32_t *m = reinterpret_cast<uint32_t *>(blk + 16384 + r * 16);
-            m[0] = f2h_host(0.001f + (rnd() & 255) * 1e-5f) | ((uint32_t)f2h_host(0.0005f + (rnd() & 255) * 1e-5f) << 16);
-            m[1] = rnd() & 0x3f3f3f3f; m[2] = (rnd() * 77u) & 0x3f3f3f3f; m[3] = 0;
+    const int nb = K / 256;
+    const size_t rb = dev_row_bytes(type, K), pb = (mmq_planes_bytes(type, N, K) + 255) & ~(size_t)255;
+    if (!pb) { printf("no planes of type %d\n", type); return 1; }
+    std::vector<uint8_t> hw(rb * N);                            // device rows: any byte is a code, a scale or a min; the block scales are chosen
+    for (auto &b : hw) b = zeros ? 0 : (uint8_t)rnd();
+    for (int r = 0; r < N && !zeros; r++)
+        for (int b = 0; b < nb; b++) {
+            const uint16_t d = f2h_host(0.001f + (rnd() & 255) * 1e-5f), dmin = f2h_host(0.0005f + (rnd() & 255) * 1e-5f);
+            uint8_t *row = hw.data() + rb * r;
+            if (type == T_Q4_K || type == T_Q5_K) { uint8_t *blk = row + (size_t)b * (type == T_Q4_K ? 144 : 176); memcpy(blk, &d, 2); memcpy(blk + 2, &dmin, 2); }
+            else if (type == T_Q6_K) memcpy(row + (size_t)nb * 208 + 2 * b, &d, 2);
+            else { printf("Q4_K, Q5_K or Q6_K (%d, %d, %d)\n", T_Q4_K, T_Q5_K, T_Q6_K); return 1; }
         }
-    }
-    if (zeros) std::fill(hp.begin(), hp.end(), 0);
-    uint8_t *planes; CK(hipMalloc(&planes, hp.size())); CK(hipMemcpy(planes, hp.data(), hp.size(), hipMemcpyHostToDevice));
+    const int copies = (int)std::max<size_t>(2, std::min<size_t>(64, ((size_t)600 << 20) / pb));
+    uint8_t *w, *planes;
+    CK(hipMalloc(&w, hw.size())); CK(hipMemcpy(w, hw.data(), hw.size(), hipMemcpyHostToDevice)); CK(hipMalloc(&planes, pb * copies));
+    for (int i = 0; i < copies; i++) CK(launch_mmq_expand(type, w, rb, N, K, planes + pb * i, nullptr));
     std::vector<int8_t> haq((size_t)T * K); std::vector<float> had((size_t)T * nb); std::vector<int16_t> hbs((size_t)T * K / 16);
     for (auto &v : haq) v = zeros ? 0 : (int8_t)((int)(rnd() % 255) - 127);
     for (auto &v : had) v = 0.01f + (rnd() & 1023) * 1e-4f;
@@ -63,10 +67,10 @@ int main(int argc, char **argv) {
     MMQWorkspace wsp; wsp.bytes = (size_t)4 * T * N * 4; CK(hipMalloc(&wsp.p, wsp.bytes));
     auto run = [&](int tiles, float *out, int split = 0) {
         mmq_set_tiles(tiles); mmq_set_split(split);
-        CK(launch_mmq_planes(type, planes, N, K, T, q, bh, bl, out, N, nullptr, nullptr, wsp));
+        for (int i = 0; i < copies; i++) CK(launch_mmq_planes(type, planes + pb * i, N, K, T, q, bh, bl, out, N, nullptr, nullptr, wsp));
         CK(hipDeviceSynchronize());
         CK(hipEventRecord(e0));
-        for (int i = 0; i < reps; i++) CK(launch_mmq_planes(type, planes, N, K, T, q, bh, bl, out, N, nullptr, nullptr, wsp));
+        for (int i = 0; i < reps; i++) CK(launch_mmq_planes(type, planes + pb * (i % copies), N, K, T, q, bh, bl, out, N, nullptr, nullptr, wsp));
         CK(hipEventRecord(e1)); CK(hipEventSynchronize(e1));
         float ms; CK(hipEventElapsedTime(&ms, e0, e1));
         return ms * 1e3f / reps;
