@@ -140,8 +140,9 @@ __global__ __launch_bounds__(256) void flash_attn_planes_kernel(const AttnArgs a
 // 32-block of nibbles, unpacked to the int8 codes nibble - 8 on its way into LDS (elements 0..15 from the low nibbles, 16..31 from the high ones), V codes
 // likewise; scores (vec_dot_q4_0_q8_0: the same integer dot with those codes), scales and the f16 hi / lo split of V' = code * d_v are the q8_0 path's.
 // PL (q8_0 and f16 caches): V's planes are in memory (flash_attn_planes_kernel), so a chunk goes to LDS as it is - no registers, no conversion, no scattered LDS stores: those were 3.1 of the
-// 7.8 kilocycles of a pair of chunks and made most of the 1.1 at the barrier; now 5.2, of which the two waves of a SIMD have 2 in matrix products and 3.3 in vector instructions, which bound
-// it (probe, 32 / 8 heads of 128, q8_0; 1919 tokens behind 2048: 382 -> 276 us, 2048 behind none 174 -> 134).  The block scales' products come from the matrix unit.  The same bits.
+// 7.8 kilocycles of a pair of chunks and made most of the 1.1 at the barrier; now 5.2, in which the two waves of a SIMD issue 64 matrix instructions, 2 kilocycles, and 930 vector
+// instructions, which bound it: at 3.4 cycles each the two add up to it (profiles/prompt_attention_probe.txt, prompt_long_pmc_mfma.json; 32 / 8 heads of 128, q8_0;
+// 1919 tokens behind 2048: 382 -> 276 us, 2048 behind none 174 -> 134).  The block scales' products come from the matrix unit.  The same bits.
 // (Tried: one of a SIMD's two waves half a chunk behind, its P.V beside the other's scores, in a third buffer: nothing.  Integer sums that start at the f32 bias: nothing.)
 template <int R, bool F16, int KH, int QS, int DH = 128, bool Q4 = false, bool PL = false>
 __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel(const AttnArgs a, const void *planes) {

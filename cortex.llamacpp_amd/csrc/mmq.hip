@@ -1088,9 +1088,10 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
 // pairs: a wave in an MFMA phase of its own leaves the vector unit idle, and one in a fold of its own the matrix cores.
 //
 // What bounds it: gate | up of an 8B layer (14336 x 4096 twice, Q4_K, 512 tokens) is 448 workgroups, two rounds of the 256 CUs of which the second is three quarters full; in each a SIMD issues
-// 2176 MFMAs of 32 cycles, so both rounds are 58 us at 2.4 GHz; but MFMAs of random operands alone run at 1.9 GHz here, with ten f32 instructions a pair of them at 1.5: the card's power.  What
-// instructions and bytes cost comes on top of the MFMAs, whichever unit has room: of a round of 73 us (2048 tokens) the MFMAs are 47, the fold 15, the expansion of codes 6, the activations'
-// way to LDS 3 to 6.  So bytes were taken out where instructions do not cost as much (us, before -> now, with weights from HBM): planes of 2 B a weight against Q4_K codes of 0.63 B: gate | up at 130, 256
+// 2176 MFMAs of 32 cycles, so both rounds are 58 us at 2.4 GHz; but MFMAs of random operands alone run at 1.6 GHz here, with ten f32 instructions a pair of them at 1.5, of zeros at 2.4: the
+// card's power.  What instructions and bytes cost comes on top of the MFMAs, whichever unit has room: of a round of 70 us (2048 tokens) the expansion of codes is 16, the fold 12, and what is
+// left without both 42 (copies of the kernel without the one, the other, both); of 55 with all-zero operands the activations' way to LDS is 3.  profiles/prompt_contraction.txt.
+// So bytes were taken out where instructions do not cost as much (us, before -> now, with weights from HBM): planes of 2 B a weight against Q4_K codes of 0.63 B: gate | up at 130, 256
 // and 512 tokens 70 -> 49, 79 -> 61, 159 -> 153; Q5_K as 1.5 B (a byte and a nibble: 6 instructions a K-step; as codes of a byte, 17, eight layers of a 7B model at 512 tokens 3179 us, as planes 3035,
 // so 2956): experts of an 8x7B layer, 611 tokens, gate | up 544 -> 455.
 // Tried, and slower: two 128 x 128 workgroups per CU, each with planes of its own (192 KiB), by 4 %; 16 x 16 x 64 MFMA tiles, which read twice the registers per product, the same; touching the

@@ -6,7 +6,7 @@ cd "$(dirname "$0")/.."
 name=$1; extra=$2; shift 2
 mkdir -p tools/bin/libs /tmp/libvar_$name
 B=cortex.llamacpp_amd/build
-F="--offload-arch=gfx950 -O3 -std=c++17 -fPIC -ffp-contract=off -fvisibility=hidden -Wall -Wno-unused-function -x hip"
+F="--offload-arch=gfx950 -O3 -Xclang -target-feature -Xclang -packed-fp32-ops -std=c++17 -fPIC -ffp-contract=off -fvisibility=hidden -Wall -Wno-unused-function -x hip"
 objs=""
 # (the objects the tree's library was linked from: build.py writes the list - the build directory may hold objects of the other experiments setting)
 for o in $(cat $B/linked_objects.txt); do

@@ -4,7 +4,7 @@
   pass 2: SQ_INSTS_VALU SQ_INSTS_MFMA SQ_INSTS_VALU_MFMA_MOPS_I8 GRBM_GUI_ACTIVE
 SQ_VALU_MFMA_BUSY_CYCLES = 32 per v_mfma_i32_32x32x32_i8, summed over SIMDs; GRBM_GUI_ACTIVE is summed over the 8 XCDs:
 available SIMD-cycles = GRBM_GUI_ACTIVE / 8 * 256 CUs * 4 SIMDs.
-usage: tools/pmc_prefill.py <pass1.db> <pass2.db> <out.json> [note]"""
+usage: tools/pmc_prefill.py <pass1.db> <pass2.db> <out.json> [prompt tokens]"""
 import json
 import sqlite3
 import sys
@@ -24,8 +24,7 @@ def load(path):
 
 
 a, b = load(sys.argv[1]), load(sys.argv[2])
-out = {"source": "two rocprofv3 --pmc passes with --kernel-trace over python3 tools/decode_loop.py 1 512 (MI355_NO_GRAPHS=1 MI355_PROFILER_SAFE=1)"
-                 + (": " + sys.argv[4] if len(sys.argv) > 4 else ""),
+out = {"source": "two rocprofv3 --pmc passes with --kernel-trace over python3 tools/decode_loop.py 1 %s (MI355_NO_GRAPHS=1 MI355_PROFILER_SAFE=1)" % (sys.argv[4] if len(sys.argv) > 4 else "512"),
        "units": __doc__.split("\n")[3:6], "kernels": {}}
 for k in sorted(set(a) | set(b)):
     c = dict(a.get(k, {})); c.update(b.get(k, {}))
