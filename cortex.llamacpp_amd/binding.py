@@ -89,6 +89,7 @@ SYMBOLS = {
     "mi355_debug_q80_plan": (_i32, [_i32] * 3),
     "mi355_debug_attn_plan": (_i32, [_i32] * 7),
     "mi355_debug_attn_planes_plan": (C.c_int64, [_i32] * 6),
+    "mi355_debug_attn_planes_taken": (_i32, [_i32] * 7),
     "mi355_set_embeddings": (None, [_vp, _i32]),
     "mi355_get_embeddings_ith": (C.POINTER(C.c_float), [_vp, _i32]),
     "mi355_synchronize": (None, [_vp]),

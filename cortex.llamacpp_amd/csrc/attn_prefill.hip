@@ -784,15 +784,30 @@ size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int H, int G, int
     const size_t b = (size_t)((n_ctx + CK - 1) / CK) * G * plane_chunk_bytes(f16, D);
     return b <= ((size_t)256 << 20) ? b : 0;
 }
-// The planes of the scanned cells cost 6 us a layer at 4096 cells of eight kv heads, and spare a query tile 2 of 5 parts of its time: from eight tiles on that see all the cells, or as many more
-// as they see less of them (us, planes / every tile on its own: 1919 tokens behind 2048 a layer 276 + 7 / 382; four tiles break even).
-bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible) {
-    const int tiles = (T + QT * fa_sub_tiles(H / G) - 1) / (QT * fa_sub_tiles(H / G));
-    return (long)tiles * std::min(n_kv, visible) >= 8L * n_kv;
+// The planes of the scanned cells cost 3 to 6 us a layer at up to 4096 cells of eight kv heads, and spare a query tile two of five parts of its time with a chunk.  So from eight tiles on that see
+// all the cells, or as many more as they see less of them (1919 tokens behind 2048 276 + 7 us a layer, every tile on its own 382; four tiles break even), and enough keys a query that what is
+// spared is more than the first chunk's way from memory, which nothing hides (us a layer, own conversion | planes and kernel; tokens behind cells).  Both sides of 256 k (token, key) pairs:
+//   32 / 8 heads of 128, q8_0   520 / 0 36.6 | 40.0, 600 / 0 40.6 | 41.8, 700 / 0 45.4 | 45.9, 850 / 0 57.4 | 54.7, 520 / 300 54.5 | 52.1, 1024 / 0 75.6 | 60.0
+//   64 / 8 heads of 128, f16    260 / 0 26.0 | 28.2, 520 / 0 36.4 | 39.4, 700 / 0 46.8 | 47.9, 750 / 0 53.2 | 53.8, and q8_0 with fewer, as its conversion takes more: 600 / 0 51.5 | 51.6,
+//   40 / 8 of them 520 / 0 55.9 | 57.1, 600 / 0 58.4 | 55.2, 700 / 0 68.4 | 62.5
+// Eight waves that share the conversion of 64-wide f16 values spare little, and where they are several workgroups to a tile only what every query sees counts:
+//   32 / 4 heads of 64, f16     1024 / 0 38.7 | 39.9, 1600 / 0 58.4 | 63.8, 2000 / 0 80.6 | 85.8, 1600 / 500 82.2 | 83.5, 850 / 300 46.7 | 43.3, 2000 / 1000 131.6 | 125.9
+//   64 / 8 (one workgroup)      1600 / 0 87.3 | 86.7, 2000 / 0 124.5 | 111.5
+// Several prompts of one batch, 32 / 8 heads of 128, q8_0: 2 x 1000 168.7 | 139.6, 4 x 500 120.5 | 105.6, 12 x 160 49.7 | 50.5.
+static bool fa_planes_pay(int type_v, long T, int R, int n_kv, int seen, long keys2) {       // keys2: twice a query's keys on average
+    const int q = QT * fa_sub_tiles(R);
+    return (T + q - 1) / q * seen >= 8L * n_kv && T * keys2 >= (R > 4 && type_v != T_F16 ? 400000 : 512000);
+}
+bool flash_attn_prefill_planes_pay(int type_v, int T, int H, int G, int D, int n_kv, int visible) {
+    const int R = H / G, seen = std::min(n_kv, visible);
+    const long keys2 = std::max(2L * seen - T, (long)seen);    // (several conversations in the batch: half of what the longest one's last query sees)
+    if (!fa_planes_pay(type_v, T, R, n_kv, seen, keys2)) return false;
+    return !(type_v == T_F16 && D == 64 && R == 8 && 3 * keys2 < 5L * T && flash_attn_prefill_splits(T, H, G, D, seen) > 1);
 }
 size_t flash_attn_prefill_planes_wanted(int type_k, int type_v, int H, int G, int D, int n_ctx, int n_ubatch) {
     const size_t b = flash_attn_prefill_planes_bytes(type_k, type_v, H, G, D, n_ctx);
-    return b && flash_attn_prefill_planes_pay(n_ubatch, H, G, 1, 1) ? b : 0;
+    const long T = std::min(n_ubatch, n_ctx);
+    return b && fa_planes_pay(type_v, T, H / G, n_ctx, n_ctx, 2L * n_ctx - T) ? b : 0;
 }
 
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *v_planes) {

@@ -288,6 +288,9 @@ int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv
 int64_t mi355_debug_attn_planes_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_ctx, int32_t n_ubatch) {
     return (int64_t)flash_attn_prefill_planes_wanted(type_kv, type_kv, n_head, n_head_kv, head_dim, n_ctx, n_ubatch);
 }
+int32_t mi355_debug_attn_planes_taken(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t n_visible) {
+    return flash_attn_prefill_planes_bytes(type_kv, type_kv, n_head, n_head_kv, head_dim, n_cells) && flash_attn_prefill_planes_pay(type_kv, n_tokens, n_head, n_head_kv, head_dim, n_cells, n_visible);
+}
 int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int32_t type_v, int32_t type_o, int32_t n_embd, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
                                   int32_t type_kv, int32_t n_kv, int32_t *slots_out) {
     int slots = 0;

@@ -176,7 +176,7 @@ bool mmq_planes_swiglu_ok(int type_gate, int type_up, int n_rows, int K, int T);
 hipError_t launch_mmq_planes_swiglu(int type, const uint8_t *planes_gate, const uint8_t *planes_up, int n_rows, int K, int T, const ActQuant &q,
                                     float *out, int ld_out, hipStream_t st);
 bool mmq_ksplit_applicable(int type, int K, int T);
-// ... and preferred over the planes kernels for a tensor (or the concatenation of a launch's) of n_rows rows.  has_planes: the pre-expanded planes exist; sum_free: the caller
+// ... and preferred over the planes kernels for a tensor (or the concatenation of a launch's) of n_rows rows.  has_planes: the tensor has its planes; sum_free: the caller
 // takes a K split's partial sums as they are (launch_mmq_planes's parts); pair: n_rows rows each of ffn_gate and ffn_up
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair = false);
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
@@ -672,7 +672,7 @@ int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max);
 // planes (nullable): flash_attn_prefill_planes_bytes() for the V planes of the scanned cells, made once for all query tiles
 hipError_t launch_flash_attn_prefill(const AttnArgs &a, hipStream_t st, void *planes = nullptr);
 size_t flash_attn_prefill_planes_bytes(int type_k, int type_v, int H, int G, int D, int n_ctx);     // of a cache; 0: no such form, or more than 256 MiB
-bool flash_attn_prefill_planes_pay(int T, int H, int G, int n_kv, int visible);               // n_kv cells scanned, of which a query can see at most `visible`
+bool flash_attn_prefill_planes_pay(int type_v, int T, int H, int G, int D, int n_kv, int visible);    // n_kv cells scanned, of which a query can see at most `visible`
 size_t flash_attn_prefill_planes_wanted(int type_k, int type_v, int H, int G, int D, int n_ctx, int n_ubatch);      // by a decoder's context: 0 too where no batch is long enough for them to pay
 // a short batch of one sequence, a short text through the encoder: the same in another split of the work (attn_cols.hip); pf_splits = flash_attn_cols_splits
 bool flash_attn_cols_applicable(const AttnArgs &a);

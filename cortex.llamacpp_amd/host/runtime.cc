@@ -1620,7 +1620,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             // extra workgroup would scan the whole cell table)
             aa.pf_splits = cols ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(T, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
             while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
-            void *const planes = !cols && flash_attn_prefill_planes_pay(T, H, G, n_kv_max, cur_max_pos_ + 1) ? att_planes_ : nullptr;
+            void *const planes = !cols && flash_attn_prefill_planes_pay(cp.type_v, T, H, G, D, n_kv_max, cur_max_pos_ + 1) ? att_planes_ : nullptr;
             HIP_TRY(cols ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_, planes));
         }
         prof_mark("attn");

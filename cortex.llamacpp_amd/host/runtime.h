@@ -29,7 +29,7 @@ struct DevTensor {
     size_t row_bytes = 0;   // device row stride
     size_t bytes = 0;       // device bytes
     size_t ggml_bytes = 0;  // on-disk bytes
-    uint8_t *planes = nullptr;   // pre-expanded MFMA operand planes for prompt processing (mmq.hip), optional
+    uint8_t *planes = nullptr;   // MFMA operand planes for prompt processing, or the codes that the kernel makes them of (mmq.hip), optional
     size_t planes_bytes = 0;
     bool valid() const { return data != nullptr; }
 };

@@ -68,7 +68,7 @@ typedef struct mi355_model_params {
     /* row split over RCCL (see mi355_tp_init below; new keys proposed in SURVEY.md §2b) */
     int32_t tp_rank;        /* 0 when tp_size <= 1 */
     int32_t tp_size;        /* 1 = whole model on this GPU */
-    /* prompt-processing copy of the projection weights as pre-expanded int8 MFMA operand planes (up to 2 B / weight):
+    /* prompt-processing copy of the projection weights as int8 MFMA operand planes, or what they are made of (0.6 to 2 B / weight):
      * -1 = keep it when device memory allows (default), 0 = never (expand on the fly), 1 = required */
     int32_t prefill_planes;
 } mi355_model_params;
@@ -187,6 +187,8 @@ MI355_API int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t
 /* host logic only: bytes that a decoder's context of n_ctx cells (K and V of type_kv) and n_ubatch tokens a micro-batch keeps for the V planes of a prompt's attention
    (csrc/attn_prefill.hip); 0 where no micro-batch takes that form */
 MI355_API int64_t mi355_debug_attn_planes_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_ctx, int32_t n_ubatch);
+/* host logic only: 1 = n_tokens in the prompt kernel over n_cells cells, of which a query can see n_visible at most, take that form */
+MI355_API int32_t mi355_debug_attn_planes_taken(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t n_visible);
 /* llama_set_embeddings (ctx.cc:299) */
 MI355_API void    mi355_set_embeddings(mi355_context *ctx, int32_t enabled);
 /* llama_get_embeddings_ith (ctx.cc:1042-1044): final-norm hidden state (n_embd floats, host memory) of batch row i of the

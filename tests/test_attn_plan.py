@@ -46,3 +46,23 @@ def test_planes_workspace(pkg, model, n, bytes_):
 def test_no_planes_workspace_without_a_form(pkg, model):
     """64-wide heads in threes, fives, sixes, sevens; a q4_0 cache; more than eight query heads to a kv head; other widths."""
     assert pkg.load_library().mi355_debug_attn_planes_plan(*model, 4096, 2048) == 0
+
+
+@pytest.mark.parametrize("model,yes,no", [
+    (L8, [(850, 0), (520, 300), (1024, 0), (1919, 2048), (300, 2000)], [(520, 0), (600, 0), (700, 0), (224, 3500)]),
+    ((F16, 64, 8, 128), [(850, 0), (600, 300), (1024, 0)], [(260, 0), (520, 0), (700, 0)]),
+    ((Q8_0, 40, 8, 128), [(700, 0), (520, 300)], [(420, 0), (520, 0)]),
+    (L7, [(1000, 0), (2000, 2000)], [(896, 3000)]),
+    (SMALL, [(850, 300), (800, 1100), (2000, 1000), (1024, 1000)], [(1024, 0), (1600, 0), (2000, 0), (1600, 500)]),
+    ((F16, 64, 8, 64), [(2000, 0), (1600, 500)], [(520, 0), (950, 0)]),
+])
+def test_planes_where_they_pay(pkg, model, yes, no):
+    """Launches timed with and without the V planes of a prompt's attention, the planes' own launch among them: fresh prompts of few keys convert for themselves."""
+    taken = pkg.load_library().mi355_debug_attn_planes_taken
+    assert [c for c in yes if taken(*model, c[0], sum(c), sum(c)) != 1] == [] and [c for c in no if taken(*model, c[0], sum(c), sum(c)) != 0] == []
+
+
+def test_planes_of_several_conversations(pkg):
+    """Four prompts of 500 tokens in one batch: a query sees 250 keys of 2000 on average, as many as in the prompt alone, for four times the tiles; sixteen of 125 see too few for the cells scanned."""
+    taken = pkg.load_library().mi355_debug_attn_planes_taken
+    assert taken(*L8, 2000, 2000, 500) == 1 and taken(*L8, 2000, 2000, 125) == 0
