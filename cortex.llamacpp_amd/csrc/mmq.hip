@@ -1594,6 +1594,8 @@ static int planes2_split(int n_rows, int K, int T, const MMQWorkspace &wsp, bool
 // workspace allows it.  The choice is by the two launches' times.  Both are whole rounds of one workgroup a CU, and a round is its super-blocks and a start (us): K-split, 32 rows x 64
 // tokens, an eighth of the super-blocks of 5.2 and 3.5; tiles, the part's super-blocks of 1.5 + T / 128, to 128 tokens of Q6_K, which they read as two bytes a weight, 2 + T / 128, and 7, and 4
 // more where the parts' sum is a launch of its own.
+// From 97 to 128 tokens a workgroup has four tiles of 32 and takes as long as at 128: gate | up of 5632 x 2048, Q4_K, at 100 tokens 24.4 / 27.0, ten layers of it at 97, 100 and 112 with the
+// tiles 929, 933, 940 us and without 905, 911, 919.
 // Measured with weights from HBM, Q4_K, K-split / tiles without the sum's launch, at 72, 128 and 256 tokens (Q5_K costs either kernel a tenth more):
 //   2048 x 2048   9/13 9/15 10/18     2048 x 5632  18/18 19/20 20/24    1536 x 8960   23/23 27/27 26/34     gate | up of 5632 x 2048    25/24 25/27 44/32
 //   3072 x 3072  11/14 12/16 19/19    3072 x 8192  24/22 24/25 43/31    5120 x 5120   28/17 28/19 42/24     gate | up of 8192 x 3072    40/32 41/37 74/44
@@ -1608,7 +1610,7 @@ static bool tiles_beat_ksplit(int type, int n_rows, int K, int T, MMQWorkspace w
     if (!takes) return n_rows >= 8192 && !(pair && T <= 128);  // (then the planes kernel below, by rows; ffn_gate | ffn_up are one launch here and two there)
     const auto up = [](long a, long b) { return (double)((a + b - 1) / b); };
     const double here = up(up(rows, 32) * up(T, 64), num_cu()) * (5.2 * nb / 8 + 3.5);
-    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * (((type == T_Q6_K && T <= 128 ? 2.0 : 1.5) + T / 128.0) * up(nb, parts) + 7.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
+    const double tiles = up(up(rows, P2_ROWS) * up(T, P2_TOK) * parts, num_cu()) * (((type == T_Q6_K && T <= 128 ? 2.0 : 1.5) + (T > 96 && T < 128 ? 128 : T) / 128.0) * up(nb, parts) + 7.0) + (parts > 1 && !sum_free ? 4.0 : 0.0);
     return tiles < here;
 }
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair) {

@@ -70,6 +70,12 @@ def test_from_65_tokens_by_the_bytes_of_a_type(plan, n):
         assert [plan(t, 4096, 14336, n, 0, 1) for t in (Q4_K, Q5_K)] == [PLANES] * 2
 
 
+@pytest.mark.parametrize("n", [97, 100, 112, 113, 128])
+def test_the_fourth_tile_of_32_tokens(plan, n):
+    """gate | up of 5632 x 2048 from 97 tokens on: the tiles take as long as at 128, 27 us, the K-split kernel 24."""
+    assert [plan(t, 5632, 2048, n, 1, 0) for t in (Q4_K, Q5_K, Q6_K)] == [KSPLIT] * 3
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("n", [161, 180, 212, 256])
 def test_the_square_tensor_of_4096_columns(plan, t, n):
