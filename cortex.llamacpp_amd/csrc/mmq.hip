@@ -1082,7 +1082,7 @@ __global__ __launch_bounds__(NTHREADS) void mmq_planes_kernel(const uint8_t *pla
 // steps ahead of the first token tile.  The 256 x 256 activation codes come by LDS-DMA one super-block ahead (two buffers, one barrier per super-block):
 //   codes  64 KiB = [token 0..255][16 pieces of 16 B]; piece p of token t sits in slot p ^ (t & 15) (applied on the SOURCE side of the DMA, whose LDS side is
 //          lane-linear), so the 16 lanes of a ds_read_b128 phase hit all 64 banks
-//   block sums 8 KiB (int16, turned into f16 in place by the wave that fetched them), the rows' words (scales, d / dmin / mins; once, for both halves), and the tokens' scales (three sets: a
+//   block sums 8 KiB (int16, turned into f16 in place by the wave that fetched them), the rows' words (scales, d / dmin / mins), and the tokens' scales (three sets: a
 //          fold reaches into the next super-block)
 // The f32 fold of a token tile (five vector instructions an output) runs BETWEEN the MFMAs of the next tile, two outputs per K-step, on the other of two accumulator
 // pairs: a wave in an MFMA phase of its own leaves the vector unit idle, and one in a fold of its own the matrix cores.
@@ -1132,8 +1132,8 @@ __device__ __forceinline__ gbytes *scalar_ptr(const void *p) {
     const uint64_t v = (uint64_t)p;
     return (gbytes *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32);
 }
-// NT: token tiles of 32; FULL: every token of the workgroup's tile exists
-template <int FORM, int NT, bool FULL>
+// NT: token tiles of 32; FULL: every token of the workgroup's tile exists.  SHARED: the rows' words, the same for both halves, come once, by the first (codes: two sets do not fit)
+template <int FORM, int NT, bool FULL, bool SHARED>
 __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int sb_lo, int nb, int tok0, int tid, int tw, uint8_t *smem_wg, float (&facc)[4][16]) {
     constexpr bool MINS = FORM != PF_SIGNED, PACKED = FORM >= PF_CODES;
     constexpr int SH = plane_shift(FORM), BLOCK = plane_block(FORM), WORDS = plane_words(FORM);
@@ -1141,18 +1141,20 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
     const int n = lane & 31, kg = lane >> 5;
     const int nb_all = a.K >> 8;
-    const uint8_t *sm_bs = smem_wg + P2_BS + tw * 4096, *sm_meta = smem_wg + P2_META, *sm_yd = smem_wg + P2_YD + tw * P2_YDB, *sm_a = smem_wg + tw * 32768;
+    const uint8_t *sm_bs = smem_wg + P2_BS + tw * 4096, *sm_yd = smem_wg + P2_YD + tw * P2_YDB, *sm_a = smem_wg + tw * 32768;
+    const unsigned meta_at = FORM == PF_CODES ? (unsigned)wave * 1024u : (unsigned)((SHARED ? 0 : tw * 4) + wave) * 512u;
+    const uint8_t *sm_meta = smem_wg + P2_META + meta_at;
     const unsigned lds0 = lds_addr32(smem_wg);
     const int last = a.T - 1 - tok0;                            // (tokens past the end read the last one; never stored)
     auto dma = [&](int sb, int buf, int y3) {                   // tokens 32 wave .. + 31 of super-block sb, and the scale words of the wave's rows
         const unsigned dst = lds0 + (unsigned)buf * P2_BUF;
         int l = lane;
         asm volatile("" : "+v"(l));                             // (the offsets are formed here, every time: hoisted out of the loop they would cost ten registers)
-        if (tw == 0) {                                          // (both halves' rows are the same)
+        if (!SHARED || tw == 0) {
             const uint8_t *mw = (const uint8_t *)scalar_ptr((const uint8_t *)blk0 + (size_t)sb * BLOCK + WORDS);
-            const unsigned to = dst + P2_META + (unsigned)wave * 1024u;
+            const unsigned to = dst + P2_META + meta_at;
             if (FORM == PF_CODES) dma16_s(mw, l * 16u, to);
-            else { dma4_s(mw, l * 4u, to + 512u); dma4_s(mw + 256, l * 4u, to + 768u); }
+            else { dma4_s(mw, l * 4u, to); dma4_s(mw + 256, l * 4u, to + 256u); }
         }
         const size_t sbg = (size_t)(sb_lo + sb);
         if (NT == 4 || wave < NT) {
@@ -1209,7 +1211,7 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     convert(0);
     __syncthreads();
-    const bool nib = FORM == PF_MINS && __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(sm_meta + 512 + 12));       // Q2_K planes: sixteen 4-bit mins
+    const bool nib = FORM == PF_MINS && __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int *>(smem_wg + P2_META + (SHARED ? 0 : tw * 2048) + 12));       // Q2_K planes: sixteen 4-bit mins
 
     i32x16 H[2], L[2];                                          // [tile parity]
     f32x16 ms;
@@ -1245,10 +1247,10 @@ __device__ __forceinline__ void planes2_loop(gbytes *blk0, const P2Args &a, int 
         asm volatile("" : "+v"(x));
         auto ld_a = [&](int t, int j) { return *reinterpret_cast<const i32x4 *>(sm_a + sbuf + t * 8192 + (x ^ (unsigned)(32 * j))); };
         i32x4 A[2];
-        u32x4 meta = *reinterpret_cast<const u32x4 *>(sm_meta + sbuf + wave * 1024 + 512 + n * 16);
+        u32x4 meta = *reinterpret_cast<const u32x4 *>(sm_meta + sbuf + (FORM == PF_CODES ? 512 : 0) + n * 16);
         A[0] = ld_a(0, 0); A[1] = ld_a(0, 1);
         uint32_t sw = 0;
-        auto scales = [&](int c) { if (FORM == PF_CODES) sw = *reinterpret_cast<const uint32_t *>(sm_meta + sbuf + wave * 1024 + n * 16 + c * 4); };
+        auto scales = [&](int c) { if (FORM == PF_CODES) sw = *reinterpret_cast<const uint32_t *>(sm_meta + sbuf + n * 16 + c * 4); };
         auto expand = [&](auto J) { constexpr int j = J.value; if constexpr (PACKED) expand_words<FORM, j>(raw[j >> 1], sw, B[j][0], B[j][1]); };
         scales(0);
         __builtin_amdgcn_sched_barrier(0);
@@ -1350,7 +1352,10 @@ __device__ __forceinline__ void planes2_body(const P2Args &a, const PlanesOut &p
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) facc[t][r] = 0.0f;
-#define P2_LOOP(NTV, FULLV) planes2_loop<FORM, NTV, FULLV>(blk0, a, sb_lo, nb, tok0, tid, tw, smem, facc)
+    // In mmq_planes2_kernel a half of fewer than four tiles fetches its rows' words itself (a second half of four means a first one): there the branch costs more than the requests, in gate | up and
+    // the experts' launches, which fill the chip, less (us, once | by each half: 4096 x 14336 of Q6_K at 129 and 160 tokens 51.6 | 50.0, 53.5 | 51.1, of Q5_K at 80 37.8 | 36.5; gate | up of
+    // 14336 x 4096 at 80 tokens of Q6_K 57.2 | 58.6, at 300 of Q5_K 107.9 | 109.6, at 1000 297 | 300).
+#define P2_LOOP(NTV, FULLV) planes2_loop<FORM, NTV, FULLV, ONE || NTV == 4 || FORM == PF_CODES>(blk0, a, sb_lo, nb, tok0, tid, tw, smem, facc)
     if (nt == 4 && T - tok0 >= 128) P2_LOOP(4, true);
     else if (nt == 4) P2_LOOP(4, false);
     else if (nt == 3) P2_LOOP(3, false);
