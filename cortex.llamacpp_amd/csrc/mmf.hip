@@ -19,6 +19,8 @@ namespace {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 // WT = 32 x 32 tiles a wave holds per side: 2 -> a workgroup covers 128 x 128 outputs, 1 -> 64 x 64 (four times the workgroups: shapes whose 128-tiles would leave
 // most of the 256 CUs idle - the LLaVA tower's 577 x 1024 projections are 40 of them).  Every output is the same chain of matrix-core steps over k either way.
@@ -241,8 +243,9 @@ namespace {
 // The encoder's projections (T tokens of one text against f16 weights of a few hundred to a few thousand columns): a product is 19 MB of weights at the most and
 // some microseconds of anything, so what counts is one trip to memory, enough workgroups and no launches around it.  Measured on nomic-embed (768 / 3072 columns)
 // at 187 tokens, us: 768 x 768 30 with the 64 x 64 direct
-// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; now Q | K | V 7.6, output 6.1, gate | up 11.6, down 9.6.  Here:
-//   * 32 rows x 32 TT tokens per workgroup (432 workgroups for Q | K | V at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
+// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; here, launches back to back, Q | K | V 6.1, output 3.8, gate | up 9.5, down 7.1, and
+// Q | K | V and gate | up of 768 columns as mmf16_rows_kernel below has them 5.1 and 9.0:
+//   * 32 rows x 32 TT tokens per workgroup (144 workgroups for the output at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
 //     both operands - all of them for 768 columns - are requested before the first matrix step;
 //   * a request is whole 128-byte lines of eight rows; the operands (16 bytes of 32 rows) are made through LDS of the wave's own, pieces of a row turned by its number.  Asked for as
 //     operands, 32 lines per request: gate | up 20.8 us at 187 tokens and 92 at 1800;
@@ -341,6 +344,19 @@ __global__ __launch_bounds__(64 * NW, EPI == FEW_SWIGLU && NW == 4 && TT == 1 ? 
     };
 #pragma unroll
     for (int u = 0; u < PD; u++) { fetch(s[u], u); __builtin_amdgcn_sched_barrier(0); }               // (in the order of their use: a wait for one slot is not one for the next)
+    // what a plain product adds on its way out, behind them (asked for there it was a trip to memory of its own, 0.3 to 0.5 us a launch): a thread's outputs are all of one weight row
+    constexpr int NE = (1024 * TT + 64 * NW - 1) / (64 * NW);
+    const int er = tid & 31, en = n0 + er;
+    float rv[EPI == FEW_PLAIN ? NE : 1], bv = 0.0f;
+    if constexpr (EPI == FEW_PLAIN) {
+        const int nn = en < a.N ? en : a.N - 1;
+        if (a.bias) bv = a.bias[nn];
+        if (a.resid) {
+#pragma unroll
+            for (int j = 0; j < NE; j++) { const int g = t0 + (tid >> 5) + 2 * NW * j; rv[j] = a.resid[(size_t)(g < a.T ? g : a.T - 1) * a.N + nn]; }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     int i = 0;
     for (; i + PD < cn; i += PD)                             // (no branch around a request: it would become a wait for all of them)
 #pragma unroll
@@ -364,8 +380,10 @@ __global__ __launch_bounds__(64 * NW, EPI == FEW_SWIGLU && NW == 4 && TT == 1 ? 
                 *reinterpret_cast<f32x4 *>(part + (((wave * NP + p) * TT + t) * 32 + m) * LD + 8 * q + 4 * kg) =
                     f32x4{acc[p][t][4 * q], acc[p][t][4 * q + 1], acc[p][t][4 * q + 2], acc[p][t][4 * q + 3]};
     __syncthreads();
-    for (int e = tid; e < 1024 * TT; e += 64 * NW) {
-        const int row = e & 31, t = e >> 5, gt = t0 + t, n = n0 + row;
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+        const int row = er, t = (tid >> 5) + 2 * NW * j, gt = t0 + t, n = en;
+        if (t >= 32 * TT) break;
         float v[NP];
 #pragma unroll
         for (int p = 0; p < NP; p++) {
@@ -389,24 +407,147 @@ __global__ __launch_bounds__(64 * NW, EPI == FEW_SWIGLU && NW == 4 && TT == 1 ? 
             if constexpr (EPI == FEW_SWIGLU) a.out_h[o] = (_Float16)((v[0] / (1.0f + expf(-v[0]))) * v[1]);
             else {
                 float y = v[0];
-                if (a.bias) y = y + a.bias[n];
-                if (a.resid) y = a.resid[o] + y;
+                if (a.bias) y = y + bv;
+                if (a.resid) y = rv[j] + y;
                 a.out[o] = y;
             }
         }
     }
 }
-template <int NW, int EPI, bool XF>
-void few_launch(const MMF16Few &a, hipStream_t st) {
+// Two products of the same tokens (gate and up, or the halves of 64-wide heads) where K is at most ROWS_K columns and there are few workgroups: 32 rows of each x 32 tokens per workgroup, whose
+// activation rows are whole in LDS, staged once by all; of the eight waves four take the one product and four the other, a chunk of 64 columns in four each, all of a wave's weights
+// requested at once.  What bounds such a launch is a wave's own chain of instructions - one or two waves a SIMD, some thousand of them - and in the form above a wave stages both products and the
+// tokens for itself.  768 columns, us, this form / that one: Q | K | V at 40, 187, 300, 700, 1000 tokens 4.9 / 5.9, 5.1 / 5.9, 6.9 / 7.6, 11.4 / 12.1, 14.1 / 16.5, at 1800 24.5 / 23.4; gate | up at
+// 40, 187, 300, 400, 700 5.0 / 5.3, 9.1 / 9.3, 11.1 / 11.3, 13.4 / 13.2, 23.4 / 21.3.  Twelve waves, two chunks each: 5.2 and, with one workgroup a CU, 11.8 at 187.  With the LayerNorm in front of
+// it in the launch, every workgroup norming its rows: 7.9 and 15.1, a launch of the norm is 2.7.
+constexpr int ROWS_K = 768;
+template <int EPI>
+__global__ __launch_bounds__(512, 4) void mmf16_rows_kernel(const MMF16Few a) {
+    constexpr int ROWS = EPI == FEW_ROPE ? 64 : 32, KJ = ROWS_K / 64, NK = 4, PD = KJ / NK, LD = 36;
+    constexpr int X_BYTES = 32 * KJ * 128, W_BYTES = 8 * 4096;
+    static_assert(8 * 32 * LD * 4 <= X_BYTES + W_BYTES && KJ % NK == 0 && KJ % 2 == 0, "the partial tiles take the operands' place");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[X_BYTES + W_BYTES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), p = wave & 1, ks = wave >> 1, m = lane & 31, kg = lane >> 5;
+    const int n0 = blockIdx.x * ROWS, t0 = blockIdx.y * 32, nc = a.K >> 6, r8 = lane >> 3, c8 = lane & 7;
+    uint8_t *const sx = smem, *const sw = smem + X_BYTES + wave * 4096;
+    // the tokens' rows, sixteen threads a row (past the end the last one's; a piece past K is the row's first, and not staged), then the wave's chunks of its product's rows
+    const int row = tid >> 4, l16 = tid & 15;
+    f16x8 v[KJ / 2];
+    {
+        const int gt = t0 + row < a.T ? t0 + row : a.T - 1;
+        const unsigned o = ((unsigned)gt * (unsigned)a.K + 8u * l16) * 2u;
+#pragma unroll
+        for (int j = 0; j < KJ / 2; j++) v[j] = *reinterpret_cast<const f16x8 *>(reinterpret_cast<const uint8_t *>(a.X) + (o + (128 * j + 8 * l16 < a.K ? 256u * j : 0u)));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t *const W = reinterpret_cast<const uint8_t *>(p ? a.W2 : a.W);
+    unsigned wrow[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { const int g = n0 + r8 + 8 * i; wrow[i] = ((unsigned)(g < a.N ? g : a.N - 1) * (unsigned)a.K + 8u * c8) * 2u; }
+    f16x8 w[PD][4];
+#pragma unroll
+    for (int u = 0; u < PD; u++) {
+        const unsigned k = 128u * (unsigned)(ks + NK * u < nc ? ks + NK * u : nc - 1);
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[u][j] = *reinterpret_cast<const f16x8 *>(W + (wrow[j] + k));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // a thread's output: a token and a pair of rows of either product; what the pairs are turned by, and their cell
+    const int et = tid >> 4, er = 2 * (tid & 15), gt = t0 + et;
+    f32x4 cv = {0.0f, 0.0f, 0.0f, 0.0f};
+    int cl = 0;
+    if constexpr (EPI == FEW_ROPE) { const int q = gt < a.T ? gt : a.T - 1; cv = *reinterpret_cast<const f32x4 *>(a.cs + (size_t)q * 64 + 2 * er); cl = a.cell[q]; }
+    __builtin_amdgcn_sched_barrier(0);
+    // (a chunk of a row is 128 bytes; piece c of row r at c ^ (r & 7): no bank conflicts either way)
+#pragma unroll
+    for (int j = 0; j < KJ / 2; j++) { const int c = 2 * j + (l16 >> 3); if (c < nc) *reinterpret_cast<f16x8 *>(sx + (row * KJ + c) * 128 + 16 * ((l16 & 7) ^ (row & 7))) = v[j]; }
+    __syncthreads();
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < PD; u++) {
+        const int c = ks + NK * u;
+        if (c < nc) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) *reinterpret_cast<f16x8 *>(sw + (r8 + 8 * j) * 128 + 16 * (c8 ^ r8)) = w[u][j];
+            __builtin_amdgcn_wave_barrier();                 // (a wave's LDS accesses are made in order)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int o = 16 * ((2 * j + kg) ^ (m & 7));
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8 *>(sw + m * 128 + o), *reinterpret_cast<const f16x8 *>(sx + (m * KJ + c) * 128 + o), acc, 0, 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    __syncthreads();
+    float *const part = reinterpret_cast<float *>(smem);     // (registers as in mmf16_few_kernel)
+#pragma unroll
+    for (int q = 0; q < 4; q++) *reinterpret_cast<f32x4 *>(part + (wave * 32 + m) * LD + 8 * q + 4 * kg) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    __syncthreads();
+    if (gt >= a.T || n0 + er >= a.N) return;
+    f32x2 y[2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+#pragma unroll
+    for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) y[q] += *reinterpret_cast<const f32x2 *>(part + ((2 * k + q) * 32 + et) * LD + er);
+    if constexpr (EPI == FEW_SWIGLU) {
+        *reinterpret_cast<f16x2 *>(a.out_h + (size_t)gt * a.N + n0 + er) = f16x2{(_Float16)((y[0].x / (1.0f + expf(-y[0].x))) * y[1].x), (_Float16)((y[0].y / (1.0f + expf(-y[0].y))) * y[1].y)};
+    } else {
+        const int E = a.N / 3, s = (n0 >= E) + (n0 >= 2 * E), c0 = n0 - s * E;         // (a head is a whole tile, a segment whole heads)
+        if (s < 2) {
+            const f32x2 c = {cv.x, cv.z}, sn = {cv.y, cv.w}, b0 = y[0], b1 = y[1];
+            y[0] = b0 * c - b1 * sn;
+            y[1] = b0 * sn + b1 * c;
+        }
+        if (s == 0) { float *q = a.out + (size_t)gt * E + c0 + er; *reinterpret_cast<f32x2 *>(q) = y[0]; *reinterpret_cast<f32x2 *>(q + 32) = y[1]; }
+        else {
+            uint16_t *d = (s == 1 ? a.kc : a.vc) + ((size_t)(c0 >> 6) * a.n_ctx + cl) * 64 + er;
+            *reinterpret_cast<unsigned *>(d) = (unsigned)f2h(y[0].x) | ((unsigned)f2h(y[0].y) << 16);
+            *reinterpret_cast<unsigned *>(d + 32) = (unsigned)f2h(y[1].x) | ((unsigned)f2h(y[1].y) << 16);
+        }
+    }
+}
+template <int NW, int EPI, int TT, int PD, bool XF>
+void few_go(const MMF16Few &a, hipStream_t st) {
     const int rows = EPI == FEW_ROPE ? 64 : 32;
-    const unsigned gx = (unsigned)((a.N + rows - 1) / rows), gy = (unsigned)((a.T + 31) / 32);
-    // two token tiles per workgroup, the weights read half as often, once there are enough workgroups: gate | up at 187 tokens (576 workgroups of one tile) 11.5 us with one
-    // tile and 12.4 with two, at 700 (2112) 24.5 and 23.3; down at 700 (528) 21.2 and 22.0, at 1800 (1368) 42.3 and 34.8.  Not for f32 rows: 17.5 and 18.0 at 1800
-    if constexpr (!XF) if (gx * gy * (rows / 32) >= 1280) {
-        hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 2, 2, XF>), dim3(gx, (gy + 1) / 2), dim3(64 * NW), 0, st, a);
+    hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, TT, PD, XF>), dim3((unsigned)((a.N + rows - 1) / rows), (unsigned)((a.T + 32 * TT - 1) / (32 * TT))), dim3(64 * NW), 0, st, a);
+}
+// two products: the form above, or a workgroup's waves sharing K.  Of the latter two token tiles per workgroup, the weights read half as often, once there are enough workgroups
+template <int NW, int EPI>
+void few_two(const MMF16Few &a, hipStream_t st) {
+    const int rows = EPI == FEW_ROPE ? 64 : 32, wg = (a.N + rows - 1) / rows * ((a.T + 31) / 32);
+    // (Q | K | V at any number of tokens, 1800: 19.8 / 23.4; gate | up to nine workgroups a CU: 500 tokens 14.9 / 15.1, 700 20.7 / 21.7, 900 25.9 / 25.4)
+    if (a.K <= ROWS_K && a.N % 32 == 0 && (EPI == FEW_ROPE || wg <= 9 * num_cu())) {
+        hipLaunchKernelGGL((mmf16_rows_kernel<EPI>), dim3((unsigned)(a.N / rows), (unsigned)((a.T + 31) / 32)), dim3(512), 0, st, a);
         return;
     }
-    hipLaunchKernelGGL((mmf16_few_kernel<NW, EPI, 1, XF || (EPI == FEW_SWIGLU && NW == 4) ? 2 : 3, XF>), dim3(gx, gy), dim3(64 * NW), 0, st, a);
+    if (wg * (rows / 32) >= 1280) few_go<NW, EPI, 2, 2, false>(a, st);
+    else few_go<NW, EPI, 1, EPI == FEW_SWIGLU && NW == 4 ? 2 : 3, false>(a, st);
+}
+// A plain product, us, K 768 of f32 rows / K 3072 of halves, both to 768 rows.  What counts is a wave's own chain again, so as many waves as K gives chunks where a CU has one workgroup: 187 tokens,
+// twelve waves 3.8 / 7.1, four and eight 4.3 / 7.5.  Beyond, in rounds of a workgroup a CU: f32 rows on four waves (400 tokens 6.0, twelve 6.4; 1000 8.3, 10.2); halves on one, two or three token
+// tiles, whose rounds take about 7.1, 9.4 and 14.6: 400 tokens 12.5, 9.3, 12.6, 800 about 18.5, 18.4, 14.8, 1200 24.8, 19.2, 27.0, 2048 36.9, 29.5, 38.9; eight waves with one and, from 1280
+// workgroups on, two 13.2, 19.9, 26.6, 31.1.
+template <bool XF>
+void few_plain(const MMF16Few &a, hipStream_t st) {
+    const int cu = num_cu(), gx = (a.N + 31) / 32, gy = (a.T + 31) / 32;
+    if constexpr (XF) {
+        if (a.K > 1024) few_go<8, FEW_PLAIN, 1, 2, true>(a, st);
+        else if (gx * gy <= cu) few_go<12, FEW_PLAIN, 1, 1, true>(a, st);
+        else few_go<4, FEW_PLAIN, 1, 2, true>(a, st);
+        return;
+    } else {
+        if (a.K <= 1024) {
+            if (gx * gy >= 1280) few_go<4, FEW_PLAIN, 2, 2, false>(a, st); else few_go<4, FEW_PLAIN, 1, 3, false>(a, st);
+            return;
+        }
+        const auto time = [&](int tt, int round) { return (gx * ((gy + tt - 1) / tt) + cu - 1) / cu * round; };
+        const int one = time(1, 71), two = time(2, 94), three = time(3, 146);
+        if (one <= two && one <= three) few_go<12, FEW_PLAIN, 1, 2, false>(a, st);
+        else if (two <= three) few_go<12, FEW_PLAIN, 2, 1, false>(a, st);
+        else few_go<8, FEW_PLAIN, 3, 2, false>(a, st);
+    }
 }
 }  // namespace
 
@@ -417,9 +558,7 @@ bool mmf16_few_applicable(int n_rows, int K, int T) {
 hipError_t launch_mmf16_few(const uint8_t *W, int n_rows, int K, const void *x, bool x_f16, int T, float *out, const float *resid, const float *bias, hipStream_t st) {
     MMF16Few a{};
     a.W = reinterpret_cast<const _Float16 *>(W); a.X = x; a.N = n_rows; a.K = K; a.T = T; a.out = out; a.resid = resid; a.bias = bias;
-    const bool wide = K > 1024;                              // eight waves share a longer K
-    if (x_f16) { if (wide) few_launch<8, FEW_PLAIN, false>(a, st); else few_launch<4, FEW_PLAIN, false>(a, st); }
-    else { if (wide) few_launch<8, FEW_PLAIN, true>(a, st); else few_launch<4, FEW_PLAIN, true>(a, st); }
+    if (x_f16) few_plain<false>(a, st); else few_plain<true>(a, st);
     return hipGetLastError();
 }
 // out[t][n_rows] = f16(silu(W_gate x) * (W_up x)), x: [T][K] halves
@@ -427,7 +566,7 @@ hipError_t launch_mmf16_few_swiglu(const uint8_t *W_gate, const uint8_t *W_up, i
     MMF16Few a{};
     a.W = reinterpret_cast<const _Float16 *>(W_gate); a.W2 = reinterpret_cast<const _Float16 *>(W_up); a.X = xh; a.N = n_rows; a.K = K; a.T = T;
     a.out_h = reinterpret_cast<_Float16 *>(out_h);
-    if (K > 1024) few_launch<8, FEW_SWIGLU, false>(a, st); else few_launch<4, FEW_SWIGLU, false>(a, st);
+    if (K > 1024) few_two<8, FEW_SWIGLU>(a, st); else few_two<4, FEW_SWIGLU>(a, st);
     return hipGetLastError();
 }
 // the projections of E = n_head * 64 rows each of W (Q | K | V) for x: [T][K] halves; rope pairs (d, d + 32) by cs[T][64]; q [T][E], k and v into the f16 cache
@@ -436,7 +575,7 @@ hipError_t launch_mmf16_few_qkv_rope(const uint8_t *W, int E, int K, const void 
     MMF16Few a{};
     a.W = reinterpret_cast<const _Float16 *>(W); a.W2 = a.W + (size_t)32 * K; a.X = xh; a.N = 3 * E; a.K = K; a.T = T;
     a.out = q; a.cs = cs; a.cell = cell; a.kc = reinterpret_cast<uint16_t *>(kv.k); a.vc = reinterpret_cast<uint16_t *>(kv.v); a.n_ctx = n_ctx;
-    if (K > 1024) few_launch<8, FEW_ROPE, false>(a, st); else few_launch<4, FEW_ROPE, false>(a, st);
+    if (K > 1024) few_two<8, FEW_ROPE>(a, st); else few_two<4, FEW_ROPE>(a, st);
     return hipGetLastError();
 }
 

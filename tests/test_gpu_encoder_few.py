@@ -61,3 +61,11 @@ def test_cache_in_q8_0(pkg, tmp_path, n):
     """768 columns with a q8_0 cache: Q, K and V as launches of their own, rope and store behind.  A value of a block of 32 is off by up to 1 / 254 of the block's largest, 2.5 to
     3 times its root mean square: 6e-3 of a value at the root mean square of the rounding, in K and in V, through two layers: sqrt(4) * 6e-3 at the most (heads' sums average it)."""
     assert run(pkg, tmp_path, n, kv=8) <= 1.2e-2
+
+
+# one and two 64-column chunks to every wave, as many columns as are staged at once and more; one token more and less than a tile of 32, and where ffn_down takes two token tiles a
+# workgroup for the first time
+@pytest.mark.parametrize("n,n_embd,n_ff", [(33, 256, 448), (31, 512, 1088), (341, 768, 3072), (33, 1024, 2048)])
+def test_tokens_staged_whole(pkg, tmp_path, n, n_embd, n_ff):
+    """Q | K | V and gate | up with a workgroup's token rows whole in LDS (to 768 columns), ffn_down on twelve waves.  Tolerance as above."""
+    assert run(pkg, tmp_path, n, n_embd=n_embd, n_head=n_embd // 64, n_head_kv=n_embd // 64, n_ff=n_ff) <= 1.6e-3
