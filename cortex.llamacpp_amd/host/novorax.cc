@@ -249,6 +249,7 @@ bool Context::init_novorax(std::string &err) {
     const NovoraxModel &M = *model->nvx;
     const size_t T = cp.n_ubatch, W = (size_t)M.width, NC = cp.n_ctx, NS = cp.n_seq_max;
     cells_.assign(NC, KVCell());
+    cell_sums_.reset(NC);
     d_cell_pos_ = (int32_t *)dalloc(NC * 4);
     d_cell_seq_ = (uint64_t *)dalloc(NC * 8);
     if (hipHostMalloc((void **)&h_cell_pos_, NC * 4, hipHostMallocDefault) != hipSuccess ||

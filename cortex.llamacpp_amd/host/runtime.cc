@@ -609,6 +609,7 @@ bool Context::init(std::string &err) {
     if (model->nvx) return init_novorax(err);
     const size_t T = cp.n_ubatch, E = hp.n_embd, FF = hp.n_ff, G = hp.n_head_kv, D = hp.head_dim, NC = cp.n_ctx;
     cells_.assign(NC, KVCell());
+    cell_sums_.reset(NC);
     kv_.resize((size_t)hp.n_layer);
     auto plane_bytes = [&](int type, size_t &codes, size_t &scales) {
         if (type == T_F16) { codes = G * NC * D * 2; scales = 0; }
@@ -766,15 +767,15 @@ bool Context::kv_seq_rm(int seq, int p0, int p1) {
         }
     }
     int new_head = (int)cells_.size();
-    for (int i = 0; i < cells_end_; i++) {
+    cell_sums_.each(cells_, cells_end_, seq < 0 ? 0 : 1ull << seq, p0, [&](int i) {
         KVCell &c = cells_[(size_t)i];
-        if (c.pos < p0 || c.pos >= p1) continue;
+        if (c.pos < p0 || c.pos >= p1) return;
         if (seq < 0) c.seqs = 0;
         else if (c.seqs & (1ull << seq)) c.seqs &= ~(1ull << seq);
-        else continue;
+        else return;
         touch_cell(i);
         if (!c.seqs) { c.pos = -1; c.delta = 0; if (i < new_head) new_head = i; }
-    }
+    });
     if (new_head < (int)cells_.size() && new_head < head_) head_ = new_head;
     if (new_head < (int)cells_.size()) region_next_.clear();   // cells came free: the next allocation starts at its region's lowest free cell
     return true;
@@ -862,7 +863,6 @@ bool Context::alloc_cells(int n, const uint64_t *seqmask, std::vector<int> &out)
     if (R >= 64) R &= ~63;
     if ((int)region_next_.size() != NS) { region_next_.assign((size_t)NS, 0); for (int s = 0; s < NS; s++) region_next_[(size_t)s] = s * R; }
     std::vector<char> taken((size_t)NC, 0);                    // cells handed out within this call
-    auto is_free = [&](int c) { return cells_[(size_t)c].pos < 0 && !taken[(size_t)c]; };
     for (int i = 0; i < n; i++) {
         int s = seqmask[i] ? __builtin_ctzll(seqmask[i]) : 0;
         if (s >= NS) s = NS - 1;
@@ -870,12 +870,9 @@ bool Context::alloc_cells(int n, const uint64_t *seqmask, std::vector<int> &out)
         int c = -1;
         int start = region_next_[(size_t)s];
         if (start < lo || start >= hi) start = lo;
-        for (int k = 0; k < hi - lo; k++) {                    // own region first, from where the last cell went
-            int cand = start + k;
-            if (cand >= hi) cand -= hi - lo;
-            if (is_free(cand)) { c = cand; break; }
-        }
-        if (c < 0) for (int cand = 0; cand < NC; cand++) if (is_free(cand)) { c = cand; break; }   // region full: anywhere
+        c = cell_sums_.first_free(cells_, start, hi, taken);   // own region first, from where the last cell went
+        if (c < 0) c = cell_sums_.first_free(cells_, lo, start, taken);
+        if (c < 0) c = cell_sums_.first_free(cells_, 0, NC, taken);                                // region full: anywhere
         if (c < 0) return false;
         taken[(size_t)c] = 1;
         out[(size_t)i] = c;
@@ -2005,6 +2002,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         KVCell &c = cells_[(size_t)tcell[(size_t)i]];
         cells_undo_.emplace_back(tcell[(size_t)i], c);
         c.pos = pos[i]; c.seqs = seqmask[i]; c.delta = 0;
+        cell_sums_.touch(tcell[(size_t)i]);
         cells_end_ = std::max(cells_end_, tcell[(size_t)i] + 1);
     }
     while (cells_end_ > 0 && cells_[(size_t)cells_end_ - 1].pos < 0) cells_end_--;
@@ -2069,8 +2067,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
     if (attn_cols_ || ((n >= 2 || cp.n_seq_max > 1) && lists_usable)) {
         const int nch = (n_kv_ + 63) / 64;
         std::vector<uint64_t> seq_of_chunk((size_t)nch, 0ull);
-        for (int i = 0; i < n_kv_ && i < (int)cells_.size(); i++)
-            if (cells_[(size_t)i].pos >= 0) seq_of_chunk[(size_t)(i >> 6)] |= cells_[(size_t)i].seqs;
+        for (int ch = 0; ch < nch; ch++) seq_of_chunk[(size_t)ch] = cell_sums_.at(cells_, ch).seqs;
         int32_t *cnt = h_chunks_ + (size_t)64 * chunk_stride_;
         for (int t = 0; t < (lists_usable ? n : 1); t++) {
             int32_t *lst = h_chunks_ + (size_t)t * chunk_stride_;
@@ -2312,7 +2309,7 @@ int Context::decode(int n_tokens, const int32_t *tokens, const int32_t *pos, con
         const int rc = decode_ubatch(n, tokens + i0, pos + i0, seq.data() + i0, mask.data() + i0, flags.data() + i0, out_base);
         ub_embd_ = nullptr;
         if (rc != 0) {
-            for (size_t u = cells_undo_.size(); u-- > 0;) cells_[(size_t)cells_undo_[u].first] = cells_undo_[u].second;
+            for (size_t u = cells_undo_.size(); u-- > 0;) { cells_[(size_t)cells_undo_[u].first] = cells_undo_[u].second; cell_sums_.touch(cells_undo_[u].first); }
             head_ = saved_head; device_cells_known_ = false; region_next_.clear();
             return rc;
         }

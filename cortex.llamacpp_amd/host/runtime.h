@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "kv_cells.h"
 #include "../csrc/kernels.h"
 #include "gguf.h"
 #include "novorax.h"
@@ -87,12 +88,6 @@ struct Model {
 Model *config_model_load(const std::string &dir, int main_gpu, std::string &err, int &status);
 bool config_model_path(const std::string &path, std::string &dir);   // does `path` name such a folder
 Model *model_load(const std::string &path, int main_gpu, std::string &err, int &status, int prefill_planes = -1, int tp_rank = 0, int tp_size = 1);
-
-struct KVCell {
-    int32_t pos = -1;
-    int32_t delta = 0;
-    uint64_t seqs = 0;
-};
 
 void debug_raise_stream_error(unsigned code);        // tests: raise the sticky error word of the cross-workgroup kernels as a timed-out wait would
 struct ContextParams {
@@ -242,6 +237,7 @@ class Context {
     int cur_T_ = 0;                    // tokens of the micro-batch run_layers last ran (run_output: a single row needs no gather)
     std::vector<void *> allocs_;
     std::vector<KVCell> cells_;
+    CellChunks cell_sums_;
     int head_ = 0;
     bool has_shift_ = false;
     // the device's cell table follows the host's: what it holds is mirrored in pinned memory, and a batch uploads the cells between dirty_lo_ and dirty_hi_ whose mirror
@@ -251,7 +247,7 @@ class Context {
     int32_t *h_cell_pos_ = nullptr;     // pinned
     uint64_t *h_cell_seq_ = nullptr;
     std::vector<std::pair<int, KVCell>> cells_undo_;      // what the decode call in progress has overwritten
-    void touch_cell(int i) { if (dirty_lo_ >= dirty_hi_) dirty_lo_ = i; dirty_lo_ = std::min(dirty_lo_, i); dirty_hi_ = std::max(dirty_hi_, i + 1); }
+    void touch_cell(int i) { cell_sums_.touch(i); if (dirty_lo_ >= dirty_hi_) dirty_lo_ = i; dirty_lo_ = std::min(dirty_lo_, i); dirty_hi_ = std::max(dirty_hi_, i + 1); }
     int upload_cells();
 
     // device state

@@ -17,6 +17,7 @@
 #include "../../cortex.llamacpp_amd/host/engine.h"
 #include "../../cortex.llamacpp_amd/host/gguf.h"
 #include "../../cortex.llamacpp_amd/host/json.h"
+#include "../../cortex.llamacpp_amd/host/kv_cells.h"
 #include "../../cortex.llamacpp_amd/host/sampling.h"
 #include "../../cortex.llamacpp_amd/host/grammar.h"
 #include "../../cortex.llamacpp_amd/host/server_context.h"
@@ -1450,6 +1451,45 @@ static void test_safetensors_reader() {
     unlink(tmpl);
 }
 
+// Searches of the cell table by the sums over its chunks, against the same searches cell by cell: whole and part chunks, full and empty ones, cells of several sequences, after every kind of change
+static void test_cell_chunks() {
+    for (const int n : {1, 63, 64, 65, 200, 512}) {
+        std::mt19937 rng(7u + (unsigned)n);
+        const auto upto = [&](int k) { return (int)(rng() % (unsigned)k); };
+        std::vector<KVCell> cells((size_t)n);
+        CellChunks sums;
+        sums.reset((size_t)n);
+        for (int round = 0; round < 400; round++) {
+            const int lo = upto(n), hi = lo + 1 + upto(n - lo), kind = upto(4);
+            for (int i = lo; i < hi; i++) {
+                KVCell &c = cells[(size_t)i];
+                if (kind == 0) c = KVCell();
+                else if (kind == 1) { c.pos = upto(300); c.seqs = 1ull << upto(6); }
+                else if (kind == 2 && c.pos >= 0) c.seqs |= 1ull << upto(64);
+                else if (kind == 3 && c.pos >= 0 && upto(3) == 0) c.pos += 40;
+                sums.touch(i);
+            }
+            const int end = upto(n + 1), p0 = upto(320);
+            const uint64_t seqs = upto(3) ? 1ull << upto(6) : 0;
+            const auto match = [&](int i) { const KVCell &c = cells[(size_t)i]; return c.pos >= p0 && (seqs == 0 || (c.seqs & seqs) != 0); };
+            std::vector<int> want, got;
+            for (int i = 0; i < end; i++) if (match(i)) want.push_back(i);
+            sums.each(cells, end, seqs, p0, [&](int i) { if (match(i)) got.push_back(i); });
+            CHECK(want == got);
+            std::vector<char> taken((size_t)n, 0);
+            for (int k = upto(4); k > 0; k--) taken[(size_t)upto(n)] = 1;
+            int free = -1;
+            for (int i = lo; i < hi && free < 0; i++) if (cells[(size_t)i].pos < 0 && !taken[(size_t)i]) free = i;
+            CHECK(sums.first_free(cells, lo, hi, taken) == free);
+            for (int ch = 0; ch < (n + 63) / 64; ch++) {
+                uint64_t m = 0;
+                for (int i = ch * 64; i < std::min(n, ch * 64 + 64); i++) if (cells[(size_t)i].pos >= 0) m |= cells[(size_t)i].seqs;
+                CHECK(sums.at(cells, ch).seqs == m);
+            }
+        }
+    }
+}
+
 int main(int argc, char **argv) {
     if (argc == 4 && std::string(argv[1]) == "--tokenize") return tokenize_cli(argv[2], argv[3]);
     if (argc == 2 && std::string(argv[1]) == "--api-shapes") return api_shapes_cli();
@@ -1457,6 +1497,7 @@ int main(int argc, char **argv) {
     signal(SIGTERM, [](int) { const char *m = g_stage; if (write(2, "hung in: ", 9) < 0 || write(2, m, strlen(m)) < 0 || write(2, "\n", 1) < 0) {} _exit(124); });
 #define STAGE(f) do { g_stage = #f; f(); } while (0)
     STAGE(test_json);
+    STAGE(test_cell_chunks);
     STAGE(test_vocab);
     STAGE(test_vocab_wordpiece);
     STAGE(test_vocab_numeric);
