@@ -1115,6 +1115,8 @@ static bool store_fuse_enabled() {
     static const bool env_off = getenv("MI355_ATTN_STORE_FUSE") && getenv("MI355_ATTN_STORE_FUSE")[0] == '0';
     return g_store_fuse && !env_off;
 }
+static bool g_last_rows = true;
+void set_last_rows(bool on) { g_last_rows = on; }
 static bool g_late_sums = true;
 void set_late_sums(bool on) { g_late_sums = on; }
 static bool g_rope_fast = true;
@@ -1490,8 +1492,13 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
     // a prompt's K-split attn_output / ffn_down leaves its partial sums to the norm that reads x_ next (x_parts of them in mmq_ws_; x_ holds the residual till then)
     const bool late_sum = g_late_sums && rmsnorm_takes_parts(E, T) && !tp;
     int x_parts = 1;
+    // behind the last layer's K and V rows only the flagged rows are read by anyone: where they follow one another (a prompt's last token; none, of a prompt's earlier batches) that layer's
+    // attention, attn_output and feed-forward are theirs alone.  Not where the rows are shown layer by layer, or a caller has named every row's experts
+    const bool cut = g_last_rows && T > 1 && n_out_rows_ < T && (n_out_rows_ == 0 || out_first_ >= 0) && !tp && !(debug_taps_ && dbg_) && moe_forced_T_ == 0;
     for (int il = 0; il < hp.n_layer; il++) {
         const LayerWeights &L = model->layers[(size_t)il];
+        int Tn = T;                                            // rows from the attention on, and the first of them
+        float *xl = x_;
         // --- attention block
         const bool any_f = !is_quant(L.wq.type) || !is_quant(L.wk.type) || !is_quant(L.wv.type);
         const bool need_k = is_quant(L.wq.type) && !act_is_q80(L.wq.type) || is_quant(L.wk.type) && !act_is_q80(L.wk.type) || is_quant(L.wv.type) && !act_is_q80(L.wv.type);
@@ -1583,10 +1590,24 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             HIP_TRY(launch_add_qkv_bias(q_, k_, v_, L.bq.valid() ? (const float *)L.bq.data : nullptr, L.bk.valid() ? (const float *)L.bk.data : nullptr,
                                         L.bv.valid() ? (const float *)L.bv.data : nullptr, H * D, G * D, T, stream_));
         if (!qkv_in_attn) prof_mark("qkv");
+        const bool cut_here = cut && il + 1 == hp.n_layer && (!decode_attn || fast_store);
+        if (cut_here) { Tn = n_out_rows_; xl = x_ + (size_t)std::max(out_first_, 0) * E; }
+        const auto rows_of = [&](AttnArgs r) {                 // the flagged rows' part of the batch's attention; its results and its quantised rows begin at row 0
+            const size_t f = (size_t)out_first_;
+            r.q += f * (size_t)H * D; r.T = Tn; r.tok_pos += f; r.tok_seq += f;
+            if (r.tok_chunks) { r.tok_chunks += f * (size_t)r.chunk_stride; r.tok_nchunks += f; }
+            if (Tn < 3) r.out_bh = r.out_bl = nullptr;
+            return r;
+        };
         if (qkv_in_attn) {
             // the whole block ran in the launch above
         } else if (decode_attn && (fast_store || fused_step || (batch_distinct_ && store_fuse_enabled()))) {
-            if (fused_step) {
+            if (cut_here) {
+                HIP_TRY(launch_kv_store_fast(k_, v_, T, G, D, rope_cs_, ra, d_cell_, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, stream_));
+                prof_mark("rope_kv");
+                if (Tn == 0) break;
+                HIP_TRY(launch_flash_attn_decode(rows_of(aa), rope_cs_ + (size_t)out_first_ * ra.n_rot, ra, stream_));
+            } else if (fused_step) {
                 // single-token step: K rope + KV store + attention + split merge + quantise in ONE launch - and, where attn_out.hip has a form for the shape,
                 // the attn_output mat-vec with its residual add in that launch too
                 if (ao_form) {
@@ -1611,17 +1632,20 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             else
                 HIP_TRY(launch_rope_kv_store(q_, k_, v_, T, H, G, D, d_pos_, d_cell_, ra, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, rope_cs_, stream_));
             prof_mark("rope_kv");
-            aa.splits = att_splits_;
+            if (cut_here && Tn == 0) break;
+            if (cut_here) aa = rows_of(aa);
+            const bool cols_here = cut_here ? !v16 && flash_attn_cols_takes(aa, false) : cols;
+            aa.splits = cut_here ? flash_attn_pick_splits(Tn, G, n_kv_max) : att_splits_;
             // (splits balance the causal tiles of ONE long sequence: sized by what a query of this batch can see - its position + 1 -
             // not by the cache's high-water mark: 32 sequences of 50-token prompts in a 32000-cell cache need none, and every
             // extra workgroup would scan the whole cell table)
-            aa.pf_splits = cols ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(T, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
-            while (aa.pf_splits > 1 && flash_attn_workspace_floats(T, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
-            void *const planes = !cols && flash_attn_prefill_planes_pay(cp.type_v, T, H, G, D, n_kv_max, cur_max_pos_ + 1) ? att_planes_ : nullptr;
-            HIP_TRY(cols ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_, planes));
+            aa.pf_splits = cols_here ? flash_attn_cols_splits(aa) : flash_attn_prefill_splits(Tn, H, G, D, std::min(n_kv_max, cur_max_pos_ + 1));
+            while (aa.pf_splits > 1 && flash_attn_workspace_floats(Tn, H, D, aa.pf_splits) > att_part_floats_) aa.pf_splits >>= 1;
+            void *const planes = !cols_here && flash_attn_prefill_planes_pay(cp.type_v, Tn, H, G, D, n_kv_max, cur_max_pos_ + 1) ? att_planes_ : nullptr;
+            HIP_TRY(cols_here ? launch_flash_attn_cols(aa, stream_) : launch_flash_attn(aa, stream_, planes));
         }
         prof_mark("attn");
-        if (o_pl) prep_written(aq_o_, (int)L.wo.K, T);          // the attention just re-quantised its output, planes included
+        if (o_pl && Tn >= 3) prep_written(aq_o_, (int)L.wo.K, Tn);          // the attention just re-quantised its output, planes included
         else if (prep_owner_ == aq_o_.qs) prep_owner_ = nullptr;
         if (engine) {   // attn_output, gate | up, down and the next layer's Q | K | V in one launch
             HIP_TRY(launch_decode_engine(d_engine_layers_ + il, E, FF, d_engine_gran_, d_engine_epoch_, il, il == engine_probe_layer_ ? d_engine_probe_ : nullptr, stream_));
@@ -1629,20 +1653,20 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         }
         // a step's Q8_0 attn_output where it can be a weight stream: that form quantises its input itself
         bool o_fuse = false;
-        if (T == 1 && !attn_out_done && !tp && L.wo.type == T_Q8_0) {
+        if (Tn == 1 && !attn_out_done && !tp && L.wo.type == T_Q8_0) {
             MMVQArgs o{};
             o.n_seg = 1; o.K = (int)L.wo.K; o.T = 1; o.epi = EPI_ADD; o.fuse_mode = 2; o.nx = att_;
-            o.seg[0] = make_seg(L.wo, x_, E, x_, nullptr);
+            o.seg[0] = make_seg(L.wo, xl, E, xl, nullptr);
             o_fuse = mmvq_stream_applicable(o);
         }
         if (attn_out_done) {   // the mat-vec ran inside the attention launch (attn_out.hip)
-            if (tp) HIP_TRY(tp_reduce_into_x(T));
+            if (tp) HIP_TRY(tp_reduce_into_x(Tn));
         } else if (tp) {   // this rank's partial sum (rank 0 carries the residual), then the exchange: x = sum over ranks
-            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, tp_part_, E, hp.tp_rank == 0 ? x_ : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
-            HIP_TRY(tp_reduce_into_x(T));
+            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, Tn, tp_part_, E, hp.tp_rank == 0 ? xl : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
+            HIP_TRY(tp_reduce_into_x(Tn));
         } else {
             if (o_fuse) { pending_fuse_.mode = 2; pending_fuse_.x = att_; }
-            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, T, x_, E, x_, EPI_ADD, late_sum ? &x_parts : nullptr));
+            HIP_TRY(linear(L.wo, aq_o_, att_, (int)L.wo.K, Tn, xl, E, xl, EPI_ADD, late_sum ? &x_parts : nullptr));
             pending_fuse_ = Fuse();
         }
         prof_mark("attn_out");
@@ -1655,7 +1679,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             // quantisation of its own expert's activation in the prologue
             MMVQArgs one_gu{}, one_down{};
             bool one_step = false;
-            if (T == 1 && KU >= 2 && KU <= 8 && (int)cp.n_ubatch >= KU && L.gate_exps.type == L.up_exps.type) {
+            if (Tn == 1 && KU >= 2 && KU <= 8 && (int)cp.n_ubatch >= KU && L.gate_exps.type == L.up_exps.type) {
                 MMVQArgs &a = one_gu, &d = one_down;
                 a.n_seg = 2; a.K = E; a.T = 1; a.epi = EPI_SWIGLU; a.n_sel = KU; a.sel_out_stride = FF;
                 a.seg[0] = make_seg(L.gate_exps, ffn_, FF, nullptr, moe_ids_);
@@ -1663,37 +1687,37 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 chunk_act(a, aq_e_, E, 0);
                 // (RMSNorm + quantise again in the launch's prologue - the arithmetic of the norm_quant launch, so the same codes: the
                 // weight stream's gate | up form takes its activation that way, and with it the selected experts stream like the dense feed-forward does)
-                if (can_fuse(E, 1) && !act_is_q80(L.gate_exps.type)) { a.fuse_mode = 1; a.nx = x_; a.nw = (const float *)L.ffn_norm.data; a.neps = hp.eps; }
+                if (can_fuse(E, 1) && !act_is_q80(L.gate_exps.type)) { a.fuse_mode = 1; a.nx = xl; a.nw = (const float *)L.ffn_norm.data; a.neps = hp.eps; }
                 d.n_seg = 1; d.K = FF; d.T = 1; d.epi = EPI_STORE; d.fuse_mode = 2; d.nx = ffn_; d.n_sel = KU; d.sel_nx_stride = FF; d.sel_out_stride = E;
                 d.seg[0] = make_seg(L.down_exps, moe_out_, E, nullptr, moe_ids_);
                 chunk_act(d, aq_ff_, FF, 0);
                 one_step = mmvq_fast_applicable(a) && mmvq_fast_applicable(d);
             }
             // (then the norm is the router's own, and nobody reads a normed or quantised row)
-            const bool router_norm = one_step && one_gu.fuse_mode == 1 && T < group_min && x_parts == 1 && moe_router_norms(L.gate_inp.type, hp.n_expert, E);
-            if (!router_norm) HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, xn_, &aq_e_,
+            const bool router_norm = one_step && one_gu.fuse_mode == 1 && Tn < group_min && x_parts == 1 && moe_router_norms(L.gate_inp.type, hp.n_expert, E);
+            if (!router_norm) HIP_TRY(launch_rmsnorm_quant(xl, (const float *)L.ffn_norm.data, E, Tn, hp.eps, xn_, &aq_e_,
                                          !act_is_q80(L.gate_exps.type) || !act_is_q80(L.up_exps.type), act_is_q80(L.gate_exps.type) || act_is_q80(L.up_exps.type), stream_, nullptr, nullptr, mmq_ws_.p, x_parts));
             x_parts = 1;
             prep_owner_ = nullptr;
             prof_mark("norm_quant");
             if (L.gate_inp.type == T_F32 || L.gate_inp.type == T_F16) {
-                HIP_TRY(launch_moe_router(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, router_norm ? x_ : xn_, T, hp.n_expert_used, router_, moe_ids_, moe_w_, stream_,
-                                          moe_forced_T_ == T ? d_moe_forced_ + (size_t)il * T * hp.n_expert_used : nullptr, router_norm ? (const float *)L.ffn_norm.data : nullptr, hp.eps));
+                HIP_TRY(launch_moe_router(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, router_norm ? xl : xn_, Tn, hp.n_expert_used, router_, moe_ids_, moe_w_, stream_,
+                                          moe_forced_T_ == Tn ? d_moe_forced_ + (size_t)il * Tn * hp.n_expert_used : nullptr, router_norm ? (const float *)L.ffn_norm.data : nullptr, hp.eps));
             } else {
-                HIP_TRY(launch_mmv_float(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, xn_, T, router_, hp.n_expert, nullptr, stream_));
-                HIP_TRY(launch_moe_route(router_, T, hp.n_expert, hp.n_expert_used, moe_ids_, moe_w_, stream_,
-                                         moe_forced_T_ == T ? d_moe_forced_ + (size_t)il * T * hp.n_expert_used : nullptr));
+                HIP_TRY(launch_mmv_float(L.gate_inp.type, L.gate_inp.data, hp.n_expert, E, xn_, Tn, router_, hp.n_expert, nullptr, stream_));
+                HIP_TRY(launch_moe_route(router_, Tn, hp.n_expert, hp.n_expert_used, moe_ids_, moe_w_, stream_,
+                                         moe_forced_T_ == Tn ? d_moe_forced_ + (size_t)il * Tn * hp.n_expert_used : nullptr));
             }
             prof_mark("moe_route");
             const bool exps_q = is_quant(L.gate_exps.type) && is_quant(L.up_exps.type) && is_quant(L.down_exps.type);
-            if (exps_q && T >= group_min && aq_eg_.qs) {
+            if (exps_q && Tn >= group_min && aq_eg_.qs) {
                 // ggml_mul_mat_id on a batch: group the (token, rank) pairs by expert, one contiguous activation batch per
                 // expert (its weights are read once per batch, through the same batched kernels as the dense projections)
-                const int NE = hp.n_expert, GR = T * KU;
-                HIP_TRY(launch_moe_group(moe_ids_, T, KU, NE, moe_meta_, moe_slot_, moe_tok_, stream_));
+                const int NE = hp.n_expert, GR = Tn * KU;
+                HIP_TRY(launch_moe_group(moe_ids_, Tn, KU, NE, moe_meta_, moe_slot_, moe_tok_, stream_));
                 // round 5: every expert's batch in ONE launch per projection (the workgroups find their expert and token tile from the counts on the device):
                 // no host synchronisation in the layer, and ~128-token batches that half-fill a launch each become one launch that fills the chip
-                const bool grouped = T >= 32 && L.gate_exps.planes && L.up_exps.planes && L.down_exps.planes && L.gate_exps.type == L.up_exps.type &&
+                const bool grouped = Tn >= 32 && L.gate_exps.planes && L.up_exps.planes && L.down_exps.planes && L.gate_exps.type == L.up_exps.type &&
                                      L.gate_exps.N == L.up_exps.N && mmq_planes_moe_ok(L.gate_exps.type, (int)L.gate_exps.N, E) &&
                                      mmq_planes_moe_ok(L.down_exps.type, (int)L.down_exps.N, FF) && (L.gate_exps.N % 64) == 0;
                 if (grouped) {
@@ -1704,9 +1728,9 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                                                          ffn_g_, FF, stream_));
                     HIP_TRY(launch_quantize(ffn_g_, FF, GR, aq_ffg_, true, false, stream_));
                     HIP_TRY(launch_mmq_planes_moe(L.down_exps.type, L.down_exps.planes, ps_d, NE, moe_meta_, (int)L.down_exps.N, FF, GR, aq_ffg_, y_g_, E, stream_));
-                    HIP_TRY(launch_moe_scatter_combine(x_, y_g_, moe_w_, moe_slot_, T, E, KU, stream_));
+                    HIP_TRY(launch_moe_scatter_combine(xl, y_g_, moe_w_, moe_slot_, Tn, E, KU, stream_));
                     prof_mark("moe_ffn");
-                    if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
+                    if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, xl, (size_t)Tn * E * 4, hipMemcpyDeviceToDevice, stream_));
                     continue;
                 }
                 HIP_TRY(hipMemcpyAsync(h_moe_meta_, moe_meta_, (size_t)(2 * NE + 1) * 4, hipMemcpyDeviceToHost, stream_));
@@ -1751,16 +1775,16 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 }
                 bh_over_ = bl_over_ = nullptr;
                 HIP_TRY(e_exp);
-                HIP_TRY(launch_moe_scatter_combine(x_, y_g_, moe_w_, moe_slot_, T, E, KU, stream_));
+                HIP_TRY(launch_moe_scatter_combine(xl, y_g_, moe_w_, moe_slot_, Tn, E, KU, stream_));
                 prof_mark("moe_ffn");
-                if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
+                if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, xl, (size_t)Tn * E * 4, hipMemcpyDeviceToDevice, stream_));
                 continue;
             }
             if (one_step) {
                 HIP_TRY(launch_mmvq(one_gu, stream_));         // the weight stream where it has a form for the shape, else the register ring (bit-identical)
                 HIP_TRY(launch_mmvq(one_down, stream_));
             }
-            for (int t = 0; t < T && !one_step; t++) {
+            for (int t = 0; t < Tn && !one_step; t++) {
                 for (int j = 0; j < KU; j++) {
                     const int32_t *esel = moe_ids_ + (size_t)t * KU + j;
                     MMVQArgs a{};
@@ -1784,128 +1808,128 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                     MMVQArgs d{};
                     d.n_seg = 1; d.K = FF; d.T = 1; d.epi = EPI_STORE;
                     if (fuse_q) { d.fuse_mode = 2; d.nx = ffn_ + (size_t)t * FF; }
-                    d.seg[0] = make_seg(L.down_exps, moe_out_ + ((size_t)j * T + t) * E, E, nullptr, esel);
+                    d.seg[0] = make_seg(L.down_exps, moe_out_ + ((size_t)j * Tn + t) * E, E, nullptr, esel);
                     chunk_act(d, aq_ff_, FF, 0);
                     HIP_TRY(launch_mmvq(d, stream_));
                 }
             }
-            HIP_TRY(launch_moe_combine(x_, moe_out_, moe_w_, T, E, KU, (size_t)T * E, stream_));
+            HIP_TRY(launch_moe_combine(xl, moe_out_, moe_w_, Tn, E, KU, (size_t)Tn * E, stream_));
             prof_mark("moe_ffn");
         } else {
             const bool gq = is_quant(L.gate.type), uq = is_quant(L.up.type);
             const bool fk = (gq && !act_is_q80(L.gate.type)) || (uq && !act_is_q80(L.up.type));
             const bool f0 = act_is_q80(L.gate.type) || act_is_q80(L.up.type);
-            const bool fuse_ffn = gq && uq && L.gate.type == L.up.type && can_fuse(E, T);
+            const bool fuse_ffn = gq && uq && L.gate.type == L.up.type && can_fuse(E, Tn);
             Fuse fz;
             if (fuse_ffn) {
-                fz.mode = 1; fz.x = x_; fz.w = (const float *)L.ffn_norm.data; fz.eps = hp.eps;
+                fz.mode = 1; fz.x = xl; fz.w = (const float *)L.ffn_norm.data; fz.eps = hp.eps;
             } else {
-                const bool pl = fk && T >= 3;
-                HIP_TRY(launch_rmsnorm_quant(x_, (const float *)L.ffn_norm.data, E, T, hp.eps, (!gq || !uq) ? xn_ : nullptr, &aq_e_, fk, f0, stream_,
+                const bool pl = fk && Tn >= 3;
+                HIP_TRY(launch_rmsnorm_quant(xl, (const float *)L.ffn_norm.data, E, Tn, hp.eps, (!gq || !uq) ? xn_ : nullptr, &aq_e_, fk, f0, stream_,
                                              pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr, mmq_ws_.p, x_parts));
                 x_parts = 1;
                 prep_owner_ = nullptr;
-                if (pl) prep_written(aq_e_, E, T);
+                if (pl) prep_written(aq_e_, E, Tn);
                 prof_mark("norm_quant");
             }
             bool swiglu_quantised = false;
-            const bool ffn_mmq = (mmq_q80_applicable(L.gate.type, E, T) && mmq_q80_applicable(L.up.type, E, T)) ||
-                                 (mmq_applicable(L.gate.type, E, T) && mmq_applicable(L.up.type, E, T)) ||
-                                 (mmq_ksplit_applicable(L.gate.type, E, T) && mmq_ksplit_applicable(L.up.type, E, T)) ||
-                                 (planes_small(L.gate, E, T) && planes_small(L.up, E, T)) || (q80_copy(L.gate, E, T) && q80_copy(L.up, E, T));
-            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, T, L.gate.planes != nullptr, mmq_ws_, false, true) &&
-                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, T, L.up.planes != nullptr, mmq_ws_, false, true) && !fuse_ffn;
+            const bool ffn_mmq = (mmq_q80_applicable(L.gate.type, E, Tn) && mmq_q80_applicable(L.up.type, E, Tn)) ||
+                                 (mmq_applicable(L.gate.type, E, Tn) && mmq_applicable(L.up.type, E, Tn)) ||
+                                 (mmq_ksplit_applicable(L.gate.type, E, Tn) && mmq_ksplit_applicable(L.up.type, E, Tn)) ||
+                                 (planes_small(L.gate, E, Tn) && planes_small(L.up, E, Tn)) || (q80_copy(L.gate, E, Tn) && q80_copy(L.up, E, Tn));
+            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, Tn, L.gate.planes != nullptr, mmq_ws_, false, true) &&
+                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, Tn, L.up.planes != nullptr, mmq_ws_, false, true) && !fuse_ffn;
             if (gq && uq && L.gate.type == L.up.type && !ffn_mmq) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
-                HIP_TRY(mmvq_tokens(segs, 2, E, T, EPI_SWIGLU, aq_e_, stream_, fz));
+                HIP_TRY(mmvq_tokens(segs, 2, E, Tn, EPI_SWIGLU, aq_e_, stream_, fz));
             } else if (ffn_ks) {                               // batched decode step: gate and up in one launch
                 MMQSeg sg[2] = {{L.gate.data, L.gate.row_bytes, (int)L.gate.N, L.gate.type, ffn_, FF, nullptr, 0},
                                 {L.up.data, L.up.row_bytes, (int)L.up.N, L.up.type, ffn_u_, FF, nullptr, 0}};
                 const bool alike = L.gate.type == L.up.type && L.gate.N == L.up.N;
-                const bool pair = alike && (T <= 32 || mmq_few_takes(sg, 2, E, T, aq_e_, true));          // SwiGLU in the epilogue
-                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, T, mmq_few_takes(sg, 2, E, T, aq_e_, pair)));
-                HIP_TRY(launch_mmq_ksplit_multi(sg, 2, E, T, aq_e_, mmq_bh_, mmq_bl_, pair, stream_));
+                const bool pair = alike && (Tn <= 32 || mmq_few_takes(sg, 2, E, Tn, aq_e_, true));          // SwiGLU in the epilogue
+                if (L.gate.type != T_Q6_K || L.up.type != T_Q6_K) HIP_TRY(ensure_prep(aq_e_, E, Tn, mmq_few_takes(sg, 2, E, Tn, aq_e_, pair)));
+                HIP_TRY(launch_mmq_ksplit_multi(sg, 2, E, Tn, aq_e_, mmq_bh_, mmq_bl_, pair, stream_));
                 if (!pair) {
                     if (is_quant(L.down.type) && (FF % 256) == 0) {
                         const bool pl = !act_is_q80(L.down.type);
-                        HIP_TRY(launch_swiglu_quant(ffn_, ffn_u_, FF, T, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_,
+                        HIP_TRY(launch_swiglu_quant(ffn_, ffn_u_, FF, Tn, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_,
                                                     pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
                         prep_owner_ = nullptr;
-                        if (pl) prep_written(aq_ff_, FF, T);
+                        if (pl) prep_written(aq_ff_, FF, Tn);
                         swiglu_quantised = true;
                     } else {
-                        HIP_TRY(launch_swiglu(ffn_, ffn_u_, ffn_, (int64_t)T * FF, stream_));
+                        HIP_TRY(launch_swiglu(ffn_, ffn_u_, ffn_, (int64_t)Tn * FF, stream_));
                     }
                 }
-            } else if (T > 1 && !fuse_ffn && L.gate.planes && L.up.planes && L.gate.N == L.up.N && (mmq_applicable(L.gate.type, E, T) || planes_small(L.gate, E, T)) &&
-                       mmq_planes_swiglu_ok(L.gate.type, L.up.type, (int)L.gate.N, E, T)) {
+            } else if (Tn > 1 && !fuse_ffn && L.gate.planes && L.up.planes && L.gate.N == L.up.N && (mmq_applicable(L.gate.type, E, Tn) || planes_small(L.gate, E, Tn)) &&
+                       mmq_planes_swiglu_ok(L.gate.type, L.up.type, (int)L.gate.N, E, Tn)) {
                 // prompt batch on the LDS kernel: gate and up in one launch, 64 rows of each per workgroup, SwiGLU in the epilogue (one
                 // f32 result of T x FF instead of two); the quantiser for the down projection then reads half as much
-                HIP_TRY(launch_mmq_planes_swiglu(L.gate.type, L.gate.planes, L.up.planes, (int)L.gate.N, E, T, aq_e_, ffn_, FF, stream_));
+                HIP_TRY(launch_mmq_planes_swiglu(L.gate.type, L.gate.planes, L.up.planes, (int)L.gate.N, E, Tn, aq_e_, ffn_, FF, stream_));
                 if (is_quant(L.down.type) && (FF % 256) == 0) {
-                    const bool pl = !act_is_q80(L.down.type) && T >= 3;
-                    HIP_TRY(launch_quantize(ffn_, FF, T, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_, pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
+                    const bool pl = !act_is_q80(L.down.type) && Tn >= 3;
+                    HIP_TRY(launch_quantize(ffn_, FF, Tn, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_, pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
                     prep_owner_ = nullptr;
-                    if (pl) prep_written(aq_ff_, FF, T);
+                    if (pl) prep_written(aq_ff_, FF, Tn);
                     swiglu_quantised = true;
                 }
             } else {
-                if (!fuse_ffn && pending_fuse_.mode == 0 && aq_e_.qs0 && q80_rows(L.gate, E, T) && q80_rows(L.up, E, T)) {
+                if (!fuse_ffn && pending_fuse_.mode == 0 && aq_e_.qs0 && q80_rows(L.gate, E, Tn) && q80_rows(L.up, E, Tn)) {
                     const Q80Seg sg[2] = {q80_seg(L.gate, E, ffn_, FF), q80_seg(L.up, E, ffn_u_, FF)};
-                    HIP_TRY(launch_mmq_q80_multi(sg, 2, E, T, aq_e_, nullptr, stream_));
+                    HIP_TRY(launch_mmq_q80_multi(sg, 2, E, Tn, aq_e_, nullptr, stream_));
                 } else {
-                    HIP_TRY(linear(L.gate, aq_e_, xn_, E, T, ffn_, FF, nullptr, EPI_STORE));
-                    HIP_TRY(linear(L.up, aq_e_, xn_, E, T, ffn_u_, FF, nullptr, EPI_STORE));
+                    HIP_TRY(linear(L.gate, aq_e_, xn_, E, Tn, ffn_, FF, nullptr, EPI_STORE));
+                    HIP_TRY(linear(L.up, aq_e_, xn_, E, Tn, ffn_u_, FF, nullptr, EPI_STORE));
                 }
                 // prompt batch: SwiGLU and the quantisation for the down projection in one pass (no f32 round trip of T x FF)
-                if (T > 1 && is_quant(L.down.type) && (FF % 256) == 0) {
-                    const bool pl = !act_is_q80(L.down.type) && T >= 3;
-                    HIP_TRY(launch_swiglu_quant(ffn_, ffn_u_, FF, T, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_,
+                if (Tn > 1 && is_quant(L.down.type) && (FF % 256) == 0) {
+                    const bool pl = !act_is_q80(L.down.type) && Tn >= 3;
+                    HIP_TRY(launch_swiglu_quant(ffn_, ffn_u_, FF, Tn, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_,
                                                 pl ? mmq_bh_ : nullptr, pl ? mmq_bl_ : nullptr));
                     prep_owner_ = nullptr;
-                    if (pl) prep_written(aq_ff_, FF, T);
+                    if (pl) prep_written(aq_ff_, FF, Tn);
                     swiglu_quantised = true;
                 } else {
-                    HIP_TRY(launch_swiglu(ffn_, ffn_u_, ffn_, (int64_t)T * FF, stream_));
+                    HIP_TRY(launch_swiglu(ffn_, ffn_u_, ffn_, (int64_t)Tn * FF, stream_));
                 }
             }
             prof_mark("ffn_gate_up");
             static const bool fuse_down_env = !(getenv("MI355_FUSE_DOWN") && getenv("MI355_FUSE_DOWN")[0] == '0');
             // quantise inside the down-projection's prologue (once per CU, overlapped with its first weight loads)
             // (the widths listed are the ones the register-ring and weight-stream kernels take; the generic mat-vec's fused prologue would refuse others)
-            const bool fuse_down = fuse_down_env && T == 1 && (L.down.type == T_Q4_K || L.down.type == T_Q5_K || L.down.type == T_Q6_K || act_is_q80(L.down.type) ||
+            const bool fuse_down = fuse_down_env && Tn == 1 && (L.down.type == T_Q4_K || L.down.type == T_Q5_K || L.down.type == T_Q6_K || act_is_q80(L.down.type) ||
                                                                L.down.type == T_Q2_K || L.down.type == T_Q3_K) &&
                                    (FF % 256) == 0 && mmvq_fast_kb_ok((FF + 2047) / 2048);
             if (fuse_down && !tp && L.down_lo.valid() && L.down_hi.valid()) {
                 // the column halves of ffn_down, each quantising its half of the SwiGLU output in its prologue: x += W_lo a_lo; x += W_hi a_hi
                 const int Kh = (int)L.down_lo.K;
                 pending_fuse_.mode = 2; pending_fuse_.x = ffn_;
-                HIP_TRY(linear(L.down_lo, aq_ff_, ffn_, Kh, T, x_, E, x_, EPI_ADD));
+                HIP_TRY(linear(L.down_lo, aq_ff_, ffn_, Kh, Tn, xl, E, xl, EPI_ADD));
                 pending_fuse_.mode = 2; pending_fuse_.x = ffn_ + Kh;
-                HIP_TRY(linear(L.down_hi, aq_ff_, ffn_ + Kh, Kh, T, x_, E, x_, EPI_ADD));
+                HIP_TRY(linear(L.down_hi, aq_ff_, ffn_ + Kh, Kh, Tn, xl, E, xl, EPI_ADD));
                 pending_fuse_ = Fuse();
                 prof_mark("ffn_down");
-                if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
+                if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, xl, (size_t)Tn * E * 4, hipMemcpyDeviceToDevice, stream_));
                 continue;
             }
             if (fuse_down) {
                 pending_fuse_.mode = 2; pending_fuse_.x = ffn_;       // quantise inside the mat-vec prologue
             } else if (is_quant(L.down.type) && !swiglu_quantised) {
-                HIP_TRY(launch_quantize(ffn_, FF, T, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_));
+                HIP_TRY(launch_quantize(ffn_, FF, Tn, aq_ff_, !act_is_q80(L.down.type), act_is_q80(L.down.type), stream_));
                 prep_owner_ = nullptr;
                 prof_mark("quant");
             }
             if (tp) {
-                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, T, tp_part_, E, hp.tp_rank == 0 ? x_ : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
+                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, Tn, tp_part_, E, hp.tp_rank == 0 ? xl : nullptr, hp.tp_rank == 0 ? EPI_ADD : EPI_STORE));
                 pending_fuse_ = Fuse();
-                HIP_TRY(tp_reduce_into_x(T));
+                HIP_TRY(tp_reduce_into_x(Tn));
             } else {
-                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, T, x_, E, x_, EPI_ADD, late_sum && il + 1 < hp.n_layer && !(debug_taps_ && dbg_) ? &x_parts : nullptr));
+                HIP_TRY(linear(L.down, aq_ff_, ffn_, FF, Tn, xl, E, xl, EPI_ADD, late_sum && il + 1 < hp.n_layer && !(debug_taps_ && dbg_) ? &x_parts : nullptr));
             }
             pending_fuse_ = Fuse();
             prof_mark("ffn_down");
         }
-        if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, x_, (size_t)T * E * 4, hipMemcpyDeviceToDevice, stream_));
+        if (debug_taps_ && dbg_) HIP_TRY(hipMemcpyAsync(dbg_ + (size_t)il * cp.n_ubatch * E, xl, (size_t)Tn * E * 4, hipMemcpyDeviceToDevice, stream_));
     }
     return hipSuccess;
 }
@@ -1920,9 +1944,9 @@ hipError_t Context::run_output(int n_out, int out_base) {
     const HParams &hp = model->hp;
     const int E = hp.n_embd, V = hp.n_vocab;
     if (embd_on_host_) return hipSuccess;                    // (the last layer's norm stored them)
-    // (a single-token step has one row and it is the flagged one: no gather launch)
-    float *const xo = cur_T_ == 1 && n_out == 1 ? x_ : xo_;
-    if (xo != x_) HIP_TRY(launch_gather_rows_f32(x_, d_outrow_, n_out, E, xo_, stream_));
+    // rows that follow one another - a prompt's last token, a tick's all - are read where they are (gathered by a launch of their own: 4.6 us)
+    float *const xo = out_first_ >= 0 ? x_ + (size_t)out_first_ * E : xo_;
+    if (out_first_ < 0) HIP_TRY(launch_gather_rows_f32(x_, d_outrow_, n_out, E, xo_, stream_));
     if (hp.encoder) {                                        // the embeddings ARE the last layer's rows (t_embd of llm_build_bert): no final norm, no head
         HIP_TRY(hipMemcpyAsync(d_embd_ + (size_t)out_base * E, xo, (size_t)n_out * E * 4, hipMemcpyDeviceToDevice, stream_));
         prof_mark("embd");
@@ -2035,6 +2059,8 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         h_tok[i] = tokens[i]; h_pos[i] = pos[i]; h_seq[i] = seq[i]; h_cell[i] = tcell[(size_t)i]; h_mask[i] = seqmask[i];
         if (flags[i]) h_out[n_out++] = i;
     }
+    n_out_rows_ = n_out;
+    out_first_ = n_out > 0 && h_out[n_out - 1] - h_out[0] == n_out - 1 ? h_out[0] : -1;
     embd_out_ = model->hp.encoder && n_out == n && out_base == 0 ? h_embd_ : nullptr;
     embd_on_host_ = false;
     if (!one_token_) {

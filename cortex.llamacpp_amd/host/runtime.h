@@ -109,6 +109,7 @@ struct Fuse {   // fused activation prologue of the single-token mat-vec (mmvq.h
 
 void set_moe_group_min(int tokens);   // tests: batch size from which a mixture-of-experts feed-forward is grouped by expert
 void set_attn_store_fuse(bool on);   // tests: 0 = batched steps store K / V in their own launch before the attention
+void set_last_rows(bool on);         // tests: 0 = the last layer works on every row of a batch, flagged or not
 void set_late_sums(bool on);         // tests: 0 = a K split's partial sums are added by a launch of their own
 void set_rope_fast(bool on);         // tests: 0 = prompt batches rotate q / store K, V with the one-workgroup-per-token kernel
 void set_decode_engine(int on);  // 1 / 0: the layer engine (decode_engine.hip) for single-token steps of contexts created afterwards; -1: environment MI355_ENGINE / default (off)
@@ -234,7 +235,8 @@ class Context {
     void *dalloc(size_t bytes);
 
     hipStream_t stream_ = nullptr;
-    int cur_T_ = 0;                    // tokens of the micro-batch run_layers last ran (run_output: a single row needs no gather)
+    int cur_T_ = 0;                    // tokens of the micro-batch run_layers last ran
+    int n_out_rows_ = 0, out_first_ = -1;     // its flagged rows, and the first of them where they follow one another, else -1
     std::vector<void *> allocs_;
     std::vector<KVCell> cells_;
     CellChunks cell_sums_;
