@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256) void flash_attn_split_kernel(const AttnArgs a)
 #pragma unroll
         for (int j = 0; j < NCG; j++) s += accs[((size_t)j * R + r) * D + d];
         const int h = g * R + r;
-        float *dst = a.part + (((size_t)t * H + h) * a.splits + sp) * (D + 2);
+        float *dst = a.part + (((size_t)t * H + h) * a.splits + sp) * att_rec(D);
         dst[d] = s;
         if (d == 0) { dst[D] = red[2 * r]; dst[D + 1] = red[2 * r + 1]; }
     }
@@ -515,19 +515,19 @@ __global__ __launch_bounds__(256) void flash_attn_combine_kernel(const float *pa
     // their weight they cost a round trip to memory each: 7.5 us for the eleven splits of 640 cells, 37 tokens, 32 heads)
     constexpr int U = 8;
     const int hl = tid / D;
-    const float *pe = part + ((size_t)t * H + h0 + hl) * stride_s * (D + 2) + (tid - hl * D);
+    const float *pe = part + ((size_t)t * H + h0 + hl) * stride_s * att_rec(D) + (tid - hl * D);
     auto fetch = [&](int s0, float (&v)[U]) {
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = pe[(size_t)(s0 + u < splits ? s0 + u : 0) * (D + 2)];
+        for (int u = 0; u < U; u++) v[u] = pe[(size_t)(s0 + u < splits ? s0 + u : 0) * att_rec(D)];
     };
     float v[U];
     fetch(0, v);
     if (wave < hpb) {
-        const float *p = part + ((size_t)t * H + h0 + wave) * stride_s * (D + 2);
+        const float *p = part + ((size_t)t * H + h0 + wave) * stride_s * att_rec(D);
         float M = -INFINITY;
         for (int s0 = 0; s0 < splits; s0 += 64) {
             const int sidx = s0 + lane;
-            const float m = sidx < splits ? p[(size_t)sidx * (D + 2) + D] : -INFINITY;
+            const float m = sidx < splits ? p[(size_t)sidx * att_rec(D) + D] : -INFINITY;
             M = fmaxf(M, wave_max(m));
         }
         float den = 0.0f;
@@ -535,8 +535,8 @@ __global__ __launch_bounds__(256) void flash_attn_combine_kernel(const float *pa
             const int sidx = s0 + lane;
             float w = 0.0f, l = 0.0f;
             if (sidx < splits) {
-                const float m = p[(size_t)sidx * (D + 2) + D];
-                l = p[(size_t)sidx * (D + 2) + D + 1];
+                const float m = p[(size_t)sidx * att_rec(D) + D];
+                l = p[(size_t)sidx * att_rec(D) + D + 1];
                 w = (m == -INFINITY) ? 0.0f : expf(m - M);
                 wgt[wave * stride_s + sidx] = w;
             }
@@ -896,12 +896,12 @@ __global__ __launch_bounds__(256) void flash_attn_combine_wave_kernel(const floa
     float wv[HPB];                                               // lane s: the weight of split s, per head of the block
 #pragma unroll
     for (int hh = 0; hh < HPB; hh++) {
-        const float *p = part + ((size_t)t * H + h0 + hh) * splits * (D + 2);
-        const float m = lane < splits ? p[(size_t)lane * (D + 2) + D] : -INFINITY;
+        const float *p = part + ((size_t)t * H + h0 + hh) * splits * att_rec(D);
+        const float m = lane < splits ? p[(size_t)lane * att_rec(D) + D] : -INFINITY;
         const float M = fmaxf(-INFINITY, wave_max(m));
         float w = 0.0f, l = 0.0f;
         if (lane < splits) {
-            l = p[(size_t)lane * (D + 2) + D + 1];
+            l = p[(size_t)lane * att_rec(D) + D + 1];
             w = (m == -INFINITY) ? 0.0f : expf(m - M);
         }
         float den = 0.0f;
@@ -910,15 +910,15 @@ __global__ __launch_bounds__(256) void flash_attn_combine_wave_kernel(const floa
         wv[hh] = w * inv;
     }
     const int e = lane * 4, hl = e / D, d = e - hl * D;
-    const float *pr = part + ((size_t)t * H + h0 + hl) * splits * (D + 2) + d;
+    const float *pr = part + ((size_t)t * H + h0 + hl) * splits * att_rec(D) + d;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s = 0; s < splits; s++) {
         float w = 0.0f;
 #pragma unroll
         for (int hh = 0; hh < HPB; hh++) { const float wh = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wv[hh]), s)); if (hh == hl) w = wh; }
         if (w != 0.0f) {                                         // chunks with no visible cell publish only (m, l)
-            const float2 a0 = *reinterpret_cast<const float2 *>(pr + (size_t)s * (D + 2)), a1 = *reinterpret_cast<const float2 *>(pr + (size_t)s * (D + 2) + 2);
-            acc[0] += w * a0.x; acc[1] += w * a0.y; acc[2] += w * a1.x; acc[3] += w * a1.y;
+            const float4 a0 = *reinterpret_cast<const float4 *>(pr + (size_t)s * att_rec(D));
+            acc[0] += w * a0.x; acc[1] += w * a0.y; acc[2] += w * a0.z; acc[3] += w * a0.w;
         }
     }
     const int e0 = b * 256 + e;
@@ -936,8 +936,7 @@ __global__ __launch_bounds__(256) void flash_attn_combine_wave_kernel(const floa
     }
 }
 
-// (D + 32 floats per record: what attn_out.hip keeps per head and chunk - whole 128-byte lines; the other kernels use D + 2 of them)
-size_t flash_attn_workspace_floats(int T, int H, int D, int splits) { return (size_t)T * H * splits * (D + 32); }
+size_t flash_attn_workspace_floats(int T, int H, int D, int splits) { return (size_t)T * H * splits * att_rec(D); }
 
 hipError_t launch_flash_attn_combine(const AttnArgs &a, int splits, hipStream_t st) {
     if (a.D != 64 && a.D != 128) return hipErrorInvalidValue;

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
 #pragma unroll
         for (int r = 0; r < 16; r++) mine[(db * 16 + r) * 65 + lane] = O[db][r] * f;
     if (wave == 0 && kg == 0 && c.nsp > 1 && q_ok) {
-        float *rec = a.part + (((size_t)tok * a.H + h) * c.nsp + blockIdx.z) * (D + 2);
+        float *rec = a.part + (((size_t)tok * a.H + h) * c.nsp + blockIdx.z) * att_rec(D);
         rec[D] = m_nat; rec[D + 1] = l_all * adj;
     }
     __syncthreads();
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_attn_cols_kernel(const ColsA
         const int t = in ? gc / R : 0, hh = g * R + (gc - t * R);
         if (c.nsp > 1) {
             if (in) {
-                float *rec = a.part + (((size_t)t * a.H + hh) * c.nsp + blockIdx.z) * (D + 2) + d0;
+                float *rec = a.part + (((size_t)t * a.H + hh) * c.nsp + blockIdx.z) * att_rec(D) + d0;
                 *reinterpret_cast<f32x2 *>(rec) = f32x2{v[0], v[1]}; *reinterpret_cast<f32x2 *>(rec + 2) = f32x2{v[2], v[3]};
             }
             continue;

@@ -708,14 +708,11 @@ __global__ __launch_bounds__(64 * R * KH * QS, 2) void flash_attn_prefill_kernel
 
     if (nsp > 1) {                                              // partial record [D O][m][l] of (query, head, split)
         if (q_ok) {
-            float *dst = a.part + (((size_t)qt * H + h) * nsp + zsp) * (D + 2);
+            float *dst = a.part + (((size_t)qt * H + h) * nsp + zsp) * att_rec(D);
 #pragma unroll
             for (int db = 0; db < NB; db++)
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    float *o = dst + 32 * db + 8 * rq + 4 * kg;  // records are 8-byte aligned only ((D + 2) floats)
-                    o[0] = O[db][rq * 4 + 0]; o[1] = O[db][rq * 4 + 1]; o[2] = O[db][rq * 4 + 2]; o[3] = O[db][rq * 4 + 3];
-                }
+                for (int rq = 0; rq < 4; rq++) *reinterpret_cast<float4 *>(dst + 32 * db + 8 * rq + 4 * kg) = float4{O[db][rq * 4 + 0], O[db][rq * 4 + 1], O[db][rq * 4 + 2], O[db][rq * 4 + 3]};
             if (kg == 0) { dst[D] = m_run * 0.6931471805599453f; dst[D + 1] = l_run; }   // (the merge works in natural-log units)
         }
         return;
@@ -748,7 +745,7 @@ bool flash_attn_prefill_applicable(const AttnArgs &a) {
 
 // Key splits of a prompt batch.  Two things pull: the causal tiles are 1 .. n_chunks long, so a few splits balance the workgroups
 // (512 tokens: 128 (kv head, tile) pairs on 512 workgroup slots, the last 16x as long as the first - 4 splits took 3.1 -> 2.0 ms);
-// but every split leaves a (D + 2)-float record per query and head that the merge reads back (2048 tokens x 8 splits: 272 MB, a
+// but every split leaves a record of D + 2 values per query and head that the merge reads back (2048 tokens x 8 splits: 272 MB, a
 // 110 us merge per layer beside a 327 us kernel).  So: as many splits as fill ~512 workgroups (measured, 8B model: 512 tokens 4 splits
 // 1.76 ms of attention per prompt against 1.80 with 2 and 2.07 with 6; 2048 tokens NO split 7.1 ms against 8.8 with 2 - the 512
 // (kv head, tile) pairs fill the chip by themselves and the merge costs more than the imbalance), never more than a quarter of the

@@ -633,6 +633,9 @@ hipError_t launch_step_setup_embed(const int32_t *tok_pos, int T, RopeArgs ra, f
                                    const StepBlock *ring = nullptr, const unsigned *turn = nullptr);
 hipError_t launch_rope_inplace(float *x, int T, int n_head, int D, const int32_t *tok_pos, RopeArgs ra, hipStream_t st);
 
+// A record of a share of a head's keys: D weighted values, the maximum, the sum of weights; begun on a 128-byte line of its own.  (D + 2 floats one behind the other put two workgroups' values
+// on one line, and no 16-byte load is aligned.  The merge of ticks of 4, 16 and 32 conversations from 90 cells up, 32 / 8 heads of 128: 3.85, 4.69, 5.65 us so, 3.56, 4.54, 5.13 here)
+__host__ __device__ constexpr int att_rec(int D) { return D + 32; }
 struct AttnArgs {
     const float *q;          // [T][H][D] (already rotated)
     float *out;              // [T][H][D]
@@ -646,9 +649,9 @@ struct AttnArgs {
     const int32_t *n_kv_dev;   // device scalar: cells to scan (high-water mark)
     int n_kv_max;              // host upper bound used to size the grid
     float scale;
-    float *part;               // workspace [T][H][splits][D+2]
+    float *part;               // workspace [T][H][splits][att_rec(D)]
     int splits;
-    int pf_splits = 0;         // prompt kernel (attn_prefill.hip): key splits per query tile, workspace [T][H][pf_splits][D+2]; 0 / 1 = none
+    int pf_splits = 0;         // prompt kernel (attn_prefill.hip): key splits per query tile, workspace [T][H][pf_splits][att_rec(D)]; 0 / 1 = none
     // batched single-token steps: per token, the 64-cell chunks that can hold a visible cell (host-built from the cell
     // table); nullptr = every chunk of the scanned range.  tok_chunks[t * chunk_stride + i], i < tok_nchunks[t] <= splits
     const int32_t *tok_chunks = nullptr;
@@ -679,7 +682,7 @@ bool flash_attn_cols_applicable(const AttnArgs &a);
 bool flash_attn_cols_takes(const AttnArgs &a, bool one_token_kernel);      // one_token_kernel: the batch of a decoder, which has kernels for one token at a time
 int flash_attn_cols_splits(const AttnArgs &a);
 hipError_t launch_flash_attn_cols(const AttnArgs &a, hipStream_t st);
-// merge of [T][H][splits][D+2] partial records into a.out (+ quantised rows when a.out_q): attn.hip
+// merge of [T][H][splits][att_rec(D)] partial records into a.out (+ quantised rows when a.out_q): attn.hip
 hipError_t launch_flash_attn_combine(const AttnArgs &a, int splits, hipStream_t st);
 // decode-step variants (attn.hip): single round trip per workgroup; q passed UN-rotated (rope fused), NORM rope, D = 128
 bool flash_attn_decode_applicable(const AttnArgs &a, const RopeArgs &ra);
