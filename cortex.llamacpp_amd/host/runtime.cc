@@ -1115,6 +1115,10 @@ static bool store_fuse_enabled() {
     static const bool env_off = getenv("MI355_ATTN_STORE_FUSE") && getenv("MI355_ATTN_STORE_FUSE")[0] == '0';
     return g_store_fuse && !env_off;
 }
+static int attn_mode() {
+    static const int mode = getenv("MI355_ATTN_MODE") ? atoi(getenv("MI355_ATTN_MODE")) : 2;
+    return mode;
+}
 static bool g_last_rows = true;
 void set_last_rows(bool on) { g_last_rows = on; }
 static bool g_late_sums = true;
@@ -1516,7 +1520,6 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         if (o_pl) { aa.out_bh = mmq_bh_; aa.out_bl = mmq_bl_; }
         // (the single-launch step and the store-fused batched step write the new K / V rows themselves; only the third branch needs the fast store kernel)
         const bool fast_store = kv_store_fast_applicable(G, D, cp.type_k, cp.type_v, ra);
-        static const int attn_mode = getenv("MI355_ATTN_MODE") ? atoi(getenv("MI355_ATTN_MODE")) : 2;
         bool fused_step = false, attn_out_done = false;
         // (parity mode for an f16 cache: the generic launch below dispatches to the cell-by-cell kernel with fp16 V accumulation)
         const bool v16 = fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16;
@@ -1530,7 +1533,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 aa.tok_chunks = d_chunks_; aa.tok_nchunks = d_chunks_ + (size_t)64 * chunk_stride_; aa.chunk_stride = chunk_stride_;
                 aa.splits = std::max(chunk_cap_, chunk_lmax_);
             }
-            fused_step = attn_mode > 0 && flash_attn_decode_fused_applicable(aa, ra);
+            fused_step = attn_mode() > 0 && flash_attn_decode_fused_applicable(aa, ra);
         }
         // single-token step: attention + attn_output in one launch (attn_out.hip) where it has a form for the shape
         // (not where the ranks of a row split exchange through the host callback - the transport of a rig whose ranks SHARE one device: this kernel's
@@ -1541,7 +1544,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         const MMVQSeg ao_seg = make_seg(L.wo, tp ? tp_part_ : x_, E, ao_add ? x_ : nullptr, nullptr);
         AttnArgs af = aa;
         bool ao_form = false;
-        if (decode_attn && fused_step && attn_mode == 2 && !engine && il < 255 && !attn_out_off_ && !attn_out_skip_step_ && !(tp && tp_uses_host())) {
+        if (decode_attn && fused_step && attn_mode() == 2 && !engine && il < 255 && !attn_out_off_ && !attn_out_skip_step_ && !(tp && tp_uses_host())) {
             af.splits = attn_out_fused_splits(af);
             if (chunk_lmax_ > 0) af.splits = aa.splits;
             ao_form = attn_out_fused_applicable(af, ra, ao_seg, (int)L.wo.K, ao_add ? EPI_ADD : EPI_STORE);
@@ -1616,7 +1619,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                     attn_out_done = true;
                 }
                 if (!attn_out_done)
-                    HIP_TRY(launch_flash_attn_decode_fused(aa, rope_cs_, ra, k_, v_, d_cell_, attn_mode == 2 ? att_counters_ : nullptr, stream_));
+                    HIP_TRY(launch_flash_attn_decode_fused(aa, rope_cs_, ra, k_, v_, d_cell_, attn_mode() == 2 ? att_counters_ : nullptr, stream_));
             } else if (batch_distinct_ && store_fuse_enabled()) {
                 // batched step, every token of a different sequence: K rope + KV store inside the attention launch (no token reads another's new cell)
                 HIP_TRY(launch_flash_attn_decode(aa, rope_cs_, ra, stream_, k_, v_, d_cell_));
@@ -2080,15 +2083,20 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         }
     }
     bool lists_usable = false;                                 // only the split-per-chunk attention kernels walk the lists
+    bool one_fused = false;                                    // ... a single token's only in the launch that stores K and V itself
     attn_cols_ = false;                                        // every token of one and the same sequence: one list, and attn_cols.hip where it has a form for the batch
     AttnArgs aa{};
     if (!model->nvx && !model->hp.encoder) {
         const HParams &hp = model->hp;
         RopeArgs ra = rope_args(*model, false);
         aa.T = n; aa.H = hp.n_head; aa.G = hp.n_head_kv; aa.D = hp.head_dim; aa.n_ctx = (int)cp.n_ctx; aa.n_kv_max = n_kv_; aa.type_k = cp.type_k; aa.type_v = cp.type_v;
-        lists_usable = n <= 64 && flash_attn_decode_applicable(aa, ra) && kv_store_fast_applicable(aa.G, aa.D, cp.type_k, cp.type_v, ra);
-        attn_cols_ = n >= 2 && seqmask[0] != 0 && (seqmask[0] & (seqmask[0] - 1)) == 0 && std::all_of(seqmask, seqmask + n, [&](uint64_t m) { return m == seqmask[0]; }) &&
-                     !(fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16);
+        const bool fast_store = kv_store_fast_applicable(aa.G, aa.D, cp.type_k, cp.type_v, ra);
+        const bool v16 = fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16;
+        // (a store of its own in front of the kernels that walk them, or their own: without either the general attention takes the batch, which knows no lists.
+        // Sixteen conversations of 90 to 1005 cells, 32 / 4 heads of 64: 138 chunks each without a list against 17, attention and its merge 30.4 us a layer against 14.2)
+        one_fused = n == 1 && !fast_store && attn_mode() > 0;
+        lists_usable = n <= 64 && !v16 && flash_attn_decode_applicable(aa, ra) && (fast_store || one_fused || (batch_distinct_ && store_fuse_enabled()));
+        attn_cols_ = n >= 2 && seqmask[0] != 0 && (seqmask[0] & (seqmask[0] - 1)) == 0 && std::all_of(seqmask, seqmask + n, [&](uint64_t m) { return m == seqmask[0]; }) && !v16;
     }
     if (attn_cols_ || ((n >= 2 || cp.n_seq_max > 1) && lists_usable)) {
         const int nch = (n_kv_ + 63) / 64;
@@ -2109,6 +2117,10 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             }
         }
         if (chunk_lmax_ < 1) chunk_lmax_ = 1;
+        if (one_fused) {
+            aa.splits = std::min(chunk_stride_, (chunk_lmax_ + 3) & ~3);
+            lists_usable = lists_usable && flash_attn_decode_fused_applicable(aa, rope_args(*model, false));
+        }
         const size_t words = attn_cols_ ? (size_t)chunk_lmax_ : (size_t)64 * (chunk_stride_ + 1);
         if (!attn_cols_ && !lists_usable) chunk_lmax_ = 0;     // (a long batch for the prompt kernel: no lists)
         else {
