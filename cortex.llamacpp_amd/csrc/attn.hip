@@ -849,6 +849,16 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
     // once serialise (tools/bench_gridbar.hip: 25 us for 512).  Measured on the 8B step: 424 -> 448 tok/s at 4000 cells.
     // MI355_ATTN_COH=0 restores the fenced form.
     static const bool coh = !(getenv("MI355_ATTN_COH") && getenv("MI355_ATTN_COH")[0] == '0');
+    // (what a workgroup of 1024 threads holds: a step's first 256 cells)
+    if (counters && a.splits <= WHOLE_NS && a.D == WHOLE_D && (R == WHOLE_R || R == 2 * WHOLE_R)) {
+#define FADW(TK, TV) hipLaunchKernelGGL((flash_attn_decode_whole_kernel<TK, TV>), dim3(a.H / WHOLE_R), dim3(256 * WHOLE_NS), 0, st, a, cs_table, ra.n_rot, fz)
+        if (a.type_k == T_F16 && a.type_v == T_F16) FADW(T_F16, T_F16);
+        else if (a.type_k == T_Q8_0 && a.type_v == T_Q8_0) FADW(T_Q8_0, T_Q8_0);
+        else if (a.type_k == T_Q8_0) FADW(T_Q8_0, T_F16);
+        else FADW(T_F16, T_Q8_0);
+#undef FADW
+        return hipGetLastError();
+    }
 #define FAD_D(RR, TK, TV, DD) do { if (coh && counters) hipLaunchKernelGGL((flash_attn_decode_kernel<RR, TK, TV, true, true, DD>), grid, dim3(256), 0, st, a, cs_table, ra.n_rot, fz); \
                                    else hipLaunchKernelGGL((flash_attn_decode_kernel<RR, TK, TV, true, false, DD>), grid, dim3(256), 0, st, a, cs_table, ra.n_rot, fz); } while (0)
 #define FAD(RR, TK, TV) do { if (a.D == 64) FAD_D(RR, TK, TV, 64); else FAD_D(RR, TK, TV, 128); } while (0)

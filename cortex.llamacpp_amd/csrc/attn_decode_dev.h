@@ -66,40 +66,70 @@ struct DecodeFuse {
     unsigned long long *probe;
 };
 
+// a wave quantises block gb of the token's attention output, its 256 values in LDS
+template <bool COH>
+__device__ __forceinline__ void decode_quant_block(const DecodeFuse &fz, const float *x, int gb, int lane) {
+    const float4 v4 = *reinterpret_cast<const float4 *>(x + lane * 4);
+    const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+    const int e0 = gb * 256 + lane * 4;
+    if (fz.want_q8k) {
+        uint32_t packed; int bs; float dq8;
+        wave_quant_q8k(vv, lane, packed, bs, dq8);
+        cst4<COH>(fz.q.qs + e0, packed);
+        if ((lane & 3) == 0) cst2<COH>(fz.q.bsums + gb * 16 + (lane >> 2), (unsigned short)(int16_t)bs);
+        if (lane == 0) cstf<COH>(fz.q.d + gb, dq8);
+    }
+    if (fz.want_q80) {
+        uint32_t packed; float dd;
+        wave_quant_q80(vv, packed, dd);
+        cst4<COH>(fz.q.qs0 + e0, packed);
+        if ((lane & 7) == 0) cst2<COH>(fz.q.d0 + gb * 8 + (lane >> 3), f2h(dd));
+    }
+}
+
 // body of one (kv head g, chunk slot sp, token t) work item; 256 threads, every exit is workgroup-uniform
 // COH (decode_mega.hip): q / K / V of the token come from other workgroups of the same launch and the results go to
 // other workgroups of the same launch: those accesses are made device-coherent (dev_common.h) and the ticket is a relaxed
 // atomic, instead of an agent-scope release / acquire whose cache-wide write-back and invalidate cost microseconds.
 // D = 128 (default) or 64: head_dim; every lane role below is derived from it
-template <int R, int TK, int TV, bool FUSED, bool COH = false, int D = 128>
-__device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const float *cs_table, int n_rot, const DecodeFuse &fz, int g, int sp, int t) {
+// NS > 1: a workgroup of NS * 256 threads holds all chunks of R query heads from qh on, a chunk to 256 threads; their merge needs no ticket then (flash_attn_decode_whole_kernel)
+template <int R, int TK, int TV, bool FUSED, bool COH = false, int D = 128, int NS = 1>
+__device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const float *cs_table, int n_rot, const DecodeFuse &fz, int g, int sp, int t, int qh) {
     constexpr int C = 64, NB = D / 32;
     // (a q4_0 cache - TK = TV = T_Q4_0, head_dim 128 - keeps 16 nibble bytes per 32-block: a piece is a whole block, four lanes per cell)
     constexpr int KROW = TK == T_F16 ? 2 * D : TK == T_Q4_0 ? D / 2 : D, VROW = TV == T_Q4_0 ? D / 2 : D;   // bytes of a K row; bytes (halfs for f16) of a V row
     constexpr int LPC = KROW / 16;                           // lanes per cell in the score pass (16-byte pieces of a K row)
     constexpr int KP = C * LPC / 256;                       // 16-byte K pieces per thread
     constexpr int DQ = D / 4, NCG = 256 / DQ, CPG = C / NCG;   // P.V pass: DQ lanes of 4 dims, NCG cell groups of CPG cells
-    __shared__ __attribute__((aligned(16))) float qf[R * D];         // rotated q (f16-rounded for an f16 cache)
-    __shared__ __attribute__((aligned(16))) int8_t qc[R * D];        // q8_0 codes of q
-    __shared__ float qd[R * NB];
-    __shared__ __attribute__((aligned(16))) float S[R * C];          // [cell][head]: a cell's weights are read together
+    __shared__ __attribute__((aligned(16))) float qf_[NS][R * D];         // rotated q (f16-rounded for an f16 cache)
+    __shared__ __attribute__((aligned(16))) int8_t qc_[NS][R * D];        // q8_0 codes of q
+    __shared__ float qd_[NS][R * NB];
+    __shared__ __attribute__((aligned(16))) float S_[NS][R * C];          // [cell][head]: a cell's weights are read together
     // (the f16 scores and P V multiply and add in one instruction: with [head][cell] and two of them ticks of 4, 16 and 32 conversations, 32 / 8 heads of 128, took 7.40, 14.2 and 23.1 us a layer
     // instead of 7.17, 13.8 and 21.5, sixteen with 32 / 4 heads of 64 18.1 instead of 16.9 to 17.5: the chunk's arithmetic is a chain of one workgroup)
-    __shared__ float ml[R * 2];
-    __shared__ int vis[C];
-    __shared__ uint32_t ksc[C * NB / 2], vsc[C * NB / 2];           // f16 block scales of the chunk
-    __shared__ __attribute__((aligned(16))) float accs[NCG * R * D];
-    __shared__ __attribute__((aligned(16))) uint8_t newk[D * 2], newv[D * 2];   // the token's own cache row (codes or f16)
-    __shared__ uint32_t newkd[2], newvd[2];                                      // its f16 block scales, two per word
-    __shared__ int last_flag;
-    const int tid = tid_now(), lane = tid & 63, wave = tid >> 6;
+    __shared__ float ml_[NS][R * 2];
+    __shared__ int vis_[NS][C];
+    __shared__ uint32_t ksc_[NS][C * NB / 2], vsc_[NS][C * NB / 2];           // f16 block scales of the chunk
+    __shared__ __attribute__((aligned(16))) float accs_[NS][NCG * R * D];
+    __shared__ __attribute__((aligned(16))) uint8_t newk_[NS][D * 2], newv_[NS][D * 2];   // the token's own cache row (codes or f16)
+    __shared__ uint32_t newkd_[NS][2], newvd_[NS][2];                                      // its f16 block scales, two per word
+    __shared__ int last_flag, any_[NS];
+    const int sub = NS > 1 ? __builtin_amdgcn_readfirstlane(tid_now() >> 8) : 0, tid = NS > 1 ? tid_now() & 255 : tid_now(), lane = tid & 63, wave = tid >> 6;
+    float *const qf = qf_[sub], *const qd = qd_[sub], *const S = S_[sub], *const ml = ml_[sub], *const accs = accs_[sub];
+    int8_t *const qc = qc_[sub];
+    int *const vis = vis_[sub];
+    uint32_t *const ksc = ksc_[sub], *const vsc = vsc_[sub], *const newkd = newkd_[sub], *const newvd = newvd_[sub];
+    uint8_t *const newk = newk_[sub], *const newv = newv_[sub];
     const int n_ctx = a.n_ctx, H = a.H;
     if (FUSED && fz.probe && tid == 0) fz.probe[2 * (sp * a.G + g)] = wall_clock64();
     int chunk = sp;
+    bool live = true;
     if (a.tok_chunks) {                                        // walk this token's chunk list only (sequences own cache regions)
-        if (sp >= a.tok_nchunks[t]) return;
-        chunk = a.tok_chunks[(size_t)t * a.chunk_stride + sp];
-    }
+        live = sp < a.tok_nchunks[t];
+        if (NS == 1 && !live) return;
+        if (live) chunk = a.tok_chunks[(size_t)t * a.chunk_stride + sp];
+    } else if (NS > 1) live = sp < a.splits;
+    if (!live) chunk = 0;                                      // (addresses that exist; nothing of it is visible)
     const int c_lo = chunk * C;
     const size_t head_row0 = (size_t)g * n_ctx;
 
@@ -116,7 +146,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
         const int mine = (tid < C && cpos >= 0 && cpos <= tpos && ((cseq >> tseq) & 1ull)) ? 1 : 0;
         if (!__syncthreads_or(mine)) {
             if (tid < R) {
-                float *dst = a.part + (((size_t)t * H + (size_t)g * R + tid) * a.splits + sp) * att_rec(D);
+                float *dst = a.part + (((size_t)t * H + (size_t)qh + tid) * a.splits + sp) * att_rec(D);
                 dst[D] = -INFINITY; dst[D + 1] = 0.0f;
             }
             return;
@@ -131,10 +161,10 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
         if (pp < NPAIR) {
             const int r = pp / HP, i = pp % HP;
             if (fz.neox) {                                      // the pair's halves lie D / 2 apart
-                const int o = (int)((((size_t)t * H + (size_t)g * R + r) * D + i) * 4);
+                const int o = (int)((((size_t)t * H + (size_t)qh + r) * D + i) * 4);
                 qv[j] = make_float2(__uint_as_float(cld4<COH>(a.q, o)), __uint_as_float(cld4<COH>(a.q, o + HP * 4)));
             } else {
-                const coh_u32x2 qq = cld8<COH>(a.q, (int)((((size_t)t * H + (size_t)g * R + r) * D + 2 * i) * 4));
+                const coh_u32x2 qq = cld8<COH>(a.q, (int)((((size_t)t * H + (size_t)qh + r) * D + 2 * i) * 4));
                 qv[j] = make_float2(__uint_as_float(qq.x), __uint_as_float(qq.y));
             }
             csv[j] = (2 * i < n_rot) ? *reinterpret_cast<const float2 *>(cs_table + (size_t)t * n_rot + 2 * i) : make_float2(1.0f, 0.0f);
@@ -177,7 +207,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     int own_cl = -1;                                   // chunk-local index of the token's cell, if this chunk holds it
     if (FUSED) {
         const int cellnew = fz.tok_cell[t];                      // (t = 0 in a single-token step)
-        if (cellnew >= c_lo && cellnew < c_lo + C) own_cl = cellnew - c_lo;
+        if (live && cellnew >= c_lo && cellnew < c_lo + C) own_cl = cellnew - c_lo;
         if (own_cl >= 0 && wave == 0 && (lane & 31) < DQ) {      // lanes 0 .. DQ - 1: K, lanes 32 .. 32 + DQ - 1: V (whole 8-lane groups either way)
             const bool isk = lane < 32;
             const int dd = (lane & 31) * 4;
@@ -238,7 +268,11 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     }
 
     // ---- q: rotate, convert
-    if (tid < C) vis[tid] = (cpos >= 0 && cpos <= tpos && ((cseq >> tseq) & 1ull)) ? 1 : 0;
+    if (tid < C) {
+        const bool v = live && cpos >= 0 && cpos <= tpos && ((cseq >> tseq) & 1ull);
+        vis[tid] = v ? 1 : 0;
+        if (NS > 1) { const bool some = __ballot(v) != 0; if (tid == 0) any_[sub] = some; }
+    }
     if (tid < C * NB / 2) { ksc[tid] = ks2; vsc[tid] = vs2; }
 #pragma unroll
     for (int j = 0; j < PPT; j++) {
@@ -288,8 +322,10 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     }
 
     // ---- scores
+    const bool any = NS == 1 || __builtin_amdgcn_readfirstlane(any_[sub]) != 0;          // (a chunk without a visible cell: weights of zero, none of the arithmetic)
 #pragma unroll
     for (int j = 0; j < KP; j++) {
+        if (!any) break;
         const int p = tid + 256 * j;
         const int cl = p / LPC, piece = p % LPC;
         float sc[R];
@@ -350,7 +386,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
 
     // ---- softmax of the chunk: wave w -> heads w, w+4, ...; lane = cell
     for (int r = wave; r < R; r += 4) {
-        const float s = S[lane * R + r];
+        const float s = any ? S[lane * R + r] : -INFINITY;
         const float m = wave_max(s);
         const float p = (s == -INFINITY) ? 0.0f : expf(s - m);
         const float l = wave_sum(p);
@@ -365,6 +401,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     for (int r = 0; r < R; r++) { acc[r][0] = acc[r][1] = acc[r][2] = acc[r][3] = 0.0f; }
 #pragma unroll
     for (int i = 0; i < CPG; i++) {
+        if (!any) break;
         const int cl = cg + NCG * i;
         float v4[4];
         if (TV == T_F16) {
@@ -393,11 +430,38 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
         float s = 0.0f;
 #pragma unroll
         for (int j = 0; j < NCG; j++) s += accs[((size_t)j * R + r) * D + d];
-        float *dst = a.part + (((size_t)t * H + (size_t)g * R + r) * a.splits + sp) * att_rec(D);
+        if (NS > 1) { S[e] = s; continue; }                   // (the chunk's weights are spent)
+        float *dst = a.part + (((size_t)t * H + (size_t)qh + r) * a.splits + sp) * att_rec(D);
         cstf<COH>(dst + d, s);
         if (d == 0) { cstf<COH>(dst + D, ml[2 * r]); cstf<COH>(dst + D + 1, ml[2 * r + 1]); }
     }
     if (!FUSED) return;
+    if constexpr (NS > 1) {
+        // every chunk is here: the merge below, of records in LDS
+        static_assert(COH == false && D <= C && (R * D) % 256 == 0 && R <= 4 * NS && R * D <= 256 * NS, "a wave to a head, a thread to an output, whole blocks");
+        __syncthreads();
+        const int all = tid_now(), wv = __builtin_amdgcn_readfirstlane(all >> 6);
+        float *const wgt = accs_[0], *const merged = qf_[0];
+        if (wv < R) {
+            const float m = lane < NS ? ml_[lane < NS ? lane : 0][2 * wv] : -INFINITY, l = lane < NS ? ml_[lane < NS ? lane : 0][2 * wv + 1] : 0.0f;
+            const float M = wave_max(m);
+            const float w = m != -INFINITY ? expf(m - M) : 0.0f;
+            const float den = wave_sum(w * l);
+            if (lane < NS) wgt[wv * 64 + lane] = w * (1.0f / den);
+        }
+        __syncthreads();
+        if (all < R * D) {
+            const int r = all / D;
+            float s = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NS; c++) s += wgt[r * 64 + c] * S_[c][all];
+            merged[all] = s;
+            a.out[(size_t)qh * D + all] = s;
+        }
+        __syncthreads();
+        if (wv < (R * D) >> 8 && (fz.want_q8k || fz.want_q80)) decode_quant_block<COH>(fz, merged + wv * 256, ((qh * D) >> 8) + wv, lane);
+        return;
+    }
     if (fz.counters == nullptr) return;               // store-fused only: the merge runs as its own launch (batched steps: in this launch it takes as long, ticks of 2 to 16 tokens 1 % slower to 1 % faster)
     if (fz.probe && tid == 0) fz.probe[2 * (sp * a.G + g) + 1] = wall_clock64();
 
@@ -497,23 +561,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     constexpr int NBLK = (RM * D) >> 8;                // 256-blocks this ticket group owns in the H*D row
     if (wave < NBLK && (fz.want_q8k || fz.want_q80)) {
         for (int b = wave; b < NBLK; b += 4) {
-            const float4 v4 = *reinterpret_cast<const float4 *>(merged + b * 256 + lane * 4);
-            const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-            const int gb = ((hb * D) >> 8) + b;        // global block index
-            const int e0 = gb * 256 + lane * 4;
-            if (fz.want_q8k) {
-                uint32_t packed; int bs; float dq8;
-                wave_quant_q8k(vv, lane, packed, bs, dq8);
-                cst4<COH>(fz.q.qs + e0, packed);
-                if ((lane & 3) == 0) cst2<COH>(fz.q.bsums + gb * 16 + (lane >> 2), (unsigned short)(int16_t)bs);
-                if (lane == 0) cstf<COH>(fz.q.d + gb, dq8);
-            }
-            if (fz.want_q80) {
-                uint32_t packed; float dd;
-                wave_quant_q80(vv, packed, dd);
-                cst4<COH>(fz.q.qs0 + e0, packed);
-                if ((lane & 7) == 0) cst2<COH>(fz.q.d0 + gb * 8 + (lane >> 3), f2h(dd));
-            }
+            decode_quant_block<COH>(fz, merged + b * 256, ((hb * D) >> 8) + b, lane);
         }
     }
     if (fz.probe) {
@@ -522,18 +570,32 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     }
 }
 
+// (the argument segment is cold at every launch: a read of each of its lines at once, instead of one behind the other where a field is first used)
+__device__ __forceinline__ void decode_args_at_once() {
+    struct KArgs { AttnArgs a; const float *cs; int n_rot; DecodeFuse fz; };
+    const __attribute__((address_space(4))) unsigned *ka = (const __attribute__((address_space(4))) unsigned *)__builtin_amdgcn_kernarg_segment_ptr();
+    unsigned acc = 0;
+#pragma unroll
+    for (int i = 0; i < (int)((sizeof(KArgs) + 63) / 64); i++) acc ^= ka[i * 16];
+    asm volatile("" :: "s"(acc));
+}
+
 template <int R, int TK, int TV, bool FUSED, bool COH = false, int D = 128>
 __global__ __launch_bounds__(256) void flash_attn_decode_kernel(const AttnArgs a, const float *cs_table, int n_rot, const DecodeFuse fz) {
-    // (the argument segment is cold at every launch: a read of each of its lines at once, instead of one behind the other where a field is first used)
-    {
-        struct KArgs { AttnArgs a; const float *cs; int n_rot; DecodeFuse fz; };
-        const __attribute__((address_space(4))) unsigned *ka = (const __attribute__((address_space(4))) unsigned *)__builtin_amdgcn_kernarg_segment_ptr();
-        unsigned acc = 0;
-#pragma unroll
-        for (int i = 0; i < (int)((sizeof(KArgs) + 63) / 64); i++) acc ^= ka[i * 16];
-        asm volatile("" :: "s"(acc));
-    }
-    flash_attn_decode_item<R, TK, TV, FUSED, COH, D>(a, cs_table, n_rot, fz, blockIdx.x, blockIdx.y, blockIdx.z);
+    decode_args_at_once();
+    flash_attn_decode_item<R, TK, TV, FUSED, COH, D>(a, cs_table, n_rot, fz, blockIdx.x, blockIdx.y, blockIdx.z, blockIdx.x * R);
+}
+
+// A single token's step over few cells: a workgroup holds R of a kv head's query heads (of H / G: the others' workgroups read the same chunks) and all WHOLE_NS chunks, so that a record, the
+// ticket and the other workgroups' records (a trip of the fabric each) leave the chain.  The same arithmetic in the same order.  Four heads of 64: their results are one block of 256 values to
+// quantise, and four chunks of them are a CU's threads.  us a launch, 32 / 4 heads of 64, f16 cache, behind 20, 93 and 250 cells: 6.3, 6.7 and 7.1; with a workgroup a chunk and the ticket 8.7
+// (six layers' step 220 -> 203, 206 and 212)
+constexpr int WHOLE_NS = 4, WHOLE_R = 4, WHOLE_D = 64;
+template <int TK, int TV>
+__global__ __launch_bounds__(256 * WHOLE_NS) void flash_attn_decode_whole_kernel(const AttnArgs a, const float *cs_table, int n_rot, const DecodeFuse fz) {
+    decode_args_at_once();
+    const int parts = a.H / a.G / WHOLE_R;
+    flash_attn_decode_item<WHOLE_R, TK, TV, true, false, WHOLE_D, WHOLE_NS>(a, cs_table, n_rot, fz, blockIdx.x / parts, __builtin_amdgcn_readfirstlane(tid_now() >> 8), 0, blockIdx.x * WHOLE_R);
 }
 
 }  // namespace mi355

@@ -119,7 +119,7 @@ __device__ __forceinline__ void mega_mmvq(const MMVQArgs &a, uint8_t *smem, cons
 template <int R, int TK, int TV>
 __device__ __forceinline__ void mega_attention(const AttnArgs &aa, const float *cs_table, int n_rot, const DecodeFuse &fz, int items) {
     for (int it = (int)blockIdx.x; it < items; it += (int)gridDim.x) {
-        flash_attn_decode_item<R, TK, TV, true, true>(aa, cs_table, n_rot, fz, it % aa.G, it / aa.G, 0);
+        flash_attn_decode_item<R, TK, TV, true, true>(aa, cs_table, n_rot, fz, it % aa.G, it / aa.G, 0, (it % aa.G) * R);
         __syncthreads();                                         // the item's LDS is reused by the next one / the next phase
     }
 }
