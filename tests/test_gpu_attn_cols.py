@@ -128,3 +128,28 @@ def test_texts_of_two_sequences_in_one_batch(pkg, tmp_path, n):
         ref = bert_forward_f64(path, toks[:, s], np.arange(n))[-1]
         assert np.linalg.norm(got[:, s] - ref) / np.linalg.norm(ref) <= 1.6e-3
     c.close(); m.close()
+
+
+@pytest.mark.parametrize("model,past,n", [("tinyllama-1.1b", 0, 2), ("tinyllama-1.1b", 0, 3), ("tinyllama-1.1b", 61, 31), ("tinyllama-1.1b", 200, 2),     # heads of 64 in groups of eight
+                                          ("tiny-d128", 123, 5), ("tiny-d128", 124, 5), ("tiny-d128", 0, 2),                     # heads of 128: two chunks of cells, and three
+                                          ("tiny-d128-mha", 251, 4), ("tiny-d128-mha", 253, 4), ("tiny-d128-mha", 253, 3)])      # keys of their own: four chunks and five, four tokens and three
+@pytest.mark.parametrize("kv", [1, 8])
+def test_few_tokens_as_steps(pkg, tmp_path, model, past, n, kv):
+    """A few tokens as one batch, on either side of the rule that chooses their kernel, and the same as single steps.  f16 weights: what differs is the order of f32 sums and, of a q8_0
+    cache or a rounded activation, a code here and there, whose share of a logit is below 1e-3 of the largest."""
+    path = str(tmp_path / "m.gguf")
+    cfg = dataclasses.replace(pkg.gguf_synth.CONFIGS[model], n_layer=2, n_vocab=512)
+    pkg.gguf_synth.write_synthetic_llama(path, cfg, "f16", seed=5, with_vocab=False)
+    m = pkg.Model(path)
+    talk = np.random.default_rng(past + n).integers(3, 512, past + n)
+    out = []
+    for each in (n, 1):
+        c = pkg.Context(m, n_ctx=512, n_batch=256, n_ubatch=256, type_k=kv, type_v=kv)
+        if past:
+            assert c.decode(talk[:past // 2], np.arange(past // 2), 0) == 0 and c.decode(talk[past // 2:past], np.arange(past // 2, past), 0) == 0
+        for i in range(past, past + n, each):
+            assert c.decode(talk[i:i + each], np.arange(i, i + each), 0) == 0
+        out.append(np.array(c.logits(-1)))
+        c.close()
+    m.close()
+    assert np.abs(out[0] - out[1]).max() <= 1e-3 * np.abs(out[1]).max()
