@@ -518,21 +518,21 @@ static bool cols_long(const AttnArgs &a) {
 //                               22 / 200 13.3 / 12.6, 31 / 150 13.7 / 12.9, 31 / 200 13.1 / 14.6, 32 / 0 11.4 / 10.8, 40 / 0 11.3 / 11.2, 64 / 0 11.0 / 11.4
 //   32 / 32 heads of 128, f16   2 / 2100 20.4 / 17.0, 2 / 3000 21.2 / 24.0, 2 / 3900 22 / 29, 3 / 1900 17.0 / 19.2, 5 / 900 13.5 / 16.8, 12 / 400 12.3 / 16.5, 32 / 0 8.3 / 10.7
 //   32 / 4 heads of 64, f16     3 / 1900 11.7 / 15.6, 8 / 700 10.1 / 14.6, 22 / 200 7.4 / 14.4
-// A pass, us, all of 2, 4, 8, 16 and 31 tokens here / there, first behind nothing:
-//   six layers, 32 / 4 of 64, f16     0 cells 327 / 365, 374 / 414, 370 / 415, 376 / 420, 383 / 438     200  347 / 387, 391 / 441, 389 / 440, 397 / 441, 397 / 458     1500  371 / 398, 415 / 446, 415 / 471
-//     q8_0                            0  335 / 369, 387 / 419, 380 / 422, 388 / 426, 395 / 443          300  357 / 381, 405 / 431, 400 / 432, 403 / 439, 411 / 478      900  358 / 385, 407 / 434, 406 / 438
-//     32 / 8 of 64                    f16 0  349 / 375, 395 / 427, 392 / 422, 399 / 432, 400 / 452      q8_0 500  384 / 389, 432 / 443, 435 / 446, 440 / 495, 439 / 562
-//     32 / 32 of 64                   f16 300  368 / 366, 407 / 412, 415 / 410, 413 / 422, 439 / 455    q8_0 500  371 / 368, 412 / 405, 423 / 413, 414 / 435, 429 / 483
-//   eight layers, 32 / 32 of 128, f16 0  770 / 783, 606 / 618, 618 / 637, 652 / 669, 761 / 783          200  792 / 788, 642 / 632, 663 / 672     260  787 / 792, 631 / 635, 639 / 654     500  789 / 791, 619 / 635, 641 / 664
-//     32 / 8 of 128, f16              0  749 / 772, 648 / 652, 658 / 667, 674 / 685, 762 / 777          330  775 / 763, 668 / 653, 682 / 667, 697 / 702
-//       q8_0                          20  761 / 781, 648 / 650, 666 / 664, 694 / 688                    90  751 / 765, 643 / 652, 671 / 667, 689 / 691     130  768 / 770, 661 / 659, 680 / 669
-// So here with heads of 64 in groups of four and more; with heads of 128 while the cells are two chunks of 64, a q8_0 cache's to four tokens; f16 heads of 128 with keys of their own
-// from four tokens and five chunks on; else by the work.
-// (The encoder has no such kernel: 3 tokens 5.7 / 7.9 with the general one.)
+// A pass of eight layers with heads of 128, us, at 2, 4, 8, 16 and 31 tokens, here / there, behind so many cells:
+//   32 / 32, f16     0  770 / 783, 606 / 618, 618 / 637, 652 / 669, 761 / 783     200  792 / 788, 642 / 632, 663 / 672     260  787 / 792, 631 / 635, 639 / 654     500  789 / 791, 619 / 635, 641 / 664
+//   32 / 8, f16      0  749 / 772, 648 / 652, 658 / 667, 674 / 685, 762 / 777     330  775 / 763, 668 / 653, 682 / 667, 697 / 702
+//   32 / 8, q8_0     20  761 / 781, 648 / 650, 666 / 664, 694 / 688     90  751 / 765, 643 / 652, 671 / 667, 689 / 691     130  768 / 770, 661 / 659, 680 / 669
+// So here while the cells are two chunks of 64, a q8_0 cache's to four tokens, and for f16 heads with keys of their own from four tokens and five chunks on; else by the work.
+// Where no store of K and V goes with the one-token kernel (fewer than 1024 values a row, NEOX pairs), the general attention is what there is, which knows no lists and needs a merge: here
+// always.  A pass, us, at 2, 3, 8, 16 and 31 tokens, here / there:
+//   six layers, 32 / 4 of 64, f16           0  327 / 365, 371 / 414, 370 / 415, 376 / 425, 383 / 437     200  347 / 391, 397 / 452, 389 / 438     1500  355 / 387, 396 / 440
+//   32 / 8 of 64, f16                       0  337 / 365, 375 / 406, 374 / 408, 379 / 410, 387 / 433     330  368 / 382, 412 / 434, 405 / 434
+//   four layers, 28 / 4 of 128, NEOX, q8_0  130  366 / 407, 365 / 404, 377 / 414, 386 / 433, 443 / 502     1500  371 / 412, 367 / 415      f16 130  349 / 392, 353 / 392, 361 / 402, 375 / 420
+//   six layers, 12 / 2 of 128, NEOX, f16    130  404 / 458, 360 / 413, 369 / 407, 378 / 415, 407 / 413     900  394 / 440, 345 / 379
+// (Nor has the encoder a one-token kernel: 3 tokens 5.7 / 7.9 with the general one.)
 static bool cols_short(const AttnArgs &a) {
     const int ch = (cols_chunks(a) + 1) / 2, work = a.T * ch;
     const bool wide = a.D == 128, q8 = a.type_k == T_Q8_0;
-    if (!wide && a.H >= 4 * a.G) return true;
     if (a.T >= (wide && q8 ? 40 : 32)) return true;
     if (wide && ch <= 2 && (!q8 || a.T <= 4)) return true;
     if (wide && !q8 && a.H == a.G && ch >= 5 && a.T >= 4) return true;

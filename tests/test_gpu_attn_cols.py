@@ -130,8 +130,9 @@ def test_texts_of_two_sequences_in_one_batch(pkg, tmp_path, n):
     c.close(); m.close()
 
 
-@pytest.mark.parametrize("model,past,n", [("tinyllama-1.1b", 0, 2), ("tinyllama-1.1b", 0, 3), ("tinyllama-1.1b", 61, 31), ("tinyllama-1.1b", 200, 2),     # heads of 64 in groups of eight
-                                          ("tiny-d128", 123, 5), ("tiny-d128", 124, 5), ("tiny-d128", 0, 2),                     # heads of 128: two chunks of cells, and three
+@pytest.mark.parametrize("model,past,n", [("tinyllama-1.1b", 0, 2), ("tinyllama-1.1b", 0, 3), ("tinyllama-1.1b", 61, 31), ("tinyllama-1.1b", 200, 2),     # no store of K and V of its own: columns at any size
+                                          ("tiny-qwen2", 0, 3), ("tiny-qwen2", 130, 9),                                          # NEOX pairs: so there
+                                          ("tiny-d128", 123, 4), ("tiny-d128", 123, 5), ("tiny-d128", 125, 4), ("tiny-d128", 0, 2),      # two chunks of cells, and three
                                           ("tiny-d128-mha", 251, 4), ("tiny-d128-mha", 253, 4), ("tiny-d128-mha", 253, 3)])      # keys of their own: four chunks and five, four tokens and three
 @pytest.mark.parametrize("kv", [1, 8])
 def test_few_tokens_as_steps(pkg, tmp_path, model, past, n, kv):
