@@ -19,7 +19,7 @@ struct ActRows {
     uint16_t *d0 = nullptr;    // [T][K/32]
 };
 struct ActQuant : ActRows {
-    uint8_t *qf = nullptr;     // nullable: the q8_K blocks of a batch of 3 .. FEW_MAX_T rows once more, as mmq_few.hip's operands
+    uint8_t *qf = nullptr;     // nullable: the q8_K blocks of a batch of 2 .. FEW_MAX_T rows once more, as mmq_few.hip's operands
 };
 // mmq_few.hip: a block of qf is 16 rows (tokens) x one super-block, blocks [row tile][super-block].  Codes: element k of row t lies at
 // (k / 64) * 1024 + ((t & 15) + 16 * (k / 8 % 4)) * 16 + k / 32 % 2 * 8 + k % 8 - a lane's 16 bytes of a step of 64 are 8 of either half.  Behind them the block
@@ -28,7 +28,7 @@ constexpr int FEW_BH = 4096, FEW_BL = FEW_BH + 256, FEW_D = FEW_BL + 256, FEW_BL
 inline ActQuant act_for(const ActQuant *q, int T) {       // what a quantiser of T rows writes
     ActQuant r;
     if (q) r = *q;
-    if (T < 3 || T > FEW_MAX_T) r.qf = nullptr;
+    if (T < 2 || T > FEW_MAX_T) r.qf = nullptr;
     return r;
 }
 inline size_t few_bytes(int64_t K) { return K % 256 ? 0 : (size_t)(FEW_MAX_T / 16) * (size_t)(K / 256) * FEW_BLOCK; }
@@ -181,10 +181,11 @@ bool mmq_ksplit_applicable(int type, int K, int T);
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair = false);
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                                    bool swiglu, hipStream_t st);
-// mmq_few.hip: 3 .. 64 tokens of the same, bit for bit; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
+// mmq_few.hip: 3 .. 64 tokens of the same, bit for bit, and two where mmq_few_pair; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
+bool mmq_few_pair(int type, int K, int T, const ActQuant &q);
 bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu);
 hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);
-// the same as the output head: 3 .. HEAD_MAX_T rows of logits are stored to `host` too ([T][ld_out] of pinned memory; nullable) while the weights stream, and each row's arg-max
+// the same as the output head: 2 (mmq_few_pair) or 3 .. HEAD_MAX_T rows of logits are stored to `host` too ([T][ld_out] of pinned memory; nullable) while the weights stream, and each row's arg-max
 // (the lowest index of equals) to win[t].  scratch: mmq_few_head_scratch() words, zero before the first launch
 constexpr int HEAD_MAX_T = 32;
 size_t mmq_few_head_scratch();

@@ -1589,8 +1589,7 @@ void mmq_set_lds_form(int on) { g_mmq_p2 = on; }
 static int g_ksplit_max = getenv("MI355_KSPLIT_MAX") ? atoi(getenv("MI355_KSPLIT_MAX")) : 256;
 bool mmq_ksplit_applicable(int type, int K, int T) {
     // from 3 tokens: the mat-vec takes 4 + 2 + 1 tokens per pass over the weights, so 3 sequences cost 4.5 ms and 6 cost 6.4 ms a step against
-    // 3.7 ms through this kernel.  Two stay with the mat-vec, whose sums are the one-token step's bit for bit: a pair of conversations then spells the text that
-    // either spells alone (mmq_few.hip adds the super-blocks up in another order)
+    // 3.7 ms through this kernel.  Two go to mmq_few.hip or stay with the mat-vec (mmq_few_pair)
     return (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K % 256) == 0 && T >= 3 && T <= g_ksplit_max;
 }
 

@@ -671,6 +671,8 @@ void few_type(const FewArgs &a, int blocks, hipStream_t st) {
 #undef GO
 }
 
+constexpr int FEW_PAIR_K = 1280;
+
 }  // namespace
 
 // Whether a launch of T tokens is the faster one here (the sums are the same either way; us, here against the K-split kernel of mmq.hip):
@@ -679,6 +681,11 @@ void few_type(const FewArgs &a, int blocks, hipStream_t st) {
 //     take twice the instructions, there is but one round: 4096 x 4096 10.8 / 13.3, but 6144 x 4096 15.6 / 14.1 and 152064 x 3584 270 / 242;
 //   * to 64, where the operands of four token tiles leave two units in flight: gate | up, 42 / 50 (14336 x 4096), and long rows, 32.7 / 39.5 (4096 x 14336) - but 13.5 / 12.7
 //     (4096 x 4096), 112 / 77 (8192 x 28672: 512 row tiles), 318 / 217 (152064 x 3584), and Q6_K never, 549 / 233.
+// Two tokens, from rows of FEW_PAIR_K columns on.  The mat-vec's sums of two are the one-token step's only for Q6_K and while no two waves share a row, so a pair of conversations and either alone
+// are as far apart there as any two orders of a sum are (8B and 7B: logits 0.010).  us a tick of two conversations and a turn of two tokens, here / the mat-vec: eight 8B Q4_K_M layers
+// 677 / 885, 648 / 805, eight 7B Q5_K_M layers 654 / 870, 627 / 847, six layers of 2048 and 5632 columns, Q4_K_M 313 / 384, 297 / 386; of 1280 and 3584 columns a tick 293, of three 305.  Of
+// shorter rows launches are latency (1024 and 2816 columns, two 328, three 303; 512 and 1536 313, 288), and they stay with the mat-vec, whose sums come closest to the single step's.
+bool mmq_few_pair(int type, int K, int T, const ActQuant &q) { return T == 2 && q.qf && (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K & 255) == 0 && K >= FEW_PAIR_K; }
 bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu) {
     if (!q.qf || T > FEW_MAX_T) return false;
     if (T <= 16) return true;
@@ -741,7 +748,7 @@ size_t mmq_few_head_scratch() { return 1 + 2 * (size_t)HEAD_MAX_T * (size_t)num_
 //   32000 x 4096                       3: 152 / 163, 8: 173 / 188, 16: 214 / 237, 17: 245 / 268, 24: 271 / 302, 32: 315 / 346                           3: 148 / 155, 16: 185 / 199, 17: 216 / 227, 32: 255 / 267
 //   32000 x 2048                       3: 115 / 119, 8: 131 / 144, 16: 167 / 186, 17: 182 / 197, 24: 210 / 227, 32: 251 / 273                           3: 108 / 111, 16: 133 / 147, 17: 148 / 156, 32: 186 / 195
 bool mmq_few_head_takes(int type, int K, int T, const ActQuant &q) {
-    return q.qf && (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K & 255) == 0 && T >= 3 && T <= HEAD_MAX_T;
+    return q.qf && (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && (K & 255) == 0 && (T >= 3 || mmq_few_pair(type, K, T, q)) && T <= HEAD_MAX_T;
 }
 hipError_t launch_mmq_few_head(const MMQSeg &seg, int K, int T, const ActQuant &q, float *host, float *scratch, int32_t *win, hipStream_t st) {
     if (!mmq_few_head_takes(seg.type, K, T, q) || !scratch || !win || seg.resid || seg.n_rows < 1) return hipErrorInvalidValue;

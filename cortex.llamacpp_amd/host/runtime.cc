@@ -583,7 +583,7 @@ static void alloc_actq(ActQuant &q, size_t K, size_t T, bool k, bool z, std::vec
         q.qs = (int8_t *)al(T * K);
         q.d = (float *)al(T * (K / 256) * 4);
         q.bsums = (int16_t *)al(T * (K / 16) * 2);
-        if (few && T >= 3 && few_bytes((int64_t)K)) q.qf = (uint8_t *)al(few_bytes((int64_t)K));
+        if (few && T >= 2 && few_bytes((int64_t)K)) q.qf = (uint8_t *)al(few_bytes((int64_t)K));
     }
     if (z) {
         q.qs0 = (int8_t *)al(T * K);
@@ -1005,7 +1005,7 @@ hipError_t Context::linear(const DevTensor &w, const ActQuant &aq, const float *
             return launch_mmq_q80(w.data, w.row_bytes, (int)w.N, K, T, aq, out, ld_out, epi == EPI_ADD ? resid : nullptr, stream_);
         // (bh_over_ / bl_over_: the caller prepared the block-sum planes of a larger batch that aq's rows are a slice of - the expert loop)
         const int8_t *bh = bh_over_ ? bh_over_ : mmq_bh_, *bl = bh_over_ ? bl_over_ : mmq_bl_;
-        if (mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, mmq_ws_, parts != nullptr) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
+        if ((mmq_ksplit_preferred(w.type, (int)w.N, K, T, w.planes != nullptr, mmq_ws_, parts != nullptr) || mmq_few_pair(w.type, K, T, aq)) && pending_fuse_.mode == 0 && epi != EPI_SWIGLU) {   // batched decode steps, short prompts, expert batches: MFMA, K split
             const MMQSeg sg{w.data, w.row_bytes, (int)w.N, w.type, out, ld_out, epi == EPI_ADD ? resid : nullptr, 0};
             if (w.type != T_Q6_K && !bh_over_) HIP_TRY(ensure_prep(aq, K, T, mmq_few_takes(&sg, 1, K, T, aq, false)));
             return launch_mmq_ksplit_multi(&sg, 1, K, T, aq, bh, bl, false, stream_);
@@ -1038,7 +1038,7 @@ hipError_t Context::linear_multi(const DevTensor *const *ws, float *const *outs,
     int all_rows = 0;
     for (int i = 0; i < n; i++) {
         all_mmq &= mmq_applicable(ws[i]->type, K, T);
-        all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T);
+        all_ks &= mmq_ksplit_applicable(ws[i]->type, K, T) || mmq_few_pair(ws[i]->type, K, T, aq);
         all_planes &= ws[i]->planes != nullptr;
         all_rows += (int)ws[i]->N;
     }
@@ -1836,12 +1836,13 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
                 prof_mark("norm_quant");
             }
             bool swiglu_quantised = false;
+            const bool ffn_pair = mmq_few_pair(L.gate.type, E, Tn, aq_e_) && mmq_few_pair(L.up.type, E, Tn, aq_e_);
             const bool ffn_mmq = (mmq_q80_applicable(L.gate.type, E, Tn) && mmq_q80_applicable(L.up.type, E, Tn)) ||
                                  (mmq_applicable(L.gate.type, E, Tn) && mmq_applicable(L.up.type, E, Tn)) ||
-                                 (mmq_ksplit_applicable(L.gate.type, E, Tn) && mmq_ksplit_applicable(L.up.type, E, Tn)) ||
+                                 (mmq_ksplit_applicable(L.gate.type, E, Tn) && mmq_ksplit_applicable(L.up.type, E, Tn)) || ffn_pair ||
                                  (planes_small(L.gate, E, Tn) && planes_small(L.up, E, Tn)) || (q80_copy(L.gate, E, Tn) && q80_copy(L.up, E, Tn));
-            const bool ffn_ks = mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, Tn, L.gate.planes != nullptr, mmq_ws_, false, true) &&
-                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, Tn, L.up.planes != nullptr, mmq_ws_, false, true) && !fuse_ffn;
+            const bool ffn_ks = ffn_pair || (mmq_ksplit_preferred(L.gate.type, (int)L.gate.N, E, Tn, L.gate.planes != nullptr, mmq_ws_, false, true) &&
+                                mmq_ksplit_preferred(L.up.type, (int)L.up.N, E, Tn, L.up.planes != nullptr, mmq_ws_, false, true) && !fuse_ffn);
             if (gq && uq && L.gate.type == L.up.type && !ffn_mmq) {
                 MMVQSeg segs[2] = {make_seg(L.gate, ffn_, FF, nullptr, nullptr), make_seg(L.up, ffn_u_, FF, nullptr, nullptr)};
                 HIP_TRY(mmvq_tokens(segs, 2, E, Tn, EPI_SWIGLU, aq_e_, stream_, fz));
@@ -1997,7 +1998,7 @@ hipError_t Context::run_output(int n_out, int out_base) {
     } else {
         // a tick's rows: the head's launch stores them to the host and finds their arg-max (mmq_few_head_kernel)
         if (oq && pending_fuse_.mode == 0 && mmq_few_head_takes(model->output.type, E, n_out, aq_e_) &&
-            mmq_ksplit_preferred(model->output.type, V, E, n_out, model->output.planes != nullptr, mmq_ws_, false)) {
+            (mmq_few_pair(model->output.type, E, n_out, aq_e_) || mmq_ksplit_preferred(model->output.type, V, E, n_out, model->output.planes != nullptr, mmq_ws_, false))) {
             logits_on_host_ = zc_env && cp.logits_to_host && h_logits_ != nullptr;
             const MMQSeg sg{model->output.data, model->output.row_bytes, V, model->output.type, lg, V, nullptr, 0};
             HIP_TRY(launch_mmq_few_head(sg, E, n_out, aq_e_, logits_on_host_ ? h_logits_ + (size_t)out_base * V : nullptr, head_scratch_, h_argmax_ + out_base, stream_));

@@ -89,3 +89,33 @@ def test_gate_up_pair(be, t, K, N, T):  # noqa: F811
                 be.mul_mat_batch([t, t], Ws, [N, N], K, x, swiglu=True)
     finally:
         be.set_option("mmq_few", -1)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("K,N", [(1280, 8210), (2048, 4100), (2304, 17), (4096, 40), (11008, 4112), (1024, 50)])
+def test_two_tokens(be, t, K, N):  # noqa: F811
+    """Against the oracle as in test_few_tokens; from 1280 columns on the bits of the same tokens in a batch of three, below the mat-vec's."""
+    rng = np.random.default_rng(K + N + t)
+    (W,), x = inputs(rng, [t], [N], K, 3)
+    y, ref = be.mul_mat(t, W, N, K, x[:2]), oq.mul_mat(t, W, N, K, x[:2])
+    assert np.abs(y - ref).max() <= 2e-5 * np.abs(ref).max() + 1e-6
+    if K >= 1280:
+        assert np.array_equal(y, be.mul_mat(t, W, N, K, x)[:2])
+
+
+@pytest.mark.parametrize("ftype", ["q4_k_m", "q5_k_m"])
+@pytest.mark.parametrize("kv", [1, 8])
+def test_two_tokens_through_a_model(pkg, tmp_path, ftype, kv):
+    """Q | K | V, attn_output, gate | up, ffn_down and the head of two tokens: the bits of the same tokens in a batch of three (the attention is columns either way, whose sums are a token's
+    own)."""
+    path = str(tmp_path / "m.gguf")
+    pkg.gguf_synth.write_synthetic_llama(path, "tiny-e2048", ftype, seed=6, with_vocab=False)
+    m = pkg.Model(path)
+    toks, out = np.random.default_rng(kv).integers(3, m.n_vocab, 3), []
+    for n in (2, 3):
+        c = pkg.Context(m, n_ctx=256, n_batch=64, n_ubatch=64, type_k=kv, type_v=kv)
+        assert c.decode(toks[:n], np.arange(n), 0, np.ones(n, np.int8)) == 0
+        out.append([np.array(c.logits(i)) for i in range(2)] + [np.array([c.argmax(i) for i in range(2)])])
+        c.close()
+    m.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
