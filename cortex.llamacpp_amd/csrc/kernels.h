@@ -181,7 +181,7 @@ bool mmq_ksplit_applicable(int type, int K, int T);
 bool mmq_ksplit_preferred(int type, int n_rows, int K, int T, bool has_planes, MMQWorkspace wsp, bool sum_free, bool pair = false);
 hipError_t launch_mmq_ksplit_multi(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, const int8_t *bh, const int8_t *bl,
                                    bool swiglu, hipStream_t st);
-// mmq_few.hip: 3 .. 64 tokens of the same, bit for bit, and two where mmq_few_pair; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
+// mmq_few.hip: 3 .. 64 tokens of the same, bit for bit, and two where mmq_few_pair says so; launch_mmq_ksplit_multi goes there where mmq_few_takes says so, and wants no block-sum planes then
 bool mmq_few_pair(int type, int K, int T, const ActQuant &q);
 bool mmq_few_takes(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu);
 hipError_t launch_mmq_few(const MMQSeg *segs, int n_seg, int K, int T, const ActQuant &q, bool swiglu, hipStream_t st);

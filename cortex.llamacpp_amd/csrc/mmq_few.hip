@@ -1,4 +1,4 @@
-// mmq_few.hip — the K-split contraction of 3 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
+// mmq_few.hip — the K-split contraction of 2 .. 64 tokens  Y[t][r] = dot(W[r,:], act_q8K[t,:])  (continuous-batching ticks, the short turn of a conversation):
 // K-quant weights in their GGUF form, Q8_K activations, int8 matrix cores, the integer of ggml_vec_dot_q{4,5,6}_K_q8_K per (row, token, super-block).
 //
 // What bounds it: the weights, read once from HBM (0.56 .. 0.82 B each), and beside them the vector instructions per unit, ~200 for Q4_K and 280 for Q6_K at 48 tokens and their waits (two
