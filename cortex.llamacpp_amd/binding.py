@@ -84,6 +84,7 @@ SYMBOLS = {
     "mi355_debug_engine_steps": (C.c_int64, [_vp]),
     "mi355_debug_fused_skipped_steps": (C.c_int64, [_vp]),
     "mi355_debug_qkv_attn_launches": (C.c_int64, [_vp]),
+    "mi355_debug_batch_route": (_i32, [_vp, C.POINTER(C.c_int32)]),
     "mi355_debug_qkv_attn_plan": (C.c_int64, [C.c_int32] * 10 + [C.POINTER(C.c_int32)]),
     "mi355_debug_batch_plan": (_i32, [_i32] * 6),
     "mi355_debug_q80_plan": (_i32, [_i32] * 3),
@@ -682,6 +683,11 @@ class Context:
 
     def qkv_attn_launches(self) -> int:
         return int(self.lib.mi355_debug_qkv_attn_launches(self.h))
+
+    def batch_route(self):
+        """What the last micro-batch took (1: chunk lists, 2: columns) and the words of chunk lists that it uploaded (diagnosis)."""
+        words = C.c_int32(0)
+        return int(self.lib.mi355_debug_batch_route(self.h, C.byref(words))), int(words.value)
 
     def engine_steps(self) -> int:
         """Single-token steps that ran through the layer engine (one persistent launch per layer; diagnosis)."""

@@ -262,6 +262,10 @@ int64_t mi355_debug_mega_steps(const mi355_context *ctx) { return ctx->c->mega_s
 int64_t mi355_debug_engine_steps(const mi355_context *ctx) { return ctx->c->engine_steps; }
 int64_t mi355_debug_fused_skipped_steps(const mi355_context *ctx) { return ctx->c->fused_skipped_steps; }
 int64_t mi355_debug_qkv_attn_launches(const mi355_context *ctx) { return ctx->c->qkv_attn_launches; }
+int32_t mi355_debug_batch_route(const mi355_context *ctx, int32_t *list_words) {
+    if (list_words) *list_words = ctx->c->list_words;
+    return ctx->c->batch_route;
+}
 int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int32_t n_tokens, int32_t pair, int32_t sum_free) {
     MMQWorkspace wsp;
     wsp.bytes = (size_t)num_cu() * 128 * 256 * sizeof(float);

@@ -1474,7 +1474,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         ma.out_q = &aq_o_; ma.out_q8k = !act_is_q80(wo0.type); ma.out_q80 = false;
         ma.splits = flash_attn_decode_splits(n_kv_max);
         if (chunk_lmax_ > 0) {
-            ma.tok_chunks = d_chunks_; ma.tok_nchunks = d_chunks_ + (size_t)64 * chunk_stride_; ma.chunk_stride = chunk_stride_;
+            ma.tok_chunks = d_chunks_ + 64; ma.tok_nchunks = d_chunks_; ma.chunk_stride = chunk_stride_;
             ma.splits = std::max(chunk_cap_, chunk_lmax_);
         }
         mega = flash_attn_decode_fused_applicable(ma, ra);      // (more than 64 chunks: the per-launch path merges them)
@@ -1525,12 +1525,12 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         const bool v16 = fa_v_acc_f16_enabled() && cp.type_k == T_F16 && cp.type_v == T_F16;
         // a batch of one sequence: (token, head) pairs as columns of one product against its keys (attn_cols.hip)
         const bool cols = attn_cols_;
-        if (cols) { aa.chunks = d_chunks_; aa.n_chunks = chunk_lmax_; }
+        if (cols) { aa.chunks = d_chunks_ + 64; aa.n_chunks = chunk_lmax_; }
         const bool decode_attn = !v16 && !cols && flash_attn_decode_applicable(aa, ra);
         if (decode_attn) {
             aa.splits = flash_attn_decode_splits(n_kv_max);
             if (chunk_lmax_ > 0) {                             // per-token chunk lists (decode_ubatch): batched steps, or regions in use
-                aa.tok_chunks = d_chunks_; aa.tok_nchunks = d_chunks_ + (size_t)64 * chunk_stride_; aa.chunk_stride = chunk_stride_;
+                aa.tok_chunks = d_chunks_ + 64; aa.tok_nchunks = d_chunks_; aa.chunk_stride = chunk_stride_;
                 aa.splits = std::max(chunk_cap_, chunk_lmax_);
             }
             fused_step = attn_mode() > 0 && flash_attn_decode_fused_applicable(aa, ra);
@@ -2074,6 +2074,7 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
     // continuous-batching steps (a few tokens, usually one per sequence): each token scans only the 64-cell chunks that
     // hold cells of its own sequence instead of the whole cache
     chunk_lmax_ = 0;
+    batch_route = list_words = 0;
     batch_distinct_ = n >= 2 && n <= 64;                       // every token in exactly one sequence, no two in the same one (a continuous-batching step)
     {
         uint64_t seen = 0;
@@ -2103,16 +2104,15 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         const int nch = (n_kv_ + 63) / 64;
         std::vector<uint64_t> seq_of_chunk((size_t)nch, 0ull);
         for (int ch = 0; ch < nch; ch++) seq_of_chunk[(size_t)ch] = cell_sums_.at(cells_, ch).seqs;
-        int32_t *cnt = h_chunks_ + (size_t)64 * chunk_stride_;
         for (int t = 0; t < (lists_usable ? n : 1); t++) {
-            int32_t *lst = h_chunks_ + (size_t)t * chunk_stride_;
+            int32_t *lst = h_chunks_ + 64 + (size_t)t * chunk_stride_;
             int c = 0;
             const uint64_t bit = 1ull << (seq[t] & 63);
             for (int ch = 0; ch < nch; ch++) if (seq_of_chunk[(size_t)ch] & bit) lst[c++] = ch;
-            cnt[t] = c;
+            h_chunks_[t] = c;
             chunk_lmax_ = std::max(chunk_lmax_, c);
             if (attn_cols_) {                                  // (by the chunks that hold its cells; which those are, and with them the order of the sums, follows the cells it was dealt)
-                aa.chunks = d_chunks_; aa.n_chunks = c;
+                aa.chunks = d_chunks_ + 64; aa.n_chunks = c;
                 // (without lists the general attention is what it would be beside; heads of 64 within one chunk of cells keep to the order of its sums, and a greedy answer's near ties to their side)
                 attn_cols_ = c > 0 && flash_attn_cols_takes(aa, lists_usable || (c == 1 && aa.D == 64));
                 if (attn_cols_) break;
@@ -2121,11 +2121,16 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
         if (chunk_lmax_ < 1) chunk_lmax_ = 1;
         if (one_fused) {
             aa.splits = std::min(chunk_stride_, (chunk_lmax_ + 3) & ~3);
-            lists_usable = lists_usable && flash_attn_decode_fused_applicable(aa, rope_args(*model, false));
+            // (all the chunks there are: a list says no more than their number)
+            lists_usable = lists_usable && h_chunks_[0] < nch && flash_attn_decode_fused_applicable(aa, rope_args(*model, false));
         }
-        const size_t words = attn_cols_ ? (size_t)chunk_lmax_ : (size_t)64 * (chunk_stride_ + 1);
         if (!attn_cols_ && !lists_usable) chunk_lmax_ = 0;     // (a long batch for the prompt kernel: no lists)
         else {
+            // the counts, and the lists of this batch's tokens as far as they reach: a single step's some hundred bytes, not the 64 lists of a longer batch
+            const int t = attn_cols_ ? 0 : n - 1;
+            const size_t words = 64 + (size_t)t * chunk_stride_ + h_chunks_[t];
+            batch_route = attn_cols_ ? ROUTE_COLS : ROUTE_LISTS;
+            list_words = (int)words;
             stage_pending_ = true;
             if (hipMemcpyAsync(d_chunks_, h_chunks_, words * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) { last_error = "chunk list upload failed"; return -1; }
         }

@@ -115,10 +115,12 @@ void set_rope_fast(bool on);         // tests: 0 = prompt batches rotate q / sto
 void set_decode_engine(int on);  // 1 / 0: the layer engine (decode_engine.hip) for single-token steps of contexts created afterwards; -1: environment MI355_ENGINE / default (off)
 void set_decode_mega(bool on);   // tests: compare the whole-step kernel with the per-launch path (read when a context first decodes one token)
 
+enum { ROUTE_LISTS = 1, ROUTE_COLS = 2 };   // (diagnosis: mi355_debug_batch_route)
 class Context {
   public:
     int64_t engine_steps = 0;          // single-token steps issued through the layer engine (graph replays included)
     int64_t qkv_attn_launches = 0;     // launches that ran a layer's Q | K | V inside its attention + attn_output launch (attn_out.hip QF)
+    int batch_route = 0, list_words = 0;      // the last micro-batch's: ROUTE_*, words of chunk lists uploaded
     int64_t fused_skipped_steps = 0;   // single-token steps that took the wait-free launches because another context of the device held the cross-workgroup-wait kernel
     int64_t mega_steps = 0;            // single-token steps issued as one whole-step launch (graph replays included)
     Context(Model *m, const ContextParams &p);
@@ -309,7 +311,7 @@ class Context {
     float *embd_out_ = nullptr;                      // an encoder's batch whose tokens are all flagged: where its last norm stores their rows, too (h_embd_)
     bool embd_on_host_ = false;                      // ... and did
     // batched single-token steps: per-token lists of the 64-cell chunks that hold cells of the token's sequence
-    int32_t *h_chunks_ = nullptr, *d_chunks_ = nullptr;     // [64][chunk_stride_] lists, then [64] counts
+    int32_t *h_chunks_ = nullptr, *d_chunks_ = nullptr;     // [64] counts, then [64][chunk_stride_] lists
     int chunk_stride_ = 0, chunk_lmax_ = 0, chunk_cap_ = 0;   // cap = grid size used for the lists (>= lmax; rounded up for graph reuse)                 // lmax = longest list of the current batch (0 = lists not in use)
     // whole-step kernel (decode_mega.hip): per-layer descriptors in device memory, barrier words, pinned time-out flag
     MegaLayer *d_mega_layers_ = nullptr;

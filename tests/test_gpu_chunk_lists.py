@@ -37,3 +37,27 @@ def test_conversations_against_one_alone(be, pkg, tmp_models, cfg, kv, n_ctx):  
             assert rel_err(rows[s][i], c.logits()) <= FLIP_TOL, (s, i)
         c.close()
     m.close()
+
+
+@pytest.mark.parametrize("cfg,kv", [("tiny-tl-2l", "f16"), ("tiny-qwen2", "q8_0")])
+def test_a_single_step_uploads_its_own_list(be, pkg, tmp_models, cfg, kv):  # noqa: F811
+    """A lone token among the cells of others walks a list; the counts and that list are uploaded, no others.  Where its sequence holds every chunk there is no list to upload: the launches, and
+    the bits, of a context of one sequence."""
+    m = pkg.Model(make(pkg, tmp_models, cfg, "q4_k_m"))
+    toks = np.random.default_rng(3).integers(3, m.n_vocab, 260)
+    rows = []
+    for n_seq in (1, 4):
+        c = pkg.Context(m, n_ctx=1024, n_seq_max=n_seq, type_k=KV[kv], type_v=KV[kv])
+        assert c.decode(toks[:130], np.arange(130)) == 0
+        assert c.decode([int(toks[130])], [130]) == 0
+        assert c.batch_route() == (0, 0)
+        rows.append(c.logits().copy())
+        if n_seq > 1:
+            assert c.decode(toks[:70], np.arange(70), [2] * 70) == 0
+            assert c.decode([int(toks[70])], [70], [2]) == 0
+            assert c.batch_route() == (1, 64 + 2)
+            assert c.decode([int(toks[131])], [131], [0]) == 0
+            assert c.batch_route() == (1, 64 + 3)
+        c.close()
+    assert np.array_equal(*rows)
+    m.close()
