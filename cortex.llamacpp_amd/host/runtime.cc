@@ -2113,8 +2113,8 @@ int Context::decode_ubatch(int n, const int32_t *tokens, const int32_t *pos, con
             chunk_lmax_ = std::max(chunk_lmax_, c);
             if (attn_cols_) {                                  // (by the chunks that hold its cells; which those are, and with them the order of the sums, follows the cells it was dealt)
                 aa.chunks = d_chunks_ + 64; aa.n_chunks = c;
-                // (without lists the general attention is what it would be beside; heads of 64 within one chunk of cells keep to the order of its sums, and a greedy answer's near ties to their side)
-                attn_cols_ = c > 0 && flash_attn_cols_takes(aa, lists_usable || (c == 1 && aa.D == 64));
+                // (without lists the general attention is what it would be beside)
+                attn_cols_ = c > 0 && flash_attn_cols_takes(aa, lists_usable);
                 if (attn_cols_) break;
             }
         }

@@ -88,6 +88,32 @@ def test_weights_and_values_as_in_f32(be, tkv, H, G, D, shares, what):  # noqa: 
         oq.set_fa_v_acc_f32(0)
 
 
+@pytest.mark.parametrize("tkv", [Q8_0, F16])
+@pytest.mark.parametrize("H,G", [(32, 4), (32, 8), (12, 12)])
+@pytest.mark.parametrize("T", [2, 5, 31])
+def test_within_one_chunk_against_64_bits(be, tkv, H, G, T):  # noqa: F811
+    """Heads of 64 over at most 64 cells: the columns and the general attention, either of which a short batch can come to, are as far from 64 bits.  A weight is a score's exp, whose error is that of
+    a sum of 64 products of f32 (2^-24 of it each, in quadrature 8 * 6e-8 of a term, the scores near 1) and an output another sum of up to 64: 5e-7 of the output's norm."""
+    D, rng = 64, np.random.default_rng(H * 10 + G + T)
+    n = int(rng.integers(T, 65))
+    kc, vc = (np.stack([oq.quantize(tkv, r) for r in rng.standard_normal((n, G * D)).astype(np.float32)]) for _ in range(2))
+    k, v = (np.stack([oq.dequantize(tkv, r, G * D) for r in rows]).astype(np.float64).reshape(n, G, D) for rows in (kc, vc))
+    q = (1.5 * rng.standard_normal((T, H, D))).astype(np.float32)
+    qq = np.stack([oq.dequantize(tkv, oq.quantize(tkv, r.reshape(-1)), H * D) for r in q]).astype(np.float64).reshape(T, H, D)
+    pos = np.arange(n - T, n, dtype=np.int32)
+    s = np.einsum("thd,nhd->thn", qq, np.repeat(k, H // G, 1)) / 8.0
+    s[np.broadcast_to(np.arange(n)[None, None, :] > pos[:, None, None], s.shape)] = -np.inf
+    w = np.exp(s - s.max(-1, keepdims=True))
+    ref = np.einsum("thn,nhd->thd", w / w.sum(-1, keepdims=True), np.repeat(v, H // G, 1))
+    try:
+        for form in (0, 1):
+            be.set_option("attn_cols", form)
+            out = be.flash_attn(q, H, G, D, tkv, kc, tkv, vc, np.arange(n, dtype=np.int32), pos, 1 / 8)
+            assert np.linalg.norm(out - ref) <= 5e-7 * np.linalg.norm(ref), form
+    finally:
+        be.set_option("attn_cols", 0)
+
+
 @pytest.mark.parametrize("kv", [1, 8])
 @pytest.mark.parametrize("past,n", [(0, 2), (70, 21), (900, 5), (300, 150)])
 def test_a_turn_among_other_conversations(pkg, tmp_path, kv, past, n):
@@ -150,6 +176,8 @@ def test_few_tokens_as_steps(pkg, tmp_path, model, past, n, kv):
             assert c.decode(talk[:past // 2], np.arange(past // 2), 0) == 0 and c.decode(talk[past // 2:past], np.arange(past // 2, past), 0) == 0
         for i in range(past, past + n, each):
             assert c.decode(talk[i:i + each], np.arange(i, i + each), 0) == 0
+        if model in ("tinyllama-1.1b", "tiny-qwen2") and each > 1:                                  # (no one-token kernel beside it: by the work, not by the number of cells)
+            assert c.batch_route()[0] == 2
         out.append(np.array(c.logits(-1)))
         c.close()
     m.close()
