@@ -685,7 +685,7 @@ class Context:
         return int(self.lib.mi355_debug_qkv_attn_launches(self.h))
 
     def batch_route(self):
-        """What the last micro-batch took (1: chunk lists, 2: columns) and the words of chunk lists that it uploaded (diagnosis)."""
+        """What the last micro-batch took (1: chunk lists, 2: columns, 4: the last layer on the flagged rows alone) and the words of chunk lists that it uploaded (diagnosis)."""
         words = C.c_int32(0)
         return int(self.lib.mi355_debug_batch_route(self.h, C.byref(words))), int(words.value)
 

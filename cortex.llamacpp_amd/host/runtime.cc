@@ -1593,8 +1593,10 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
             HIP_TRY(launch_add_qkv_bias(q_, k_, v_, L.bq.valid() ? (const float *)L.bq.data : nullptr, L.bk.valid() ? (const float *)L.bk.data : nullptr,
                                         L.bv.valid() ? (const float *)L.bv.data : nullptr, H * D, G * D, T, stream_));
         if (!qkv_in_attn) prof_mark("qkv");
-        const bool cut_here = cut && il + 1 == hp.n_layer && (!decode_attn || fast_store);
-        if (cut_here) { Tn = n_out_rows_; xl = x_ + (size_t)std::max(out_first_, 0) * E; }
+        // the one-token kernel, with a store of K and V in front of it or inside; else columns, or the general attention behind its own
+        const bool own_attn = decode_attn && (fast_store || fused_step || (batch_distinct_ && store_fuse_enabled()));
+        const bool cut_here = cut && il + 1 == hp.n_layer && (!own_attn || fast_store);      // (not where only the attention's launch stores the rows' K and V)
+        if (cut_here) { batch_route |= ROUTE_LAST_ROWS; Tn = n_out_rows_; xl = x_ + (size_t)std::max(out_first_, 0) * E; }
         const auto rows_of = [&](AttnArgs r) {                 // the flagged rows' part of the batch's attention; its results and its quantised rows begin at row 0
             const size_t f = (size_t)out_first_;
             r.q += f * (size_t)H * D; r.T = Tn; r.tok_pos += f; r.tok_seq += f;
@@ -1604,7 +1606,7 @@ hipError_t Context::run_layers(int T, int n_kv_cap) {
         };
         if (qkv_in_attn) {
             // the whole block ran in the launch above
-        } else if (decode_attn && (fast_store || fused_step || (batch_distinct_ && store_fuse_enabled()))) {
+        } else if (own_attn) {
             if (cut_here) {
                 HIP_TRY(launch_kv_store_fast(k_, v_, T, G, D, rope_cs_, ra, d_cell_, kv_[(size_t)il], cp.type_k, cp.type_v, (int)cp.n_ctx, stream_));
                 prof_mark("rope_kv");

@@ -115,7 +115,7 @@ void set_rope_fast(bool on);         // tests: 0 = prompt batches rotate q / sto
 void set_decode_engine(int on);  // 1 / 0: the layer engine (decode_engine.hip) for single-token steps of contexts created afterwards; -1: environment MI355_ENGINE / default (off)
 void set_decode_mega(bool on);   // tests: compare the whole-step kernel with the per-launch path (read when a context first decodes one token)
 
-enum { ROUTE_LISTS = 1, ROUTE_COLS = 2 };   // (diagnosis: mi355_debug_batch_route)
+enum { ROUTE_LISTS = 1, ROUTE_COLS = 2, ROUTE_LAST_ROWS = 4 };   // (diagnosis: mi355_debug_batch_route)
 class Context {
   public:
     int64_t engine_steps = 0;          // single-token steps issued through the layer engine (graph replays included)

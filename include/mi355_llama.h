@@ -171,7 +171,8 @@ MI355_API int64_t mi355_debug_fused_skipped_steps(const mi355_context *ctx);
    per layer for the whole attention block of a single-token step; "qkv_attn_fused" 0 / MI355_QKV_ATTN_FUSED=0 keeps Q | K | V a launch of its own).  Counts
    launches issued eagerly or while a graph was captured, not graph replays. */
 MI355_API int64_t mi355_debug_qkv_attn_launches(const mi355_context *ctx);
-/* diagnosis: what the context's last micro-batch took.  1: each token's attention walks a list of its own sequence's 64-cell chunks, 2: attention in columns (csrc/attn_cols.hip), added up.
+/* diagnosis: what the context's last micro-batch took.  1: each token's attention walks a list of its own sequence's 64-cell chunks, 2: attention in columns (csrc/attn_cols.hip), 4: its last layer
+   worked on the flagged rows alone behind K and V, added up.
    *list_words (nullable): the 32-bit words of chunk lists that it uploaded */
 MI355_API int32_t mi355_debug_batch_route(const mi355_context *ctx, int32_t *list_words);
 /* host logic only (no GPU needed): would a single-token step of a layer with these tensor types (MI355_TYPE_*) and this geometry run its Q | K | V inside the attention
