@@ -271,11 +271,11 @@ int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int
     wsp.bytes = (size_t)num_cu() * 128 * 256 * sizeof(float);
     wsp.p = reinterpret_cast<float *>(wsp.bytes);               // (looked at for being there)
     if (n_rows < 1 || n_cols < 256 || n_cols % 256 || n_tokens < 1) return 0;
-    if (mmq_ksplit_preferred(type, n_rows, n_cols, n_tokens, mmq_planes_bytes(type, n_rows, n_cols) != 0, wsp, sum_free != 0, pair != 0)) {
+    ActQuant q;
+    q.qf = reinterpret_cast<uint8_t *>(wsp.p);
+    if (mmq_few_pair(type, n_cols, n_tokens, q) || mmq_ksplit_preferred(type, n_rows, n_cols, n_tokens, mmq_planes_bytes(type, n_rows, n_cols) != 0, wsp, sum_free != 0, pair != 0)) {
         MMQSeg sg[2] = {};
         for (MMQSeg &s : sg) { s.n_rows = n_rows; s.type = type; }
-        ActQuant q;
-        q.qf = reinterpret_cast<uint8_t *>(wsp.p);
         return mmq_few_takes(sg, pair ? 2 : 1, n_cols, n_tokens, q, pair != 0) ? 1 : 2;
     }
     return mmq_applicable(type, n_cols, n_tokens) ? 3 : 0;

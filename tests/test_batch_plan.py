@@ -29,8 +29,11 @@ def test_from_129_tokens_by_time(plan, t, n):
 
 
 def test_around_the_ranges_ends(plan):
-    """One and two rows are mat-vecs, whose sums a single step's are; from 257 tokens on the K-split kernel is out, whatever the shape."""
-    assert [plan(Q4_K, 2048, 2048, n, 0, 0) for n in (1, 2, 3, 128, 129, 256, 257)] == [MATVEC, MATVEC, FEW, KSPLIT, KSPLIT, KSPLIT, PLANES]
+    """One row is a mat-vec, and two of fewer than 1280 columns; from 257 tokens on the K-split kernel is out, whatever the shape."""
+    assert [plan(Q4_K, 2048, 2048, n, 0, 0) for n in (1, 2, 3, 128, 129, 256, 257)] == [MATVEC, FEW, FEW, KSPLIT, KSPLIT, KSPLIT, PLANES]
+    for t in (Q4_K, Q5_K, Q6_K):
+        assert [plan(t, r, c, 2, p, 0) for r, c, p in [(4096, 1280, 0), (128256, 4096, 0), (14336, 4096, 1), (4096, 1024, 0), (2816, 1024, 1)]] == [FEW, FEW, FEW, MATVEC, MATVEC]
+    assert plan(10, 4096, 4096, 2, 0, 0) == MATVEC            # (Q2_K has no contraction of few tokens)
     assert [plan(Q4_K, 8192, 4096, n, 0, 0) for n in (65, 128, 129)] == [PLANES] * 3
     assert plan(Q4_K, 2048, 2000, 64, 0, 0) == MATVEC
 
