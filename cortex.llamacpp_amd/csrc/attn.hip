@@ -802,15 +802,16 @@ bool flash_attn_decode_fused_applicable(const AttnArgs &a, const RopeArgs &ra) {
 // diagnosis: MI355_ATTN_PROBE=1 makes the fused decode attention stamp its phases (DecodeFuse::probe); the stamps of the
 // LAST launch are summarised on stderr by attn_probe_report() (called when a context is destroyed)
 static unsigned long long *g_attn_probe = nullptr;
+constexpr int ATT_PROBE_WORDS = 4096 + 8 * 256;   // start and end of 2048 items; eight words a kv head
 static int g_attn_probe_G = 0, g_attn_probe_splits = 0;
 static unsigned long long *attn_probe_buffer() {
     static const bool on = getenv("MI355_ATTN_PROBE") && getenv("MI355_ATTN_PROBE")[0] == '1';
-    if (on && !g_attn_probe && hipMalloc((void **)&g_attn_probe, (4096 + 64) * 8) == hipSuccess) (void)hipMemset(g_attn_probe, 0, (4096 + 64) * 8);
+    if (on && !g_attn_probe && hipMalloc((void **)&g_attn_probe, ATT_PROBE_WORDS * 8) == hipSuccess) (void)hipMemset(g_attn_probe, 0, ATT_PROBE_WORDS * 8);
     return g_attn_probe;
 }
 void attn_probe_report() {
     if (!g_attn_probe || g_attn_probe_G <= 0) return;
-    std::vector<unsigned long long> t(4096 + 64);
+    std::vector<unsigned long long> t(ATT_PROBE_WORDS);
     (void)hipDeviceSynchronize();
     if (hipMemcpy(t.data(), g_attn_probe, t.size() * 8, hipMemcpyDeviceToHost) != hipSuccess) return;
     const int n = std::min(2048, g_attn_probe_G * g_attn_probe_splits);
@@ -843,7 +844,7 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
     fz.neox = ra.neox;
     if (a.out_q) fz.q = *a.out_q;
     fz.want_q8k = (int)(a.out_q && a.out_q8k); fz.want_q80 = (int)(a.out_q && a.out_q80);
-    fz.probe = attn_probe_buffer();
+    fz.probe = a.G <= 256 && a.G * a.splits <= 2048 ? attn_probe_buffer() : nullptr;
     // The chunk partials are published with write-through stores and a relaxed ticket instead of an agent-scope release /
     // acquire per workgroup: that pair is a write-back + invalidate of the whole L2, and hundreds of workgroups issuing it at
     // once serialise (tools/bench_gridbar.hip: 25 us for 512).  Measured on the 8B step: 424 -> 448 tok/s at 4000 cells.
@@ -851,12 +852,14 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
     static const bool coh = !(getenv("MI355_ATTN_COH") && getenv("MI355_ATTN_COH")[0] == '0');
     // (what a workgroup of 1024 threads holds: a step's first 256 cells)
     if (counters && a.splits <= WHOLE_NS && a.D == WHOLE_D && (R == WHOLE_R || R == 2 * WHOLE_R)) {
-#define FADW(TK, TV) hipLaunchKernelGGL((flash_attn_decode_whole_kernel<TK, TV>), dim3(a.H / WHOLE_R), dim3(256 * WHOLE_NS), 0, st, a, cs_table, ra.n_rot, fz)
+#define FADP(TK, TV, P) hipLaunchKernelGGL((flash_attn_decode_whole_kernel<TK, TV, P>), dim3(a.H / WHOLE_R), dim3(256 * WHOLE_NS), 0, st, a, cs_table, ra.n_rot, fz)
+#define FADW(TK, TV) do { if (fz.probe) FADP(TK, TV, true); else FADP(TK, TV, false); } while (0)
         if (a.type_k == T_F16 && a.type_v == T_F16) FADW(T_F16, T_F16);
         else if (a.type_k == T_Q8_0 && a.type_v == T_Q8_0) FADW(T_Q8_0, T_Q8_0);
         else if (a.type_k == T_Q8_0) FADW(T_Q8_0, T_F16);
         else FADW(T_F16, T_Q8_0);
 #undef FADW
+#undef FADP
         return hipGetLastError();
     }
 #define FAD_D(RR, TK, TV, DD) do { if (coh && counters) hipLaunchKernelGGL((flash_attn_decode_kernel<RR, TK, TV, true, true, DD>), grid, dim3(256), 0, st, a, cs_table, ra.n_rot, fz); \

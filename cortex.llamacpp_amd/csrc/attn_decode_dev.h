@@ -439,8 +439,10 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
     if constexpr (NS > 1) {
         // every chunk is here: the merge below, of records in LDS
         static_assert(COH == false && D <= C && (R * D) % 256 == 0 && R <= 4 * NS && R * D <= 256 * NS, "a wave to a head, a thread to an output, whole blocks");
+        if (fz.probe && tid == 0) fz.probe[2 * (sp * a.G + g) + 1] = wall_clock64();
         __syncthreads();
         const int all = tid_now(), wv = __builtin_amdgcn_readfirstlane(all >> 6);
+        if (fz.probe && all == 0) fz.probe[4096 + 8 * g] = wall_clock64();
         float *const wgt = accs_[0], *const merged = qf_[0];
         if (wv < R) {
             const float m = lane < NS ? ml_[lane < NS ? lane : 0][2 * wv] : -INFINITY, l = lane < NS ? ml_[lane < NS ? lane : 0][2 * wv + 1] : 0.0f;
@@ -450,6 +452,7 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
             if (lane < NS) wgt[wv * 64 + lane] = w * (1.0f / den);
         }
         __syncthreads();
+        if (fz.probe && all == 0) fz.probe[4096 + 8 * g + 1] = wall_clock64();
         if (all < R * D) {
             const int r = all / D;
             float s = 0.0f;
@@ -459,7 +462,12 @@ __device__ __forceinline__ void flash_attn_decode_item(const AttnArgs &a, const 
             a.out[(size_t)qh * D + all] = s;
         }
         __syncthreads();
+        if (fz.probe && all == 0) fz.probe[4096 + 8 * g + 2] = wall_clock64();
         if (wv < (R * D) >> 8 && (fz.want_q8k || fz.want_q80)) decode_quant_block<COH>(fz, merged + wv * 256, ((qh * D) >> 8) + wv, lane);
+        if (fz.probe && wv == 0) {                            // (the block's wave)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (lane == 0) fz.probe[4096 + 8 * g + 3] = wall_clock64();
+        }
         return;
     }
     if (fz.counters == nullptr) return;               // store-fused only: the merge runs as its own launch (batched steps: in this launch it takes as long, ticks of 2 to 16 tokens 1 % slower to 1 % faster)
@@ -591,9 +599,11 @@ __global__ __launch_bounds__(256) void flash_attn_decode_kernel(const AttnArgs a
 // quantise, and four chunks of them are a CU's threads.  us a launch, 32 / 4 heads of 64, f16 cache, behind 20, 93 and 250 cells: 6.3, 6.7 and 7.1; with a workgroup a chunk and the ticket 8.7
 // (six layers' step 220 -> 203, 206 and 212)
 constexpr int WHOLE_NS = 4, WHOLE_R = 4, WHOLE_D = 64;
-template <int TK, int TV>
-__global__ __launch_bounds__(256 * WHOLE_NS) void flash_attn_decode_whole_kernel(const AttnArgs a, const float *cs_table, int n_rot, const DecodeFuse fz) {
+template <int TK, int TV, bool PROBE>
+__global__ __launch_bounds__(256 * WHOLE_NS) void flash_attn_decode_whole_kernel(const AttnArgs a, const float *cs_table, int n_rot, const DecodeFuse fz_) {
     decode_args_at_once();
+    DecodeFuse fz = fz_;
+    if (!PROBE) fz.probe = nullptr;                            // (looked at behind every phase it is 0.1 us of the 7.1 behind 250 cells)
     const int parts = a.H / a.G / WHOLE_R;
     flash_attn_decode_item<WHOLE_R, TK, TV, true, false, WHOLE_D, WHOLE_NS>(a, cs_table, n_rot, fz, blockIdx.x / parts, __builtin_amdgcn_readfirstlane(tid_now() >> 8), 0, blockIdx.x * WHOLE_R);
 }

@@ -1,4 +1,9 @@
 """A single token's attention over up to four chunks of 64 cells with heads of 64: all of a head's chunks in one workgroup."""
+import os
+import re
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -38,3 +43,31 @@ def test_steps_at_the_edges_of_chunks(be, pkg, tmp_models, cfg, tk, tv, n_seq): 
         c.close(); m.close(); oc.close(); om.close()
     finally:
         oq.set_fa_v_acc_f32(0)
+
+
+PROBED = """
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+from __graft_entry__ import load_pkg
+pkg = load_pkg()
+be = pkg.Backend()
+m = pkg.Model(sys.argv[1])
+c = pkg.Context(m, n_ctx=512)
+n = int(sys.argv[2])
+assert c.decode(np.arange(3, 3 + n), np.arange(n)) == 0 and c.decode([5], [n]) == 0
+c.close(); m.close()
+"""
+
+
+@pytest.mark.parametrize("n,items", [(100, 4 * 4), (300, 4 * 8)])           # one workgroup's four chunks of each of four kv heads; a workgroup a chunk of 512 cells
+def test_probe_reports_either_form(be, pkg, tmp_models, n, items):  # noqa: F811
+    """MI355_ATTN_PROBE=1: every item's start and end and the merges' phases, in order."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", PROBED % root, make(pkg, tmp_models, "tiny-tl-2l", "q4_k_m"), str(n)], capture_output=True, text=True, timeout=100, cwd=root,
+                       env=dict(os.environ, MI355_ATTN_PROBE="1"))
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = re.search(r"attn probe: (\d+) workgroups", r.stderr)
+    assert got and int(got.group(1)) == items, r.stderr[-2000:]
+    merges = re.findall(r"merge: ticket at (\S+) us, weights \+(\S+), sums \+(\S+), stores \+(\S+) -> done at (\S+) us", r.stderr)
+    assert len(merges) == 4 and all(0 <= float(x) < 1000 for row in merges for x in row), merges
