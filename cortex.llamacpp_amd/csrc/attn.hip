@@ -834,6 +834,8 @@ void attn_probe_report() {
     }
 }
 
+static bool g_attn_whole = true;
+void set_attn_whole(bool on) { g_attn_whole = on; }
 hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_table, RopeArgs ra, const float *knew, const float *vnew,
                                           const int32_t *tok_cell, unsigned *counters, hipStream_t st) {
     const int R = a.H / a.G;
@@ -851,7 +853,7 @@ hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_tab
     // MI355_ATTN_COH=0 restores the fenced form.
     static const bool coh = !(getenv("MI355_ATTN_COH") && getenv("MI355_ATTN_COH")[0] == '0');
     // (what a workgroup of 1024 threads holds: a step's first 256 cells)
-    if (counters && a.splits <= WHOLE_NS && a.D == WHOLE_D && (R == WHOLE_R || R == 2 * WHOLE_R)) {
+    if (g_attn_whole && counters && a.splits <= WHOLE_NS && a.D == WHOLE_D && (R == WHOLE_R || R == 2 * WHOLE_R)) {
 #define FADP(TK, TV, P) hipLaunchKernelGGL((flash_attn_decode_whole_kernel<TK, TV, P>), dim3(a.H / WHOLE_R), dim3(256 * WHOLE_NS), 0, st, a, cs_table, ra.n_rot, fz)
 #define FADW(TK, TV) do { if (fz.probe) FADP(TK, TV, true); else FADP(TK, TV, false); } while (0)
         if (a.type_k == T_F16 && a.type_v == T_F16) FADW(T_F16, T_F16);

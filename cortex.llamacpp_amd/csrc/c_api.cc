@@ -955,6 +955,7 @@ int mi355_debug_set_option(const char *name, int32_t value) {
     if (!strcmp(name, "attn_seqs")) { g_op_attn_seqs = value < 1 || value > 32 ? 1 : value; return MI355_OK; }
     if (!strcmp(name, "attn_spare")) { g_op_attn_spare = value < 0 ? 0 : value; return MI355_OK; }
     if (!strcmp(name, "attn_cols")) { g_op_attn_cols = value < 0 || value > 64 ? 0 : value; return MI355_OK; }     // mi355_op_flash_attn: attn_cols.hip with so many shares of the keys
+    if (!strcmp(name, "attn_whole")) { set_attn_whole(value != 0); return MI355_OK; }
     if (!strcmp(name, "last_rows")) { set_last_rows(value != 0); return MI355_OK; }
     if (!strcmp(name, "late_sums")) { set_late_sums(value != 0); return MI355_OK; }
     if (!strcmp(name, "rope_fast")) { set_rope_fast(value != 0); return MI355_OK; }

@@ -692,6 +692,7 @@ hipError_t launch_flash_attn_decode(const AttnArgs &a, const float *cs_table, Ro
                                     const float *vnew = nullptr, const int32_t *tok_cell = nullptr);   // knew..: KV store inside (tokens of different sequences)
 // one launch per layer for a single-token step: KV store + attention + split merge + quantise (a.splits set by the caller)
 bool flash_attn_decode_fused_applicable(const AttnArgs &a, const RopeArgs &ra);
+void set_attn_whole(bool on);   // tests: 0 = a single token's attention over few cells of 64-wide heads with a workgroup a chunk, as over more (read when a step's launches are built)
 void attn_probe_report();   // MI355_ATTN_PROBE=1: phase timing of the last fused decode attention launch, on stderr
 hipError_t launch_flash_attn_decode_fused(const AttnArgs &a, const float *cs_table, RopeArgs ra, const float *knew, const float *vnew,
                                           const int32_t *tok_cell, unsigned *counters, hipStream_t st);

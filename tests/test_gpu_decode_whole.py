@@ -45,6 +45,33 @@ def test_steps_at_the_edges_of_chunks(be, pkg, tmp_models, cfg, tk, tv, n_seq): 
         oq.set_fa_v_acc_f32(0)
 
 
+@pytest.mark.parametrize("n_seq", [1, 3])
+@pytest.mark.parametrize("cfg,tk,tv", [("tiny-gqa4", "f16", "f16"), ("tiny-gqa4", "q8_0", "f16"), ("tiny-gqa4", "f16", "q8_0"), ("tiny-tl-2l", "f16", "f16"), ("tiny-tl-2l", "q8_0", "q8_0")])
+def test_bits_of_the_general_form(be, pkg, tmp_models, cfg, tk, tv, n_seq):  # noqa: F811
+    """The same arithmetic in the same order as a workgroup a chunk and their merge behind a ticket: a chunk's sums, the chunks' weights, and the outputs' sum chunk by chunk."""
+    m = pkg.Model(make(pkg, tmp_models, cfg, "q4_k_m"))
+    toks, out = np.random.default_rng(9).integers(3, m.n_vocab, 258), []
+    try:
+        for whole in (1, 0):
+            be.set_option("attn_whole", whole)
+            c = pkg.Context(m, n_ctx=1024, n_seq_max=n_seq, type_k=KV[tk], type_v=KV[tv])
+            sq, have, rows = n_seq - 1, 0, []
+            if sq:
+                assert c.decode(toks[:70], np.arange(70), [0] * 70) == 0
+            for n in (0, 1, 2, 31, 63, 64, 65, 127, 128, 130, 191, 192, 230, 254, 255):
+                if n > have:
+                    assert c.decode(toks[have:n], np.arange(have, n), [sq] * (n - have), np.zeros(n - have, np.int8)) == 0
+                assert c.decode([int(toks[n])], [n], [sq], [1]) == 0
+                rows.append(c.logits(0).copy())
+                have = n + 1
+            out.append(np.stack(rows))
+            c.close()
+    finally:
+        be.set_option("attn_whole", 1)
+    m.close()
+    assert np.array_equal(*out)
+
+
 PROBED = """
 import sys
 sys.path.insert(0, %r)
