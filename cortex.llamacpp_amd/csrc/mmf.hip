@@ -243,8 +243,8 @@ namespace {
 // The encoder's projections (T tokens of one text against f16 weights of a few hundred to a few thousand columns): a product is 19 MB of weights at the most and
 // some microseconds of anything, so what counts is one trip to memory, enough workgroups and no launches around it.  Measured on nomic-embed (768 / 3072 columns)
 // at 187 tokens, us: 768 x 768 30 with the 64 x 64 direct
-// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; here, launches back to back, Q | K | V 6.1, output 3.8, gate | up 9.5, down 7.1, and
-// Q | K | V and gate | up of 768 columns as mmf16_rows_kernel below has them 5.1 and 9.0:
+// kernel above (36 workgroups, one load in flight, 32 lines per request), gate and up 21 each, down about 60; here, in a pass, output 5.0 and down 8.1, Q | K | V 7.7 and gate | up 10.7, and
+// the latter two, of 768 columns, as mmf16_rows_kernel below has them 5.7 and 10.0:
 //   * 32 rows x 32 TT tokens per workgroup (144 workgroups for the output at 187 tokens); the NW waves share K, chunk by chunk of 64, and a wave's first PD chunks of
 //     both operands - all of them for 768 columns - are requested before the first matrix step;
 //   * a request is whole 128-byte lines of eight rows; the operands (16 bytes of 32 rows) are made through LDS of the wave's own, pieces of a row turned by its number.  Asked for as
@@ -417,9 +417,8 @@ __global__ __launch_bounds__(64 * NW, EPI == FEW_SWIGLU && NW == 4 && TT == 1 ? 
 // Two products of the same tokens (gate and up, or the halves of 64-wide heads) where K is at most ROWS_K columns and there are few workgroups: 32 rows of each x 32 tokens per workgroup, whose
 // activation rows are whole in LDS, staged once by all; of the eight waves four take the one product and four the other, a chunk of 64 columns in four each, all of a wave's weights
 // requested at once.  What bounds such a launch is a wave's own chain of instructions - one or two waves a SIMD, some thousand of them - and in the form above a wave stages both products and the
-// tokens for itself.  768 columns, us, this form / that one: Q | K | V at 40, 187, 300, 700, 1000 tokens 4.9 / 5.9, 5.1 / 5.9, 6.9 / 7.6, 11.4 / 12.1, 14.1 / 16.5, at 1800 24.5 / 23.4; gate | up at
-// 40, 187, 300, 400, 700 5.0 / 5.3, 9.1 / 9.3, 11.1 / 11.3, 13.4 / 13.2, 23.4 / 21.3.  Twelve waves, two chunks each: 5.2 and, with one workgroup a CU, 11.8 at 187.  With the LayerNorm in front of
-// it in the launch, every workgroup norming its rows: 7.9 and 15.1, a launch of the norm is 2.7.
+// tokens for itself (both forms' times: few_two).  Twelve waves, two chunks each: no faster and, with one workgroup a CU, gate | up of 187 tokens 11.8 instead of 9.1 us.  With the LayerNorm in front
+// of it in the launch, every workgroup norming its rows: 7.9 and 15.1 instead of 5.1 and 9.1, a launch of the norm is 2.7.  (These back to back, half a microsecond to one less than in a pass.)
 constexpr int ROWS_K = 768;
 template <int EPI>
 __global__ __launch_bounds__(512, 4) void mmf16_rows_kernel(const MMF16Few a) {
@@ -430,7 +429,7 @@ __global__ __launch_bounds__(512, 4) void mmf16_rows_kernel(const MMF16Few a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), p = wave & 1, ks = wave >> 1, m = lane & 31, kg = lane >> 5;
     const int n0 = blockIdx.x * ROWS, t0 = blockIdx.y * 32, nc = a.K >> 6, r8 = lane >> 3, c8 = lane & 7;
     uint8_t *const sx = smem, *const sw = smem + X_BYTES + wave * 4096;
-    // the tokens' rows, sixteen threads a row (past the end the last one's; a piece past K is the row's first, and not staged), then the wave's chunks of its product's rows
+    // the tokens' rows, sixteen threads a row (past the end the last one's; a piece past K is the thread's first, and not staged: K is 128 or more), then the wave's chunks of its product's rows
     const int row = tid >> 4, l16 = tid & 15;
     f16x8 v[KJ / 2];
     {
@@ -517,15 +516,18 @@ void few_go(const MMF16Few &a, hipStream_t st) {
 template <int NW, int EPI>
 void few_two(const MMF16Few &a, hipStream_t st) {
     const int rows = EPI == FEW_ROPE ? 64 : 32, wg = (a.N + rows - 1) / rows * ((a.T + 31) / 32);
-    // (Q | K | V at any number of tokens, 1800: 19.8 / 23.4; gate | up to nine workgroups a CU: 500 tokens 14.9 / 15.1, 700 20.7 / 21.7, 900 25.9 / 25.4)
-    if (a.K <= ROWS_K && a.N % 32 == 0 && (EPI == FEW_ROPE || wg <= 9 * num_cu())) {
+    // us in a pass of 768 columns, that form / the shared K, medians of two profiled runs of each in turn, at 40, 187, 300, 400, 500, 600, 700, 800, 900, 1000, 1400, 1800 and 2000 tokens:
+    //   Q | K | V   5.4 / 7.0, 5.7 / 7.7, 7.3 / 8.8, 7.6 / 9.3, 9.5 / 11.8, 10.1 / 14.1, 11.3 / 13.8, 11.8 / 14.3, 13.4 / 15.9, 14.1 / 18.6, 18.2 / 22.7, 21.8 / 25.7, 23.3 / 29.4
+    //   gate | up   6.0 / 6.1, 10.1 / 10.7, 12.3 / 12.7, 14.8 / 15.1, 17.0 / 17.0, 20.5 / 20.4, 22.5 / 23.4, 24.8 / 24.2, 27.1 / 27.4, 29.2 / 27.7, 39.2 / 37.4, 49.3 / 45.2, 54.1 / 49.1
+    // So Q | K | V at any number, gate | up to nine workgroups a CU (768 tokens of 3072 rows)
+    if (a.K >= 128 && a.K <= ROWS_K && a.N % 32 == 0 && (EPI == FEW_ROPE || wg <= 9 * num_cu())) {
         hipLaunchKernelGGL((mmf16_rows_kernel<EPI>), dim3((unsigned)(a.N / rows), (unsigned)((a.T + 31) / 32)), dim3(512), 0, st, a);
         return;
     }
     if (wg * (rows / 32) >= 1280) few_go<NW, EPI, 2, 2, false>(a, st);
     else few_go<NW, EPI, 1, EPI == FEW_SWIGLU && NW == 4 ? 2 : 3, false>(a, st);
 }
-// A plain product, us, K 768 of f32 rows / K 3072 of halves, both to 768 rows.  What counts is a wave's own chain again, so as many waves as K gives chunks where a CU has one workgroup: 187 tokens,
+// A plain product, us back to back, K 768 of f32 rows / K 3072 of halves, both to 768 rows.  What counts is a wave's own chain again, so as many waves as K gives chunks where a CU has one workgroup: 187 tokens,
 // twelve waves 3.8 / 7.1, four and eight 4.3 / 7.5.  Beyond, in rounds of a workgroup a CU: f32 rows on four waves (400 tokens 6.0, twelve 6.4; 1000 8.3, 10.2); halves on one, two or three token
 // tiles, whose rounds take about 7.1, 9.4 and 14.6: 400 tokens 12.5, 9.3, 12.6, 800 about 18.5, 18.4, 14.8, 1200 24.8, 19.2, 27.0, 2048 36.9, 29.5, 38.9; eight waves with one and, from 1280
 // workgroups on, two 13.2, 19.9, 26.6, 31.1.
