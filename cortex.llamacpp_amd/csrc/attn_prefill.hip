@@ -769,7 +769,7 @@ int flash_attn_prefill_splits(int T, int H, int G, int D, int n_kv_max) {
     if (s > n_chunks / (4 * kh)) s = n_chunks / (4 * kh);        // (~4 chunks per half and workgroup at least)
     if (s > 8) s = 8;
     if (env > 0) s = env;
-    while (s > 1 && (size_t)T * H * s * (D + 2) * sizeof(float) > ((size_t)512 << 20)) s >>= 1;
+    while (s > 1 && flash_attn_workspace_floats(T, H, D, s) * sizeof(float) > ((size_t)512 << 20)) s >>= 1;
     return s < 1 ? 1 : s;
 }
 

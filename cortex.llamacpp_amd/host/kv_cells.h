@@ -24,7 +24,6 @@ class CellChunks {
     };
     void reset(size_t n_cells) { sums_.assign((n_cells + 63) / 64, Sum()); stale_.assign(sums_.size(), 0); }
     void touch(int cell) { stale_[(size_t)cell >> 6] = 1; }
-    void touch_all() { std::fill(stale_.begin(), stale_.end(), (uint8_t)1); }
     const Sum &at(const std::vector<KVCell> &cells, int chunk) {
         Sum &s = sums_[(size_t)chunk];
         if (stale_[(size_t)chunk]) {

@@ -1349,7 +1349,6 @@ bool Context::engine_prepare() {
 // passes), attn_output (+ bias), residual, LayerNorm, SwiGLU feed-forward, residual, LayerNorm.  The output is the last layer's hidden state; there is no head.
 // K / V rows go through the context's cache like a prompt batch's (the whole sequence is one micro-batch: Context::decode checks that).
 hipError_t Context::run_layers_encoder(int T, int n_kv_cap) {
-    cur_T_ = T;
     const HParams &hp = model->hp;
     const int E = hp.n_embd, FF = hp.n_ff, H = hp.n_head, G = hp.n_head_kv, D = hp.head_dim;
     RopeArgs ra = rope_args(*model, true);
@@ -1454,7 +1453,6 @@ hipError_t Context::launch_setup(int T, bool mega) {
 
 hipError_t Context::run_layers(int T, int n_kv_cap) {
     if (model->hp.encoder) return run_layers_encoder(T, n_kv_cap);
-    cur_T_ = T;
     const HParams &hp = model->hp;
     const int E = hp.n_embd, FF = hp.n_ff, H = hp.n_head, G = hp.n_head_kv, D = hp.head_dim;
     RopeArgs ra = rope_args(*model, true);

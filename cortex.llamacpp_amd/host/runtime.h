@@ -237,8 +237,8 @@ class Context {
     void *dalloc(size_t bytes);
 
     hipStream_t stream_ = nullptr;
-    int cur_T_ = 0;                    // tokens of the micro-batch run_layers last ran
-    int n_out_rows_ = 0, out_first_ = -1;     // its flagged rows, and the first of them where they follow one another, else -1
+    int cur_T_ = 0;                    // tokens of the micro-batch run_layers_novorax last ran (run_output_novorax: a single row needs no gather)
+    int n_out_rows_ = 0, out_first_ = -1;     // flagged rows of the micro-batch in work, and the first of them where they follow one another, else -1
     std::vector<void *> allocs_;
     std::vector<KVCell> cells_;
     CellChunks cell_sums_;
