@@ -21,7 +21,7 @@ def be(pkg):
 # test_prefill_layers_logits_and_greedy_ids: the cases whose 24 teacher-forced steps hold TWO near ties of the CPU logits that the HIP path resolves the other
 # way (every other case: at most one) -> the largest relative top-2 gap such a flip may have (measured gaps in the comment; FLIP_TOL bounds any flip at 6e-2)
 TWO_FLIP_CASES = {
-    ("tiny-qwen2-1.5b-2l:70", "q4_k_m", "f16"): 1e-2,      # steps 6 and 15: gaps 7.8e-3 and 4.4e-3 of the logit scale (round 5, gpurun_out/r5_flips.txt)
+    ("tiny-qwen2-1.5b-2l:70", "q4_k_m", "f16"): 1e-2,      # steps 6 and 15: gaps 7.8e-3 and 4.4e-3 of the logit scale
     ("tiny-r3:40", "q4_k_m", "q8_0"): 1e-2,                # steps 7 and 14: gaps 4.8e-3 and 1.5e-3
     ("tiny-tl-2l", "q4_k_m", "f16"): 2e-3,                 # steps 5 and 16: gaps 1.2e-3 and 1.3e-4 (columns in the prompt; with the general attention's sums one of them)
 }
