@@ -177,7 +177,7 @@ def test_few_tokens_as_steps(pkg, tmp_path, model, past, n, kv):
         for i in range(past, past + n, each):
             assert c.decode(talk[i:i + each], np.arange(i, i + each), 0) == 0
         if model in ("tinyllama-1.1b", "tiny-qwen2") and each > 1:                                  # (no one-token kernel beside it: by the work, not by the number of cells)
-            assert c.batch_route()[0] == 2
+            assert c.batch_route()[0] & 2
         out.append(np.array(c.logits(-1)))
         c.close()
     m.close()
