@@ -287,7 +287,10 @@ int32_t mi355_debug_q80_plan(int32_t n_rows, int32_t n_cols, int32_t n_tokens) {
 int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder) {
     AttnArgs a{};
     a.T = n_tokens; a.H = n_head; a.G = n_head_kv; a.D = head_dim; a.n_ctx = a.n_kv_max = n_cells; a.type_k = a.type_v = type_kv;
-    return flash_attn_cols_takes(a, !encoder) ? flash_attn_cols_splits(a) : 0;
+    RopeArgs ra{};
+    ra.n_rot = head_dim;
+    const bool beside = !encoder && n_tokens <= 64 && flash_attn_decode_applicable(a, ra) && kv_store_fast_applicable(n_head_kv, head_dim, type_kv, type_kv, ra);
+    return flash_attn_cols_takes(a, beside) ? flash_attn_cols_splits(a) : 0;
 }
 int64_t mi355_debug_attn_planes_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_ctx, int32_t n_ubatch) {
     return (int64_t)flash_attn_prefill_planes_wanted(type_kv, type_kv, n_head, n_head_kv, head_dim, n_ctx, n_ubatch);

@@ -185,8 +185,8 @@ MI355_API int64_t mi355_debug_qkv_attn_plan(int32_t type_q, int32_t type_k, int3
 MI355_API int32_t mi355_debug_batch_plan(int32_t type, int32_t n_rows, int32_t n_cols, int32_t n_tokens, int32_t pair, int32_t sum_free);
 /* host logic only: rows and tokens of a wave in the kernel that a batch of n_tokens rows against a Q8_0 tensor of n_rows x n_cols takes (csrc/mmq_q80.hip): 16, 32 or 64; 0 the mat-vec */
 MI355_API int32_t mi355_debug_q80_plan(int32_t n_rows, int32_t n_cols, int32_t n_tokens);
-/* host logic only: does the attention of n_tokens of one conversation (encoder: of a text) over n_cells cells of type_kv go through csrc/attn_cols.hip?  Returns the number of workgroups
-   that share a tile's keys there, 0 = the one-token or the prompt kernel */
+/* host logic only: does the attention of n_tokens of one conversation (encoder: of a text; else rope of neighbouring pairs) over n_cells cells of type_kv go through csrc/attn_cols.hip?  Returns the number of workgroups
+   that share a tile's keys there, 0 = the one-token, the general or the prompt kernel */
 MI355_API int32_t mi355_debug_attn_plan(int32_t type_kv, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t n_tokens, int32_t n_cells, int32_t encoder);
 /* host logic only: bytes that a decoder's context of n_ctx cells (K and V of type_kv) and n_ubatch tokens a micro-batch keeps for the V planes of a prompt's attention
    (csrc/attn_prefill.hip); 0 where no micro-batch takes that form */

@@ -2,7 +2,7 @@
 import pytest
 
 F16, Q8_0 = 1, 8
-L8, L7, SMALL, TEXT = (Q8_0, 32, 8, 128), (F16, 32, 32, 128), (F16, 32, 4, 64), (F16, 12, 12, 64)
+L8, L7, MID, SMALL, TEXT = (Q8_0, 32, 8, 128), (F16, 32, 32, 128), (F16, 32, 16, 64), (F16, 32, 4, 64), (F16, 12, 12, 64)
 
 
 @pytest.fixture(scope="module")
@@ -14,7 +14,9 @@ def takes(pkg):
 @pytest.mark.parametrize("model,yes,no", [
     (L8, [(2, 2100), (3, 1900), (5, 1495), (14, 700), (31, 200), (40, 0), (37, 160), (64, 613)], [(2, 700), (5, 900), (8, 700), (12, 400), (22, 200), (31, 150), (32, 0), (1, 3900)]),
     (L7, [(2, 3000), (3, 1900), (5, 900), (12, 400), (32, 0)], [(2, 2100), (14, 200)]),
-    (SMALL, [(3, 1900), (8, 700), (22, 200)], [(14, 200), (2, 700)]),
+    (MID, [(3, 1900), (8, 700), (22, 200)], [(14, 200), (2, 700)]),
+    (SMALL, [(2, 0), (3, 0), (31, 20), (3, 1900), (8, 700), (22, 200), (14, 200), (2, 700)], []),                  # fewer than 1024 values of K a row: no one-token kernel beside the columns
+    ((Q8_0, 28, 4, 128), [(2, 0), (2, 60), (8, 500), (31, 30)], []),
 ])
 def test_short_batches(takes, model, yes, no):
     assert [c for c in yes if not takes(model, *c)] == [] and [c for c in no if takes(model, *c)] == []
